@@ -27,10 +27,12 @@
 // row groups with long windows (decode) cut every window into runs of key tiles over
 // gridDim.z; a second kernel merges the runs.
 #include "common.h"
+#include "attn_tile.h"
+#include "window_attn.h"
 using namespace sm;
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+
 
 // cap * tanh(v / cap) and ln(1 + x) on the hardware's exp2 / log2 / reciprocal units: a prompt
 // evaluates them once per (query, key, head), where the library forms (tanhf, log1pf) cost more
@@ -41,8 +43,6 @@ __device__ __forceinline__ float fast_tanh(float x) {
 }
 
 #define WM_LDK 36   // keys per transposed value row in LDS (32 + padding), in bf16
-
-enum { KEYS_WINDOW = 0, KEYS_BLOCKS = 1, KEYS_KEPT = 2 };
 
 template <int NK, int NV2, int KEYS, int MAPS>  // D padded to NK * 32, V padded to NV2 * 32
 __global__ void __launch_bounds__(64)
@@ -331,11 +331,12 @@ window_attn_mfma_k(const bf16* __restrict__ q, int ldq, const bf16* __restrict__
 }
 
 // Merges the runs of a split window: out = sum_z e^(m_z - M) acc_z / sum_z e^(m_z - M) l_z.
-// One block per (unit, head block, pair); the weights of the runs are formed once in LDS.
+// One block per (unit, head block, pair); the weights of the runs are formed once in LDS.  NP: pairs
+// of a record.
 __global__ void window_attn_merge_k(const float* __restrict__ part, const int* __restrict__ units,
                                     bf16* __restrict__ out, int ldo, int H, int G, int V, int HS,
                                     int splits, int VP, float out_scale,
-                                    const bf16* __restrict__ gate, int ldg, int gate_pc) {
+                                    const bf16* __restrict__ gate, int ldg, int gate_pc, int NP) {
   __shared__ float sw[65];
   const int r0 = units[2 * blockIdx.x], nr = units[2 * blockIdx.x + 1];
   const int HG = H / G, hblocks = (HG + HS - 1) / HS;
@@ -343,9 +344,9 @@ __global__ void window_attn_merge_k(const float* __restrict__ part, const int* _
   const int m = blockIdx.z;
   const int mr = m / HS, ms = hb0 + m % HS;
   if (mr >= nr || ms >= HG) return;
-  const float* rec = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * splits * 16 * (VP + 2) +
+  const float* rec = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * splits * NP * (VP + 2) +
                      (size_t)m * (VP + 2);
-  const size_t zs = (size_t)16 * (VP + 2);   // stride between runs
+  const size_t zs = (size_t)NP * (VP + 2);   // stride between runs
   if (threadIdx.x < 64) {
     int z = threadIdx.x;
     float mz = z < splits ? rec[z * zs + VP] : -INFINITY;
@@ -380,7 +381,7 @@ __global__ void window_attn_merge_k(const float* __restrict__ part, const int* _
 __global__ void __launch_bounds__(128)
 diff_attn_merge_k(const float* __restrict__ part, const int* __restrict__ units, bf16* __restrict__ out,
                   int ldo, int H, int G, int V, int HS, int splits, int VP, float out_scale, float lam,
-                  float eps) {
+                  float eps, int NP) {
   __shared__ float sw[2][65];
   __shared__ float red[16];
   const int nr = units[2 * blockIdx.x + 1], r0 = units[2 * blockIdx.x];
@@ -389,7 +390,7 @@ diff_attn_merge_k(const float* __restrict__ part, const int* __restrict__ units,
   const int m = blockIdx.z;
   const int mr = m / HS, ms = hb0 + m % HS;
   if (mr >= nr || ms >= HG) return;
-  const size_t ms_ = (size_t)16 * (VP + 2), zs = 2 * ms_;   // strides between maps and runs
+  const size_t ms_ = (size_t)NP * (VP + 2), zs = 2 * ms_;   // strides between maps and runs
   const float* rec = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * splits * zs + (size_t)m * (VP + 2);
   {
     const int u = threadIdx.x >> 6, z = threadIdx.x & 63;   // a wavefront per map
@@ -431,11 +432,6 @@ diff_attn_merge_k(const float* __restrict__ part, const int* __restrict__ units,
   }
 }
 
-static int pad32(int n) {   // 32-channel steps the kernel is instantiated for
-  int s = (n + 31) / 32;
-  return s <= 1 ? 1 : s <= 2 ? 2 : s <= 4 ? 4 : 8;
-}
-
 static int head_slots(int HG) {
   int hs = 1;
   while (hs < HG && hs < 16) hs *= 2;
@@ -444,20 +440,24 @@ static int head_slots(int HG) {
 
 extern "C" {
 
+// (row, head) pairs of a row group: a wavefront's, or (tile) those of a workgroup of window_attn_tile_k
+static int group_pairs(int tile) { return tile ? WINDOW_TILE_PAIRS : 16; }
+
 // floats of workspace for `splits` runs per window (0 when splits <= 1)
-long p2p_sm_window_attn_mfma_ws(int U, int H, int G, int V, int splits, int maps) {
+long p2p_sm_window_attn_mfma_ws(int U, int H, int G, int V, int splits, int maps, int tile) {
   if (splits <= 1 || G < 1 || H % G) return 0;
   int HG = H / G, HS = head_slots(HG);
-  return (long)U * G * ((HG + HS - 1) / HS) * splits * maps * 16 * (pad32(V) * 32 + 2);
+  return (long)U * G * ((HG + HS - 1) / HS) * splits * maps * group_pairs(tile) * (window_pad32(V) * 32 + 2);
 }
 
+// tile: the units are cut for window_attn_tile_k (64 / HS rows), which then runs instead
 int p2p_sm_window_attn_mfma(const void* q, int ldq, const void* pool, const int* bt,
                             int max_pages, const int* row_ent, const int* pos, const int* units,
                             int U, const float* sink, float scale, int win, void* out, int ldo,
                             int H, int G, int D, int V, int page, int splits, float* part,
                             float out_scale, float cap, const float* r1, const float* r2,
                             const void* gate, int ldg, int gate_pc, const void* blk, int P, int keep,
-                            int maps, float lam, float eps, hipStream_t st) {
+                            int maps, float lam, float eps, int tile, hipStream_t st) {
   if (U <= 0) return 0;
   // blocks stand for what lies before the window, kept tokens lie there as they are: one or the other;
   // the difference of two maps is normed, so nothing else comes after it
@@ -467,9 +467,16 @@ int p2p_sm_window_attn_mfma(const void* q, int ldq, const void* pool, const int*
       win < 1 || ldq % 8 || (r1 && !r2) || cap < 0.0f || (blk && (P < 1 || r1)))
     return (int)hipErrorInvalidValue;
   if (splits < 1 || splits > 64 || (splits > 1 && !part)) return (int)hipErrorInvalidValue;
-  int HG = H / G, HS = head_slots(HG);
-  dim3 grid(U, G * ((HG + HS - 1) / HS), splits), block(64);
-  int nk = pad32(D), nv = pad32(V);
+  const int HG = H / G, HS = head_slots(HG), hblocks = (HG + HS - 1) / HS;
+  const WindowArgs a = {(const bf16*)q, ldq, (const bf16*)pool, bt, max_pages, row_ent, pos, units, U, sink,
+                        scale, win, (bf16*)out, ldo, H, G, D, V, page, HS, splits, part, out_scale, cap, r1,
+                        r2, (const bf16*)gate, ldg, gate_pc, (const bf16*)blk, P, keep, lam, eps};
+  const int nk = window_pad32(D), nv = window_pad32(V);
+  int err = 0;
+  if (tile) {
+    err = window_attn_tile(a, maps, st);
+  } else {
+    const dim3 grid(U, G * hblocks, splits), block(64);
 #define WMB(NKK, NVV, KEYS, MAPS)                                                              \
   do {                                                                                         \
     size_t shm = (size_t)(MAPS * 16 * (NKK * 32 + 8) + NVV * 32 * WM_LDK) * 2;                 \
@@ -485,14 +492,6 @@ int p2p_sm_window_attn_mfma(const void* q, int ldq, const void* pool, const int*
     else if (blk) WMB(NKK, NVV, KEYS_BLOCKS, 1);                                               \
     else if (keep) WMB(NKK, NVV, KEYS_KEPT, 1);                                                \
     else WMB(NKK, NVV, KEYS_WINDOW, 1);                                                        \
-    if (splits > 1 && maps == 2)                                                               \
-      hipLaunchKernelGGL(diff_attn_merge_k, dim3(grid.x, grid.y, 16), dim3(128), 0, st, part,  \
-                         units, (bf16*)out, ldo, H, G, V, HS, splits, NVV * 32, out_scale, lam, \
-                         eps);                                                                 \
-    else if (splits > 1)                                                                       \
-      hipLaunchKernelGGL(window_attn_merge_k, dim3(grid.x, grid.y, 16), dim3(128), 0, st,      \
-                         part, units, (bf16*)out, ldo, H, G, V, HS, splits, NVV * 32,          \
-                         out_scale, (const bf16*)gate, ldg, gate_pc);                          \
   } while (0)
 #define WMV(NKK)                 \
   do {                           \
@@ -501,13 +500,23 @@ int p2p_sm_window_attn_mfma(const void* q, int ldq, const void* pool, const int*
     else if (nv == 4) WM(NKK, 4);\
     else WM(NKK, 8);             \
   } while (0)
-  if (nk == 1) WMV(1);
-  else if (nk == 2) WMV(2);
-  else if (nk == 4) WMV(4);
-  else WMV(8);
+    if (nk == 1) WMV(1);
+    else if (nk == 2) WMV(2);
+    else if (nk == 4) WMV(4);
+    else WMV(8);
 #undef WMV
 #undef WM
 #undef WMB
+    err = (int)hipGetLastError();
+  }
+  if (err || splits == 1) return err;
+  const dim3 mg(U, G * hblocks, group_pairs(tile));
+  if (maps == 2)
+    hipLaunchKernelGGL(diff_attn_merge_k, mg, dim3(128), 0, st, part, units, (bf16*)out, ldo, H, G, V, HS,
+                       splits, nv * 32, out_scale, lam, eps, group_pairs(tile));
+  else
+    hipLaunchKernelGGL(window_attn_merge_k, mg, dim3(128), 0, st, part, units, (bf16*)out, ldo, H, G, V, HS,
+                       splits, nv * 32, out_scale, (const bf16*)gate, ldg, gate_pc, group_pairs(tile));
   return (int)hipGetLastError();
 }
 

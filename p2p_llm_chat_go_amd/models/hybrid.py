@@ -343,6 +343,13 @@ class StepBatch:
                 self.ids.device)
         return u
 
+    def attn_units(self, rows_per_wave: int):
+        """(row groups, rows they were cut to) for an attention layer (``ops.seqmix.attn_unit_rows``)."""
+        rows = self._units.get(("rows", rows_per_wave))
+        if rows is None:
+            rows = self._units[("rows", rows_per_wave)] = sm.attn_unit_rows(rows_per_wave, self.ent_host)
+        return self.units(rows), rows
+
 
 # ---------------------------------------------------------------------------- mixers
 class Mixer:
@@ -674,9 +681,10 @@ class WindowAttention(Mixer):
         sm.qk_norm_rope_store(proj, H, G, D, V, self.qnorm, self.knorm, self.inv_freq, b.pos,
                               b.cache_rows, pool if own else None, self.eps, q,
                               per_head=self.PER_HEAD, half=self.HALF, rm=self.rot_mag)
-        units = b.units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) else None
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
+            else (None, None)
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
-                       out, PAGE, H, G, D, V, units=units, max_keys=b.max_keys, out_scale=out_scale,
+                       out, PAGE, H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale,
                        keep=self.keep)
         return out
 
@@ -739,9 +747,10 @@ class BiasedAttention(Mixer):
         nq, nkv = H * D, G * (D + V)
         q = torch.empty(b.R, nq, device=proj.device, dtype=proj.dtype)
         sm.qtemp_kv_store(proj, nq, nkv, self.qt_coef, self.qt_every, b.pos, b.cache_rows, pool, q)
-        units = b.units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) else None
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
+            else (None, None)
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
-                       out, PAGE, H, G, D, V, units=units, max_keys=b.max_keys, out_scale=out_scale,
+                       out, PAGE, H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale,
                        softcap=self.cap, dist=(self.r1, self.r2), gate=proj[:, nq + nkv:])
         return out
 
@@ -805,9 +814,10 @@ class ConvAttention(Mixer):
         sm.conv_rope_norm_store(proj, H, G, D, V, self.cw, cache.state[layer]["tail"], self.inv_freq,
                                 self.temp, b.pos, b.cache_rows, pool, self.eps, q, b.ent, b.ent_host,
                                 b.row_ent, b.block_tables, PAGE, blk=blk, every=self.pool)
-        units = b.units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) else None
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
+            else (None, None)
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, out, PAGE,
-                       H, G, D, V, units=units, max_keys=b.max_keys, out_scale=out_scale,
+                       H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale,
                        gate=proj[:, self.C:], gate_channels=True, blk=blk, every=self.pool)
         return out
 
@@ -882,9 +892,10 @@ class DiffAttention(Mixer):
         sm.conv_rope_norm_store(proj, H, G, D, V, self.cw, cache.state[layer]["tail"], self.inv_freq, None,
                                 b.pos, b.cache_rows, pool if own else None, self.eps, q, b.ent, b.ent_host,
                                 b.row_ent, b.block_tables, PAGE, maps=2, norm=False, rm=self.rot_mag)
-        units = b.units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) else None
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
+            else (None, None)
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, out, PAGE,
-                       H, G, D, V, units=units, max_keys=b.max_keys, out_scale=out_scale * (1.0 - self.diff),
+                       H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale * (1.0 - self.diff),
                        keep=self.keep, diff=(self.lam, self.eps))
         return out
 

@@ -142,7 +142,7 @@ _SIGS = {
                                 c_void_p, c_int, c_void_p, c_float, c_int, c_void_p, c_int, c_int,
                                 c_int, c_int, c_int, c_int, c_int, c_void_p, c_float, c_float,
                                 c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int,
-                                c_int, c_int, c_float, c_float, c_void_p],
+                                c_int, c_int, c_float, c_float, c_int, c_void_p],
     "p2p_sm_hgrn2_scan": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                           c_int, c_void_p, c_int, c_int, c_int, c_int, c_float, c_float, c_int,
                           c_void_p],
@@ -936,6 +936,15 @@ def latent_mfma_ok(qa, cache) -> bool:
             and cache.data_ptr() % 16 == 0 and os.environ.get("P2P_LATENT_MFMA", "1") != "0")
 
 
+def _tiled_units(unit_rows, rows_per_wave: int) -> int:
+    """1 when units were cut for the kernel whose wavefronts share key tiles, 0 for one wavefront each."""
+    if unit_rows is None or unit_rows == rows_per_wave:
+        return 0
+    if unit_rows != 4 * rows_per_wave:
+        raise ValueError("row groups of %d, a wavefront takes %d" % (unit_rows, rows_per_wave))
+    return 1
+
+
 LATENT_SPLIT_BLOCKS = 512   # split windows while a step has fewer blocks than this
 
 
@@ -1411,6 +1420,16 @@ def window_rows_per_wave(HG: int) -> int:
     return latent_rows_per_wave(HG)
 
 
+def attn_unit_rows(rows_per_wave: int, ent_host: list) -> int:
+    """Rows per group (``make_units``) that a step's attention is cut into: those of one wavefront, or
+    four times as many for the kernels whose four wavefronts share the key tiles.  Those win as
+    soon as half of their rows are taken (a group of a decoded token leaves three of the four
+    wavefronts idle)."""
+    tile = 4 * rows_per_wave
+    groups = sum(-(-e[1] // tile) for e in ent_host)
+    return tile if 2 * sum(e[1] for e in ent_host) >= groups * tile else rows_per_wave
+
+
 def window_mfma_ok(q, pool, D: int, V: int) -> bool:
     """The matrix-core kernel serves bf16 with key / value sizes that are multiples of 8 up to
     256 and 16-byte aligned rows.  P2P_WINDOW_MFMA=0 switches it off."""
@@ -1423,7 +1442,7 @@ def window_mfma_ok(q, pool, D: int, V: int) -> bool:
 def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: int, out, page: int,
                 H: int, G: int, D: int, V: int, units=None, max_keys=None, out_scale: float = 1.0,
                 softcap: float = 0.0, dist=None, gate=None, gate_channels: bool = False,
-                blk=None, every: int = 0, keep: int = 0, diff=None):
+                blk=None, every: int = 0, keep: int = 0, diff=None, unit_rows=None):
     """Grouped-query attention over a paged key/value pool with a causal sliding window and a
     softmax sink.
 
@@ -1448,7 +1467,9 @@ def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: in
     same values; head h leaves as o = a_1 - lam a_2, divided by sqrt(mean(o^2) + eps) over its V
     channels, times out_scale (no sink, gate or blk).
     units: ``make_units(entries, window_rows_per_wave(H // G))`` on the device; with it bf16
-    inputs run on the matrix cores (``window_mfma_ok``)."""
+    inputs run on the matrix cores (``window_mfma_ok``).  unit_rows: the rows that the units were
+    cut to where they are others, four times as many (``attn_unit_rows``): groups of rows that
+    share key tiles."""
     R = q.shape[0]
     HG = H // G
     M = 2 if diff is not None else 1
@@ -1519,16 +1540,17 @@ def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: in
         assert units.dtype == torch.int32 and units.is_contiguous() and units.shape[1] == 2
         U = units.shape[0]
         hs = 16 // window_rows_per_wave(HG)
+        tile = _tiled_units(unit_rows, window_rows_per_wave(HG))
         blocks = U * G * (-(-HG // hs))
         splits = 1
         if max_keys is not None and blocks < LATENT_SPLIT_BLOCKS:
             most = min(max_keys, win + keep) + (max(0, max_keys - win) // every if blk is not None else 0)
-            splits = max(1, min(-(-most // 64), LATENT_SPLIT_BLOCKS // blocks, 64))
+            splits = max(1, min(-(-most // (256 if tile else 64)), LATENT_SPLIT_BLOCKS // blocks, 64))
         part = None
         if splits > 1:
             L = lib()
             L.p2p_sm_window_attn_mfma_ws.restype = c_long
-            part = torch.empty(L.p2p_sm_window_attn_mfma_ws(U, H, G, V, splits, M), device=q.device,
+            part = torch.empty(L.p2p_sm_window_attn_mfma_ws(U, H, G, V, splits, M, tile), device=q.device,
                                dtype=torch.float32)
         _chk(lib().p2p_sm_window_attn_mfma(q.data_ptr(), q.stride(0), pool.data_ptr(),
                                            block_tables.data_ptr(), block_tables.shape[1],
@@ -1538,7 +1560,7 @@ def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: in
                                            out_scale, softcap, _lib.ptr(r1), _lib.ptr(r2),
                                            _lib.ptr(gate), ldg, gpc, _lib.ptr(blk), every, keep, M,
                                            diff[0] if M == 2 else 0.0, diff[1] if M == 2 else 0.0,
-                                           _st(q)), "window_attn_mfma")
+                                           tile, _st(q)), "window_attn_mfma")
         return out
     dst = out if M == 1 else torch.empty(R, H * 2 * V, device=q.device, dtype=torch.float32)
     _chk(lib().p2p_sm_window_attn(q.data_ptr(), q.stride(0), pool.data_ptr(),

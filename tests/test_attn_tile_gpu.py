@@ -1,0 +1,86 @@
+"""The attention kernels whose wavefronts share key tiles in LDS against the PyTorch rendering of the
+same ops: row groups that are full, ragged and of one row, portions that begin inside a sequence,
+tiles cut by the window's ends, key lists of blocks and of kept tokens, windows cut into runs."""
+import pytest
+import torch
+
+from p2p_llm_chat_go_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+PAGE = 64
+# portions (rows, first position): tile remainders, a long prefix, a single row among them
+STEPS = {"prompts": ([129, 37, 64], [0, 0, 64]), "portions": ([70, 9, 1], [3, 180, 131]), "short": ([5], [0])}
+
+
+def _step(name, seed):
+    lens, starts = STEPS[name]
+    ent, r0 = [], 0
+    for i, (n, s) in enumerate(zip(lens, starts)):
+        ent.append((r0, n, s, i))
+        r0 += n
+    row_ent = torch.tensor([i for i, e in enumerate(ent) for _ in range(e[1])], dtype=torch.int32)
+    pos = torch.tensor([e[2] + k for e in ent for k in range(e[1])], dtype=torch.int32)
+    g = torch.Generator().manual_seed(seed)
+    bt = (torch.randperm(len(ent) * 3, generator=g) + 1).to(torch.int32).view(len(ent), 3)
+    return ent, row_ent, pos, bt, r0, g
+
+
+def _close(got, want):
+    # probabilities and results are rounded to bf16 (2^-9 each) beside values of about one: a weighted
+    # mean of values up to 4.5 in size is off by at most 2 * 2^-9 * 4.5 = 1.8e-2
+    torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1e-2, atol=1.8e-2)
+
+
+@pytest.mark.parametrize("step", sorted(STEPS))
+@pytest.mark.parametrize("H,G,D,V", [(8, 2, 128, 128), (3, 1, 24, 40), (4, 4, 16, 8), (34, 2, 8, 16),
+                                     (4, 2, 136, 200), (16, 1, 64, 256)])
+@pytest.mark.parametrize("form", ["window", "sink", "biased", "blocks", "kept", "maps"])
+def test_window_attention_tiles(step, H, G, D, V, form):
+    ent, row_ent, pos, bt, R, g = _step(step, 3)
+    M = 2 if form == "maps" else 1
+    win = {"window": 1 << 30, "biased": 1 << 30, "sink": 33, "blocks": 50, "kept": 21, "maps": 40}[form]
+    q = torch.randn(R, H * M * D, generator=g).bfloat16()
+    pool = torch.randn((int(bt.max()) + 1) * PAGE, G * (M * D + V), generator=g).bfloat16()
+    sink, kw, dev = None, dict(out_scale=0.7), {}
+    if form == "sink":
+        sink = torch.randn(H, generator=g)
+    if form == "biased":
+        sink = torch.zeros(H)
+        dev.update(dist=(torch.rand(H, generator=g) * 2, torch.rand(H, generator=g) * 0.3),
+                   gate=torch.randn(R, H + 3, generator=g).bfloat16())
+        kw.update(softcap=9.0)
+    if form == "blocks":
+        dev.update(blk=torch.randn((int(bt.max()) + 1) * sm.blocks_per_page(PAGE, 12), G * (D + V),
+                                   generator=g).bfloat16(), gate=torch.randn(R, H * V, generator=g).bfloat16())
+        kw.update(every=12, gate_channels=True)
+    if form in ("kept", "maps"):
+        kw.update(keep=9)
+    if form == "maps":
+        kw.update(diff=(0.4, 1e-4))
+    scale = 1.3 / D ** 0.5
+    want = sm.window_attn(q, pool, bt, row_ent, pos, sink, scale, win, torch.empty(R, H * V).bfloat16(), PAGE, H, G,
+                          D, V, **kw, **dev)
+    to = lambda t: tuple(x.to(DEV) for x in t) if isinstance(t, tuple) else t.to(DEV) if t is not None else None
+    rows = 4 * sm.window_rows_per_wave(H // G)
+    units = sm.make_units(ent, rows).to(DEV)
+    dev = {k: to(v) for k, v in dev.items()}
+    for max_keys in (None, 700):    # whole key lists / cut into runs
+        out = torch.full((R, H * V + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        sm.window_attn(to(q), to(pool), to(bt), to(row_ent), to(pos), to(sink), scale, win, out[:, :H * V], PAGE, H, G,
+                       D, V, units=units, unit_rows=rows, max_keys=max_keys, **kw, **dev)
+        _close(out[:, :H * V], want)
+        assert bool((out[:, H * V:] == 7.0).all())
+
+
+def test_group_size():
+    one = [(i, 1, 5, i) for i in range(8)]
+    assert sm.attn_unit_rows(4, one) == 4                     # decoded tokens
+    assert sm.attn_unit_rows(4, [(0, 300, 0, 0)]) == 16       # a prompt
+    assert sm.attn_unit_rows(4, [(0, 300, 0, 0)] + [(300 + i, 1, 9, i + 1) for i in range(8)]) == 16
+    assert sm.attn_unit_rows(4, [(0, 7, 0, 0)]) == 4          # less than half of one group
+    q = torch.zeros(2, 8, dtype=torch.bfloat16, device=DEV)
+    z = torch.zeros(2, dtype=torch.int32, device=DEV)
+    with pytest.raises(ValueError):
+        sm.window_attn(q, torch.zeros(64, 16, dtype=torch.bfloat16, device=DEV), z.view(2, 1), z, z, None, 1.0, 1, q,
+                       PAGE, 1, 1, 8, 8, units=sm.make_units([(0, 2, 0, 0)], 16).to(DEV), unit_rows=5)
