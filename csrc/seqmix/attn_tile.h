@@ -37,6 +37,10 @@ __device__ __forceinline__ unsigned lds_address(const void* p) {
 }
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
+// What is computed from x after this is computed after this: keeps a loop's addresses out of registers
+// that its accumulators need.
+__device__ __forceinline__ void again(int& x) { asm volatile("" : "+v"(x)); }
+
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ bf16x8 to_bf16(f32x8 v) { return __builtin_convertvector(v, bf16x8); }
 

@@ -14,11 +14,9 @@
 // transposed to LDS, where the second product reads them as B operands.  One wavefront per
 // workgroup, no cross-wave synchronisation.  `units` (int32 x 2: first row, rows) lists the
 // row groups; a group never spans two portions.
-#include "common.h"
+#include "attn_tile.h"
+#include "latent_attn.h"
 using namespace sm;
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define LM_LDK 36   // keys per transposed row in LDS (32 + padding), in bf16: rows 72 bytes apart
                     // spread the four key-index slices over different banks
@@ -193,18 +191,19 @@ latent_attn_mfma_k(const bf16* __restrict__ qa, long sqh, long sqr, const bf16* 
 }
 
 // Merges the runs of a split window: out = sum_z e^(m_z - M) acc_z / sum_z e^(m_z - M) l_z.
-// One block per (unit, head group, pair); the weights of the runs are formed once in LDS.
+// One block per (unit, head group, pair); the weights of the runs are formed once in LDS.  NP: pairs of a
+// record.
 __global__ void latent_attn_merge_k(const float* __restrict__ part, const int* __restrict__ units,
                                     bf16* __restrict__ out, long soh, long sor, int H, int rank,
-                                    int HS, int splits, int RP) {
+                                    int HS, int splits, int RP, int NP) {
   __shared__ float sw[65];
   const int r0 = units[2 * blockIdx.x], nr = units[2 * blockIdx.x + 1];
   const int m = blockIdx.z;
   const int mr = m / HS, mh = blockIdx.y * HS + m % HS;
   if (mr >= nr || mh >= H) return;
-  const float* rec = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * splits * 16 * (RP + 2) +
+  const float* rec = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * splits * NP * (RP + 2) +
                      (size_t)m * (RP + 2);
-  const size_t zs = (size_t)16 * (RP + 2);   // stride between runs
+  const size_t zs = (size_t)NP * (RP + 2);   // stride between runs
   if (threadIdx.x < 64) {
     int z = threadIdx.x;
     float mz = z < splits ? rec[z * zs + RP] : -INFINITY;
@@ -242,44 +241,62 @@ int p2p_sm_latent_attn_mfma_rows(int H) {
   return 16 / hs;
 }
 
+// the rank the kernels are instantiated for, in steps of 32
+static int padded(int rank) {
+  const int n = (rank + 31) / 32;
+  return n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : n <= 8 ? 8 : 16;
+}
+
+// 1 when latent_attn_tile_k serves this rank; its row groups are four times as long
+static int tiled(int rank, int tile) { return tile && padded(rank) > 1; }
+
 // floats of workspace for `splits` runs per window (0 when splits <= 1)
-long p2p_sm_latent_attn_mfma_ws(int U, int H, int rank, int splits) {
+long p2p_sm_latent_attn_mfma_ws(int U, int H, int rank, int splits, int tile) {
   if (splits <= 1) return 0;
   int HS = 16 / p2p_sm_latent_attn_mfma_rows(H);
-  int n = (rank + 31) / 32;
-  int N = n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : n <= 8 ? 8 : 16;
-  return (long)U * ((H + HS - 1) / HS) * splits * 16 * (N * 32 + 2);
+  return (long)U * ((H + HS - 1) / HS) * splits * (tiled(rank, tile) ? LATENT_TILE_PAIRS : 16) *
+         (padded(rank) * 32 + 2);
 }
 
 // splits > 1: each window is cut into that many runs of key tiles (decode steps: few rows,
-// long windows), partial results in `part` (p2p_sm_latent_attn_mfma_ws floats), then merged
+// long windows), partial results in `part` (p2p_sm_latent_attn_mfma_ws floats), then merged.
+// tile: the units are cut for latent_attn_tile_k, which then runs instead
 int p2p_sm_latent_attn_mfma(const void* qa, long sqh, long sqr, const void* cache, const int* bt,
                             int max_pages, const int* row_ent, const int* pos, const int* units,
                             int U, const float* sink, float scale, int win, void* out, long soh,
-                            long sor, int H, int rank, int page, int splits, float* part,
+                            long sor, int H, int rank, int page, int splits, float* part, int tile,
                             hipStream_t st) {
   if (U <= 0) return 0;
-  if (!p2p_sm_latent_attn_mfma_ok(H, rank) || win < 1) return (int)hipErrorInvalidValue;
+  if (!p2p_sm_latent_attn_mfma_ok(H, rank) || win < 1 || (tile && !tiled(rank, tile)))
+    return (int)hipErrorInvalidValue;
   if (splits < 1 || splits > 64 || (splits > 1 && !part)) return (int)hipErrorInvalidValue;
   int HS = 16 / p2p_sm_latent_attn_mfma_rows(H);
-  dim3 grid(U, (H + HS - 1) / HS, splits), block(64);
+  const dim3 grid(U, (H + HS - 1) / HS, splits), block(64);
+  const int n = padded(rank), np = tile ? LATENT_TILE_PAIRS : 16;
+  int err = 0;
+  if (tile) {
+    const LatentArgs a = {(const bf16*)qa, sqh, sqr, (const bf16*)cache, bt, max_pages, row_ent, pos, units,
+                          U, sink, scale, win, (bf16*)out, soh, sor, H, rank, page, HS, splits, part};
+    err = latent_attn_tile(a, st);
+  } else {
 #define LM(N)                                                                                  \
   do {                                                                                         \
     size_t shm = (size_t)(16 * (N * 32 + 8) + N * 32 * LM_LDK) * 2;                            \
     hipLaunchKernelGGL((latent_attn_mfma_k<N>), grid, block, shm, st, (const bf16*)qa, sqh,    \
                        sqr, (const bf16*)cache, bt, max_pages, row_ent, pos, units, sink,      \
                        scale, win, (bf16*)out, soh, sor, H, rank, page, HS, splits, part);     \
-    if (splits > 1)                                                                            \
-      hipLaunchKernelGGL(latent_attn_merge_k, dim3(grid.x, grid.y, 16), dim3(128), 0, st, part, \
-                         units, (bf16*)out, soh, sor, H, rank, HS, splits, N * 32);            \
   } while (0)
-  int n = (rank + 31) / 32;
-  if (n <= 1) LM(1);
-  else if (n <= 2) LM(2);
-  else if (n <= 4) LM(4);
-  else if (n <= 8) LM(8);
-  else LM(16);
+    if (n == 1) LM(1);
+    else if (n == 2) LM(2);
+    else if (n == 4) LM(4);
+    else if (n == 8) LM(8);
+    else LM(16);
 #undef LM
+    err = (int)hipGetLastError();
+  }
+  if (err || splits == 1) return err;
+  hipLaunchKernelGGL(latent_attn_merge_k, dim3(grid.x, grid.y, np), dim3(128), 0, st, part, units, (bf16*)out,
+                     soh, sor, H, rank, HS, splits, n * 32, np);
   return (int)hipGetLastError();
 }
 

@@ -343,8 +343,11 @@ class StepBatch:
                 self.ids.device)
         return u
 
-    def attn_units(self, rows_per_wave: int):
-        """(row groups, rows they were cut to) for an attention layer (``ops.seqmix.attn_unit_rows``)."""
+    def attn_units(self, rows_per_wave: int, shared: bool = True):
+        """(row groups, rows they were cut to) for an attention layer (``ops.seqmix.attn_unit_rows``;
+        not ``shared``: the layer has no kernel of shared key tiles)."""
+        if not shared:
+            return self.units(rows_per_wave), rows_per_wave
         rows = self._units.get(("rows", rows_per_wave))
         if rows is None:
             rows = self._units[("rows", rows_per_wave)] = sm.attn_unit_rows(rows_per_wave, self.ent_host)
@@ -607,9 +610,10 @@ class LatentAttention(Mixer):
         sm.rmsnorm(proj[:, H * D:H * D + r], self.cnorm, self.eps, pool, out_rows=b.cache_rows)
         qa = torch.bmm(proj[:, :H * D].view(b.R, H, D).transpose(0, 1), self.uk)   # [H, R, rank]
         ol = torch.empty_like(qa)
-        units = b.units(sm.latent_rows_per_wave(H)) if sm.latent_mfma_ok(qa, pool) else None
+        units, rows = b.attn_units(sm.latent_rows_per_wave(H), pool.shape[1] > 32) if sm.latent_mfma_ok(qa, pool) \
+            else (None, None)
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
-                       ol, PAGE, units=units, max_keys=b.max_keys)
+                       ol, PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
         o = torch.bmm(ol, self.uvt)                                                # [H, R, V]
         gated = torch.empty(b.R, H * V, device=h.device, dtype=h.dtype)
         sm.sigmoid_gate(o, proj[:, H * D + r:], gated, H, V)
@@ -986,9 +990,10 @@ class RopeLatentAttention(Mixer):
         if nrot2 < Rd:
             qa[:, :, r + nrot2:] = q3[:, :, D + nrot2:].transpose(0, 1)
         ol = torch.empty_like(qa)
-        units = b.units(sm.latent_rows_per_wave(H)) if sm.latent_mfma_ok(qa, pool) else None
+        units, rows = b.attn_units(sm.latent_rows_per_wave(H), pool.shape[1] > 32) if sm.latent_mfma_ok(qa, pool) \
+            else (None, None)
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, ol,
-                       PAGE, units=units, max_keys=b.max_keys)
+                       PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
         if not self.HEAD_GATE:
             torch.bmm(ol[:, :, :r], self.uvt, out=out.unflatten(1, (H, V)).transpose(0, 1))
             if out_scale != 1.0:

@@ -89,7 +89,7 @@ _SIGS = {
                            c_int, c_int, c_int, c_int, c_void_p],
     "p2p_sm_latent_attn_mfma": [c_void_p, c_long, c_long, c_void_p, c_void_p, c_int, c_void_p,
                                 c_void_p, c_void_p, c_int, c_void_p, c_float, c_int, c_void_p,
-                                c_long, c_long, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
+                                c_long, c_long, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
     "p2p_sm_tanh": [c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "p2p_sm_sigmoid_gate": [c_void_p, c_long, c_long, c_void_p, c_int, c_void_p, c_int, c_int,
                             c_int, c_int, c_int, c_int, c_void_p],
@@ -949,7 +949,7 @@ LATENT_SPLIT_BLOCKS = 512   # split windows while a step has fewer blocks than t
 
 
 def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: int, out,
-                page: int, units=None, max_keys=None):
+                page: int, units=None, max_keys=None, unit_rows=None):
     """Windowed attention over cached latents with a softmax sink.
 
     qa [H, R, rank] (any strides, last = 1): the queries already carried into latent space
@@ -961,7 +961,9 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
     the matching query part to qa; the columns of out beyond the latent are then not used.
     units: ``make_units(entries, latent_rows_per_wave(H))`` on the device; with
     it, bf16 inputs run on the matrix cores (``latent_mfma_ok``).  max_keys: an upper bound of
-    the keys any row sees (host side; lets a step of few rows split its windows)."""
+    the keys any row sees (host side; lets a step of few rows split its windows).  unit_rows: the rows
+    that the units were cut to where they are others, four times as many (``attn_unit_rows``; latents of
+    more than 32 numbers): groups of rows that share key tiles."""
     H, R, rank = qa.shape
     if not qa.is_cuda:
         bt = block_tables.long()
@@ -990,14 +992,15 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
         # so that the step fills the chip; the runs are merged by a second small kernel
         U = units.shape[0]
         hg = -(-H // (16 // latent_rows_per_wave(H)))
+        tile = _tiled_units(unit_rows, latent_rows_per_wave(H))
         splits = 1
         if max_keys is not None and U * hg < LATENT_SPLIT_BLOCKS:
-            splits = max(1, min(-(-min(max_keys, win) // 64), LATENT_SPLIT_BLOCKS // (U * hg), 64))
+            splits = max(1, min(-(-min(max_keys, win) // (256 if tile else 64)), LATENT_SPLIT_BLOCKS // (U * hg), 64))
         part = None
         if splits > 1:
             L = lib()
             L.p2p_sm_latent_attn_mfma_ws.restype = c_long
-            n = L.p2p_sm_latent_attn_mfma_ws(U, H, rank, splits)
+            n = L.p2p_sm_latent_attn_mfma_ws(U, H, rank, splits, tile)
             part = torch.empty(n, device=qa.device, dtype=torch.float32)
         _chk(lib().p2p_sm_latent_attn_mfma(qa.data_ptr(), qa.stride(0), qa.stride(1),
                                            cache.data_ptr(), block_tables.data_ptr(),
@@ -1005,7 +1008,7 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
                                            pos.data_ptr(), units.data_ptr(), units.shape[0],
                                            _lib.ptr(sink), scale, win, out.data_ptr(),
                                            out.stride(0), out.stride(1), H, rank, page, splits,
-                                           _lib.ptr(part), _st(qa)),
+                                           _lib.ptr(part), tile, _st(qa)),
              "latent_attn_mfma")
         return out
     if not latent_attn_ok(H, rank):

@@ -84,3 +84,23 @@ def test_group_size():
     with pytest.raises(ValueError):
         sm.window_attn(q, torch.zeros(64, 16, dtype=torch.bfloat16, device=DEV), z.view(2, 1), z, z, None, 1.0, 1, q,
                        PAGE, 1, 1, 8, 8, units=sm.make_units([(0, 2, 0, 0)], 16).to(DEV), unit_rows=5)
+
+
+@pytest.mark.parametrize("step", sorted(STEPS))
+@pytest.mark.parametrize("H,rank", [(16, 512), (3, 64), (1, 72), (34, 40), (8, 256), (5, 328), (16, 128)])
+@pytest.mark.parametrize("win,sunk", [(1 << 30, False), (37, True), (64, False)])
+def test_latent_attention_tiles(step, H, rank, win, sunk):
+    ent, row_ent, pos, bt, R, g = _step(step, 7)
+    qa = torch.randn(H, R, rank + 8, generator=g).bfloat16()[:, :, :rank]
+    cache = torch.randn((int(bt.max()) + 1) * PAGE, rank, generator=g).bfloat16()
+    sink = torch.randn(H, generator=g) if sunk else None
+    scale = 1.3 / rank ** 0.5
+    want = sm.latent_attn(qa, cache, bt, row_ent, pos, sink, scale, win, torch.empty(H, R, rank).bfloat16(), PAGE)
+    rows = 4 * sm.latent_rows_per_wave(H)
+    units = sm.make_units(ent, rows).to(DEV)
+    for max_keys in (None, 700):    # whole windows / cut into runs
+        out = torch.full((H, R, rank), 7.0, dtype=torch.bfloat16, device=DEV)
+        q2 = torch.empty(H, R, rank + 8, dtype=torch.bfloat16, device=DEV)[:, :, :rank].copy_(qa)
+        sm.latent_attn(q2, *(t.to(DEV) for t in (cache, bt, row_ent, pos)), sink.to(DEV) if sunk else None, scale, win,
+                       out, PAGE, units=units, unit_rows=rows, max_keys=max_keys)
+        _close(out, want)
