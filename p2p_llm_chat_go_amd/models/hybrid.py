@@ -610,8 +610,7 @@ class LatentAttention(Mixer):
         sm.rmsnorm(proj[:, H * D:H * D + r], self.cnorm, self.eps, pool, out_rows=b.cache_rows)
         qa = torch.bmm(proj[:, :H * D].view(b.R, H, D).transpose(0, 1), self.uk)   # [H, R, rank]
         ol = torch.empty_like(qa)
-        units, rows = b.attn_units(sm.latent_rows_per_wave(H), pool.shape[1] > 32) if sm.latent_mfma_ok(qa, pool) \
-            else (None, None)
+        units, rows = b.attn_units(sm.latent_rows_per_wave(H), sm.latent_mfma_ok(qa, pool) and pool.shape[1] > 32)
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
                        ol, PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
         o = torch.bmm(ol, self.uvt)                                                # [H, R, V]
@@ -685,8 +684,7 @@ class WindowAttention(Mixer):
         sm.qk_norm_rope_store(proj, H, G, D, V, self.qnorm, self.knorm, self.inv_freq, b.pos,
                               b.cache_rows, pool if own else None, self.eps, q,
                               per_head=self.PER_HEAD, half=self.HALF, rm=self.rot_mag)
-        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
-            else (None, None)
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G), sm.window_mfma_ok(q, pool, D, V))
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
                        out, PAGE, H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale,
                        keep=self.keep)
@@ -751,8 +749,7 @@ class BiasedAttention(Mixer):
         nq, nkv = H * D, G * (D + V)
         q = torch.empty(b.R, nq, device=proj.device, dtype=proj.dtype)
         sm.qtemp_kv_store(proj, nq, nkv, self.qt_coef, self.qt_every, b.pos, b.cache_rows, pool, q)
-        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
-            else (None, None)
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G), sm.window_mfma_ok(q, pool, D, V))
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
                        out, PAGE, H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale,
                        softcap=self.cap, dist=(self.r1, self.r2), gate=proj[:, nq + nkv:])
@@ -818,8 +815,7 @@ class ConvAttention(Mixer):
         sm.conv_rope_norm_store(proj, H, G, D, V, self.cw, cache.state[layer]["tail"], self.inv_freq,
                                 self.temp, b.pos, b.cache_rows, pool, self.eps, q, b.ent, b.ent_host,
                                 b.row_ent, b.block_tables, PAGE, blk=blk, every=self.pool)
-        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
-            else (None, None)
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G), sm.window_mfma_ok(q, pool, D, V))
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, out, PAGE,
                        H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale,
                        gate=proj[:, self.C:], gate_channels=True, blk=blk, every=self.pool)
@@ -896,8 +892,7 @@ class DiffAttention(Mixer):
         sm.conv_rope_norm_store(proj, H, G, D, V, self.cw, cache.state[layer]["tail"], self.inv_freq, None,
                                 b.pos, b.cache_rows, pool if own else None, self.eps, q, b.ent, b.ent_host,
                                 b.row_ent, b.block_tables, PAGE, maps=2, norm=False, rm=self.rot_mag)
-        units, rows = b.attn_units(sm.window_rows_per_wave(H // G)) if sm.window_mfma_ok(q, pool, D, V) \
-            else (None, None)
+        units, rows = b.attn_units(sm.window_rows_per_wave(H // G), sm.window_mfma_ok(q, pool, D, V))
         sm.window_attn(q, pool, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, out, PAGE,
                        H, G, D, V, units=units, unit_rows=rows, max_keys=b.max_keys, out_scale=out_scale * (1.0 - self.diff),
                        keep=self.keep, diff=(self.lam, self.eps))
@@ -990,8 +985,7 @@ class RopeLatentAttention(Mixer):
         if nrot2 < Rd:
             qa[:, :, r + nrot2:] = q3[:, :, D + nrot2:].transpose(0, 1)
         ol = torch.empty_like(qa)
-        units, rows = b.attn_units(sm.latent_rows_per_wave(H), pool.shape[1] > 32) if sm.latent_mfma_ok(qa, pool) \
-            else (None, None)
+        units, rows = b.attn_units(sm.latent_rows_per_wave(H), sm.latent_mfma_ok(qa, pool) and pool.shape[1] > 32)
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, ol,
                        PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
         if not self.HEAD_GATE:

@@ -90,6 +90,11 @@ _SIGS = {
     "p2p_sm_latent_attn_mfma": [c_void_p, c_long, c_long, c_void_p, c_void_p, c_int, c_void_p,
                                 c_void_p, c_void_p, c_int, c_void_p, c_float, c_int, c_void_p,
                                 c_long, c_long, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
+    "p2p_sm_attn_f32": [c_void_p, c_long, c_long, c_long, c_void_p, c_int, c_int, c_void_p, c_int,
+                        c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_float, c_int, c_void_p,
+                        c_long, c_long, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                        c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
+                        c_int, c_int, c_int, c_void_p],
     "p2p_sm_tanh": [c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "p2p_sm_sigmoid_gate": [c_void_p, c_long, c_long, c_void_p, c_int, c_void_p, c_int, c_int,
                             c_int, c_int, c_int, c_int, c_void_p],
@@ -936,6 +941,35 @@ def latent_mfma_ok(qa, cache) -> bool:
             and cache.data_ptr() % 16 == 0 and os.environ.get("P2P_LATENT_MFMA", "1") != "0")
 
 
+def attn_f32_ok(q, pool, D: int, V: int) -> bool:
+    """The fp32 matrix-instruction kernel serves float32 with key / value sizes that are multiples of 4
+    up to 512 and 16-byte aligned rows; it needs row groups (``units``)."""
+    return (q.is_cuda and q.dtype == torch.float32 and D % 4 == 0 and V % 4 == 0 and 4 <= D <= 512
+            and 4 <= V <= 512 and all(st % 4 == 0 for st in q.stride()[:-1]) and q.data_ptr() % 16 == 0
+            and pool.data_ptr() % 16 == 0 and pool.shape[1] % 4 == 0)
+
+
+def _attn_f32(q, sqh: int, sqr: int, sqm: int, pool, vbase: int, block_tables, row_ent, pos, units, sink, scale,
+              win: int, out, soh: int, sor: int, som: int, H: int, G: int, D: int, V: int, page: int, most,
+              out_scale: float = 1.0, cap: float = 0.0, r1=None, r2=None, gate=None, ldg: int = 0, gpc: int = 0,
+              blk=None, every: int = 0, keep: int = 0, maps: int = 1):
+    """most: a bound of the keys a row sees (None: windows are not cut).  A step of fewer workgroups
+    than two per CU cuts its windows into runs of at least 128 keys (two tiles per wavefront)."""
+    U, hs = units.shape[0], 16 // latent_rows_per_wave(H // G)
+    blocks, splits = U * G * maps * (-(-(H // G) // hs)), 1
+    if most is not None and blocks < LATENT_SPLIT_BLOCKS:
+        splits = max(1, min(-(-most // 128), LATENT_SPLIT_BLOCKS // blocks, 64))
+    L, part = lib(), None
+    if splits > 1:
+        L.p2p_sm_attn_f32_ws.restype = c_long
+        part = torch.empty(L.p2p_sm_attn_f32_ws(U, H, G, V, splits, maps), device=q.device, dtype=torch.float32)
+    _chk(L.p2p_sm_attn_f32(q.data_ptr(), sqh, sqr, sqm, pool.data_ptr(), pool.shape[1], vbase, block_tables.data_ptr(),
+                           block_tables.shape[1], row_ent.data_ptr(), pos.data_ptr(), units.data_ptr(), U,
+                           _lib.ptr(sink), scale, win, out.data_ptr(), soh, sor, som, H, G, D, V, page, splits,
+                           _lib.ptr(part), out_scale, cap, _lib.ptr(r1), _lib.ptr(r2), _lib.ptr(gate), ldg, gpc,
+                           _lib.ptr(blk), every, keep, maps, _st(q)), "attn_f32")
+
+
 def _tiled_units(unit_rows, rows_per_wave: int) -> int:
     """1 when units were cut for the kernel whose wavefronts share key tiles, 0 for one wavefront each."""
     if unit_rows is None or unit_rows == rows_per_wave:
@@ -960,7 +994,8 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
     part outside the latent (a rotated part shared by the heads) appends it to the cached row and
     the matching query part to qa; the columns of out beyond the latent are then not used.
     units: ``make_units(entries, latent_rows_per_wave(H))`` on the device; with
-    it, bf16 inputs run on the matrix cores (``latent_mfma_ok``).  max_keys: an upper bound of
+    it, bf16 inputs run on the matrix cores (``latent_mfma_ok``) and float32 ones on the fp32
+    matrix instruction (``attn_f32_ok``).  max_keys: an upper bound of
     the keys any row sees (host side; lets a step of few rows split its windows).  unit_rows: the rows
     that the units were cut to where they are others, four times as many (``attn_unit_rows``; latents of
     more than 32 numbers): groups of rows that share key tiles."""
@@ -1010,6 +1045,13 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
                                            out.stride(0), out.stride(1), H, rank, page, splits,
                                            _lib.ptr(part), tile, _st(qa)),
              "latent_attn_mfma")
+        return out
+    if units is not None and attn_f32_ok(qa, cache, rank, rank) and \
+            not _tiled_units(unit_rows, latent_rows_per_wave(H)):
+        assert units.dtype == torch.int32 and units.is_contiguous() and units.shape[1] == 2
+        _attn_f32(qa, qa.stride(0), qa.stride(1), 0, cache, 0, block_tables, row_ent, pos, units, sink, scale, win, out,
+                  out.stride(0), out.stride(1), 0, H, 1, rank, rank, page,
+                  None if max_keys is None else min(max_keys, win))
         return out
     if not latent_attn_ok(H, rank):
         raise ValueError("latent_attn: %d heads x latent %d exceed the kernel's tile" % (H, rank))
@@ -1470,7 +1512,8 @@ def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: in
     same values; head h leaves as o = a_1 - lam a_2, divided by sqrt(mean(o^2) + eps) over its V
     channels, times out_scale (no sink, gate or blk).
     units: ``make_units(entries, window_rows_per_wave(H // G))`` on the device; with it bf16
-    inputs run on the matrix cores (``window_mfma_ok``).  unit_rows: the rows that the units were
+    inputs run on the matrix cores (``window_mfma_ok``), float32 ones on the fp32 matrix instruction
+    (``attn_f32_ok``).  unit_rows: the rows that the units were
     cut to where they are others, four times as many (``attn_unit_rows``): groups of rows that
     share key tiles."""
     R = q.shape[0]
@@ -1566,13 +1609,22 @@ def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: in
                                            tile, _st(q)), "window_attn_mfma")
         return out
     dst = out if M == 1 else torch.empty(R, H * 2 * V, device=q.device, dtype=torch.float32)
-    _chk(lib().p2p_sm_window_attn(q.data_ptr(), q.stride(0), pool.data_ptr(),
-                                  block_tables.data_ptr(), block_tables.shape[1],
-                                  row_ent.data_ptr(), pos.data_ptr(), _lib.ptr(sink), scale, win,
-                                  dst.data_ptr(), dst.stride(0), R, H, G, D, V, page,
-                                  out_scale if M == 1 else 1.0,
-                                  softcap, _lib.ptr(r1), _lib.ptr(r2), _lib.ptr(gate), ldg, gpc,
-                                  _lib.ptr(blk), every, keep, M, _f32(q), _st(q)), "window_attn")
+    if units is not None and attn_f32_ok(q, pool, D, V) and not _tiled_units(unit_rows, window_rows_per_wave(HG)):
+        assert units.dtype == torch.int32 and units.is_contiguous() and units.shape[1] == 2
+        most = None
+        if max_keys is not None:
+            most = min(max_keys, win + keep) + (max(0, max_keys - win) // every if blk is not None else 0)
+        _attn_f32(q, M * D, q.stride(0), D, pool, G * M * D, block_tables, row_ent, pos, units, sink, scale, win, dst,
+                  M * V, dst.stride(0), V, H, G, D, V, page, most, out_scale if M == 1 else 1.0, softcap, r1, r2, gate,
+                  ldg, gpc, blk, every, keep, M)
+    else:
+        _chk(lib().p2p_sm_window_attn(q.data_ptr(), q.stride(0), pool.data_ptr(),
+                                      block_tables.data_ptr(), block_tables.shape[1],
+                                      row_ent.data_ptr(), pos.data_ptr(), _lib.ptr(sink), scale, win,
+                                      dst.data_ptr(), dst.stride(0), R, H, G, D, V, page,
+                                      out_scale if M == 1 else 1.0,
+                                      softcap, _lib.ptr(r1), _lib.ptr(r2), _lib.ptr(gate), ldg, gpc,
+                                      _lib.ptr(blk), every, keep, M, _f32(q), _st(q)), "window_attn")
     if M == 2:
         _chk(lib().p2p_sm_diff_combine(dst.data_ptr(), dst.stride(0), out.data_ptr(), out.stride(0), R, H, V,
                                        diff[0], diff[1], out_scale, _f32(out), _st(q)), "diff_combine")

@@ -1,5 +1,5 @@
 """The attention kernels whose wavefronts share key tiles in LDS against the PyTorch rendering of the
-same ops: row groups that are full, ragged and of one row, portions that begin inside a sequence,
+same ops, and the fp32 kernels of the same inputs: row groups that are full, ragged and of one row, portions that begin inside a sequence,
 tiles cut by the window's ends, key lists of blocks and of kept tokens, windows cut into runs."""
 import pytest
 import torch
@@ -27,6 +27,11 @@ def _step(name, seed):
 
 
 def _close(got, want):
+    if want.dtype == torch.float32:
+        # scores of size up to about 8 from sums of up to 512 products, off by a few 1e-6; weights of fp32
+        # exponentials and a weighted mean of values of about one carry that on
+        torch.testing.assert_close(got.cpu(), want, rtol=2e-5, atol=2e-5)
+        return
     # probabilities and results are rounded to bf16 (2^-9 each) beside values of about one: a weighted
     # mean of values up to 4.5 in size is off by at most 2 * 2^-9 * 4.5 = 1.8e-2
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1e-2, atol=1.8e-2)
@@ -36,37 +41,39 @@ def _close(got, want):
 @pytest.mark.parametrize("H,G,D,V", [(8, 2, 128, 128), (3, 1, 24, 40), (4, 4, 16, 8), (34, 2, 8, 16),
                                      (4, 2, 136, 200), (16, 1, 64, 256)])
 @pytest.mark.parametrize("form", ["window", "sink", "biased", "blocks", "kept", "maps"])
-def test_window_attention_tiles(step, H, G, D, V, form):
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_window_attention_tiles(step, H, G, D, V, form, dt):
     ent, row_ent, pos, bt, R, g = _step(step, 3)
     M = 2 if form == "maps" else 1
     win = {"window": 1 << 30, "biased": 1 << 30, "sink": 33, "blocks": 50, "kept": 21, "maps": 40}[form]
-    q = torch.randn(R, H * M * D, generator=g).bfloat16()
-    pool = torch.randn((int(bt.max()) + 1) * PAGE, G * (M * D + V), generator=g).bfloat16()
+    q = torch.randn(R, H * M * D, generator=g).to(dt)
+    pool = torch.randn((int(bt.max()) + 1) * PAGE, G * (M * D + V), generator=g).to(dt)
     sink, kw, dev = None, dict(out_scale=0.7), {}
     if form == "sink":
         sink = torch.randn(H, generator=g)
     if form == "biased":
         sink = torch.zeros(H)
         dev.update(dist=(torch.rand(H, generator=g) * 2, torch.rand(H, generator=g) * 0.3),
-                   gate=torch.randn(R, H + 3, generator=g).bfloat16())
+                   gate=torch.randn(R, H + 3, generator=g).to(dt))
         kw.update(softcap=9.0)
     if form == "blocks":
         dev.update(blk=torch.randn((int(bt.max()) + 1) * sm.blocks_per_page(PAGE, 12), G * (D + V),
-                                   generator=g).bfloat16(), gate=torch.randn(R, H * V, generator=g).bfloat16())
+                                   generator=g).to(dt), gate=torch.randn(R, H * V, generator=g).to(dt))
         kw.update(every=12, gate_channels=True)
     if form in ("kept", "maps"):
         kw.update(keep=9)
     if form == "maps":
         kw.update(diff=(0.4, 1e-4))
     scale = 1.3 / D ** 0.5
-    want = sm.window_attn(q, pool, bt, row_ent, pos, sink, scale, win, torch.empty(R, H * V).bfloat16(), PAGE, H, G,
+    want = sm.window_attn(q, pool, bt, row_ent, pos, sink, scale, win, torch.empty(R, H * V).to(dt), PAGE, H, G,
                           D, V, **kw, **dev)
     to = lambda t: tuple(x.to(DEV) for x in t) if isinstance(t, tuple) else t.to(DEV) if t is not None else None
-    rows = 4 * sm.window_rows_per_wave(H // G)
+    # four wavefronts' rows for bf16, one's for fp32
+    rows = (4 if dt == torch.bfloat16 else 1) * sm.window_rows_per_wave(H // G)
     units = sm.make_units(ent, rows).to(DEV)
     dev = {k: to(v) for k, v in dev.items()}
     for max_keys in (None, 700):    # whole key lists / cut into runs
-        out = torch.full((R, H * V + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        out = torch.full((R, H * V + 8), 7.0, dtype=dt, device=DEV)
         sm.window_attn(to(q), to(pool), to(bt), to(row_ent), to(pos), to(sink), scale, win, out[:, :H * V], PAGE, H, G,
                        D, V, units=units, unit_rows=rows, max_keys=max_keys, **kw, **dev)
         _close(out[:, :H * V], want)
@@ -89,18 +96,19 @@ def test_group_size():
 @pytest.mark.parametrize("step", sorted(STEPS))
 @pytest.mark.parametrize("H,rank", [(16, 512), (3, 64), (1, 72), (34, 40), (8, 256), (5, 328), (16, 128)])
 @pytest.mark.parametrize("win,sunk", [(1 << 30, False), (37, True), (64, False)])
-def test_latent_attention_tiles(step, H, rank, win, sunk):
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_latent_attention_tiles(step, H, rank, win, sunk, dt):
     ent, row_ent, pos, bt, R, g = _step(step, 7)
-    qa = torch.randn(H, R, rank + 8, generator=g).bfloat16()[:, :, :rank]
-    cache = torch.randn((int(bt.max()) + 1) * PAGE, rank, generator=g).bfloat16()
+    qa = torch.randn(H, R, rank + 8, generator=g).to(dt)[:, :, :rank]
+    cache = torch.randn((int(bt.max()) + 1) * PAGE, rank, generator=g).to(dt)
     sink = torch.randn(H, generator=g) if sunk else None
     scale = 1.3 / rank ** 0.5
-    want = sm.latent_attn(qa, cache, bt, row_ent, pos, sink, scale, win, torch.empty(H, R, rank).bfloat16(), PAGE)
-    rows = 4 * sm.latent_rows_per_wave(H)
+    want = sm.latent_attn(qa, cache, bt, row_ent, pos, sink, scale, win, torch.empty(H, R, rank).to(dt), PAGE)
+    rows = (4 if dt == torch.bfloat16 else 1) * sm.latent_rows_per_wave(H)
     units = sm.make_units(ent, rows).to(DEV)
     for max_keys in (None, 700):    # whole windows / cut into runs
-        out = torch.full((H, R, rank), 7.0, dtype=torch.bfloat16, device=DEV)
-        q2 = torch.empty(H, R, rank + 8, dtype=torch.bfloat16, device=DEV)[:, :, :rank].copy_(qa)
+        out = torch.full((H, R, rank), 7.0, dtype=dt, device=DEV)
+        q2 = torch.empty(H, R, rank + 8, dtype=dt, device=DEV)[:, :, :rank].copy_(qa)
         sm.latent_attn(q2, *(t.to(DEV) for t in (cache, bt, row_ent, pos)), sink.to(DEV) if sunk else None, scale, win,
                        out, PAGE, units=units, unit_rows=rows, max_keys=max_keys)
         _close(out, want)
