@@ -11,15 +11,12 @@
 // r * top + k; every expert gets the list of its slots (cnt / rows).
 //
 // expert_gemm: for expert e and each of its slots s: out[s] = x[s / x_div] . W_e^T.  Rows are
-// gathered through the slot lists, so only experts with rows read their weights.  bf16 runs
-// on the matrix cores (a 16 x 64 tile with K split over the wavefronts for decode-sized steps,
-// an LDS-staged 128 x 128 tile for prompts); fp32 and odd shapes run a tiled FMA kernel.  A
+// gathered through the slot lists, so only experts with rows read their weights.  Rows of a multiple of 16
+// bytes run on the matrix cores (a 16 x 64 tile with K split over the wavefronts for decode-sized steps,
+// LDS-staged 128 x 128 or 64 x 64 tiles for prompts); odd shapes run a tiled FMA kernel.  A
 // slot's result does not depend on which other slots share its tile.
-#include "common.h"
+#include "attn_tile.h"
 using namespace sm;
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // best (value, index) over the wavefront; ties go to the lower index
 __device__ __forceinline__ void wave_argmax(float& v, int& i) {
@@ -40,60 +37,13 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// score: 0 sigmoid, 1 softmax over all experts, 2 the logits themselves for the choice and the
-// softmax over the chosen logits as weights.  bias (optional, [E]): added to the logits.
-// corr (optional, [E]): added to the scores for the choice only.  gscore: a group is ranked by 0 the sum of its two best choice scores, 1 its
-// best choice score.
-template <typename T>
-__global__ void __launch_bounds__(256)
-group_route_k(const T* __restrict__ h, int ldh, const float* __restrict__ wr, int W, int E, int top,
-              int groups, int keep, int score, const float* __restrict__ corr, int gscore,
-              int* __restrict__ ids, float* __restrict__ wts, int* __restrict__ cnt,
-              int* __restrict__ rows, int ldr, const float* __restrict__ bias, int renorm,
-              float wscale) {
-  extern __shared__ float smem[];
-  float* sh = smem;          // [W] the row in fp32
-  float* ss = sh + W;        // [E] scores (the weights of the chosen)
-  float* sc = ss + E;        // [E] choice scores; -inf marks "cannot be chosen (any more)"
-  float* sgs = sc + E;       // [groups] group scores
-  float* stop = sgs + groups;   // [top] the chosen logits (score 2) or scores (renorm)
-  const int r = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int i = threadIdx.x; i < W; i += blockDim.x) sh[i] = ldf(h, (size_t)r * ldh + i);
-  __syncthreads();
-  // four experts at a time per wavefront: their weight loads are independent and go out together
-  for (int e0 = wave * 4; e0 < E; e0 += nw * 4) {
-    const float* w0 = wr + (size_t)e0 * W;
-    const float* w1 = wr + (size_t)min(e0 + 1, E - 1) * W;
-    const float* w2 = wr + (size_t)min(e0 + 2, E - 1) * W;
-    const float* w3 = wr + (size_t)min(e0 + 3, E - 1) * W;
-    float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f, d3 = 0.0f;
-#pragma unroll 4
-    for (int i = lane; i < W; i += 64) {
-      float x = sh[i];
-      d0 += x * w0[i];
-      d1 += x * w1[i];
-      d2 += x * w2[i];
-      d3 += x * w3[i];
-    }
-    d0 = wave_sum(d0);
-    d1 = wave_sum(d1);
-    d2 = wave_sum(d2);
-    d3 = wave_sum(d3);
-    if (lane == 0) {
-      if (bias) {
-        d0 += bias[e0];
-        d1 += bias[min(e0 + 1, E - 1)];
-        d2 += bias[min(e0 + 2, E - 1)];
-        d3 += bias[min(e0 + 3, E - 1)];
-      }
-      ss[e0] = score ? d0 : sigmoidf_(d0);
-      if (e0 + 1 < E) ss[e0 + 1] = score ? d1 : sigmoidf_(d1);
-      if (e0 + 2 < E) ss[e0 + 2] = score ? d2 : sigmoidf_(d2);
-      if (e0 + 3 < E) ss[e0 + 3] = score ? d3 : sigmoidf_(d3);
-    }
-  }
-  __syncthreads();
-  if (wave != 0) return;
+// The choice of one row by one wavefront: ss holds its E logits (sigmoids for score 0) and becomes its scores.
+// place(k, e): the row's k-th expert is e (called by lane 0).
+template <typename P>
+__device__ __forceinline__ void choose_experts(int r, int lane, float* ss, float* sc, float* sgs, float* stop, int E,
+                                               int top, int groups, int keep, int score,
+                                               const float* __restrict__ corr, int gscore, int* __restrict__ ids,
+                                               float* __restrict__ wts, int renorm, float wscale, P place) {
   if (score == 1) {   // softmax over all experts
     float mx = -INFINITY;
     for (int e = lane; e < E; e += 64) mx = fmaxf(mx, ss[e]);
@@ -152,8 +102,7 @@ group_route_k(const T* __restrict__ h, int ldh, const float* __restrict__ wr, in
       ids[slot] = bi;
       if (score == 2 || renorm) stop[k] = ss[bi];
       else wts[slot] = ss[bi] * wscale;
-      int at = atomicAdd(&cnt[bi], 1);
-      rows[(size_t)bi * ldr + at] = slot;
+      place(k, bi);
     }
     wave_sync();
   }
@@ -171,6 +120,129 @@ group_route_k(const T* __restrict__ h, int ldh, const float* __restrict__ wr, in
     for (int k = lane; k < top; k += 64) sum += stop[k];
     sum = wave_sum(sum) + 1e-20f;
     for (int k = lane; k < top; k += 64) wts[r * top + k] = stop[k] / sum * wscale;
+  }
+}
+
+// score: 0 sigmoid, 1 softmax over all experts, 2 the logits themselves for the choice and the
+// softmax over the chosen logits as weights.  bias (optional, [E]): added to the logits.
+// corr (optional, [E]): added to the scores for the choice only.  gscore: a group is ranked by 0 the sum of its two best choice scores, 1 its
+// best choice score.
+template <typename T>
+__global__ void __launch_bounds__(256)
+group_route_k(const T* __restrict__ h, int ldh, const float* __restrict__ wr, int W, int E, int top,
+              int groups, int keep, int score, const float* __restrict__ corr, int gscore,
+              int* __restrict__ ids, float* __restrict__ wts, int* __restrict__ cnt,
+              int* __restrict__ rows, int ldr, const float* __restrict__ bias, int renorm,
+              float wscale) {
+  extern __shared__ float smem[];
+  float* sh = smem;          // [W] the row in fp32
+  float* ss = sh + W;        // [E] scores (the weights of the chosen)
+  float* sc = ss + E;        // [E] choice scores; -inf marks "cannot be chosen (any more)"
+  float* sgs = sc + E;       // [groups] group scores
+  float* stop = sgs + groups;   // [top] the chosen logits (score 2) or scores (renorm)
+  const int r = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  for (int i = threadIdx.x; i < W; i += blockDim.x) sh[i] = ldf(h, (size_t)r * ldh + i);
+  __syncthreads();
+  // four experts at a time per wavefront: their weight loads are independent and go out together
+  for (int e0 = wave * 4; e0 < E; e0 += nw * 4) {
+    const float* w0 = wr + (size_t)e0 * W;
+    const float* w1 = wr + (size_t)min(e0 + 1, E - 1) * W;
+    const float* w2 = wr + (size_t)min(e0 + 2, E - 1) * W;
+    const float* w3 = wr + (size_t)min(e0 + 3, E - 1) * W;
+    float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f, d3 = 0.0f;
+#pragma unroll 4
+    for (int i = lane; i < W; i += 64) {
+      float x = sh[i];
+      d0 += x * w0[i];
+      d1 += x * w1[i];
+      d2 += x * w2[i];
+      d3 += x * w3[i];
+    }
+    d0 = wave_sum(d0);
+    d1 = wave_sum(d1);
+    d2 = wave_sum(d2);
+    d3 = wave_sum(d3);
+    if (lane == 0) {
+      if (bias) {
+        d0 += bias[e0];
+        d1 += bias[min(e0 + 1, E - 1)];
+        d2 += bias[min(e0 + 2, E - 1)];
+        d3 += bias[min(e0 + 3, E - 1)];
+      }
+      ss[e0] = score ? d0 : sigmoidf_(d0);
+      if (e0 + 1 < E) ss[e0 + 1] = score ? d1 : sigmoidf_(d1);
+      if (e0 + 2 < E) ss[e0 + 2] = score ? d2 : sigmoidf_(d2);
+      if (e0 + 3 < E) ss[e0 + 3] = score ? d3 : sigmoidf_(d3);
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  choose_experts(r, lane, ss, sc, sgs, stop, E, top, groups, keep, score, corr, gscore, ids, wts, renorm, wscale,
+                 [&](int k, int e) { rows[(size_t)e * ldr + atomicAdd(&cnt[e], 1)] = r * top + k; });
+}
+
+// The same for prompts: a workgroup takes 16 rows, a wavefront each, and the experts' slot counts go up by one
+// atomic per workgroup and expert instead of one per slot (4096 of them on eight addresses took most of the
+// 57 us that 2048 rows of 2048 numbers needed; 20 us now, 606 rows of 1024 14 instead of 21).  Two or four rows
+// per wavefront, with the weights read once for them, measured 22 and 31 us: the chain of one row's sums
+// and choices is what is left.  A logit's sum has the order it has above.
+template <typename T>
+__global__ void __launch_bounds__(1024)
+group_route_rows_k(const T* __restrict__ h, int ldh, const float* __restrict__ wr, int R, int W, int E, int top,
+                   int groups, int keep, int score, const float* __restrict__ corr, int gscore, int* __restrict__ ids,
+                   float* __restrict__ wts, int* __restrict__ cnt, int* __restrict__ rows, int ldr,
+                   const float* __restrict__ bias, int renorm, float wscale) {
+  extern __shared__ float smem[];
+  float* ss = smem;                      // [16][E]
+  float* sc = ss + 16 * E;               // [16][E]
+  float* sgs = sc + 16 * E;              // [16][groups]
+  float* stop = sgs + 16 * groups;       // [16][top]
+  int* scnt = (int*)(stop + 16 * top);   // [E] slots of this workgroup, then the place of its first
+  int* spick = scnt + E;                 // [16][top] expert
+  int* sat = spick + 16 * top;           // [16][top] place among the workgroup's
+  const int lane = threadIdx.x & 63, m = threadIdx.x >> 6, r = blockIdx.x * 16 + m;
+  for (int e = threadIdx.x; e < E; e += 1024) scnt[e] = 0;
+  const T* x = h + (size_t)min(r, R - 1) * ldh;
+  for (int e0 = 0; e0 < E; e0 += 4) {
+    const float* w[4];
+    float d[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      w[u] = wr + (size_t)min(e0 + u, E - 1) * W;
+      d[u] = 0.0f;
+    }
+#pragma unroll 4
+    for (int i = lane; i < W; i += 64) {
+      const float xv = ldf(x, i);
+#pragma unroll
+      for (int u = 0; u < 4; u++) d[u] += xv * w[u][i];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      float v = wave_sum(d[u]);
+      if (lane == 0 && e0 + u < E) {
+        if (bias) v += bias[e0 + u];
+        ss[m * E + e0 + u] = score ? v : sigmoidf_(v);
+      }
+    }
+  }
+  __syncthreads();   // scnt is clear
+  if (r < R)
+    choose_experts(r, lane, ss + m * E, sc + m * E, sgs + m * groups, stop + m * top, E, top, groups, keep, score, corr,
+                   gscore, ids, wts, renorm, wscale, [&](int k, int e) {
+                     spick[m * top + k] = e;
+                     sat[m * top + k] = atomicAdd(&scnt[e], 1);
+                   });
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 1024) {
+    const int n = scnt[e];
+    if (n) scnt[e] = atomicAdd(&cnt[e], n);
+  }
+  __syncthreads();
+  const int slots = min(16, R - (int)blockIdx.x * 16) * top;
+  for (int i = threadIdx.x; i < slots; i += 1024) {
+    const int e = spick[i];
+    rows[(size_t)e * ldr + scnt[e] + sat[i]] = blockIdx.x * 16 * top + i;
   }
 }
 
@@ -251,16 +323,30 @@ __device__ __forceinline__ float plain_epi(float v, int epi) {
   return v;
 }
 
-// bf16 on the matrix cores, few slots per expert (decode-sized steps): a block takes 16 slots x
+// one step of an accumulator: a 16-byte fragment of 16 slots' rows times one of 16 weight rows
+template <typename T>
+__device__ __forceinline__ f32x4 mfma_piece(uint4 a, uint4 b, f32x4 c) {
+  if constexpr (sizeof(T) == 2) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  } else {
+    const f32x4 x = __builtin_bit_cast(f32x4, a), y = __builtin_bit_cast(f32x4, b);
+#pragma unroll
+    for (int i = 0; i < 4; i++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], c, 0, 0, 0);
+    return c;
+  }
+}
+
+// Few slots per expert (decode-sized steps), on the matrix cores: a block takes 16 slots x
 // 64 output columns of one expert and its four wavefronts split K among themselves, so the
 // chain of dependent loads is a quarter as long; each wavefront walks its share in steps of 32
-// with one A fragment (the gathered rows) and four B fragments (16 weight rows each), the next
-// step's fragments in flight while the current products run; the four partial tiles are
-// added through LDS.
+// with one A fragment (the gathered rows) and four B fragments (16 weight rows each), four steps'
+// fragments in flight while the current products run; the four partial tiles are added through LDS.  fp32 takes half the K per step (a fragment is 16 bytes of a row) and four products.
+template <typename T>
 __global__ void __launch_bounds__(256)
-expert_gemm_mfma_k(const bf16* __restrict__ x, int ldx, int x_div, const bf16* __restrict__ w,
+expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restrict__ w,
                    const int* __restrict__ cnt, const int* __restrict__ rows, int ldr,
-                   bf16* __restrict__ out, int ldo, int N, int K, int E, int TMP, int epi, float limit, float alpha) {
+                   T* __restrict__ out, int ldo, int N, int K, int E, int TMP, int epi, float limit, float alpha) {
+  constexpr int EP = 16 / sizeof(T), KS = 4 * EP;   // numbers per fragment, per step
   __shared__ f32x4 red[3][4][64];
   int e, m0, nt;
   if (!find_tile(cnt, E, 16, TMP, e, m0, nt)) return;
@@ -268,41 +354,43 @@ expert_gemm_mfma_k(const bf16* __restrict__ x, int ldx, int x_div, const bf16* _
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, quad = lane >> 4;
   const int mi = m0 + n16;
   const int slot = mi < c ? rows[(size_t)e * ldr + mi] : -1;
-  const int kq = ((K + 127) / 128) * 32;          // K per wavefront, a multiple of 32
+  const int kq = ((K + 4 * KS - 1) / (4 * KS)) * KS;   // K per wavefront, a multiple of the step
   const int kb = wave * kq, ke = min(K, kb + kq);
-  const bf16* xa = slot >= 0 ? x + (size_t)(slot / x_div) * ldx + quad * 8 : nullptr;
-  const bf16* wb[4];
+  // rows that do not exist (a slot or column beyond the last) are others, their products are dropped; past
+  // the wavefront's share of K both operands are zero
+  const T* xa = x + (size_t)(max(slot, 0) / x_div) * ldx + quad * EP;
+  const T* wb[4];
 #pragma unroll
-  for (int t = 0; t < 4; t++) {
-    int n = n0 + t * 16 + n16;
-    wb[t] = n < N ? w + ((size_t)e * N + n) * K + quad * 8 : nullptr;
-  }
+  for (int t = 0; t < 4; t++) wb[t] = w + ((size_t)e * N + min(n0 + t * 16 + n16, N - 1)) * K + quad * EP;
   f32x4 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint4 zero = make_uint4(0, 0, 0, 0);
-  uint4 av, bv[4];
-  {
-    bool kin = kb + quad * 8 < ke;                 // K is a multiple of 8
-    av = (xa && kin) ? *(const uint4*)(xa + kb) : zero;
+  // DEPTH steps in flight
+  constexpr int DEPTH = 4;
+  uint4 av[DEPTH], bv[DEPTH][4];
+  auto load = [&](int k, uint4& a, uint4 (&b)[4]) {
+    const bool in = k + quad * EP < ke;            // K is a multiple of EP
+    const int at = in ? k : 0;
+    a = *(const uint4*)(xa + at);
 #pragma unroll
-    for (int t = 0; t < 4; t++) bv[t] = (wb[t] && kin) ? *(const uint4*)(wb[t] + kb) : zero;
-  }
-  for (int k0 = kb; k0 < ke; k0 += 32) {
-    const int kn = k0 + 32;
-    const bool nin = kn + quad * 8 < ke;
-    uint4 an = (xa && nin) ? *(const uint4*)(xa + kn) : zero;
-    uint4 bn[4];
+    for (int t = 0; t < 4; t++) b[t] = *(const uint4*)(wb[t] + at);
+    if (!in) {
+      a = zero;
 #pragma unroll
-    for (int t = 0; t < 4; t++) bn[t] = (wb[t] && nin) ? *(const uint4*)(wb[t] + kn) : zero;
-    bf16x8 af = __builtin_bit_cast(bf16x8, av);
+      for (int t = 0; t < 4; t++) b[t] = zero;
+    }
+  };
 #pragma unroll
-    for (int t = 0; t < 4; t++)
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, __builtin_bit_cast(bf16x8, bv[t]),
-                                                        acc[t], 0, 0, 0);
-    av = an;
+  for (int d = 0; d < DEPTH; d++) load(kb + d * KS, av[d], bv[d]);
+  for (int k0 = kb; k0 < ke; k0 += DEPTH * KS) {
 #pragma unroll
-    for (int t = 0; t < 4; t++) bv[t] = bn[t];
+    for (int d = 0; d < DEPTH; d++) {
+#pragma unroll
+      for (int t = 0; t < 4; t++) acc[t] = mfma_piece<T>(av[d], bv[d][t], acc[t]);
+      if (k0 + (DEPTH + d) * KS < ke) load(k0 + (DEPTH + d) * KS, av[d], bv[d]);
+      else av[d] = zero;
+    }
   }
   if (wave > 0) {
 #pragma unroll
@@ -324,126 +412,147 @@ expert_gemm_mfma_k(const bf16* __restrict__ x, int ldx, int x_div, const bf16* _
       for (int t = 0; t < 4; t += 2) {
         int n = n0 + t * 16;
         if (n + 16 + n16 < N)
-          out[(size_t)so * ldo + n / 2 + n16] =
-              __float2bfloat16(glu_epi(acc[t][i], acc[t + 1][i], epi, limit, alpha));
+          stf(out, (size_t)so * ldo + n / 2 + n16, glu_epi(acc[t][i], acc[t + 1][i], epi, limit, alpha));
       }
       continue;
     }
 #pragma unroll
     for (int t = 0; t < 4; t++) {
       int n = n0 + t * 16 + n16;
-      if (n < N) out[(size_t)so * ldo + n] = __float2bfloat16(plain_epi(acc[t][i], epi));
+      if (n < N) stf(out, (size_t)so * ldo + n, plain_epi(acc[t][i], epi));
     }
   }
 }
 
-// Many slots per expert (prompts): a block of 2 x 2 wavefronts takes 128 slots x 128 columns
-// and walks K in steps of 64.  The gathered A rows and the weight rows of a step are loaded
-// with coalesced 16-byte reads (8 threads per row), kept in registers while the previous step
-// computes, and handed to the MFMA fragments through LDS (rows 144 bytes apart).  Each
-// wavefront owns 64 x 64 (4 x 4 MFMA tiles); 16-slot tiles beyond the expert's count are skipped.
-#define EB_LD 72   // bf16 per LDS row: 64 + 8
-__global__ void __launch_bounds__(256)
-expert_gemm_mfma_big_k(const bf16* __restrict__ x, int ldx, int x_div, const bf16* __restrict__ w,
-                       const int* __restrict__ cnt, const int* __restrict__ rows, int ldr,
-                       bf16* __restrict__ out, int ldo, int N, int K, int E, int TMP, int epi, float limit, float alpha) {
-  __shared__ __align__(16) unsigned short sA[128 * EB_LD];
-  __shared__ __align__(16) unsigned short sB[128 * EB_LD];
-  __shared__ int sslot[128];
+// Many slots per expert (prompts): a block of 2 x 2 wavefronts takes BM slots x BN columns and walks K in
+// steps of 128 bytes per row (64 bf16, 32 fp32).  The gathered rows and the weight rows of a step are copied
+// straight into LDS (attn_tile.h) while the step before is multiplied; their 16-byte pieces are permuted
+// so that a fragment's 16 rows spread over all banks.  A wavefront owns BM/2 x BN/2; 16-slot tiles
+// beyond the expert's count are skipped.  bf16: one v_mfma_f32_16x16x32_bf16 per pair of 16-byte fragments;
+// fp32: four v_mfma_f32_16x16x4_f32, component by component.
+//
+// Bound by LDS reads and the copies' latency (two or three blocks per CU).  8 experts, 4096 slots, width 2048,
+// gate and up of 1024: 70 us (490 TFLOP/s) and 40 us for the two products against 229 and 117 with register
+// staging, one step at a time; 1212 slots at width 1024: 10.7 and 8.7 us (64 x 64 tiles) against 53 and 29;
+// fp32, 1012 slots, width 1024 and 512: 44 and 24 us against 185 and 94 on vector instructions.
+template <typename T, int BM, int BN>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
+expert_gemm_tile_k(const T* __restrict__ x, int ldx, int x_div, const T* __restrict__ w,
+                   const int* __restrict__ cnt, const int* __restrict__ rows, int ldr, T* __restrict__ out, int ldo,
+                   int N, int K, int E, int TMP, int epi, float limit, float alpha) {
+  constexpr int EP = 16 / sizeof(T), KS = 8 * EP;          // numbers per piece, per step
+  constexpr int FM = BM / 32, FN = BN / 32;                // 16 x 16 tiles of a wavefront
+  constexpr int STAGE = (BM + BN) * 128;
+  extern __shared__ __align__(16) unsigned char tile[];    // [2][BM rows | BN rows] of 128 bytes
+  __shared__ int sslot[BM];
   int e, m0, nt;
-  if (!find_tile(cnt, E, 128, TMP, e, m0, nt)) return;
-  const int c = cnt[e], n0 = nt * 128;
-  const int tid = threadIdx.x;
-  if (tid < 128) sslot[tid] = m0 + tid < c ? rows[(size_t)e * ldr + m0 + tid] : -1;
+  if (!find_tile(cnt, E, BM, TMP, e, m0, nt)) return;
+  const int c = cnt[e], n0 = nt * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), n16 = lane & 15, quad = lane >> 4;
+  if (tid < BM) sslot[tid] = m0 + tid < c ? rows[(size_t)e * ldr + m0 + tid] : -1;
   __syncthreads();
-  const int lane = tid & 63, wave = tid >> 6, n16 = lane & 15, quad = lane >> 4;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  const int nmt = max(0, min(4, (c - (m0 + wm) + 15) / 16));
-  // this thread's four 16-byte pieces of the A and B tiles: row = (tid + 256 u) / 8
-  const int c8 = (tid & 7) * 8;
-  const bf16* pa[4];
-  const bf16* pb[4];
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+  const int nmt = max(0, min(FM, (c - (m0 + wm) + 15) / 16));
+  // thread t copies pieces t, t + 256, ..; rows that do not exist are the tile's first, their products are dropped
+  const int sw = ((tid >> 4) & 7), c8 = ((tid & 7) ^ sw) * EP;   // row r = tid / 8 (+ 32 i) has pieces ^ (r / 2 % 8)
+  const T* pa[BM / 32];
+  const T* pb[BN / 32];
 #pragma unroll
-  for (int u = 0; u < 4; u++) {
-    int r = (tid + 256 * u) >> 3;
-    int sl = sslot[r];
-    pa[u] = sl >= 0 ? x + (size_t)(sl / x_div) * ldx + c8 : nullptr;
-    pb[u] = n0 + r < N ? w + ((size_t)e * N + n0 + r) * K + c8 : nullptr;
+  for (int i = 0; i < BM / 32; i++) {
+    const int sl = sslot[(tid >> 3) + 32 * i];
+    pa[i] = x + (size_t)((sl >= 0 ? sl : sslot[0]) / x_div) * ldx;
   }
-  const uint4 zero = make_uint4(0, 0, 0, 0);
-  uint4 ra[4], rb[4];
 #pragma unroll
-  for (int u = 0; u < 4; u++) {
-    bool kin = c8 < K;
-    ra[u] = (pa[u] && kin) ? *(const uint4*)pa[u] : zero;
-    rb[u] = (pb[u] && kin) ? *(const uint4*)pb[u] : zero;
-  }
-  f32x4 acc[4][4];
+  for (int i = 0; i < BN / 32; i++) pb[i] = w + ((size_t)e * N + min(n0 + (tid >> 3) + 32 * i, N - 1)) * K;
+  const unsigned lds0 = lds_address(tile) + wave * 1024;
+  auto copy_step = [&](int k0, int st) {
+    const int k = k0 + c8 < K ? k0 + c8 : 0;   // past the end: any numbers, struck out below
+    const unsigned dst = lds0 + st * STAGE;
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+    for (int i = 0; i < BM / 32; i++) copy_lds16(pa[i] + k, dst + i * 4096);
 #pragma unroll
-    for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += 64) {
+    for (int i = 0; i < BN / 32; i++) copy_lds16(pb[i] + k, dst + BM * 128 + i * 4096);
+  };
+  f32x4 acc[FM][FN];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      int r = (tid + 256 * u) >> 3;
-      *(uint4*)(sA + r * EB_LD + c8) = ra[u];
-      *(uint4*)(sB + r * EB_LD + c8) = rb[u];
-    }
-    __syncthreads();
-    const int kn = k0 + 64;
-    if (kn < K) {
-      bool kin = kn + c8 < K;
+  for (int a = 0; a < FM; a++)
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        ra[u] = (pa[u] && kin) ? *(const uint4*)(pa[u] + kn) : zero;
-        rb[u] = (pb[u] && kin) ? *(const uint4*)(pb[u] + kn) : zero;
-      }
-    }
+    for (int b = 0; b < FN; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  copy_step(0, 0);
+  int st = 0;
+  for (int k0 = 0; k0 < K; k0 += KS, st ^= 1) {
+    tile_wait();
+    __syncthreads();   // the step has landed, the other stage is free
+    if (k0 + KS < K) copy_step(k0 + KS, st ^ 1);
+    const unsigned char* sA = tile + st * STAGE + (wm + n16) * 128;
+    const unsigned char* sB = tile + st * STAGE + BM * 128 + (wn + n16) * 128;
+    uint4 af[2][FM], bf[2][FN];
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
-      bf16x8 bfr[4];
+      const int at = ((kk * 4 + quad) ^ ((n16 >> 1) & 7)) * 16;
 #pragma unroll
-      for (int b = 0; b < 4; b++)
-        bfr[b] = __builtin_bit_cast(bf16x8, *(const uint4*)(sB + (wn + b * 16 + n16) * EB_LD +
-                                                             kk * 32 + quad * 8));
+      for (int b = 0; b < FN; b++) bf[kk][b] = *(const uint4*)(sB + b * 2048 + at);
 #pragma unroll
-      for (int a = 0; a < 4; a++) {
-        if (a < nmt) {
-          bf16x8 av = __builtin_bit_cast(bf16x8, *(const uint4*)(sA + (wm + a * 16 + n16) * EB_LD +
-                                                                  kk * 32 + quad * 8));
-#pragma unroll
-          for (int b = 0; b < 4; b++)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bfr[b], acc[a][b], 0, 0, 0);
-        }
-      }
+      for (int a = 0; a < FM; a++) af[kk][a] = *(const uint4*)(sA + a * 2048 + at);
     }
-    __syncthreads();
+    if (k0 + KS > K) {   // the last step of a K that is no multiple: zeros past its end
+#pragma unroll
+      for (int kk = 0; kk < 2; kk++)
+        if (k0 + (kk * 4 + quad) * EP >= K) {
+#pragma unroll
+          for (int a = 0; a < FM; a++) af[kk][a] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+          for (int b = 0; b < FN; b++) bf[kk][b] = make_uint4(0, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+      for (int a = 0; a < FM; a++)
+        if (a < nmt) {
+#pragma unroll
+          for (int b = 0; b < FN; b++) acc[a][b] = mfma_piece<T>(af[kk][a], bf[kk][b], acc[a][b]);
+        }
   }
 #pragma unroll
-  for (int a = 0; a < 4; a++) {
+  for (int a = 0; a < FM; a++) {
     if (a >= nmt) continue;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      int so = sslot[wm + a * 16 + quad * 4 + i];
+      const int so = sslot[wm + a * 16 + quad * 4 + i];
       if (so < 0) continue;
       if (epi == 1 || epi == 3) {
 #pragma unroll
-        for (int b = 0; b < 4; b += 2) {
-          int n = n0 + wn + b * 16;
+        for (int b = 0; b < FN; b += 2) {
+          const int n = n0 + wn + b * 16;
           if (n + 16 + n16 < N)
-            out[(size_t)so * ldo + n / 2 + n16] =
-                __float2bfloat16(glu_epi(acc[a][b][i], acc[a][b + 1][i], epi, limit, alpha));
+            stf(out, (size_t)so * ldo + n / 2 + n16, glu_epi(acc[a][b][i], acc[a][b + 1][i], epi, limit, alpha));
         }
         continue;
       }
 #pragma unroll
-      for (int b = 0; b < 4; b++) {
-        int n = n0 + wn + b * 16 + n16;
-        if (n < N) out[(size_t)so * ldo + n] = __float2bfloat16(plain_epi(acc[a][b][i], epi));
+      for (int b = 0; b < FN; b++) {
+        const int n = n0 + wn + b * 16 + n16;
+        if (n < N) stf(out, (size_t)so * ldo + n, plain_epi(acc[a][b][i], epi));
       }
     }
   }
+}
+
+template <typename T, int BM, int BN>
+static int launch_expert_tile(const void* x, int ldx, int x_div, const void* w, const int* cnt, const int* rows, int ldr,
+                              void* out, int ldo, int E, int N, int K, int slots, int epi, float limit, float alpha,
+                              hipStream_t st) {
+  const int tmp = (((slots + BM - 1) / BM + E) + 7) & ~7;
+  const size_t shm = (size_t)2 * (BM + BN) * 128;
+  if (shm > 48 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)expert_gemm_tile_k<T, BM, BN>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+    if (e != hipSuccess) return (int)e;
+  }
+  hipLaunchKernelGGL((expert_gemm_tile_k<T, BM, BN>), dim3(tmp * ((N + BN - 1) / BN)), dim3(256), shm, st, (const T*)x,
+                     ldx, x_div, (const T*)w, cnt, rows, ldr, (T*)out, ldo, N, K, E, tmp, epi, limit, alpha);
+  return (int)hipGetLastError();
 }
 
 // any type, any shape: 32 slots x 64 columns per block, K staged through LDS 32 at a time
@@ -545,6 +654,14 @@ int p2p_sm_group_route(const void* h, int ldh, const float* wr, int R, int W, in
     return (int)hipErrorInvalidValue;
   size_t shm = (size_t)(W + 2 * E + groups + top) * 4;
   if (shm > 64 * 1024) return (int)hipErrorInvalidValue;
+  const size_t many = (size_t)(16 * (2 * E + groups + 3 * top) + E) * 4;
+  // one row per workgroup takes 13 us up to 100 rows and 18 at 500; sixteen per workgroup 14 at 600
+  if (R >= 256 && many <= 48 * 1024) {
+    SM_DISPATCH_T(f32, hipLaunchKernelGGL(group_route_rows_k<T>, dim3((R + 15) / 16), dim3(1024), many, st,
+                                           (const T*)h, ldh, wr, R, W, E, top, groups, keep, score, corr,
+                                           gscore, ids, wts, cnt, rows, ldr, bias, renorm, wscale));
+    return (int)hipGetLastError();
+  }
   SM_DISPATCH_T(f32, hipLaunchKernelGGL(group_route_k<T>, dim3(R), dim3(256), shm, st,
                                          (const T*)h, ldh, wr, W, E, top, groups, keep, score, corr,
                                          gscore, ids, wts, cnt, rows, ldr, bias, renorm, wscale));
@@ -561,18 +678,24 @@ int p2p_sm_expert_gemm(const void* x, int ldx, int x_div, const void* w, const i
   if (total_slots <= 0 || E <= 0) return 0;
   if (x_div < 1 || N < 1 || K < 1 || ((epi == 1 || epi == 3) && N % 32))
     return (int)hipErrorInvalidValue;
-  if (!f32 && K % 8 == 0 && ldx % 8 == 0 && ((size_t)x & 15) == 0 && ((size_t)w & 15) == 0) {
-    if (total_slots >= 64 * E) {   // prompts: the large tile
-      int tmp = (((total_slots + 127) / 128 + E) + 7) & ~7;
-      dim3 grid(tmp * ((N + 127) / 128));
-      hipLaunchKernelGGL(expert_gemm_mfma_big_k, grid, dim3(256), 0, st, (const bf16*)x, ldx, x_div,
-                         (const bf16*)w, cnt, rows, ldr, (bf16*)out, ldo, N, K, E, tmp, epi, limit, alpha);
-      return (int)hipGetLastError();
+  const int ep = f32 ? 4 : 8;   // numbers per 16 bytes
+  if (K % ep == 0 && ldx % ep == 0 && ((size_t)x & 15) == 0 && ((size_t)w & 15) == 0) {
+    if (total_slots >= 64 * E) {   // prompts: tiles
+      // the larger tile needs fewer reads per product, the smaller one gives every CU a block: 160 large
+      // tiles 35 us against 27 (width 2048, 1212 slots), 432 large ones 37.6 against 43 (2400 slots)
+      const long big = (long)((total_slots + 127) / 128 + E) * ((N + 127) / 128);
+#define ET(T, BM, BN)                                                                                        \
+  return launch_expert_tile<T, BM, BN>(x, ldx, x_div, w, cnt, rows, ldr, out, ldo, E, N, K, total_slots, epi, \
+                                       limit, alpha, st)
+      if (f32) ET(float, 64, 64);
+      if (big >= 384) ET(bf16, 128, 128);
+      ET(bf16, 64, 64);
+#undef ET
     }
     int tmp = (((total_slots + 15) / 16 + E) + 7) & ~7;
     dim3 grid(tmp * ((N + 63) / 64));
-    hipLaunchKernelGGL(expert_gemm_mfma_k, grid, dim3(256), 0, st, (const bf16*)x, ldx, x_div,
-                       (const bf16*)w, cnt, rows, ldr, (bf16*)out, ldo, N, K, E, tmp, epi, limit, alpha);
+    SM_DISPATCH_T(f32, hipLaunchKernelGGL(expert_gemm_mfma_k<T>, grid, dim3(256), 0, st, (const T*)x, ldx, x_div,
+                                           (const T*)w, cnt, rows, ldr, (T*)out, ldo, N, K, E, tmp, epi, limit, alpha));
     return (int)hipGetLastError();
   }
   int tmp = (((total_slots + 31) / 32 + E) + 7) & ~7;

@@ -1,0 +1,70 @@
+"""Routing of many rows and the tiled expert products against the PyTorch rendering of the same ops:
+experts without slots and with one, counts off the tiles' grid, row lengths that end inside a step,
+columns that end inside a tile, both tile sizes, the activations."""
+import pytest
+import torch
+
+from p2p_llm_chat_go_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("R,W,E,top,groups,keep,kw", [
+    (256, 72, 8, 2, 1, 1, dict(score="top_softmax", bias=True)),
+    (301, 200, 12, 3, 4, 2, dict()),
+    (1000, 64, 70, 5, 7, 3, dict(score="softmax", group_score="max", renorm=True, scale=1.5)),
+    (259, 40, 3, 1, 1, 1, dict(score="softmax", corr=True))])
+def test_routing_of_many_rows(dt, R, W, E, top, groups, keep, kw):
+    g = torch.Generator().manual_seed(2)
+    h, wr = torch.randn(R, W, generator=g).to(dt), torch.randn(E, W, generator=g) / W ** 0.5
+    extra = {k: torch.randn(E, generator=g) * 0.3 for k in ("bias", "corr") if kw.get(k)}
+    kw = dict(kw, **extra)
+    res = []
+    for dev in ("cpu", DEV):
+        ids, wts = torch.empty(R, top, dtype=torch.int32, device=dev), torch.empty(R, top, device=dev)
+        cnt, rows = torch.empty(E, dtype=torch.int32, device=dev), torch.full((E, R * top), -1, dtype=torch.int32, device=dev)
+        k2 = {k: v.to(dev) if isinstance(v, torch.Tensor) else v for k, v in kw.items()}
+        sm.group_route(h.to(dev), wr.to(dev), top, groups, keep, ids, wts, cnt, rows, **k2)
+        res.append([t.cpu() for t in (ids, wts, cnt, rows)])
+    (i1, w1, _c1, _r1), (i2, w2, c2, r2) = res
+    # two scores that differ by less than fp32 sums may come in either order
+    assert (i1 != i2).float().mean() < 0.005
+    same = (i1 == i2).all(1)
+    torch.testing.assert_close(w2[same], w1[same], rtol=1e-5, atol=1e-6)
+    # every slot is in its expert's list, once
+    for e in range(E):
+        assert sorted(r2[e, :int(c2[e])].tolist()) == (i2.reshape(-1) == e).nonzero()[:, 0].tolist()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts,N,K", [
+    ([0, 1, 130, 400, 17], 100, 40),        # 64 x 64 tiles; K ends inside a step of either type
+    ([700, 129, 300], 5152, 72),            # 128 x 128 tiles (bf16)
+    ([3, 0, 1], 160, 200)])                 # few slots
+@pytest.mark.parametrize("act", [None, "silu_glu", "relu2", "limit"])
+def test_expert_products(dt, counts, N, K, act):
+    if act in ("silu_glu", "limit"):
+        N = N // 32 * 32
+    g = torch.Generator().manual_seed(4)
+    E, S = len(counts), sum(counts)
+    order = torch.randperm(S, generator=g).to(torch.int32)
+    rows, at = torch.zeros(E, S, dtype=torch.int32), 0
+    for e, n in enumerate(counts):
+        rows[e, :n] = order[at:at + n]
+        at += n
+    cnt = torch.tensor(counts, dtype=torch.int32)
+    x = torch.randn((S + 1) // 2, K + 8, generator=g).to(dt)[:, :K]       # two slots per row, strided
+    w = (torch.randn(E, N, K, generator=g) / K ** 0.5).to(dt)
+    kw = {"silu_glu": dict(silu_glu=True), "relu2": dict(relu2=True), "limit": dict(act_limit=0.9), None: {}}[act]
+    F = N // 2 if act in ("silu_glu", "limit") else N
+    want = sm.expert_gemm(x, 2, w, cnt, rows, torch.zeros(S, F, dtype=dt), S, **kw)
+    x2 = torch.empty((S + 1) // 2, K + 8, dtype=dt, device=DEV)[:, :K].copy_(x)
+    out = torch.full((S, F + 8), 7.0, dtype=dt, device=DEV)
+    sm.expert_gemm(x2, 2, w.to(DEV), cnt.to(DEV), rows.to(DEV), out[:, :F], S, **kw)
+    # sums of K products of about 1 / sqrt(K): fp32 rounding in either order, one rounding to bf16 (of values
+    # up to about 5, squared under relu2: up to 25)
+    tol = dict(rtol=1e-2, atol=2e-2) if dt == torch.bfloat16 else dict(rtol=2e-5, atol=1e-5)
+    torch.testing.assert_close(out[:, :F].cpu().float(), want.float(), **tol)
+    assert bool((out[:, F:] == 7.0).all())
