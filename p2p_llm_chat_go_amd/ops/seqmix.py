@@ -52,7 +52,7 @@ _SIGS = {
                                                     c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                                     c_void_p, c_int, c_void_p, c_int, c_int, c_int,
                                                     c_float, c_int, c_void_p],
-    "p2p_sm_mamba_scan_chunked": [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p,
+    "p2p_sm_mamba_scan_chunked": [c_void_p, c_int, c_void_p, c_int, c_int, c_void_p,
                                   c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int,
                                   c_int, c_void_p],
@@ -822,13 +822,13 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
     if N > 256 or P > 256:
         raise ValueError("mamba_scan: state %d / value %d sizes above 256" % (N, P))
     E = ent.shape[0]
-    if _chunked(ent_host):
-        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, zx.device)
+    if max(e[1] for e in ent_host) >= LIGHT_MIN:
+        vent, cent = chunk_tables(ent_host, min(SCAN_CHUNK or LIGHT_CHUNK, LIGHT_CHUNK), zx.device)
         NV = vent.shape[0]
         tmp = torch.empty(NV, H, N, P, device=zx.device, dtype=torch.float32)
         decay = torch.empty(NV, H, device=zx.device, dtype=torch.float32)
         _chk(lib().p2p_sm_mamba_scan_chunked(
-            conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), xoff, dtoff, dt_bias.data_ptr(),
+            conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), dtoff, dt_bias.data_ptr(),
             A_log.data_ptr(), Dp.data_ptr(), state.data_ptr(), tmp.data_ptr(), decay.data_ptr(),
             vent.data_ptr(), NV, cent.data_ptr(), E, y.data_ptr(), H, P, N, G, _f32(zx),
             _st(zx)), "mamba_scan_chunked")

@@ -165,3 +165,30 @@ def test_latent_attn(dt, H, rank, win):
                            win, torch.empty(H, R, rank, dtype=dt, device=DEV), page, units=units,
                            max_keys=140)
         torch.testing.assert_close(d.cpu().float(), a.float(), **_tol(dt))
+
+
+@pytest.mark.parametrize("lens,starts", [([130, 64, 1], [0, 7, 3]), ([65], [0]), ([33, 200], [5, 0])])
+@pytest.mark.parametrize("H,P,N,G", [(4, 64, 128, 2), (2, 30, 17, 1), (1, 256, 256, 1)])
+@pytest.mark.parametrize("steep", [False, True])
+def test_mamba_long_portions(lens, starts, H, P, N, G, steep):
+    """Chunks of 64 on the matrix instruction: remainders, single-chunk portions beside long ones, and
+    decays so steep that a quotient of running products would overflow."""
+    g = torch.Generator().manual_seed(6)
+    inner, C = H * P, H * P + 2 * G * N
+    slots = len(lens) + 1
+    ent_h, ent, _row_ent, R = _ents(lens, starts, list(range(len(lens)))[::-1])
+    conv = torch.randn(R, C, generator=g)
+    zx = torch.randn(R, 2 * inner + 2 * G * N + H, generator=g)
+    dtb, Dp = torch.randn(H, generator=g) + (3.0 if steep else 0.0), torch.randn(H, generator=g)
+    Al = torch.rand(H, generator=g) + (3.0 if steep else -1.0)
+    S0, T0 = torch.randn(slots, H, N, P, generator=g), torch.zeros(slots, 3, C)
+    res = []
+    for dev in ("cpu", DEV):
+        S, T = S0.clone().to(dev), T0.clone().to(dev)
+        y = sm.mamba_scan(conv.to(dev), zx.to(dev), inner, inner + C, dtb.to(dev), Al.to(dev), Dp.to(dev), S, T,
+                          ent.to(dev), ent_h, torch.empty(R, inner, device=dev), H, P, N, G)
+        res.append((y.cpu(), S.cpu()))
+    (y1, s1), (y2, s2) = res
+    # sums of up to 64 x 256 fp32 products in another order, exponents of sums of 64 steps
+    for a, b in ((y1, y2), (s1, s2)):
+        torch.testing.assert_close(b, a, rtol=1e-4, atol=1e-5 * float(a.abs().max()))
