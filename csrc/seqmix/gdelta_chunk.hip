@@ -1,0 +1,384 @@
+// The generalized delta rule over long portions in chunks of up to 64 tokens on the fp32 matrix instruction
+// (v_mfma_f32_16x16x4_f32: products and sums in fp32), head sizes up to 64.  Per head and token
+//   S <- diag(w) S - (a * u)(u^T S) + k v^T,   o = S^T r,   u = k / sqrt(|k|^2 + 1e-6),   w = exp(-e^-1/2 sigmoid(.))
+// With W(s, t) the product of the decays after token s up to t, the rows p_t = u_t^T S_(t-1) of a chunk obey
+//   p_t + sum_{s<t} (u_t W(s,t-1) a_s u_s) p_s = (u_t W(-1,t-1)) S_0 + sum_{s<t} (u_t W(s,t-1) k_s) v_s,
+// a unit lower triangular system: P = G S_0 + H.  What leaves the chunk is linear in S_0 as well:
+//   S_end = T S_0 + L,   T = W(-1,end) - sum_s W(s,end) a_s u_s G_s,  L = sum_s W(s,end) (k_s v_s^T - a_s u_s H_s)
+//   o_t   = Q_t S_0 + O_t,   Q_t = r_t W(-1,t) - sum_{s<=t} (r_t W(s,t) a_s u_s) G_s,  O_t likewise with k_s v_s, H_s
+// gdelta_chunk_k forms T, L, Q, O of every (chunk, head); gdelta_chain_k walks the chunks, S <- T S + L;
+// gdelta_out_k forms o = Q S_0 + O with the head norm, weight and gate.
+//
+// W(s, t) is taken apart into exp(c_t - m) and exp(m - c_s), c the running sum of the log decays and m its value
+// after 32 tokens: a log decay lies between -0.61 and 0, so neither exponent passes 20 in size and both
+// factors are as exact as the product of up to 64 decays.  The system is solved in blocks of 16 rows, the
+// blocks on the diagonal by their inverses.
+//
+// A chunk and head are about 700 matrix instructions per wavefront.  The walk of gdelta_scan_k (once for L and T, once
+// for the outputs) took 2 x 205 us for 2048 tokens and 32 heads of 64, and the chain 654 us of 32 dependent products on
+// 32 workgroups with scalar sums; the three kernels here take 164, 36 and 20 us.
+#include "common.h"
+using namespace sm;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define GC 64               // tokens of a chunk, and the padded head size
+#define GLD 68              // row length in LDS: 16 rows x 16 bytes and 4 rows x 16 numbers both spread over the banks
+#define GD_DECAY_SCALE 0.6065306597126334f  // exp(-1/2)
+
+#define MFMA4(a, b, c) __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0)
+
+struct GdeltaArgs {
+  const void *r, *k, *v, *g, *a;
+  int ld;
+  const void* lo;
+  int ldlo;
+  const float *w0, *ab, *normw;
+  float* state;
+  float *trn, *loc, *qq, *oo;   // scratch, [chunks, H, 64, 64] each; loc becomes the state before every chunk
+  const int *vent, *cent;
+  void* out;
+  int ldo, H, D;
+  float eps;
+};
+
+template <typename T>
+__global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
+  extern __shared__ __align__(16) float smem[];
+  float* sU = smem;                  // u exp(c_(t-1) - m), later the weights of v_s in p_t
+  float* sR = sU + GC * GLD;         // r exp(c_t - m),     later the weights of p_s in o_t
+  float* sK = sR + GC * GLD;         // k exp(m - c_s)
+  float* sA = sK + GC * GLD;         // a u exp(m - c_s)
+  float* sL = sA + GC * GLD;         // weights of p_s in p_t
+  float* sB = sL + GC * GLD;         // weights of v_s in o_t
+  __shared__ float sTot[4][GC], sMid[GC], sEnd[GC];
+  __shared__ __align__(16) float sD[4][16][20];   // inverses of the blocks on the diagonal
+  const int c = blockIdx.x, h = blockIdx.y, D = p.D;
+  const Entry en = load_entry(p.vent, c);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, quad = lane >> 4;
+  // a lane's channel of the wavefront's 16 tokens
+  {
+    const int col = h * D + min(lane, D - 1);
+    const bool in = lane < D;
+    const float w0 = p.w0[col], ab = p.ab[col];
+    float kv[16], rv[16], av[16], lw[16], cw[16], sum = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int t = wave * 16 + q;
+      const size_t row = (size_t)(en.row0 + min(t, en.n - 1));
+      const bool have = in && t < en.n;
+      kv[q] = have ? ldf((const T*)p.k, row * p.ld + col) : 0.0f;
+      rv[q] = have ? ldf((const T*)p.r, row * p.ld + col) : 0.0f;
+      av[q] = sigmoidf_(ldf((const T*)p.a, row * p.ld + col) + ab);
+      lw[q] = have ? -GD_DECAY_SCALE * sigmoidf_(ldf((const T*)p.lo, row * p.ldlo + col) + w0) : 0.0f;
+      sum += lw[q];
+      cw[q] = sum;
+    }
+    sTot[wave][lane] = sum;
+    __syncthreads();
+    const float t0 = sTot[0][lane], t1 = sTot[1][lane], t2 = sTot[2][lane], t3 = sTot[3][lane];
+    const float mid = t0 + t1, before = wave == 0 ? 0.0f : wave == 1 ? t0 : wave == 2 ? mid : mid + t2;
+    if (wave == 0) {
+      sMid[lane] = expf(mid);
+      sEnd[lane] = expf(t2 + t3);   // to the chunk's end, from m
+    }
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int at = (wave * 16 + q) * GLD + lane;
+      const float u = kv[q] * (1.0f / sqrtf(wave_sum(kv[q] * kv[q]) + 1e-6f));
+      const float x = before + cw[q] - mid, down = expf(-x);
+      sU[at] = u * expf(x - lw[q]);
+      sR[at] = rv[q] * expf(x);
+      sK[at] = kv[q] * down;
+      sA[at] = av[q] * u * down;
+    }
+  }
+  // values as operands: token 16 b + quad * 4 + e, this wavefront's 16 columns
+  const int vc = wave * 16 + n16;
+  f32x4 V[4];
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int t = b * 16 + quad * 4 + e;
+      V[b][e] = (t < en.n && vc < D) ? ldf((const T*)p.v, (size_t)(en.row0 + t) * p.ld + h * D + vc) : 0.0f;
+    }
+  __syncthreads();
+  // the four tables of weights: this wavefront's 16 rows t, s <= t
+  f32x4 akk[4], auu[4], bk[4], bu[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) akk[j] = auu[j] = bk[j] = bu[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kk = 0; kk < 4; kk++) {
+    const int at = kk * 16 + quad * 4;
+    const f32x4 u = *(const f32x4*)(sU + (wave * 16 + n16) * GLD + at);
+    const f32x4 r = *(const f32x4*)(sR + (wave * 16 + n16) * GLD + at);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (j <= wave) {
+        const f32x4 kd = *(const f32x4*)(sK + (j * 16 + n16) * GLD + at);
+        const f32x4 ad = *(const f32x4*)(sA + (j * 16 + n16) * GLD + at);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          akk[j] = MFMA4(u[e], kd[e], akk[j]);
+          auu[j] = MFMA4(u[e], ad[e], auu[j]);
+          bk[j] = MFMA4(r[e], kd[e], bk[j]);
+          bu[j] = MFMA4(r[e], ad[e], bu[j]);
+        }
+      }
+  }
+  // G starts as U, Q as R: this wavefront's 16 columns
+  f32x4 G[4], Q[4];
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int at = (b * 16 + quad * 4 + e) * GLD + vc;
+      G[b][e] = sU[at];
+      Q[b][e] = sR[at];
+    }
+  __syncthreads();   // U and R have been read
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    if (j <= wave) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int t = wave * 16 + quad * 4 + e, s = j * 16 + n16, at = t * GLD + s;
+        sU[at] = s < t ? akk[j][e] : 0.0f;
+        sL[at] = s < t ? auu[j][e] : 0.0f;
+        sB[at] = s <= t ? bk[j][e] : 0.0f;
+        sR[at] = s <= t ? bu[j][e] : 0.0f;
+      }
+    }
+  __syncthreads();
+  // the inverse of this wavefront's block on the diagonal, a column per lane
+  {
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      float v = i == n16 ? 1.0f : 0.0f;
+#pragma unroll
+      for (int q = 0; q < i; q++) v = fmaf(-sL[(wave * 16 + i) * GLD + wave * 16 + q], x[q], v);
+      x[i] = v;
+    }
+    if (quad == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) sD[wave][i][n16] = x[i];
+    }
+  }
+  // right side of H
+  f32x4 Hm[4];
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    Hm[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j <= b; j++) {
+      const f32x4 f = *(const f32x4*)(sU + (b * 16 + n16) * GLD + j * 16 + quad * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) Hm[b] = MFMA4(f[e], V[j][e], Hm[b]);
+    }
+  }
+  __syncthreads();   // the inverses
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+#pragma unroll
+    for (int j = 0; j < b; j++) {
+      const f32x4 f = *(const f32x4*)(sL + (b * 16 + n16) * GLD + j * 16 + quad * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        G[b] = MFMA4(-f[e], G[j][e], G[b]);
+        Hm[b] = MFMA4(-f[e], Hm[j][e], Hm[b]);
+      }
+    }
+    const f32x4 f = *(const f32x4*)&sD[b][n16][quad * 4];
+    f32x4 g = {0.f, 0.f, 0.f, 0.f}, x = g;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      g = MFMA4(f[e], G[b][e], g);
+      x = MFMA4(f[e], Hm[b][e], x);
+    }
+    G[b] = g;
+    Hm[b] = x;
+  }
+  const size_t base = ((size_t)c * p.H + h) * GC * GC;
+  const float emid = sMid[vc];
+  // outputs: Q and O
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    f32x4 O = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j <= b; j++) {
+      const f32x4 fu = *(const f32x4*)(sR + (b * 16 + n16) * GLD + j * 16 + quad * 4);
+      const f32x4 fk = *(const f32x4*)(sB + (b * 16 + n16) * GLD + j * 16 + quad * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        Q[b] = MFMA4(-fu[e], G[j][e], Q[b]);
+        O = MFMA4(-fu[e], Hm[j][e], O);
+        O = MFMA4(fk[e], V[j][e], O);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const size_t at = base + (b * 16 + quad * 4 + e) * GC + vc;
+      p.qq[at] = Q[b][e] * emid;
+      p.oo[at] = O[e];
+    }
+  }
+  // the end of the chunk: T and L
+#pragma unroll
+  for (int it = 0; it < 4; it++) {
+    f32x4 tr = {0.f, 0.f, 0.f, 0.f}, lc = tr;
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int at = (b * 16 + quad * 4 + e) * GLD + it * 16 + n16;
+        const float ad = sA[at], kd = sK[at];
+        tr = MFMA4(ad, G[b][e], tr);
+        lc = MFMA4(kd, V[b][e], lc);
+        lc = MFMA4(-ad, Hm[b][e], lc);
+      }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int i = it * 16 + quad * 4 + e;
+      const float end = sEnd[i];
+      p.trn[base + i * GC + vc] = (i == vc ? end * emid : 0.0f) - end * tr[e] * emid;
+      p.loc[base + i * GC + vc] = end * lc[e];
+    }
+  }
+}
+
+// S <- T S + L over each portion's chunks, 16 columns of a head per workgroup, a wavefront per 16 rows; the state before
+// a chunk replaces its L.  What a chunk needs from memory does not depend on the state: it is read a chunk ahead.
+__global__ void __launch_bounds__(256) gdelta_chain_k(GdeltaArgs p) {
+  __shared__ float sS[2][GC][17];
+  const int c0 = p.cent[4 * blockIdx.z], nc = p.cent[4 * blockIdx.z + 1], start = p.cent[4 * blockIdx.z + 2],
+            slot = p.cent[4 * blockIdx.z + 3];
+  const int h = blockIdx.y, D = p.D;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, quad = lane >> 4;
+  const int col = blockIdx.x * 16 + n16, row = wave * 16 + quad * 4;   // C layout: rows row .. row + 3
+  float* sg = p.state + ((size_t)slot * p.H + h) * D * D;
+  f32x4 cur;
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    cur[e] = (start > 0 && row + e < D && col < D) ? sg[(size_t)(row + e) * D + col] : 0.0f;
+  const size_t step = (size_t)p.H * GC * GC;
+  const float* tp = p.trn + (size_t)c0 * step + (size_t)h * GC * GC + (wave * 16 + n16) * GC + quad * 4;
+  float* lp = p.loc + (size_t)c0 * step + (size_t)h * GC * GC + row * GC + col;
+  f32x4 T[4], L;
+  auto load = [&](int c, f32x4 (&t)[4], f32x4& l) {
+#pragma unroll
+    for (int b = 0; b < 4; b++) t[b] = *(const f32x4*)(tp + c * step + b * 16);
+#pragma unroll
+    for (int e = 0; e < 4; e++) l[e] = lp[c * step + e * GC];
+  };
+  load(0, T, L);
+  for (int c = 0; c < nc; c++) {
+    f32x4 Tn[4], Ln;
+    if (c + 1 < nc) load(c + 1, Tn, Ln);
+    float(*S)[17] = sS[c & 1];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      S[row + e][n16] = cur[e];
+      lp[c * step + e * GC] = cur[e];
+    }
+    __syncthreads();
+    f32x4 a[4];
+    a[0] = L;
+    a[1] = a[2] = a[3] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) a[b] = MFMA4(T[b][e], S[b * 16 + quad * 4 + e][n16], a[b]);
+    cur = (a[0] + a[1]) + (a[2] + a[3]);
+#pragma unroll
+    for (int b = 0; b < 4; b++) T[b] = Tn[b];
+    L = Ln;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    if (row + e < D && col < D) sg[(size_t)(row + e) * D + col] = cur[e];
+}
+
+// o = Q S + O, head norm, weight and gate; a wavefront per 16 tokens, column n16 * 4 + j in tile j
+template <typename T>
+__global__ void __launch_bounds__(256) gdelta_out_k(GdeltaArgs p) {
+  const int c = blockIdx.x, h = blockIdx.y, D = p.D;
+  const Entry en = load_entry(p.vent, c);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, quad = lane >> 4;
+  if (wave * 16 >= en.n) return;
+  const size_t base = ((size_t)c * p.H + h) * GC * GC;
+  const float* qp = p.qq + base + (wave * 16 + n16) * GC + quad * 4;
+  const float* sp = p.loc + base + quad * 4 * GC + n16 * 4;
+  const float* op = p.oo + base + (wave * 16 + quad * 4) * GC + n16 * 4;
+  f32x4 q[4], s[4][4], o[4], acc[4];
+#pragma unroll
+  for (int b = 0; b < 4; b++) q[b] = *(const f32x4*)(qp + b * 16);
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) s[b][e] = *(const f32x4*)(sp + (b * 16 + e) * GC);
+#pragma unroll
+  for (int e = 0; e < 4; e++) o[e] = *(const f32x4*)(op + e * GC);
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[j][e] = o[e][j];
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[j] = MFMA4(q[b][e], s[b][e][j], acc[j]);
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int t = wave * 16 + quad * 4 + e;
+    float ss = 0.0f;   // columns beyond D are zero
+#pragma unroll
+    for (int j = 0; j < 4; j++) ss += acc[j][e] * acc[j][e];
+#pragma unroll
+    for (int m = 8; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
+    const float rs = 1.0f / sqrtf(ss / (float)D + p.eps);
+    if (t >= en.n) continue;
+    const size_t row = (size_t)(en.row0 + t);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int i = n16 * 4 + j, at = h * D + i;
+      if (i < D)
+        stf((T*)p.out, row * p.ldo + at, acc[j][e] * rs * p.normw[at] * sigmoidf_(ldf((const T*)p.g, row * p.ld + at)));
+    }
+  }
+}
+
+extern "C" {
+
+// 1 when the kernels serve this head size
+int p2p_sm_gdelta_chunk_ok(int D) { return D >= 1 && D <= GC; }
+
+// vent [NV]: the portions' chunks of at most 64 tokens as entries (row0, n, 1, chunk index); tmp: 4 fp32 buffers of
+// [NV, H, 64, 64]; cent: per portion (first chunk, chunks, first position, slot)
+int p2p_sm_gdelta_chunk(const void* r, const void* k, const void* v, const void* g, const void* a, int ld,
+                        const void* lo, int ldlo, const float* w0, const float* ab, const float* normw, float* state,
+                        float* tmp, const int* vent, int NV, const int* cent, int E, void* out, int ldo, int H, int D,
+                        float eps, int f32, hipStream_t st) {
+  if (E <= 0 || NV <= 0) return 0;
+  if (!p2p_sm_gdelta_chunk_ok(D)) return (int)hipErrorInvalidValue;
+  const size_t sz = (size_t)NV * H * GC * GC;
+  const GdeltaArgs p = {r, k, v, g, a, ld, lo, ldlo, w0, ab, normw, state, tmp, tmp + sz, tmp + 2 * sz, tmp + 3 * sz,
+                        vent, cent, out, ldo, H, D, eps};
+  constexpr int shm = 6 * GC * GLD * 4;
+  static const hipError_t attr = [] {
+    const hipError_t e = hipFuncSetAttribute((const void*)gdelta_chunk_k<float>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    return e != hipSuccess ? e
+                           : hipFuncSetAttribute((const void*)gdelta_chunk_k<bf16>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+  }();
+  if (attr != hipSuccess) return (int)attr;
+  SM_DISPATCH_T(f32, hipLaunchKernelGGL(gdelta_chunk_k<T>, dim3(NV, H), dim3(256), shm, st, p));
+  hipLaunchKernelGGL(gdelta_chain_k, dim3((D + 15) / 16, H, E), dim3(256), 0, st, p);
+  SM_DISPATCH_T(f32, hipLaunchKernelGGL(gdelta_out_k<T>, dim3(NV, H), dim3(256), 0, st, p));
+  return (int)hipGetLastError();
+}
+
+}  // extern "C"

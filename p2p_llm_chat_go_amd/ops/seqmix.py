@@ -48,6 +48,10 @@ _SIGS = {
     "p2p_sm_gdelta_scan": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                             c_void_p, c_void_p, c_int, c_void_p, c_int, c_int,
                                             c_int, c_float, c_int, c_void_p],
+    "p2p_sm_gdelta_chunk": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p,
+                                                    c_void_p, c_void_p, c_void_p, c_void_p, c_int,
+                                                    c_void_p, c_int, c_void_p, c_int, c_int, c_int,
+                                                    c_float, c_int, c_void_p],
     "p2p_sm_gdelta_scan_chunked": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                                     c_void_p, c_int, c_void_p, c_int, c_int, c_int,
@@ -663,6 +667,7 @@ def _chunked(ent_host) -> bool:
 
 # ------------------------------------------------------------------ generalized delta rule
 GD_DECAY_SCALE = math.exp(-0.5)
+GD_MATRIX_MAX = 64    # head sizes of the matrix-instruction chunks (larger ones walk theirs)
 
 
 def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: int, D: int,
@@ -702,6 +707,15 @@ def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: 
     assert ent.dtype == torch.int32 and ent.is_contiguous() and ent.shape[1] == 4
     if D > 256:
         raise ValueError("gdelta_scan: head size %d > 256" % D)
+    if D <= GD_MATRIX_MAX and max(e[1] for e in ent_host) >= LIGHT_MIN:
+        vent, cent = chunk_tables(ent_host, min(SCAN_CHUNK or LIGHT_CHUNK, LIGHT_CHUNK), r.device)
+        tmp = torch.empty(4, vent.shape[0], H, 64, 64, device=r.device, dtype=torch.float32)
+        _chk(lib().p2p_sm_gdelta_chunk(
+            r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), a.data_ptr(), ld,
+            lo.data_ptr(), lo.stride(0), w0.data_ptr(), ab.data_ptr(), normw.data_ptr(),
+            state.data_ptr(), tmp.data_ptr(), vent.data_ptr(), vent.shape[0], cent.data_ptr(), E,
+            out.data_ptr(), out.stride(0), H, D, eps, _f32(r), _st(r)), "gdelta_chunk")
+        return out
     if _chunked(ent_host):
         vent, cent = chunk_tables(ent_host, SCAN_CHUNK, r.device)
         tmp = torch.empty(3, vent.shape[0], H, D, D, device=r.device, dtype=torch.float32)

@@ -192,3 +192,28 @@ def test_mamba_long_portions(lens, starts, H, P, N, G, steep):
     # sums of up to 64 x 256 fp32 products in another order, exponents of sums of 64 steps
     for a, b in ((y1, y2), (s1, s2)):
         torch.testing.assert_close(b, a, rtol=1e-4, atol=1e-5 * float(a.abs().max()))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,starts", [([130, 64, 1], [0, 7, 3]), ([65], [0]), ([33, 200], [5, 0])])
+@pytest.mark.parametrize("H,D", [(4, 64), (2, 33), (1, 5)])
+@pytest.mark.parametrize("decay", [-20.0, 0.0, 20.0])
+def test_gdelta_long_portions(dt, lens, starts, H, D, decay):
+    """Chunks of 64 on the matrix instruction: remainders, single-chunk portions beside long ones, decays of one, mixed,
+    and the strongest there are."""
+    g = torch.Generator().manual_seed(8)
+    n, slots = H * D, len(lens) + 1
+    ent_h, ent, _row_ent, R = _ents(lens, starts, list(range(len(lens)))[::-1])
+    proj, lo = torch.randn(R, 5 * n + 3, generator=g).to(dt), torch.randn(R, n, generator=g).to(dt)
+    w0, ab, nw = torch.randn(n, generator=g) + decay, torch.randn(n, generator=g), torch.randn(n, generator=g)
+    S0 = torch.randn(slots, H, D, D, generator=g)
+    res = []
+    for dev in ("cpu", DEV):
+        S, p = S0.clone().to(dev), proj.to(dev)
+        o = sm.gdelta_scan(*[p[:, i * n:(i + 1) * n] for i in range(5)], lo.to(dev), w0.to(dev), ab.to(dev), nw.to(dev), S,
+                           ent.to(dev), ent_h, torch.empty(R, n, dtype=dt, device=dev), H, D, 1e-5)
+        res.append((o.cpu().float(), S.cpu()))
+    (o1, s1), (o2, s2) = res
+    # 200 tokens of fp32 sums in another order; without decay nothing is forgotten on the way
+    torch.testing.assert_close(s2, s1, rtol=2e-4, atol=2e-5 * float(s1.abs().max()))
+    torch.testing.assert_close(o2, o1, **(_tol(dt) if dt == torch.bfloat16 else dict(rtol=1e-3, atol=2e-4)))
