@@ -107,7 +107,6 @@ import json
 import os
 
 import torch
-import torch.nn.functional as F
 
 from ..ops import PAGE
 from ..ops import seqmix as sm
@@ -395,10 +394,10 @@ class Mixer:
 
     def forward_proj(self, proj, b: "StepBatch", cache, layer: int):
         mid = torch.empty(b.R, self.n_mid, device=proj.device, dtype=proj.dtype)
-        return F.linear(self.mix(proj, b, cache, layer, mid), self.wo, self.b_out)
+        return sm.linear(self.mix(proj, b, cache, layer, mid), self.wo, self.b_out)
 
     def forward(self, h, b: "StepBatch", cache, layer: int):
-        return self.forward_proj(F.linear(h, self.w_in, self.b_in), b, cache, layer)
+        return self.forward_proj(sm.linear(h, self.w_in, self.b_in), b, cache, layer)
 
 
 class GeneralDelta(Mixer):
@@ -431,15 +430,15 @@ class GeneralDelta(Mixer):
 
     def forward(self, h, b, cache, layer):
         n = self.n
-        proj = F.linear(h, self.w_in)
+        proj = sm.linear(h, self.w_in)
         low = proj[:, 5 * n:]
         sm.tanh_(low)
-        lo = F.linear(low, self.w2)
+        lo = sm.linear(low, self.w2)
         out = torch.empty(b.R, n, device=h.device, dtype=h.dtype)
         sm.gdelta_scan(proj[:, 0:n], proj[:, n:2 * n], proj[:, 2 * n:3 * n], proj[:, 3 * n:4 * n],
                        proj[:, 4 * n:5 * n], lo, self.w0, self.ab, self.normw,
                        cache.state[layer]["S"], b.ent, b.ent_host, out, self.H, self.D, self.eps)
-        return F.linear(out, self.wo)
+        return sm.linear(out, self.wo)
 
 
 class Mamba2(Mixer):
@@ -475,7 +474,7 @@ class Mamba2(Mixer):
 
     def forward(self, h, b, cache, layer):
         st = cache.state[layer]
-        zx = F.linear(h, self.w_in)
+        zx = sm.linear(h, self.w_in)
         conv = torch.empty(b.R, self.C, device=h.device, dtype=torch.float32)
         sm.mamba_conv(zx, self.inner, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, conv)
         y = torch.empty(b.R, self.inner, device=h.device, dtype=torch.float32)
@@ -483,7 +482,7 @@ class Mamba2(Mixer):
                       st["S"], st["tail"], b.ent, b.ent_host, y, self.H, self.P, self.N, self.G)
         yn = torch.empty(b.R, self.inner, device=h.device, dtype=h.dtype)
         sm.rmsnorm(y, self.normw, self.eps, yn, parts=self.ng)
-        return F.linear(yn, self.wo)
+        return sm.linear(yn, self.wo)
 
 
 class Mamba1(Mixer):
@@ -523,7 +522,7 @@ class Mamba1(Mixer):
         st, I = cache.state[layer], self.I
         x = torch.empty(b.R, I, device=proj.device, dtype=proj.dtype)
         sm.mamba_conv(proj, 0, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, x, roll=True)
-        xp = F.linear(x, self.w_x)
+        xp = sm.linear(x, self.w_x)
         sm.selective_scan(x, xp, self.rank, self.w_dt, self.dtb, self.A2, self.Dp, proj[:, I:2 * I],
                           st["S"], b.ent, b.ent_host, out)
         if out_scale != 1.0:
@@ -606,7 +605,7 @@ class LatentAttention(Mixer):
     def forward(self, h, b, cache, layer):
         H, D, V, r = self.H, self.D, self.V, self.rank
         pool = cache.paged[layer]
-        proj = F.linear(h, self.w_in)
+        proj = sm.linear(h, self.w_in)
         sm.rmsnorm(proj[:, H * D:H * D + r], self.cnorm, self.eps, pool, out_rows=b.cache_rows)
         qa = torch.bmm(proj[:, :H * D].view(b.R, H, D).transpose(0, 1), self.uk)   # [H, R, rank]
         ol = torch.empty_like(qa)
@@ -616,7 +615,7 @@ class LatentAttention(Mixer):
         o = torch.bmm(ol, self.uvt)                                                # [H, R, V]
         gated = torch.empty(b.R, H * V, device=h.device, dtype=h.dtype)
         sm.sigmoid_gate(o, proj[:, H * D + r:], gated, H, V)
-        return F.linear(gated, self.wo)
+        return sm.linear(gated, self.wo)
 
 
 class WindowAttention(Mixer):
@@ -970,7 +969,7 @@ class RopeLatentAttention(Mixer):
             cq = torch.empty(R, qr, device=dev, dtype=dt)
             sm.latent_prep(proj, qr, r, Rd, self.qnorm, self.cnorm, self.inv_freq, b.pos, b.cache_rows,
                            pool, self.eps, cq, rm=self.rot_mag)
-            q = F.linear(cq, self.uq)                                              # [R, H*(D+Rd)]
+            q = sm.linear(cq, self.uq)                                              # [R, H*(D+Rd)]
         else:
             qr = H * (D + Rd)
             q = proj[:, :qr]
@@ -1096,8 +1095,8 @@ class GatedDelta(Mixer):
         conv = torch.empty(b.R, C, device=proj.device, dtype=torch.float32)
         sm.mamba_conv(proj, 0, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, conv)
         sm.conv_tail_roll(proj, 0, st["tail"], b.ent, b.ent_host, C)
-        araw = F.linear(proj[:, C + H:C + H + self.ra], self.w_a2)
-        gate = F.linear(proj[:, C + H + self.ra:C + H + self.ra + self.rg], self.w_g2)
+        araw = sm.linear(proj[:, C + H:C + H + self.ra], self.w_a2)
+        gate = sm.linear(proj[:, C + H + self.ra:C + H + self.ra + self.rg], self.w_g2)
         sm.gated_delta_scan(conv, araw, proj[:, C:C + H], gate, self.A_log, self.dt_bias, self.normw,
                             st["S"], b.ent, b.ent_host, out, H, self.G, self.D, self.V, self.eps,
                             out_scale=out_scale)
@@ -1271,10 +1270,10 @@ class DenseFF:
         """gu = [gate | up] projections of the input."""
         act = torch.empty(gu.shape[0], self.F, device=gu.device, dtype=gu.dtype)
         self.fill(gu, None, act)
-        return F.linear(act, self.w_down)
+        return sm.linear(act, self.w_down)
 
     def forward(self, h):
-        return self.forward_proj(F.linear(h, self.w_gu))
+        return self.forward_proj(sm.linear(h, self.w_gu))
 
 
 class MoEFF:
@@ -1414,10 +1413,10 @@ class SoftmaxMoEFF:
     def forward(self, h):
         y = self.routed(h)
         if self.Fs:
-            proj = F.linear(h, self.w_in)
+            proj = sm.linear(h, self.w_in)
             mid = torch.empty(h.shape[0], self.Fs, device=h.device, dtype=h.dtype)
             sm.relu2_gate(proj, proj[:, self.Fs:self.Fs + 1], mid)
-            y = y + F.linear(mid, self.w_out)
+            y = y + sm.linear(mid, self.w_out)
         return y
 
 
@@ -1509,8 +1508,8 @@ class TopMoEFF:
         y = sm.expert_combine(y, wts, torch.empty(h.shape[0], self.width, device=h.device, dtype=h.dtype))
         if self.Fs:
             mid = torch.empty(h.shape[0], self.Fs, device=h.device, dtype=h.dtype)
-            sm.glu_act(F.linear(h, self.w_in), mid, "silu")
-            y = y + F.linear(mid, self.w_out)
+            sm.glu_act(sm.linear(h, self.w_in), mid, "silu")
+            y = y + sm.linear(mid, self.w_out)
         return y
 
 
@@ -1853,7 +1852,7 @@ class HybridModel:
 
     def _head(self, hn):
         cfg, w = self.cfg, self.w
-        y = F.linear(hn, w.head)
+        y = sm.linear(hn, w.head)
         if not cfg.logit_softcap and cfg.logit_scale == 1.0:
             return y.float()
         return sm.softcap(y, cfg.logit_softcap, torch.empty(y.shape, device=y.device, dtype=torch.float32),
@@ -1884,10 +1883,10 @@ class HybridModel:
             elif moe[i]:
                 mid = proj = None
                 if L.ff.n_mid:
-                    proj = F.linear(h, L.ff.w_in)
+                    proj = sm.linear(h, L.ff.w_in)
                     mid = torch.empty(R, L.ff.n_mid, device=dev, dtype=self.dtype)
                 routed = L.ff.fill_routed(proj, h, mid, cnts[sum(moe[:i]), :L.ff.E])
-                y = F.linear(mid, L.ff.w_out) if mid is not None else None
+                y = sm.linear(mid, L.ff.w_out) if mid is not None else None
             else:
                 y = L.ff.forward(h)
             if k + 1 < len(subs):
@@ -1937,15 +1936,15 @@ class HybridModel:
                          w1=L.norm1, out1=h1, w2=n2, out2=o2, routed=routed)
             mm = L.mixer.n_mid
             mid = torch.empty(R, L.w_out_all.shape[1], device=self.device, dtype=self.dtype)
-            L.mixer.mix(F.linear(h1, L.mixer.w_in, L.mixer.b_in), b, self.cache, k, mid[:, :mm])
+            L.mixer.mix(sm.linear(h1, L.mixer.w_in, L.mixer.b_in), b, self.cache, k, mid[:, :mm])
             extra = routed = None
             if L.ff is not None:
-                proj = F.linear(h2, L.ff.w_in) if L.ff.w_in is not None else None
+                proj = sm.linear(h2, L.ff.w_in) if L.ff.w_in is not None else None
                 if moe[k]:
                     routed = L.ff.fill_routed(proj, h2, mid[:, mm:], cnts[sum(moe[:k]), :L.ff.E])
                 else:
                     extra = L.ff.fill(proj, h2, mid[:, mm:])
-            y = F.linear(mid, L.w_out_all)
+            y = sm.linear(mid, L.w_out_all)
         sm.add_norm2(x, y, extra, routed=routed)
         if layer_out is not None:
             layer_out.append(x.clone())
@@ -1967,11 +1966,11 @@ class HybridModel:
         parts, eps = cfg.norm_groups, cfg.eps
         for i, L in enumerate(w.layers):
             n = L.mixer.w_in.shape[0]
-            proj = F.linear(h, L.w_in1)
+            proj = sm.linear(h, L.w_in1)
             m = L.mixer.forward_proj(proj[:, :n], b, self.cache, i)
             sm.gate_norm_add(x, m, proj[:, n:], L.rg1b, L.norm1, parts, eps, next_out=nxt)
             if L.ff is not None:
-                proj = F.linear(h, L.w_in2)
+                proj = sm.linear(h, L.w_in2)
                 if L.ff.w_in is None:
                     f, gate = L.ff.forward(h), proj
                 else:
@@ -2019,12 +2018,12 @@ class HybridModel:
         h = torch.empty(b.R, cfg.width, device=self.device, dtype=self.dtype)
         sm.rmsnorm(x, w.layers[0].norm1, cfg.eps, h)
         for i, L in enumerate(w.layers):
-            proj = F.linear(h, L.w_in_all)
+            proj = sm.linear(h, L.w_in_all)
             nm, mm = L.mixer.w_in.shape[0], L.mixer.n_mid
             mid = torch.empty(b.R, L.w_out_all.shape[1], device=self.device, dtype=self.dtype)
             L.mixer.mix(proj[:, :nm], b, self.cache, i, mid[:, :mm])
             extra = L.ff.fill(proj[:, nm:], h, mid[:, mm:]) if L.ff is not None else None
-            y = F.linear(mid, L.w_out_all)
+            y = sm.linear(mid, L.w_out_all)
             nxt = w.layers[i + 1].norm1 if i + 1 < len(w.layers) else None
             sm.add_norm(x, y, extra, cfg.eps, next_w=nxt, next_out=h)
             if layer_out is not None:

@@ -33,6 +33,7 @@ import os
 import threading
 
 import torch
+import torch.nn.functional as F
 
 from . import _lib
 
@@ -48,6 +49,8 @@ _SIGS = {
     "p2p_sm_gdelta_scan": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                             c_void_p, c_void_p, c_int, c_void_p, c_int, c_int,
                                             c_int, c_float, c_int, c_void_p],
+    "p2p_sm_skinny": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                      c_void_p],
     "p2p_sm_gdelta_chunk": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                                     c_void_p, c_int, c_void_p, c_int, c_int, c_int,
@@ -294,6 +297,41 @@ def embed_rows(embed, ids, out, h_out=None, scale: float = 1.0):
                                  _lib.ptr(h_out), ldh, R, W, scale, _f32(embed), _st(out)),
          "embed_rows")
     return out
+
+
+def _skinny(x, w) -> bool:
+    """Products that ``csrc/seqmix/skinny.hip`` takes from the library.  Where the lines lie (bf16 / fp32,
+    a captured graph, library -> kernel in us): at most 16 rows of one matrix instruction; K, because one
+    workgroup walks all of it (8 rows, 2048 x 8192: 12.9 -> 15.0, 2048 x 4096: 12.5 -> 8.3; fp32
+    2048 x 4096: 13.2 -> 15.0, 2048 x 2048: 10.5 -> 8.5); N, because every workgroup reads the
+    activations again (8 rows, 32000 x 2048: 33.7 -> 33.1; 16 rows, 10272 x 2048: 14.6 -> 15.9,
+    4608 x 2048: 12.0 -> 10.9; fp32 4608 x 2048: 14.1 -> 16.4); fp32 from 1024 columns on (96 x 2048:
+    6.7 -> 7.7, bf16 5.4 -> 4.8).  The rest: what 16-byte loads need."""
+    M, K = x.shape
+    N = w.shape[0]
+    if not (0 < M <= 16 and x.is_cuda and w.is_cuda and x.dtype == w.dtype and w.shape[1] == K
+            and x.stride(1) == 1 and w.is_contiguous()):
+        return False
+    if x.dtype == torch.bfloat16:
+        fits, ep = K <= 4096 and N <= (16384 if M <= 8 else 8192), 8
+    elif x.dtype == torch.float32:
+        fits, ep = K <= 2048 and N >= 1024 and N * K <= 8 << 20, 4
+    else:
+        return False
+    return (fits and K >= ep and K % ep == 0 and x.stride(0) % ep == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def linear(x, w, b=None):
+    """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, the shapes of ``_skinny`` on a
+    kernel for few rows."""
+    if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
+            b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
+        return F.linear(x, w, b)
+    y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
+    _chk(lib().p2p_sm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), _lib.ptr(b), y.data_ptr(), x.shape[0],
+                             w.shape[0], x.shape[1], _f32(x), _st(x)), "skinny")
+    return y
 
 
 def rmsnorm(x, w, eps, out, parts: int = 1, in_rows=None, out_rows=None):

@@ -217,3 +217,21 @@ def test_gdelta_long_portions(dt, lens, starts, H, D, decay):
     # 200 tokens of fp32 sums in another order; without decay nothing is forgotten on the way
     torch.testing.assert_close(s2, s1, rtol=2e-4, atol=2e-5 * float(s1.abs().max()))
     torch.testing.assert_close(o2, o1, **(_tol(dt) if dt == torch.bfloat16 else dict(rtol=1e-3, atol=2e-4)))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 7, 16, 17])
+@pytest.mark.parametrize("N,K", [(1, 8), (1024, 4), (1040, 64), (1031, 1000), (1025, 2048), (33, 4096), (16, 4104)])
+@pytest.mark.parametrize("off,bias", [(0, False), (8, True), (3, True)])
+def test_linear_few_rows(dt, M, N, K, off, bias):
+    """Edges of the 16 columns, of the 128-byte pieces and of the eight wavefronts' turns, strided and unaligned
+    rows; shapes on both sides of the rule."""
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(M, K + 24, generator=g).to(dt).to(DEV)[:, off:off + K]
+    w, b = torch.randn(N, K, generator=g).to(dt).to(DEV), torch.randn(N, generator=g).to(dt).to(DEV) if bias else None
+    y = sm.linear(x, w, b)
+    ref = x.double() @ w.double().t() + (b.double() if bias else 0.0)
+    # one rounding of the result, and K products summed in fp32: eps |x| |w| sqrt(K) with room for the tail
+    eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -23
+    torch.testing.assert_close(y.double(), ref, rtol=eps, atol=8 * 2.0 ** -24 * K + 1e-6)
+    assert y.dtype == dt and y.is_contiguous()
