@@ -235,3 +235,28 @@ def test_linear_few_rows(dt, M, N, K, off, bias):
     eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -23
     torch.testing.assert_close(y.double(), ref, rtol=eps, atol=8 * 2.0 ** -24 * K + 1e-6)
     assert y.dtype == dt and y.is_contiguous()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [4, 256, 260, 1023, 1024, 1028, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("off", [0, 4, 1])   # first column of the rows and vectors: aligned for one wide load, or not
+def test_row_passes_by_width(dt, n, off):
+    """The row passes at the edges of the widths that a form takes, and on rows that wide loads cannot take."""
+    g = torch.Generator().manual_seed(10)
+    R = 5
+    x, big = torch.randn(R, n, generator=g), torch.randn(R, 3 * n + 12, generator=g).to(dt)
+    vecs = torch.randn(4, 2 * n + 8, generator=g)
+    res = []
+    for dev in ("cpu", DEV):
+        b, v = big.to(dev), [t.to(dev)[off:off + n] for t in vecs]
+        ya, yb = b[:, off:off + n], b[:, n + 4 + off:n + 4 + off + n]
+        out = [torch.zeros(R, n + 8, dtype=dt, device=dev)[:, off:off + n] for _ in range(5)]
+        x1 = sm.norm_scale_add(x.clone().to(dev), ya, v[0], v[1], 1e-5, v[2], out[0])
+        x2 = sm.add_norm(x.clone().to(dev), ya, yb, 1e-5, v[0], out[1])
+        x3 = sm.add_norm2(x.clone().to(dev), ya, yb, vec=v[3], eps=1e-5, w1=v[0], out1=out[2], w2=v[1][:1], out2=out[3])
+        parts = 2 if n % 2 == 0 else 1
+        sm.rmsnorm(ya, v[1], 1e-5, out[4], parts=parts)
+        res.append([t.float().cpu() for t in [x1, x2, x3] + out])
+    # sums of up to 4100 fp32 squares in another order, then one rounding; the two wide inputs double the scale
+    for p, q in zip(*res):
+        torch.testing.assert_close(q, p, **(_tol(dt) if dt == torch.bfloat16 else dict(rtol=1e-5, atol=1e-5)))
