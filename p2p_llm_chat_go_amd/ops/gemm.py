@@ -269,6 +269,19 @@ def _code(wt, M, epi, norm, waves):
     return _TUNE.get(tune_key(wt, M, epi, norm), 0)
 
 
+def _untuned(wt, x, epi) -> int:
+    """Launch code of a shape the table does not hold.  Logits of 16 rows and more (the table's LM head entry is the
+    greedy one) go to the wide kernel, which reads the activations once per 128 columns instead of once per
+    16: 128256 x 4096 at 8 / 16 / 17 / 32 / 64 rows, skinny 172 / 207 / 227 / 304 / 533 us, wide 175 / 189 / 176 /
+    188 / 221; 32000 x 4096 46 / 56 / 63 / 82 / 164 and 50 / 53 / 48 / 50 / 55.  Fewer columns than fill the chip
+    with workgroups of 128 (250 at 32000) would split K and keep the skinny kernel."""
+    N, K = tiled_shape(wt)
+    if (epi == EPI_F32 and 16 <= x.shape[0] <= SKINNY_MAX_M and N >= 128 * 250 and not _is_f8(wt)
+            and wide_ok(N, K, epi) and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0):
+        return WIDE_FLAG | WIDE16
+    return 0
+
+
 def tile_weight(w: torch.Tensor) -> torch.Tensor:
     """[N, K] (nn.Linear layout) -> fragment-major [N/16, K/32, 64, 8]."""
     N, K = w.shape
@@ -351,7 +364,7 @@ def skinny_gemm(wt: torch.Tensor, x: torch.Tensor, epi: int = EPI_STORE, norm: b
         xs = x[m0:m0 + mc]
         os_ = out[m0:m0 + mc]
         wp, sp = _wptr(wt)
-        code = _code(wt, mc, epi, norm, waves)
+        code = _code(wt, mc, epi, norm, waves) or _untuned(wt, xs, epi)
         if code & PERSIST_FLAG:
             _lib.experimental()  # the persistent GEMV's library (its symbol, found by dlsym)
         if code & AFRAG_FLAG and not x_packed:
