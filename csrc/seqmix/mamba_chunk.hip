@@ -6,12 +6,14 @@
 //                position 0); the last one is the slot's new state
 //   output pass  y_t = exp(c_t) S^T C_t + sum_{s <= t} exp(c_t - c_s) dt_s (C_t . B_s) x_s + D x_t,  y *= silu(z)
 // Every exponent is <= 0, so nothing overflows whatever the step sizes are.  One workgroup of four wavefronts per
-// (chunk, head); sizes are padded to multiples of 16 with zeros in LDS, rows are laid out so that the
-// lanes of a fragment read hit different banks.
+// (chunk, head); sizes are padded to multiples of 16 with zeros in LDS.
 //
 // The walk of mamba_scan_k does the same 1 074 M state updates of a prompt of 2048 tokens (64 heads, 128 x 64 states)
 // twice, token after token: 240 us each, bound by the chain per token.  The matrix form does 3.7 MFLOP per chunk and
-// head, bound by LDS reads per product and by staging B and C from L2 for every head: 61 + 30 + 137 us.
+// head: 46 + 30 + 87 us, bound by each workgroup's chain (inputs into LDS, then products) with three workgroups
+// per CU; the output pass's products alone take 31 us at the card's fp32 rate.  LDS is read four numbers at a
+// time: with one number per read, C and the weights in LDS too, and one row's load in flight per thread while staging,
+// the passes took 61 + 30 + 137.
 #include "common.h"
 using namespace sm;
 
@@ -19,10 +21,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define MC 64   // tokens of a chunk
 
-// row lengths in LDS: fragments that take 16 rows x 4 neighbours want ld = 4 mod 64, fragments that take 4
-// rows x 16 neighbours ld = 16 mod 64
+// row lengths in LDS: reads of four neighbours by 16 lanes, a row each, want ld = 4 mod 64; reads of two neighbours
+// by 2 x 16 lanes along two rows ld = 32 mod 64; reads of four neighbours along a row take any
 static __host__ __device__ __forceinline__ int ld_rows(int n) { return n + ((4 - n) & 63); }
-static __host__ __device__ __forceinline__ int ld_cols(int n) { return n + ((16 - n) & 63); }
+static __host__ __device__ __forceinline__ int ld_pairs(int n) { return n + ((32 - n) & 63); }
 
 struct MambaChunkArgs {
   const float* conv;   // [R, C] = x | B | C after the convolution
@@ -36,13 +38,18 @@ struct MambaChunkArgs {
   int H, P, N, G, NV, vec;
 };
 
-// dt and c of the chunk's tokens (zero steps beyond it) by the first wavefront
+// dt and c of the chunk's tokens (zero steps beyond it) by the first wavefront: the loads, then the rest once
+// other loads are under way too
 template <typename T>
-__device__ __forceinline__ void chunk_steps(const MambaChunkArgs& a, const Entry& en, int h, float* sdt, float* sc) {
+__device__ __forceinline__ float chunk_dt(const MambaChunkArgs& a, const Entry& en, int h) {
+  const int t = threadIdx.x;
+  return t < en.n && t < 64 ? ldf((const T*)a.zx, (size_t)(en.row0 + t) * a.ldz + a.dtoff + h) : 0.0f;
+}
+__device__ __forceinline__ void chunk_steps(const MambaChunkArgs& a, const Entry& en, int h, float raw, float* sdt,
+                                            float* sc) {
   if (threadIdx.x >= 64) return;
   const int t = threadIdx.x;
-  float dt = 0.0f;
-  if (t < en.n) dt = softplusf_(ldf((const T*)a.zx, (size_t)(en.row0 + t) * a.ldz + a.dtoff + h) + a.dt_bias[h]);
+  const float dt = t < en.n ? softplusf_(raw + a.dt_bias[h]) : 0.0f;
   float c = -expf(a.A_log[h]) * dt;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -53,65 +60,99 @@ __device__ __forceinline__ void chunk_steps(const MambaChunkArgs& a, const Entry
   sc[t] = c;
 }
 
-// n rows of `width` numbers of src (row stride ld) -> dst [MC][ldd] times scale(t); zeros up to `pad` columns and in
-// rows n .. MC-1
-template <typename F>
+// n rows of `width` numbers of src (row stride ld) -> dst [MC][ldd]; zeros up to `pad` (a multiple of 16, at most
+// 256) columns and in rows n .. MC-1
 __device__ __forceinline__ void stage(const float* __restrict__ src, size_t ld, int n, int width, int pad, float* dst,
-                                      int ldd, int vec, F scale) {
-  if (vec) {   // four numbers per load
-    const int w4 = pad / 4;
-    for (int i = threadIdx.x; i < MC * w4; i += 256) {
-      const int t = i / w4, c = i % w4 * 4;
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if (t < n && c < width) v = *(const f32x4*)(src + (size_t)t * ld + c) * scale(t);
-      *(f32x4*)(dst + t * ldd + c) = v;
+                                      int ldd, int vec) {
+  if (vec) {   // 16 lanes take 64 columns of a row, four rows' loads in flight
+    const int t0 = threadIdx.x >> 4;
+#pragma unroll 1
+    for (int c = (threadIdx.x & 15) * 4; c < pad; c += 64) {
+      const float* p = src + min(c, width - 4);
+      f32x4 v[MC / 16];
+#pragma unroll
+      for (int u = 0; u < MC / 16; u++) v[u] = *(const f32x4*)(p + (size_t)min(t0 + u * 16, n - 1) * ld);
+#pragma unroll
+      for (int u = 0; u < MC / 16; u++)
+        *(f32x4*)(dst + (t0 + u * 16) * ldd + c) = c < width && t0 + u * 16 < n ? v[u] : f32x4{0.f, 0.f, 0.f, 0.f};
     }
     return;
   }
   for (int i = threadIdx.x; i < MC * pad; i += 256) {
     const int t = i / pad, c = i % pad;
-    dst[t * ldd + c] = (t < n && c < width) ? src[(size_t)t * ld + c] * scale(t) : 0.0f;
+    dst[t * ldd + c] = (t < n && c < width) ? src[(size_t)t * ld + c] : 0.0f;
   }
 }
+
+// Columns of 16 * NPT numbers as the lanes hold them: lane i16 has G = min(NPT, 4) neighbours of every 16 * G, so one
+// LDS read (or store) of G numbers serves G fragments.  The same freedom on k: a fragment of four products may hold
+// any four rows as long as both operands hold the same ones.
+template <int NPT>
+struct Cols {
+  static constexpr int G = NPT < 4 ? NPT : 4;
+  static __device__ __forceinline__ int at(int j, int i16) { return j / G * 16 * G + i16 * G + j % G; }
+};
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 template <typename T, int NPT>   // value size padded to NPT * 16
 __global__ void __launch_bounds__(256) mamba_local_k(MambaChunkArgs a) {
   extern __shared__ __align__(16) float smem[];
   __shared__ float sdt[MC], sc[MC];
+  typedef Cols<NPT> CP;
   const int c = blockIdx.x, h = blockIdx.y, N = a.N, P = a.P;
   const Entry en = load_entry(a.vent, c);
-  const int NP = (N + 15) & ~15, PP = NPT * 16, LDB = ld_cols(NP), LDX = ld_cols(PP);
+  const int NP = (N + 31) & ~31, PP = NPT * 16, LDB = ld_pairs(NP), LDX = PP;
   float* sB = smem;
   float* sX = smem + MC * LDB;
-  chunk_steps<T>(a, en, h, sdt, sc);
-  __syncthreads();
+  const float raw = chunk_dt<T>(a, en, h);
   const float* row = a.conv + (size_t)en.row0 * a.C;
-  const float end = sc[en.n - 1];
-  stage(row + a.H * P + (h / (a.H / a.G)) * N, a.C, en.n, N, NP, sB, LDB, a.vec,
-        [&](int t) { return sdt[t] * expf(end - sc[t]); });
-  stage(row + h * P, a.C, en.n, P, PP, sX, LDX, a.vec, [](int) { return 1.0f; });
-  if (threadIdx.x == 0) a.decay[(size_t)c * a.H + h] = expf(end);
+  stage(row + a.H * P + (h / (a.H / a.G)) * N, a.C, en.n, N, NP, sB, LDB, a.vec);
+  stage(row + h * P, a.C, en.n, P, PP, sX, LDX, a.vec);
+  chunk_steps(a, en, h, raw, sdt, sc);
+  if (threadIdx.x < 64) {   // within the first wavefront
+    const float end = __shfl(sc[threadIdx.x], en.n - 1, 64);
+    sdt[threadIdx.x] *= expf(end - sc[threadIdx.x]);
+    if (threadIdx.x == 0) a.decay[(size_t)c * a.H + h] = expf(end);
+  }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
   const int steps = (en.n + 3) / 4;
   float* out = a.cs + ((size_t)c * a.H + h) * N * P;
-  for (int nt = wave; nt * 16 < NP; nt += 4) {
-    f32x4 acc[NPT];
+  for (int nb = wave * 32; nb < NP; nb += 128) {   // rows nb + 2 i16 and the one after it
+    f32x4 acc[2][NPT];
 #pragma unroll
-    for (int j = 0; j < NPT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int j = 0; j < NPT; j++) acc[u][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
     for (int s = 0; s < steps; s++) {
-      const float b = sB[(4 * s + k4) * LDB + nt * 16 + i16];
+      const f32x2 b = *(const f32x2*)(sB + (4 * s + k4) * LDB + nb + 2 * i16) * sdt[4 * s + k4];
+      float x[NPT];
 #pragma unroll
-      for (int j = 0; j < NPT; j++)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b, sX[(4 * s + k4) * LDX + j * 16 + i16], acc[j], 0, 0, 0);
+      for (int j = 0; j < NPT; j++) x[j] = sX[(4 * s + k4) * LDX + CP::at(j, i16)];
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int j = 0; j < NPT; j++) acc[u][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u], x[j], acc[u][j], 0, 0, 0);
     }
 #pragma unroll
-    for (int j = 0; j < NPT; j++)
+    for (int u = 0; u < 2; u++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int n = nt * 16 + k4 * 4 + r, p = j * 16 + i16;
-        if (n < N && p < P) out[(size_t)n * P + p] = acc[j][r];
+        const int n = nb + 2 * (k4 * 4 + r) + u;
+        if (n >= N) continue;
+        float* o = out + (size_t)n * P;
+        if (CP::G == 4 && a.vec) {
+#pragma unroll
+          for (int j = 0; j < NPT; j += 4) {
+            const int p = CP::at(j, i16);
+            if (p < P) *(f32x4*)(o + p) = f32x4{acc[u][j][r], acc[u][j + 1][r], acc[u][(j + 2) % NPT][r], acc[u][(j + 3) % NPT][r]};
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < NPT; j++)
+            if (CP::at(j, i16) < P) o[CP::at(j, i16)] = acc[u][j][r];
+        }
       }
   }
 }
@@ -148,67 +189,88 @@ template <typename T, int NPT>
 __global__ void __launch_bounds__(256) mamba_out_k(MambaChunkArgs a) {
   extern __shared__ __align__(16) float smem[];
   __shared__ float sdt[MC], sc[MC];
+  typedef Cols<NPT> CP;
   const int c = blockIdx.x, h = blockIdx.y, N = a.N, P = a.P, inner = a.H * P;
   const Entry en = load_entry(a.vent, c);
   const int n = en.n;
-  const int NP = (N + 15) & ~15, PP = NPT * 16, LDC = ld_rows(NP), LDX = ld_cols(PP), LDW = MC + 4;
-  float* sC = smem;                             // later the weights of the second product
-  float* sB = smem + MC * max(LDC, LDW);        // later x
-  float* sX = sB;
-  float* sW = smem;                             // [MC][LDW]
+  const int NP = (N + 15) & ~15, PP = NPT * 16, LDB = ld_rows(NP), LDX = PP;
+  float* sB = smem;
+  float* sX = smem + MC * LDB;
   const float* row = a.conv + (size_t)en.row0 * a.C;
   const float* bc = row + inner + (h / (a.H / a.G)) * N;
-  auto one = [](int) { return 1.0f; };
-  chunk_steps<T>(a, en, h, sdt, sc);
-  stage(bc + a.G * N, a.C, n, N, NP, sC, LDC, a.vec, one);
-  stage(bc, a.C, n, N, NP, sB, LDC, a.vec, one);
+  const float raw = chunk_dt<T>(a, en, h);
+  stage(bc, a.C, n, N, NP, sB, LDB, a.vec);
+  stage(row + h * P, a.C, n, P, PP, sX, LDX, a.vec);
+  chunk_steps(a, en, h, raw, sdt, sc);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
   const int r0 = wave * 16;                     // this wavefront's 16 tokens
-  f32x4 w[MC / 16], acc[NPT];                   // C_t . B_s;  S^T C_t, then y
+  if (r0 >= n) return;
+  // w[j]: (B_s . C_t) with s = 16 j + 4 k4 + r down and t = r0 + i16 across, which is the layout that the product
+  // with x wants its left operand in;  acc: S^T C_t, then y, tokens r0 + 4 k4 + r down
+  f32x4 w[MC / 16], acc[NPT];
 #pragma unroll
   for (int j = 0; j < MC / 16; j++) w[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < NPT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (r0 < n) {
-    const float* S = a.cs + ((size_t)c * a.H + h) * N * P;
-#pragma unroll 4
-    for (int s = 0; s < NP / 4; s++) {
-      const float q = sC[(r0 + i16) * LDC + 4 * s + k4];        // zero beyond N
-      const float* Sr = S + (size_t)min(4 * s + k4, N - 1) * P;
-      float b[NPT];
+  const float* S = a.cs + ((size_t)c * a.H + h) * N * P;
+  const float* Ct = bc + a.G * N + (size_t)min(r0 + i16, n - 1) * a.C;
+  for (int q = 0; q < NP; q += 16) {
+    const int n0 = q + 4 * k4;                  // this lane's four state rows
+    f32x4 ct = {0.f, 0.f, 0.f, 0.f};            // zero beyond N
+    float st[4][NPT];
+    if (a.vec) {
+      if (n0 < N) ct = *(const f32x4*)(Ct + n0);
+    } else {
 #pragma unroll
-      for (int j = 0; j < NPT; j++) b[j] = Sr[min(j * 16 + i16, P - 1)];
-#pragma unroll
-      for (int j = 0; j < MC / 16; j++)
-        if (j <= wave)
-          w[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(q, sB[(j * 16 + i16) * LDC + 4 * s + k4], w[j], 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < NPT; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(q, b[j], acc[j], 0, 0, 0);
+      for (int i = 0; i < 4; i++)
+        if (n0 + i < N) ct[i] = Ct[n0 + i];
     }
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const float m = expf(sc[r0 + k4 * 4 + r]);
+    for (int i = 0; i < 4; i++) {
+      const float* Sr = S + (size_t)min(n0 + i, N - 1) * P;
+      if (CP::G == 4 && a.vec) {
 #pragma unroll
-      for (int j = 0; j < NPT; j++) acc[j][r] *= m;
+        for (int j = 0; j < NPT; j += 4) {
+          const f32x4 v = *(const f32x4*)(Sr + min(CP::at(j, i16), P - 4));
+#pragma unroll
+          for (int g = 0; g < 4; g++) st[i][(j + g) % NPT] = v[g];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NPT; j++) st[i][j] = Sr[min(CP::at(j, i16), P - 1)];
+      }
     }
+#pragma unroll
+    for (int j = 0; j < MC / 16; j++)
+      if (j <= wave) {
+        const f32x4 bs = *(const f32x4*)(sB + (j * 16 + i16) * LDB + n0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bs[i], ct[i], w[j], 0, 0, 0);
+      }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < NPT; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ct[i], st[i][j], acc[j], 0, 0, 0);
   }
-  __syncthreads();   // B and C have been read
-  stage(row + h * P, a.C, n, P, PP, sX, LDX, a.vec, one);
 #pragma unroll
-  for (int j = 0; j < MC / 16; j++)
+  for (int r = 0; r < 4; r++) {
+    const float m = expf(sc[r0 + k4 * 4 + r]);
+#pragma unroll
+    for (int j = 0; j < NPT; j++) acc[j][r] *= m;
+  }
+  const float ce = sc[r0 + i16];
+#pragma unroll
+  for (int j = 0; j < MC / 16; j++) {
+    if (j > wave) continue;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int t = r0 + k4 * 4 + r, s = j * 16 + i16;
-      sW[t * LDW + s] = s <= t ? w[j][r] * expf(sc[t] - sc[s]) * sdt[s] : 0.0f;
-    }
-  __syncthreads();
-  if (r0 >= n) return;
-  for (int s = 0; s < (wave + 1) * 4; s++) {
-    const float q = sW[(r0 + i16) * LDW + 4 * s + k4];
+      const int s = j * 16 + k4 * 4 + r;
+      const float v = s <= r0 + i16 ? w[j][r] * expf(ce - sc[s]) * sdt[s] : 0.0f;
 #pragma unroll
-    for (int j = 0; j < NPT; j++)
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(q, sX[(4 * s + k4) * LDX + j * 16 + i16], acc[j], 0, 0, 0);
+      for (int k = 0; k < NPT; k++)
+        acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, sX[s * LDX + CP::at(k, i16)], acc[k], 0, 0, 0);
+    }
   }
   const float Dh = a.Dp[h];
 #pragma unroll
@@ -216,21 +278,23 @@ __global__ void __launch_bounds__(256) mamba_out_k(MambaChunkArgs a) {
     const int t = r0 + k4 * 4 + r;
     if (t >= n) continue;
     const size_t at = (size_t)(en.row0 + t);
+    const T* zr = (const T*)a.zx + at * a.ldz + h * P;
+    float* yr = a.y + at * inner + h * P;
 #pragma unroll
     for (int j = 0; j < NPT; j++) {
-      const int p = j * 16 + i16;
-      if (p >= P) continue;
-      const float z = ldf((const T*)a.zx, at * a.ldz + h * P + p);
-      a.y[at * inner + h * P + p] = (acc[j][r] + Dh * sX[t * LDX + p]) * (z * sigmoidf_(z));
+      const int p = CP::at(j, i16);
+      if (p < P) {
+        const float z = ldf(zr, p);
+        yr[p] = (acc[j][r] + Dh * sX[t * LDX + p]) * (z * sigmoidf_(z));
+      }
     }
   }
 }
 
 template <typename T, int NPT>
 static int launch_chunks(const MambaChunkArgs& a, int E, hipStream_t st) {
-  const int NP = (a.N + 15) & ~15, PP = NPT * 16, lc = ld_rows(NP), lx = ld_cols(PP);
-  const size_t shm1 = (size_t)MC * (ld_cols(NP) + lx) * 4;
-  const size_t shm2 = (size_t)MC * ((lc > MC + 4 ? lc : MC + 4) + (lc > lx ? lc : lx)) * 4;
+  const size_t shm1 = (size_t)MC * (ld_pairs((a.N + 31) & ~31) + NPT * 16) * 4;
+  const size_t shm2 = (size_t)MC * (ld_rows((a.N + 15) & ~15) + NPT * 16) * 4;
   static const hipError_t attr = [] {
     const hipError_t e = hipFuncSetAttribute((const void*)mamba_local_k<T, NPT>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);

@@ -168,7 +168,7 @@ def test_latent_attn(dt, H, rank, win):
 
 
 @pytest.mark.parametrize("lens,starts", [([130, 64, 1], [0, 7, 3]), ([65], [0]), ([33, 200], [5, 0])])
-@pytest.mark.parametrize("H,P,N,G", [(4, 64, 128, 2), (2, 30, 17, 1), (1, 256, 256, 1)])
+@pytest.mark.parametrize("H,P,N,G", [(4, 64, 128, 2), (2, 30, 17, 1), (1, 256, 256, 1), (3, 36, 20, 1), (2, 100, 44, 1)])
 @pytest.mark.parametrize("steep", [False, True])
 def test_mamba_long_portions(lens, starts, H, P, N, G, steep):
     """Chunks of 64 on the matrix instruction: remainders, single-chunk portions beside long ones, and
