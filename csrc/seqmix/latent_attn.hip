@@ -5,6 +5,7 @@
 // Causal sliding window: position i sees j with 0 <= i - j < win.  The softmax denominator
 // holds one more term exp(sink_h) with no key and no value: the running maximum starts at
 // sink_h and the running sum at 1.
+// For shapes that neither the matrix-core kernel nor, for float32 models, attn_f32.hip takes.
 // One block per (query row, group of heads); keys stream through LDS in tiles with an online
 // softmax in fp32.  The group size and the key tile are chosen so that a block's LDS fits.
 #include "common.h"

@@ -1,6 +1,6 @@
 // Grouped-query attention over a paged key/value pool: the pass that prepares its inputs and
-// the attention kernel in fp32 arithmetic (float32 models, shapes the matrix-core kernel does
-// not take).
+// the attention kernel in fp32 arithmetic (shapes that neither the matrix-core kernel nor, for
+// float32 models, attn_f32.hip takes).
 //
 // qk_norm_rope_store_k: one projection buffer holds q (H heads x D) | k (G x D) | v (G x V) of a
 // row.  q and k are RMS-normalised and weighted -- with one mean square per row (heads not
