@@ -260,3 +260,14 @@ def test_row_passes_by_width(dt, n, off):
     # sums of up to 4100 fp32 squares in another order, then one rounding; the two wide inputs double the scale
     for p, q in zip(*res):
         torch.testing.assert_close(q, p, **(_tol(dt) if dt == torch.bfloat16 else dict(rtol=1e-5, atol=1e-5)))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("F,off", [(4, 0), (1020, 0), (1023, 0), (1028, 4), (1028, 1), (1, 0)])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+def test_glu_act_by_width(dt, F, off, act):
+    """Four channels per thread at the edges of a block, and the widths and rows that take one."""
+    gu = (torch.randn(3, 2 * F + 8, generator=torch.Generator().manual_seed(11)) * 2).to(dt)
+    res = [sm.glu_act(gu.to(d)[:, off:off + 2 * F], torch.zeros(3, F + 4, dtype=dt, device=d)[:, :F], act).cpu()
+           for d in ("cpu", DEV)]
+    torch.testing.assert_close(res[1], res[0], **_tol(dt))
