@@ -86,9 +86,12 @@ window_attn_tile_k(WindowArgs a) {
     return pages[t / page] * SB + (t % page) / a.P;
   };
 
-  // Copies of a tile: thread t takes 16-byte pieces t, t + 256, .. of its rows.  Channels beyond D and V
-  // (which meet zero queries, or columns that are not written) are some channels of the same row.
+  // Copies of a tile: thread t takes 16-byte pieces t, t + 256, .. of its rows, as long as there are any (32 rows of
+  // four pieces are two wavefronts' work).  Channels beyond D and V (which meet zero queries, or columns that
+  // are not written) are some channels of the same row.
   constexpr int CK = (KT * PK + 255) / 256, CV = (KT * PV + 255) / 256;
+  static_assert(KT * PK % 64 == 0 && KT * PV % 64 == 0, "a copy is a whole wavefront's");
+  auto mine = [&](int c, int pieces) { return pieces % 256 == 0 || c * 256 + wave * 64 < pieces; };
   int ok_[CK], ov_[CV];                                   // byte offsets within a page's rows
 #pragma unroll
   for (int i = 0; i < CK; i++) {
@@ -107,12 +110,14 @@ window_attn_tile_k(WindowArgs a) {
     if (BLK && i < heads) {
 #pragma unroll
       for (int c = 0; c < CK; c++) {
+        if (!mine(c, KT * PK)) continue;
         const int r = (c * 256 + tid) / PK;
         copy_lds16((const char*)a.blk + ((size_t)srow[st][r] - r) * ldpool * 2 + ok_[c],
                    base + c * 4096);
       }
 #pragma unroll
       for (int c = 0; c < CV; c++) {
+        if (!mine(c, KT * PV)) continue;
         const int r = (c * 256 + tid) / PV;
         copy_lds16((const char*)a.blk + ((size_t)srow[st][r] - r) * ldpool * 2 + ov_[c],
                    vbase + c * 4096);
@@ -126,11 +131,13 @@ window_attn_tile_k(WindowArgs a) {
     if (lo > 0 || hi < KT - 1) {
 #pragma unroll
       for (int c = 0; c < CK; c++) {
+        if (!mine(c, KT * PK)) continue;
         const int r = (c * 256 + tid) / PK;
         copy_lds16_at(src, ok_[c] + (min(max(r, lo), hi) - r) * ldpool * 2, base + c * 4096);
       }
 #pragma unroll
       for (int c = 0; c < CV; c++) {
+        if (!mine(c, KT * PV)) continue;
         const int r = (c * 256 + tid) / PV;
         copy_lds16_at(src, ov_[c] + (min(max(r, lo), hi) - r) * ldpool * 2,
                       vbase + c * 4096);
@@ -138,9 +145,11 @@ window_attn_tile_k(WindowArgs a) {
       return;
     }
 #pragma unroll
-    for (int c = 0; c < CK; c++) copy_lds16_at(src, ok_[c], base + c * 4096);
+    for (int c = 0; c < CK; c++)
+      if (mine(c, KT * PK)) copy_lds16_at(src, ok_[c], base + c * 4096);
 #pragma unroll
-    for (int c = 0; c < CV; c++) copy_lds16_at(src, ov_[c], vbase + c * 4096);
+    for (int c = 0; c < CV; c++)
+      if (mine(c, KT * PV)) copy_lds16_at(src, ov_[c], vbase + c * 4096);
   };
   auto token_page = [&](int i) { return BLK && i < heads ? 0 : pages[place(i) / page]; };
   auto token_row = [&](int i, int pg) {                   // the pool row of a tile's first token

@@ -80,6 +80,14 @@ def test_window_attention_tiles(step, H, G, D, V, form, dt):
         assert bool((out[:, H * V:] == 7.0).all())
 
 
+@pytest.mark.parametrize("step", ["portions", "prompts"])
+@pytest.mark.parametrize("H,G,D,V", [(4, 2, 32, 256), (4, 2, 256, 32), (4, 2, 128, 24), (2, 1, 16, 136), (8, 2, 72, 32)])
+@pytest.mark.parametrize("form", ["window", "sink", "blocks", "kept", "maps"])
+def test_window_attention_tiles_of_one_narrow_side(step, H, G, D, V, form):
+    """Tiles of 32 keys whose key or value rows are so short that two wavefronts copy them."""
+    test_window_attention_tiles(step, H, G, D, V, form, torch.bfloat16)
+
+
 def test_group_size():
     one = [(i, 1, 5, i) for i in range(8)]
     assert sm.attn_unit_rows(4, one) == 4                     # decoded tokens
