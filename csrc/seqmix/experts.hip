@@ -358,10 +358,10 @@ expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
   const int kb = wave * kq, ke = min(K, kb + kq);
   // rows that do not exist (a slot or column beyond the last) are others, their products are dropped; past
   // the wavefront's share of K both operands are zero
-  const T* xa = x + (size_t)(max(slot, 0) / x_div) * ldx + quad * EP;
+  const T* xa = x + (size_t)(max(slot, 0) / x_div) * ldx;
   const T* wb[4];
 #pragma unroll
-  for (int t = 0; t < 4; t++) wb[t] = w + ((size_t)e * N + min(n0 + t * 16 + n16, N - 1)) * K + quad * EP;
+  for (int t = 0; t < 4; t++) wb[t] = w + ((size_t)e * N + min(n0 + t * 16 + n16, N - 1)) * K;
   f32x4 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -371,7 +371,7 @@ expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
   uint4 av[DEPTH], bv[DEPTH][4];
   auto load = [&](int k, uint4& a, uint4 (&b)[4]) {
     const bool in = k + quad * EP < ke;            // K is a multiple of EP
-    const int at = in ? k : 0;
+    const int at = in ? k + quad * EP : 0;         // else the row's start, which is there whatever K is
     a = *(const uint4*)(xa + at);
 #pragma unroll
     for (int t = 0; t < 4; t++) b[t] = *(const uint4*)(wb[t] + at);

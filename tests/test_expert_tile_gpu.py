@@ -68,3 +68,25 @@ def test_expert_products(dt, counts, N, K, act):
     tol = dict(rtol=1e-2, atol=2e-2) if dt == torch.bfloat16 else dict(rtol=2e-5, atol=1e-5)
     torch.testing.assert_close(out[:, :F].cpu().float(), want.float(), **tol)
     assert bool((out[:, F:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts", [[3, 0, 1], [130, 70]])    # few slots / tiles
+@pytest.mark.parametrize("N,K", [(48, 8), (64, 16), (20, 24), (70, 4), (33, 12)])
+def test_expert_products_of_short_rows(dt, counts, N, K):
+    """Rows shorter than one step of the kernels, the last ones at the end of their tensors."""
+    if dt == torch.bfloat16 and K % 8:
+        K *= 2
+    g = torch.Generator().manual_seed(5)
+    E, S = len(counts), sum(counts)
+    rows, at = torch.zeros(E, S, dtype=torch.int32), 0
+    for e, n in enumerate(counts):
+        rows[e, :n] = torch.arange(at, at + n)
+        at += n
+    cnt = torch.tensor(counts, dtype=torch.int32)
+    x, w = torch.randn(S, K, generator=g).to(dt), (torch.randn(E, N, K, generator=g) / K ** 0.5).to(dt)
+    want = sm.expert_gemm(x, 1, w, cnt, rows, torch.zeros(S, N, dtype=dt), S)
+    out = sm.expert_gemm(x.to(DEV), 1, w.to(DEV), cnt.to(DEV), rows.to(DEV), torch.zeros(S, N, dtype=dt, device=DEV), S)
+    # up to 24 products of about 1 / sqrt(K) in fp32, one rounding to bf16 of values up to about 5
+    tol = dict(rtol=1e-2, atol=2e-2) if dt == torch.bfloat16 else dict(rtol=2e-5, atol=1e-5)
+    torch.testing.assert_close(out.cpu().float(), want.float(), **tol)
