@@ -351,7 +351,7 @@ expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
   int e, m0, nt;
   if (!find_tile(cnt, E, 16, TMP, e, m0, nt)) return;
   const int c = cnt[e], n0 = nt * 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, quad = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6), n16 = lane & 15, quad = lane >> 4;
   const int mi = m0 + n16;
   const int slot = mi < c ? rows[(size_t)e * ldr + mi] : -1;
   const int kq = ((K + 4 * KS - 1) / (4 * KS)) * KS;   // K per wavefront, a multiple of the step
@@ -386,10 +386,11 @@ expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
   for (int k0 = kb; k0 < ke; k0 += DEPTH * KS) {
 #pragma unroll
     for (int d = 0; d < DEPTH; d++) {
+      if (k0 + d * KS < ke) {   // what a place held before must not meet zeros: it need not be finite
 #pragma unroll
-      for (int t = 0; t < 4; t++) acc[t] = mfma_piece<T>(av[d], bv[d][t], acc[t]);
+        for (int t = 0; t < 4; t++) acc[t] = mfma_piece<T>(av[d], bv[d][t], acc[t]);
+      }
       if (k0 + (DEPTH + d) * KS < ke) load(k0 + (DEPTH + d) * KS, av[d], bv[d]);
-      else av[d] = zero;
     }
   }
   if (wave > 0) {

@@ -90,3 +90,20 @@ def test_expert_products_of_short_rows(dt, counts, N, K):
     # up to 24 products of about 1 / sqrt(K) in fp32, one rounding to bf16 of values up to about 5
     tol = dict(rtol=1e-2, atol=2e-2) if dt == torch.bfloat16 else dict(rtol=2e-5, atol=1e-5)
     torch.testing.assert_close(out.cpu().float(), want.float(), **tol)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("K", [640, 200, 136])    # steps of a wavefront's share off the depth of its loads
+def test_small_expert_products_with_infinite_weights(dt, K):
+    """An infinite weight gives an infinite result, and only in its column."""
+    g = torch.Generator().manual_seed(6)
+    N, S = 70, 5
+    x, w = torch.randn(S, K, generator=g).abs().to(dt), torch.randn(1, N, K, generator=g).to(dt)
+    for k in (40, K - 3):
+        w[0, k % N, k] = float("inf")
+    cnt, rows = torch.tensor([S], dtype=torch.int32), torch.arange(S, dtype=torch.int32)[None]
+    want = x.double() @ w[0].double().T
+    out = sm.expert_gemm(x.to(DEV), 1, w.to(DEV), cnt.to(DEV), rows.to(DEV), torch.zeros(S, N, dtype=dt, device=DEV), S).cpu()
+    fin = want.isfinite()
+    assert torch.equal(out[~fin].double(), want[~fin]) and (~fin).sum() == 2 * S
+    torch.testing.assert_close(out[fin].double(), want[fin], rtol=1e-2 if dt == torch.bfloat16 else 1e-5, atol=1e-4)
