@@ -121,11 +121,12 @@ attn_f32_k(AttnF32Args a) {
     for (int e = 0; e < 4; e++)
       vrow[e] = (const float*)__shfl((unsigned long long)krow, quad * 4 + e, 64) + voff;
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
-    const float* kp = krow + koff + quad * 4;
+    const float* kp = krow + koff;
     const float* qp = smem + n16 * LDQ + quad * 4;
 #pragma unroll 8
     for (int c = 0; c < DP; c += 16) {
-      f32x4 kv = *(const f32x4*)(kp + (c + quad * 4 < D ? c : 0));
+      // beyond D: the key's start (D may be less than the 16 numbers of a step), which meets zeros
+      const f32x4 kv = *(const f32x4*)(kp + (c + quad * 4 < D ? c + quad * 4 : 0));
       const f32x4 qv = *(const f32x4*)(qp + c);   // zero beyond D
       s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[0], qv[0], s0, 0, 0, 0);
       s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[1], qv[1], s1, 0, 0, 0);

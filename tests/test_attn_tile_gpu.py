@@ -120,3 +120,30 @@ def test_latent_attention_tiles(step, H, rank, win, sunk, dt):
         sm.latent_attn(q2, *(t.to(DEV) for t in (cache, bt, row_ent, pos)), sink.to(DEV) if sunk else None, scale, win,
                        out, PAGE, units=units, unit_rows=rows, max_keys=max_keys)
         _close(out, want)
+
+
+@pytest.mark.parametrize("step", sorted(STEPS))
+@pytest.mark.parametrize("size", [4, 8, 12, 20])
+def test_fp32_keys_shorter_than_a_step(step, size):
+    """Nothing beside a key's own numbers is read with it: here all of that is not a number."""
+    ent, row_ent, pos, bt, R, g = _step(step, 9)
+    H, units = 3, None
+    q = torch.randn(R, H * size, generator=g)
+    top = (int(bt.max()) + 1) * PAGE
+    full = torch.full((top, size), float("nan"))
+    for r in range(R):      # only the rows that belong to the sequences
+        for j in range(int(pos[r]) + 1):
+            full[int(bt[int(row_ent[r]), j // PAGE]) * PAGE + j % PAGE] = 0.0
+    keep = full[:, 0] == 0.0
+    full[keep] = torch.randn(int(keep.sum()), size, generator=g)
+    units = sm.make_units(ent, sm.latent_rows_per_wave(H)).to(DEV)
+    qa = q.view(R, H, size).transpose(0, 1).contiguous()
+    want = sm.latent_attn(qa, full, bt, row_ent, pos, None, 0.5, 40, torch.empty(H, R, size), PAGE)
+    out = sm.latent_attn(*(t.to(DEV) for t in (qa, full, bt, row_ent, pos)), None, 0.5, 40,
+                         torch.empty(H, R, size, device=DEV), PAGE, units=units)
+    _close(out, want)
+    pool = torch.cat([full, full[:, :4]], 1).contiguous()    # key of `size`, value of four numbers
+    want = sm.window_attn(q, pool, bt, row_ent, pos, None, 0.5, 40, torch.empty(R, H * 4), PAGE, H, 1, size, 4)
+    out = sm.window_attn(*(t.to(DEV) for t in (q, pool, bt, row_ent, pos)), None, 0.5, 40,
+                         torch.empty(R, H * 4, device=DEV), PAGE, H, 1, size, 4, units=units)
+    _close(out, want)
