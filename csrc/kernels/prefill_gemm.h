@@ -471,9 +471,12 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
       for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int s2 = 0; s2 < splitk; ++s2) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FM; ++i) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] += base[((size_t)s2 * FM * FN + i * FN + j) * NT + tid];
+        // 256 x 256: all rows' loads in flight beside 128 accumulators would not fit the registers
+        if constexpr (BM * BN >= 256 * 256) __builtin_amdgcn_sched_barrier(0);
+      }
     }
     if constexpr (NORM) {
       if (tid < BM) {

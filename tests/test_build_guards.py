@@ -38,3 +38,16 @@ def test_wide_gemm_compiles_without_scratch(tmp_path):
     assert r.returncode == 0, r.stdout[-3000:]
     assert "Function Name: _ZN4wide16wide_gemm_kernel" in r.stdout
     B.check_no_scratch(src, r.stdout)
+
+
+@pytest.mark.parametrize("lib", ["seqmix", "kernels", "experimental"])
+def test_no_library_is_compiled_with_packed_fp32(lib, tmp_path, monkeypatch):
+    cmds = []
+    monkeypatch.setattr(B, "_run", lambda cmd, cwd=None: cmds.append(cmd) or open(cmd[-1], "w").close() or "")
+    for name in ("LIBDIR", "BUILDDIR"):
+        monkeypatch.setattr(B, name, str(tmp_path))
+    for name in ("KERNEL_LIB", "SEQMIX_LIB", "EXPERIMENTAL_LIB"):
+        monkeypatch.setattr(B, name, str(tmp_path / name))
+    B.build_seqmix(force=True) if lib == "seqmix" else B.build_kernels(force=True, experimental=lib == "experimental")
+    compiles = [" ".join(c) for c in cmds if "-c" in c]
+    assert compiles and all("-Xclang -target-feature -Xclang -packed-fp32-ops" in c for c in compiles)
