@@ -37,6 +37,8 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+#define LOWEST_SCORE -3.402823466e+38f
+
 // The choice of one row by one wavefront: ss holds its E logits (sigmoids for score 0) and becomes its scores.
 // place(k, e): the row's k-th expert is e (called by lane 0).
 template <typename P>
@@ -58,7 +60,9 @@ __device__ __forceinline__ void choose_experts(int r, int lane, float* ss, float
     sum = wave_sum(sum);
     for (int e = lane; e < E; e += 64) ss[e] = ss[e] / sum;
   }
-  for (int e = lane; e < E; e += 64) sc[e] = corr ? ss[e] + corr[e] : ss[e];
+  // choice scores are above -inf, which marks what cannot be chosen (any more): a score that is not a number or
+  // -inf counts as the lowest, so that every pick is an expert
+  for (int e = lane; e < E; e += 64) sc[e] = fmaxf(corr ? ss[e] + corr[e] : ss[e], LOWEST_SCORE);
   wave_sync();
   const int per = E / groups;
   if (keep < groups) {
@@ -69,7 +73,7 @@ __device__ __forceinline__ void choose_experts(int r, int lane, float* ss, float
         if (v > b1) { b2 = b1; b1 = v; }
         else if (v > b2) b2 = v;
       }
-      sgs[g] = b1 + ((per > 1 && gscore == 0) ? b2 : 0.0f);
+      sgs[g] = fmaxf(b1 + ((per > 1 && gscore == 0) ? b2 : 0.0f), LOWEST_SCORE);
     }
     wave_sync();
     // keep the best groups: pick `keep` times, then strike out the experts of the others

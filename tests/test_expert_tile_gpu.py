@@ -107,3 +107,30 @@ def test_small_expert_products_with_infinite_weights(dt, K):
     fin = want.isfinite()
     assert torch.equal(out[~fin].double(), want[~fin]) and (~fin).sum() == 2 * S
     torch.testing.assert_close(out[fin].double(), want[fin], rtol=1e-2 if dt == torch.bfloat16 else 1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("R", [3, 300])      # a row per workgroup / sixteen
+@pytest.mark.parametrize("score,groups,keep", [("sigmoid", 1, 1), ("softmax", 4, 2), ("top_softmax", 4, 1)])
+def test_routing_of_rows_that_are_not_finite(R, score, groups, keep):
+    """Every slot goes to an expert that exists and is in that expert's list, whatever the scores are; the other
+    rows' choices are as they were."""
+    g = torch.Generator().manual_seed(3)
+    W, E, top = 40, 12, 3
+    h, wr = torch.randn(R, W, generator=g), torch.randn(E, W, generator=g)
+    corr = torch.randn(E, generator=g)
+    bad = h.clone()
+    bad[1], bad[2, 7], bad[R - 1, 3] = float("nan"), float("inf"), -3e38
+    low = torch.full((E,), float("-inf"))     # no expert wanted
+    res = []
+    for x, c in ((h, corr), (bad, corr), (h, low)):
+        ids, wts = torch.full((R, top), -1, dtype=torch.int32, device=DEV), torch.empty(R, top, device=DEV)
+        cnt, rows = torch.empty(E, dtype=torch.int32, device=DEV), torch.full((E, R * top), -1, dtype=torch.int32, device=DEV)
+        sm.group_route(x.to(DEV), wr.to(DEV), top, groups, keep, ids, wts, cnt, rows, score=score, corr=c.to(DEV))
+        ids, cnt, rows = ids.cpu(), cnt.cpu(), rows.cpu()
+        assert int(ids.min()) >= 0 and int(ids.max()) < E
+        assert all(len(set(r)) == top for r in ids.tolist())
+        for e in range(E):
+            assert sorted(rows[e, :int(cnt[e])].tolist()) == (ids.reshape(-1) == e).nonzero()[:, 0].tolist()
+        res.append(ids)
+    same = [r for r in range(R) if r not in (1, 2, R - 1)]
+    assert torch.equal(res[0][same], res[1][same])
