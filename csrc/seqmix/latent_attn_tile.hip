@@ -51,7 +51,6 @@ latent_attn_tile_k(LatentArgs a) {
     i_lo += blockIdx.y * per;
     i_hi = min(i_hi, i_lo + per - 1);
   }
-  const bool first = blockIdx.y == 0;   // the sink is counted by the first run only
 
   // Copies of a tile: thread t takes 16-byte pieces t, t + 256, ..  Numbers beyond the rank (which meet zero
   // queries, or columns that are not written) are some numbers of the same row; a tile that reaches over
@@ -83,9 +82,8 @@ latent_attn_tile_k(LatentArgs a) {
     qf[kk] = __builtin_bit_cast(bf16x8, v);
   }
   const float sl2 = a.scale * LOG2E_;
-  const bool sunk = first && a.sink != nullptr;   // no sink: an ordinary softmax
-  float m_run = pvalid ? (sunk ? a.sink[ph] * LOG2E_ : NO_KEY_YET) : 0.0f;   // in powers of two
-  float l_part = (pvalid && quad == 0 && sunk) ? 1.0f : 0.0f;
+  float m_run = pvalid ? NO_KEY_YET : 0.0f;   // in powers of two
+  float l_part = 0.0f;
   f32x4 acc[4][CT];   // pairs 16 m + quad * 4 + e, columns (wave * CT + t) * 16 + n16
 #pragma unroll
   for (int m = 0; m < 4; m++)
@@ -207,25 +205,38 @@ latent_attn_tile_k(LatentArgs a) {
   }
   float l = l_part + __shfl_xor(l_part, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  m_run *= 1.0f / LOG2E_;   // natural from here on
+  // the sink joins the finished sums (see window_attn_tile.hip)
+  float sf = 1.0f;          // rescales the sums of this lane's pair
+  int pair = threadIdx.x & 15;
+  again(pair);              // (its row and head are not kept in registers until here)
+  if (a.sink && blockIdx.y == 0 && (wave * 16 + pair) / a.HS < nr && h0 + pair % a.HS < a.H) {
+    const float sink = a.sink[h0 + pair % a.HS], m = fmaxf(m_run, sink);
+    sf = expf(m_run - m);
+    l = l * sf + expf(sink - m);
+    m_run = m;
+  }
+  __syncthreads();   // the last tile's factors have been read
+  if (quad == 0) sAl[wave * 16 + n16] = a.splits > 1 ? sf : l != 0.0f ? sf / l : 0.0f;
+  __syncthreads();
   if (a.splits > 1) {
     // partial record of this run: [64 pairs][RP + 2] = unnormalised sums, running max (natural), sum
     float* rec = a.part + (((size_t)unit * hg + at % hg) * a.splits + blockIdx.y) * 64 * (RP + 2);
     if (quad == 0) {
-      rec[(wave * 16 + n16) * (RP + 2) + RP] = m_run * (1.0f / LOG2E_);
+      rec[(wave * 16 + n16) * (RP + 2) + RP] = m_run;
       rec[(wave * 16 + n16) * (RP + 2) + RP + 1] = l;
     }
 #pragma unroll
-    for (int m = 0; m < 4; m++)
+    for (int m = 0; m < 4; m++) {
+      const f32x4 f = *(const f32x4*)(sAl + m * 16 + quad * 4);
 #pragma unroll
       for (int e = 0; e < 4; e++)
 #pragma unroll
         for (int t = 0; t < CT; t++)
-          rec[(m * 16 + quad * 4 + e) * (RP + 2) + (wave * CT + t) * 16 + n16] = acc[m][t][e];
+          rec[(m * 16 + quad * 4 + e) * (RP + 2) + (wave * CT + t) * 16 + n16] = acc[m][t][e] * f[e];
+    }
     return;
   }
-  __syncthreads();   // the last tile's factors have been read
-  if (quad == 0) sAl[wave * 16 + n16] = l > 0.0f ? 1.0f / l : 0.0f;
-  __syncthreads();
 #pragma unroll
   for (int m = 0; m < 4; m++) {
     const f32x4 inv = *(const f32x4*)(sAl + m * 16 + quad * 4);

@@ -78,7 +78,6 @@ window_attn_tile_k(WindowArgs a) {
     i_lo = blockIdx.y * per;
     i_hi = min(i_hi, i_lo + per - 1);
   }
-  const bool first = blockIdx.y == 0;                     // the sink is counted by the first run only
   // first place of a tile: block or token number
   auto place = [&](int i) { return ((BLK || KEPT) && i < heads ? i : i - heads + t_lo) * KT; };
   auto block_row = [&](int j) {                           // of the pool of blocks; past the last: the last
@@ -172,13 +171,12 @@ window_attn_tile_k(WindowArgs a) {
   const float sl2 = a.scale * LOG2E_;
   const float cap2 = a.cap * LOG2E_, capx = a.cap > 0.0f ? 2.0f * sl2 / a.cap : 0.0f;
   const float pr1 = (pvalid && a.r1) ? a.r1[ph] : 0.0f, pr2 = (pvalid && a.r1) ? a.r2[ph] : 0.0f;
-  const bool sunk = first && a.sink != nullptr;   // no sink: an ordinary softmax
   float m_run[MAPS], l_part[MAPS];                // maxima in powers of two
   f32x4 acc[MAPS][NT];
 #pragma unroll
   for (int u = 0; u < MAPS; u++) {
-    m_run[u] = pvalid ? (sunk ? a.sink[ph] * LOG2E_ : NO_KEY_YET) : 0.0f;
-    l_part[u] = (pvalid && quad == 0 && sunk) ? 1.0f : 0.0f;
+    m_run[u] = pvalid ? NO_KEY_YET : 0.0f;
+    l_part[u] = 0.0f;
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -342,6 +340,18 @@ window_attn_tile_k(WindowArgs a) {
   for (int u = 0; u < MAPS; u++) {
     l[u] = l_part[u] + __shfl_xor(l_part[u], 16, 64);
     l[u] += __shfl_xor(l[u], 32, 64);
+    m_run[u] *= 1.0f / LOG2E_;   // natural from here on
+  }
+  // The sink joins the finished sums (of the first run of a window that is cut).  Scores are taken less the running
+  // maximum before it moves: one that began with a sink far below them would swallow their low bits.
+  float sf = 1.0f;               // rescales the sums of this lane's pair
+  int pair = lane & 15;
+  again(pair);                   // (its row and head are not kept in registers until here)
+  if (MAPS == 1 && a.sink && blockIdx.y == 0 && (wave * 16 + pair) / a.HS < nr && hb0 + pair % a.HS < HG) {
+    const float sink = a.sink[g * HG + hb0 + pair % a.HS], m = fmaxf(m_run[0], sink);
+    sf = expf(m_run[0] - m);
+    l[0] = l[0] * sf + expf(sink - m);
+    m_run[0] = m;
   }
   if (a.splits > 1) {
     // partial record of this run: [map][64 pairs][VP + 2] = unnormalised sums, running max (natural), sum
@@ -350,13 +360,15 @@ window_attn_tile_k(WindowArgs a) {
 #pragma unroll
     for (int u = 0; u < MAPS; u++, rec += 64 * (VP + 2)) {
       if (quad == 0) {
-        rec[n16 * (VP + 2) + VP] = m_run[u] * (1.0f / LOG2E_);
+        rec[n16 * (VP + 2) + VP] = m_run[u];
         rec[n16 * (VP + 2) + VP + 1] = l[u];
       }
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < 4; i++) {
+        const float f = MAPS == 1 ? __shfl(sf, quad * 4 + i, 64) : 1.0f;
 #pragma unroll
-        for (int t = 0; t < NT; t++) rec[(quad * 4 + i) * (VP + 2) + t * 16 + n16] = acc[u][t][i];
+        for (int t = 0; t < NT; t++) rec[(quad * 4 + i) * (VP + 2) + t * 16 + n16] = acc[u][t][i] * f;
+      }
     }
     return;
   }
@@ -364,7 +376,7 @@ window_attn_tile_k(WindowArgs a) {
   for (int i = 0; i < 4; i++) {
     const int m = wave * 16 + quad * 4 + i, mr = m / a.HS, ms = hb0 + m % a.HS;
     const float l0 = __shfl(l[0], quad * 4 + i, 64);
-    const float i0 = l0 > 0.0f ? 1.0f / l0 : 0.0f;
+    const float i0 = l0 != 0.0f ? (MAPS == 1 ? __shfl(sf, quad * 4 + i, 64) : 1.0f) / l0 : 0.0f;
     if constexpr (MAPS == 2) {
       const float l1 = __shfl(l[1], quad * 4 + i, 64);
       const float i1 = l1 > 0.0f ? a.lam / l1 : 0.0f;
