@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(256)
 attn_f32_k(AttnF32Args a) {
   constexpr int VP = NB * 64;
   extern __shared__ __align__(16) float smem[];   // queries [16][LDQ], at the end sums [16][VP]
-  __shared__ float sM[4][16], sL[4][16];
+  __shared__ float sM[5][16], sL[5][16];          // per wavefront, then all together
   const int tid = threadIdx.x, lane = tid & 63, n16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int HG = a.H / a.G, hblocks = (HG + a.HS - 1) / a.HS;
@@ -102,9 +102,7 @@ attn_f32_k(AttnF32Args a) {
       v = *(const f32x4*)(a.q + (g * HG + ms) * a.sqh + (r0 + mr) * a.sqr + map * a.sqm + c);
     *(f32x4*)(smem + m * LDQ + c) = v;
   }
-  const bool sunk = a.sink != nullptr && blockIdx.z == 0 && wave == 0;   // counted once
-  float m_run = pvalid ? (sunk ? a.sink[ph] : -1e30f) : 0.0f;
-  float l_part = (pvalid && quad == 0 && sunk) ? 1.0f : 0.0f;
+  float m_run = pvalid ? -1e30f : 0.0f, l_part = 0.0f;
   const float pr1 = (pvalid && a.r1) ? a.r1[ph] : 0.0f, pr2 = (pvalid && a.r1) ? a.r2[ph] : 0.0f;
   f32x4 acc[NB * 4];   // pairs quad * 4 + e, column (t / 4) * 64 + n16 * 4 + t % 4
 #pragma unroll
@@ -181,7 +179,7 @@ attn_f32_k(AttnF32Args a) {
       }
     krow = nxt;
   }
-  // the wavefronts' sums under their common maximum, one after the other
+  // the wavefronts' sums under their common maximum, one after the other; the sink (of the first run) is a fifth
   float l = l_part + __shfl_xor(l_part, 16, 64);
   l += __shfl_xor(l, 32, 64);
   if (quad == 0) {
@@ -189,12 +187,19 @@ attn_f32_k(AttnF32Args a) {
     sL[wave][n16] = l;
   }
   __syncthreads();   // (and every wavefront is past its queries)
+  if (tid < 16) {
+    const bool sunk = a.sink && blockIdx.z == 0 && tid / a.HS < nr && hb0 + tid % a.HS < HG;
+    const float sink = sunk ? a.sink[g * HG + hb0 + tid % a.HS] : -INFINITY;
+    const float m = fmaxf(fmaxf(fmaxf(sM[0][tid], sM[1][tid]), fmaxf(sM[2][tid], sM[3][tid])), sink);
+    float sum = expf(sink - m);
+    for (int w = 0; w < 4; w++) sum += sL[w][tid] * expf(sM[w][tid] - m);
+    sM[4][tid] = m;
+    sL[4][tid] = sum;
+  }
+  __syncthreads();
   float f[4];
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const int m = quad * 4 + e;
-    f[e] = expf(sM[wave][m] - fmaxf(fmaxf(sM[0][m], sM[1][m]), fmaxf(sM[2][m], sM[3][m])));
-  }
+  for (int e = 0; e < 4; e++) f[e] = expf(sM[wave][quad * 4 + e] - sM[4][quad * 4 + e]);
   for (int w = 0; w < 4; w++) {
     if (wave == w) {
 #pragma unroll
@@ -217,20 +222,15 @@ attn_f32_k(AttnF32Args a) {
     if (rec) {
       rec[m * (VP + 2) + c] = smem[i];
       if (c == 0) {
-        const float M = fmaxf(fmaxf(sM[0][m], sM[1][m]), fmaxf(sM[2][m], sM[3][m]));
-        float L = 0.0f;
-        for (int w = 0; w < 4; w++) L += sL[w][m] * expf(sM[w][m] - M);
-        rec[m * (VP + 2) + VP] = M;
-        rec[m * (VP + 2) + VP + 1] = L;
+        rec[m * (VP + 2) + VP] = sM[4][m];
+        rec[m * (VP + 2) + VP + 1] = sL[4][m];
       }
       continue;
     }
-    const float M = fmaxf(fmaxf(sM[0][m], sM[1][m]), fmaxf(sM[2][m], sM[3][m]));
-    float L = 0.0f;
-    for (int w = 0; w < 4; w++) L += sL[w][m] * expf(sM[w][m] - M);
+    const float L = sL[4][m];
     const int h = g * HG + ms;
     a.out[h * a.soh + (r0 + mr) * a.sor + map * a.som + c] =
-        L > 0.0f ? smem[i] / L * out_factor(a, r0 + mr, h, c) : 0.0f;
+        L != 0.0f ? smem[i] / L * out_factor(a, r0 + mr, h, c) : 0.0f;
   }
 }
 
@@ -261,7 +261,7 @@ __global__ void __launch_bounds__(128) attn_f32_merge_k(AttnF32Args a, int VP) {
   for (int c = threadIdx.x; c < a.V; c += blockDim.x) {
     float num = 0.0f;
     for (int z = 0; z < a.splits; z++) num += sw[z] * rec[z * zs + c];
-    a.out[h * a.soh + (r0 + mr) * a.sor + map * a.som + c] = d > 0.0f ? num / d * out_factor(a, r0 + mr, h, c) : 0.0f;
+    a.out[h * a.soh + (r0 + mr) * a.sor + map * a.som + c] = d != 0.0f ? num / d * out_factor(a, r0 + mr, h, c) : 0.0f;
   }
 }
 

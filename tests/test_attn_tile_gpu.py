@@ -147,3 +147,24 @@ def test_fp32_keys_shorter_than_a_step(step, size):
     out = sm.window_attn(*(t.to(DEV) for t in (q, pool, bt, row_ent, pos)), None, 0.5, 40,
                          torch.empty(R, H * 4, device=DEV), PAGE, H, 1, size, 4, units=units)
     _close(out, want)
+
+
+@pytest.mark.parametrize("max_keys", [None, 700])
+@pytest.mark.parametrize("what", ["score", "sink"])
+def test_fp32_rows_that_are_not_a_number_say_so(what, max_keys):
+    """A query, or a sink, that is not a number gives a result that is not one, in its row (head) only."""
+    ent, row_ent, pos, bt, R, g = _step("portions", 4)
+    H, D = 3, 16
+    q, pool = torch.randn(R, H * D, generator=g), torch.randn((int(bt.max()) + 1) * PAGE, 2 * D, generator=g)
+    sink = torch.zeros(H)
+    if what == "sink":
+        sink[1] = float("nan")
+    else:
+        q[5, D + 2] = float("nan")
+    units = sm.make_units(ent, sm.window_rows_per_wave(H)).to(DEV)
+    want = sm.window_attn(q, pool, bt, row_ent, pos, sink, 0.3, 40, torch.empty(R, H * D), PAGE, H, 1, D, D)
+    out = sm.window_attn(*(t.to(DEV) for t in (q, pool, bt, row_ent, pos, sink)), 0.3, 40, torch.empty(R, H * D, device=DEV),
+                         PAGE, H, 1, D, D, units=units, max_keys=max_keys).cpu()
+    lost = want.isnan()
+    assert lost.any() and torch.equal(lost, out.isnan())
+    _close(out[~lost], want[~lost])
