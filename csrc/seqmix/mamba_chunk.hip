@@ -5,7 +5,10 @@
 //   chain        S_next = exp(c_(n-1)) S + L over each portion's chunks, from the slot's state (or zero at
 //                position 0); the last one is the slot's new state
 //   output pass  y_t = exp(c_t) S^T C_t + sum_{s <= t} exp(c_t - c_s) dt_s (C_t . B_s) x_s + D x_t,  y *= silu(z)
-// Every exponent is <= 0, so nothing overflows whatever the step sizes are.  One workgroup of four wavefronts per
+// Every exponent is <= 0, so nothing overflows whatever the step sizes are.  The running sums are kept in 64 bits and
+// differences rounded after they are taken: c grows with every token (to -64 at A = 16 and steps of 0.06), and the
+// weight between two tokens must not carry the rounding of what decayed before both (off by 1e-5 with drawn steps
+// at A = 16, by 5e-4 where small steps follow large ones, against 1e-7).  One workgroup of four wavefronts per
 // (chunk, head); sizes are padded to multiples of 16 with zeros in LDS.
 //
 // The walk of mamba_scan_k does the same 1 074 M state updates of a prompt of 2048 tokens (64 heads, 128 x 64 states)
@@ -39,21 +42,21 @@ struct MambaChunkArgs {
 };
 
 // dt and c of the chunk's tokens (zero steps beyond it) by the first wavefront: the loads, then the rest once
-// other loads are under way too
+// other loads are under way too.  A step below -200 counts as -200: exp() of either is zero, and sums stay finite.
 template <typename T>
 __device__ __forceinline__ float chunk_dt(const MambaChunkArgs& a, const Entry& en, int h) {
   const int t = threadIdx.x;
   return t < en.n && t < 64 ? ldf((const T*)a.zx, (size_t)(en.row0 + t) * a.ldz + a.dtoff + h) : 0.0f;
 }
 __device__ __forceinline__ void chunk_steps(const MambaChunkArgs& a, const Entry& en, int h, float raw, float* sdt,
-                                            float* sc) {
+                                            double* sc) {
   if (threadIdx.x >= 64) return;
   const int t = threadIdx.x;
   const float dt = t < en.n ? softplusf_(raw + a.dt_bias[h]) : 0.0f;
-  float c = -expf(a.A_log[h]) * dt;
+  double c = fmaxf(-expf(a.A_log[h]) * dt, -200.0f);
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const float v = __shfl_up(c, o, 64);
+    const double v = __shfl_up(c, o, 64);
     if (t >= o) c += v;
   }
   sdt[t] = dt;
@@ -97,7 +100,8 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 template <typename T, int NPT>   // value size padded to NPT * 16
 __global__ void __launch_bounds__(256) mamba_local_k(MambaChunkArgs a) {
   extern __shared__ __align__(16) float smem[];
-  __shared__ float sdt[MC], sc[MC];
+  __shared__ float sdt[MC];
+  __shared__ double sc[MC];
   typedef Cols<NPT> CP;
   const int c = blockIdx.x, h = blockIdx.y, N = a.N, P = a.P;
   const Entry en = load_entry(a.vent, c);
@@ -110,9 +114,9 @@ __global__ void __launch_bounds__(256) mamba_local_k(MambaChunkArgs a) {
   stage(row + h * P, a.C, en.n, P, PP, sX, LDX, a.vec);
   chunk_steps(a, en, h, raw, sdt, sc);
   if (threadIdx.x < 64) {   // within the first wavefront
-    const float end = __shfl(sc[threadIdx.x], en.n - 1, 64);
-    sdt[threadIdx.x] *= expf(end - sc[threadIdx.x]);
-    if (threadIdx.x == 0) a.decay[(size_t)c * a.H + h] = expf(end);
+    const double end = __shfl(sc[threadIdx.x], en.n - 1, 64);
+    sdt[threadIdx.x] *= expf((float)(end - sc[threadIdx.x]));
+    if (threadIdx.x == 0) a.decay[(size_t)c * a.H + h] = expf((float)end);
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
@@ -188,7 +192,8 @@ __global__ void __launch_bounds__(256) mamba_chain_k(MambaChunkArgs a) {
 template <typename T, int NPT>
 __global__ void __launch_bounds__(256) mamba_out_k(MambaChunkArgs a) {
   extern __shared__ __align__(16) float smem[];
-  __shared__ float sdt[MC], sc[MC];
+  __shared__ float sdt[MC];
+  __shared__ double sc[MC];
   typedef Cols<NPT> CP;
   const int c = blockIdx.x, h = blockIdx.y, N = a.N, P = a.P, inner = a.H * P;
   const Entry en = load_entry(a.vent, c);
@@ -255,18 +260,18 @@ __global__ void __launch_bounds__(256) mamba_out_k(MambaChunkArgs a) {
   }
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    const float m = expf(sc[r0 + k4 * 4 + r]);
+    const float m = expf((float)sc[r0 + k4 * 4 + r]);
 #pragma unroll
     for (int j = 0; j < NPT; j++) acc[j][r] *= m;
   }
-  const float ce = sc[r0 + i16];
+  const double ce = sc[r0 + i16];
 #pragma unroll
   for (int j = 0; j < MC / 16; j++) {
     if (j > wave) continue;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int s = j * 16 + k4 * 4 + r;
-      const float v = s <= r0 + i16 ? w[j][r] * expf(ce - sc[s]) * sdt[s] : 0.0f;
+      const float v = s <= r0 + i16 ? w[j][r] * expf((float)(ce - sc[s])) * sdt[s] : 0.0f;
 #pragma unroll
       for (int k = 0; k < NPT; k++)
         acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, sX[s * LDX + CP::at(k, i16)], acc[k], 0, 0, 0);

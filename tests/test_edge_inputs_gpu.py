@@ -67,3 +67,45 @@ def test_sinks_of_any_size(dt, tiled, max_keys, win):
     got = sm.latent_attn(*_to(a), torch.empty(H, R, D, dtype=dt, device=DEV), PAGE, units=units,
                          unit_rows=_rows(dt, per, tiled), max_keys=max_keys)
     torch.testing.assert_close(got.cpu().float(), want.float(), **_tol(dt))
+
+
+# ------------------------------------------------------------------ decays
+def _err(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("steps", ["even", "drawn", "large first"])
+@pytest.mark.parametrize("lens", [[64], [300, 40]])
+def test_mamba_scan_decays_in_64_bits(steps, lens):
+    """A weight between two tokens is as exact as the decays between them, whatever decayed before (A = 16)."""
+    g = torch.Generator().manual_seed(5)
+    H, P, N, G = 2, 64, 128, 1
+    inner, C = H * P, H * P + 2 * N
+    ent_h, r0 = [], 0
+    for i, n in enumerate(lens):
+        ent_h.append((r0, n, 7, i))
+        r0 += n
+    ent, R = torch.tensor(ent_h, dtype=torch.int32), r0
+    conv, zx = torch.randn(R, C, generator=g), torch.randn(R, 2 * inner + 2 * N + H, generator=g)
+    raw = {"even": torch.full((R, H), math.log(math.expm1(0.05))), "drawn": torch.randn(R, H, generator=g) - 2,
+           "large first": torch.where((torch.arange(R) % 64 < 32)[:, None], torch.randn(R, H, generator=g) + 4,
+                                      torch.full((R, H), -7.0))}[steps]
+    zx[:, inner + C:] = raw
+    Al, Dp, zero = torch.full((H,), math.log(16.0)), torch.randn(H, generator=g), torch.zeros(H)
+    S0 = torch.randn(len(lens), H, N, P, generator=g)
+    S, T = S0.clone().to(DEV), torch.zeros(len(lens), 3, C, device=DEV)
+    y = sm.mamba_scan(conv.to(DEV), zx.to(DEV), inner, inner + C, zero.to(DEV), Al.to(DEV), Dp.to(DEV), S, T,
+                      ent.to(DEV), ent_h, torch.empty(R, inner, device=DEV), H, P, N, G).cpu()
+    x, B, Cc = (t.double() for t in conv.split([inner, N, N], -1))
+    dt, A = torch.nn.functional.softplus(raw.double(), threshold=1e9), -torch.exp(Al.double())
+    z, want, ends = zx[:, :inner].double(), torch.empty(R, inner, dtype=torch.float64), []
+    for row0, n, _s, slot in ent_h:
+        st = S0[slot].double()
+        for t in range(row0, row0 + n):
+            xt = x[t].view(H, P)
+            st = torch.exp(A * dt[t])[:, None, None] * st + B[t][None, :, None] * (dt[t][:, None] * xt)[:, None]
+            want[t] = ((Cc[t] @ st + Dp.double()[:, None] * xt).reshape(inner)) * z[t] * torch.sigmoid(z[t])
+        ends.append(st)
+    # fp32 products and sums: a few roundings of 6e-8; a step of 4 at A = 16 carries its own rounding times 64
+    assert _err(y, want) < 6e-7
+    assert _err(S.cpu(), torch.stack(ends)) < 6e-7
