@@ -74,4 +74,43 @@ __device__ __forceinline__ bf16x8 read_keys_by_channel(const unsigned short* til
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// A place out of a row's sight has weight zero, but 0 * inf is nan: through the tiles' products a value that is not finite
+// reaches rows of the group that do not see it.  Groups whose sums are not finite are therefore done again pair by pair,
+// by a wavefront each, over the places that the pair's row sees.  Slow and rare; it stands behind the tile loop, whose
+// registers it must not take (a second walk through the tiles cost 13 % by its spills).
+__device__ __forceinline__ bool not_finite(f32x4 v) {
+  bool bad = false;
+#pragma unroll
+  for (int e = 0; e < 4; e++) bad |= !(fabsf(v[e]) < INFINITY);
+  return bad;
+}
+
+__device__ __forceinline__ float wave_dot(const bf16* x, const bf16* y, int n) {
+  float s = 0.0f;
+  for (int c = threadIdx.x & 63; c < n; c += 64) s = fmaf(ldf(x, c), ldf(y, c), s);
+  return wave_sum(s);
+}
+
+// softmax sums of one pair; a lane has every 64th channel
+template <int NC>
+struct PairSums {
+  float m, l, o[NC];
+  __device__ __forceinline__ void begin(float sink, bool sunk) {   // natural units
+    m = sunk ? sink : -1e30f;
+    l = sunk ? 1.0f : 0.0f;
+#pragma unroll
+    for (int t = 0; t < NC; t++) o[t] = 0.0f;
+  }
+  __device__ __forceinline__ void add(float s, const bf16* v, int V) {
+    const float up = fmaxf(m, s), f = m == up ? 1.0f : expf(m - up), w = expf(s - up);
+    m = up;
+    l = l * f + w;
+#pragma unroll
+    for (int t = 0; t < NC; t++) {
+      const int c = t * 64 + (threadIdx.x & 63);
+      o[t] = c < V ? o[t] * f + w * ldf(v, c) : 0.0f;
+    }
+  }
+};
+
 }  // namespace sm

@@ -33,7 +33,7 @@ latent_attn_tile_k(LatentArgs a) {
   extern __shared__ __align__(16) unsigned short lds[];   // [2][KT latents]
   __shared__ __align__(16) unsigned short sP[64 * KT];    // weights [pair][slot], see read_keys_by_channel
   __shared__ __align__(16) float sAl[64];                 // rescale factors of this tile, then the sums
-  __shared__ int sUp[4];                                  // wavefront w's pairs are rescaled
+  __shared__ int sUp[4], sBad[4];                         // wavefront w's pairs are rescaled; its sums are not finite
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), n16 = lane & 15, quad = lane >> 4;
   const int hg = (a.H + a.HS - 1) / a.HS, at = folded_block(), unit = a.U - 1 - at / hg, h0 = (at % hg) * a.HS;
   const int r0 = a.units[2 * unit], nr = a.units[2 * unit + 1];
@@ -203,6 +203,40 @@ latent_attn_tile_k(LatentArgs a) {
       if (NT2 == 16) __builtin_amdgcn_sched_barrier(0);
     }
   }
+  bool bad = false;
+#pragma unroll
+  for (int m = 0; m < 4; m++)
+#pragma unroll
+    for (int t = 0; t < CT; t++) bad |= not_finite(acc[m][t]);
+  bad = __any(bad);
+  if (lane == 0) sBad[wave] = bad;
+  __syncthreads();   // (and the last tile's factors have been read)
+  if (__builtin_expect(uniform(sBad[0] | sBad[1] | sBad[2] | sBad[3]), 0)) {   // see not_finite()
+#pragma unroll 1
+    for (int m = wave * 16; m < wave * 16 + 16; m++) {
+      const int row = r0 + m / a.HS, h = h0 + m % a.HS;
+      if (m / a.HS >= nr || h >= a.H) continue;
+      const int p = a.pos[row];
+      PairSums<RP / 64> sums;
+      sums.begin(a.sink ? a.sink[h] : 0.0f, a.sink && blockIdx.y == 0);
+#pragma unroll 1
+      for (int j = max(i_lo * KT, max(0, p - win + 1)); j <= min(p, i_hi * KT + KT - 1); j++) {
+        const bf16* c = a.cache + ((size_t)pages[j / page] * page + j % page) * rank;
+        sums.add(wave_dot(a.qa + (size_t)h * a.sqh + (size_t)row * a.sqr, c, rank) * a.scale, c, rank);
+      }
+      float* rec = a.part + (((size_t)unit * hg + at % hg) * a.splits + blockIdx.y) * 64 * (RP + 2) + m * (RP + 2);
+      const float f = a.splits > 1 ? 1.0f : sums.l != 0.0f ? 1.0f / sums.l : 0.0f;
+#pragma unroll
+      for (int t = 0; t < RP / 64; t++) {
+        const int c = t * 64 + lane;
+        if (c >= rank) continue;
+        if (a.splits > 1) rec[c] = sums.o[t];
+        else a.out[(size_t)h * a.soh + (size_t)row * a.sor + c] = __float2bfloat16(sums.o[t] * f);
+      }
+      if (a.splits > 1 && lane == 0) rec[RP] = sums.m, rec[RP + 1] = sums.l;
+    }
+    return;
+  }
   float l = l_part + __shfl_xor(l_part, 16, 64);
   l += __shfl_xor(l, 32, 64);
   m_run *= 1.0f / LOG2E_;   // natural from here on
@@ -216,7 +250,6 @@ latent_attn_tile_k(LatentArgs a) {
     l = l * sf + expf(sink - m);
     m_run = m;
   }
-  __syncthreads();   // the last tile's factors have been read
   if (quad == 0) sAl[wave * 16 + n16] = a.splits > 1 ? sf : l != 0.0f ? sf / l : 0.0f;
   __syncthreads();
   if (a.splits > 1) {

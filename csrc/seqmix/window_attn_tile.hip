@@ -335,6 +335,68 @@ window_attn_tile_k(WindowArgs a) {
     if (BLK && i + 2 < heads && i + 2 <= i_hi && tid < KT) srow[st][tid] = nrow;   // read after the next barrier
   }
   if (!wlive) return;
+  bool bad = false;
+#pragma unroll
+  for (int u = 0; u < MAPS; u++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) bad |= not_finite(acc[u][t]);
+  if (__builtin_expect(__any(bad), 0)) {   // see not_finite()
+#pragma unroll 1
+    for (int m = wave * 16; m < wave * 16 + 16; m++) {
+      const int row = r0 + m / a.HS, hs = hb0 + m % a.HS, h = g * HG + hs;
+      if (m / a.HS >= nr || hs >= HG) continue;
+      const int p = a.pos[row], blocks = BLK ? max(0, p - win + 1) / a.P : 0;
+      PairSums<(VP + 63) / 64> sums[MAPS];
+#pragma unroll
+      for (int u = 0; u < MAPS; u++) sums[u].begin(a.sink ? a.sink[h] : 0.0f, MAPS == 1 && a.sink && blockIdx.y == 0);
+#pragma unroll 1
+      for (int x = i_lo * KT; x < (i_hi + 1) * KT; x++) {
+        const int i = x / KT, j = place(i) + x % KT;
+        const bool head = (BLK || KEPT) && i < heads;
+        if (!(head ? j < (BLK ? blocks : nb) : j <= p && (j > p - win || (KEPT && j >= nb && j < a.keep)))) continue;
+        const bf16* kr = BLK && head ? a.blk + (size_t)block_row(j) * ldpool
+                                     : a.pool + ((size_t)pages[j / page] * page + j % page) * ldpool;
+#pragma unroll
+        for (int u = 0; u < MAPS; u++) {
+          float s = wave_dot(a.q + (size_t)row * a.ldq + (size_t)(h * MAPS + u) * D, kr + koff + u * D, D) * a.scale;
+          if (a.cap > 0.0f) s = a.cap * tanhf(s / a.cap);
+          if (a.r1) s -= a.r1[h] * log1pf(a.r2[h] * (float)(p - j));
+          sums[u].add(s, kr + voff, V);
+        }
+      }
+      if (a.splits > 1) {
+        float* rec = a.part + (((size_t)unit * gh + gb) * a.splits + blockIdx.y) * MAPS * 64 * (VP + 2) + m * (VP + 2);
+#pragma unroll
+        for (int u = 0; u < MAPS; u++, rec += 64 * (VP + 2)) {
+#pragma unroll
+          for (int t = 0; t < (VP + 63) / 64; t++)
+            if (t * 64 + lane < V) rec[t * 64 + lane] = sums[u].o[t];
+          if (lane == 0) rec[VP] = sums[u].m, rec[VP + 1] = sums[u].l;
+        }
+        continue;
+      }
+      float ss = 0.0f, f = sums[0].l != 0.0f ? 1.0f / sums[0].l : 0.0f;
+      if constexpr (MAPS == 2) {
+        const float f1 = sums[1].l != 0.0f ? a.lam / sums[1].l : 0.0f;
+#pragma unroll
+        for (int t = 0; t < (VP + 63) / 64; t++) {
+          sums[0].o[t] = sums[0].o[t] * f - sums[1].o[t] * f1;
+          ss += sums[0].o[t] * sums[0].o[t];
+        }
+        f = 1.0f / sqrtf(wave_sum(ss) / (float)V + a.eps);
+      }
+      f *= a.out_scale;
+      const bf16* gr = a.gate + (size_t)row * a.ldg + (size_t)h * (a.gate_pc ? V : 1);
+#pragma unroll
+      for (int t = 0; t < (VP + 63) / 64; t++) {
+        const int c = t * 64 + lane;
+        if (c >= V) continue;
+        const float gv = a.gate ? sigmoidf_(__bfloat162float(gr[a.gate_pc ? c : 0])) : 1.0f;
+        a.out[(size_t)row * a.ldo + (size_t)h * V + c] = __float2bfloat16(sums[0].o[t] * f * gv);
+      }
+    }
+    return;
+  }
   float l[MAPS];
 #pragma unroll
   for (int u = 0; u < MAPS; u++) {

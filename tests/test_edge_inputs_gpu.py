@@ -69,6 +69,50 @@ def test_sinks_of_any_size(dt, tiled, max_keys, win):
     torch.testing.assert_close(got.cpu().float(), want.float(), **_tol(dt))
 
 
+# ------------------------------------------------------------------ tokens that are not finite
+@pytest.mark.parametrize("dt", [torch.bfloat16])
+@pytest.mark.parametrize("bad", [INF, -INF, NAN])
+@pytest.mark.parametrize("max_keys", [None, 700])
+@pytest.mark.parametrize("form", ["window", "blocks", "kept", "maps", "latent", "latent512"])
+def test_attention_keeps_values_that_are_not_finite_to_later_rows(dt, bad, max_keys, form):
+    """Position 70's value is not finite: rows before it, and rows whose window has passed it, are as they were."""
+    ent, row_ent, pos, bt, R, g = _step([150, 40], [0, 37], 2)
+    H, D = 4, 64 if form != "latent512" else 512
+    M = 2 if form == "maps" else 1
+    win = 50 if form != "window" else 1 << 30
+    latent = form.startswith("latent")
+    width = D if latent else (M + 1) * D
+    pool = torch.randn((int(bt.max()) + 1) * PAGE, width, generator=g).to(dt)
+    q = torch.randn(R, H * M * D, generator=g).to(dt)
+    kw = {"blocks": dict(every=16), "kept": dict(keep=9), "maps": dict(diff=(0.4, 1e-4))}.get(form, {})
+    if form == "blocks":
+        kw["blk"] = torch.randn((int(bt.max()) + 1) * sm.blocks_per_page(PAGE, 16), width, generator=g).to(dt)
+        kw["blk"][int(bt[0, 1]) * 4, D + 3] = bad        # the block of tokens 64 .. 79
+    if form == "kept":
+        pool[int(bt[0, 0]) * PAGE + 4, D + 3] = bad      # a kept token, seen by all rows from there on
+    else:
+        pool[int(bt[0, 1]) * PAGE + 6, width - D + 3] = bad
+    per = sm.window_rows_per_wave(H)
+    units = sm.make_units(ent, _rows(dt, per, True)).to(DEV)
+    more = dict(units=units, unit_rows=_rows(dt, per, True), max_keys=max_keys)
+    if latent:
+        a = (q.view(R, H, D).transpose(0, 1).contiguous(), pool, bt, row_ent, pos, None, 0.05, win)
+        want = sm.latent_attn(*a, torch.empty(H, R, D, dtype=dt), PAGE)
+        got = sm.latent_attn(*_to(a), torch.empty(H, R, D, dtype=dt, device=DEV), PAGE, **more)
+        # a latent is key and value: the rows that see it are lost as a whole
+        lost = ~want.isfinite()
+    else:
+        a = (q, pool, bt, row_ent, pos, None, 0.1, win)
+        want = sm.window_attn(*a, torch.empty(R, H * D, dtype=dt), PAGE, H, 1, D, D, **kw)
+        got = sm.window_attn(*_to(a), torch.empty(R, H * D, dtype=dt, device=DEV), PAGE, H, 1, D, D, **more,
+                             **{k: _to(v) for k, v in kw.items()})
+        lost = ~want.isfinite()
+    assert lost.any() and not lost.all()
+    got = got.cpu()
+    assert torch.equal(lost, ~got.isfinite())
+    torch.testing.assert_close(got[~lost].float(), want[~lost].float(), **_tol(dt))
+
+
 # ------------------------------------------------------------------ decays
 def _err(a, b):
     return float((a.double() - b).norm() / b.norm())
