@@ -17,10 +17,8 @@
 // wavefront.  Two prompts of 389 and 117 rows, 8 heads: latents of 512 numbers 114 us against 4330 us for
 // latent_attn_k (one workgroup per row, scalar products); 8 heads of 128 on 2, capped and penalised, 47
 // against 300 for window_attn_k.
-#include "common.h"
+#include "attn_tile.h"
 using namespace sm;
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 struct AttnF32Args {
   const float* q;
@@ -56,6 +54,7 @@ attn_f32_k(AttnF32Args a) {
   constexpr int VP = NB * 64;
   extern __shared__ __align__(16) float smem[];   // queries [16][LDQ], at the end sums [16][VP]
   __shared__ float sM[5][16], sL[5][16];          // per wavefront, then all together
+  __shared__ int sBad[4];                         // a wavefront's sums are not finite
   const int tid = threadIdx.x, lane = tid & 63, n16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int HG = a.H / a.G, hblocks = (HG + a.HS - 1) / a.HS;
@@ -186,7 +185,43 @@ attn_f32_k(AttnF32Args a) {
     sM[wave][n16] = m_run;
     sL[wave][n16] = l;
   }
+  float z = 0.0f;
+#pragma unroll
+  for (int t = 0; t < NB * 4; t++) not_finite(acc[t], z);
+  const bool bad = __any(z != z);
+  if (lane == 0) sBad[wave] = bad;
   __syncthreads();   // (and every wavefront is past its queries)
+  if (__builtin_expect(uniform(sBad[0] | sBad[1] | sBad[2] | sBad[3]), 0)) {   // see not_finite()
+#pragma unroll 1
+    for (int m = wave * 4; m < wave * 4 + 4; m++) {
+      const int row = r0 + m / a.HS, hs = hb0 + m % a.HS, h = g * HG + hs;
+      if (m / a.HS >= nr || hs >= HG) continue;
+      const int p = a.pos[row], blocks = a.blk ? max(0, p - win + 1) / a.P : 0;
+      PairSums<NB> sums;
+      sums.begin(a.sink ? a.sink[h] : 0.0f, a.sink && blockIdx.z == 0);
+#pragma unroll 1
+      for (int u = t_lo * 16; u < min(t_hi * 16, last + 1); u++) {
+        const int j = u < nb ? u : u + shift;
+        if (!(a.blk && u < nb ? u < blocks : j <= p && (j > p - win || (!a.blk && j < a.keep)))) continue;
+        const float* kr = key_row(u);
+        float s = wave_dot(a.q + h * a.sqh + row * a.sqr + map * a.sqm, kr + koff, D) * a.scale;
+        if (a.cap > 0.0f) s = a.cap * tanhf(s / a.cap);
+        if (a.r1) s -= a.r1[h] * log1pf(a.r2[h] * (float)(p - j));
+        sums.add(s, kr + voff, V);
+      }
+      float* rec = a.part + (((size_t)unit * gridDim.y + blockIdx.y) * a.splits + blockIdx.z) * 16 * (VP + 2) + m * (VP + 2);
+#pragma unroll
+      for (int t = 0; t < NB; t++) {
+        const int c = t * 64 + lane;
+        if (c >= V) continue;
+        if (a.splits > 1) rec[c] = sums.o[t];
+        else a.out[h * a.soh + row * a.sor + map * a.som + c] =
+            sums.l != 0.0f ? sums.o[t] / sums.l * out_factor(a, row, h, c) : 0.0f;
+      }
+      if (a.splits > 1 && lane == 0) rec[VP] = sums.m, rec[VP + 1] = sums.l;
+    }
+    return;
+  }
   if (tid < 16) {
     const bool sunk = a.sink && blockIdx.z == 0 && tid / a.HS < nr && hb0 + tid % a.HS < HG;
     const float sink = sunk ? a.sink[g * HG + hb0 + tid % a.HS] : -INFINITY;

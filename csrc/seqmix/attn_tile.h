@@ -78,14 +78,14 @@ __device__ __forceinline__ bf16x8 read_keys_by_channel(const unsigned short* til
 // reaches rows of the group that do not see it.  Groups whose sums are not finite are therefore done again pair by pair,
 // by a wavefront each, over the places that the pair's row sees.  Slow and rare; it stands behind the tile loop, whose
 // registers it must not take (a second walk through the tiles cost 13 % by its spills).
-__device__ __forceinline__ bool not_finite(f32x4 v) {
-  bool bad = false;
+// z: 0 while all numbers are finite, then nan
+__device__ __forceinline__ void not_finite(f32x4 v, float& z) {
 #pragma unroll
-  for (int e = 0; e < 4; e++) bad |= !(fabsf(v[e]) < INFINITY);
-  return bad;
+  for (int e = 0; e < 4; e++) z = fmaf(v[e], 0.0f, z);
 }
 
-__device__ __forceinline__ float wave_dot(const bf16* x, const bf16* y, int n) {
+template <typename T>
+__device__ __forceinline__ float wave_dot(const T* x, const T* y, int n) {
   float s = 0.0f;
   for (int c = threadIdx.x & 63; c < n; c += 64) s = fmaf(ldf(x, c), ldf(y, c), s);
   return wave_sum(s);
@@ -101,7 +101,8 @@ struct PairSums {
 #pragma unroll
     for (int t = 0; t < NC; t++) o[t] = 0.0f;
   }
-  __device__ __forceinline__ void add(float s, const bf16* v, int V) {
+  template <typename T>
+  __device__ __forceinline__ void add(float s, const T* v, int V) {
     const float up = fmaxf(m, s), f = m == up ? 1.0f : expf(m - up), w = expf(s - up);
     m = up;
     l = l * f + w;

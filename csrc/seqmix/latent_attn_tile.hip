@@ -203,12 +203,12 @@ latent_attn_tile_k(LatentArgs a) {
       if (NT2 == 16) __builtin_amdgcn_sched_barrier(0);
     }
   }
-  bool bad = false;
+  float z = 0.0f;
 #pragma unroll
   for (int m = 0; m < 4; m++)
 #pragma unroll
-    for (int t = 0; t < CT; t++) bad |= not_finite(acc[m][t]);
-  bad = __any(bad);
+    for (int t = 0; t < CT; t++) not_finite(acc[m][t], z);
+  const bool bad = __any(z != z);
   if (lane == 0) sBad[wave] = bad;
   __syncthreads();   // (and the last tile's factors have been read)
   if (__builtin_expect(uniform(sBad[0] | sBad[1] | sBad[2] | sBad[3]), 0)) {   // see not_finite()

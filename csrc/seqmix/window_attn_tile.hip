@@ -335,12 +335,12 @@ window_attn_tile_k(WindowArgs a) {
     if (BLK && i + 2 < heads && i + 2 <= i_hi && tid < KT) srow[st][tid] = nrow;   // read after the next barrier
   }
   if (!wlive) return;
-  bool bad = false;
+  float z = 0.0f;
 #pragma unroll
   for (int u = 0; u < MAPS; u++)
 #pragma unroll
-    for (int t = 0; t < NT; t++) bad |= not_finite(acc[u][t]);
-  if (__builtin_expect(__any(bad), 0)) {   // see not_finite()
+    for (int t = 0; t < NT; t++) not_finite(acc[u][t], z);
+  if (__builtin_expect(__any(z != z), 0)) {   // see not_finite()
 #pragma unroll 1
     for (int m = wave * 16; m < wave * 16 + 16; m++) {
       const int row = r0 + m / a.HS, hs = hb0 + m % a.HS, h = g * HG + hs;

@@ -70,7 +70,7 @@ def test_sinks_of_any_size(dt, tiled, max_keys, win):
 
 
 # ------------------------------------------------------------------ tokens that are not finite
-@pytest.mark.parametrize("dt", [torch.bfloat16])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("bad", [INF, -INF, NAN])
 @pytest.mark.parametrize("max_keys", [None, 700])
 @pytest.mark.parametrize("form", ["window", "blocks", "kept", "maps", "latent", "latent512"])
