@@ -18,10 +18,8 @@
 // per CU; the output pass's products alone take 31 us at the card's fp32 rate.  LDS is read four numbers at a
 // time: with one number per read, C and the weights in LDS too, and one row's load in flight per thread while staging,
 // the passes took 61 + 30 + 137.
-#include "common.h"
+#include "attn_tile.h"
 using namespace sm;
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define MC 64   // tokens of a chunk
 
@@ -277,15 +275,36 @@ __global__ void __launch_bounds__(256) mamba_out_k(MambaChunkArgs a) {
   for (int j = 0; j < MC / 16; j++) {
     if (j > wave) continue;
     f32x4 p[NPT];
+    float v[4];
 #pragma unroll
     for (int k = 0; k < NPT; k++) p[k] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int s = j * 16 + k4 * 4 + r;
-      const float v = s <= r0 + i16 ? w[j][r] * expf((float)(ce - sc[s])) * sdt[s] : 0.0f;
+      v[r] = s <= r0 + i16 ? w[j][r] * expf((float)(ce - sc[s])) * sdt[s] : 0.0f;
 #pragma unroll
       for (int k = 0; k < NPT; k++)
-        p[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, sX[s * LDX + CP::at(k, i16)], p[k], 0, 0, 0);
+        p[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[r], sX[s * LDX + CP::at(k, i16)], p[k], 0, 0, 0);
+    }
+    if (j == wave) {   // a later token of the block weighs zero, but its input need not be finite: 0 * inf is nan
+      float z = 0.0f;
+#pragma unroll
+      for (int k = 0; k < NPT; k++) not_finite(p[k], z);
+      if (__builtin_expect(__any(z != z), 0)) {
+#pragma unroll
+        for (int k = 0; k < NPT; k++) p[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int u = 0; u < 4; u++)      // token 4 q + u of the block
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const float f = __shfl(v[u], q * 16 + 4 * k4 + r, 64);
+              if (4 * q + u > 4 * k4 + r) continue;
+#pragma unroll
+              for (int k = 0; k < NPT; k++) p[k][r] = fmaf(f, sX[(r0 + 4 * q + u) * LDX + CP::at(k, i16)], p[k][r]);
+            }
+      }
     }
 #pragma unroll
     for (int k = 0; k < NPT; k++) acc[k] += p[k];

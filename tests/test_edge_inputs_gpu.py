@@ -113,6 +113,40 @@ def test_attention_keeps_values_that_are_not_finite_to_later_rows(dt, bad, max_k
     torch.testing.assert_close(got[~lost].float(), want[~lost].float(), **_tol(dt))
 
 
+@pytest.mark.parametrize("where", ["x", "B", "C", "dt", "z"])
+@pytest.mark.parametrize("bad", [INF, NAN])
+@pytest.mark.parametrize("P", [64, 40, 200])
+def test_mamba_scan_keeps_tokens_that_are_not_finite_to_later_ones(where, bad, P):
+    g = torch.Generator().manual_seed(3)
+    H, N, G = 2, 32, 1
+    inner, C = H * P, H * P + 2 * N
+    lens, at = [130, 40], 74
+    ent_h = [(0, 130, 0, 0), (130, 40, 9, 1)]
+    ent = torch.tensor(ent_h, dtype=torch.int32)
+    R = sum(lens)
+    conv, zx = torch.randn(R, C, generator=g), torch.randn(R, 2 * inner + 2 * N + H, generator=g)
+    dtb, Al, Dp = (torch.randn(H, generator=g) for _ in range(3))
+    S0, T0 = torch.randn(2, H, N, P, generator=g), torch.zeros(2, 3, C)
+    if where == "dt":
+        zx[at, inner + C] = bad                  # head 0's step size
+    elif where == "z":
+        zx[at, 5] = bad
+    else:
+        conv[at, {"x": 5, "B": inner + 5, "C": inner + N + 5}[where]] = bad
+    res = []
+    for dev in ("cpu", DEV):
+        S = S0.clone().to(dev)
+        y = sm.mamba_scan(conv.to(dev), zx.to(dev), inner, inner + C, dtb.to(dev), Al.to(dev), Dp.to(dev), S,
+                          T0.clone().to(dev), ent.to(dev), ent_h, torch.empty(R, inner, device=dev), H, P, N, G)
+        res.append((y.cpu(), S.cpu()))
+    (y1, s1), (y2, s2) = res
+    for a, b in ((y1, y2), (s1, s2)):
+        ok = a.isfinite()
+        assert not ok.all() or where in ("C", "z") and a is s1
+        assert torch.equal(ok, b.isfinite())
+        torch.testing.assert_close(b[ok], a[ok], rtol=1e-4, atol=1e-5 * float(a[ok].abs().max()))
+
+
 # ------------------------------------------------------------------ decays
 def _err(a, b):
     return float((a.double() - b).norm() / b.norm())
