@@ -16,6 +16,8 @@
 // 600 tokens, decays near 1, mixed and strongest): outputs 1.6e-7, 1.4e-7, 1.4e-7, the walk 1.6e-7, 1.4e-7, 1.5e-7;
 // states 1.7e-7, 1.2e-7, 0.8e-7, the walk 1.4e-7, 0.6e-7, 0.4e-7, a walk of chunks 1.7e-7, 1.2e-7, 0.9e-7.
 // The system is solved in blocks of 16 rows, the blocks on the diagonal by their inverses.
+// A weight of zero stands for "not before this token" in these products, and 0 * inf is nan: a chunk and head whose
+// inputs are not all finite is walked token by token instead, so that tokens before such an input are what they were.
 //
 // A chunk and head are about 700 matrix instructions per wavefront.  The walk of gdelta_scan_k (once for L and T, once
 // for the outputs) took 2 x 205 us for 2048 tokens and 32 heads of 64, and the chain 654 us of 32 dependent products on
@@ -45,6 +47,67 @@ struct GdeltaArgs {
   float eps;
 };
 
+// T, L, Q and O of a chunk and head by its tokens in order: a thread takes 16 rows of a column of T and of L
+template <typename T>
+__device__ __forceinline__ void walk_chunk(const GdeltaArgs& p, const Entry& en, int c, int h, float* smem) {
+  float *sr = smem, *sk = sr + GC * GLD, *su = sk + GC * GLD, *sa = su + GC * GLD, *sw = sa + GC * GLD, *sv = sw + GC * GLD;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, D = p.D;
+  const int vc = wave * 16 + (lane & 15), i0 = (lane >> 4) * 16;
+  const int col = h * D + min(lane, D - 1);
+  for (int t = wave; t < en.n; t += 4) {   // a wavefront's own places below: no wait needed in between
+    const size_t row = (size_t)(en.row0 + t);
+    const int at = t * GLD + lane;
+    const bool in = lane < D;
+    const float k = in ? ldf((const T*)p.k, row * p.ld + col) : 0.0f;
+    const float u = k * (1.0f / sqrtf(wave_sum(k * k) + 1e-6f));
+    sr[at] = in ? ldf((const T*)p.r, row * p.ld + col) : 0.0f;
+    sk[at] = k;
+    su[at] = u;
+    sa[at] = in ? sigmoidf_(ldf((const T*)p.a, row * p.ld + col) + p.ab[col]) * u : 0.0f;
+    sw[at] = in ? expf(-GD_DECAY_SCALE * sigmoidf_(ldf((const T*)p.lo, row * p.ldlo + col) + p.w0[col])) : 1.0f;
+    sv[at] = in ? ldf((const T*)p.v, row * p.ld + col) : 0.0f;
+  }
+  __syncthreads();
+  float S[16], M[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) S[q] = 0.0f, M[q] = i0 + q == vc ? 1.0f : 0.0f;
+  auto over_rows = [](float x) {   // the sum over a column's four threads
+    x += __shfl_xor(x, 16, 64);
+    return x + __shfl_xor(x, 32, 64);
+  };
+  const size_t base = ((size_t)c * p.H + h) * GC * GC;
+  for (int t = 0; t < en.n; t++) {
+    const int at = t * GLD + i0;
+    float ds = 0.0f, dm = 0.0f, os = 0.0f, om = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      ds += su[at + q] * S[q];
+      dm += su[at + q] * M[q];
+    }
+    ds = over_rows(ds);
+    dm = over_rows(dm);
+    const float v = sv[t * GLD + vc];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      S[q] = sw[at + q] * S[q] - sa[at + q] * ds + sk[at + q] * v;
+      M[q] = sw[at + q] * M[q] - sa[at + q] * dm;
+      os += S[q] * sr[at + q];
+      om += M[q] * sr[at + q];
+    }
+    os = over_rows(os);
+    om = over_rows(om);
+    if (i0 == 0) {
+      p.oo[base + t * GC + vc] = os;
+      p.qq[base + t * GC + vc] = om;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    p.loc[base + (i0 + q) * GC + vc] = S[q];
+    p.trn[base + (i0 + q) * GC + vc] = M[q];
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
   extern __shared__ __align__(16) float smem[];
@@ -60,6 +123,7 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
   const int c = blockIdx.x, h = blockIdx.y, D = p.D;
   const Entry en = load_entry(p.vent, c);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, quad = lane >> 4;
+  float odd = 0.0f;   // becomes nan with an input that is not finite
   // a lane's channel of the wavefront's 16 tokens
   {
     const int col = h * D + min(lane, D - 1);
@@ -93,9 +157,11 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
       sU[at] = (float)(u * up);
       up *= w[q];
       const double down = 1.0 / up;
+      const float kd = (float)(kv[q] * down), ad = (float)((double)(av[q] * u) * down);
       sR[at] = (float)(rv[q] * up);
-      sK[at] = (float)(kv[q] * down);
-      sA[at] = (float)((double)(av[q] * u) * down);
+      sK[at] = kd;
+      sA[at] = ad;
+      odd += 0.0f * kd + 0.0f * ad;
     }
   }
   // values as operands: token 16 b + quad * 4 + e, this wavefront's 16 columns
@@ -107,8 +173,12 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
     for (int e = 0; e < 4; e++) {
       const int t = b * 16 + quad * 4 + e;
       V[b][e] = (t < en.n && vc < D) ? ldf((const T*)p.v, (size_t)(en.row0 + t) * p.ld + h * D + vc) : 0.0f;
+      odd += 0.0f * V[b][e];
     }
-  __syncthreads();
+  if (__syncthreads_or(odd != 0.0f)) {
+    walk_chunk<T>(p, en, c, h, smem);
+    return;
+  }
   // the four tables of weights: this wavefront's 16 rows t, s <= t
   f32x4 akk[4], auu[4], bk[4], bu[4];
 #pragma unroll
@@ -355,9 +425,9 @@ __global__ void __launch_bounds__(256) gdelta_out_k(GdeltaArgs p) {
 #pragma unroll
   for (int e = 0; e < 4; e++) {
     const int t = wave * 16 + quad * 4 + e;
-    float ss = 0.0f;   // columns beyond D are zero
+    float ss = 0.0f;   // a column beyond D is zero, or nan after a walk
 #pragma unroll
-    for (int j = 0; j < 4; j++) ss += acc[j][e] * acc[j][e];
+    for (int j = 0; j < 4; j++) ss += n16 * 4 + j < D ? acc[j][e] * acc[j][e] : 0.0f;
 #pragma unroll
     for (int m = 8; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
     const float rs = 1.0f / sqrtf(ss / (float)D + p.eps);

@@ -147,6 +147,37 @@ def test_mamba_scan_keeps_tokens_that_are_not_finite_to_later_ones(where, bad, P
         torch.testing.assert_close(b[ok], a[ok], rtol=1e-4, atol=1e-5 * float(a[ok].abs().max()))
 
 
+@pytest.mark.parametrize("where", ["r", "k", "v", "g", "a", "lo"])
+@pytest.mark.parametrize("bad", [INF, NAN])
+@pytest.mark.parametrize("D", [64, 40, 7])
+def test_gdelta_scan_keeps_tokens_that_are_not_finite_to_later_ones(where, bad, D):
+    g = torch.Generator().manual_seed(4)
+    H, at = 2, 74
+    n = H * D
+    ent_h = [(0, 130, 0, 0), (130, 40, 9, 1)]
+    ent, R = torch.tensor(ent_h, dtype=torch.int32), 170
+    proj, lo = torch.randn(R, 5 * n, generator=g), torch.randn(R, n, generator=g)
+    w0, ab, nw = (torch.randn(n, generator=g) for _ in range(3))
+    S0 = torch.randn(2, H, D, D, generator=g)
+    if where == "lo":
+        lo[at, D - 1] = bad                      # in head 0, as below
+    else:
+        proj[at, "rkvga".index(where) * n + D - 1] = bad
+    res = []
+    for dev in ("cpu", DEV):
+        S, p = S0.clone().to(dev), proj.to(dev)
+        o = sm.gdelta_scan(*[p[:, i * n:(i + 1) * n] for i in range(5)], lo.to(dev), w0.to(dev), ab.to(dev), nw.to(dev),
+                           S, ent.to(dev), ent_h, torch.empty(R, n, device=dev), H, D, 1e-5)
+        res.append((o.cpu(), S.cpu()))
+    (o1, s1), (o2, s2) = res
+    harmless = bad == INF and where in ("g", "a", "lo")   # behind a sigmoid
+    assert o1.isfinite().all() == harmless
+    for a, b in ((o1, o2), (s1, s2)):
+        ok = a.isfinite()
+        assert torch.equal(ok, b.isfinite())
+        torch.testing.assert_close(b[ok], a[ok], rtol=1e-4, atol=1e-4)   # as in the tests of ordinary inputs
+
+
 # ------------------------------------------------------------------ decays
 def _err(a, b):
     return float((a.double() - b).norm() / b.norm())
