@@ -657,10 +657,12 @@ def ff_act(gu, out, limit: float, alpha: float = 1.702):
 
 
 # ------------------------------------------------------------------ recurrences in chunks
-# A portion of at least 2 * SCAN_CHUNK tokens is scanned in chunks of SCAN_CHUNK tokens that
-# run side by side (local pass, chain over the chunks, output pass); shorter steps -- decode,
-# small portions -- walk their tokens in one pass.  Both recurrences are linear in the state,
-# so the chunked form computes the same sums in another order (fp32 throughout).
+# Long portions are scanned in chunks that run side by side (local pass, chain over the chunks, output pass); shorter
+# steps -- decode, small portions -- walk their tokens in one pass.  The recurrences are linear in the state, so the
+# chunked form computes the same sums in another order (fp32 throughout).  Scans that walk their chunks too take
+# chunks of SCAN_CHUNK tokens from 2 * SCAN_CHUNK on.  Mamba-2 and the generalized delta rule with heads of up to
+# GD_MATRIX_MAX have chunks as matrix products, of SCAN_CHUNK tokens too but no more than LIGHT_CHUNK, from
+# LIGHT_MIN on.  0: all of these walk.
 SCAN_CHUNK = int(os.environ.get("P2P_SCAN_CHUNK", "64"))
 
 
@@ -701,6 +703,11 @@ def chunk_tables(ent_host: list, chunk: int, device):
 
 def _chunked(ent_host) -> bool:
     return SCAN_CHUNK > 0 and max(e[1] for e in ent_host) >= 2 * SCAN_CHUNK
+
+
+def _matrix_chunks(ent_host) -> int:
+    """Tokens per chunk of the matrix-product form of this step's scans, 0: they walk."""
+    return min(SCAN_CHUNK, LIGHT_CHUNK) if max(e[1] for e in ent_host) >= LIGHT_MIN else 0
 
 
 # ------------------------------------------------------------------ generalized delta rule
@@ -745,8 +752,9 @@ def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: 
     assert ent.dtype == torch.int32 and ent.is_contiguous() and ent.shape[1] == 4
     if D > 256:
         raise ValueError("gdelta_scan: head size %d > 256" % D)
-    if D <= GD_MATRIX_MAX and max(e[1] for e in ent_host) >= LIGHT_MIN:
-        vent, cent = chunk_tables(ent_host, min(SCAN_CHUNK or LIGHT_CHUNK, LIGHT_CHUNK), r.device)
+    chunk = _matrix_chunks(ent_host) if D <= GD_MATRIX_MAX else 0
+    if chunk > 0:
+        vent, cent = chunk_tables(ent_host, chunk, r.device)
         tmp = torch.empty(4, vent.shape[0], H, 64, 64, device=r.device, dtype=torch.float32)
         _chk(lib().p2p_sm_gdelta_chunk(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), a.data_ptr(), ld,
@@ -874,8 +882,9 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
     if N > 256 or P > 256:
         raise ValueError("mamba_scan: state %d / value %d sizes above 256" % (N, P))
     E = ent.shape[0]
-    if max(e[1] for e in ent_host) >= LIGHT_MIN:
-        vent, cent = chunk_tables(ent_host, min(SCAN_CHUNK or LIGHT_CHUNK, LIGHT_CHUNK), zx.device)
+    chunk = _matrix_chunks(ent_host)
+    if chunk > 0:
+        vent, cent = chunk_tables(ent_host, chunk, zx.device)
         NV = vent.shape[0]
         tmp = torch.empty(NV, H, N, P, device=zx.device, dtype=torch.float32)
         decay = torch.empty(NV, H, device=zx.device, dtype=torch.float32)

@@ -135,6 +135,27 @@ def test_mamba(dt, H, P, N, G, K, scan_chunk):
         torch.testing.assert_close(T_g.cpu()[[2, 0, 3]], T_c[[2, 0, 3]], rtol=0, atol=0)
 
 
+@pytest.fixture
+def walks(monkeypatch):
+    """SCAN_CHUNK = 0: no scan forms chunks, whatever its portions are."""
+    def tables(*_a):
+        raise AssertionError("a scan formed chunks")
+    monkeypatch.setattr(sm, "SCAN_CHUNK", 0)
+    monkeypatch.setattr(sm, "chunk_tables", tables)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D", [(2, 40), (3, 20), (1, 72), (2, 64), (1, 136), (2, 7)])
+def test_gdelta_walks(dt, H, D, walks):
+    test_gdelta(dt, H, D, 0)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,P,N,G,K", [(6, 40, 24, 3, 3), (2, 72, 80, 2, 2), (2, 200, 256, 1, 4), (8, 64, 128, 4, 4)])
+def test_mamba_walks(dt, H, P, N, G, K, walks):
+    test_mamba(dt, H, P, N, G, K, 0)
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,rank,win", [(6, 120, 36), (3, 40, 7), (5, 96, 200), (16, 512, 33), (20, 64, 64), (1, 8, 3)])
 def test_latent_attn(dt, H, rank, win):
