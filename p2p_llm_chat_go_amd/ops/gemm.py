@@ -272,11 +272,12 @@ def _code(wt, M, epi, norm, waves):
 def _untuned(wt, x, epi) -> int:
     """Launch code of a shape the table does not hold.  Logits of 16 rows and more (the table's LM head entry is the
     greedy one) go to the wide kernel, which reads the activations once per 128 columns instead of once per
-    16: 128256 x 4096 at 8 / 16 / 17 / 32 / 64 rows, skinny 172 / 207 / 227 / 304 / 533 us, wide 175 / 189 / 176 /
-    188 / 221; 32000 x 4096 46 / 56 / 63 / 82 / 164 and 50 / 53 / 48 / 50 / 55.  Fewer columns than fill the chip
-    with workgroups of 128 (250 at 32000) would split K and keep the skinny kernel."""
+    16, where its workgroups of 128 columns are more than half the CUs: no more than that and it cuts K, whose sums
+    then have another order.  us, skinny / wide at K = 4096, 8, 16, 17, 32 and 64 rows: 128256 columns 173 / 174,
+    213 / 185, 231 / 171, 314 / 183, 530 / 207; 32000 columns 44 / 46, 52 / 47, 54 / 43, 82 / 44, 160 / 47; 18432
+    columns 26 / 30, 34 / 33, 34 / 29, 44 / 31, 91 / 38; 16512 columns 24 / 30, 34 / 32, 34 / 28, 44 / 31, 90 / 38."""
     N, K = tiled_shape(wt)
-    if (epi == EPI_F32 and 16 <= x.shape[0] <= SKINNY_MAX_M and N >= 128 * 250 and not _is_f8(wt)
+    if (epi == EPI_F32 and 16 <= x.shape[0] <= SKINNY_MAX_M and N > 128 * 128 and not _is_f8(wt)
             and wide_ok(N, K, epi) and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0):
         return WIDE_FLAG | WIDE16
     return 0

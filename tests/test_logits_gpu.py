@@ -9,7 +9,7 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 48, 64, 70])
-@pytest.mark.parametrize("N,K", [(32000, 256), (32128, 1280), (31984, 512), (32000, 288)])
+@pytest.mark.parametrize("N,K", [(32000, 256), (32128, 1280), (31984, 512), (32000, 288), (16384, 512), (16512, 4096), (20480, 256)])
 @pytest.mark.parametrize("norm", [False, True])
 def test_logits_by_rows(M, N, K, norm):
     g = torch.Generator(device=DEV).manual_seed(M + K)
