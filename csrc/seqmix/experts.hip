@@ -660,8 +660,11 @@ int p2p_sm_group_route(const void* h, int ldh, const float* wr, int R, int W, in
   size_t shm = (size_t)(W + 2 * E + groups + top) * 4;
   if (shm > 64 * 1024) return (int)hipErrorInvalidValue;
   const size_t many = (size_t)(16 * (2 * E + groups + 3 * top) + E) * 4;
-  // one row per workgroup takes 13 us up to 100 rows and 18 at 500; sixteen per workgroup 14 at 600
-  if (R >= 256 && many <= 48 * 1024) {
+  // Sixteen rows per workgroup take as long as one row's E sums of W products by one wavefront, whatever R is (until
+  // the chip is full); one row per workgroup takes its slots' atomics, R of them, and shares a row's sums among four
+  // wavefronts.  us, one / sixteen: E * W = 8192, 256 rows 10.0 / 10.9, 606 rows 18.3 / 11.1; 16384, 606 rows 19 /
+  // 17; 65536, 1024 rows 40 / 54, 2048 rows 68 / 55; 262144, 2048 rows 92 / 188
+  if (R >= 256 && (size_t)R * 28 >= (size_t)E * W && many <= 48 * 1024) {
     SM_DISPATCH_T(f32, hipLaunchKernelGGL(group_route_rows_k<T>, dim3((R + 15) / 16), dim3(1024), many, st,
                                            (const T*)h, ldh, wr, R, W, E, top, groups, keep, score, corr,
                                            gscore, ids, wts, cnt, rows, ldr, bias, renorm, wscale));

@@ -15,7 +15,10 @@ DEV = "cuda:0"
     (256, 72, 8, 2, 1, 1, dict(score="top_softmax", bias=True)),
     (301, 200, 12, 3, 4, 2, dict()),
     (1000, 64, 70, 5, 7, 3, dict(score="softmax", group_score="max", renorm=True, scale=1.5)),
-    (259, 40, 3, 1, 1, 1, dict(score="softmax", corr=True))])
+    (259, 40, 3, 1, 1, 1, dict(score="softmax", corr=True)),
+    # many experts: a row per workgroup up to R * 28 = E * W, sixteen from there on
+    (300, 100, 128, 8, 8, 3, dict(renorm=True)), (365, 80, 128, 8, 8, 3, dict()), (366, 80, 128, 8, 8, 3, dict()),
+    (1300, 72, 256, 8, 1, 1, dict(score="softmax"))])
 def test_routing_of_many_rows(dt, R, W, E, top, groups, keep, kw):
     g = torch.Generator().manual_seed(2)
     h, wr = torch.randn(R, W, generator=g).to(dt), torch.randn(E, W, generator=g) / W ** 0.5
