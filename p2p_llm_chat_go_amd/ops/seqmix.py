@@ -705,6 +705,24 @@ def _chunked(ent_host) -> bool:
     return SCAN_CHUNK > 0 and max(e[1] for e in ent_host) >= 2 * SCAN_CHUNK
 
 
+def portion_tables(ent_host: list, chunk: int, least: int, device):
+    """``chunk_tables`` of the portions of at least ``least`` tokens, and the other portions as entries (None where
+    there are none): these walk in a launch of their own.  A decoded token beside a prompt costs a whole chunk
+    otherwise (64 tokens and 31 decoded ones, Mamba-2 with 64 heads of 128 x 64: 263 us in chunks, 80 walked)."""
+    kept = getattr(ent_host, "tables", None)
+    key = (chunk, least, str(device))
+    if kept is not None and key in kept:
+        return kept[key]
+    vent, cent = scan_chunks([e for e in ent_host if e[1] >= least], chunk)
+    short = [tuple(e) for e in ent_host if e[1] < least]
+    V, E = vent.shape[0], cent.shape[0]
+    every = torch.cat([vent, cent, torch.tensor(short, dtype=torch.int32).view(-1, 4)]).to(device)
+    out = every[:V], every[V:V + E], every[V + E:] if short else None
+    if kept is not None:
+        kept[key] = out
+    return out
+
+
 def _matrix_chunks(ent_host) -> int:
     """Tokens per chunk of the matrix-product form of this step's scans, 0: they walk."""
     return min(SCAN_CHUNK, LIGHT_CHUNK) if max(e[1] for e in ent_host) >= LIGHT_MIN else 0
@@ -754,15 +772,16 @@ def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: 
         raise ValueError("gdelta_scan: head size %d > 256" % D)
     chunk = _matrix_chunks(ent_host) if D <= GD_MATRIX_MAX else 0
     if chunk > 0:
-        vent, cent = chunk_tables(ent_host, chunk, r.device)
+        vent, cent, ent = portion_tables(ent_host, chunk, LIGHT_MIN, r.device)
         tmp = torch.empty(4, vent.shape[0], H, 64, 64, device=r.device, dtype=torch.float32)
         _chk(lib().p2p_sm_gdelta_chunk(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), a.data_ptr(), ld,
             lo.data_ptr(), lo.stride(0), w0.data_ptr(), ab.data_ptr(), normw.data_ptr(),
-            state.data_ptr(), tmp.data_ptr(), vent.data_ptr(), vent.shape[0], cent.data_ptr(), E,
+            state.data_ptr(), tmp.data_ptr(), vent.data_ptr(), vent.shape[0], cent.data_ptr(), cent.shape[0],
             out.data_ptr(), out.stride(0), H, D, eps, _f32(r), _st(r)), "gdelta_chunk")
-        return out
-    if _chunked(ent_host):
+        if ent is None:
+            return out
+    elif _chunked(ent_host):
         vent, cent = chunk_tables(ent_host, SCAN_CHUNK, r.device)
         tmp = torch.empty(3, vent.shape[0], H, D, D, device=r.device, dtype=torch.float32)
         _chk(lib().p2p_sm_gdelta_scan_chunked(
@@ -774,7 +793,7 @@ def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: 
     _chk(lib().p2p_sm_gdelta_scan(r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(),
                                   a.data_ptr(), ld, lo.data_ptr(), lo.stride(0), w0.data_ptr(),
                                   ab.data_ptr(), normw.data_ptr(), state.data_ptr(),
-                                  ent.data_ptr(), E, out.data_ptr(), out.stride(0), H, D, eps,
+                                  ent.data_ptr(), ent.shape[0], out.data_ptr(), out.stride(0), H, D, eps,
                                   _f32(r), _st(r)), "gdelta_scan")
     return out
 
@@ -882,21 +901,21 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
     if N > 256 or P > 256:
         raise ValueError("mamba_scan: state %d / value %d sizes above 256" % (N, P))
     E = ent.shape[0]
-    chunk = _matrix_chunks(ent_host)
+    chunk, walk = _matrix_chunks(ent_host), ent
     if chunk > 0:
-        vent, cent = chunk_tables(ent_host, chunk, zx.device)
+        vent, cent, walk = portion_tables(ent_host, chunk, LIGHT_MIN, zx.device)
         NV = vent.shape[0]
         tmp = torch.empty(NV, H, N, P, device=zx.device, dtype=torch.float32)
         decay = torch.empty(NV, H, device=zx.device, dtype=torch.float32)
         _chk(lib().p2p_sm_mamba_scan_chunked(
             conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), dtoff, dt_bias.data_ptr(),
             A_log.data_ptr(), Dp.data_ptr(), state.data_ptr(), tmp.data_ptr(), decay.data_ptr(),
-            vent.data_ptr(), NV, cent.data_ptr(), E, y.data_ptr(), H, P, N, G, _f32(zx),
+            vent.data_ptr(), NV, cent.data_ptr(), cent.shape[0], y.data_ptr(), H, P, N, G, _f32(zx),
             _st(zx)), "mamba_scan_chunked")
-    else:
+    if walk is not None:
         _chk(lib().p2p_sm_mamba_scan(conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), xoff, dtoff,
                                      dt_bias.data_ptr(), A_log.data_ptr(), Dp.data_ptr(),
-                                     state.data_ptr(), tail.data_ptr(), ent.data_ptr(), E,
+                                     state.data_ptr(), tail.data_ptr(), walk.data_ptr(), walk.shape[0],
                                      y.data_ptr(), H, P, N, G, Km1 + 1, _f32(zx), _st(zx)),
              "mamba_scan")
     _chk(lib().p2p_sm_mamba_tail(zx.data_ptr(), zx.stride(0), xoff, tail.data_ptr(),

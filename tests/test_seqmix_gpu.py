@@ -156,6 +156,18 @@ def test_mamba_walks(dt, H, P, N, G, K, walks):
     test_mamba(dt, H, P, N, G, K, 0)
 
 
+@pytest.mark.parametrize("lens,starts", [([64, 1, 5, 1], [0, 9, 0, 3]), ([1, 130, 1, 70, 31], [2, 4, 7, 0, 6])])
+@pytest.mark.parametrize("scan", ["gdelta", "mamba"])
+def test_decoded_tokens_beside_prompts_form_no_chunks(lens, starts, scan, monkeypatch):
+    cut, whole = [], sm.scan_chunks
+    monkeypatch.setattr(sm, "scan_chunks", lambda e, c: (cut.extend(x[1] for x in e), whole(e, c))[1])
+    if scan == "gdelta":
+        test_gdelta_long_portions(torch.float32, lens, starts, 2, 64, 0.0)
+    else:
+        test_mamba_long_portions(lens, starts, 4, 64, 128, 2, False)
+    assert sorted(cut) == sorted(n for n in lens if n > 31)
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,rank,win", [(6, 120, 36), (3, 40, 7), (5, 96, 200), (16, 512, 33), (20, 64, 64), (1, 8, 3)])
 def test_latent_attn(dt, H, rank, win):
