@@ -5,8 +5,8 @@
 // walked in order.  The per-token vectors (r, k, v, decay w, removal rate a) are staged
 // through LDS a chunk of tokens at a time, with the decay and the rate evaluated while
 // staging.  The head's outputs are RMS-normalised, weighted and gated as each chunk
-// finishes.  Long portions run as chunks side by side: gdelta_chunk.hip for head sizes up to 64,
-// modes 1 and 2 + gdelta_combine_k above.
+// finishes.  Long portions run as chunks side by side: as matrix products in gdelta_chunk.hip, or
+// (head sizes above 64, many chunks of small heads) modes 1 and 2 + gdelta_combine_k.
 #include "common.h"
 using namespace sm;
 
@@ -246,7 +246,7 @@ int p2p_sm_gdelta_scan(const void* r, const void* k, const void* v, const void* 
                                  ldo, H, D, eps, 0, nullptr, f32, st);
 }
 
-// Long portions in chunks that run side by side (head sizes above 64; the others: gdelta_chunk.hip): every
+// Long portions in chunks that run side by side that are walked: every
 // chunk's local end state and transition matrix, a chain over each portion's chunks, then every chunk again from its true initial
 // state.  vent: the chunks as entries (row0, n, 1, chunk index); tmp: 3 fp32 buffers of
 // [chunks, H, D, D] (local, transition, init); cent: per portion (first chunk, chunks, first
@@ -270,7 +270,8 @@ int p2p_sm_gdelta_scan_chunked(const void* r, const void* k, const void* v, cons
   size_t shm = (size_t)(TI + 3) * DS * 4;
   int nw = 256 / threads;   // groups of `threads` per block
 #define GC(P) hipLaunchKernelGGL((gdelta_combine_k<P>), dim3(E * H), dim3(threads * nw), shm, st, loc, trn, ini, state, cent, H, D, TI)
-  if (D <= 128) GC(128);
+  if (D <= 32) GC(32);
+  else if (D <= 128) GC(128);
   else GC(256);
 #undef GC
   err = (int)hipGetLastError();

@@ -660,9 +660,9 @@ def ff_act(gu, out, limit: float, alpha: float = 1.702):
 # Long portions are scanned in chunks that run side by side (local pass, chain over the chunks, output pass); shorter
 # steps -- decode, small portions -- walk their tokens in one pass.  The recurrences are linear in the state, so the
 # chunked form computes the same sums in another order (fp32 throughout).  Scans that walk their chunks too take
-# chunks of SCAN_CHUNK tokens from 2 * SCAN_CHUNK on.  Mamba-2 and the generalized delta rule with heads of up to
-# GD_MATRIX_MAX have chunks as matrix products, of SCAN_CHUNK tokens too but no more than LIGHT_CHUNK, from
-# LIGHT_MIN on.  0: all of these walk.
+# chunks of SCAN_CHUNK tokens from 2 * SCAN_CHUNK on.  Mamba-2 (portions from LIGHT_MIN on) and the generalized delta
+# rule (_gdelta_portions) have chunks as matrix products, of SCAN_CHUNK tokens too but no more than LIGHT_CHUNK.
+# 0: all of these walk.
 SCAN_CHUNK = int(os.environ.get("P2P_SCAN_CHUNK", "64"))
 
 
@@ -731,6 +731,31 @@ def _matrix_chunks(ent_host) -> int:
 # ------------------------------------------------------------------ generalized delta rule
 GD_DECAY_SCALE = math.exp(-0.5)
 GD_MATRIX_MAX = 64    # head sizes of the matrix-instruction chunks (larger ones walk theirs)
+GD_MATRIX_MIN = 48    # shortest portions that may take them
+
+
+def _gdelta_portions(ent_host, H: int, D: int) -> int:
+    """Shortest portion of this step that runs as matrix products of chunks (0: none does).  A chunk and head holds a CU
+    (104 KB of LDS) for about 45 us, whatever its head size (padded to 64): 45 us for up to 256 of them, then 0.17 us
+    each.  What it is set against, us, other form -> matrix products:
+    a walk of 1.1 us per token of the longest portion, all heads and portions side by side: 32 tokens of 32 heads of 64
+    38 -> 46, 48 tokens 55 -> 47, 8 portions of 64 and 32 heads of 64 76 -> 66, 64 heads of 32 64 -> 107, 4 of 127 and
+    64 heads of 32 115 -> 106, 8 of 100 and 64 heads of 64 130 -> 200; so up to 6 chunks and heads per token;
+    from 128 tokens on chunks that are walked, whose cost falls with the head size: 4 portions of 1024 and 64 heads of
+    64 1705 -> 924, 64 heads of 32 643 -> 867, 64 heads of 16 709 -> 855, 32 heads of 32 432 -> 374."""
+    chunk = min(SCAN_CHUNK, LIGHT_CHUNK)
+    if chunk <= 0 or D > GD_MATRIX_MAX:
+        return 0
+
+    def chunks(least, below):
+        return H * sum(-(-e[1] // chunk) for e in ent_host if least <= e[1] < below)
+
+    long, some = chunks(128, math.inf), chunks(GD_MATRIX_MIN, 128)
+    if D <= 32 and long > 2048:
+        return 0
+    if some and some <= 6 * max(e[1] for e in ent_host if e[1] < 128) - 128:
+        return GD_MATRIX_MIN
+    return 128 if long else 0
 
 
 def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: int, D: int,
@@ -770,9 +795,9 @@ def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: 
     assert ent.dtype == torch.int32 and ent.is_contiguous() and ent.shape[1] == 4
     if D > 256:
         raise ValueError("gdelta_scan: head size %d > 256" % D)
-    chunk = _matrix_chunks(ent_host) if D <= GD_MATRIX_MAX else 0
-    if chunk > 0:
-        vent, cent, ent = portion_tables(ent_host, chunk, LIGHT_MIN, r.device)
+    least = _gdelta_portions(ent_host, H, D)
+    if least > 0:
+        vent, cent, ent = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, r.device)
         tmp = torch.empty(4, vent.shape[0], H, 64, 64, device=r.device, dtype=torch.float32)
         _chk(lib().p2p_sm_gdelta_chunk(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), a.data_ptr(), ld,

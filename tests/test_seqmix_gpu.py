@@ -156,6 +156,21 @@ def test_mamba_walks(dt, H, P, N, G, K, walks):
     test_mamba(dt, H, P, N, G, K, 0)
 
 
+@pytest.mark.parametrize("lens,H,D,form", [
+    ([47], 2, 64, "walk"), ([48, 47, 1], 2, 64, "matrix"), ([64] * 8, 33, 20, "walk"), ([64] * 8, 32, 20, "matrix"),
+    ([128] + [64] * 8, 33, 20, "matrix"), ([1100], 128, 8, "chunks"), ([1000, 3], 128, 8, "matrix"), ([130, 5], 2, 72, "chunks")])
+def test_gdelta_forms(lens, H, D, form, monkeypatch):
+    """Both sides of the lines between the walk, walked chunks and matrix products."""
+    ran = []
+    for nm in ("p2p_sm_gdelta_scan", "p2p_sm_gdelta_scan_chunked", "p2p_sm_gdelta_chunk"):
+        f = getattr(sm.lib(), nm)
+        monkeypatch.setattr(sm.lib(), nm, lambda *a, f=f, nm=nm: (ran.append(nm), f(*a))[1])
+    test_gdelta_long_portions(torch.float32, lens, [3 * i for i in range(len(lens))], H, D, 0.0)
+    assert ran[0] == {"walk": "p2p_sm_gdelta_scan", "chunks": "p2p_sm_gdelta_scan_chunked",
+                      "matrix": "p2p_sm_gdelta_chunk"}[form]
+    assert len(ran) == (2 if form == "matrix" and min(lens) < 48 or lens[0] == 128 else 1)
+
+
 @pytest.mark.parametrize("lens,starts", [([64, 1, 5, 1], [0, 9, 0, 3]), ([1, 130, 1, 70, 31], [2, 4, 7, 0, 6])])
 @pytest.mark.parametrize("scan", ["gdelta", "mamba"])
 def test_decoded_tokens_beside_prompts_form_no_chunks(lens, starts, scan, monkeypatch):
@@ -165,7 +180,7 @@ def test_decoded_tokens_beside_prompts_form_no_chunks(lens, starts, scan, monkey
         test_gdelta_long_portions(torch.float32, lens, starts, 2, 64, 0.0)
     else:
         test_mamba_long_portions(lens, starts, 4, 64, 128, 2, False)
-    assert sorted(cut) == sorted(n for n in lens if n > 31)
+    assert sorted(cut) == sorted(n for n in lens if n >= (48 if scan == "gdelta" else 32))
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
