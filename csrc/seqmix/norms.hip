@@ -608,10 +608,15 @@ int p2p_sm_add_norm2(float* x, const void* a, int lda, const void* b, int ldb, c
                    (((ws1 ? (size_t)w1 : 0) | (ws2 ? (size_t)w2 : 0)) % 16) == 0 &&
                    ((size_t)a | (size_t)b | (size_t)h1 | (size_t)h2 | (size_t)cy) % a4 == 0 &&
                    (lda | ldb | ld1 | ld2 | ldcy) % 4 == 0;
-  SM_DISPATCH_T(f32, ROW_FORMS(row_form(n, by4),
-                               hipLaunchKernelGGL((add_norm2_k<T, VE, NC>), dim3(R), dim3(256), 0, st, x,
-                                                  (const T*)a, lda, (const T*)b, ldb, rows, vec, n, eps, w1, ws1,
-                                                  (T*)h1, ld1, w2, ws2, (T*)h2, ld2, (const T*)cy, ldcy, cw, top)));
+#define AN2(VE, NC)                                                                                                \
+  hipLaunchKernelGGL((add_norm2_k<T, VE, NC>), dim3(R), dim3(256), 0, st, x, (const T*)a, lda, (const T*)b, ldb,   \
+                     rows, vec, n, eps, w1, ws1, (T*)h1, ld1, w2, ws2, (T*)h2, ld2, (const T*)cy, ldcy, cw, top)
+  // rows that one number per load takes: this pass loads up to six operands, so the smallest form that holds the row
+  // (2048 rows of 510 numbers with registers for 1024 / 4096: 6.6 / 10.4 us, of 1502 with 2048 / 4096: 10.0 / 14.2)
+  if (!by4 && n <= 1024) SM_DISPATCH_T(f32, AN2(1, 4));
+  else if (!by4 && n <= 2048) SM_DISPATCH_T(f32, AN2(1, 8));
+  else SM_DISPATCH_T(f32, ROW_FORMS(row_form(n, by4), AN2(VE, NC)));
+#undef AN2
   return (int)hipGetLastError();
 }
 
