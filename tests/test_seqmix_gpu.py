@@ -311,7 +311,7 @@ def test_row_passes_by_width(dt, n, off):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("F,off", [(4, 0), (1020, 0), (1023, 0), (1028, 4), (1028, 1), (1, 0)])
+@pytest.mark.parametrize("F,off", [(4, 0), (252, 0), (256, 0), (1020, 0), (1023, 0), (1028, 4), (1028, 1), (1, 0)])
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
 def test_glu_act_by_width(dt, F, off, act):
     """Four channels per thread at the edges of a block, and the widths and rows that take one."""
