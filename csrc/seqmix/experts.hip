@@ -343,9 +343,13 @@ __device__ __forceinline__ f32x4 mfma_piece(uint4 a, uint4 b, f32x4 c) {
 // Few slots per expert (decode-sized steps), on the matrix cores: a block takes 16 slots x
 // 64 output columns of one expert and its four wavefronts split K among themselves, so the
 // chain of dependent loads is a quarter as long; each wavefront walks its share in steps of 32
-// with one A fragment (the gathered rows) and four B fragments (16 weight rows each), four steps'
-// fragments in flight while the current products run; the four partial tiles are added through LDS.  fp32 takes half the K per step (a fragment is 16 bytes of a row) and four products.
-template <typename T>
+// with one A fragment (the gathered rows) and four B fragments (16 weight rows each), DEPTH steps'
+// fragments in flight while the current products run; the four partial tiles are added through LDS.  fp32 takes half
+// the K per step (a fragment is 16 bytes of a row) and four products.
+// Four steps where a wavefront's share is longer than 8, two (76 instead of 116 registers) where it is shorter: rows
+// of 512 numbers, 1024 columns, 128 experts of 40 slots, four / two steps 83 / 68 us, rows of 2048 with 64 experts of 16
+// slots and 2048 columns 160 / 163.
+template <typename T, int DEPTH>
 __global__ void __launch_bounds__(256)
 expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restrict__ w,
                    const int* __restrict__ cnt, const int* __restrict__ rows, int ldr,
@@ -370,8 +374,6 @@ expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
 #pragma unroll
   for (int t = 0; t < 4; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint4 zero = make_uint4(0, 0, 0, 0);
-  // DEPTH steps in flight
-  constexpr int DEPTH = 4;
   uint4 av[DEPTH], bv[DEPTH][4];
   auto load = [&](int k, uint4& a, uint4 (&b)[4]) {
     const bool in = k + quad * EP < ke;            // K is a multiple of EP
@@ -702,8 +704,12 @@ int p2p_sm_expert_gemm(const void* x, int ldx, int x_div, const void* w, const i
     }
     int tmp = (((total_slots + 15) / 16 + E) + 7) & ~7;
     dim3 grid(tmp * ((N + 63) / 64));
-    SM_DISPATCH_T(f32, hipLaunchKernelGGL(expert_gemm_mfma_k<T>, grid, dim3(256), 0, st, (const T*)x, ldx, x_div,
-                                           (const T*)w, cnt, rows, ldr, (T*)out, ldo, N, K, E, tmp, epi, limit, alpha));
+#define EM(DEPTH)                                                                                                     \
+  SM_DISPATCH_T(f32, hipLaunchKernelGGL((expert_gemm_mfma_k<T, DEPTH>), grid, dim3(256), 0, st, (const T*)x, ldx, x_div, \
+                                         (const T*)w, cnt, rows, ldr, (T*)out, ldo, N, K, E, tmp, epi, limit, alpha))
+    if (K > 128 * ep) EM(4);   // 4 wavefronts x 8 steps of 4 pieces
+    else EM(2);
+#undef EM
     return (int)hipGetLastError();
   }
   int tmp = (((total_slots + 31) / 32 + E) + 7) & ~7;
