@@ -304,18 +304,27 @@ def _skinny(x, w) -> bool:
     a captured graph, library -> kernel in us): at most 16 rows of one matrix instruction; K, because one
     workgroup walks all of it (8 rows, 2048 x 8192: 12.9 -> 15.0, 2048 x 4096: 12.5 -> 8.3; fp32
     2048 x 4096: 13.2 -> 15.0, 2048 x 2048: 10.5 -> 8.5); N, because every workgroup reads the
-    activations again (8 rows, 32000 x 2048: 33.7 -> 33.1; 16 rows, 10272 x 2048: 14.6 -> 15.9,
-    4608 x 2048: 12.0 -> 10.9; fp32 4608 x 2048: 14.1 -> 16.4); fp32 from 1024 columns on (96 x 2048:
-    6.7 -> 7.7, bf16 5.4 -> 4.8).  The rest: what 16-byte loads need."""
+    activations again, the more so the more rows there are and the longer they are (8 rows, 12288 x 2048: 14.8 -> 13.8,
+    16384 x 1536: 13.0 -> 13.9, 6144 x 3072: 11.9 -> 13.0, 4096 x 4096: 15.6 -> 9.9; 16 rows, 8192 x 2048: 13.1 -> 11.9,
+    10272 x 2048: 14.6 -> 15.9, 6144 x 3072: 12.0 -> 16.1; 4 rows, 12288 x 4096: 24.1 -> 21.1; fp32, 16 rows,
+    8192 x 1024: 13.1 -> 12.2, 16384 x 512: 9.9 -> 12.1, 4608 x 2048: 14.1 -> 16.4); few columns only where the chain of
+    loads is short (bf16, 16 rows, 96 x 2048: 5.5 -> 5.5, 96 x 4096: 7.9 -> 8.9, 8 rows 7.9 -> 7.6; fp32 96 x 2048: 6.7 ->
+    7.7, 1024 x 2048 16 rows 8.6 -> 9.8, 8 rows 8.7 -> 8.5).  The rest: what 16-byte loads need."""
     M, K = x.shape
     N = w.shape[0]
     if not (0 < M <= 16 and x.is_cuda and w.is_cuda and x.dtype == w.dtype and w.shape[1] == K
             and x.stride(1) == 1 and w.is_contiguous()):
         return False
     if x.dtype == torch.bfloat16:
-        fits, ep = K <= 4096 and N <= (16384 if M <= 8 else 8192), 8
+        ep = 8
+        if K <= 2048:
+            fits = N <= ((16384 if K <= 1024 else 12288) if M <= 8 else 8192)
+        else:
+            fits = K <= 4096 and N <= (12288 if M <= 4 else 4096) and (N >= 256 or M <= 8)
     elif x.dtype == torch.float32:
-        fits, ep = K <= 2048 and N >= 1024 and N * K <= 8 << 20, 4
+        ep = 4
+        fits = (K <= 2048 and 1024 <= N and N * K <= 8 << 20 and (N <= 8192 or K <= 256 or M <= 4)
+                and (M <= 8 or K <= 1024 or N >= 2048))
     else:
         return False
     return (fits and K >= ep and K % ep == 0 and x.stride(0) % ep == 0
