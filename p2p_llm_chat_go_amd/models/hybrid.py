@@ -342,14 +342,15 @@ class StepBatch:
                 self.ids.device)
         return u
 
-    def attn_units(self, rows_per_wave: int, shared: bool = True):
+    def attn_units(self, rows_per_wave: int, shared: bool = True, latent: int = 0):
         """(row groups, rows they were cut to) for an attention layer (``ops.seqmix.attn_unit_rows``;
         not ``shared``: the layer has no kernel of shared key tiles)."""
         if not shared:
             return self.units(rows_per_wave), rows_per_wave
-        rows = self._units.get(("rows", rows_per_wave))
+        key = ("rows", rows_per_wave, latent)
+        rows = self._units.get(key)
         if rows is None:
-            rows = self._units[("rows", rows_per_wave)] = sm.attn_unit_rows(rows_per_wave, self.ent_host)
+            rows = self._units[key] = sm.attn_unit_rows(rows_per_wave, self.ent_host, latent)
         return self.units(rows), rows
 
 
@@ -609,7 +610,8 @@ class LatentAttention(Mixer):
         sm.rmsnorm(proj[:, H * D:H * D + r], self.cnorm, self.eps, pool, out_rows=b.cache_rows)
         qa = torch.bmm(proj[:, :H * D].view(b.R, H, D).transpose(0, 1), self.uk)   # [H, R, rank]
         ol = torch.empty_like(qa)
-        units, rows = b.attn_units(sm.latent_rows_per_wave(H), sm.latent_mfma_ok(qa, pool) and pool.shape[1] > 32)
+        units, rows = b.attn_units(sm.latent_rows_per_wave(H), sm.latent_mfma_ok(qa, pool) and pool.shape[1] > 32,
+                                   pool.shape[1])
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
                        ol, PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
         o = torch.bmm(ol, self.uvt)                                                # [H, R, V]
@@ -984,7 +986,8 @@ class RopeLatentAttention(Mixer):
         if nrot2 < Rd:
             qa[:, :, r + nrot2:] = q3[:, :, D + nrot2:].transpose(0, 1)
         ol = torch.empty_like(qa)
-        units, rows = b.attn_units(sm.latent_rows_per_wave(H), sm.latent_mfma_ok(qa, pool) and pool.shape[1] > 32)
+        units, rows = b.attn_units(sm.latent_rows_per_wave(H), sm.latent_mfma_ok(qa, pool) and pool.shape[1] > 32,
+                                   pool.shape[1])
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, ol,
                        PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
         if not self.HEAD_GATE:

@@ -1096,6 +1096,15 @@ def _tiled_units(unit_rows, rows_per_wave: int) -> int:
 LATENT_SPLIT_BLOCKS = 512   # split windows while a step has fewer blocks than this
 
 
+def _key_runs(blocks: int, most: int, tile: int) -> int:
+    """Runs of keys that the windows of a step of few workgroups are cut into.  A wavefront takes runs of 64 keys, four
+    wavefronts that share key tiles runs of 256: shorter ones cost more in the merge than they gain (100 rows and 12
+    decoded ones, windows of 256, 16 heads of 128, 256 / 64 keys: 11.9 / 14.1 us), unless the step has so few
+    workgroups that its chip is mostly idle (8 rows at 500, latents of 512: 26.6 / 17.9; 16 heads of 256: 18.8 / 12.9)."""
+    run = 256 if tile and (most <= 128 or blocks * -(-most // 64) > 128) else 64
+    return max(1, min(-(-most // run), LATENT_SPLIT_BLOCKS // blocks, 64))
+
+
 def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: int, out,
                 page: int, units=None, max_keys=None, unit_rows=None):
     """Windowed attention over cached latents with a softmax sink.
@@ -1144,7 +1153,7 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
         tile = _tiled_units(unit_rows, latent_rows_per_wave(H))
         splits = 1
         if max_keys is not None and U * hg < LATENT_SPLIT_BLOCKS:
-            splits = max(1, min(-(-min(max_keys, win) // (256 if tile else 64)), LATENT_SPLIT_BLOCKS // (U * hg), 64))
+            splits = _key_runs(U * hg, min(max_keys, win), tile)
         part = None
         if splits > 1:
             L = lib()
@@ -1579,13 +1588,17 @@ def window_rows_per_wave(HG: int) -> int:
     return latent_rows_per_wave(HG)
 
 
-def attn_unit_rows(rows_per_wave: int, ent_host: list) -> int:
+def attn_unit_rows(rows_per_wave: int, ent_host: list, latent: int = 0) -> int:
     """Rows per group (``make_units``) that a step's attention is cut into: those of one wavefront, or
     four times as many for the kernels whose four wavefronts share the key tiles.  Those win as
     soon as half of their rows are taken (a group of a decoded token leaves three of the four
-    wavefronts idle)."""
+    wavefronts idle).  ``latent``: size of a layer's latents; up to 128 they are so short that only portions of more
+    than 32 rows pay for sharing (16 heads, latents of 64, a wavefront each / shared: 16 rows 6.2 / 7.5 us, 16
+    portions of 20 6.7 / 7.7, 16 of 5 at 300 10.6 / 12.6, one of 33 7.5 / 7.5, 8 of 100 11.3 / 9.8)."""
     tile = 4 * rows_per_wave
     groups = sum(-(-e[1] // tile) for e in ent_host)
+    if 0 < latent <= 128 and max(e[1] for e in ent_host) <= 32:
+        return rows_per_wave
     return tile if 2 * sum(e[1] for e in ent_host) >= groups * tile else rows_per_wave
 
 
@@ -1705,7 +1718,7 @@ def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: in
         splits = 1
         if max_keys is not None and blocks < LATENT_SPLIT_BLOCKS:
             most = min(max_keys, win + keep) + (max(0, max_keys - win) // every if blk is not None else 0)
-            splits = max(1, min(-(-most // (256 if tile else 64)), LATENT_SPLIT_BLOCKS // blocks, 64))
+            splits = _key_runs(blocks, most, tile)
         part = None
         if splits > 1:
             L = lib()
