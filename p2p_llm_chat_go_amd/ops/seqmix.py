@@ -669,8 +669,8 @@ def ff_act(gu, out, limit: float, alpha: float = 1.702):
 # Long portions are scanned in chunks that run side by side (local pass, chain over the chunks, output pass); shorter
 # steps -- decode, small portions -- walk their tokens in one pass.  The recurrences are linear in the state, so the
 # chunked form computes the same sums in another order (fp32 throughout).  Scans that walk their chunks too take
-# chunks of SCAN_CHUNK tokens from 2 * SCAN_CHUNK on.  Mamba-2 (portions from LIGHT_MIN on) and the generalized delta
-# rule (_gdelta_portions) have chunks as matrix products, of SCAN_CHUNK tokens too but no more than LIGHT_CHUNK.
+# chunks of SCAN_CHUNK tokens from 2 * SCAN_CHUNK on.  Mamba-2 and the generalized delta rule have chunks as matrix
+# products, of SCAN_CHUNK tokens too but no more than LIGHT_CHUNK, for the portions that matrix_portions names.
 # 0: all of these walk.
 SCAN_CHUNK = int(os.environ.get("P2P_SCAN_CHUNK", "64"))
 
@@ -716,8 +716,7 @@ def _chunked(ent_host) -> bool:
 
 def portion_tables(ent_host: list, chunk: int, least: int, device):
     """``chunk_tables`` of the portions of at least ``least`` tokens, and the other portions as entries (None where
-    there are none): these walk in a launch of their own.  A decoded token beside a prompt costs a whole chunk
-    otherwise (64 tokens and 31 decoded ones, Mamba-2 with 64 heads of 128 x 64: 263 us in chunks, 80 walked)."""
+    there are none), which walk in a launch of their own."""
     kept = getattr(ent_host, "tables", None)
     key = (chunk, least, str(device))
     if kept is not None and key in kept:
@@ -732,39 +731,45 @@ def portion_tables(ent_host: list, chunk: int, least: int, device):
     return out
 
 
-def _matrix_chunks(ent_host) -> int:
-    """Tokens per chunk of the matrix-product form of this step's scans, 0: they walk."""
-    return min(SCAN_CHUNK, LIGHT_CHUNK) if max(e[1] for e in ent_host) >= LIGHT_MIN else 0
+def matrix_portions(ent_host: list, heads: int, first: float, start: float, each: float, token: float) -> int:
+    """Shortest portion of a step that a scan with chunks as matrix products takes there, 0: all walk.  Chunks of all
+    heads cost ``first`` us, or ``start`` and ``each`` per chunk and head where that is more; a walk, all its portions and
+    heads side by side, ``token`` us per token of the longest.  So decoded tokens beside a prompt join its
+    chunks while these leave CUs idle and walk in a launch of their own where they do not (64 tokens and 31 decoded ones,
+    Mamba-2, all in chunks / apart: 32 heads of 16 x 64 42 / 32 us, 64 heads of 128 x 64 261 / 70; 200 tokens and 8
+    portions of 20: 29 / 53 and 97 / 76).  Portions from 128 tokens on are always chunks, a step below LIGHT_MIN walks."""
+    chunk = min(SCAN_CHUNK, LIGHT_CHUNK)
+    lens = sorted((e[1] for e in ent_host), reverse=True)
+    if chunk <= 0 or lens[0] < LIGHT_MIN:
+        return 0
+    best, least, chunks = 2.0 + token * lens[0] if lens[0] < 128 else math.inf, 0, 0
+    for n, shorter in zip(lens, lens[1:] + [0]):
+        chunks += -(-n // chunk)
+        if shorter == n:
+            continue
+        cost = max(first, start + each * chunks * heads) + (2.0 + token * shorter if shorter else 0.0)
+        if cost < best and shorter < 128:
+            best, least = cost, n
+    return least
 
 
 # ------------------------------------------------------------------ generalized delta rule
 GD_DECAY_SCALE = math.exp(-0.5)
 GD_MATRIX_MAX = 64    # head sizes of the matrix-instruction chunks (larger ones walk theirs)
-GD_MATRIX_MIN = 48    # shortest portions that may take them
 
 
 def _gdelta_portions(ent_host, H: int, D: int) -> int:
-    """Shortest portion of this step that runs as matrix products of chunks (0: none does).  A chunk and head holds a CU
-    (104 KB of LDS) for about 45 us, whatever its head size (padded to 64): 45 us for up to 256 of them, then 0.17 us
-    each.  What it is set against, us, other form -> matrix products:
-    a walk of 1.1 us per token of the longest portion, all heads and portions side by side: 32 tokens of 32 heads of 64
-    38 -> 46, 48 tokens 55 -> 47, 8 portions of 64 and 32 heads of 64 76 -> 66, 64 heads of 32 64 -> 107, 4 of 127 and
-    64 heads of 32 115 -> 106, 8 of 100 and 64 heads of 64 130 -> 200; so up to 6 chunks and heads per token;
-    from 128 tokens on chunks that are walked, whose cost falls with the head size: 4 portions of 1024 and 64 heads of
-    64 1705 -> 924, 64 heads of 32 643 -> 867, 64 heads of 16 709 -> 855, 32 heads of 32 432 -> 374."""
-    chunk = min(SCAN_CHUNK, LIGHT_CHUNK)
-    if chunk <= 0 or D > GD_MATRIX_MAX:
+    """``matrix_portions`` of the generalized delta rule.  A chunk and head holds a CU (104 KB of LDS) for about 45 us,
+    whatever its head size (padded to 64): 45 us for up to 256 of them, then 0.17 us each; a walk takes 1.15 us per
+    token, heads of 17 to 32 numbers 0.92.  us, walk -> matrix products: 32 tokens of 32 heads of 64 38 -> 46, 48 tokens
+    55 -> 47, 8 portions of 64 and 32 heads of 64 76 -> 66, 64 heads of 32 64 -> 107, 4 of 127 and 64 heads of 32 115 ->
+    106.  From 128 tokens on it is set against chunks that are walked, whose cost falls with the head size: 4 portions of
+    1024 and 64 heads of 64 1705 -> 924, 64 heads of 32 643 -> 867, 64 heads of 16 709 -> 855, 32 heads of 32 432 -> 374."""
+    if D > GD_MATRIX_MAX:
         return 0
-
-    def chunks(least, below):
-        return H * sum(-(-e[1] // chunk) for e in ent_host if least <= e[1] < below)
-
-    long, some = chunks(128, math.inf), chunks(GD_MATRIX_MIN, 128)
-    if D <= 32 and long > 2048:
+    if D <= 32 and H * sum(-(-e[1] // LIGHT_CHUNK) for e in ent_host if e[1] >= 128) > 2048:
         return 0
-    if some and some <= 6 * max(e[1] for e in ent_host if e[1] < 128) - 128:
-        return GD_MATRIX_MIN
-    return 128 if long else 0
+    return matrix_portions(ent_host, H, 46.0, 22.0, 0.17, 0.92 if 16 < D <= 32 else 1.15)
 
 
 def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: int, D: int,
@@ -935,9 +940,11 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
     if N > 256 or P > 256:
         raise ValueError("mamba_scan: state %d / value %d sizes above 256" % (N, P))
     E = ent.shape[0]
-    chunk, walk = _matrix_chunks(ent_host), ent
-    if chunk > 0:
-        vent, cent, walk = portion_tables(ent_host, chunk, LIGHT_MIN, zx.device)
+    # us, measured from 8 heads of 256 x 256 to 64 of 16 x 16 (``matrix_portions``)
+    walk, first = ent, 20.0 + 0.001 * N * P
+    least = matrix_portions(ent_host, H, first, first, 1.1e-5 * N * P, 3.1 if N * P > 32768 else 1.15)
+    if least > 0:
+        vent, cent, walk = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, zx.device)
         NV = vent.shape[0]
         tmp = torch.empty(NV, H, N, P, device=zx.device, dtype=torch.float32)
         decay = torch.empty(NV, H, device=zx.device, dtype=torch.float32)

@@ -156,31 +156,35 @@ def test_mamba_walks(dt, H, P, N, G, K, walks):
     test_mamba(dt, H, P, N, G, K, 0)
 
 
-@pytest.mark.parametrize("lens,H,D,form", [
-    ([47], 2, 64, "walk"), ([48, 47, 1], 2, 64, "matrix"), ([64] * 8, 33, 20, "walk"), ([64] * 8, 32, 20, "matrix"),
-    ([128] + [64] * 8, 33, 20, "matrix"), ([1100], 128, 8, "chunks"), ([1000, 3], 128, 8, "matrix"), ([130, 5], 2, 72, "chunks")])
-def test_gdelta_forms(lens, H, D, form, monkeypatch):
-    """Both sides of the lines between the walk, walked chunks and matrix products."""
+GD_FORMS = [
+    # portions, heads, head size, the form that runs first, the portions that are in it
+    ([38], 2, 64, "walk", [38]), ([40], 2, 64, "matrix", [40]), ([40, 5], 2, 32, "walk", [40, 5]),
+    ([64] * 8, 33, 40, "matrix", [64] * 8), ([64] * 8, 40, 40, "walk", [64] * 8),
+    ([100, 40, 1], 32, 64, "matrix", [100, 40, 1]), ([64, 1, 5, 1], 256, 8, "matrix", [64]),
+    ([1100], 128, 8, "chunks", [1100]), ([1000, 3], 128, 8, "matrix", [1000]), ([130, 5], 2, 72, "chunks", [130, 5])]
+
+
+@pytest.mark.parametrize("lens,H,D,form,first", GD_FORMS)
+def test_gdelta_forms(lens, H, D, form, first, monkeypatch):
+    """Both sides of the lines between the walk, walked chunks and matrix products; what is left walks."""
     ran = []
     for nm in ("p2p_sm_gdelta_scan", "p2p_sm_gdelta_scan_chunked", "p2p_sm_gdelta_chunk"):
         f = getattr(sm.lib(), nm)
         monkeypatch.setattr(sm.lib(), nm, lambda *a, f=f, nm=nm: (ran.append(nm), f(*a))[1])
     test_gdelta_long_portions(torch.float32, lens, [3 * i for i in range(len(lens))], H, D, 0.0)
-    assert ran[0] == {"walk": "p2p_sm_gdelta_scan", "chunks": "p2p_sm_gdelta_scan_chunked",
-                      "matrix": "p2p_sm_gdelta_chunk"}[form]
-    assert len(ran) == (2 if form == "matrix" and min(lens) < 48 or lens[0] == 128 else 1)
+    names = {"walk": "p2p_sm_gdelta_scan", "chunks": "p2p_sm_gdelta_scan_chunked", "matrix": "p2p_sm_gdelta_chunk"}
+    assert ran == [names[form]] + ([names["walk"]] if first != lens else [])
 
 
-@pytest.mark.parametrize("lens,starts", [([64, 1, 5, 1], [0, 9, 0, 3]), ([1, 130, 1, 70, 31], [2, 4, 7, 0, 6])])
-@pytest.mark.parametrize("scan", ["gdelta", "mamba"])
-def test_decoded_tokens_beside_prompts_form_no_chunks(lens, starts, scan, monkeypatch):
+@pytest.mark.parametrize("lens,H,P,N,first", [
+    ([31, 1], 4, 64, 128, []), ([32], 4, 64, 128, [32]), ([130, 1, 20], 4, 64, 128, [130, 20, 1]),
+    ([64, 1, 5, 1], 128, 64, 128, [64]), ([1, 130, 1, 70, 31], 128, 64, 128, [130, 70, 31])])
+def test_mamba_portions_in_chunks(lens, H, P, N, first, monkeypatch):
+    """Decoded tokens join a prompt's chunks where that is cheap and walk where it is not."""
     cut, whole = [], sm.scan_chunks
     monkeypatch.setattr(sm, "scan_chunks", lambda e, c: (cut.extend(x[1] for x in e), whole(e, c))[1])
-    if scan == "gdelta":
-        test_gdelta_long_portions(torch.float32, lens, starts, 2, 64, 0.0)
-    else:
-        test_mamba_long_portions(lens, starts, 4, 64, 128, 2, False)
-    assert sorted(cut) == sorted(n for n in lens if n >= (48 if scan == "gdelta" else 32))
+    test_mamba_long_portions(lens, [2 * i for i in range(len(lens))], H, P, N, 2, False)
+    assert sorted(cut) == sorted(first)
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
