@@ -739,6 +739,10 @@ def matrix_portions(ent_host: list, heads: int, first: float, start: float, each
     Mamba-2, all in chunks / apart: 32 heads of 16 x 64 42 / 32 us, 64 heads of 128 x 64 261 / 70; 200 tokens and 8
     portions of 20: 29 / 53 and 97 / 76).  Portions from 128 tokens on are always chunks, a step below LIGHT_MIN walks."""
     chunk = min(SCAN_CHUNK, LIGHT_CHUNK)
+    kept = getattr(ent_host, "tables", None)
+    key = (chunk, heads, first, each, token)
+    if kept is not None and key in kept:
+        return kept[key]
     lens = sorted((e[1] for e in ent_host), reverse=True)
     if chunk <= 0 or lens[0] < LIGHT_MIN:
         return 0
@@ -750,6 +754,8 @@ def matrix_portions(ent_host: list, heads: int, first: float, start: float, each
         cost = max(first, start + each * chunks * heads) + (2.0 + token * shorter if shorter else 0.0)
         if cost < best and shorter < 128:
             best, least = cost, n
+    if kept is not None:
+        kept[key] = least
     return least
 
 
@@ -1105,10 +1111,11 @@ LATENT_SPLIT_BLOCKS = 512   # split windows while a step has fewer blocks than t
 
 def _key_runs(blocks: int, most: int, tile: int) -> int:
     """Runs of keys that the windows of a step of few workgroups are cut into.  A wavefront takes runs of 64 keys, four
-    wavefronts that share key tiles runs of 256: shorter ones cost more in the merge than they gain (100 rows and 12
-    decoded ones, windows of 256, 16 heads of 128, 256 / 64 keys: 11.9 / 14.1 us), unless the step has so few
-    workgroups that its chip is mostly idle (8 rows at 500, latents of 512: 26.6 / 17.9; 16 heads of 256: 18.8 / 12.9)."""
-    run = 256 if tile and (most <= 128 or blocks * -(-most // 64) > 128) else 64
+    wavefronts that share key tiles runs of 256: shorter ones cost more in the merge than they gain (150 rows, 16 heads
+    of 128, 256 / 64 keys: 10.5 / 14.2 us, 100 rows and 12 decoded ones, windows of 256: 11.9 / 14.1), unless the windows
+    are long and the workgroups so few that the chip is mostly idle (8 rows at 500, latents of 512: 26.6 / 17.9; 16
+    heads of 256: 18.8 / 12.9; 32 rows at 300, latents of 512: 24.0 / 21.5, at 1000 27.7 / 32.6)."""
+    run = 256 if tile and (most < 256 or blocks * -(-most // 64) >= 128) else 64
     return max(1, min(-(-most // run), LATENT_SPLIT_BLOCKS // blocks, 64))
 
 

@@ -97,8 +97,8 @@ def test_group_size():
     assert [sm.attn_unit_rows(1, [(0, n, 0, 0)], 64) for n in (32, 33)] == [1, 4]     # short latents
     assert sm.attn_unit_rows(1, [(0, 16, 0, 0)], 256) == 4
     # few workgroups: runs of 64 keys; more, or short windows: of 256 where wavefronts share tiles
-    assert [sm._key_runs(16, 500, t) for t in (0, 1)] == [8, 8] and sm._key_runs(17, 500, 1) == 2
-    assert sm._key_runs(2, 128, 1) == 1 and sm._key_runs(40, 5000, 1) == 12
+    assert [sm._key_runs(15, 500, t) for t in (0, 1)] == [8, 8] and sm._key_runs(16, 500, 1) == 2
+    assert sm._key_runs(2, 255, 1) == 1 and sm._key_runs(2, 256, 1) == 4 and sm._key_runs(40, 5000, 1) == 12
     q = torch.zeros(2, 8, dtype=torch.bfloat16, device=DEV)
     z = torch.zeros(2, dtype=torch.int32, device=DEV)
     with pytest.raises(ValueError):
