@@ -14,7 +14,7 @@
 //
 // The walk of mamba_scan_k does the same 1 074 M state updates of a prompt of 2048 tokens (64 heads, 128 x 64 states)
 // twice, token after token: 240 us each, bound by the chain per token.  The matrix form does 3.7 MFLOP per chunk and
-// head: 46 + 30 + 87 us, bound by each workgroup's chain (inputs into LDS, then products) with three workgroups
+// head: 47 + 30 + 93 us, bound by each workgroup's chain (inputs into LDS, then products) with three workgroups
 // per CU; the output pass's products alone take 31 us at the card's fp32 rate.  LDS is read four numbers at a
 // time: with one number per read, C and the weights in LDS too, and one row's load in flight per thread while staging,
 // the passes took 61 + 30 + 137.
