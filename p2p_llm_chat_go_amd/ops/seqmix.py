@@ -1861,7 +1861,7 @@ def gla_scan(proj, low0: int, rank: int, wa2, za, inv_tau: float, normw, state, 
     vent = cent = cs = cd = None
     NV = 0
     matrix = max(D, V) <= GLA_MAX
-    if max(e[1] for e in ent_host) >= (GLA_MIN if matrix else 2 * SCAN_CHUNK):
+    if max(e[1] for e in ent_host) >= GLA_MIN if matrix else _chunked(ent_host):
         vent, cent = chunk_tables(ent_host, LIGHT_CHUNK if matrix else SCAN_CHUNK, proj.device)
         NV = vent.shape[0]
         cs = torch.empty(NV, H, D, V, device=proj.device, dtype=torch.float32)

@@ -236,6 +236,14 @@ def test_gla_scan(dt, H, D, V, rank, tau, step):
             assert float(d) < 0.02
 
 
+@pytest.mark.parametrize("step", sorted(STEPS))
+@pytest.mark.parametrize("H,D,V,rank,tau", [c for c in GLA if max(c[1:3]) > 128])
+def test_gla_scan_without_chunks(H, D, V, rank, tau, step, monkeypatch):
+    """A chunk size of 0: sizes that have no matrix products walk."""
+    monkeypatch.setattr(sm, "SCAN_CHUNK", 0)
+    test_gla_scan(torch.float32, H, D, V, rank, tau, step)
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("E,top,groups,keep", [(12, 2, 2, 1), (8, 3, 4, 2), (6, 1, 1, 1), (70, 5, 7, 3), (4, 4, 2, 2)])
 def test_router_rescaled(dt, E, top, groups, keep):
