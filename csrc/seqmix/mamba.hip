@@ -97,7 +97,7 @@ mamba_scan_k(const float* __restrict__ conv, int C, const T* __restrict__ zx, in
   int e = blockIdx.x / H, h = blockIdx.x % H;
   Entry en = load_entry(ent, e);
   if (en.n <= 0) return;
-  extern __shared__ float smem[];
+  extern __shared__ __align__(16) float smem[];
   const int NPAD = NS * NSUB;
   float* sB = smem;                  // [CT][NPAD]
   float* sC = sB + CT * NPAD;        // [CT][NPAD]
@@ -155,10 +155,18 @@ mamba_scan_k(const float* __restrict__ conv, int C, const T* __restrict__ zx, in
         const float* bb = sB + t * NPAD + n0;
         const float* cc = sC + t * NPAD + n0;
         float acc = 0.0f;
+        // B and C come eight rows at a time, four per read: two at a time, each waited for, the reads were most of the
+        // chain (31 tokens, 64 heads of 128 x 64 37.3 -> 26.1 us)
 #pragma unroll
-        for (int q = 0; q < NSUB; q++) {
-          S[q] = dA * S[q] + dx * bb[q];
-          acc += S[q] * cc[q];
+        for (int q0 = 0; q0 < NSUB; q0 += 8) {
+          float b[8], c[8];
+          *(float4*)b = *(const float4*)(bb + q0), *(float4*)(b + 4) = *(const float4*)(bb + q0 + 4);
+          *(float4*)c = *(const float4*)(cc + q0), *(float4*)(c + 4) = *(const float4*)(cc + q0 + 4);
+#pragma unroll
+          for (int q = 0; q < 8; q++) {
+            S[q0 + q] = dA * S[q0 + q] + dx * b[q];
+            acc += S[q0 + q] * c[q];
+          }
         }
         sy[(t * NS + ns) * P + p] = acc;
       }

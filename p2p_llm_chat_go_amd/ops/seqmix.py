@@ -948,7 +948,7 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
     E = ent.shape[0]
     # us, measured from 8 heads of 256 x 256 to 64 of 16 x 16 (``matrix_portions``)
     walk, first = ent, 20.0 + 0.001 * N * P
-    least = matrix_portions(ent_host, H, first, first, 1.1e-5 * N * P, 3.1 if N * P > 32768 else 1.15)
+    least = matrix_portions(ent_host, H, first, first, 1.3e-5 * N * P, 2.1 if N * P > 32768 else 0.8)
     if least > 0:
         vent, cent, walk = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, zx.device)
         NV = vent.shape[0]

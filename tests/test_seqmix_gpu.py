@@ -177,7 +177,7 @@ def test_gdelta_forms(lens, H, D, form, first, monkeypatch):
 
 
 @pytest.mark.parametrize("lens,H,P,N,first", [
-    ([31, 1], 4, 64, 128, []), ([32], 4, 64, 128, [32]), ([130, 1, 20], 4, 64, 128, [130, 20, 1]),
+    ([31, 1], 4, 64, 128, []), ([32], 4, 64, 128, []), ([36], 4, 64, 128, [36]), ([130, 1, 20], 4, 64, 128, [130, 20, 1]),
     ([64, 1, 5, 1], 128, 64, 128, [64]), ([1, 130, 1, 70, 31], 128, 64, 128, [130, 70, 31])])
 def test_mamba_portions_in_chunks(lens, H, P, N, first, monkeypatch):
     """Decoded tokens join a prompt's chunks where that is cheap and walk where it is not."""
