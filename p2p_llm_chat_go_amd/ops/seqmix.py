@@ -766,7 +766,7 @@ GD_MATRIX_MAX = 64    # head sizes of the matrix-instruction chunks (larger ones
 
 def _gdelta_portions(ent_host, H: int, D: int) -> int:
     """``matrix_portions`` of the generalized delta rule.  A chunk and head holds a CU (104 KB of LDS) for about 45 us,
-    whatever its head size (padded to 64): 45 us for up to 256 of them, then 0.17 us each; a walk takes 1.15 us per
+    whatever its head size (padded to 64): 46 us for up to 128 of them, 0.16 us for each one more; a walk takes 1.15 us per
     token, heads of 17 to 32 numbers 0.92.  us, walk -> matrix products: 32 tokens of 32 heads of 64 38 -> 46, 48 tokens
     55 -> 47, 8 portions of 64 and 32 heads of 64 76 -> 66, 64 heads of 32 64 -> 107, 4 of 127 and 64 heads of 32 115 ->
     106.  From 128 tokens on it is set against chunks that are walked, whose cost falls with the head size: 4 portions of
@@ -775,7 +775,7 @@ def _gdelta_portions(ent_host, H: int, D: int) -> int:
         return 0
     if D <= 32 and H * sum(-(-e[1] // LIGHT_CHUNK) for e in ent_host if e[1] >= 128) > 2048:
         return 0
-    return matrix_portions(ent_host, H, 46.0, 22.0, 0.17, 0.92 if 16 < D <= 32 else 1.15)
+    return matrix_portions(ent_host, H, 46.0, 26.0, 0.16, 0.92 if 16 < D <= 32 else 1.15)
 
 
 def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: int, D: int,
