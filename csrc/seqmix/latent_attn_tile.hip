@@ -13,15 +13,14 @@
 //
 // What bounds it: LDS reads, 32 KB for the first product and 12 KB for the second per wavefront and tile
 // at rank 512, and the copies; two workgroups fit a CU as long as a wavefront keeps to 256 registers (a
-// spill's reload would wait for the copies: 292 us instead of 128).  16 heads, rank 512, 2048 rows: 128 us
-// (540 TFLOP/s) against 704 us for latent_attn_mfma_k; a window of 1024: 84 against 490; 300 rows 26
-// against 66; 8 heads of rank 256 with the window 41 against 119.
+// spill's reload would wait for the copies: 292 us instead of 128).  16 heads, rank 512, 2048 rows: 152 us
+// (450 TFLOP/s; 133 with a maximum that lagged, see window_attn_tile.hip) against 706 us for latent_attn_mfma_k; a window
+// of 256: 45 against 184; 32 heads of rank 256 143 against 456.
 #include "attn_tile.h"
 #include "latent_attn.h"
 using namespace sm;
 
 #define LOG2E_ 1.4426950408889634f
-#define RESCALE_AT 8.0f     // powers of two
 #define NO_KEY_YET -1e30f   // running maximum of a pair that has seen no key
 
 template <int NT2>  // rank padded to NT2 * 32
@@ -150,7 +149,7 @@ latent_attn_tile_k(LatentArgs a) {
     for (int sub = 0; sub < 2; sub++)
 #pragma unroll
       for (int e = 0; e < 4; e++) tmax = fmaxf(tmax, s[sub][e]);
-    const bool rescale = __any(tmax > (fresh ? -INFINITY : RESCALE_AT));
+    const bool rescale = __any(tmax > (fresh ? -INFINITY : 0.0f));
     if (rescale) {
       tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
       tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
@@ -165,17 +164,18 @@ latent_attn_tile_k(LatentArgs a) {
     }
     if (lane == 0) sUp[wave] = rescale;
     f32x8 pw;
-    float psum = 0.0f;
+    float psum = 0.0f;   // of the weights as the product has them
 #pragma unroll
     for (int sub = 0; sub < 2; sub++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const float p = exp2_(s[sub][e]);   // 0 for keys out of sight
-        psum += p;
-        pw[sub * 4 + e] = p;
+        pw[sub * 4 + e] = exp2_(s[sub][e]);   // 0 for keys out of sight
       }
+    const bf16x8 pb = to_bf16(pw);
+#pragma unroll
+    for (int e = 0; e < 8; e++) psum += (float)pb[e];
     l_part += psum;
-    *(bf16x8*)(sP + (wave * 16 + n16) * KT + quad * 8) = to_bf16(pw);
+    *(bf16x8*)(sP + (wave * 16 + n16) * KT + quad * 8) = pb;
     __syncthreads();   // the weights are in LDS
     const int4 up4 = *(const int4*)sUp;
     const int ups[4] = {up4.x, up4.y, up4.z, up4.w};

@@ -10,8 +10,11 @@
 // is read once per 64 pairs and the wait for it is hidden by the products and the other workgroups
 // of the CU.  Per tile and wavefront:
 //   S^T[KT keys x 16 pairs] = K . Q^T     (K rows from LDS, Q in registers)
-//   online softmax in the accumulator layout; the running maximum follows only when a score passes
-//   it by more than 8 powers of two, so most tiles need no exchange between lanes and no rescaling
+//   online softmax in the accumulator layout; tiles in which no pair's maximum moves need no exchange between lanes
+//   and no rescaling.  The largest weight is one, which bf16 holds exactly, and the sum is that of the rounded weights:
+//   with a maximum that lagged by up to 2^8 and the sum of the unrounded ones, results were up to 18 % further off a
+//   64-bit run than window_attn_mfma_k's where few keys dominate (scores of deviation 3.4: 1.96e-3 against 1.74e-3, now
+//   1.72e-3; 2048 rows 48 -> 56 us)
 //   O[16 pairs x V] += P . V              (V read transposed from the same row-major tile)
 //
 // All operands of a product are read before it starts (two wavefronts per SIMD leave the registers for
@@ -19,9 +22,8 @@
 //
 // What bounds it: with plain scores the LDS reads (a wavefront reads the whole tile for 16 pairs) and
 // the copies, then the exponentials; with capped and penalised scores the exponentials and logarithms.
-// 2048 rows, 16 heads on 4, D = V = 128: 45 us (380 TFLOP/s) against 286 us for window_attn_mfma_k; capped
-// and penalised 53 against 310; a window of 1024: 32 against 169; 512 rows 14.4 against 61; 4096 rows
-// 120 (570 TFLOP/s) against 806.
+// 2048 rows, 16 heads on 4, D = V = 128: 56 us (300 TFLOP/s) against 276 us for window_attn_mfma_k; a window of 256 20
+// against 58; 32 heads on 8, D = V = 64: 62 against 264.
 //
 // Grid: one dimension, (row group, key/value head, head block) with the last row groups first (they
 // see the most keys), key/value heads innermost so that an XCD's workgroups share few heads; y:
@@ -32,7 +34,6 @@
 using namespace sm;
 
 #define LOG2E_ 1.4426950408889634f
-#define RESCALE_AT 8.0f     // powers of two
 #define NO_KEY_YET -1e30f   // running maximum of a pair that has seen no key
 
 template <int NK, int NV2, int KEYS, int MAPS, int KT>
@@ -215,6 +216,7 @@ window_attn_tile_k(WindowArgs a) {
                             : j0 + KT - 1 > p_lo || j0 <= p_hi - win;
       const int jl = j0 + quad * 4;                // this lane's places: jl + sub * 16 + i
       f32x8 pw[MAPS][NS / 2];
+      bf16x8 pf[MAPS][NS / 2];
       bf16x8 vf[NT][NS / 2];
 #pragma unroll
       for (int u = 0; u < MAPS; u++) {
@@ -289,7 +291,7 @@ window_attn_tile_k(WindowArgs a) {
         for (int sub = 0; sub < NS; sub++)
 #pragma unroll
           for (int e = 0; e < 4; e++) tmax = fmaxf(tmax, s[sub][e]);
-        if (__any(tmax > (fresh ? -INFINITY : RESCALE_AT))) {
+        if (__any(tmax > (fresh ? -INFINITY : 0.0f))) {
           tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
           tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
           const bool none = fresh && tmax == -INFINITY;
@@ -308,22 +310,21 @@ window_attn_tile_k(WindowArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; e++) acc[u][t][e] *= al[e];
         }
-        float psum = 0.0f;
+        float psum = 0.0f;   // of the weights as the product has them
 #pragma unroll
         for (int sub = 0; sub < NS; sub++)
 #pragma unroll
           for (int e = 0; e < 4; e++) {
-            const float p = exp2_(s[sub][e]);   // 0 for places out of sight
-            psum += p;
-            pw[u][sub >> 1][(sub & 1) * 4 + e] = p;
+            pw[u][sub >> 1][(sub & 1) * 4 + e] = exp2_(s[sub][e]);   // 0 for places out of sight
           }
+#pragma unroll
+        for (int hf = 0; hf < NS / 2; hf++) {
+          pf[u][hf] = to_bf16(pw[u][hf]);
+#pragma unroll
+          for (int e = 0; e < 8; e++) psum += (float)pf[u][hf][e];
+        }
         l_part[u] += psum;
       }
-      bf16x8 pf[MAPS][NS / 2];
-#pragma unroll
-      for (int u = 0; u < MAPS; u++)
-#pragma unroll
-        for (int hf = 0; hf < NS / 2; hf++) pf[u][hf] = to_bf16(pw[u][hf]);
 #pragma unroll
       for (int t = 0; t < NT; t++)
 #pragma unroll
