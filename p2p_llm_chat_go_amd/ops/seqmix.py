@@ -1109,13 +1109,14 @@ def _tiled_units(unit_rows, rows_per_wave: int) -> int:
 LATENT_SPLIT_BLOCKS = 512   # split windows while a step has fewer blocks than this
 
 
-def _key_runs(blocks: int, most: int, tile: int) -> int:
+def _key_runs(blocks: int, most: int, tile: int, few: int = 128) -> int:
     """Runs of keys that the windows of a step of few workgroups are cut into.  A wavefront takes runs of 64 keys, four
     wavefronts that share key tiles runs of 256: shorter ones cost more in the merge than they gain (150 rows, 16 heads
     of 128, 256 / 64 keys: 10.5 / 14.2 us, 100 rows and 12 decoded ones, windows of 256: 11.9 / 14.1), unless the windows
-    are long and the workgroups so few that the chip is mostly idle (8 rows at 500, latents of 512: 26.6 / 17.9; 16
-    heads of 256: 18.8 / 12.9; 32 rows at 300, latents of 512: 24.0 / 21.5, at 1000 27.7 / 32.6)."""
-    run = 256 if tile and (most < 256 or blocks * -(-most // 64) >= 128) else 64
+    are long and fewer than ``few`` workgroups with runs of 64 leave the chip mostly idle (8 rows at 500, latents of 512:
+    26.6 / 17.9; 16 heads of 256: 18.8 / 12.9; 32 rows at 300, latents of 512: 24.0 / 21.5, at 1000 27.7 / 32.6; latents of
+    96, 64 rows at 1000, 136 workgroups: 14.5 / 13.0)."""
+    run = 256 if tile and (most < 256 or blocks * -(-most // 64) >= few) else 64
     return max(1, min(-(-most // run), LATENT_SPLIT_BLOCKS // blocks, 64))
 
 
@@ -1167,7 +1168,7 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
         tile = _tiled_units(unit_rows, latent_rows_per_wave(H))
         splits = 1
         if max_keys is not None and U * hg < LATENT_SPLIT_BLOCKS:
-            splits = _key_runs(U * hg, min(max_keys, win), tile)
+            splits = _key_runs(U * hg, min(max_keys, win), tile, 160 if rank <= 128 else 128)
         part = None
         if splits > 1:
             L = lib()
@@ -1607,11 +1608,12 @@ def attn_unit_rows(rows_per_wave: int, ent_host: list, latent: int = 0) -> int:
     four times as many for the kernels whose four wavefronts share the key tiles.  Those win as
     soon as half of their rows are taken (a group of a decoded token leaves three of the four
     wavefronts idle).  ``latent``: size of a layer's latents; up to 128 they are so short that only portions of more
-    than 32 rows pay for sharing (16 heads, latents of 64, a wavefront each / shared: 16 rows 6.2 / 7.5 us, 16
-    portions of 20 6.7 / 7.7, 16 of 5 at 300 10.6 / 12.6, one of 33 7.5 / 7.5, 8 of 100 11.3 / 9.8)."""
+    than 32 rows pay for sharing, up to 64 of more than 64 (a wavefront each / shared, us: 16 heads, latents of 64, 16
+    rows 6.2 / 7.5, 16 portions of 20 6.7 / 7.7, 8 of 40 7.9 / 8.5, one of 64 7.8 / 8.4, one of 96 10.1 / 9.3, 8 of 100
+    11.5 / 10.4; 8 heads, latents of 128, 16 rows 7.7 / 8.1, 8 of 40 9.5 / 9.2)."""
     tile = 4 * rows_per_wave
     groups = sum(-(-e[1] // tile) for e in ent_host)
-    if 0 < latent <= 128 and max(e[1] for e in ent_host) <= 32:
+    if 0 < latent <= 128 and max(e[1] for e in ent_host) <= (64 if latent <= 64 else 32):
         return rows_per_wave
     return tile if 2 * sum(e[1] for e in ent_host) >= groups * tile else rows_per_wave
 

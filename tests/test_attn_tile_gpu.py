@@ -94,7 +94,8 @@ def test_group_size():
     assert sm.attn_unit_rows(4, [(0, 300, 0, 0)]) == 16       # a prompt
     assert sm.attn_unit_rows(4, [(0, 300, 0, 0)] + [(300 + i, 1, 9, i + 1) for i in range(8)]) == 16
     assert sm.attn_unit_rows(4, [(0, 7, 0, 0)]) == 4          # less than half of one group
-    assert [sm.attn_unit_rows(1, [(0, n, 0, 0)], 64) for n in (32, 33)] == [1, 4]     # short latents
+    assert [sm.attn_unit_rows(1, [(0, n, 0, 0)], 128) for n in (32, 33)] == [1, 4]    # short latents
+    assert [sm.attn_unit_rows(1, [(0, n, 0, 0)], 64) for n in (64, 65)] == [1, 4]
     assert sm.attn_unit_rows(1, [(0, 16, 0, 0)], 256) == 4
     # few workgroups: runs of 64 keys; more, or short windows: of 256 where wavefronts share tiles
     assert [sm._key_runs(15, 500, t) for t in (0, 1)] == [8, 8] and sm._key_runs(16, 500, 1) == 2
