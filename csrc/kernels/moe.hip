@@ -223,6 +223,133 @@ __global__ __launch_bounds__(256) void moe_router_logits_kernel(const bf16* __re
   }
 }
 
+// Routing of many rows (prompts above 64 rows, the all-to-all's chunks): logits, softmax, top-k and weights of 16 rows
+// per workgroup, then every local expert's slot list.  Eight wavefronts split H; the logits are one 16-column fragment on
+// the matrix cores, summed in the order of the few-row product (skinny_gemm.hip), so a row's choice does not depend on
+// how many rows there are.  One launch of that product takes 64 rows in one workgroup and 20 us, the choice of all rows
+// in one workgroup 20 us more: 700 rows of 4096 numbers took 240 us in 12 launches.
+__global__ __launch_bounds__(512) void moe_route_rows_kernel(const bf16* __restrict__ h, int ldh, int R, int H,
+                                                             const bf16x8* __restrict__ rt, float eps, int E, int K,
+                                                             int* __restrict__ topk_ids,
+                                                             float* __restrict__ topk_w) {
+  constexpr int WAVES = 8;
+  __shared__ f32x4 red[WAVES - 1][64];
+  __shared__ float red_ss[WAVES][16];
+  __shared__ float s_logit[16][17];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+  const int r0 = blockIdx.x * 16, S = H >> 5;
+  const int s0 = S * w / WAVES, s1 = S * (w + 1) / WAVES;
+  const bf16* hp = h + (size_t)min(r0 + r, R - 1) * ldh + 8 * q;
+  const bf16x8* wp = rt + lane;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float ss = 0.f;
+#pragma unroll 8
+  for (int s = s0; s < s1; ++s) {
+    const bf16x8 a = *reinterpret_cast<const bf16x8*>(hp + (size_t)s * 32);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, wp[(size_t)s * 64], acc, 0, 0, 0);
+    ss = sumsq8(a, ss);
+  }
+  ss += __shfl_xor(ss, 16, 64);
+  ss += __shfl_xor(ss, 32, 64);
+  if (w > 0) red[w - 1][lane] = acc;
+  if (q == 0) red_ss[w][r] = ss;
+  __syncthreads();
+  if (w != 0) return;
+#pragma unroll
+  for (int ww = 0; ww < WAVES - 1; ++ww) acc += red[ww][lane];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float t = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < WAVES; ++ww) t += red_ss[ww][q * 4 + j];
+    s_logit[q * 4 + j][r] = acc[j] * rsqrtf(t / (float)H + eps);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (lane >= 16 || r0 + lane >= R) return;
+  // one lane per row; the sums and choices of moe_route_kernel
+  float p[16];
+  float m = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    p[e] = s_logit[lane][e];
+    if (e < E) m = fmaxf(m, p[e]);
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e)
+    if (e < E) {
+      p[e] = __expf(p[e] - m);
+      sum += p[e];
+    }
+  unsigned taken = 0;
+  int sel[MAX_K];
+  float ws[MAX_K];
+  float wsum = 0.f;
+#pragma unroll
+  for (int k = 0; k < MAX_K; ++k) {
+    if (k >= K) break;
+    int best = -1;
+    float bv = -1.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (e < E && !(taken >> e & 1u) && p[e] > bv) {
+        bv = p[e];
+        best = e;
+      }
+    if (best >= 0) taken |= 1u << best;
+    sel[k] = best;
+    ws[k] = bv / sum;
+    wsum += ws[k];
+  }
+  const size_t slot = (size_t)(r0 + lane) * K;
+#pragma unroll
+  for (int k = 0; k < MAX_K; ++k)
+    if (k < K) {
+      topk_ids[slot + k] = sel[k];
+      topk_w[slot + k] = ws[k] / wsum;
+    }
+}
+
+// Slot lists, one workgroup per local expert, slots in ascending order: 4 slots per thread and round
+__global__ __launch_bounds__(512) void moe_lists_kernel(const int* __restrict__ topk_ids, int n, int e_lo,
+                                                        int* __restrict__ cnt, int* __restrict__ rows,
+                                                        int rows_stride) {
+  __shared__ int s_wave[2][8];
+  const int e = e_lo + blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int* list = rows + (size_t)blockIdx.x * rows_stride;
+  int at = 0, buf = 0;
+  for (int b = 0; b < n; b += 2048, buf ^= 1) {
+    const int i = b + threadIdx.x * 4;
+    bool hit[4];
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      hit[j] = i + j < n && topk_ids[i + j] == e;
+      c += hit[j];
+    }
+    int incl = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    if (lane == 63) s_wave[buf][w] = incl;
+    __syncthreads();   // the other half of s_wave is written next, so one barrier per round is enough
+    int pos = at + incl - c;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int x = s_wave[buf][v];
+      if (v < w) pos += x;
+      at += x;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (hit[j]) list[pos++] = i + j;
+  }
+  if (threadIdx.x == 0) cnt[blockIdx.x] = at;
+}
+
 // accumulate=1: h[r] += sum_k o[r*K+k] over local experts;  0: out[r] = that sum.
 __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16* __restrict__ o, int ldo_,
                                                           const int* __restrict__ topk_ids, int K,
@@ -406,6 +533,22 @@ P2P_API int p2p_moe_router_route(const void* h, int ldh, int R, int H, const voi
   }
 #undef P2P_ROUTER_CASE
   return (int)hipErrorInvalidValue;
+}
+
+// The same for any R; rt: the router padded to 16 rows, fragment-major (ops.tile_weight), H % 32 == 0, E <= 16.
+// e_local == 0: the choice only (cnt and rows are not touched).
+P2P_API int p2p_moe_route_rows(const void* h, int ldh, int R, int H, const void* rt, float eps, int E, int K, int e_lo,
+                               int e_local, int* topk_ids, float* topk_w, int* cnt, int* rows, int rows_stride,
+                               hipStream_t st) {
+  if (E <= 0 || E > 16 || K <= 0 || K > MAX_K || K > E || R <= 0 || H % 32 || ldh % 8 || ((uintptr_t)h % 16) ||
+      e_local < 0 || (e_local > 0 && rows_stride < R))
+    return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(moe_route_rows_kernel, dim3((R + 15) / 16), dim3(512), 0, st, (const bf16*)h, ldh, R, H,
+                     (const bf16x8*)rt, eps, E, K, topk_ids, topk_w);
+  if (e_local > 0)
+    hipLaunchKernelGGL(moe_lists_kernel, dim3(e_local), dim3(512), 0, st, topk_ids, R * K, e_lo, cnt, rows,
+                       rows_stride);
+  return (int)hipGetLastError();
 }
 
 // logits [R, >= E] fp32 of rstd(h) h Wr^T, one workgroup per row (prefill chunks).

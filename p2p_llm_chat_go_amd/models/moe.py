@@ -114,12 +114,8 @@ def moe_forward_tiled(model, lw, ws, R):
         m = ws.moe_big = MoeWorkspace(cfg, ws.max_rows, model.device, e_local,
                                       lw.w13.shape[1] * 16 // 2)
     h = ws.h[:R]
-    rt = router_tiled(lw)
-    for r0 in range(0, R, CHUNK):
-        rc = min(CHUNK, R - r0)
-        ops.skinny_gemm(rt, h[r0:r0 + rc], ops.EPI_F32, norm=True, out=m.logits[r0:r0 + rc],
-                        eps=cfg.eps)
-    moe_ops.moe_route(m.logits[:R], E, K, e_lo, e_local, m.topk_ids, m.topk_w, m.cnt, m.rows)
+    moe_ops.moe_route_rows(h, router_tiled(lw), E, K, m.topk_ids, m.topk_w, e_lo, e_local, m.cnt, m.rows,
+                           eps=cfg.eps)
     moe_ops.grouped_gemm(lw.w13, m.cnt, m.rows, h, K, R, ops.EPI_SILU, m.act, norm=True,
                          eps=cfg.eps)
     moe_ops.grouped_gemm(lw.w2, m.cnt, m.rows, m.act, 1, R, ops.EPI_STORE, m.o, row_w=m.topk_w)
@@ -181,16 +177,9 @@ def moe_forward_a2a(model, lw, ws, R):
         buf = ws.a2a = _Grow(dev)
     n_slots = R * K
     # routing: logits (RMSNorm folded) -> top-k ids / renormalised weights
-    logits = buf.get("logits", R, 16, torch.float32)
-    for r0 in range(0, R, CHUNK):
-        rc = min(CHUNK, R - r0)
-        ops.skinny_gemm(router_tiled(lw), h[r0:r0 + rc], ops.EPI_F32, norm=True,
-                        out=logits[r0:r0 + rc], eps=cfg.eps)
     topk_ids = buf.get("topk_ids", n_slots, None, torch.int32)
     topk_w = buf.get("topk_w", n_slots, None, torch.float32)
-    dummy_rows = buf.get("route_rows", 1, R, torch.int32)
-    dummy_cnt = buf.get("route_cnt", 1, None, torch.int32)
-    moe_ops.moe_route(logits, E, K, 0, 0, topk_ids, topk_w, dummy_cnt, dummy_rows)
+    moe_ops.moe_route_rows(h, router_tiled(lw), E, K, topk_ids, topk_w, eps=cfg.eps)
     ipc = getattr(comm, "ep_ipc", None)
     if ipc is not None and dev.type == "cuda" and ipc.fits(n_slots):
         return _a2a_ipc(model, lw, buf, ipc, h, topk_ids, topk_w, R)

@@ -111,6 +111,8 @@ _SIGS = {
                       c_void_p, c_void_p, c_int, c_void_p],
     "p2p_moe_router_route": [c_void_p, c_int, c_int, c_int, c_void_p, c_float, c_int, c_int, c_int,
                              c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+    "p2p_moe_route_rows": [c_void_p, c_int, c_int, c_int, c_void_p, c_float, c_int, c_int, c_int, c_int,
+                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "p2p_moe_a2a_dispatch": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int,
                              c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                              c_void_p],

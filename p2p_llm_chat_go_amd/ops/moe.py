@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .gemm import EPI_SILU, EPI_STORE, _ref, tiled_shape
+from .gemm import EPI_F32, EPI_SILU, EPI_STORE, _ref, tiled_shape
 
 
 def moe_route(logits, E, K, e_lo, e_local, topk_ids, topk_w, cnt, rows):
@@ -53,6 +53,27 @@ def moe_router_route(h, wr, E, K, e_lo, e_local, topk_ids, topk_w, cnt, rows, ep
                                       cnt.data_ptr(), rows.data_ptr(), rows.stride(0),
                                       _lib.stream_ptr(h.device)), "moe_router_route")
     return topk_ids, topk_w
+
+
+def moe_route_rows(h, rt, E, K, topk_ids, topk_w, e_lo=0, e_local=0, cnt=None, rows=None, eps=1e-5):
+    """Router and routing of any number of rows: logits rstd(h) * h @ Wr^T (``rt``: the router padded to 16 rows,
+    RMSNorm gain folded in, tiled by ``ops.tile_weight``), then the choice of ``moe_route`` and, with ``e_local`` > 0,
+    the slot lists, in ascending order."""
+    R, H = h.shape
+    if h.device.type != "cuda":
+        logits = _ref(rt, h, EPI_F32, True, torch.empty(R, 16), eps)
+        if not e_local:
+            cnt, rows = torch.zeros(0, dtype=torch.int32), None
+        return moe_route(logits, E, K, e_lo, e_local, topk_ids, topk_w, cnt, rows)
+    if h.dtype != torch.bfloat16 or rt.dtype != torch.bfloat16 or not rt.is_contiguous() or h.stride(1) != 1:
+        raise TypeError("moe_route_rows: h and rt must be bf16 (rt contiguous)")
+    if tiled_shape(rt) != (16, H):
+        raise ValueError("moe_route_rows: the router must be padded to 16 rows of %d" % H)
+    L = _lib.lib()
+    _lib.check(L.p2p_moe_route_rows(h.data_ptr(), h.stride(0), R, H, rt.data_ptr(), float(eps), E, K, e_lo, e_local,
+                                    topk_ids.data_ptr(), topk_w.data_ptr(), _lib.ptr(cnt), _lib.ptr(rows),
+                                    rows.stride(0) if rows is not None else 0, _lib.stream_ptr(h.device)),
+               "moe_route_rows")
 
 
 def moe_router_logits(h, wr, E, logits, eps=1e-5):

@@ -728,6 +728,33 @@ def test_moe_route_grouped_combine(R, E, K, e_lo, e_local):
     assert _rel(b[3] - h, a[3] - h) < 2e-2
 
 
+@pytest.mark.parametrize("R,E,K,e_lo,e_local,H", [(1, 8, 2, 0, 8, 4096), (16, 4, 1, 0, 4, 512), (17, 8, 2, 2, 4, 64),
+                                                   (700, 8, 2, 0, 8, 4096), (1025, 16, 8, 8, 8, 256), (90, 5, 3, 0, 0, 96)])
+def test_moe_route_rows(R, E, K, e_lo, e_local, H):
+    """Routing of many rows: the few-row product's logits bit for bit, the choice of moe_route on them, lists ascending."""
+    from p2p_llm_chat_go_amd.ops import moe as M
+
+    torch.manual_seed(R + E)
+    h = torch.randn(R, H).to(torch.bfloat16).to(DEV)
+    pad = torch.zeros(16, H, dtype=torch.bfloat16)
+    pad[:E] = (torch.randn(E, H) * 0.3).to(torch.bfloat16)
+    rt = ops.tile_weight(pad).to(DEV)
+    logits = torch.cat([ops.skinny_gemm(rt, h[r:r + 64], ops.EPI_F32, norm=True, waves=8) for r in range(0, R, 64)])
+
+    def bufs():
+        return [torch.full((R * K,), -7, dtype=torch.int32, device=DEV), torch.zeros(R * K, device=DEV),
+                torch.zeros(e_local, dtype=torch.int32, device=DEV),
+                torch.zeros(e_local, R, dtype=torch.int32, device=DEV)]
+    want, got = bufs(), bufs()
+    M.moe_route(logits, E, K, e_lo, e_local, *want)
+    M.moe_route_rows(h, rt, E, K, got[0], got[1], e_lo, e_local, *(got[2:] if e_local else ()))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2])
+    assert torch.allclose(got[1], want[1], rtol=1e-6)   # sums of the same exponentials, up to fused multiplies
+    for e in range(e_local):
+        c = int(want[2][e])
+        assert got[3][e, :c].tolist() == sorted(want[3][e, :c].tolist())
+
+
 # ------------------------------------------------------------ tiled (prefill) GEMM
 # (version, tile, splitk[, parallel split-K reduction]); split-K grids of at most one block
 # per CU with splitk | 8 take the parallel reduction unless the 4th field is 0
