@@ -33,6 +33,15 @@ __device__ __forceinline__ bf16x8 lds_rd(const bf16x8* p) {
   return v;
 }
 
+// the same from byte address `at` + OFF: reads at fixed distances share one address register
+template <int OFF>
+__device__ __forceinline__ bf16x8 lds_rd_at(unsigned at) {
+  static_assert(OFF >= 0 && OFF < 65536, "16-bit offset");
+  bf16x8 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
+  return v;
+}
+
 // wait for every outstanding LDS read; the empty asms re-define each fragment AFTER the wait,
 // so nothing that uses them can be scheduled before it
 template <int N>

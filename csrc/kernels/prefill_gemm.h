@@ -1046,8 +1046,9 @@ static __global__ __launch_bounds__(256) void row_rstd_kernel(const bf16* __rest
 // never grown while capturing (the GEMM then keeps the in-loop sums)
 static SplitWs g_rstd_ws;
 static int g_pre_rstd = 1;  // 0: always in-loop sums (A/B)
-static const float* pre_rstd(const void* X, int ldx, int M, int K, float eps, hipStream_t st) {
-  if (!g_pre_rstd || M < 128 || (ldx % 8) || (K % 8) || ((uintptr_t)X % 16)) return nullptr;
+static const float* pre_rstd(const void* X, int ldx, int M, int K, float eps, hipStream_t st,
+                             int min_rows = 128) {
+  if (!g_pre_rstd || M < min_rows || (ldx % 8) || (K % 8) || ((uintptr_t)X % 16)) return nullptr;
   const size_t bytes = (size_t)M * sizeof(float);
   if (g_rstd_ws.bytes < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

@@ -17,6 +17,7 @@
 // NORM: each thread always loads the same 4 rows at the same k offset, so it
 // accumulates their sum of squares on the fly; 3 xor-shuffles finish each row.
 #include "gemm_epilogue.h"
+#include "moe_gemm.h"
 #include "prefill_gemm.h"
 
 namespace {
@@ -317,9 +318,7 @@ P2P_API int p2p_tiled_gemm_argmax(const void* Wt, const void* X, int ldx, int M,
   return tiled_dispatch(Wt, X, ldx, M, K, N, EPI_ARGMAX, 1, keys, 0, eps, ea, stream);
 }
 
-// Grouped (MoE) expert GEMM on the LDS-tiled MFMA kernel (prefill_gemm.h, MOE mode):
-// one launch, grid (m-tiles x n-tiles, experts); see p2p_grouped_gemm for the
-// arguments.  Every expert's weights stream once per m-tile of its own rows.
+// Grouped (MoE) expert GEMM for prompts (moe_gemm.h): one launch; see p2p_grouped_gemm for the arguments.
 P2P_API int p2p_grouped_gemm_tiled(const void* Wt, long long w_stride, int n_experts,
                                    const int* cnt, const int* rows, int rows_stride, int x_div,
                                    const float* row_w, const void* X, int ldx, int max_rows,
@@ -335,28 +334,21 @@ P2P_API int p2p_grouped_gemm_tiled(const void* Wt, long long w_stride, int n_exp
   ea.row_w = row_w;
   ea.w_stride = w_stride;
   ea.n_experts = n_experts;
-  // normed (w13): the token rows' rstd once (X has max_rows rows), then the NORM = false
-  // kernel with the rstd applied per slot in the epilogue (prefill_gemm.h, pre_rstd)
-  if (norm && (epi == EPI_SILU || epi == EPI_STORE)) {
-    if (const float* r = pre_rstd(X, ldx, max_rows, K, eps, stream)) {
-      if (epi == EPI_SILU && N % 256) return (int)hipErrorInvalidValue;
-      ea.rstd_in = r;
-      return epi == EPI_SILU
-                 ? launch_moe<128, 128, EPI_SILU, false>(Wt, X, ldx, max_rows, K, N, N / 32, out,
-                                                         ldo, eps, ea, stream)
-                 : launch_moe<128, 128, EPI_STORE, false>(Wt, X, ldx, max_rows, K, N, 0, out, ldo,
-                                                          eps, ea, stream);
-    }
+  // normed (w13): the token rows' rstd once (X has max_rows rows), applied per slot at the end
+  if ((epi == EPI_SILU && norm && N % 256 == 0) || epi == EPI_STORE) {
+    if (norm) ea.rstd_in = pre_rstd(X, ldx, max_rows, K, eps, stream, 1);
+    if (!norm || ea.rstd_in)
+      return epi == EPI_SILU ? launch_moe_gemm<EPI_SILU>(Wt, X, ldx, max_rows, K, N, out, ldo, ea, stream)
+                             : launch_moe_gemm<EPI_STORE>(Wt, X, ldx, max_rows, K, N, out, ldo, ea, stream);
   }
+  // no buffer for the rstd (a capture before the first eager call): sums of squares in the k loop
   if (epi == EPI_SILU) {
     if (!norm || N % 256) return (int)hipErrorInvalidValue;
     return launch_moe<128, 128, EPI_SILU, true>(Wt, X, ldx, max_rows, K, N, N / 32, out, ldo, eps,
                                                 ea, stream);
   }
   if (epi == EPI_STORE)
-    return norm ? launch_moe<128, 128, EPI_STORE, true>(Wt, X, ldx, max_rows, K, N, 0, out, ldo,
-                                                        eps, ea, stream)
-                : launch_moe<128, 128, EPI_STORE, false>(Wt, X, ldx, max_rows, K, N, 0, out, ldo,
-                                                         eps, ea, stream);
+    return launch_moe<128, 128, EPI_STORE, true>(Wt, X, ldx, max_rows, K, N, 0, out, ldo, eps, ea,
+                                                 stream);
   return (int)hipErrorInvalidValue;
 }

@@ -755,6 +755,48 @@ def test_moe_route_rows(R, E, K, e_lo, e_local, H):
         assert got[3][e, :c].tolist() == sorted(want[3][e, :c].tolist())
 
 
+@pytest.mark.parametrize("counts,H,F", [([1, 0, 64, 65], 64, 128), ([16, 17, 129, 0, 255], 128, 256),
+                                        ([320, 321, 5], 192, 128), ([192, 700, 0, 1, 193, 256], 448, 128),
+                                        ([3] * 67, 64, 128)])
+def test_moe_grouped_tile_heights(counts, H, F):
+    """Grouped product of prompts over every tile height, K from one stage on, experts beyond a wavefront's lanes: against
+    fp32 (rounding of one bf16 result and of the SwiGLU's reciprocal: under 2^-8 of a row's largest)."""
+    from p2p_llm_chat_go_amd.ops import moe as M
+
+    E, R = len(counts), max(max(counts), 65)
+    g = torch.Generator().manual_seed(sum(counts))
+    x = torch.randn(R, H, generator=g).to(torch.bfloat16).to(DEV)
+    wn = (torch.randn(E, 2 * F, H, generator=g) * H ** -0.5).to(torch.bfloat16)
+    w2 = (torch.randn(E, 128, 64, generator=g) * 0.1).to(torch.bfloat16)
+    wt, w2t = (torch.stack([ops.tile_weight(m) for m in w]).to(DEV) for w in (wn, w2))
+    n = sum(counts)
+    slots = torch.randperm(n, generator=g).int()
+    cnt = torch.tensor(counts, dtype=torch.int32, device=DEV)
+    rows = torch.full((E, R), -1, dtype=torch.int32)
+    o = 0
+    for e, c in enumerate(counts):
+        rows[e, :c] = slots[o:o + c]
+        o += c
+    rd, xd = rows.to(DEV), (n + R - 1) // R
+    act = torch.full((n, F), float("nan"), dtype=torch.bfloat16, device=DEV)
+    M.grouped_gemm(wt, cnt, rd, x, xd, R, ops.EPI_SILU, act, norm=True)
+    y = torch.randn(n, 64, generator=g).to(torch.bfloat16).to(DEV)
+    tw = torch.rand(n, generator=g).to(DEV)
+    out = torch.full((n, 128), float("nan"), dtype=torch.bfloat16, device=DEV)
+    M.grouped_gemm(w2t, cnt, rd, y, 1, R, ops.EPI_STORE, out, row_w=tw)
+    xf = x.float()
+    xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5)
+    for e, c in enumerate(counts):
+        if not c:
+            continue
+        s = rows[e, :c].long().to(DEV)
+        z = xf[s // xd] @ wn[e].float().to(DEV).T
+        ref = torch.nn.functional.silu(z[:, :F]) * z[:, F:]
+        assert (act[s].float() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
+        ref = (y[s].float() @ w2[e].float().to(DEV).T) * tw[s][:, None]
+        assert (out[s].float() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
+
+
 # ------------------------------------------------------------ tiled (prefill) GEMM
 # (version, tile, splitk[, parallel split-K reduction]); split-K grids of at most one block
 # per CU with splitk | 8 take the parallel reduction unless the 4th field is 0
