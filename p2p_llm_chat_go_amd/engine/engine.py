@@ -340,7 +340,6 @@ class Engine:
             last[r[0]] = j
         g.load(g.host_meta(rows, block_tables, last))
         if sampled:
-            g.samp._key = None  # the native loop may have written these slots directly
             g.samp.load(list(sampling))
         g.replay()
         return g.first[:B]

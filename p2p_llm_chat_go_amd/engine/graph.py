@@ -21,6 +21,7 @@ import torch
 
 from .. import ops
 from ..ops import PAGE
+from .sampling import HostImage, SamplerSlots
 
 
 class DecodeState:
@@ -32,18 +33,18 @@ class DecodeState:
         self.max_pages = max_pages
         self.max_steps = max_steps
         self.max_ctx = max_ctx
-        # ids | pos | ctx | slots | block tables: views of ONE device buffer, so `load`
+        # ids | pos | ctx | slots | block tables | step: views of ONE device buffer, so `load`
         # refreshes a batch's whole state with one host->device copy
-        self.meta = torch.zeros(B * (4 + max_pages), device=dev, dtype=i32)
+        n = B * (4 + max_pages)
+        state = torch.zeros(n + 1, device=dev, dtype=i32)
+        self.meta, self.step = state[:n], state[n:]
+        self.image = HostImage(state)
         self.ids, self.pos, self.ctx, self.slots = (self.meta[k * B:(k + 1) * B] for k in range(4))
         self.bt = self.meta[4 * B:].view(B, max_pages)
         self.ctx.fill_(1)
         self.row_bt = torch.arange(B, device=dev, dtype=i32)
         self.hist = torch.zeros(B, max_steps, device=dev, dtype=i32)
-        self.step = torch.zeros(1, device=dev, dtype=i32)
         self.ws = model.new_workspace(B, max_ctx)
-        from .sampling import SamplerSlots
-
         self.samp = SamplerSlots(B, dev)  # sampled graphs read these (ops.sample)
         if model.tp > 1:  # vocab-parallel sampling: per-shard top-128 candidates, gathered
             W = model.tp
@@ -64,20 +65,20 @@ class DecodeState:
     def load(self, ids, pos, block_tables):
         """ids/pos: int lists (n <= B); block_tables: list of page lists."""
         n = len(ids)
-        B = self.B
+        B, P = self.B, self.max_pages
         assert n <= B
-        self.step.zero_()
         self.ws.keys.zero_()
-        host = torch.zeros(B * (4 + self.max_pages), dtype=torch.int32)
-        bt = host[4 * B:].view(B, self.max_pages)
+        host = self.image.fill()   # rows >= n: dummies (page 0, position 0)
+        host[:] = 0
+        bt = host[4 * B:4 * B + B * P].reshape(B, P)
         for b, pages in enumerate(block_tables):
-            bt[b, :len(pages)] = torch.tensor(pages, dtype=torch.int32)
+            bt[b, :len(pages)] = pages
         p = host[B:2 * B]
-        p[:n] = torch.tensor(pos, dtype=torch.int32)
-        host[:n] = torch.tensor(ids, dtype=torch.int32)
+        p[:n] = pos
+        host[:n] = ids
         host[2 * B:3 * B] = p + 1
-        host[3 * B:4 * B] = bt.gather(1, (p // PAGE).long()[:, None])[:, 0] * PAGE + p % PAGE
-        self.meta.copy_(host, non_blocking=True)  # rows >= n: dummies (page 0, position 0)
+        host[3 * B:4 * B] = bt[np.arange(B), p // PAGE] * PAGE + p % PAGE
+        self.image.send()
 
     def body_logits(self):
         """Forward only (sampling mode): logits of every row in ws.logits."""
@@ -246,7 +247,7 @@ class DecodeGraph:
 
     def step_sampled(self, params: list, n: int = 1):
         """n decode steps with per-row SamplingParams (temperature <= 0 rows stay greedy):
-        the parameters are loaded into device slots (only when they change), then each
+        the parameters are loaded into device slots, then each
         step is one replay -- forward, ops.sample and advance are all in the graph."""
         assert not self.greedy
         self.state.samp.load(params)
@@ -298,6 +299,7 @@ class PrefillGraph:
             self.offsets[name] = (o, n)
             o += n
         self.meta = torch.zeros(o, device=dev, dtype=torch.int32)
+        self.image = HostImage(self.meta)
         v = {name: self.meta[a:a + n] for name, (a, n) in self.offsets.items()}
         self.bt = v["bt"].view(S + 1, max_pages)
         self.seq, self.pos, self.ids, self.slots, self.ctx = (v[k] for k in ("seq", "pos", "ids",
@@ -308,8 +310,6 @@ class PrefillGraph:
         self.first = torch.zeros(S, device=dev, dtype=torch.int32)
         self.samp = None
         if not greedy:  # per-sequence sampling parameters, read by the captured ops.sample
-            from .sampling import SamplerSlots
-
             self.samp = SamplerSlots(S, dev)
             if model.tp > 1:  # vocab-parallel draw: top-128 per shard, one all-gather
                 W = model.tp
@@ -364,7 +364,8 @@ class PrefillGraph:
         return torch.from_numpy(host)
 
     def load(self, host: torch.Tensor):
-        self.meta.copy_(host, non_blocking=True)
+        self.image.fill()[:] = host.numpy()
+        self.image.send()
 
     # ------------------------------------------------------------------ device side
     def body(self):

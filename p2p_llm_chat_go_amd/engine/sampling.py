@@ -50,29 +50,58 @@ class SamplingParams:
                    stop_on_eos=not bool(o.get("ignore_eos", False)))
 
 
+class HostImage:
+    """Page-locked host image of a device buffer that is filled anew for every step.  From pageable memory a copy
+    is a staging round trip of some 35 us that the host waits for; from here it is queued like a launch.  The
+    image is written again only once its last copy has been read (``fill`` waits for that)."""
+
+    def __init__(self, dev: torch.Tensor):
+        self.dev = dev
+        cuda = dev.device.type == "cuda"
+        self.host = torch.zeros(dev.shape, dtype=dev.dtype, pin_memory=cuda)
+        self.sent = torch.cuda.Event() if cuda else None
+        self.busy = False
+
+    def fill(self):
+        """The image as a numpy array, free to be written."""
+        if self.busy:
+            self.sent.synchronize()
+            self.busy = False
+        return self.host.numpy()
+
+    def send(self):
+        self.dev.copy_(self.host, non_blocking=True)
+        if self.sent is not None:
+            self.sent.record(torch.cuda.current_stream(self.dev.device))
+            self.busy = True
+
+
+_PADDING = (0.0, 40, 0.9, 0)   # a row no sequence has: greedy, and the same in every step
+
+
 class SamplerSlots:
     """Per-row sampling parameters of a decode batch as device tensors, read by the
     graph-captured ``ops.sample`` launch (so a sampled decode step replays like a
-    greedy one).  ``load`` copies only when the batch's parameters change."""
+    greedy one): views of one buffer, which ``load`` fills with one copy (each time: the native loop writes them too)."""
 
     def __init__(self, B: int, device):
         self.B = B
-        self.temp = torch.zeros(B, device=device, dtype=torch.float32)
-        self.topk = torch.full((B,), 40, device=device, dtype=torch.int32)
-        self.topp = torch.full((B,), 0.9, device=device, dtype=torch.float32)
-        self.seeds = torch.zeros(B, device=device, dtype=torch.int64)
-        self._key = None
+        o = (3 * B + 1) // 2 * 2   # the seeds' 64-bit words after three 32-bit ones per row
+        self.buf = torch.zeros(o + 2 * B, device=device, dtype=torch.int32)
+        self.image = HostImage(self.buf)
+        (self.temp, self.topk, self.topp, self.seeds), self.parts = (
+            (v[:B].view(torch.float32), v[B:2 * B], v[2 * B:3 * B].view(torch.float32), v[o:].view(torch.int64))
+            for v in (self.buf, self.image.host))
+        self.load([])
 
     def load(self, params: list):
-        params = list(params[:self.B]) + [SamplingParams()] * (self.B - len(params))
-        key = tuple((p.temperature, p.top_k, p.top_p, p.resolved_seed()) for p in params)
-        if key == self._key:
-            return
-        self.temp.copy_(torch.tensor([k[0] for k in key], dtype=torch.float32))
-        self.topk.copy_(torch.tensor([k[1] for k in key], dtype=torch.int32))
-        self.topp.copy_(torch.tensor([k[2] for k in key], dtype=torch.float32))
-        self.seeds.copy_(torch.tensor([k[3] for k in key], dtype=torch.int64))
-        self._key = key
+        params = params[:self.B]
+        rows = [(p.temperature, p.top_k, p.top_p, p.resolved_seed()) for p in params]
+        rows += [_PADDING] * (self.B - len(rows))
+        self.image.fill()
+        for view, col in zip(self.parts, zip(*rows)):
+            view.numpy()[:] = col
+        self.image.send()
 
 
 def sample(logits: torch.Tensor, params: list, pos) -> torch.Tensor:
