@@ -75,6 +75,11 @@ __device__ __forceinline__ void dma_lds(const void* g, const void* l) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(m0)
                  : "memory", "m0");
 }
+// the same with a wave-uniform address and a lane's byte offset from it, to LDS byte address l (wave-uniform)
+__device__ __forceinline__ void dma_lds16(const void* base, unsigned off, unsigned l) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(l)
+               : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // a streamed (non-temporal) 16-byte global load into registers, counted like the DMAs

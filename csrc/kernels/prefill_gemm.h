@@ -42,7 +42,7 @@ struct SplitArgs {
   f32x4* slab;         // [tiles][splitk][FM*FN][NT] partial accumulators
   float* ss_slab;      // [tiles][splitk][BM] partial row sums of squares
   unsigned* counters;  // [tiles], zeroed before the launch
-  // parallel reduction (every slice reduces 8/splitk of the tile's waves; all slices of a
+  // parallel reduction (every slice reduces its part of the tile's fragment rows; all slices of a
   // tile must be resident together -- the host enables it only for grids <= the CU count):
   unsigned* gen;       // [tiles] generation, bumped by each tile's last arriver
   int* err;            // set if a slice waited past the spin bound (results invalid)
@@ -104,27 +104,58 @@ __device__ __forceinline__ void wait_tiles(int pending) {
   wait_vmcnt<0>();
 }
 
+// an address that is the same for all lanes, in scalar registers
+__device__ __forceinline__ const char* wave_address(const void* p) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+  return reinterpret_cast<const char*>((uint64_t)hi << 32 | lo);
+}
+
+// scalar arguments that are to be in registers from here on
+template <typename T>
+__device__ __forceinline__ void pin_scalar(const T& v) {
+  asm volatile("" ::"s"(v));
+}
+template <typename... T>
+__device__ __forceinline__ void pin_scalars(const T&... v) {
+  (pin_scalar(v), ...);
+}
+
 // MOE: grouped expert GEMM (ea.moe_*): blockIdx.y = local expert e, whose rows are the
 // slots rows[e][i] (i < min(cnt[e], M)); A row of slot s = X[s / x_div], output row s
 // (scaled by row_w[s]).  m-tiles past the expert's count exit at once, so one launch
 // covers every expert at any M and each expert's weights stream once per m-tile.
-template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, bool MOE = false>
-__global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
+//
+// NWV = 4 (128-row tiles): four wavefronts of 64 x BN/2 instead of eight of 64 x 32, each the only one on its SIMD.  Eight
+// in step read a half stage, waited, multiplied it, and issued the copies between: 1900 cycles per stage for 512 cycles
+// of products.  Four read the next half stage under the products of the present one, and issue their copies (a
+// scalar address and a lane's constant offset) between the products: 1440 cycles.  Reads ahead alone gave 1600; a fifth
+// wavefront that touched the lines of stages further ahead, so that copies find them in the L2, nothing.
+template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, bool MOE = false, int NWV = 8>
+__global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
                                                           const bf16* __restrict__ X, int ldx,
                                                           int M, int K, int m_tiles, int n_tiles,
                                                           int up_off, void* __restrict__ out,
                                                           int ldo, float eps, EpiArgs ea,
                                                           SplitArgs sp) {
-  constexpr int FM = BM / 32;        // 16-row fragments per wave (2 x 4 wave grid)
-  constexpr int FN = BN / 64;        // 16-col groups per wave
+  constexpr bool PIPE = NWV == 4;
+  constexpr int NT = NWV * 64;
+  constexpr int WN = NWV / 2;        // 2 x WN wave grid
+  constexpr int FM = BM / 32;        // 16-row fragments per wave
+  constexpr int FN = BN / (16 * WN);  // 16-col groups per wave
   constexpr int AB = BM / 16 * 2;    // A fragment blocks per stage (x 1 KiB)
   constexpr int BB = BN / 16 * 2;    // B fragment blocks per stage
   constexpr int STAGE = (AB + BB) * 64;  // bf16x8 per stage
-  constexpr int AI = AB / 8, BI = BB / 8;  // blocks per wave per stage
+  constexpr int AI = AB / NWV, BI = BB / NWV;  // blocks per wave per stage
   constexpr int L = AI + BI;               // LDS-DMA instructions per thread per stage
-  static_assert(AB % 8 == 0 && BB % 8 == 0, "tile");
+  static_assert(AB % NWV == 0 && BB % NWV == 0, "tile");
+  static_assert(!PIPE || (STAGES >= 3 && !MOE), "the stage after the present one is read ahead");
   static_assert(FM >= 1 && FN >= 2, "tile");
-  __shared__ __attribute__((aligned(16))) bf16x8 lds[STAGES * STAGE];
+  // PIPE: given at the launch.  A static 160 KiB tells the compiler that one wavefront per SIMD is all there can be, and it
+  // moves the accumulators through AGPRs, four copies per product
+  extern __shared__ __attribute__((aligned(16))) bf16x8 lds_given[];
+  __shared__ __attribute__((aligned(16))) bf16x8 lds_own[PIPE ? 1 : STAGES * STAGE];
+  bf16x8* lds = PIPE ? lds_given : lds_own;
 
   const int splitk = SPLIT ? sp.splitk : 1;
   const int nb = m_tiles * n_tiles * splitk;
@@ -147,7 +178,7 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
   // 12-22 % of the GEMM, profiles/r2_norm_cost.jsonl); applied in the epilogue
   const bool pre = !NORM && ea.rstd_in != nullptr;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 2, wn = w & 3;
+  const int wm = w / WN, wn = w % WN;
   const int S = K >> 5;
   const int nk_all = K / BK;
   const int kt0 = split * nk_all / splitk, kt1 = (split + 1) * nk_all / splitk;
@@ -165,17 +196,19 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
   const bf16* asrc[AI];
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
-    const int blk = w + 8 * i;  // = mi * 2 + ks
+    const int blk = w + NWV * i;  // = mi * 2 + ks
     const int mi = blk >> 1, ks = blk & 1;
     int row = m0 + 16 * mi + (lane & 15);
+    // PIPE: 8 rows x 128 bytes per block, 16-byte chunks of row R permuted by R & 7 (see the phased kernel)
+    if constexpr (PIPE) row = m0 + 8 * blk + (lane >> 3);
     row = row < M ? row : M - 1;
     if constexpr (MOE) row = mrows[row] / ea.x_div;
-    asrc[i] = X + (size_t)row * ldx + 32 * ks + 8 * (lane >> 4);
+    asrc[i] = X + (size_t)row * ldx + (PIPE ? 8 * ((lane & 7) ^ (lane >> 3)) : 32 * ks + 8 * (lane >> 4));
   }
   const bf16x8* bsrc[BI];
 #pragma unroll
   for (int i = 0; i < BI; ++i) {
-    const int blk = w + 8 * i;  // = gi * 2 + ks
+    const int blk = w + NWV * i;  // = gi * 2 + ks
     bsrc[i] = Wt + ((size_t)group_of(blk >> 1) * S + (blk & 1)) * 64 + lane;
   }
 
@@ -184,9 +217,9 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
   auto issue = [&](int kt, int st) {
     bf16x8* base = lds + st * STAGE;
 #pragma unroll
-    for (int i = 0; i < AI; ++i) ldsp::dma_lds<16>(asrc[i] + kt * BK, base + (w + 8 * i) * 64);
+    for (int i = 0; i < AI; ++i) ldsp::dma_lds<16>(asrc[i] + kt * BK, base + (w + NWV * i) * 64);
 #pragma unroll
-    for (int i = 0; i < BI; ++i) ldsp::dma_lds<16>(bsrc[i] + (size_t)kt * 2 * 64, base + (AB + w + 8 * i) * 64);
+    for (int i = 0; i < BI; ++i) ldsp::dma_lds<16>(bsrc[i] + (size_t)kt * 2 * 64, base + (AB + w + NWV * i) * 64);
   };
 
   int bgi[FN];
@@ -211,37 +244,135 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
 
   // ---- STAGES-deep LDS-DMA pipeline: counted vmcnt + raw barriers, so the
   // younger stages stay in flight across the barrier (no vmcnt(0) drain) ----
+  if constexpr (!PIPE)
 #pragma unroll
-  for (int t = 0; t < STAGES - 1; ++t)
-    if (t < n) issue(kt0 + t, t);
-  for (int t = 0; t < n; ++t) {
-    wait_tiles<L, STAGES>(min(STAGES - 2, n - 1 - t));  // tile t landed (this thread's part)
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();                       // ... and every other wave's part
-    if (t + STAGES - 1 < n) issue(kt0 + t + STAGES - 1, (t + STAGES - 1) % STAGES);
-    const bf16x8* sa = lds + (t % STAGES) * STAGE;
-    const bf16x8* sb = sa + AB * 64;
+    for (int t = 0; t < STAGES - 1; ++t)
+      if (t < n) issue(kt0 + t, t);
+  if constexpr (PIPE) {
+    // copies: a wave-uniform address per stage, a lane's offset that stays
+    const char* abase = wave_address(X + (size_t)m0 * ldx + (size_t)kt0 * BK);
+    constexpr int HALF = EPI == EPI_SILU ? BI / 2 : BI;   // SwiGLU: a wave's first copies are gate columns, the rest up
+    constexpr int TILE_GROUPS = EPI == EPI_SILU ? BN / 32 : BN / 16;
+    static_assert(EPI != EPI_SILU || BI % 2 == 0, "halves");
+    const char* bbase = wave_address(Wt + ((size_t)nt_i * TILE_GROUPS * S + (size_t)kt0 * 2) * 64);
+    const size_t to_up = EPI == EPI_SILU ? (size_t)up_off * S * 1024 : 0;
+    unsigned aoff[AI], boff[BI];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 af[FM], bfr[FN];
+    for (int i = 0; i < AI; ++i) aoff[i] = (unsigned)((const char*)asrc[i] - reinterpret_cast<const char*>(X + (size_t)m0 * ldx));
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bfr[j] = ldsp::lds_rd(sb + (bgi[j] * 2 + ks) * 64 + lane);
+    for (int i = 0; i < BI; ++i)
+      boff[i] = (unsigned)((const char*)(bsrc[i] + (size_t)kt0 * 128) - bbase - (i < HALF ? 0 : to_up));
+    const unsigned lds0 = ldsp::lds_off(lds) + __builtin_amdgcn_readfirstlane(w) * 1024;
+    auto copy = [&](int i, int t) {   // the i-th of this wave's L copies of stage t
+      const unsigned l = lds0 + (t % STAGES) * (STAGE * 16) + (i < AI ? i : AB / NWV + i - AI) * (NWV * 1024);
+      if (i < AI) ldsp::dma_lds16(abase + (size_t)t * (BK * 2), aoff[i < AI ? i : 0], l);
+      else ldsp::dma_lds16(bbase + (i - AI < HALF ? 0 : to_up) + (size_t)t * 2048, boff[i < AI ? 0 : i - AI], l);
+    };
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = ldsp::lds_rd(sa + ((wm * FM + i) * 2 + ks) * 64 + lane);
-      ldsp::lds_wait(af, bfr);
-      // keep the MFMA cluster together against the co-resident wave (guide T5)
-      __builtin_amdgcn_s_setprio(1);
+    for (int t = 0; t < STAGES - 1; ++t)
+      if (t < n)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < L; ++i) copy(i, t);
+    // (LDS reads as plain loads: the copies are asm, so the compiler waits for exactly what a product needs)
+    const int ar = (wm * FM * 16 + (lane & 15)) * 8, aq = lane >> 4, ax = lane & 7;
+    auto read = [&](int t, int ks, bf16x8(&af)[FM], bf16x8(&bfr)[FN]) {
+      const bf16x8* sa = lds + (t % STAGES) * STAGE;
+      const bf16x8* sb = sa + AB * 64 + lane;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) af[i] = sa[ar + i * 128 + ((4 * ks + aq) ^ ax)];
+#pragma unroll
+      for (int j = 0; j < FN; ++j) bfr[j] = sb[(bgi[j] * 2 + ks) * 64];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // between(i): what is issued behind the products of fragment row i
+    auto products = [&](const bf16x8(&af)[FM], const bf16x8(&bfr)[FN], auto&& between) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
 #pragma unroll
         for (int j = 0; j < FN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_s_setprio(0);
-      if constexpr (NORM) {  // RMSNorm sums: fragment i by wave wn == i % 4 (VALU spread)
+        __builtin_amdgcn_sched_barrier(0);
+        between(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (NORM) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          if ((i & 3) != wn) continue;
-          ss[i] = sumsq8(af[i], ss[i]);
+        for (int i = 0; i < FM; ++i)
+          if (i % WN == wn) ss[i] = sumsq8(af[i], ss[i]);
+      }
+    };
+    auto nothing = [](int) {};
+    auto meet = [] {
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");   // (the barrier alone does not order reads of LDS)
+    };
+    bf16x8 a0[FM], b0[FN], a1[FM], b1[FN];
+    // stages 0 .. STAGES - 2 are under way; stage 0 alone has to be there
+    wait_tiles<L, STAGES>(min(STAGES - 2, n - 1));
+    meet();
+    // the epilogue's arguments are loaded now, and lgkmcnt(0) is seen by the compiler: with a scalar load under way where
+    // the loop begins it waits for all LDS reads before each product
+    pin_scalars(out, ldo, eps, ea.rstd_in);
+    if constexpr (EPI == EPI_QKV_ROPE)
+      pin_scalars(ea.pos, ea.slots, ea.cs, ea.q_out, ea.ldq, ea.kc, ea.vc, ea.Hq, ea.Hkv);
+    if constexpr (EPI == EPI_ARGMAX) pin_scalars(ea.col_offset);
+    if constexpr (SPLIT) pin_scalars(sp.splitk, sp.slab, sp.ss_slab, sp.counters, sp.gen, sp.err, sp.parallel);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    read(0, 0, a0, b0);
+    int t = 0;
+    for (; t + STAGES - 1 < n; ++t) {
+      read(t, 1, a1, b1);
+      products(a0, b0, nothing);
+      wait_vmcnt<(STAGES - 3) * L>();   // stage t + 1 is there, for every wave once they met
+      meet();
+      read(t + 1, 0, a0, b0);
+      // the slot of the stage that is copied held stage t - 1, whose reads every wave had used up before it met the others
+      products(a1, b1, [&](int i) {
+#pragma unroll
+        for (int c = i * L / FM; c < (i + 1) * L / FM; ++c) copy(c, t + STAGES - 1);
+      });
+    }
+    for (; t + 1 < n; ++t) {
+      read(t, 1, a1, b1);
+      products(a0, b0, nothing);
+      wait_tiles<L, STAGES - 1>(min(STAGES - 3, n - 2 - t));
+      meet();
+      read(t + 1, 0, a0, b0);
+      products(a1, b1, nothing);
+    }
+    read(t, 1, a1, b1);
+    products(a0, b0, nothing);
+    products(a1, b1, nothing);
+  } else {
+    for (int t = 0; t < n; ++t) {
+      wait_tiles<L, STAGES>(min(STAGES - 2, n - 1 - t));  // tile t landed (this thread's part)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();                       // ... and every other wave's part
+      if (t + STAGES - 1 < n) issue(kt0 + t + STAGES - 1, (t + STAGES - 1) % STAGES);
+      const bf16x8* sa = lds + (t % STAGES) * STAGE;
+      const bf16x8* sb = sa + AB * 64;
+  #pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        bf16x8 af[FM], bfr[FN];
+  #pragma unroll
+        for (int j = 0; j < FN; ++j) bfr[j] = ldsp::lds_rd(sb + (bgi[j] * 2 + ks) * 64 + lane);
+  #pragma unroll
+        for (int i = 0; i < FM; ++i) af[i] = ldsp::lds_rd(sa + ((wm * FM + i) * 2 + ks) * 64 + lane);
+        ldsp::lds_wait(af, bfr);
+        // keep the MFMA cluster together against the co-resident wave (guide T5)
+        __builtin_amdgcn_s_setprio(1);
+  #pragma unroll
+        for (int i = 0; i < FM; ++i)
+  #pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        if constexpr (NORM) {  // RMSNorm sums: fragment i by wave wn == i % 4 (VALU spread)
+  #pragma unroll
+          for (int i = 0; i < FM; ++i) {
+            if ((i & 3) != wn) continue;
+            ss[i] = sumsq8(af[i], ss[i]);
+          }
         }
       }
     }
@@ -254,7 +385,7 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
   if constexpr (NORM) {
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      if ((i & 3) != wn) continue;
+      if (i % WN != wn) continue;
       float v = ss[i];
       v += __shfl_xor(v, 16, 64);
       v += __shfl_xor(v, 32, 64);
@@ -270,7 +401,8 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
   }
   // ---- epilogue of one wave's accumulators (wave grid position wm_, wn_) ----
   const int r = lane & 15, q = lane >> 4;
-  auto epilogue = [&](int wm_, int wn_, const f32x4 (&ac)[FM][FN], auto&& scale_of) {
+  // (fragment rows i0 .. i1 - 1)
+  auto epilogue = [&](int wm_, int wn_, const f32x4 (&ac)[FM][FN], auto&& scale_of, int i0, int i1) {
     int bg[FN];
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
@@ -283,6 +415,7 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
     }
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
+      if (i < i0 || i >= i1) continue;
       // one fragment row's epilogue operands as one batch (residual values; the rows'
       // positions -> (cos, sin) and KV slots): per element, between the stores they may
       // alias, they were FN x 4 dependent round trips per fragment row
@@ -374,8 +507,8 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
     // registers for the shared reduction would spill its main loop)
     if (BM * BN <= 128 * 256 && sp.parallel) {
       // ---- parallel split-K: write-through slabs, one generation flip per tile, then
-      // every slice reduces and stores 8/splitk of the tile's waves (no serial reducer,
-      // no release fence) ----
+      // every slice reduces and stores its part of the tile (no serial reducer, no release
+      // fence) ----
       const __amdgpu_buffer_rsrc_t rsl = raw_rsrc(sp.slab);
       const size_t tile_v = (size_t)tile * splitk * (FM * FN) * NT;  // f32x4 index of slice 0
 #pragma unroll
@@ -407,10 +540,14 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
         }
       }
       __syncthreads();
-      constexpr int kWavesPerTile = NT / 64;
-      const int vw_n = kWavesPerTile / splitk;  // host guarantees splitk | 8
-      if (w >= vw_n) return;
-      const int vw = split * vw_n + w;  // the tile wave whose accumulators this wave finishes
+      // the tile's NWV * FM fragment rows go to the slices in equal runs (host guarantees splitk | 8), and a slice's
+      // run to its waves in shares that lie within one wave's rows
+      const int units = NWV * FM / splitk;
+      int share = (units + NWV - 1) / NWV;
+      while (FM % share || units % share) ++share;
+      if (w * share >= units) return;
+      const int unit = split * units + w * share;
+      const int vw = unit / FM, i0 = unit % FM, i1 = i0 + share;  // whose accumulators this wave finishes
       // acc is dead after the slab stores: it becomes the total (one fragment row of
       // loads in flight at a time keeps the 256x256 tile inside its register budget)
 #pragma unroll
@@ -420,6 +557,7 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
       for (int s2 = 0; s2 < splitk; ++s2) {
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
+          if (i < i0 || i >= i1) continue;
           f32x4 part[FN];
 #pragma unroll
           for (int j = 0; j < FN; ++j)
@@ -429,15 +567,18 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
           for (int j = 0; j < FN; ++j) acc[i][j] += part[j];
         }
       }
-      epilogue(vw >> 2, vw & 3, acc, [&](int i, int jj) {
-        const int rl = (vw >> 2) * (BM / 2) + 16 * i + 4 * q + jj;
-        if constexpr (!NORM) return rstd_pre(rl);
-        float t = 0.f;
-        for (int s2 = 0; s2 < splitk; ++s2)
-          t += __hip_atomic_load(&sp.ss_slab[((size_t)tile * splitk + s2) * BM + rl],
-                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return rstd_of(t);
-      });
+      epilogue(
+          vw / WN, vw % WN, acc,
+          [&](int i, int jj) {
+            const int rl = (vw / WN) * (BM / 2) + 16 * i + 4 * q + jj;
+            if constexpr (!NORM) return rstd_pre(rl);
+            float t = 0.f;
+            for (int s2 = 0; s2 < splitk; ++s2)
+              t += __hip_atomic_load(&sp.ss_slab[((size_t)tile * splitk + s2) * BM + rl],
+                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return rstd_of(t);
+          },
+          i0, i1);
       return;
     }
     // ---- serial split-K: agent-scope release/acquire through a per-tile ticket; every
@@ -491,11 +632,14 @@ __global__ __launch_bounds__(NT) void prefill_gemm_kernel(const bf16x8* __restri
     if (tid == 0) sp.counters[tile] = 0;
   }
 
-  epilogue(wm, wn, acc, [&](int i, int jj) {
-    const int rl = wm * (BM / 2) + 16 * i + 4 * q + jj;
-    if constexpr (!NORM) return rstd_pre(rl);
-    return rstd_of(ss_row[rl]);
-  });
+  epilogue(
+      wm, wn, acc,
+      [&](int i, int jj) {
+        const int rl = wm * (BM / 2) + 16 * i + 4 * q + jj;
+        if constexpr (!NORM) return rstd_pre(rl);
+        return rstd_of(ss_row[rl]);
+      },
+      0, FM);
 }
 
 // ---------------------------------------------------------------------------------
@@ -824,12 +968,25 @@ static int cu_count() {
   return cached[dev] > 0 ? cached[dev] : 0;
 }
 
+// Wavefronts of a tile shape: four (prefill_gemm_kernel, NWV) where a workgroup has 128 rows and a CU to itself
+template <int BM, int BN>
+constexpr int waves_for() {
+  return BM == 128 && BN <= 192 ? 4 : 8;
+}
+
+// (128 x 192 leaves no registers for a reduction)
+template <int BM, int BN>
+constexpr bool splits_k() {
+  return BN != 192;
+}
+
 // LDS stages per tile shape.  Measured on MI355X (bench/prefill_gemm_bench.py): the
 // 64-row tiles are latency-bound streams and want 3-4 stages in flight; the 128/256-row
 // tiles are MFMA-bound at large M, where two blocks share a CU and hide each other's
 // loads, and lose more to 1-block/CU occupancy than they gain from depth.
 template <int BM, int BN>
 constexpr int stages_for() {
+  if constexpr (waves_for<BM, BN>() == 4) return (160 * 1024) / ((BM + BN) * BK * 2);
   if constexpr (BM >= 128) return 2;
   return BN <= 128 ? 4 : 3;
 }
@@ -842,7 +999,7 @@ constexpr int stages_for() {
 // (profiles/r2_prefill_gemm_deep_stages.jsonl): deep applies from 128 rows.
 template <int BM, int BN>
 constexpr int deep_stages_for() {
-  if constexpr (BM < 128) return stages_for<BM, BN>();
+  if constexpr (BM < 128 || waves_for<BM, BN>() == 4) return stages_for<BM, BN>();
   constexpr int stage_bytes = (BM + BN) * BK * 2;
   constexpr int most = (160 * 1024) / stage_bytes;
   return most > 6 ? 6 : (most < 2 ? 2 : most);
@@ -856,27 +1013,35 @@ template <int BM, int BN, int EPI, bool NORM, int STAGES>
 int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_tiles, int n_tiles,
                   int up_off, void* out, int ldo, float eps, const EpiArgs& ea, hipStream_t st,
                   int splitk, char* ws, int par) {
+  constexpr int NWV = waves_for<BM, BN>();
+  constexpr size_t SHM = NWV == 4 ? (size_t)STAGES * (BM + BN) * BK * sizeof(bf16) : 0;
   const int tiles = m_tiles * n_tiles;
-  if (splitk > 1) {
-    constexpr int FM = BM / 32, FN = BN / 64;
-    const size_t slab = (size_t)tiles * splitk * FM * FN * NT * sizeof(f32x4);
-    // counters live at the END of the workspace at a fixed offset from the end so a
-    // grown workspace keeps them zeroed; see split_ws.  Layout of that region (u32):
-    // [0, n/2) arrival tickets, [n/2, n-1) generations, [n-1] the fault word.
-    unsigned* ctr = (unsigned*)(ws + g_split_ws.bytes - kCounterBytes);
-    constexpr size_t nw = kCounterBytes / sizeof(unsigned);
-    int* fw = p2p_split_fault_word_ptr(st);
-    SplitArgs sp{splitk, (f32x4*)ws, (float*)(ws + slab), ctr, ctr + nw / 2,
-                 fw ? fw : (int*)(ctr + nw - 1), par};
-    hipLaunchKernelGGL((prefill_gemm_kernel<BM, BN, EPI, NORM, true, STAGES>),
-                       dim3(tiles * splitk), dim3(NT), 0, st, (const bf16x8*)Wt,
-                       (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, sp);
-    return (int)hipGetLastError();
+  auto with_lds = [](const void* k) {
+    return SHM ? hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SHM) : hipSuccess;
+  };
+  if constexpr (splits_k<BM, BN>()) {
+    if (splitk > 1) {
+      constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, true, STAGES, false, NWV>;
+      if (const hipError_t e = with_lds((const void*)kernel)) return (int)e;
+      const size_t slab = (size_t)tiles * splitk * BM * BN * sizeof(float);
+      // counters live at the END of the workspace at a fixed offset from the end so a
+      // grown workspace keeps them zeroed; see split_ws.  Layout of that region (u32):
+      // [0, n/2) arrival tickets, [n/2, n-1) generations, [n-1] the fault word.
+      unsigned* ctr = (unsigned*)(ws + g_split_ws.bytes - kCounterBytes);
+      constexpr size_t nw = kCounterBytes / sizeof(unsigned);
+      int* fw = p2p_split_fault_word_ptr(st);
+      SplitArgs sp{splitk, (f32x4*)ws, (float*)(ws + slab), ctr, ctr + nw / 2,
+                   fw ? fw : (int*)(ctr + nw - 1), par};
+      hipLaunchKernelGGL(kernel, dim3(tiles * splitk), dim3(NWV * 64), SHM, st, (const bf16x8*)Wt,
+                         (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, sp);
+      return (int)hipGetLastError();
+    }
   }
   SplitArgs none{1, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-  hipLaunchKernelGGL((prefill_gemm_kernel<BM, BN, EPI, NORM, false, STAGES>), dim3(tiles), dim3(NT), 0,
-                     st, (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off,
-                     out, ldo, eps, ea, none);
+  constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, false, STAGES, false, NWV>;
+  if (const hipError_t e = with_lds((const void*)kernel)) return (int)e;
+  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(NWV * 64), SHM, st, (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles,
+                     n_tiles, up_off, out, ldo, eps, ea, none);
   return (int)hipGetLastError();
 }
 
@@ -890,7 +1055,8 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
   const int tiles = m_tiles * n_tiles;
   const int nk = K / BK;
   const int cus = cu_count();
-  const bool deep_auto = DEEP > SHALLOW && g_deep == 1 && cus > 0 && tiles <= cus;
+  constexpr int NWV = waves_for<BM, BN>();   // four: one workgroup per CU whatever the grid
+  const bool deep_auto = (DEEP > SHALLOW || NWV == 4) && g_deep == 1 && cus > 0 && tiles <= cus;
   // too few tiles to fill 256 CUs: split K so every CU gets work (>= 4 k-tiles per slice)
   // (measured on MI355X at 8B shapes: ~400 blocks, >= 16 k-tiles per slice); the deep
   // variant keeps the grid at one block per CU instead (power-of-two slices <= CUs/tiles)
@@ -904,12 +1070,11 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
   } else {
     splitk = std::min(8, std::max(1, std::min(400 / tiles, nk / 16)));
   }
-  splitk = std::max(1, std::min(splitk, nk / 4));
+  splitk = splits_k<BM, BN>() ? std::max(1, std::min(splitk, nk / 4)) : 1;
   char* ws = nullptr;
   int par = 0;
   if (splitk > 1 && (size_t)tiles * sizeof(unsigned) < kCounterBytes / 2) {
-    constexpr int FM = BM / 32, FN = BN / 64;
-    const size_t slab = (size_t)tiles * splitk * FM * FN * NT * sizeof(f32x4);
+    const size_t slab = (size_t)tiles * splitk * BM * BN * sizeof(float);
     const size_t ssb = (size_t)tiles * splitk * BM * sizeof(float);
     if (!(split_ws(slab + ssb, st, &ws) && slab + ssb < 0x7FFFFFFF)) splitk = 1;
     par = g_split_parallel && (8 % splitk) == 0 && cus > 0 && tiles * splitk <= cus;
@@ -967,47 +1132,43 @@ int launch_tile(int tile, const void* Wt, const void* X, int ldx, int M, int K, 
     case 6: return launch<320, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 7: return launch<192, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 8: return launch<192, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
+    case 9:
+      if constexpr (EPI != EPI_SILU)   // (gate and up of 14336 columns do not divide by 96)
+        return launch<128, 192, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
   }
   return (int)hipErrorInvalidValue;
 }
 
 // Largest tile that still gives about one block per CU; N must divide.  M <= 64
-// uses the 64-row tiles (no MFMA work or DMA on padding rows beyond one tile).
-// 129-192 and 257-320 rows (batched chat prompts: 8 peers x ~36-44 tokens) take ONE
-// m-tile of 192 / 320 rows: at these M the tiles are bound by the per-CU LDS-DMA fill
-// rate, so the bytes staged per useful output decide, and 128-row tiles would stream
-// every weight column 2-3 times (25 % padding) while 256x256 pads up to 44 %.
-static int g_tile8 = 1;  // the 192 x 256 gate_up pick below (A/B switch: p2p_prefill_tile8)
+// uses the 64-row tiles (no MFMA work or DMA on padding rows beyond one tile).  128-row tiles run on four
+// wavefronts that read ahead (prefill_gemm_kernel, NWV).  llama3.1-8B, cold weights, us, eight wavefronts in step (and
+// the tiles of 192 and 320 rows picked beside them) / now: o 128 rows 29 / 22, 400 rows 41 / 33, 1024 rows 64 / 50;
+// down 43 / 37, 101 / 75, 186 / 135 (890 TFLOP/s); qkv 27 / 24, 54 / 39, 95 / 55.  What is left there is each
+// wavefront's own chain: a wait for all wavefronts per 64 numbers of K beside 512 cycles of products.
+static int g_tile8 = 1;  // the 192 x 256 gate_up picks below (A/B switch: p2p_prefill_tile8)
 static int pick_tile(int M, int N, int K) {
   if (M <= 64) return N % 128 == 0 ? 4 : 0;
   // (one-m-tile 384 / 448-row tiles for 321-448 rows measured 1.1-1.3x SLOWER than the
   // 128x128 split-K / phased 256x256 picks below and were removed:
   // profiles/r3_prefill_tiles_384_448.jsonl)
-  // (257-320 rows: the one-m-tile 320x128 pays on the wide gate_up only; o_proj at 288 rows
-  // took 64 us with it and 39 with 128x128 split-K, cold weights:
-  // profiles/r5_prefill_gemm_cold_vs_hipblaslt.jsonl)
-  // (129-192 rows, N <= 4096 with K <= 4096 -- o_proj: 32 one-m-tile tiles take split-K 4 at
-  // most, 128 blocks; 128 x 128 split-K 4 fills the 256 CUs: 30.8 vs 37.7 us for llama3.1-8B
-  // o_proj at 192 rows, cold weights, profiles/r6_prefill_gemm_sweep_cold.jsonl)
-  const bool short_k = N <= 4096 && K <= 4096;
-  if (N % 128 == 0 && ((M > 128 && M <= 192 && !short_k) || (M > 256 && M <= 320 && N >= 16384)))
-    return M <= 192 ? 7 : 6;
-  // qkv-width projections (4096 < N <= 8192) in the 384-row bucket (8 peers x ~44-token
-  // prompts): 192 x 128 tiles, split-K 2 by launch()'s rule -- llama3.1-8B qkv+RoPE 49.2 vs
-  // 57.0 us with 128 x 128 (144 tiles on 256 CUs, unsplit), cold weights
-  // (profiles/r6_prefill_gemm_384_cold.jsonl); o_proj / down (N = 4096) and gate_up measured
-  // best on their picks below
-  if (N % 128 == 0 && M > 320 && M <= 384 && N > 4096 && N <= 8192) return 7;
-  // SwiGLU-width projections (N >= 16384: gate_up) in the 384-row bucket: 192 x 256 tiles (2 x
-  // N/256, no padding rows) instead of the phased 256 x 256 (384 -> 512 rows): 2-8 us faster
-  // per launch in every round of an order-balanced A/B (bench/tile_ab.py,
-  // profiles/r6_tile_ab_gate_up_384.jsonl)
-  if (g_tile8 && N % 256 == 0 && M > 320 && M <= 384 && N >= 16384) return 8;
+  if (N >= 16384) {
+    // SwiGLU-width projections (gate_up of llama3.1-8B, us, cold weights).  129-192 rows: one m-tile of 192 rows,
+    // 78 beside 80 with 128 x 128.  257-384 and 513-768 rows: 192 x 256 tiles waste fewer rows than the phased
+    // 256 x 256: 288 rows 106 / 112 (320 x 128: 112), 352 rows 107 / 108, 600 rows 195 / 204, 768 rows 198 / 208;
+    // 416 rows 193 / 115, 896 rows 278 / 217
+    if (N % 128 == 0 && M > 128 && M <= 192) return 7;
+    if (g_tile8 && N % 256 == 0 && ((M > 256 && M <= 384) || (M > 512 && M <= 768))) return 8;
+  }
   const int cand[3][3] = {{1, 256, 256}, {2, 128, 256}, {3, 128, 128}};
   int best = 0;
+  const long cus = cu_count() > 0 ? cu_count() : 256, rows128 = (M + 127) / 128;
   for (auto& c : cand) {
     if (N % c[2]) continue;
     const long blocks = (long)((M + c[1] - 1) / c[1]) * (N / c[2]);
+    // 128 x 192 where it takes one round of the CUs and 128 x 128 two: qkv of llama3.1-8B at 700 and 1024 rows
+    // 49 and 53 us beside 71 and 78 (128 x 256: 78 and 80); where 128 x 128 takes one round it is the faster one
+    // (512 rows 42 beside 49)
+    if (c[0] != 1 && N % 192 == 0 && rows128 * (N / 192) <= cus && N % 128 == 0 && rows128 * (N / 128) > cus) return 9;
     if (!best) best = c[0];
     // the phased 256x256 kernel pays from ~160 tiles (profiles/r2_prefill_gemm_phased.jsonl)
     if (blocks >= (c[0] == 1 ? 160 : 200)) return c[0];
@@ -1079,7 +1240,7 @@ static int prefill_dispatch(const void* Wt, const void* X, int ldx, int M, int K
   using namespace pgemm;
   if (M <= 0 || K % BK) return (int)hipErrorInvalidValue;
   int tile = g_prefill_tile ? g_prefill_tile : pick_tile(M, N, K);
-  const int bn = (tile == 3 || tile == 4 || tile == 6 || tile == 7) ? 128 : 256;
+  const int bn = (tile == 3 || tile == 4 || tile == 6 || tile == 7) ? 128 : tile == 9 ? 192 : 256;
   if (!tile || N % bn) return (int)hipErrorInvalidValue;
   const int up_off = (epi == EPI_SILU) ? N / 32 : 0;
   // normed projections from 128 rows: rstd by row_rstd_kernel, GEMM without in-loop sums

@@ -850,6 +850,47 @@ def test_tiled_gemm(M, epi, tiled_cfg):
     assert _rel(out.cpu(), ref) < 1e-2
 
 
+@pytest.mark.parametrize("epi", ["store", "store_norm", "resid", "f32", "silu"])
+@pytest.mark.parametrize("tile,splitk,nk", [(t, 1, n) for t in (3, 9) for n in (1, 2, 3, 4, 5, 6, 11)] +
+                         [(3, 2, 9), (3, 4, 17), (3, 8, 33), (3, 3, 12)])
+def test_tiled_gemm_read_ahead(epi, tile, splitk, nk):
+    """128-row tiles on four wavefronts: K from one stage to more than the ring holds, rows that fill a tile and that do
+    not, K slices of uneven length, against fp32 (rounding of one bf16 result: 2^-8 of the largest)."""
+    from p2p_llm_chat_go_amd.ops.gemm import set_tiled_min_m, tiled_config
+
+    if tile == 9 and epi == "silu":
+        pytest.skip("not built")
+    K, N = 64 * nk, 768
+    g = torch.Generator().manual_seed(nk * 10 + splitk)
+    W = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    Wt = ops.tile_weight(W).to(DEV)
+    tiled_config(2, tile, splitk)
+    set_tiled_min_m(1)
+    try:
+        for M in (1, 127, 128, 257):
+            x = torch.randn(M, K + 64, generator=g).to(torch.bfloat16)[:, :K]   # rows with a gap
+            acc = x.float() @ W.float().t()
+            xd = x.to(DEV) if M == 1 else torch.empty(M, K + 64, dtype=torch.bfloat16, device=DEV)[:, :K].copy_(x)
+            if epi in ("store_norm", "silu", "f32"):
+                acc = acc * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)
+            if epi == "resid":
+                h = torch.randn(M, N, generator=g).to(torch.bfloat16)
+                out = ops.skinny_gemm(Wt, xd, ops.EPI_RESID, out=h.to(DEV))
+                acc = acc + h.float()
+            elif epi == "silu":
+                out = ops.skinny_gemm(Wt, xd, ops.EPI_SILU, norm=True)
+                acc = torch.nn.functional.silu(acc[:, :N // 2]) * acc[:, N // 2:]
+            elif epi == "f32":
+                out = ops.skinny_gemm(Wt, xd, ops.EPI_F32, norm=True)
+            else:
+                out = ops.skinny_gemm(Wt, xd, ops.EPI_STORE, norm=epi == "store_norm")
+            bound = 1e-5 if epi == "f32" else 2 ** -8
+            assert (out.float().cpu() - acc).abs().max() <= bound * acc.abs().max(), M
+    finally:
+        set_tiled_min_m(65)
+        tiled_config(2, 0, 0)
+
+
 @pytest.mark.parametrize("deep", [0, 2])
 @pytest.mark.parametrize("splitk", [1, 4])
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
