@@ -227,7 +227,7 @@ def lib():
 
 
 def _st(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.stream_ptr(t.device)
 
 
 def _f32(t) -> int:
