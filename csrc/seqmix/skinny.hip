@@ -86,89 +86,6 @@ __global__ void __launch_bounds__(512) skinny_k(SkinnyArgs a) {
     if (quad * 4 + e < a.M) stf((T*)a.y, (size_t)(quad * 4 + e) * a.N + n, acc[e] + b);
 }
 
-// The same for the rows of a short prompt, bf16: a workgroup takes 32 rows x 64 columns, its eight wavefronts the K index
-// 128 bytes at a time in turn, straight from memory into fragments, two such pieces in flight; each finishes one of the
-// eight 16 x 16 parts.
-//
-// A short prompt is bound by the host: a vendor product costs it 22 us (the library looks its kernel up at each call), this
-// one 5, and a pass has 22 to 25 of them.  The kernel itself is bound by what a CU can take in (some 40 KB/us): 64 rows,
-// 1024 x 1024 7.8 us (library 6.6), 8192 x 1024 8.5 (9.0), 2048 x 2048 13.3 (8.9), 10272 x 2048 28.7 (14.3).
-// `_rows` in ops/seqmix.py draws the line.
-__global__ void __launch_bounds__(512) rows_k(SkinnyArgs a) {
-  typedef bf16 T;
-  constexpr int WAVES = 8, MT = 2, NT = 4;
-  constexpr int EP = 16 / sizeof(T), KB = 8 * EP;   // numbers per fragment, per 128 bytes
-  __shared__ f32x4 red[WAVES][MT * NT][64];
-  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6), n16 = lane & 15, quad = lane >> 4;
-  const int n0 = blockIdx.x * 64, m0 = blockIdx.y * 32, K = a.K;
-  // rows that do not exist are the last ones, their results are dropped
-  const T *xp[MT], *wp[NT];
-#pragma unroll
-  for (int t = 0; t < MT; t++) xp[t] = (const T*)a.x + (size_t)min(m0 + t * 16 + n16, a.M - 1) * a.ldx + quad * EP;
-#pragma unroll
-  for (int t = 0; t < NT; t++) wp[t] = (const T*)a.w + (size_t)min(n0 + t * 16 + n16, a.N - 1) * K + quad * EP;
-  f32x4 acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; i++)
-#pragma unroll
-    for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  uint4 av[2][2][MT], bv[2][2][NT];
-  auto load = [&](int k, uint4 (&A)[2][MT], uint4 (&B)[2][NT]) {   // a piece past K is zero
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-      const int at = k + s * 4 * EP;
-      const bool in = at + quad * EP < K;
-      const int o = in ? at : -quad * EP;
-#pragma unroll
-      for (int t = 0; t < NT; t++) B[s][t] = *(const uint4*)(wp[t] + o);
-#pragma unroll
-      for (int t = 0; t < MT; t++) A[s][t] = *(const uint4*)(xp[t] + o);
-      if (!in) {
-#pragma unroll
-        for (int t = 0; t < NT; t++) B[s][t] = make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < MT; t++) A[s][t] = make_uint4(0, 0, 0, 0);
-      }
-    }
-  };
-  const int kb = wave * KB, step = WAVES * KB;
-#pragma unroll
-  for (int d = 0; d < 2; d++)
-    if (kb + d * step < K) load(kb + d * step, av[d], bv[d]);
-  for (int k0 = kb; k0 < K; k0 += 2 * step) {
-#pragma unroll
-    for (int d = 0; d < 2; d++) {
-      const int k = k0 + d * step;
-      if (k < K) {
-#pragma unroll
-        for (int s = 0; s < 2; s++)
-#pragma unroll
-          for (int i = 0; i < MT; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j++) acc[i][j] = mfma_frag<T>(av[d][s][i], bv[d][s][j], acc[i][j]);
-        if (k + 2 * step < K) load(k + 2 * step, av[d], bv[d]);
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < MT; i++)
-#pragma unroll
-    for (int j = 0; j < NT; j++) red[wave][i * NT + j][lane] = acc[i][j];
-  __syncthreads();
-  // eight 16 x 16 parts, one per wavefront
-  const int i = wave / NT, n = n0 + (wave % NT) * 16 + n16;
-  f32x4 s = red[0][wave][lane];
-#pragma unroll
-  for (int w = 1; w < WAVES; w++) s += red[w][wave][lane];
-  if (n >= a.N) return;
-  const float b = a.bias ? ldf((const T*)a.bias, n) : 0.0f;
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const int m = m0 + i * 16 + quad * 4 + e;
-    if (m < a.M) stf((T*)a.y, (size_t)m * a.N + n, s[e] + b);
-  }
-}
-
 extern "C" {
 
 // x rows are ldx numbers apart and, like w, aligned to 16 bytes; y [M, N] is packed
@@ -179,15 +96,6 @@ int p2p_sm_skinny(const void* x, int ldx, const void* w, const void* bias, void*
   if (M > 16 || K < ep || K % ep || ldx % ep || (size_t)x % 16 || (size_t)w % 16) return (int)hipErrorInvalidValue;
   const SkinnyArgs a = {x, w, bias, y, ldx, M, N, K};
   SM_DISPATCH_T(f32, hipLaunchKernelGGL((skinny_k<T>), dim3((N + 15) / 16), dim3(512), 0, st, a));
-  return (int)hipGetLastError();
-}
-
-// the same arguments, any number of rows, bf16
-int p2p_sm_rows(const void* x, int ldx, const void* w, const void* bias, void* y, int M, int N, int K, hipStream_t st) {
-  if (M <= 0 || N <= 0) return 0;
-  if (M > 65535 * 32 || K < 8 || K % 8 || ldx % 8 || (size_t)x % 16 || (size_t)w % 16) return (int)hipErrorInvalidValue;
-  const SkinnyArgs a = {x, w, bias, y, ldx, M, N, K};
-  hipLaunchKernelGGL(rows_k, dim3((N + 63) / 64, (M + 31) / 32), dim3(512), 0, st, a);
   return (int)hipGetLastError();
 }
 

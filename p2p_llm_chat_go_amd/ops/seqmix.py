@@ -51,7 +51,6 @@ _SIGS = {
                                             c_int, c_float, c_int, c_void_p],
     "p2p_sm_skinny": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                       c_void_p],
-    "p2p_sm_rows": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "p2p_sm_gdelta_chunk": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                                     c_void_p, c_int, c_void_p, c_int, c_int, c_int,
@@ -332,37 +331,15 @@ def _skinny(x, w) -> bool:
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def _rows(x, w) -> bool:
-    """Products of 17 rows and more that ``rows_k`` (``csrc/seqmix/skinny.hip``) takes from the library: those that cost
-    the GPU no more over the library's kernel than the host saves by not asking for one, 17 us.  One round of the CUs with
-    rows of up to 2048 numbers (7 to 13 us beside 5 to 9), two with up to 1024 (15 beside 9 to 11).  Whole prompts of 20 /
-    100 / 256 / 512 tokens, us, library -> this: Regesun, width 1024, 8 layers 1147 -> 868, 1229 -> 981, 1268 -> 1113,
-    1332 -> 1205, width 2048 1132 -> 919, 1246 -> 1167, 1269 -> 1217, 1412 -> 1393; Rasepel 1193 -> 895, 1322 -> 1119,
-    1336 -> 1192, 1409 -> 1310; without the bound on K and rounds, width 2048, 256 tokens 1205 -> 1557.  In a captured
-    graph the host costs nothing and the library's kernels are the faster ones."""
-    M, K = x.shape
-    N = w.shape[0]
-    tiles = (N + 63) // 64 * ((M + 31) // 32)
-    return (x.dtype == torch.bfloat16 and K <= 2048 and tiles <= (512 if K <= 1024 else 256) and x.is_cuda and w.is_cuda
-            and w.dtype == x.dtype and w.shape[1] == K and x.stride(1) == 1 and w.is_contiguous() and K >= 8
-            and K % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and not (x.requires_grad or w.requires_grad) and not torch.cuda.is_current_stream_capturing())
-
-
 def linear(x, w, b=None):
     """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, the shapes of ``_skinny`` on a
-    kernel for few rows, those of ``_rows`` on one for short prompts."""
-    if x.dim() != 2 or (b is not None and not (b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
-        return F.linear(x, w, b)
-    few = x.shape[0] <= 16
-    if not (_skinny(x, w) if few else _rows(x, w)):
+    kernel for few rows."""
+    if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
+            b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
         return F.linear(x, w, b)
     y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
-    at = (x.data_ptr(), x.stride(0), w.data_ptr(), _lib.ptr(b), y.data_ptr(), x.shape[0], w.shape[0], x.shape[1])
-    if few:
-        _chk(lib().p2p_sm_skinny(*at, _f32(x), _st(x)), "skinny")
-    else:
-        _chk(lib().p2p_sm_rows(*at, _st(x)), "rows")
+    _chk(lib().p2p_sm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), _lib.ptr(b), y.data_ptr(), x.shape[0],
+                             w.shape[0], x.shape[1], _f32(x), _st(x)), "skinny")
     return y
 
 

@@ -323,42 +323,3 @@ def test_glu_act_by_width(dt, F, off, act):
     res = [sm.glu_act(gu.to(d)[:, off:off + 2 * F], torch.zeros(3, F + 4, dtype=dt, device=d)[:, :F], act).cpu()
            for d in ("cpu", DEV)]
     torch.testing.assert_close(res[1], res[0], **_tol(dt))
-
-
-@pytest.mark.parametrize("K", [8, 56, 64, 520, 1024, 1032, 2048])
-@pytest.mark.parametrize("M,N", [(17, 1), (31, 64), (32, 65), (33, 2048), (100, 96), (255, 130)])
-def test_linear_of_short_prompts(M, N, K):
-    """``sm.linear`` on ``rows_k`` (tails of its 32 x 64 tiles and of its pieces of K, rows with a gap, a bias) against fp32:
-    one rounding of the result, 2^-8 of a row's largest; a row that is not finite stays by itself."""
-    g = torch.Generator().manual_seed(M * 7 + N + K)
-    x = torch.randn(M, K + 8, generator=g).bfloat16().to(DEV)[:, :K]
-    w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
-    b = torch.randn(N, generator=g).bfloat16().to(DEV)
-    assert sm._rows(x, w)
-    ref = x.double() @ w.double().T
-    for bias in (None, b):
-        want = ref if bias is None else ref + bias.double()
-        got = sm.linear(x, w, bias).double()
-        assert ((got - want).abs() <= 2 ** -8 * want.abs() + 1e-5 * ref.abs().amax(1, keepdim=True)).all()
-    y = sm.linear(x, w)
-    x[M // 2, K - 1] = float("inf")
-    z = sm.linear(x, w)
-    keep = torch.arange(M, device=DEV) != M // 2
-    assert torch.equal(z[keep], y[keep]) and not torch.isfinite(z[M // 2]).all()
-
-
-def test_linear_under_capture_and_with_gradients_is_the_librarys():
-    x = torch.randn(64, 1024, device=DEV).bfloat16()
-    w = torch.randn(256, 1024, device=DEV).bfloat16()
-    assert sm._rows(x, w) and not sm._rows(x.clone().requires_grad_(), w)
-    want = torch.nn.functional.linear(x, w)   # (and the library's workspace, before the capture)
-    g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
-        assert not sm._rows(x, w)
-        y = sm.linear(x, w)
-    for _ in range(3):
-        x.normal_()
-        want = torch.nn.functional.linear(x, w)
-        g.replay()
-        torch.cuda.synchronize()
-        assert torch.equal(y, want)
