@@ -20,6 +20,34 @@ template <> __device__ __forceinline__ void stf<bf16>(bf16* p, size_t i, float v
   p[i] = __float2bfloat16(v);
 }
 
+// VE neighbours (1, or 4 at an address that is a multiple of their size)
+template <int VE, typename T>
+__device__ __forceinline__ void ldv(const T* p, size_t i, float* v) {
+  if constexpr (VE == 1) {
+    v[0] = ldf(p, i);
+  } else if constexpr (sizeof(T) == 4) {
+    const float4 q = *(const float4*)(p + i);
+    v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+  } else {
+    const uint2 q = *(const uint2*)(p + i);
+    v[0] = __uint_as_float(q.x << 16), v[1] = __uint_as_float(q.x & 0xffff0000u);
+    v[2] = __uint_as_float(q.y << 16), v[3] = __uint_as_float(q.y & 0xffff0000u);
+  }
+}
+template <int VE, typename T>
+__device__ __forceinline__ void stv(T* p, size_t i, const float* v) {
+  if constexpr (VE == 1) {
+    stf(p, i, v[0]);
+  } else if constexpr (sizeof(T) == 4) {
+    *(float4*)(p + i) = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+    bf16 o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) stf(o, j, v[j]);
+    *(uint2*)(p + i) = __builtin_bit_cast(uint2, o);
+  }
+}
+
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float softplusf_(float x) {
   return fmaxf(x, 0.0f) + log1pf(expf(-fabsf(x)));

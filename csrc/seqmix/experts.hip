@@ -632,20 +632,25 @@ expert_gemm_fma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restri
 
 // out[r] = sum_k wts[r, k] * y[r * top + k]; a slot whose expert index is >= n_real (ids given)
 // stands for an expert that hands its input back: its term is wts * x[r]
-template <typename T>
+// VE channels per thread (2048 rows of 2048, two experts each, one / four: 12.8 / 7.4 us)
+template <typename T, int VE>
 __global__ void expert_combine_k(const T* __restrict__ y, int ldy, const float* __restrict__ wts,
                                  T* __restrict__ out, int ldo, int top, int n,
                                  const int* __restrict__ ids, int n_real, const T* __restrict__ x,
                                  int ldx) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
+  int c = (blockIdx.x * blockDim.x + threadIdx.x) * VE, r = blockIdx.y;
   if (c >= n) return;
-  float s = 0.0f;
+  float s[VE];
+#pragma unroll
+  for (int j = 0; j < VE; j++) s[j] = 0.0f;
   for (int k = 0; k < top; k++) {
     bool same = ids && ids[r * top + k] >= n_real;
-    float v = same ? ldf(x, (size_t)r * ldx + c) : ldf(y, (size_t)(r * top + k) * ldy + c);
-    s += wts[r * top + k] * v;
+    float v[VE];
+    ldv<VE>(same ? x : y, same ? (size_t)r * ldx + c : (size_t)(r * top + k) * ldy + c, v);
+#pragma unroll
+    for (int j = 0; j < VE; j++) s[j] += wts[r * top + k] * v[j];
   }
-  stf(out, (size_t)r * ldo + c, s);
+  stv<VE>(out, (size_t)r * ldo + c, s);
 }
 
 extern "C" {
@@ -725,9 +730,15 @@ int p2p_sm_expert_combine(const void* y, int ldy, const float* wts, void* out, i
                           int f32, hipStream_t st) {
   if (R <= 0) return 0;
   if (ids && !x) return (int)hipErrorInvalidValue;
-  dim3 g((n + 255) / 256, R), b(256);
-  SM_DISPATCH_T(f32, hipLaunchKernelGGL(expert_combine_k<T>, g, b, 0, st, (const T*)y, ldy, wts,
-                                         (T*)out, ldo, top, n, ids, n_real, (const T*)x, ldx));
+  const size_t al = f32 ? 16 : 8;
+#define COMBINE(VE)                                                                                                  \
+  SM_DISPATCH_T(f32, hipLaunchKernelGGL((expert_combine_k<T, VE>), dim3((n + 256 * VE - 1) / (256 * VE), R), dim3(256), \
+                                         0, st, (const T*)y, ldy, wts, (T*)out, ldo, top, n, ids, n_real, (const T*)x, ldx))
+  if (n % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && ((size_t)y | (size_t)out) % al == 0 &&
+      (!ids || (ldx % 4 == 0 && (size_t)x % al == 0)))
+    COMBINE(4);
+  else COMBINE(1);
+#undef COMBINE
   return (int)hipGetLastError();
 }
 

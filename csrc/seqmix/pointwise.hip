@@ -11,16 +11,22 @@ __global__ void tanh_k(T* x, int ld, int n, int R) {
   if (c < n) stf(x, (size_t)r * ld + c, tanhf(ldf(x, (size_t)r * ld + c)));
 }
 
-// out[r, h * V + v] = o[h * soh + r * sor + v] * sigmoid(g[r * ldg + h * V + v])
-template <typename T>
+// out[r, h * V + v] = o[h * soh + r * sor + v] * sigmoid(g[r * ldg + h * V + v]); VE channels per thread (2048 rows of
+// 2048, one / four: 10.1 / 6.8 us)
+template <typename T, int VE>
 __global__ void sigmoid_gate_k(const T* __restrict__ o, long soh, long sor, const T* __restrict__ g,
                                int ldg, T* __restrict__ out, int ldo, int H, int V,
                                int per_head) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
+  int c = (blockIdx.x * blockDim.x + threadIdx.x) * VE, r = blockIdx.y;
   if (c >= H * V) return;
   int h = c / V, v = c % V;
-  float x = ldf(o, (size_t)h * soh + (size_t)r * sor + v);
-  stf(out, (size_t)r * ldo + c, x * sigmoidf_(ldf(g, (size_t)r * ldg + (per_head ? h : c))));
+  float x[VE], z[VE];
+  ldv<VE>(o, (size_t)h * soh + (size_t)r * sor + v, x);
+  if (per_head) z[0] = ldf(g, (size_t)r * ldg + h);
+  else ldv<VE>(g, (size_t)r * ldg + c, z);
+#pragma unroll
+  for (int j = 0; j < VE; j++) x[j] *= sigmoidf_(z[per_head ? 0 : j]);
+  stv<VE>(out, (size_t)r * ldo + c, x);
 }
 
 template <typename T>
@@ -143,9 +149,16 @@ int p2p_sm_tanh(void* x, int ld, int n, int R, int f32, hipStream_t st) {
 int p2p_sm_sigmoid_gate(const void* o, long soh, long sor, const void* gt, int ldg, void* out,
                         int ldo, int R, int H, int V, int per_head, int f32, hipStream_t st) {
   if (R <= 0) return 0;
-  dim3 g((H * V + 255) / 256, R), b(256);
-  SM_DISPATCH_T(f32, hipLaunchKernelGGL(sigmoid_gate_k<T>, g, b, 0, st, (const T*)o, soh, sor,
-                                         (const T*)gt, ldg, (T*)out, ldo, H, V, per_head));
+  const size_t al = f32 ? 16 : 8;
+#define GATE(VE)                                                                                             \
+  SM_DISPATCH_T(f32, hipLaunchKernelGGL((sigmoid_gate_k<T, VE>), dim3((H * V + 256 * VE - 1) / (256 * VE), R), \
+                                         dim3(256), 0, st, (const T*)o, soh, sor, (const T*)gt, ldg, (T*)out, ldo, H, V, \
+                                         per_head))
+  if (V % 4 == 0 && soh % 4 == 0 && sor % 4 == 0 && ldo % 4 == 0 && ((size_t)o | (size_t)out) % al == 0 &&
+      (per_head || (ldg % 4 == 0 && (size_t)gt % al == 0)))
+    GATE(4);
+  else GATE(1);
+#undef GATE
   return (int)hipGetLastError();
 }
 
