@@ -431,10 +431,8 @@ class GeneralDelta(Mixer):
 
     def forward(self, h, b, cache, layer):
         n = self.n
-        proj = sm.linear(h, self.w_in)
-        low = proj[:, 5 * n:]
-        sm.tanh_(low)
-        lo = sm.linear(low, self.w2)
+        proj = sm.linear(h, self.w_in, tanh_from=5 * n)
+        lo = sm.linear(proj[:, 5 * n:], self.w2)
         out = torch.empty(b.R, n, device=h.device, dtype=h.dtype)
         sm.gdelta_scan(proj[:, 0:n], proj[:, n:2 * n], proj[:, 2 * n:3 * n], proj[:, 3 * n:4 * n],
                        proj[:, 4 * n:5 * n], lo, self.w0, self.ab, self.normw,
@@ -477,10 +475,11 @@ class Mamba2(Mixer):
         st = cache.state[layer]
         zx = sm.linear(h, self.w_in)
         conv = torch.empty(b.R, self.C, device=h.device, dtype=torch.float32)
-        sm.mamba_conv(zx, self.inner, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, conv)
+        single = all(e[1] == 1 for e in b.ent_host)   # their tails move on in the convolution's launch
+        sm.mamba_conv(zx, self.inner, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, conv, roll=single)
         y = torch.empty(b.R, self.inner, device=h.device, dtype=torch.float32)
         sm.mamba_scan(conv, zx, self.inner, self.inner + self.C, self.dt_bias, self.A_log, self.Dp,
-                      st["S"], st["tail"], b.ent, b.ent_host, y, self.H, self.P, self.N, self.G)
+                      st["S"], st["tail"], b.ent, b.ent_host, y, self.H, self.P, self.N, self.G, roll=not single)
         yn = torch.empty(b.R, self.inner, device=h.device, dtype=h.dtype)
         sm.rmsnorm(y, self.normw, self.eps, yn, parts=self.ng)
         return sm.linear(yn, self.wo)
@@ -596,7 +595,8 @@ class LatentAttention(Mixer):
         # keys and values are never formed: the query is carried into latent space with
         # W_uk (per head [D, rank]) and the attended latent leaves through W_uv^T
         self.uk = get("uk").to(dev, dtype).view(H, D, r).contiguous()
-        self.uvt = get("uv").to(dev, dtype).view(H, V, r).transpose(1, 2).contiguous()
+        self.uv = get("uv").to(dev, dtype).view(H, V, r).contiguous()
+        self.uvt = self.uv.transpose(1, 2).contiguous()
         self.sink = _vec(get("sink"), dev)
         self.wo = get("o").to(dev, dtype).contiguous()
 
@@ -614,9 +614,8 @@ class LatentAttention(Mixer):
                                    pool.shape[1])
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
                        ol, PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
-        o = torch.bmm(ol, self.uvt)                                                # [H, R, V]
         gated = torch.empty(b.R, H * V, device=h.device, dtype=h.dtype)
-        sm.sigmoid_gate(o, proj[:, H * D + r:], gated, H, V)
+        sm.heads_gated(ol, self.uv, self.uvt, proj[:, H * D + r:], gated)
         return sm.linear(gated, self.wo)
 
 
@@ -955,7 +954,8 @@ class RopeLatentAttention(Mixer):
         if self.QUERY_LATENT:
             self.qnorm, self.uq = _vec(get("dq.norm"), dev), get("uq").to(dev, dtype).contiguous()
         self.uk = get("uk").to(dev, dtype).view(H, D, r).contiguous()
-        self.uvt = get("uv").to(dev, dtype).view(H, V, r).transpose(1, 2).contiguous()
+        self.uv = get("uv").to(dev, dtype).view(H, V, r).contiguous()
+        self.uvt = self.uv.transpose(1, 2).contiguous()
         self.inv_freq = sm.rope_inv_freq(self.rot_base, self.rot_dims, dev, self.rot_scaling)
         self.rot_mag = sm.rope_magnitude(self.rot_scaling)
         self.wo = get("o").to(dev, dtype).contiguous()
@@ -995,8 +995,7 @@ class RopeLatentAttention(Mixer):
             if out_scale != 1.0:
                 out.mul_(out_scale)
             return out
-        o = torch.bmm(ol[:, :, :r], self.uvt)                                      # [H, R, V]
-        sm.sigmoid_gate(o, proj[:, qr + r + Rd:], out, H, V, per_head=True)
+        sm.heads_gated(ol[:, :, :r], self.uv, self.uvt, proj[:, qr + r + Rd:], out, per_head=True)
         if out_scale != 1.0:
             out.mul_(out_scale)
         return out

@@ -49,8 +49,10 @@ _SIGS = {
     "p2p_sm_gdelta_scan": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                             c_void_p, c_void_p, c_int, c_void_p, c_int, c_int,
                                             c_int, c_float, c_int, c_void_p],
-    "p2p_sm_skinny": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+    "p2p_sm_skinny": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                       c_void_p],
+    "p2p_sm_skinny_heads": [c_void_p, ctypes.c_long, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int,
+                            c_int, c_int, c_int, c_int, c_void_p],
     "p2p_sm_gdelta_chunk": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                                     c_void_p, c_int, c_void_p, c_int, c_int, c_int,
@@ -331,16 +333,38 @@ def _skinny(x, w) -> bool:
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def linear(x, w, b=None):
+def linear(x, w, b=None, tanh_from=None):
     """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, the shapes of ``_skinny`` on a
-    kernel for few rows."""
+    kernel for few rows.  tanh_from: columns from there on pass a tanh (of the rounded result)."""
     if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
             b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
-        return F.linear(x, w, b)
+        y = F.linear(x, w, b)
+        if tanh_from is not None:
+            tanh_(y[:, tanh_from:])
+        return y
     y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
     _chk(lib().p2p_sm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), _lib.ptr(b), y.data_ptr(), x.shape[0],
-                             w.shape[0], x.shape[1], _f32(x), _st(x)), "skinny")
+                             w.shape[0], x.shape[1], w.shape[0] if tanh_from is None else tanh_from, _f32(x),
+                             _st(x)), "skinny")
     return y
+
+
+def heads_gated(x, w, wt, g, out, per_head: bool = False):
+    """out[r, h*V + v] = (sum_k x[h, r, k] wt[h, k, v]) * sigmoid(g[r, h*V + v]), or with ``per_head`` sigmoid(g[r, h]);
+    x [H, R, K], wt [H, K, V] and the same weights as w [H, V, K], which a step of few rows reads."""
+    H, R, K = x.shape
+    V = w.shape[1]
+    if (0 < R <= 16 and x.is_cuda and x.dtype == torch.bfloat16 and K >= 8 and K % 8 == 0 and x.stride(2) == 1
+            and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        _rows2d(g, "g")
+        _rows2d(out, "out")
+        assert w.shape == (H, V, K) and w.is_contiguous() and w.dtype == g.dtype == out.dtype == x.dtype
+        assert g.shape[0] == R and g.shape[1] >= (H if per_head else H * V) and out.shape == (R, H * V)
+        _chk(lib().p2p_sm_skinny_heads(x.data_ptr(), x.stride(0), x.stride(1), w.data_ptr(), g.data_ptr(), g.stride(0),
+                                       1 if per_head else 0, out.data_ptr(), out.stride(0), R, H, V, K, _st(x)),
+             "skinny_heads")
+        return out
+    return sigmoid_gate(torch.bmm(x, wt), g, out, H, V, per_head=per_head)
 
 
 def rmsnorm(x, w, eps, out, parts: int = 1, in_rows=None, out_rows=None):
@@ -907,10 +931,11 @@ def conv_tail_roll(zx, xoff: int, tail, ent, ent_host, C: int, skip_single: bool
 
 
 def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail, ent, ent_host,
-               y, H: int, P: int, N: int, G: int):
+               y, H: int, P: int, N: int, G: int, roll: bool = True):
     """Selective state-space scan.  conv fp32 [R, H*P + 2*G*N] = silu(conv(x | B | C)); zx the
     input projection (z at column 0, raw x|B|C at xoff, dt at dtoff).  state fp32
-    [slots, H, N, P].  Writes y * silu(z) as fp32 [R, H*P] and rolls the convolution tail."""
+    [slots, H, N, P].  Writes y * silu(z) as fp32 [R, H*P] and, with ``roll``, rolls the
+    convolution tail (a step of single tokens has that from ``mamba_conv``)."""
     R, C = conv.shape
     inner = H * P
     Km1 = tail.shape[1]
@@ -930,7 +955,7 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
                 z = zx[t, :inner].float()
                 y[t] = yy.reshape(inner) * (z * torch.sigmoid(z))
             state[slot] = S
-            if Km1:
+            if Km1 and roll:
                 raw = zx[row0:row0 + n, xoff:xoff + C].float()
                 prev = tail[slot] if start > 0 else torch.zeros(Km1, C)
                 tail[slot] = torch.cat([prev, raw], 0)[-Km1:]
@@ -965,8 +990,9 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
                                      state.data_ptr(), tail.data_ptr(), walk.data_ptr(), walk.shape[0],
                                      y.data_ptr(), H, P, N, G, Km1 + 1, _f32(zx), _st(zx)),
              "mamba_scan")
-    _chk(lib().p2p_sm_mamba_tail(zx.data_ptr(), zx.stride(0), xoff, tail.data_ptr(),
-                                 ent.data_ptr(), E, C, Km1 + 1, 0, _f32(zx), _st(zx)), "mamba_tail")
+    if roll:
+        _chk(lib().p2p_sm_mamba_tail(zx.data_ptr(), zx.stride(0), xoff, tail.data_ptr(),
+                                     ent.data_ptr(), E, C, Km1 + 1, 0, _f32(zx), _st(zx)), "mamba_tail")
     return y
 
 

@@ -323,3 +323,60 @@ def test_glu_act_by_width(dt, F, off, act):
     res = [sm.glu_act(gu.to(d)[:, off:off + 2 * F], torch.zeros(3, F + 4, dtype=dt, device=d)[:, :F], act).cpu()
            for d in ("cpu", DEV)]
     torch.testing.assert_close(res[1], res[0], **_tol(dt))
+
+
+@pytest.mark.parametrize("R,H,V,K,per_head", [(1, 16, 128, 512, False), (8, 3, 40, 72, False), (16, 2, 24, 448, True),
+                                              (9, 1, 1, 8, True), (17, 2, 24, 64, False)])
+def test_heads_gated(R, H, V, K, per_head):
+    """Products of few rows per head with the gate in the epilogue: as the library's product, rounded, and the gate pass
+    (one bf16 step apart where the sums round differently), also from rows with a gap and into rows with a gap."""
+    g = torch.Generator().manual_seed(R + V)
+    x = torch.randn(H, R, K + 8, generator=g).bfloat16().to(DEV)[:, :, :K]
+    w = (torch.randn(H, V, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    gate = torch.randn(R, H * V + 3, generator=g).bfloat16().to(DEV)
+    out = torch.full((R, H * V + 5), 7.0, device=DEV).bfloat16()
+    wt = w.transpose(1, 2).contiguous()
+    sm.heads_gated(x, w, wt, gate, out[:, :H * V], per_head=per_head)
+    o = torch.stack([x[h].double() @ w[h].double().T for h in range(H)])
+    z = torch.sigmoid(gate.double())
+    z = z[:, :H].repeat_interleave(V, 1) if per_head else z[:, :H * V]
+    want = o.permute(1, 0, 2).reshape(R, H * V) * z
+    assert ((out[:, :H * V].double() - want).abs() <= 2 ** -7 * want.abs() + 1e-5 * o.abs().max()).all()
+    assert (out[:, H * V:] == 7).all()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 300])
+def test_linear_with_tanh_columns(dt, M):
+    """tanh of the columns from one on: bit for bit the product and then the pass over them."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, 1024, generator=g).to(dt).to(DEV)
+    w = (torch.randn(1104, 1024, generator=g) / 32).to(dt).to(DEV)
+    for at in (0, 1072, 1087, 1104):
+        want = sm.linear(x, w)
+        if at < 1104:
+            sm.tanh_(want[:, at:])
+        assert torch.equal(sm.linear(x, w, tanh_from=at), want) or at == 1104
+
+
+def test_mamba_tails_move_in_the_convolution():
+    """A step of single tokens: outputs, states and tails are those of a convolution that leaves its tails to the scan."""
+    g = torch.Generator().manual_seed(5)
+    H, P, N, G, K, E = 4, 64, 32, 2, 4, 5
+    inner = H * P
+    C = inner + 2 * G * N
+    zx = torch.randn(E, 2 * inner + 2 * G * N + H, generator=g).bfloat16().to(DEV)
+    cw, cb = torch.randn(C, K, generator=g).to(DEV), torch.randn(C, generator=g).to(DEV)
+    dtb, al, dp = (torch.randn(H, generator=g).to(DEV) for _ in range(3))
+    ent_h, ent, row_ent, R = _ents([1] * E, [3, 0, 7, 1, 9], [4, 0, 2, 1, 3])
+    got = []
+    for roll in (False, True):
+        S, T = torch.randn(6, H, N, P, generator=torch.Generator().manual_seed(1)).to(DEV), torch.randn(
+            6, K - 1, C, generator=torch.Generator().manual_seed(2)).to(DEV)
+        conv = torch.empty(R, C, device=DEV)
+        sm.mamba_conv(zx, inner, cw, cb, T, ent.to(DEV), ent_h, row_ent.to(DEV), conv, roll=roll)
+        y = torch.empty(R, inner, device=DEV)
+        sm.mamba_scan(conv, zx, inner, inner + C, dtb, al, dp, S, T, ent.to(DEV), ent_h, y, H, P, N, G, roll=not roll)
+        got.append((y, S, T))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
