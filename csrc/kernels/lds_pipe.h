@@ -80,6 +80,10 @@ __device__ __forceinline__ void dma_lds16(const void* base, unsigned off, unsign
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(l)
                : "memory", "m0");
 }
+// the same from an address per lane
+__device__ __forceinline__ void dma_lds16(const void* g, unsigned l) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(l) : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // a streamed (non-temporal) 16-byte global load into registers, counted like the DMAs

@@ -14,10 +14,12 @@
 // L2), and the row tiles of one column tile follow each other (its weights are in the L2 for the second).
 //
 // Gate and up (28672 x 4096) / down (4096 x 14336) of 8 experts, 2 per row, us, 128 x 128 tiles with one launch
-// dimension per expert / this: 65 rows 437 / 315 and 220 / 158, 400 rows 1240 / 380 and 580 / 180, 700 rows 752 / 500 and
-// 548 / 242, 1024 rows 1270 / 618 and 640 / 323.  Up to about 200 rows the weight stream (5.9 TB/s) is the bound, above
-// the reads of LDS beside the matrix products.  Half a stage read ahead of its products measured the same, two stages
-// in flight for rows and weights alike (every wavefront copying both) 5 to 40 % slower.
+// dimension per expert / this: 65 rows 437 / 315 and 220 / 158, 400 rows 1240 / 385 and 580 / 185, 700 rows 752 / 455
+// to 490 and 548 / 225, 1024 rows 1270 / 620 and 640 / 323.  Up to about 200 rows the weight stream (5.9 TB/s) is the
+// bound, above that what a CU takes in, rows from the L2 and weights together, at some 40 KB/us.  Half a stage read ahead of its products measured the same, two stages
+// in flight for rows and weights alike (every wavefront copying both) 5 to 40 % slower; copies issued before the reads
+// instead of between the products 2 to 5 % slower from 400 rows on, but for tiles of more than 256 rows (down 365
+// against 323 us at 1024 rows).
 #pragma once
 #include "prefill_gemm.h"
 
@@ -130,15 +132,20 @@ __device__ __forceinline__ void moe_gemm_body(bf16x8* lds, const bf16x8* __restr
       }
     }
   };
+  const unsigned lds_a = __builtin_amdgcn_readfirstlane(ldsp::lds_off(lds)) + (w & 3) * 1024, lds_b = lds_a + SA * ASTAGE * 16;
+  auto copy_a = [&](int i, int kt) {
+    ldsp::dma_lds16(src[i] + kt * (BK * 2), lds_a + (kt % SA) * (ASTAGE * 16) + i * 4096);
+  };
+  auto copy_b = [&](int i, int kt) {
+    ldsp::dma_lds16(src[i] + (size_t)kt * 2048, lds_b + (kt % SB) * (BSTAGE * 16) + i * 4096);
+  };
   auto issue_a = [&](int kt) {
-    bf16x8* base = lds + (kt % SA) * ASTAGE + w * 64;
 #pragma unroll
-    for (int i = 0; i < LA; ++i) ldsp::dma_lds<16>(src[i] + kt * (BK * 2), base + i * 256);
+    for (int i = 0; i < LA; ++i) copy_a(i, kt);
   };
   auto issue_b = [&](int kt) {
-    bf16x8* base = ldsb + (kt % SB) * BSTAGE + (w - 4) * 64;
 #pragma unroll
-    for (int i = 0; i < LB; ++i) ldsp::dma_lds<16>(src[i] + (size_t)kt * 2048, base + i * 256);
+    for (int i = 0; i < LB; ++i) copy_b(i, kt);
   };
   auto prologue = [&]() {
     if (rows_wave) {
@@ -158,15 +165,18 @@ __device__ __forceinline__ void moe_gemm_body(bf16x8* lds, const bf16x8* __restr
   // all stages of a wave that has LIVE fragment rows
   auto walk = [&](auto live) {
     constexpr int LIVE = decltype(live)::value;
+    constexpr bool BETWEEN = LIVE > 0 && NL < 5;   // copies go out between products; a ring of two stages wants them first
     for (int t = 0; t < n; ++t) {
       if (rows_wave) wait_stages<LA, SA - 2>(n - 1 - t);   // this wavefront's copies of stage t have landed
       else wait_stages<LB, SB - 2>(n - 1 - t);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();                        // ... and every other's; the stage before is used up
-      if (rows_wave) {
-        if (t + SA - 1 < n) issue_a(t + SA - 1);
-      } else if (t + SB - 1 < n) {
-        issue_b(t + SB - 1);
+      const int ahead = t + (rows_wave ? SA : SB) - 1;     // the stage this wavefront copies next
+      if constexpr (!BETWEEN) {
+        if (ahead < n) {
+          if (rows_wave) issue_a(ahead);
+          else issue_b(ahead);
+        }
       }
       if constexpr (LIVE > 0) {
         const unsigned sa = (t % SA) * (ASTAGE * 16), sb = fb + (t % SB) * (BSTAGE * 16);
@@ -180,10 +190,24 @@ __device__ __forceinline__ void moe_gemm_body(bf16x8* lds, const bf16x8* __restr
           ldsp::lds_wait(af, bfr);
           __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-          for (int i = 0; i < LIVE; ++i)
+          for (int i = 0; i < LIVE; ++i) {
 #pragma unroll
             for (int j = 0; j < FN; ++j)
               acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
+            if (BETWEEN && ks == 0) {
+              __builtin_amdgcn_sched_barrier(0);
+              if (ahead < n) {
+                if (rows_wave) {
+#pragma unroll
+                  for (int c = i * LA / LIVE; c < (i + 1) * LA / LIVE; ++c) copy_a(c, ahead);
+                } else {
+#pragma unroll
+                  for (int c = i * LB / LIVE; c < (i + 1) * LB / LIVE; ++c) copy_b(c, ahead);
+                }
+              }
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
           __builtin_amdgcn_s_setprio(0);
         }
       }
