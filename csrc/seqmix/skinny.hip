@@ -1,18 +1,20 @@
 // Matrix products of few rows: y[m, n] = sum_k x[m, k] W[n, k] (+ bias[n]), m < M <= 16, weights as a checkpoint has
 // them (row-major [N, K]), bf16 or fp32 with fp32 sums, one rounding at the end.
 //
-// A step of few rows reads every weight once and does little else, so the kernel is built around the loads: a
-// workgroup takes 16 rows of W, its eight wavefronts take the K index 128 bytes at a time in turn (together they
-// read 1 KB of each row), and each keeps two such pieces of all 16 rows in flight while it multiplies
-// (v_mfma_f32_16x16x32_bf16; fp32: four v_mfma_f32_16x16x4_f32 per 16-byte fragment).  The eight partial sums meet
-// in LDS.
-//
-// Bound by the weight stream at large N * K and by the chain of one launch otherwise (about 2.3 us at K = 32; the
-// activations are read by every workgroup, which is what 16 rows cost over one).  8 rows in bf16, in a captured
-// graph, microseconds, vendor product -> this: 1024 x 1024 5.8 -> 3.8, 4096 x 1024 6.1 -> 4.3, 2048 x 2048
-// 8.3 -> 5.4, 2048 x 4096 12.5 -> 8.3, 10304 x 2048 15.9 -> 13.2 (3.2 TB/s), one row 16.0 -> 11.6; fp32 1024 x 1024
-// 8.2 -> 5.4, 2048 x 2048 10.5 -> 8.5.  32 columns per workgroup leave half as many workgroups (2048 x 2048: 7.4),
-// 16 wavefronts or four pieces in flight measured the same within 0.2.
+// A step of few rows reads every weight once and does little else, so the kernels are built around the loads: a
+// workgroup takes 16 rows of W at a time, its eight wavefronts take the K index 128 bytes at a time in turn (together
+// they read 1 KB of each row) and multiply (v_mfma_f32_16x16x32_bf16; fp32: four v_mfma_f32_16x16x4_f32 per 16-byte
+// fragment).  The eight partial sums meet in LDS.  Bound by the weight stream at large N * K and by the chain of one
+// launch otherwise (about 2.3 us at K = 32).  Two kernels with the same sums in the same order:
+//  * walk_k, where four such pieces hold K (2048 numbers of bf16, 1024 of fp32): a workgroup reads the activations
+//    once, keeps them in registers and walks over tiles of 16 columns; the next tile's weights (up to 64 KB) are
+//    asked for in one burst while this one is multiplied and summed.
+//  * skinny_k, above and for few columns: one tile per workgroup, two pieces of weights and activations in flight.
+// In a captured graph with cold weights, us, vendor product / skinny_k / walk_k.  bf16, 8 rows: 2048 x 2048 11.2 / 6.0 /
+// 5.8, 4096 x 2048 11.7 / 6.7 / 6.2, 10304 x 2048 14.5 / 13.6 / 11.0, 18432 x 2048 58.7 / 21.3 / 17.0 (4.4 TB/s),
+// 32000 x 2048 34.5 / 32.5 / 26.5 (4.9), 16384 x 512 11.7 / 6.5 / 5.4; 16 rows 10304 x 2048 14.5 / 16.1 / 11.4, one
+// row 14.5 / 11.9 / 10.4.  fp32, 8 rows: 4096 x 1024 11.5 / 6.9 / 6.5, 16384 x 1024 18.2 / 19.5 / 15.5.  Eight pieces in
+// registers are no better: fp32 4096 x 2048 13.0 / 10.2 / 11.1, bf16 2048 x 4096 14.9 / 8.8 / 8.6.
 #include "attn_tile.h"
 using namespace sm;
 
@@ -38,6 +40,22 @@ __device__ __forceinline__ f32x4 mfma_frag(uint4 a, uint4 b, f32x4 c) {
 #pragma unroll
     for (int i = 0; i < 4; i++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], c, 0, 0, 0);
     return c;
+  }
+}
+
+// rows quad * 4 .. + 3 of column n of product p
+template <typename T>
+__device__ __forceinline__ void store_tile(const SkinnyArgs& a, int p, int n, int quad, f32x4 acc) {
+  const float b = a.bias ? ldf((const T*)a.bias, n) : 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int m = quad * 4 + e;
+    if (m >= a.M) break;
+    T o[1];
+    stf(o, 0, acc[e] + b);
+    if (n >= a.tanh_from) stf(o, 0, tanhf(ldf(o, 0)));
+    if (a.g) stf(o, 0, ldf(o, 0) * sigmoidf_(ldf((const T*)a.g, (size_t)m * a.ldg + (a.per_head ? p : p * a.N + n))));
+    ((T*)a.y)[p * a.yb + (size_t)m * a.ldy + n] = o[0];
   }
 }
 
@@ -88,17 +106,96 @@ __global__ void __launch_bounds__(512) skinny_k(SkinnyArgs a) {
   if (wave > 0 || n >= a.N) return;
 #pragma unroll
   for (int w = 0; w < WAVES - 1; w++) acc += red[w][lane];
-  const float b = a.bias ? ldf((const T*)a.bias, n) : 0.0f;
+  store_tile<T>(a, p, n, quad, acc);
+}
+
+// NP: pieces of 128 bytes per wavefront that hold a row of K numbers
+template <typename T, int NP>
+__global__ void __launch_bounds__(512) walk_k(SkinnyArgs a) {
+  constexpr int WAVES = 8;
+  constexpr int EP = 16 / sizeof(T), KB = 8 * EP;   // numbers per fragment, per 128 bytes
+  // by turns: the next tile's sums go to the other half, and the one after that starts behind the next barrier
+  __shared__ f32x4 red[2][WAVES][64];
+  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6), n16 = lane & 15, quad = lane >> 4;
+  const int p = blockIdx.y, tiles = (a.N + 15) / 16, stride = gridDim.x;
+  // rows that do not exist are the last ones, their results are dropped
+  const T* xp = (const T*)a.x + p * a.xb + (size_t)min(n16, a.M - 1) * a.ldx;
+  auto row = [&](int t) { return (const T*)a.w + p * a.wb + (size_t)min(t * 16 + n16, a.N - 1) * a.K; };
+  uint4 av[NP][2], bv[NP][2];
+  int at[NP][2];   // a fragment past K reads the row's first numbers and counts as zero on both sides
+  bool in[NP][2];
+  int t = blockIdx.x;
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const int m = quad * 4 + e;
-    if (m >= a.M) break;
-    T o[1];
-    stf(o, 0, acc[e] + b);
-    if (n >= a.tanh_from) stf(o, 0, tanhf(ldf(o, 0)));
-    if (a.g) stf(o, 0, ldf(o, 0) * sigmoidf_(ldf((const T*)a.g, (size_t)m * a.ldg + (a.per_head ? p : p * a.N + n))));
-    ((T*)a.y)[p * a.yb + (size_t)m * a.ldy + n] = o[0];
+  for (int i = 0; i < NP; i++)
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const int k = (i * WAVES + wave) * KB + (s * 4 + quad) * EP;
+      in[i][s] = k < a.K;
+      at[i][s] = in[i][s] ? k : 0;
+    }
+#pragma unroll
+  for (int i = 0; i < NP; i++)
+#pragma unroll
+    for (int s = 0; s < 2; s++) av[i][s] = *(const uint4*)(xp + at[i][s]);
+  const T* first = row(t);
+#pragma unroll
+  for (int i = 0; i < NP; i++)
+#pragma unroll
+    for (int s = 0; s < 2; s++) bv[i][s] = *(const uint4*)(first + at[i][s]);
+#pragma unroll
+  for (int i = 0; i < NP; i++)
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+      if (!in[i][s]) av[i][s] = make_uint4(0, 0, 0, 0);
+  for (int turn = 0; t < tiles; t += stride, turn++) {
+    const bool more = t + stride < tiles;
+    const T* next = row(t + stride);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    // the whole tile is there before the first of the next one is asked for: asked for one by one, as each is used, the
+    // halves of a line come apart (32000 x 2048 31 us, this 26.5)
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const uint4 w = in[i][s] ? bv[i][s] : make_uint4(0, 0, 0, 0);
+        acc = mfma_frag<T>(av[i][s], w, acc);
+        if (more) bv[i][s] = *(const uint4*)(next + at[i][s]);
+      }
+    f32x4 (&sums)[WAVES][64] = red[turn & 1];
+    sums[wave][lane] = acc;
+    // a barrier that leaves the loads in flight
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (wave == (turn & (WAVES - 1))) {
+      acc = sums[0][lane];
+#pragma unroll
+      for (int w = 1; w < WAVES; w++) acc += sums[w][lane];
+      const int n = t * 16 + n16;
+      if (n < a.N) store_tile<T>(a, p, n, quad, acc);
+    }
   }
+}
+
+// One workgroup per CU, all products together, each with the same number of tiles but for the last ones (8 rows in bf16,
+// 10304 x 2048: 215 workgroups 11.1 us, 256 11.3, 322 14.0, 512 11.8); two where a tile is only 16 KB (16384 x 512: 5.5
+// beside 6.4, while 16384 x 1024 has 8.5 beside 8.2).
+static int walkers(int tiles, int products, int pieces) {
+  const int most = max(1, 256 * (pieces > 1 ? 1 : 2) / products), each = (tiles + most - 1) / most;
+  return (tiles + each - 1) / each;
+}
+
+template <typename T>
+static void launch_skinny(const SkinnyArgs& a, int products, hipStream_t st) {
+  const int tiles = (a.N + 15) / 16, pieces = (a.K + 64 * 16 / (int)sizeof(T) - 1) / (64 * 16 / (int)sizeof(T));
+  const dim3 g(walkers(tiles, products, pieces), products), b(512);
+  // long rows of few columns: a tile per workgroup either way, and what comes first is multiplied first (8 rows, skinny_k /
+  // walk_k: fp32 1024 x 1024 5.3 / 5.6, 2048 x 1024 6.0 / 6.2, 3072 x 1024 6.3 / 6.3, bf16 96 x 2048 5.0 / 5.1, 2048 x 2048
+  // 5.9 / 5.8; two pieces, bf16 1024 x 1024 3.8 / 3.7)
+  if (pieces > 4 || (pieces > 2 && tiles < 128)) hipLaunchKernelGGL((skinny_k<T>), dim3(tiles, products), b, 0, st, a);
+  else if (pieces == 4) hipLaunchKernelGGL((walk_k<T, 4>), g, b, 0, st, a);
+  else if (pieces == 3) hipLaunchKernelGGL((walk_k<T, 3>), g, b, 0, st, a);
+  else if (pieces == 2) hipLaunchKernelGGL((walk_k<T, 2>), g, b, 0, st, a);
+  else hipLaunchKernelGGL((walk_k<T, 1>), g, b, 0, st, a);
 }
 
 extern "C" {
@@ -111,7 +208,7 @@ int p2p_sm_skinny(const void* x, int ldx, const void* w, const void* bias, void*
   const int ep = f32 ? 4 : 8;
   if (M > 16 || K < ep || K % ep || ldx % ep || (size_t)x % 16 || (size_t)w % 16) return (int)hipErrorInvalidValue;
   const SkinnyArgs a = {x, w, bias, y, ldx, M, N, K, N, 0, 0, 0, tanh_from, nullptr, 0, 0};
-  SM_DISPATCH_T(f32, hipLaunchKernelGGL((skinny_k<T>), dim3((N + 15) / 16), dim3(512), 0, st, a));
+  SM_DISPATCH_T(f32, launch_skinny<T>(a, 1, st));
   return (int)hipGetLastError();
 }
 
@@ -124,7 +221,7 @@ int p2p_sm_skinny_heads(const void* x, long xb, int ldx, const void* w, const vo
   if (M > 16 || H > 65535 || K < 8 || K % 8 || ldx % 8 || xb % 8 || (size_t)x % 16 || (size_t)w % 16 || !g)
     return (int)hipErrorInvalidValue;
   const SkinnyArgs a = {x, w, nullptr, y, ldx, M, N, K, ldy, xb, (long)N * K, N, N, g, ldg, per_head};
-  hipLaunchKernelGGL((skinny_k<bf16>), dim3((N + 15) / 16, H), dim3(512), 0, st, a);
+  launch_skinny<bf16>(a, H, st);
   return (int)hipGetLastError();
 }
 

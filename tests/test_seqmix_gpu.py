@@ -346,6 +346,29 @@ def test_heads_gated(R, H, V, K, per_head):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,part", [(1, 1, 1), (8, 17, 9), (16, 4096, 64), (5, 4112, 65), (8, 8203, 128), (16, 13000, 2),
+                                      (3, 8200, 256), (2, 4120, 257), (16, 50, 511),
+                                      (7, 5000, 161), (2, 2040, 192), (4, 2032, 192)])
+def test_few_row_products_walk_over_columns(dt, M, N, part):
+    """K of ``part`` 16-byte fragments: one to four pieces per wavefront and beyond, whole ones and rests; one to several
+    tiles per workgroup, the last one cut; rows with a gap.  Against 64 bits: one rounding of the result and one of each
+    of the K sums in fp32."""
+    K = part * (16 // dt.itemsize)
+    g = torch.Generator().manual_seed(part)
+    x = torch.randn(M, K + 16, generator=g).to(dt).to(DEV)[:, :K]
+    w = torch.randn(N, K, generator=g).to(dt).to(DEV)
+    b = torch.randn(N, generator=g).to(dt).to(DEV)
+    y = torch.full((M + 1, N), 7.0, dtype=dt, device=DEV)
+    sm._chk(sm.lib().p2p_sm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), b.data_ptr(), y.data_ptr(), M, N, K, N,
+                                   int(dt == torch.float32), sm._st(x)), "skinny")
+    want = x.double() @ w.double().T + b.double()
+    size = x.double().abs() @ w.double().abs().T + b.double().abs()
+    half = 2.0 ** -24 if dt == torch.float32 else 2.0 ** -8
+    assert ((y[:M].double() - want).abs() <= half * want.abs() + (K + 1) * 2.0 ** -23 * size).all()
+    assert (y[M] == 7).all()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 300])
 def test_linear_with_tanh_columns(dt, M):
     """tanh of the columns from one on: bit for bit the product and then the pass over them."""
