@@ -219,6 +219,28 @@ def test_latent_attn(dt, H, rank, win):
         torch.testing.assert_close(d.cpu().float(), a.float(), **_tol(dt))
 
 
+@pytest.mark.parametrize("runs", [1, 2, 3, 5])
+@pytest.mark.parametrize("H,rank,win,sunk", [(3, 72, 300, True), (20, 200, 131, False), (1, 384, 65, True), (16, 512, 300, True)])
+def test_latent_attn_shared_by_wavefronts(monkeypatch, H, rank, win, sunk, runs):
+    """Latents over 64 numbers in a step: 64 keys of four wavefronts, runs of an odd number of 32 keys, runs that are
+    empty, units of one to 16 rows, padded ranks."""
+    monkeypatch.setattr(sm, "_key_runs", lambda *a: runs)
+    g = torch.Generator().manual_seed(H)
+    page = 48
+    cache = torch.randn(page * 16, rank, generator=g).bfloat16()
+    bt = torch.randperm(16, generator=g).to(torch.int32).view(2, 8)
+    pos = torch.tensor(list(range(280, 299)) + [0, 63], dtype=torch.int32)
+    row_ent = torch.tensor([0] * 19 + [1, 1], dtype=torch.int32)
+    qa = (torch.randn(H, 21, rank, generator=g) * 0.2).bfloat16()
+    sink = torch.randn(H, generator=g) if sunk else None
+    want = sm.latent_attn(qa, cache, bt, row_ent, pos, sink, 0.2, win, torch.empty(H, 21, rank).bfloat16(), page)
+    units = sm.make_units([(0, 19, 280, 0), (19, 1, 0, 1), (20, 1, 63, 1)], sm.latent_rows_per_wave(H)).to(DEV)
+    got = sm.latent_attn(qa.to(DEV), cache.to(DEV), bt.to(DEV), row_ent.to(DEV), pos.to(DEV), None if sink is None else
+                         sink.to(DEV), 0.2, win, torch.empty(H, 21, rank, device=DEV).bfloat16(), page, units=units,
+                         max_keys=300)
+    torch.testing.assert_close(got.cpu().float(), want.float(), **_tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("lens,starts", [([130, 64, 1], [0, 7, 3]), ([65], [0]), ([33, 200], [5, 0])])
 @pytest.mark.parametrize("H,P,N,G", [(4, 64, 128, 2), (2, 30, 17, 1), (1, 256, 256, 1), (3, 36, 20, 1), (2, 100, 44, 1)])
 @pytest.mark.parametrize("steep", [False, True])
