@@ -43,8 +43,8 @@ __device__ __forceinline__ f32x4 mfma_frag(uint4 a, uint4 b, f32x4 c) {
   }
 }
 
-// rows quad * 4 .. + 3 of column n of product p
-template <typename T>
+// rows quad * 4 .. + 3 of column n of product p.  ACT: with the tanh and the gate, whose code a plain product need not fetch
+template <typename T, bool ACT>
 __device__ __forceinline__ void store_tile(const SkinnyArgs& a, int p, int n, int quad, f32x4 acc) {
   const float b = a.bias ? ldf((const T*)a.bias, n) : 0.0f;
 #pragma unroll
@@ -53,13 +53,15 @@ __device__ __forceinline__ void store_tile(const SkinnyArgs& a, int p, int n, in
     if (m >= a.M) break;
     T o[1];
     stf(o, 0, acc[e] + b);
-    if (n >= a.tanh_from) stf(o, 0, tanhf(ldf(o, 0)));
-    if (a.g) stf(o, 0, ldf(o, 0) * sigmoidf_(ldf((const T*)a.g, (size_t)m * a.ldg + (a.per_head ? p : p * a.N + n))));
+    if constexpr (ACT) {
+      if (n >= a.tanh_from) stf(o, 0, tanhf(ldf(o, 0)));
+      if (a.g) stf(o, 0, ldf(o, 0) * sigmoidf_(ldf((const T*)a.g, (size_t)m * a.ldg + (a.per_head ? p : p * a.N + n))));
+    }
     ((T*)a.y)[p * a.yb + (size_t)m * a.ldy + n] = o[0];
   }
 }
 
-template <typename T>
+template <typename T, bool ACT>
 __global__ void __launch_bounds__(512) skinny_k(SkinnyArgs a) {
   constexpr int WAVES = 8, DEPTH = 2;
   constexpr int EP = 16 / sizeof(T), KB = 8 * EP;   // numbers per fragment, per 128 bytes
@@ -106,11 +108,11 @@ __global__ void __launch_bounds__(512) skinny_k(SkinnyArgs a) {
   if (wave > 0 || n >= a.N) return;
 #pragma unroll
   for (int w = 0; w < WAVES - 1; w++) acc += red[w][lane];
-  store_tile<T>(a, p, n, quad, acc);
+  store_tile<T, ACT>(a, p, n, quad, acc);
 }
 
 // NP: pieces of 128 bytes per wavefront that hold a row of K numbers
-template <typename T, int NP>
+template <typename T, int NP, bool ACT>
 __global__ void __launch_bounds__(512) walk_k(SkinnyArgs a) {
   constexpr int WAVES = 8;
   constexpr int EP = 16 / sizeof(T), KB = 8 * EP;   // numbers per fragment, per 128 bytes
@@ -171,7 +173,7 @@ __global__ void __launch_bounds__(512) walk_k(SkinnyArgs a) {
 #pragma unroll
       for (int w = 1; w < WAVES; w++) acc += sums[w][lane];
       const int n = t * 16 + n16;
-      if (n < a.N) store_tile<T>(a, p, n, quad, acc);
+      if (n < a.N) store_tile<T, ACT>(a, p, n, quad, acc);
     }
   }
 }
@@ -184,18 +186,24 @@ static int walkers(int tiles, int products, int pieces) {
   return (tiles + each - 1) / each;
 }
 
-template <typename T>
-static void launch_skinny(const SkinnyArgs& a, int products, hipStream_t st) {
+template <typename T, bool ACT>
+static void launch_tiles(const SkinnyArgs& a, int products, hipStream_t st) {
   const int tiles = (a.N + 15) / 16, pieces = (a.K + 64 * 16 / (int)sizeof(T) - 1) / (64 * 16 / (int)sizeof(T));
   const dim3 g(walkers(tiles, products, pieces), products), b(512);
   // long rows of few columns: a tile per workgroup either way, and what comes first is multiplied first (8 rows, skinny_k /
   // walk_k: fp32 1024 x 1024 5.3 / 5.6, 2048 x 1024 6.0 / 6.2, 3072 x 1024 6.3 / 6.3, bf16 96 x 2048 5.0 / 5.1, 2048 x 2048
   // 5.9 / 5.8; two pieces, bf16 1024 x 1024 3.8 / 3.7)
-  if (pieces > 4 || (pieces > 2 && tiles < 128)) hipLaunchKernelGGL((skinny_k<T>), dim3(tiles, products), b, 0, st, a);
-  else if (pieces == 4) hipLaunchKernelGGL((walk_k<T, 4>), g, b, 0, st, a);
-  else if (pieces == 3) hipLaunchKernelGGL((walk_k<T, 3>), g, b, 0, st, a);
-  else if (pieces == 2) hipLaunchKernelGGL((walk_k<T, 2>), g, b, 0, st, a);
-  else hipLaunchKernelGGL((walk_k<T, 1>), g, b, 0, st, a);
+  if (pieces > 4 || (pieces > 2 && tiles < 128)) hipLaunchKernelGGL((skinny_k<T, ACT>), dim3(tiles, products), b, 0, st, a);
+  else if (pieces == 4) hipLaunchKernelGGL((walk_k<T, 4, ACT>), g, b, 0, st, a);
+  else if (pieces == 3) hipLaunchKernelGGL((walk_k<T, 3, ACT>), g, b, 0, st, a);
+  else if (pieces == 2) hipLaunchKernelGGL((walk_k<T, 2, ACT>), g, b, 0, st, a);
+  else hipLaunchKernelGGL((walk_k<T, 1, ACT>), g, b, 0, st, a);
+}
+
+template <typename T>
+static void launch_skinny(const SkinnyArgs& a, int products, hipStream_t st) {
+  if (a.g || a.tanh_from < a.N) launch_tiles<T, true>(a, products, st);
+  else launch_tiles<T, false>(a, products, st);
 }
 
 extern "C" {
