@@ -185,10 +185,14 @@ class DecodeGraph:
                           % (e, traceback.format_exc()))
             torch.cuda.synchronize(st.model.device)
             st.reset_dummy()
+            torch.cuda.synchronize(st.model.device)
             self.graph = None
             return self
-        torch.cuda.synchronize(st.model.device)
         st.reset_dummy()
+        # The native loop and a group's followers load the state on streams of their own, which do not wait for
+        # this one: a fill still queued here would overwrite the rows they load (with eight ranks on one device
+        # it came late in nearly every run, and the reply went its own way from there)
+        torch.cuda.synchronize(st.model.device)
         self.graph = g
         return self
 

@@ -11,6 +11,7 @@ import torch
 
 from p2p_llm_chat_go_amd import ops
 from p2p_llm_chat_go_amd.engine import Engine
+from p2p_llm_chat_go_amd.engine.graph import DecodeGraph
 from p2p_llm_chat_go_amd.models import TINY_LLAMA
 from p2p_llm_chat_go_amd.models.reference import (random_state_dict, reference_forward,
                                                   reference_greedy)
@@ -365,3 +366,44 @@ def test_prefill_graph_equals_eager_gpu(lens):
         eager.kv.allocator.free(pages)
         lg = lg[0].float().cpu()
         assert abs(float(lg[a[j]] - lg[b[j]])) < 2e-2 * float(lg.abs().max()), (j, a, b)
+
+
+@pytest.mark.parametrize("greedy", [True, False])
+@pytest.mark.parametrize("captured", [True, False])
+def test_decode_capture_leaves_no_work_behind(monkeypatch, greedy, captured):
+    """The native loop and its followers load a captured graph's state on streams of their own, which do not
+    wait for torch's: whatever the capture queues on the state must be done when it returns."""
+    import contextlib
+
+    log = []
+
+    class State:
+        model = type("M", (), {"device": torch.device("cuda", 0), "comm": None})()
+
+        def reset_dummy(self):
+            log.append("fill")
+
+        def body(self):
+            log.append("body")
+            if not captured and log.count("body") > 2:
+                raise RuntimeError("not capturable")
+
+        body_sampled = body
+
+    class Stream:
+        def __init__(self, *a):
+            pass
+
+        def wait_stream(self, other):
+            pass
+
+    monkeypatch.setattr(torch.cuda, "Stream", Stream)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream())
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", object)
+    monkeypatch.setattr(torch.cuda, "graph", lambda *a, **k: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: log.append("wait"))
+    with contextlib.nullcontext() if captured else pytest.warns(UserWarning):
+        g = DecodeGraph(State(), greedy=greedy).capture()
+    assert (g.graph is not None) == captured
+    assert log[-1] == "wait" and "fill" in log, log

@@ -90,28 +90,14 @@ def test_group_native_loop_matches_python_lockstep(world):
     # every reply in full, the seeded sampled one (request 2) included: both loops run a
     # chunk shape eagerly until its n-th use and through its captured graph after, and the
     # two forms' logits are pinned directly by test_tp_prefill_graph_matches_eager below
-    # (bit-identical at 2 / 4 / 8 ranks).  Open (round 6): at 8 virtual ranks the NATIVE
-    # loop's sampled reply left the Python loop's on 2 of 4 runs, at a different token each
-    # time (the Python loop's reply was the same on every run; bench/group_determinism.py
-    # runs each loop twice), while every greedy reply matched; inside ONE group the reply is
-    # stable (12 repeats, both loops: `group_determinism.py --repeat 12`, gpurun_out/r6y_rep8.log),
-    # and the round-6 final GPU tier run matched.  Until the cause is found, a world-8 sampled
-    # mismatch is reported as an expected failure, not hidden behind a shorter check.
-    open_issue = None
+    # (bit-identical at 2 / 4 / 8 ranks)
     for i, (a, b) in enumerate(zip(seq_n, seq_p)):
         assert a["eval_count"] == b["eval_count"]
-        if i == 2 and world == 8 and a["response"] != b["response"]:
-            open_issue = ("known intermittent: the native loop's seeded sampled reply at 8 "
-                          "virtual ranks left the Python loop's (native %r vs python %r)"
-                          % (a["response"][:80], b["response"][:80]))
-            continue
         assert a["response"] == b["response"], (i, a["response"], b["response"])
     # concurrent (batched decode, riders in prompt chunks): every reply complete (the
     # batch shapes differ from the sequential run's, so bf16 rounding may flip near-ties)
     for a, b in zip(conc_n, seq_p):
         assert a is not None and a["done"] and a["eval_count"] == b["eval_count"]
-    if open_issue:
-        pytest.xfail(open_issue)
 
 
 def test_group_follower_fault_fails_the_step():
