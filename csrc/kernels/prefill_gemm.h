@@ -1116,6 +1116,17 @@ int launch_phased(const void* Wt, const void* X, int ldx, int M, int K, int N, i
   return (int)hipGetLastError();
 }
 
+// 128 x 128 tiles of eight wavefronts and two stages, of which a CU takes two
+template <int EPI, bool NORM>
+int launch_pairs(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off, void* out, int ldo, float eps,
+                 const EpiArgs& ea, hipStream_t st) {
+  const int m_tiles = (M + 127) / 128, n_tiles = N / 128;
+  SplitArgs none{1, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
+  hipLaunchKernelGGL((prefill_gemm_kernel<128, 128, EPI, NORM, false, 2>), dim3(m_tiles * n_tiles), dim3(NT), 0, st,
+                     (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, none);
+  return (int)hipGetLastError();
+}
+
 template <int EPI, bool NORM>
 int launch_tile(int tile, const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off,
                 void* out, int ldo, float eps, const EpiArgs& ea, hipStream_t st) {
@@ -1129,52 +1140,70 @@ int launch_tile(int tile, const void* Wt, const void* X, int ldx, int M, int K, 
     case 3: return launch<128, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 4: return launch<64, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 5: return launch<64, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
-    case 6: return launch<320, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
+    case 6: return launch_pairs<EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 7: return launch<192, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 8: return launch<192, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 9:
-      if constexpr (EPI != EPI_SILU)   // (gate and up of 14336 columns do not divide by 96)
+      if constexpr (EPI != EPI_SILU)
         return launch<128, 192, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
   }
   return (int)hipErrorInvalidValue;
 }
 
-// Largest tile that still gives about one block per CU; N must divide.  M <= 64
+// Whether launch_tile has this tile for N columns with this epilogue (128 x 192 is not built for SwiGLU)
+static bool tile_fits(int tile, int N, int epi) {
+  static const int columns[] = {0, 256, 256, 128, 128, 256, 128, 128, 256, 192};
+  return tile >= 1 && tile <= 9 && N % columns[tile] == 0 && (tile != 9 || epi != EPI_SILU);
+}
+
+// The tile of a shape, 0 where N does not divide.  M <= 64
 // uses the 64-row tiles (no MFMA work or DMA on padding rows beyond one tile).  128-row tiles run on four
 // wavefronts that read ahead (prefill_gemm_kernel, NWV).  llama3.1-8B, cold weights, us, eight wavefronts in step (and
 // the tiles of 192 and 320 rows picked beside them) / now: o 128 rows 29 / 22, 400 rows 41 / 33, 1024 rows 64 / 50;
 // down 43 / 37, 101 / 75, 186 / 135 (890 TFLOP/s); qkv 27 / 24, 54 / 39, 95 / 55.  What is left there is each
 // wavefront's own chain: a wait for all wavefronts per 64 numbers of K beside 512 cycles of products.
 static int g_tile8 = 1;  // the 192 x 256 gate_up picks below (A/B switch: p2p_prefill_tile8)
-static int pick_tile(int M, int N, int K) {
-  if (M <= 64) return N % 128 == 0 ? 4 : 0;
+static int pick_tile(int M, int N, int K, int epi) {
+  if (N % 128) return 0;
+  if (M <= 64) return 4;
+  const int cus = cu_count() > 0 ? cu_count() : 256;
+  auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * (N / bn); };
   // (one-m-tile 384 / 448-row tiles for 321-448 rows measured 1.1-1.3x SLOWER than the
   // 128x128 split-K / phased 256x256 picks below and were removed:
   // profiles/r3_prefill_tiles_384_448.jsonl)
   if (N >= 16384) {
     // SwiGLU-width projections (gate_up of llama3.1-8B, us, cold weights).  129-192 rows: one m-tile of 192 rows,
     // 78 beside 80 with 128 x 128.  257-384 and 513-768 rows: 192 x 256 tiles waste fewer rows than the phased
-    // 256 x 256: 288 rows 106 / 112 (320 x 128: 112), 352 rows 107 / 108, 600 rows 195 / 204, 768 rows 198 / 208;
-    // 416 rows 193 / 115, 896 rows 278 / 217
-    if (N % 128 == 0 && M > 128 && M <= 192) return 7;
-    if (g_tile8 && N % 256 == 0 && ((M > 256 && M <= 384) || (M > 512 && M <= 768))) return 8;
+    // 256 x 256: 288 rows 106 / 112, 352 rows 107 / 108, 600 rows 195 / 204, 768 rows 198 / 208;
+    // 416 rows 193 / 115, 896 rows 278 / 217.  Not where they take a round of the CUs more (20480 x 2560, 600 rows:
+    // 131 / 73), nor up to 200 of them, where launch() cuts K as well (24576 x 4096, 300 rows: 138 / 105; 16384 x 2048:
+    // 74 beside 48 with 192 x 128)
+    if (M > 128 && M <= 192) return 7;
+    if (g_tile8 && N % 256 == 0 && ((M > 256 && M <= 384) || (M > 512 && M <= 768)) && tiles(192, 256) > 200 &&
+        (tiles(192, 256) - 1) / cus == (tiles(256, 256) - 1) / cus)
+      return 8;
   }
-  const int cand[3][3] = {{1, 256, 256}, {2, 128, 256}, {3, 128, 128}};
-  int best = 0;
-  const long cus = cu_count() > 0 ? cu_count() : 256, rows128 = (M + 127) / 128;
-  for (auto& c : cand) {
-    if (N % c[2]) continue;
-    const long blocks = (long)((M + c[1] - 1) / c[1]) * (N / c[2]);
-    // 128 x 192 where it takes one round of the CUs and 128 x 128 two: qkv of llama3.1-8B at 700 and 1024 rows
-    // 49 and 53 us beside 71 and 78 (128 x 256: 78 and 80); where 128 x 128 takes one round it is the faster one
-    // (512 rows 42 beside 49)
-    if (c[0] != 1 && N % 192 == 0 && rows128 * (N / 192) <= cus && N % 128 == 0 && rows128 * (N / 128) > cus) return 9;
-    if (!best) best = c[0];
-    // the phased 256x256 kernel pays from ~160 tiles (profiles/r2_prefill_gemm_phased.jsonl)
-    if (blocks >= (c[0] == 1 ? 160 : 200)) return c[0];
-    best = c[0];
-  }
-  return best;
+  // the phased 256x256 kernel pays from ~160 tiles (profiles/r2_prefill_gemm_phased.jsonl)
+  if (N % 256 == 0 && tiles(256, 256) >= 160) return 1;
+  const long small = tiles(128, 128);
+  if (small <= cus) return 3;
+  // 128 x 128 takes more than one round, a workgroup per CU: a larger tile that takes one.  us, 128 x 128 / 192 x 128 /
+  // 128 x 192 / 128 x 256: normed 9216 x 4096, 448 rows 74 / 68 / 50 / 78; llama3.1-8B qkv, 700 rows 71 / - / 49 / 78;
+  // residual 6144 x 2048, 700 rows 57 / 47 / 44 / 54; SwiGLU 12288 x 2048, 384 rows 46 / 39 / - / 43, 11264 x 2048, 300
+  // rows 40 / 38 / - / 43; where only the last fits SwiGLU 6144 x 1024, 1024 rows 30 / 35 / - / 26, 24576 x 4096, 256
+  // rows 82 / 110 / - / 79, 200 rows 76 / 111 / - / 78
+  const bool tall = tiles(192, 128) <= cus, resid = epi == EPI_RESID;
+  if (!(resid && K <= 1024) && tile_fits(9, N, epi) && tiles(128, 192) <= cus) return 9;
+  if (tall) return 7;
+  // no tile takes one.  Two workgroups on a CU hide what one waits for: the reads of the residual, the first and the last
+  // stages of a short K (pairs / 128 x 192 / 128 x 256: residual 3072 x 1024, 2048 rows 35 / 37 / 38, 11264 x 2368, 456
+  // rows 57 / - / 64, 22016 x 4096, 256 rows 95 / - / 91; pairs / 128 x 128: 8320 x 1024, 600 rows 28 / 31,
+  // 8320 x 4096, 600 rows 77 / 72, residual 86 / 91); over more rounds 192 x 128 has fewer (10112 x 768, 2167 rows
+  // 55 / 58 / 69 with 128 x 128, 8320 x 4096, 1042 rows 110 / 137 / 105)
+  const bool two = small <= 2 * cus;
+  if (N % 256 == 0) return resid && two && K <= 3072 ? 6 : 2;
+  if (two) return K <= (resid ? 4096 : 1024) ? 6 : 3;
+  return resid || K <= 2048 ? 7 : 3;
 }
 
 // Per-row RMSNorm statistics for the prefill GEMMs (one wave per row, every 16-byte load
@@ -1239,9 +1268,8 @@ static int prefill_dispatch(const void* Wt, const void* X, int ldx, int M, int K
                          hipStream_t st) {
   using namespace pgemm;
   if (M <= 0 || K % BK) return (int)hipErrorInvalidValue;
-  int tile = g_prefill_tile ? g_prefill_tile : pick_tile(M, N, K);
-  const int bn = (tile == 3 || tile == 4 || tile == 6 || tile == 7) ? 128 : tile == 9 ? 192 : 256;
-  if (!tile || N % bn) return (int)hipErrorInvalidValue;
+  const int tile = g_prefill_tile ? g_prefill_tile : pick_tile(M, N, K, epi);
+  if (!tile_fits(tile, N, epi)) return (int)hipErrorInvalidValue;
   const int up_off = (epi == EPI_SILU) ? N / 32 : 0;
   // normed projections from 128 rows: rstd by row_rstd_kernel, GEMM without in-loop sums
   if (norm && !ea.moe_cnt) {

@@ -210,6 +210,10 @@ def lib():
         if fn is not None:
             fn.argtypes = [c_int, c_int, c_int]
             fn.restype = None
+        fn = getattr(L, "p2p_prefill_tile", None)
+        if fn is not None:
+            fn.argtypes = [c_int, c_int, c_int, c_int]
+            fn.restype = c_int
         fn = getattr(L, "p2p_tiled_split_parallel", None)
         if fn is not None:
             fn.argtypes = [c_int]

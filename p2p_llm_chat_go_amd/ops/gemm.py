@@ -226,9 +226,9 @@ def _want_tiled(wt, M, N, K, epi, norm, waves) -> bool:
 
 
 def tiled_config(version: int = 2, tile: int = 0, splitk: int = 0):
-    """Prefill GEMM selection: version 2 = 8-wave LDS-DMA kernel (tile 0 = heuristic,
-    1 = 256x256, 2 = 128x256, 3 = 128x128; splitk 0 = heuristic, 1 = off, n = forced),
-    version 1 = register-staged 128x128."""
+    """Prefill GEMM selection: version 2 = LDS-DMA kernels (tile 0 = heuristic,
+    1 = 256x256, 2 = 128x256, 3 = 128x128, ... 9, see p2p_tiled_gemm_config; splitk 0 = heuristic,
+    1 = off, n = forced), version 1 = register-staged 128x128."""
     _lib.lib().p2p_tiled_gemm_config(int(version), int(tile), int(splitk))
 
 

@@ -1,7 +1,9 @@
 """Layouts the GEMM kernels rely on (CPU): fragment-major activations (ops.gemm.pack_frag)
 and weights (tile_weight) follow the v_mfma_f32_16x16x32_bf16 operand layout."""
+import pytest
 import torch
 
+from p2p_llm_chat_go_amd.ops import _lib
 from p2p_llm_chat_go_amd.ops import gemm as G
 
 
@@ -25,3 +27,21 @@ def test_pack_frag_layout():
 def test_tile_weight_roundtrip():
     w = torch.randn(64, 128).to(torch.bfloat16)
     assert torch.equal(G.untile_weight(G.tile_weight(w)), w)
+
+
+@pytest.mark.skipif(not _lib.available(), reason="kernel library not built")
+@pytest.mark.parametrize("epi", [G.EPI_STORE, G.EPI_RESID, G.EPI_SILU, G.EPI_F32, G.EPI_QKV_ROPE, G.EPI_ARGMAX])
+def test_every_width_of_128_columns_has_a_tile(epi):
+    """The heuristic gives every shape that tiles (K a multiple of 64, N of 128; SwiGLU: of 256) a tile that is built for
+    its epilogue; none is left to the register-staged kernel behind it.  (128 x 192 tiles are not built for SwiGLU:
+    feed-forwards of 3072 to 18432 columns whose gate and up divide by 192 were.)"""
+    L = _lib.lib()
+    for N in range(256 if epi == G.EPI_SILU else 128, 40960, 256 if epi == G.EPI_SILU else 128):
+        for M in (1, 64, 65, 100, 128, 129, 192, 193, 200, 256, 257, 300, 384, 385, 512, 513, 640, 641, 768, 1024, 2048, 4100):
+            assert L.p2p_prefill_tile(M, N, 1024, epi) > 0, (M, N)
+    for ffn, M in ((3072, 1024), (4608, 640), (6144, 400), (6912, 300), (9216, 200), (12288, 200), (18432, 100)):
+        assert L.p2p_prefill_tile(M, 2 * ffn, 4096, G.EPI_SILU) not in (0, 9)
+    assert L.p2p_prefill_tile(700, 6144, 4096, G.EPI_QKV_ROPE) == 9   # one round of 128 x 192
+    assert L.p2p_prefill_tile(700, 6144, 4096, G.EPI_SILU) == 7       # ... and of 192 x 128
+    assert L.p2p_prefill_tile(2048, 3072, 1024, G.EPI_RESID) == 6     # short rows: two tiles to a CU
+    assert L.p2p_prefill_tile(300, 100, 1024, epi) == 0 and L.p2p_prefill_tile(300, 256, 100, epi) == 0
