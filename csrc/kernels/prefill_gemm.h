@@ -121,17 +121,12 @@ __device__ __forceinline__ void pin_scalars(const T&... v) {
   (pin_scalar(v), ...);
 }
 
-// MOE: grouped expert GEMM (ea.moe_*): blockIdx.y = local expert e, whose rows are the
-// slots rows[e][i] (i < min(cnt[e], M)); A row of slot s = X[s / x_div], output row s
-// (scaled by row_w[s]).  m-tiles past the expert's count exit at once, so one launch
-// covers every expert at any M and each expert's weights stream once per m-tile.
-//
 // NWV = 4 (128-row tiles): four wavefronts of 64 x BN/2 instead of eight of 64 x 32, each the only one on its SIMD.  Eight
 // in step read a half stage, waited, multiplied it, and issued the copies between: 1900 cycles per stage for 512 cycles
 // of products.  Four read the next half stage under the products of the present one, and issue their copies (a
 // scalar address and a lane's constant offset) between the products: 1440 cycles.  Reads ahead alone gave 1600; a fifth
 // wavefront that touched the lines of stages further ahead, so that copies find them in the L2, nothing.
-template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, bool MOE = false, int NWV = 8>
+template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, int NWV = 8>
 __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
                                                           const bf16* __restrict__ X, int ldx,
                                                           int M, int K, int m_tiles, int n_tiles,
@@ -149,7 +144,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
   constexpr int AI = AB / NWV, BI = BB / NWV;  // blocks per wave per stage
   constexpr int L = AI + BI;               // LDS-DMA instructions per thread per stage
   static_assert(AB % NWV == 0 && BB % NWV == 0, "tile");
-  static_assert(!PIPE || (STAGES >= 3 && !MOE), "the stage after the present one is read ahead");
+  static_assert(!PIPE || STAGES >= 3, "the stage after the present one is read ahead");
   static_assert(FM >= 1 && FN >= 2, "tile");
   // PIPE: given at the launch.  A static 160 KiB tells the compiler that one wavefront per SIMD is all there can be, and it
   // moves the accumulators through AGPRs, four copies per product
@@ -165,14 +160,6 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
   int mt_i, nt_i;
   grouped_tile(tile, m_tiles, n_tiles, mt_i, nt_i);
   const int m0 = mt_i * BM;
-  const int* mrows = nullptr;
-  if constexpr (MOE) {
-    const int e = blockIdx.y;
-    M = min(ea.moe_cnt[e], M);
-    if (m0 >= M) return;  // block-uniform: this expert has fewer rows
-    Wt += (size_t)e * ea.w_stride;
-    mrows = ea.moe_rows + (size_t)e * ea.rows_stride;
-  }
   // rows' RMSNorm rstd precomputed by row_rstd_kernel (ea.rstd_in): the host launches the
   // NORM = false instantiation, so no sums of squares ride in the k loop (they cost
   // 12-22 % of the GEMM, profiles/r2_norm_cost.jsonl); applied in the epilogue
@@ -202,7 +189,6 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
     // PIPE: 8 rows x 128 bytes per block, 16-byte chunks of row R permuted by R & 7 (see the phased kernel)
     if constexpr (PIPE) row = m0 + 8 * blk + (lane >> 3);
     row = row < M ? row : M - 1;
-    if constexpr (MOE) row = mrows[row] / ea.x_div;
     asrc[i] = X + (size_t)row * ldx + (PIPE ? 8 * ((lane & 7) ^ (lane >> 3)) : 32 * ks + 8 * (lane >> 4));
   }
   const bf16x8* bsrc[BI];
@@ -429,7 +415,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
           const int m = m0 + wm_ * (BM / 2) + 16 * i + 4 * q + jj;
           posv[jj] = 0;
           slotv[jj] = -1;
-          if constexpr (EPI == EPI_QKV_ROPE && !MOE)
+          if constexpr (EPI == EPI_QKV_ROPE)
             if (m < M) {
               posv[jj] = ea.pos[m];
               slotv[jj] = ea.slots[m];
@@ -437,11 +423,11 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
           for (int j = 0; j < FN; ++j) {
             resv[jj][j] = 0.f;
-            if constexpr (EPI == EPI_RESID && !MOE)
+            if constexpr (EPI == EPI_RESID)
               if (m < M) resv[jj][j] = (float)reinterpret_cast<const bf16*>(out)[(size_t)m * ldo + (nt_i * (BN / 16) + bg[j]) * 16 + r];
           }
         }
-        if constexpr (EPI == EPI_QKV_ROPE && !MOE) {
+        if constexpr (EPI == EPI_QKV_ROPE) {
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
@@ -460,25 +446,21 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const int rl = wm_ * (BM / 2) + 16 * i + 4 * q + jj;
-        int m = m0 + rl;
+        const int m = m0 + rl;
         const bool valid = m < M;
-        float scale = scv[jj];
-        if constexpr (MOE) {
-          m = valid ? mrows[m] : 0;  // output row = the slot
-          if (ea.row_w && valid) scale *= ea.row_w[m];
-        }
+        const float scale = scv[jj];
         if constexpr (EPI == EPI_SILU) {
           constexpr int H = FN / 2;
 #pragma unroll
           for (int j = 0; j < H; ++j)
             epi_store<EPI>(m, valid, nt_i * (BN / 32) + wn_ * H + j, r, ac[i][j][jj] * scale,
                            ac[i][j + H][jj] * scale, out, ldo, ea);
-        } else if constexpr (EPI == EPI_QKV_ROPE && !MOE) {
+        } else if constexpr (EPI == EPI_QKV_ROPE) {
 #pragma unroll
           for (int j = 0; j < FN; ++j)
             epi_store<EPI>(m, valid, nt_i * (BN / 16) + bg[j], r, ac[i][j][jj] * scale, 0.f, out,
                            ldo, ea, csv[jj][j], valid ? slotv[jj] : -1);
-        } else if constexpr (EPI == EPI_RESID && !MOE) {
+        } else if constexpr (EPI == EPI_RESID) {
 #pragma unroll
           for (int j = 0; j < FN; ++j)
             if (valid)
@@ -495,10 +477,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
   };
   auto rstd_of = [&](float t) { return rsqrtf(t / (float)K + eps); };
   auto rstd_pre = [&](int rl) {
-    if (!pre) return 1.f;
-    int m = min(m0 + rl, M - 1);
-    if constexpr (MOE) m = mrows[m] / ea.x_div;  // the slot's token row of X
-    return ea.rstd_in[m];
+    return pre ? ea.rstd_in[min(m0 + rl, M - 1)] : 1.f;
   };
 
   if constexpr (SPLIT) {
@@ -1021,7 +1000,7 @@ int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_ti
   };
   if constexpr (splits_k<BM, BN>()) {
     if (splitk > 1) {
-      constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, true, STAGES, false, NWV>;
+      constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, true, STAGES, NWV>;
       if (const hipError_t e = with_lds((const void*)kernel)) return (int)e;
       const size_t slab = (size_t)tiles * splitk * BM * BN * sizeof(float);
       // counters live at the END of the workspace at a fixed offset from the end so a
@@ -1038,7 +1017,7 @@ int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_ti
     }
   }
   SplitArgs none{1, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-  constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, false, STAGES, false, NWV>;
+  constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, false, STAGES, NWV>;
   if (const hipError_t e = with_lds((const void*)kernel)) return (int)e;
   hipLaunchKernelGGL(kernel, dim3(tiles), dim3(NWV * 64), SHM, st, (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles,
                      n_tiles, up_off, out, ldo, eps, ea, none);
@@ -1089,19 +1068,6 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
   }
   return launch_stages<BM, BN, EPI, NORM, SHALLOW>(Wt, X, ldx, M, K, m_tiles, n_tiles, up_off, out,
                                                    ldo, eps, ea, st, splitk, ws, par);
-}
-
-template <int BM, int BN, int EPI, bool NORM>
-int launch_moe(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off, void* out,
-               int ldo, float eps, const EpiArgs& ea, hipStream_t st) {
-  constexpr int STAGES = stages_for<BM, BN>();
-  const int m_tiles = (M + BM - 1) / BM;
-  const int n_tiles = N / BN;
-  SplitArgs none{1, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-  hipLaunchKernelGGL((prefill_gemm_kernel<BM, BN, EPI, NORM, false, STAGES, true>),
-                     dim3(m_tiles * n_tiles, ea.n_experts), dim3(NT), 0, st, (const bf16x8*)Wt,
-                     (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, none);
-  return (int)hipGetLastError();
 }
 
 static int g_phased = 1;  // 256x256 tiles: phased pipeline (1) or the 2-stage kernel (0)
@@ -1236,9 +1202,8 @@ static __global__ __launch_bounds__(256) void row_rstd_kernel(const bf16* __rest
 // never grown while capturing (the GEMM then keeps the in-loop sums)
 static SplitWs g_rstd_ws;
 static int g_pre_rstd = 1;  // 0: always in-loop sums (A/B)
-static const float* pre_rstd(const void* X, int ldx, int M, int K, float eps, hipStream_t st,
-                             int min_rows = 128) {
-  if (!g_pre_rstd || M < min_rows || (ldx % 8) || (K % 8) || ((uintptr_t)X % 16)) return nullptr;
+static const float* pre_rstd(const void* X, int ldx, int M, int K, float eps, hipStream_t st) {
+  if (!g_pre_rstd || M < 128 || (ldx % 8) || (K % 8) || ((uintptr_t)X % 16)) return nullptr;
   const size_t bytes = (size_t)M * sizeof(float);
   if (g_rstd_ws.bytes < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1272,7 +1237,7 @@ static int prefill_dispatch(const void* Wt, const void* X, int ldx, int M, int K
   if (!tile_fits(tile, N, epi)) return (int)hipErrorInvalidValue;
   const int up_off = (epi == EPI_SILU) ? N / 32 : 0;
   // normed projections from 128 rows: rstd by row_rstd_kernel, GEMM without in-loop sums
-  if (norm && !ea.moe_cnt) {
+  if (norm) {
     if (const float* r = pre_rstd(X, ldx, M, K, eps, st)) {
       EpiArgs e2 = ea;
       e2.rstd_in = r;

@@ -324,14 +324,16 @@ P2P_API int p2p_tiled_gemm_argmax(const void* Wt, const void* X, int ldx, int M,
   return tiled_dispatch(Wt, X, ldx, M, K, N, EPI_ARGMAX, 1, keys, 0, eps, ea, stream);
 }
 
-// Grouped (MoE) expert GEMM for prompts (moe_gemm.h): one launch; see p2p_grouped_gemm for the arguments.
+// Grouped (MoE) expert GEMM for prompts (moe_gemm.h); see p2p_grouped_gemm for the arguments.  norm: the rows' rstd (X
+// has max_rows rows) go to `rstd`, a buffer of the caller's, so that calls on several streams or devices share nothing.
 P2P_API int p2p_grouped_gemm_tiled(const void* Wt, long long w_stride, int n_experts,
                                    const int* cnt, const int* rows, int rows_stride, int x_div,
                                    const float* row_w, const void* X, int ldx, int max_rows,
                                    int K, int N, int epi, int norm, void* out, int ldo, float eps,
-                                   hipStream_t stream) {
+                                   float* rstd, hipStream_t stream) {
   using namespace pgemm;
   if (n_experts <= 0 || max_rows <= 0 || K % pgemm::BK || N % 128) return (int)hipErrorInvalidValue;
+  if (epi == EPI_SILU ? !norm || N % 256 : epi != EPI_STORE) return (int)hipErrorInvalidValue;
   EpiArgs ea = {};
   ea.moe_cnt = cnt;
   ea.moe_rows = rows;
@@ -340,21 +342,13 @@ P2P_API int p2p_grouped_gemm_tiled(const void* Wt, long long w_stride, int n_exp
   ea.row_w = row_w;
   ea.w_stride = w_stride;
   ea.n_experts = n_experts;
-  // normed (w13): the token rows' rstd once (X has max_rows rows), applied per slot at the end
-  if ((epi == EPI_SILU && norm && N % 256 == 0) || epi == EPI_STORE) {
-    if (norm) ea.rstd_in = pre_rstd(X, ldx, max_rows, K, eps, stream, 1);
-    if (!norm || ea.rstd_in)
-      return epi == EPI_SILU ? launch_moe_gemm<EPI_SILU>(Wt, X, ldx, max_rows, K, N, out, ldo, ea, stream)
-                             : launch_moe_gemm<EPI_STORE>(Wt, X, ldx, max_rows, K, N, out, ldo, ea, stream);
+  if (norm) {
+    if (!rstd || ldx % 8 || (uintptr_t)X % 16) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(row_rstd_kernel, dim3((max_rows + 3) / 4), dim3(256), 0, stream, (const bf16*)X, ldx, max_rows, K,
+                       eps, rstd);
+    if (const hipError_t e = hipGetLastError()) return (int)e;
+    ea.rstd_in = rstd;
   }
-  // no buffer for the rstd (a capture before the first eager call): sums of squares in the k loop
-  if (epi == EPI_SILU) {
-    if (!norm || N % 256) return (int)hipErrorInvalidValue;
-    return launch_moe<128, 128, EPI_SILU, true>(Wt, X, ldx, max_rows, K, N, N / 32, out, ldo, eps,
-                                                ea, stream);
-  }
-  if (epi == EPI_STORE)
-    return launch_moe<128, 128, EPI_STORE, true>(Wt, X, ldx, max_rows, K, N, 0, out, ldo, eps, ea,
-                                                 stream);
-  return (int)hipErrorInvalidValue;
+  return epi == EPI_SILU ? launch_moe_gemm<EPI_SILU>(Wt, X, ldx, max_rows, K, N, out, ldo, ea, stream)
+                         : launch_moe_gemm<EPI_STORE>(Wt, X, ldx, max_rows, K, N, out, ldo, ea, stream);
 }

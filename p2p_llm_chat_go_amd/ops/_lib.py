@@ -106,7 +106,7 @@ _SIGS = {
                               c_float, c_void_p],
     "p2p_grouped_gemm": [c_void_p, ctypes.c_longlong, c_int, c_void_p, c_void_p, c_int, c_int,
                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
-                         c_int, c_float, c_int, c_void_p],
+                         c_int, c_float, c_int, c_void_p, c_void_p],
     "p2p_moe_route": [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                       c_void_p, c_void_p, c_int, c_void_p],
     "p2p_moe_router_route": [c_void_p, c_int, c_int, c_int, c_void_p, c_float, c_int, c_int, c_int,

@@ -113,10 +113,15 @@ def grouped_gemm(wt, cnt, rows, x, x_div, max_rows, epi, out, norm=False, row_w=
         return out
     L = _lib.lib()
     w_stride = wt[0].numel() // 8  # in bf16x8 units
+    rstd = None
+    if norm and max_rows > 64:   # the rows' scales, in a buffer of this call's own
+        if x.stride(0) % 8 or x.data_ptr() % 16:
+            x = x.clone(memory_format=torch.contiguous_format)
+        rstd = torch.empty(max_rows, dtype=torch.float32, device=x.device)
     _lib.check(L.p2p_grouped_gemm(wt.data_ptr(), w_stride, E, cnt.data_ptr(), rows.data_ptr(),
                                   rows.stride(0), x_div, _lib.ptr(row_w), x.data_ptr(), x.stride(0),
                                   max_rows, K, N, epi, int(norm), out.data_ptr(), out.stride(0),
-                                  float(eps), 0, _lib.stream_ptr(x.device)), "grouped_gemm")
+                                  float(eps), 0, _lib.ptr(rstd), _lib.stream_ptr(x.device)), "grouped_gemm")
     return out
 
 

@@ -45,3 +45,15 @@ def test_every_width_of_128_columns_has_a_tile(epi):
     assert L.p2p_prefill_tile(700, 6144, 4096, G.EPI_SILU) == 7       # ... and of 192 x 128
     assert L.p2p_prefill_tile(2048, 3072, 1024, G.EPI_RESID) == 6     # short rows: two tiles to a CU
     assert L.p2p_prefill_tile(300, 100, 1024, epi) == 0 and L.p2p_prefill_tile(300, 256, 100, epi) == 0
+
+
+@pytest.mark.skipif(not _lib.available(), reason="kernel library not built")
+def test_grouped_product_has_no_scales_of_its_own():
+    """Normed grouped products of more than 64 rows write the rows' scales to the caller's buffer and refuse a call without
+    one: a buffer inside the library was shared by every stream and device."""
+    L = _lib.lib()
+    at = 4096   # no launch is reached, so nothing is read
+    args = [at, 0, 2, at, at, 128, 1, None, at, 64, 100, 64, 256, G.EPI_SILU, 1, at, 128, 1e-5, 0]
+    assert L.p2p_grouped_gemm(*args, None, None) != 0
+    args[8] = at + 2   # rows that the scales' wide loads cannot take
+    assert L.p2p_grouped_gemm(*args, at, None) != 0

@@ -797,6 +797,41 @@ def test_moe_grouped_tile_heights(counts, H, F):
         assert (out[s].float() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
 
 
+def test_moe_grouped_on_two_streams():
+    """Normed grouped products of 65 to 127 rows on two streams at once: each call has scales of its own."""
+    from p2p_llm_chat_go_amd.ops import moe as M
+
+    E, H, F = 4, 1024, 1024
+    g = torch.Generator().manual_seed(3)
+    wt = torch.stack([ops.tile_weight((torch.randn(2 * F, H, generator=g) * H ** -0.5).to(torch.bfloat16))
+                      for _ in range(E)]).to(DEV)
+    work = []
+    for R, scale in ((65, 0.01), (127, 30.0)):
+        x = (torch.randn(R, H, generator=g) * scale).to(torch.bfloat16).to(DEV)
+        rows = torch.arange(R, dtype=torch.int32, device=DEV).repeat(E, 1)
+        rows += torch.arange(E, dtype=torch.int32, device=DEV)[:, None] * R
+        work.append((x, torch.full((E,), R, dtype=torch.int32, device=DEV), rows, R, torch.cuda.Stream()))
+
+    def run(x, cnt, rows, R):
+        out = torch.full((E * R, F), float("nan"), dtype=torch.bfloat16, device=DEV)
+        M.grouped_gemm(wt, cnt, rows, x, E, R, ops.EPI_SILU, out, norm=True)
+        return out
+
+    # (slot s of row s // E: every expert's list names other rows)
+    want = [run(*w[:4]) for w in work]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(20):
+        for w, o in zip(work, got):
+            with torch.cuda.stream(w[4]):
+                o.append(run(*w[:4]))
+    torch.cuda.synchronize()
+    for ref, outs in zip(want, got):
+        assert not ref.isnan().any()
+        for o in outs:
+            assert torch.equal(o, ref)
+
+
 # ------------------------------------------------------------ tiled (prefill) GEMM
 # (version, tile, splitk[, parallel split-K reduction]); split-K grids of at most one block
 # per CU with splitk | 8 take the parallel reduction unless the 4th field is 0
