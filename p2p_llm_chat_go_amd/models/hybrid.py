@@ -571,6 +571,13 @@ class Lightning(Mixer):
         return out
 
 
+def _value_products(w, gated=True):
+    """Latents to values [H, V, rank] for ``sm.heads_gated``: as a step of few rows reads them, where that has a kernel (else
+    None), and transposed, as the library's batched product does."""
+    return (w.contiguous() if gated and w.is_cuda and w.dtype == torch.bfloat16 else None,
+            w.transpose(1, 2).contiguous())
+
+
 class LatentAttention(Mixer):
     kind = "latent_attention"
 
@@ -595,8 +602,7 @@ class LatentAttention(Mixer):
         # keys and values are never formed: the query is carried into latent space with
         # W_uk (per head [D, rank]) and the attended latent leaves through W_uv^T
         self.uk = get("uk").to(dev, dtype).view(H, D, r).contiguous()
-        self.uv = get("uv").to(dev, dtype).view(H, V, r).contiguous()
-        self.uvt = self.uv.transpose(1, 2).contiguous()
+        self.uv, self.uvt = _value_products(get("uv").to(dev, dtype).view(H, V, r))
         self.sink = _vec(get("sink"), dev)
         self.wo = get("o").to(dev, dtype).contiguous()
 
@@ -954,8 +960,7 @@ class RopeLatentAttention(Mixer):
         if self.QUERY_LATENT:
             self.qnorm, self.uq = _vec(get("dq.norm"), dev), get("uq").to(dev, dtype).contiguous()
         self.uk = get("uk").to(dev, dtype).view(H, D, r).contiguous()
-        self.uv = get("uv").to(dev, dtype).view(H, V, r).contiguous()
-        self.uvt = self.uv.transpose(1, 2).contiguous()
+        self.uv, self.uvt = _value_products(get("uv").to(dev, dtype).view(H, V, r), self.HEAD_GATE)
         self.inv_freq = sm.rope_inv_freq(self.rot_base, self.rot_dims, dev, self.rot_scaling)
         self.rot_mag = sm.rope_magnitude(self.rot_scaling)
         self.wo = get("o").to(dev, dtype).contiguous()

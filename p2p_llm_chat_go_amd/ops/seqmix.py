@@ -362,10 +362,10 @@ def linear(x, w, b=None, tanh_from=None):
 
 def heads_gated(x, w, wt, g, out, per_head: bool = False):
     """out[r, h*V + v] = (sum_k x[h, r, k] wt[h, k, v]) * sigmoid(g[r, h*V + v]), or with ``per_head`` sigmoid(g[r, h]);
-    x [H, R, K], wt [H, K, V] and the same weights as w [H, V, K], which a step of few rows reads."""
+    x [H, R, K], wt [H, K, V] and the same weights as w [H, V, K], which a step of few rows reads (None: it takes wt too)."""
     H, R, K = x.shape
-    V = w.shape[1]
-    if (0 < R <= 16 and x.is_cuda and x.dtype == torch.bfloat16 and K >= 8 and K % 8 == 0 and x.stride(2) == 1
+    V = wt.shape[2]
+    if (w is not None and 0 < R <= 16 and x.is_cuda and x.dtype == torch.bfloat16 and K >= 8 and K % 8 == 0 and x.stride(2) == 1
             and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
         _rows2d(g, "g")
         _rows2d(out, "out")

@@ -672,3 +672,15 @@ def test_config_roundtrip_and_errors():
         eng.step([("b", [1], [0])])          # no second state slot
     with pytest.raises(MemoryError):
         eng.step([("a", [1] * PAGE, [])])    # no second page
+
+
+@pytest.mark.parametrize("dev", DEVICES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind,gated", [("rope_latent_attention", True), ("direct_latent_attention", False)])
+def test_value_products_are_kept_twice_only_where_steps_read_them(dev, dtype, kind, gated):
+    """The second layout of the values' up-projection belongs to the bf16 kernel of gated heads."""
+    m = Hy.MIXERS[kind](dict(LA["mixer"]), 48, 1e-5)
+    shapes = m.tensor_shapes()
+    m.load(lambda k: torch.randn(shapes[k]), dtype, dev)
+    assert m.uvt.shape == (3, 24, 20)
+    assert (m.uv is not None) == (gated and dev != "cpu" and dtype == torch.bfloat16)
