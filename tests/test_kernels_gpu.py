@@ -1099,9 +1099,83 @@ def test_tiled_oproj_192_rows_heuristic():
     assert ops.tiled_split_fault() == 0
 
 
+@pytest.mark.parametrize("M,forced", [(641, False), (700, False), (1024, False), (1, True), (100, True), (257, True)])
+def test_tiled_qkv_rope_and_argmax_in_192_columns(M, forced):
+    """128 x 192 tiles, which prompts of 641 to 1024 rows take at 32 + 2 x 8 heads: twelve column groups cross heads of eight
+    and the borders of q, K and V.  Every number against one rounding of each operand of the rotation and one of its
+    result; where the rows' scales are formed before the product, also the bits of 64 x 128 tiles (the same sums in the
+    same order)."""
+    from p2p_llm_chat_go_amd.models.config import LLAMA31_8B, rope_table
+    from p2p_llm_chat_go_amd.ops import _lib
+    from p2p_llm_chat_go_amd.ops.gemm import set_tiled_min_m, tiled_config
+
+    Hq, Hkv, K = 32, 8, 512
+    N, pages = (Hq + 2 * Hkv) * 128, 17
+    assert forced or _lib.lib().p2p_prefill_tile(M, N, K, ops.gemm.EPI_QKV_ROPE) == 9
+    g = torch.Generator().manual_seed(M)
+    W = (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    cs = rope_table(LLAMA31_8B, max_pos=2048)
+    pos = torch.arange(M, dtype=torch.int32) + 3
+    slots = torch.randperm(pages * 64, generator=g)[:M].to(torch.int32)
+    slots[M // 2] = -1   # a row that writes no K and V
+    Wt = ops.tile_weight(W[ops.rope_row_perm(Hq + 2 * Hkv)]).to(DEV)
+
+    def run(tile):
+        q = torch.full((M, Hq * 128), 7.0).to(torch.bfloat16).to(DEV)
+        k = torch.full((pages, Hkv, 64, 128), 7.0).to(torch.bfloat16).to(DEV)
+        v = k.clone()
+        tiled_config(2, tile, 1 if tile else 0)
+        set_tiled_min_m(1)
+        try:
+            ops.qkv_rope_gemm(Wt, x.to(DEV), pos.to(DEV), slots.to(DEV), cs.to(DEV), Hq, Hkv, q, k, v)
+        finally:
+            set_tiled_min_m(65)
+            tiled_config(2, 0, 0)
+        return q.cpu(), k.cpu(), v.cpu()
+
+    q, k, v = run(9 if forced else 0)
+    if M >= 128:
+        for a, b in zip((q, k, v), run(4)):
+            assert torch.equal(a, b)
+    xf = x.double()
+    y = (xf @ W.double().T) * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5)
+    y = y.view(M, Hq + 2 * Hkv, 128)
+    c, s = (t[pos.long()][:, None, :].double() for t in (cs[..., 0], cs[..., 1]))
+    lo, hi = y[..., :64], y[..., 64:]
+    rot = torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+    room = torch.cat([lo.abs() + hi.abs()] * 2, -1) * 2.0 ** -8 + rot.abs() * 2.0 ** -8 + 1e-4
+    got = torch.full_like(y, float("nan"))
+    got[:, :Hq] = q.double().view(M, Hq, 128)
+    w = slots >= 0
+    page, at = slots[w].long() // 64, slots[w].long() % 64
+    got[w, Hq:Hq + Hkv], got[w, Hq + Hkv:] = k[page, :, at].double(), v[page, :, at].double()
+    rot[:, Hq + Hkv:] = y[:, Hq + Hkv:]
+    ok = (got - rot).abs() <= room
+    ok[~w, Hq:] = True
+    assert ok.all()
+    rest = torch.ones(pages, 64, dtype=torch.bool)
+    rest[page, at] = False
+    assert (k.transpose(1, 2)[rest] == 7).all() and (v.transpose(1, 2)[rest] == 7).all()
+    # the head: 1152 columns are six such tiles; the chosen one's logit is the largest up to the sums' rounding
+    Wl = (torch.randn(1152, K, generator=g) * 0.05).to(torch.bfloat16)
+    lg = (xf @ Wl.double().T) * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5)
+    keys, ids = ops.new_argmax_keys(M, DEV), torch.zeros(M, dtype=torch.int32, device=DEV)
+    tiled_config(2, 9, 1)
+    set_tiled_min_m(1)
+    try:
+        ops.lm_head_argmax(ops.tile_weight(Wl).to(DEV), x.to(DEV), keys, col_offset=5000)
+    finally:
+        set_tiled_min_m(65)
+        tiled_config(2, 0, 0)
+    ops.argmax_finalize(keys, ids)
+    chosen = lg.gather(1, ids.cpu().long()[:, None] - 5000)[:, 0]
+    assert (chosen >= lg.amax(1) - 1e-4 * lg.abs().amax()).all()
+
+
 def test_tiled_qkv_rope_384_rows_heuristic():
-    """The 384-row bucket at qkv width (32 + 2 x 8 heads: N = 6144) takes 192 x 128 tiles with
-    split-K 2 by the heuristic (prefill_gemm.h pick_tile): q, K and V against the fp32 path."""
+    """The 384-row bucket at qkv width (32 + 2 x 8 heads: N = 6144), which takes 128 x 128 tiles by the heuristic
+    (prefill_gemm.h pick_tile): q, K and V against the fp32 path."""
     from p2p_llm_chat_go_amd.models.config import LLAMA31_8B, rope_table
     from p2p_llm_chat_go_amd.ops.gemm import tiled_config
 
