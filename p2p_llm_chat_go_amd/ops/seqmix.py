@@ -1147,12 +1147,15 @@ LATENT_SPLIT_BLOCKS = 512   # split windows while a step has fewer blocks than t
 
 
 def _key_runs(blocks: int, most: int, tile: int, few: int = 128) -> int:
-    """Runs of keys that the windows of a step of few workgroups are cut into.  A wavefront takes runs of 64 keys, four
-    wavefronts that share key tiles runs of 256: shorter ones cost more in the merge than they gain (150 rows, 16 heads
-    of 128, 256 / 64 keys: 10.5 / 14.2 us, 100 rows and 12 decoded ones, windows of 256: 11.9 / 14.1), unless the windows
-    are long and fewer than ``few`` workgroups with runs of 64 leave the chip mostly idle (8 rows at 500, latents of 512:
-    26.6 / 17.9; 16 heads of 256: 18.8 / 12.9; 32 rows at 300, latents of 512: 24.0 / 21.5, at 1000 27.7 / 32.6; latents of
-    96, 64 rows at 1000, 136 workgroups: 14.5 / 13.0)."""
+    """Runs of keys that the windows of a step of few workgroups are cut into.  Runs of 64 keys, where a wavefront works alone
+    and where four share 64 keys (latents above 64 numbers: one run is one pass of its loop; steps of single tokens with
+    16 heads, runs of 64 / 128 / 256, us: latents of 512, 8 rows at 500 11.8 / 15.2 / 22.5, at 2000 14.6 / 16.4 / 22.9,
+    32 rows at 500 14.9 / 17.4 / 24.3, at 1000 26.7 / 20.8 / 26.3; latents of 256, 8 rows at 500 8.7 / 10.6 / 14.7, 32
+    rows at 1000 13.3 / 12.4 / 15.7).  Of 256 where four wavefronts share key tiles (tile): shorter ones cost more in the merge
+    than they gain (150 rows, 16 heads of 128, 256 / 64 keys: 10.5 / 14.2 us, 150 rows, latents of 512 20.9 / 33.2), unless
+    the windows are long and fewer than ``few`` workgroups with runs of 64 leave the chip mostly idle (8 rows of one
+    sequence at 500, latents of 512: 27.2 / 15.3; 16 heads of 256: 18.8 / 12.9; 32 rows at 300, latents of 512: 22.5 / 17.6, at
+    1000 30.1 / 27.5; latents of 96, 64 rows at 1000, 136 workgroups: 16.5 / 14.9)."""
     run = 256 if tile and (most < 256 or blocks * -(-most // 64) >= few) else 64
     return max(1, min(-(-most // run), LATENT_SPLIT_BLOCKS // blocks, 64))
 
@@ -1645,9 +1648,12 @@ def attn_unit_rows(rows_per_wave: int, ent_host: list, latent: int = 0) -> int:
     four times as many for the kernels whose four wavefronts share the key tiles.  Those win as
     soon as half of their rows are taken (a group of a decoded token leaves three of the four
     wavefronts idle).  ``latent``: size of a layer's latents; up to 128 they are so short that only portions of more
-    than 32 rows pay for sharing, up to 64 of more than 64 (a wavefront each / shared, us: 16 heads, latents of 64, 16
+    than 32 rows share, up to 64 of more than 64 (a wavefront each / shared, us: 16 heads, latents of 64, 16
     rows 6.2 / 7.5, 16 portions of 20 6.7 / 7.7, 8 of 40 7.9 / 8.5, one of 64 7.8 / 8.4, one of 96 10.1 / 9.3, 8 of 100
-    11.5 / 10.4; 8 heads, latents of 128, 16 rows 7.7 / 8.1, 8 of 40 9.5 / 9.2)."""
+    11.5 / 10.4).  Above 64 the smaller groups have four wavefronts on 64 keys too and are the faster ones for longer than
+    these lines say (smaller / shared: latents of 128, 16 rows 5.2 / 7.9, one portion of 64 5.2 / 7.8, of 96 9.1 / 8.8, 8 of
+    40 6.5 / 7.9, 8 of 100 11.1 / 10.2; of 512, 16 rows 9.2 / 14.3, one portion of 64 9.2 / 14.4, of 96 17.6 / 16.5, 8 of 40
+    17.3 / 15.1, 8 of 100 37.3 / 20.5)."""
     tile = 4 * rows_per_wave
     groups = sum(-(-e[1] // tile) for e in ent_host)
     if 0 < latent <= 128 and max(e[1] for e in ent_host) <= (64 if latent <= 64 else 32):
