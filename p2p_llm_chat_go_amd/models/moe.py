@@ -2,7 +2,7 @@
 
 Per layer, for R rows (chunks of <= 64 rows on the skinny grouped kernel; above 64 rows
 all rows at once on the LDS-tiled grouped kernel, ``moe_forward_tiled``):
-    ids, w = top_k(softmax(rstd(h) h Wr'))   moe_router_route (+ per-expert slot lists)
+    ids, w = top_k(softmax(rstd(h) h Wr'))   moe_router_route / moe_route_rows (+ per-expert slot lists)
     act[s] = silu(g) * u of expert(s)        grouped_gemm SILU | NORM
     o[s]   = w[s] * act[s] @ W2_e            grouped_gemm STORE (row-scaled)
     h     += sum_k o[r*K + k]                moe_combine (EP/TP: partial + all-reduce)
@@ -42,7 +42,6 @@ class MoeWorkspace:
     def __init__(self, cfg, rows, device, e_local, f_local):
         K = cfg.top_k
         dev = torch.device(device)
-        self.logits = torch.zeros(rows, 16, device=dev, dtype=torch.float32)
         self.topk_ids = torch.zeros(rows * K, device=dev, dtype=torch.int32)
         self.topk_w = torch.zeros(rows * K, device=dev, dtype=torch.float32)
         self.cnt = torch.zeros(e_local, device=dev, dtype=torch.int32)
@@ -74,6 +73,7 @@ def moe_forward(model, lw, ws, R):
     e_lo = w.ep_rank * e_local
     if ws.moe is None:
         ws.moe = MoeWorkspace(cfg, CHUNK, model.device, e_local, lw.w13.shape[1] * 16 // 2)
+        ws.moe.logits = torch.zeros(CHUNK, 16, device=model.device, dtype=torch.float32)
     m = ws.moe
     K = cfg.top_k
     distributed = w.ep_size > 1 or w.tp_size > 1
@@ -104,7 +104,7 @@ def moe_forward_tiled(model, lw, ws, R):
     """Prefill / large batches (R > 64 rows): route all R rows at once, then each expert's
     gate_up and down run as ONE grouped launch of the LDS-tiled MFMA kernel over its own
     rows (``ops.moe.grouped_gemm`` with max_rows > 64), so every selected expert's weights
-    stream once per 128-row tile of its rows -- not once per 64-row chunk of the prompt."""
+    stream once for up to 320 of its rows -- not once per 64-row chunk of the prompt."""
     cfg, w = model.cfg, model.w
     E, K = cfg.n_experts, cfg.top_k
     e_local = E // w.ep_size
@@ -158,7 +158,7 @@ A2A_STATIC_MAX_BYTES = int(os.environ.get("P2P_A2A_STATIC_MAX_BYTES", str(4 << 2
 def moe_forward_a2a(model, lw, ws, R):
     """DP-attention + EP MoE layer for this rank's R rows (see module doc).
 
-    Kernels (``moe.hip``): routing (``moe_route``), dispatch (``a2a_dispatch``: slot ->
+    Kernels (``moe.hip``): routing (``moe_route_rows``), dispatch (``a2a_dispatch``: slot ->
     owner rank, row packing), slot grouping on the owner (``a2a_group``), the grouped
     expert GEMMs, and the combine (``a2a_combine``).  Two exchange forms:
       * static capacity C = R*K rows per destination -- no host sync, hipGraph-capturable
