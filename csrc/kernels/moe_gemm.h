@@ -13,11 +13,12 @@
 // tile while it stores the finished one.  Tiles of one expert are neighbours (its gathered rows stay in the XCD's
 // L2), and the row tiles of one column tile follow each other (its weights are in the L2 for the second).
 //
-// Gate and up (28672 x 4096) / down (4096 x 14336) of 8 experts, 2 per row, us, 128 x 128 tiles with one launch
-// dimension per expert / this: 65 rows 437 / 315 and 220 / 158, 400 rows 1240 / 385 and 580 / 185, 700 rows 752 / 455
-// to 490 and 548 / 225, 1024 rows 1270 / 620 and 640 / 323.  Up to about 200 rows the weight stream (5.9 TB/s) is the
-// bound, above that what a CU takes in, rows from the L2 and weights together, at some 40 KB/us.  Half a stage read ahead of its products measured the same, two stages
-// in flight for rows and weights alike (every wavefront copying both) 5 to 40 % slower; copies issued before the reads
+// Gate and up (28672 x 4096, with the rows' scales) / down (4096 x 14336) of 8 experts, 2 per row, even routing, us,
+// 128 x 128 tiles with one launch dimension per expert / this: 65 rows 366 / 318 and 220 / 156, 400 rows 1180 / 367 and
+// 583 / 187, 700 rows 678 / 425 and 541 / 226 (a model's uneven routing: 500 and 245 now), 1024 rows 1223 / 640 and
+// 630 / 315; 59 to 400 rows per expert 772 / 616 and 539 / 524.  Up to about 200 rows the weight stream (5.9 TB/s) is the
+// bound, above that what a CU takes in, rows from the L2 and weights together, at some 40 KB/us.  Half a stage read ahead
+// of its products measured the same, two stages in flight for rows and weights alike (every wavefront copying both) 5 to 40 % slower; copies issued before the reads
 // instead of between the products 2 to 5 % slower from 400 rows on, but for tiles of more than 256 rows (down 365
 // against 323 us at 1024 rows).
 #pragma once

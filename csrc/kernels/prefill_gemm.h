@@ -1,9 +1,10 @@
-// Prefill GEMM v2: 8-wave MFMA GEMM with direct global->LDS (LDS-DMA) staging.
+// Prefill GEMM v2: MFMA GEMM with direct global->LDS (LDS-DMA) staging.
 //
 //   out[m, n] = epilogue( rstd[m] * sum_k X[m, k] * W[n, k] )   (gemm_epilogue.h)
 //
-// Tile BM x BN x 64 (BM, BN in {128, 256}), 512 threads = 8 waves in a 2 (M) x 4 (N)
-// grid; wave tile (BM/2) x (BN/4) of v_mfma_f32_16x16x32_bf16 accumulators.
+// Tiles BM x BN x 64 (launch_tile has the shapes, pick_tile the choice): 512 threads = 8 waves in a 2 (M) x 4 (N)
+// grid, wave tile (BM/2) x (BN/4) of v_mfma_f32_16x16x32_bf16 accumulators; 128 x 128 and 128 x 192 on 4 waves in a
+// 2 x 2 grid (NWV below).
 // Both operands are staged with `global_load_lds_dwordx4` (one wave-instruction
 // = one 1 KiB MFMA fragment block): the LDS image is fragment-major, so every
 // operand read is a lane-linear, conflict-free ds_read_b128 and no VGPRs or
@@ -12,8 +13,8 @@
 //     contiguous;
 //   * X is row-major: lane l of a block fetches X[row0 + (l&15)][k0 + 8(l>>4) ..]
 //     (per-lane source address, lane-linear destination).
-// Two LDS stages (2 x (BM+BN) x 64 bf16 <= 128 KiB, one __shared__ array):
-// stage kt+1 is in flight while the MFMAs consume stage kt; one barrier per
+// LDS holds two to six stages of (BM+BN) x 64 bf16 (stages_for, deep_stages_for): later
+// stages are in flight while the MFMAs consume stage kt; one barrier per
 // k-tile.  Blocks sharing a weight n-tile are consecutive after the XCD remap.
 // NORM: the waves of column 0 also square the A fragments they read; a lane
 // sees 8 of every 32 k of one row, 3 shuffles finish the row's sum.
@@ -122,10 +123,10 @@ __device__ __forceinline__ void pin_scalars(const T&... v) {
 }
 
 // NWV = 4 (128-row tiles): four wavefronts of 64 x BN/2 instead of eight of 64 x 32, each the only one on its SIMD.  Eight
-// in step read a half stage, waited, multiplied it, and issued the copies between: 1900 cycles per stage for 512 cycles
-// of products.  Four read the next half stage under the products of the present one, and issue their copies (a
-// scalar address and a lane's constant offset) between the products: 1440 cycles.  Reads ahead alone gave 1600; a fifth
-// wavefront that touched the lines of stages further ahead, so that copies find them in the L2, nothing.
+// in step read a half stage, waited, multiplied it, and issued the copies between.  Four read the next half stage under
+// the products of the present one, and issue their copies (a scalar address and a lane's constant offset) between the
+// products: down of llama3.1-8B at 1024 rows, 224 stages with 512 cycles of products each, 173 -> 136 us.  A fifth
+// wavefront that touched the lines of stages further ahead, so that copies find them in the L2, gave nothing.
 template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, int NWV = 8>
 __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
                                                           const bf16* __restrict__ X, int ldx,
@@ -960,9 +961,10 @@ constexpr bool splits_k() {
 }
 
 // LDS stages per tile shape.  Measured on MI355X (bench/prefill_gemm_bench.py): the
-// 64-row tiles are latency-bound streams and want 3-4 stages in flight; the 128/256-row
-// tiles are MFMA-bound at large M, where two blocks share a CU and hide each other's
-// loads, and lose more to 1-block/CU occupancy than they gain from depth.
+// 64-row tiles are latency-bound streams and want 3-4 stages in flight; tiles of 128 rows and more
+// on eight waves are MFMA-bound at large M, where two blocks share a CU and hide each other's
+// loads, and lose more to 1-block/CU occupancy than they gain from depth; those on four waves, one
+// to a SIMD, have the CU's LDS to themselves.
 template <int BM, int BN>
 constexpr int stages_for() {
   if constexpr (waves_for<BM, BN>() == 4) return (160 * 1024) / ((BM + BN) * BK * 2);
@@ -1125,9 +1127,10 @@ static bool tile_fits(int tile, int N, int epi) {
 // The tile of a shape, 0 where N does not divide.  M <= 64
 // uses the 64-row tiles (no MFMA work or DMA on padding rows beyond one tile).  128-row tiles run on four
 // wavefronts that read ahead (prefill_gemm_kernel, NWV).  llama3.1-8B, cold weights, us, eight wavefronts in step (and
-// the tiles of 192 and 320 rows picked beside them) / now: o 128 rows 29 / 22, 400 rows 41 / 33, 1024 rows 64 / 50;
-// down 43 / 37, 101 / 75, 186 / 135 (890 TFLOP/s); qkv 27 / 24, 54 / 39, 95 / 55.  What is left there is each
-// wavefront's own chain: a wait for all wavefronts per 64 numbers of K beside 512 cycles of products.
+// the tiles of 192 and 320 rows picked beside them) / now, 128, 400 and 1024 rows: o 29 / 23, 40 / 33, 58 / 50; down
+// 42 / 41, 95 / 73, 173 / 136 (890 TFLOP/s); qkv with the rows' scales and the rotation 32 / 27, 60 / 49, 91 / 66 (780).
+// What is left there is each wavefront's own chain: a wait for all wavefronts per 64 numbers of K beside 512 cycles of
+// products.
 static int g_tile8 = 1;  // the 192 x 256 gate_up picks below (A/B switch: p2p_prefill_tile8)
 static int pick_tile(int M, int N, int K, int epi) {
   if (N % 128) return 0;
@@ -1154,7 +1157,7 @@ static int pick_tile(int M, int N, int K, int epi) {
   const long small = tiles(128, 128);
   if (small <= cus) return 3;
   // 128 x 128 takes more than one round, a workgroup per CU: a larger tile that takes one.  us, 128 x 128 / 192 x 128 /
-  // 128 x 192 / 128 x 256: normed 9216 x 4096, 448 rows 74 / 68 / 50 / 78; llama3.1-8B qkv, 700 rows 71 / - / 49 / 78;
+  // 128 x 192 / 128 x 256: normed 9216 x 4096, 448 rows 74 / 68 / 50 / 78; llama3.1-8B qkv without its rotation, 700 rows 71 / - / 49 / 78;
   // residual 6144 x 2048, 700 rows 57 / 47 / 44 / 54; SwiGLU 12288 x 2048, 384 rows 46 / 39 / - / 43, 11264 x 2048, 300
   // rows 40 / 38 / - / 43; where only the last fits SwiGLU 6144 x 1024, 1024 rows 30 / 35 / - / 26, 24576 x 4096, 256
   // rows 82 / 110 / - / 79, 200 rows 76 / 111 / - / 78
