@@ -3,7 +3,7 @@
 // Every expert's weights are read, and few rows share them: 700 rows of a model with 8 experts of 4096 x 14336 and 2 per
 // row are 175 slots per expert, 2.8 GB of weights (580 us at a copy's rate) for 490 GFLOP.  So
 //  * an expert's rows sit in ONE row tile where 320 hold them (more are cut into tiles of equal height, not into full
-//    ones and a rest), and products of 16-row fragments past the last row are left out: fragment g of a tile belongs to
+//    ones and a rest; from 256 on where the tiles then still take one round of the CUs), and products of 16-row fragments past the last row are left out: fragment g of a tile belongs to
 //    wave row g % 4, so whatever the height is the waves have the same number of them, but for one;
 //  * the column tiles are narrow (128: 1792 tiles of 28672 columns for 8 experts, seven for every CU, and 256 of 4096);
 //  * what bounds the stream is the bytes in flight per CU, so the weights' ring is as deep as LDS allows and deeper than
@@ -29,6 +29,14 @@ namespace pgemm {
 constexpr int MOE_WM = 4;            // wave rows: a tile of NL fragment rows per wave has NL * 64 rows
 constexpr int MOE_NL = 5;
 constexpr int MOE_ROWS = MOE_NL * 64;
+
+// Row tiles of an expert.  Tiles of more than 256 rows have two stages of rows in flight, which only pays for weights that
+// would be read again: where tiles of 256 rows take one round of the CUs all the same (experts of 4096 x 14336 that a rank
+// has one or two of), the smaller ones are the faster (down, us: one expert, 320 rows 254 / 149, two of 320 and 330 262 /
+// 161; 128 x 128 tiles had 199 and 224)
+__device__ __forceinline__ int moe_row_tiles(int cnt, bool tall) {
+  return tall ? (cnt + MOE_ROWS - 1) / MOE_ROWS : (cnt + 255) / 256;
+}
 
 // LDS stages of 64 numbers of K: rows NL * 8 KiB, weights 16 KiB; 160 KiB together
 template <int NL>
@@ -65,7 +73,7 @@ __device__ __forceinline__ void moe_read_b(unsigned at, bf16x8 (&f)[4]) {
 template <int EPI, int NL>
 __device__ __forceinline__ void moe_gemm_body(bf16x8* lds, const bf16x8* __restrict__ Wt, const bf16* __restrict__ X,
                                               int ldx, int M, int K, int n_tiles, int up_off, bf16* __restrict__ out,
-                                              int ldo, const EpiArgs& ea, int idx, int last, int step) {
+                                              int ldo, const EpiArgs& ea, bool tall, int idx, int last, int step) {
   constexpr int WM = MOE_WM, FN = 4, SA = Rings<NL>::A, SB = Rings<NL>::B;
   constexpr int ASTAGE = NL * 512, BSTAGE = 1024;      // bf16x8
   constexpr int LA = 2 * NL, LB = 4;                   // copies per stage of a wavefront that has them
@@ -84,7 +92,7 @@ __device__ __forceinline__ void moe_gemm_body(bf16x8* lds, const bf16x8* __restr
     int before = 0;
     for (int b = 0; b < E; b += 64) {
       const int cnt = b + lane < E ? min(ea.moe_cnt[b + lane], M) : 0;
-      const int c = (cnt + MOE_ROWS - 1) / MOE_ROWS;
+      const int c = moe_row_tiles(cnt, tall);
       int incl = c;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -290,32 +298,36 @@ __global__ __launch_bounds__(NT) void moe_gemm_kernel(const bf16x8* __restrict__
                                                       bf16* __restrict__ out, int ldo, EpiArgs ea) {
   __shared__ __attribute__((aligned(16))) bf16x8 lds[160 * 64];
   const int lane = threadIdx.x & 63;
-  // row tiles in all, and the fragment rows per wave of the tallest
-  int total = 0, tall = 0;
+  // row tiles in all and the 16-row fragments of the tallest, cut at 256 rows and at MOE_ROWS
+  int total[2] = {0, 0}, high[2] = {0, 0};
   for (int b = 0; b < ea.n_experts; b += 64) {
     const int cnt = b + lane < ea.n_experts ? min(ea.moe_cnt[b + lane], M) : 0;
-    int c = (cnt + MOE_ROWS - 1) / MOE_ROWS, h = c ? ((cnt + 15) / 16 + c - 1) / c : 0;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      c += __shfl_xor(c, o, 64);
-      h = max(h, __shfl_xor(h, o, 64));
+    for (int t = 0; t < 2; ++t) {
+      int c = moe_row_tiles(cnt, t), h = c ? ((cnt + 15) / 16 + c - 1) / c : 0;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        c += __shfl_xor(c, o, 64);
+        h = max(h, __shfl_xor(h, o, 64));
+      }
+      total[t] += c;
+      high[t] = max(high[t], h);
     }
-    total += c;
-    tall = max(tall, h);
   }
-  total = __builtin_amdgcn_readfirstlane(total) * n_tiles;
-  const int nl = (__builtin_amdgcn_readfirstlane(tall) + MOE_WM - 1) / MOE_WM;
+  const bool tall = __builtin_amdgcn_readfirstlane(total[0]) * n_tiles > (int)gridDim.x;
+  const int tiles = __builtin_amdgcn_readfirstlane(tall ? total[1] : total[0]) * n_tiles;
+  const int nl = (__builtin_amdgcn_readfirstlane(tall ? high[1] : high[0]) + MOE_WM - 1) / MOE_WM;
   // an XCD's workgroups share a contiguous run of tiles
   const int xcd = blockIdx.x & 7, step = gridDim.x >> 3;
-  const int last = (int)((long long)(xcd + 1) * total / 8);
-  const int idx = (int)((long long)xcd * total / 8) + (blockIdx.x >> 3);
+  const int last = (int)((long long)(xcd + 1) * tiles / 8);
+  const int idx = (int)((long long)xcd * tiles / 8) + (blockIdx.x >> 3);
   if (idx >= last) return;
   switch (nl) {
-    case 1: return moe_gemm_body<EPI, 1>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, idx, last, step);
-    case 2: return moe_gemm_body<EPI, 2>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, idx, last, step);
-    case 3: return moe_gemm_body<EPI, 3>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, idx, last, step);
-    case 4: return moe_gemm_body<EPI, 4>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, idx, last, step);
-    default: return moe_gemm_body<EPI, MOE_NL>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, idx, last, step);
+    case 1: return moe_gemm_body<EPI, 1>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, tall, idx, last, step);
+    case 2: return moe_gemm_body<EPI, 2>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, tall, idx, last, step);
+    case 3: return moe_gemm_body<EPI, 3>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, tall, idx, last, step);
+    case 4: return moe_gemm_body<EPI, 4>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, tall, idx, last, step);
+    default: return moe_gemm_body<EPI, MOE_NL>(lds, Wt, X, ldx, M, K, n_tiles, up_off, out, ldo, ea, tall, idx, last, step);
   }
 }
 

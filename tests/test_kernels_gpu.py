@@ -797,6 +797,46 @@ def test_moe_grouped_tile_heights(counts, H, F):
         assert (out[s].float() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
 
 
+@pytest.mark.parametrize("counts", [[257, 320, 300, 321, 640], [257], [256, 320], [513, 5, 290], [0, 319]])
+@pytest.mark.parametrize("cols", [256, 4096])
+def test_moe_grouped_heights_by_rounds(counts, cols):
+    """Experts of 257 to 320 rows stay whole only where the tiles of 256 rows would take more than a round of the CUs (4096
+    columns of five experts), and are cut into two everywhere else: against fp32 (rounding of one bf16 result and of the
+    SwiGLU's reciprocal: under 2^-8 of the largest)."""
+    from p2p_llm_chat_go_amd.ops import moe as M
+
+    E, R, H = len(counts), max(counts), 128
+    g = torch.Generator().manual_seed(sum(counts) + cols)
+    x = torch.randn(R, H, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(E, 2 * cols, H, generator=g) * H ** -0.5).to(torch.bfloat16)
+    wt = torch.stack([ops.tile_weight(m) for m in w]).to(DEV)
+    n = sum(counts)
+    slots = torch.randperm(n, generator=g).int()
+    rows, o = torch.full((E, R), -1, dtype=torch.int32), 0
+    for e, c in enumerate(counts):
+        rows[e, :c] = slots[o:o + c]
+        o += c
+    cnt, rd, xd = torch.tensor(counts, dtype=torch.int32, device=DEV), rows.to(DEV), -(-n // R)
+    act = torch.full((n, cols), float("nan"), dtype=torch.bfloat16, device=DEV)
+    M.grouped_gemm(wt, cnt, rd, x, xd, R, ops.EPI_SILU, act, norm=True)
+    tw = torch.rand(n, generator=g).to(DEV)
+    out = torch.full((n, 2 * cols), float("nan"), dtype=torch.bfloat16, device=DEV)
+    M.grouped_gemm(wt, cnt, rd, x, xd, R, ops.EPI_STORE, out, row_w=tw)
+    xf = x.float()
+    rs = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5)
+    for e, c in enumerate(counts):
+        if not c:
+            continue
+        s = rows[e, :c].long().to(DEV)
+        at = s // xd
+        z = xf[at] @ w[e].float().to(DEV).T
+        zn = z * rs[at]
+        ref = torch.nn.functional.silu(zn[:, :cols]) * zn[:, cols:]
+        assert (act[s].float() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
+        ref = z * tw[s][:, None]
+        assert (out[s].float() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
+
+
 def test_moe_grouped_on_two_streams():
     """Normed grouped products of 65 to 127 rows on two streams at once: each call has scales of its own."""
     from p2p_llm_chat_go_amd.ops import moe as M
