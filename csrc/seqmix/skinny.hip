@@ -9,7 +9,8 @@
 //  * walk_k, where four such pieces hold K (2048 numbers of bf16, 1024 of fp32): a workgroup reads the activations
 //    once, keeps them in registers and walks over tiles of 16 columns; the next tile's weights (up to 64 KB) are
 //    asked for in one burst while this one is multiplied and summed.
-//  * skinny_k, above and for few columns: one tile per workgroup, two pieces of weights and activations in flight.
+//  * skinny_k, above, for few columns and for K that fills its pieces badly: one tile per workgroup, two pieces of weights
+//    and activations in flight.
 // In a captured graph with cold weights, us, vendor product / skinny_k / walk_k.  bf16, 8 rows: 2048 x 2048 11.2 / 6.0 /
 // 5.8, 4096 x 2048 11.7 / 6.7 / 6.2, 10304 x 2048 14.5 / 13.6 / 11.0, 18432 x 2048 58.7 / 21.3 / 17.0 (4.4 TB/s),
 // 32000 x 2048 34.5 / 32.5 / 26.5 (4.9), 16384 x 512 11.7 / 6.5 / 5.4; 16 rows 10304 x 2048 14.5 / 16.1 / 11.4, one
@@ -186,14 +187,28 @@ static int walkers(int tiles, int products, int pieces) {
   return (tiles + each - 1) / each;
 }
 
+// Whether to walk; both kernels give the same sums.  A wavefront of walk_k loads whole pieces, also past K, and holds them
+// all before it multiplies, where skinny_k leaves out what is past K and multiplies what comes first.  us, bf16, skinny_k /
+// walk_k (fp32 at half the K the same within 5 %):
+//  * a tile per workgroup: 8 rows, 1024 columns, K = 64 2.3 / 2.8, 256 2.5 / 2.8, 512 2.9 / 2.8, 640 3.3 / 3.7, 1024 3.9 /
+//    3.9; three and four pieces: 2048 x 2048 5.4 / 5.5, 4096 x 2048 7.1 / 6.5, 4096 x 1792 6.5 / 6.3;
+//  * several: 8192 columns, K = 512, one row 3.8 / 3.7, 16 rows 4.5 / 4.2; K = 768, one row 4.9 / 5.2, 8 rows 5.6 / 5.5, 16
+//    rows 6.4 / 5.6; K = 896, one row 5.4 / 5.4, 8 rows 6.5 / 5.7; 16384 columns, K = 64, 8 rows 3.0 / 4.7, K = 384 5.7 /
+//    5.2, K = 640, 8 rows 8.0 / 8.0, 16 rows 9.3 / 8.3, K = 1024, 8 rows 11.2 / 8.3.
+static bool walks(int tiles, int pieces, int eighths, int M) {
+  if (pieces > 4) return false;
+  if (tiles <= 256) return eighths == 8 && (pieces <= 2 || tiles >= 192);
+  if (eighths >= 7) return true;
+  return M > 4 && eighths == 6 ? tiles >= (pieces > 1 ? 512 : 768) : M > 8 && eighths == 5 && tiles >= 768;
+}
+
 template <typename T, bool ACT>
 static void launch_tiles(const SkinnyArgs& a, int products, hipStream_t st) {
-  const int tiles = (a.N + 15) / 16, pieces = (a.K + 64 * 16 / (int)sizeof(T) - 1) / (64 * 16 / (int)sizeof(T));
+  constexpr int PIECE = 64 * 16 / (int)sizeof(T);   // numbers of K that the eight wavefronts' pieces hold
+  const int tiles = (a.N + 15) / 16, pieces = (a.K + PIECE - 1) / PIECE;
   const dim3 g(walkers(tiles, products, pieces), products), b(512);
-  // long rows of few columns: a tile per workgroup either way, and what comes first is multiplied first (8 rows, skinny_k /
-  // walk_k: fp32 1024 x 1024 5.3 / 5.6, 2048 x 1024 6.0 / 6.2, 3072 x 1024 6.3 / 6.3, bf16 96 x 2048 5.0 / 5.1, 2048 x 2048
-  // 5.9 / 5.8; two pieces, bf16 1024 x 1024 3.8 / 3.7)
-  if (pieces > 4 || (pieces > 2 && tiles < 128)) hipLaunchKernelGGL((skinny_k<T, ACT>), dim3(tiles, products), b, 0, st, a);
+  if (!walks(tiles * products, pieces, a.K * 8 / (pieces * PIECE), a.M))
+    hipLaunchKernelGGL((skinny_k<T, ACT>), dim3(tiles, products), b, 0, st, a);
   else if (pieces == 4) hipLaunchKernelGGL((walk_k<T, 4, ACT>), g, b, 0, st, a);
   else if (pieces == 3) hipLaunchKernelGGL((walk_k<T, 3, ACT>), g, b, 0, st, a);
   else if (pieces == 2) hipLaunchKernelGGL((walk_k<T, 2, ACT>), g, b, 0, st, a);

@@ -305,13 +305,14 @@ def _skinny(x, w) -> bool:
     """Products that ``csrc/seqmix/skinny.hip`` takes from the library: at most 16 rows of one matrix instruction.  Where
     the lines lie (a captured graph, cold weights, library -> kernel in us, 8 rows unless others are named):
 
-    * bf16, K up to 2048 (activations kept in registers): 12288 x 2048 16.1 -> 12.1, 24576 x 2048 37.3 -> 21.8, 128256 x
-      2048 109 -> 97, 16 rows 108 -> 97; up to 1536 by N, because a tile is small against the sums and barrier that end
-      it: 32000 x 1536 25.7 -> 20.9, 65536 x 1536 40.8 -> 40.5, 128256 x 1536 75 -> 79, 32000 x 640 15.2 -> 14.6, 65536 x
-      640 19.7 -> 27.7; up to 256 sooner: 16384 x 256 7.8 -> 5.1, 16384 x 64 4.3 -> 4.7, 32000 x 128 6.3 -> 7.3,
-      16 rows 8192 x 128 4.5 -> 4.1, 16384 x 128 4.9 -> 5.0.
+    * bf16, K up to 2048 (activations kept in registers where that pays, skinny.hip): 12288 x 2048 16.1 -> 12.1, 24576 x
+      2048 37.3 -> 21.8, 128256 x 2048 109 -> 97, 16 rows 108 -> 97; up to 1536 by N, because a tile is small against the
+      sums and barrier that end it: 32000 x 1536 25.7 -> 20.9, 65536 x 1536 40.8 -> 40.5, 128256 x 1536 75 -> 79, 32000 x
+      640 15.2 -> 13.4, 65536 x 640 19.7 -> 27.7; up to 256 sooner: 16384 x 256 6.4 -> 4.3, 16384 x 64 4.5 -> 3.0, 16 rows
+      8192 x 256 5.7 -> 3.7, 8192 x 64 3.6 -> 2.5.
     * fp32, K up to 1024, the same kernel: 12288 x 1024 31.6 -> 12.9, 32000 x 512 19.0 -> 17.3, 65536 x 512 28.8 -> 31.8,
-      32000 x 128 9.2 -> 8.3, 128256 x 1024 106 -> 92, 16384 x 768 13.8 -> 12.0; few columns stay with the library.
+      32000 x 128 9.2 -> 8.3, 50257 x 128 10.7 -> 9.4, 128256 x 64 16.9 -> 13.6, 128256 x 1024 106 -> 92, 16384 x 768 13.8 ->
+      12.0; few columns stay with the library.
     * Longer K, one workgroup per tile walks all of it: bf16 2048 x 8192 12.9 -> 15.0, 2048 x 4096 12.5 -> 8.3, 4096 x
       4096 15.6 -> 9.9, 6144 x 3072 11.9 -> 13.0, 4 rows 12288 x 4096 24.1 -> 21.1, 16 rows 96 x 4096 7.9 -> 8.9, 8 rows
       7.9 -> 7.6; fp32 2048 x 4096 13.2 -> 15.0, 2048 x 2048 10.5 -> 8.5, 16 rows 4608 x 2048 14.1 -> 16.4, 1024 x 2048
@@ -334,7 +335,7 @@ def _skinny(x, w) -> bool:
     elif x.dtype == torch.float32:
         ep = 4
         if K <= 1024:
-            fits = N >= 1024 and (N <= 32768 or K > 768)
+            fits = N >= 1024 and (N <= 32768 or K > 768 or (K <= 256 and N * K <= 8 << 20))
         else:
             fits = (K <= 2048 and 1024 <= N and N * K <= 8 << 20 and (N <= 8192 or M <= 4)
                     and (M <= 8 or N >= 2048))

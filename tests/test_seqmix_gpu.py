@@ -370,7 +370,8 @@ def test_heads_gated(R, H, V, K, per_head):
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,part", [(1, 1, 1), (8, 17, 9), (16, 4096, 64), (5, 4112, 65), (8, 8203, 128), (16, 13000, 2),
                                       (3, 8200, 256), (2, 4120, 257), (16, 50, 511),
-                                      (7, 5000, 161), (2, 2040, 192), (4, 2032, 192)])
+                                      (7, 5000, 161), (2, 2040, 192), (4, 2032, 192),
+                                      (4, 4112, 57), (16, 8210, 81), (8, 4500, 225), (4, 3080, 192)])
 def test_few_row_products_walk_over_columns(dt, M, N, part):
     """K of ``part`` 16-byte fragments: one to four pieces per wavefront and beyond, whole ones and rests; one to several
     tiles per workgroup, the last one cut; rows with a gap.  Against 64 bits: one rounding of the result and one of each
