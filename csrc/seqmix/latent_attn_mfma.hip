@@ -495,7 +495,12 @@ int p2p_sm_latent_attn_mfma(const void* qa, long sqh, long sqr, const void* cach
     err = (int)hipGetLastError();
   }
   if (err || splits == 1) return err;
-  hipLaunchKernelGGL(latent_attn_merge_k, dim3(grid.x, grid.y, np), dim3(max(64, n * 32)), 0, st, part, units, (bf16*)out,
+  // a thread per column while all workgroups are on the chip together, above that fewer, down to 128 (16 heads, latents of
+  // 512, one portion of 195 rows at 933, 3136 workgroups: 48 with 512 threads, 40 with 128; 8 portions of 113 rows, 6 heads 63
+  // / 45; 128 workgroups, 88 rows of one head at 2109 19 / 24; 8 rows of 8 heads, latents of 448 12 / 13)
+  int threads = max(64, n * 32);
+  while (threads > 128 && (long)grid.x * grid.y * np * threads > 256l * 2048) threads /= 2;
+  hipLaunchKernelGGL(latent_attn_merge_k, dim3(grid.x, grid.y, np), dim3(threads), 0, st, part, units, (bf16*)out,
                      soh, sor, H, rank, HS, splits, n * 32, np);
   return (int)hipGetLastError();
 }
