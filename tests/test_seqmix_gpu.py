@@ -348,7 +348,8 @@ def test_glu_act_by_width(dt, F, off, act):
 
 
 @pytest.mark.parametrize("R,H,V,K,per_head", [(1, 16, 128, 512, False), (8, 3, 40, 72, False), (16, 2, 24, 448, True),
-                                              (9, 1, 1, 8, True), (17, 2, 24, 64, False)])
+                                              (9, 1, 1, 8, True), (17, 2, 24, 64, False),
+                                              (8, 32, 512, 512, False), (8, 32, 513, 512, False)])
 def test_heads_gated(R, H, V, K, per_head):
     """Products of few rows per head with the gate in the epilogue: as the library's product, rounded, and the gate pass
     (one bf16 step apart where the sums round differently), also from rows with a gap and into rows with a gap."""
