@@ -13,7 +13,7 @@
 // Here a workgroup of 8 waves owns 128 output columns (SwiGLU: 64 gate + the matching
 // 64 up columns) and a K slice:
 //   * the activation slice streams through an LDS ring of D + 2 chunk slots by LDS-DMA
-//     (global_load_lds_dwordx4, fragment-major image, conflict-free ds_read_b128), or sits
+//     (global_load_lds_dwordx4 of whole lines, conflict-free ds_read_b128), or sits
 //     in LDS whole when it fits (RES), and is read by all 8 waves: 16 activation rows cost
 //     1/8 of a weight byte, not 1;
 //   * each wave streams its OWN 16-column weight group straight into VGPRs (one 1 KiB
@@ -89,10 +89,17 @@ __device__ __forceinline__ void wait_vmcnt() {
 // the reads go out as asm (the compiler inserts no wait for them) and lds_wait holds their
 // results until they land.
 __device__ __forceinline__ unsigned lds_off(const void* p) { return (unsigned)(uintptr_t)(lds_ptr_t)p; }
-__device__ __forceinline__ bf16x8 lds_rd(const bf16x8* p) {
+template <int OFF>
+__device__ __forceinline__ bf16x8 lds_rd(unsigned at) {
   bf16x8 v;
-  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(lds_off(p)));
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
   return v;
+}
+// N fragments, STEP bytes apart from OFF on
+template <int OFF, int STEP, int N, int I = 0>
+__device__ __forceinline__ void lds_rds(unsigned at, bf16x8 (&a)[N]) {
+  a[I] = lds_rd<OFF + I * STEP>(at);
+  if constexpr (I + 1 < N) lds_rds<OFF, STEP, N, I + 1>(at, a);
 }
 // The LDS DMA itself goes out as asm too: with the builtin's DMA events pending, the
 // compiler's own vmcnt tracking of the weight loads gave up (mixed event kinds on one
@@ -164,6 +171,12 @@ __device__ __forceinline__ void lds_wait(bf16x8 (&a)[N]) {
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
 }
 
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  f(std::integral_constant<int, I>{});
+  if constexpr (I + 1 < N) static_for<N, I + 1>(f);
+}
+
 // chunks of a K slice whose activations fit LDS at once (the RES variant): <= 144 KiB
 template <int MT>
 constexpr int res_chunks() { return 18 / MT; }
@@ -202,7 +215,7 @@ __global__ __launch_bounds__(NW * 64) void wide_gemm_kernel(const bf16x8* __rest
   constexpr int PER_CHUNK = AD + KW;  // vmem instructions per thread per chunk
   constexpr int NSLOT = RES ? res_chunks<MT>() : RING;
   constexpr int NSV = NQ2 * MAX_SPLIT / 4;  // row-sum granules polled per lane (split-K NORM)
-  __shared__ __attribute__((aligned(16))) bf16x8 ring[NSLOT * SLOT];
+  __shared__ __attribute__((aligned(256))) bf16x8 ring[NSLOT * SLOT];
   __shared__ float ss_l[NQ2][4][16];
   __shared__ int slot_l[64], pos_l[64];  // EPI_QKV_ROPE: the rows' KV slots and positions
 
@@ -231,26 +244,30 @@ __global__ __launch_bounds__(NW * 64) void wide_gemm_kernel(const bf16x8* __rest
 
   const int gw = SILU ? (wg < 4 ? tile * 4 + wg : tile * 4 + (wg - 4) + up_off) : tile * 8 + wg;
   const bf16x8* wsrc = Wt + (size_t)gw * S * 64 + lane;
+  // A slot holds, per m-tile, 16 rows x 512 bytes (KC k-steps); wave w copies rows 2 (w & 7) and the one after it, whole
+  // lines (1 KiB as the 16 rows x 64 bytes of one k-step's fragment comes in at 58 KB/us per CU, as lines at 95 to 100).
+  // 16-byte piece p of row R lies at p ^ R, so that a fragment's 16 rows are read without bank conflicts.
+  const int arow = 2 * wg + (lane >> 5), apiece = (lane & 31) ^ arow;
   const bf16* asrc[MT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int row = min(16 * i + (lane & 15), M - 1);
-    asrc[i] = X + (size_t)row * ldx + 8 * (lane >> 4);
-  }
+  for (int i = 0; i < MT; ++i) asrc[i] = X + (size_t)min(16 * i + arow, M - 1) * ldx;
 
-  // Chunk c's loads (nothing past the slice, c >= n).  Activations: wave w loads k-step
-  // w & 7 of the m-tiles of its parity (NW = 16: the odd wave of a pair repeats its last
+  // Chunk c's loads (nothing past the slice, c >= n).  Activations: wave w loads its two rows
+  // of the m-tiles of its parity (NW = 16: the odd wave of a pair repeats its last
   // m-tile when MT is odd, so every wave issues AD instructions -- the same bytes to the same
   // LDS place -- and the counted waits hold).  The weights go out through gload_chunk.
   auto issue_a = [&](int c) {
     bf16x8* base = ring + (c % NSLOT) * SLOT;
-    const int kk = ks0 + c * KC + min(wg, kv_of(c) - 1);
+    const int at = (ks0 + c * KC) * 32 + 8 * min(apiece, 4 * kv_of(c) - 1);   // (a partial chunk repeats its last piece)
 #pragma unroll
     for (int a = 0; a < AD; ++a) {
       const int i = min(par + NPAR * a, MT - 1);
-      dma_lds<16>(asrc[i] + (size_t)kk * 32, base + (i * KC + wg) * 64);
+      dma_lds<16>(asrc[i] + at, base + (i * KC + wg) * 64);
     }
   };
+  // byte address of this lane's piece of k-step k & 3 in a slot; k-steps 4 .. 7 lie 256 bytes, m-tiles 8 KiB further
+  const unsigned fr = (lane & 15) * 512 + (((lane & 15) ^ (lane >> 4)) << 4);
+  auto frag = [&](unsigned slot, int k) { return (slot + fr) ^ ((k & 3) << 6); };   // (slots are aligned to 256 bytes)
   auto issue_w = [&](int c, bf16x8(&wr)[KW]) {
     const int cc = min(c, n - 1);  // (addresses only; no load goes out for c >= n)
     const int kb = ks0 + cc * KC, kl = kv_of(cc) - 1;
@@ -303,7 +320,7 @@ __global__ __launch_bounds__(NW * 64) void wide_gemm_kernel(const bf16x8* __rest
       const bool ok = owns(i) && m < M;
       res[i][j] = 0.f;
       csv[i][j] = float2{1.f, 0.f};
-      if constexpr (EPI == EPI_RESID && !(SPLIT && NW == 16))
+      if constexpr (EPI == EPI_RESID && NW == 8)
         if (ok) res[i][j] = (float)reinterpret_cast<const bf16*>(out)[(size_t)m * ldo + g * 16 + r];
     }
   if constexpr (EPI == EPI_QKV_ROPE)
@@ -319,45 +336,47 @@ __global__ __launch_bounds__(NW * 64) void wide_gemm_kernel(const bf16x8* __rest
   float ss = 0.f;  // NORM: rows of m-tile (w & 3), k-steps = (w >> 2) mod NQ, this lane's 8 k
   const int sq_mt = w & 3, sq_q = w >> 2;
 
-  auto compute_kv = [&](const bf16x8* base, const bf16x8(&wr)[KW], int kv, auto full) {
+  auto compute_kv = [&](unsigned slot, const bf16x8(&wr)[KW], int kv, auto full) {
     constexpr bool FULL = decltype(full)::value;
-#pragma unroll
-    for (int j = 0; j < KW; ++j) {
+    static_for<KW>([&](auto jc) {
+      constexpr int j = decltype(jc)::value, HI = j >= KW / 2 ? 256 : 0;
       const int k = par + NPAR * j;
-      if (!FULL && k >= kv) break;
+      if (!FULL && k >= kv) return;
+      const unsigned at = frag(slot, k);
       // A fragments in flight together: every m-tile's (one at a time for MT = 4 at NW = 16)
       constexpr int AB = (NW == 16 && MT == 4) ? 1 : MT;
-#pragma unroll
-      for (int i0 = 0; i0 < MT; i0 += AB) {
+      static_for<MT / AB>([&](auto ic) {
+        constexpr int i0 = decltype(ic)::value * AB;
         bf16x8 a[AB];
-#pragma unroll
-        for (int i = 0; i < AB; ++i) a[i] = lds_rd(base + ((i0 + i) * KC + k) * 64 + lane);
+        lds_rds<i0 * 8192 + HI, 8192>(at, a);
         lds_wait(a);
 #pragma unroll
         for (int i = 0; i < AB; ++i)
           acc[i0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], wr[j], acc[i0 + i], 0, 0, 0);
-      }
-    }
+      });
+    });
     if constexpr (NORM) {
       if (sq_mt < MT) {
         // reads in flight together: all of the chunk's at NW = 8, one at NW = 16 (128 VGPRs)
         constexpr int NS = KC / NQ, NB = NW == 16 ? 1 : NS;
-#pragma unroll
-        for (int u0 = 0; u0 < NS; u0 += NB) {
+        const unsigned mt_at = slot + sq_mt * 8192;
+        static_for<NS / NB>([&](auto uc) {
+          constexpr int u0 = decltype(uc)::value * NB;
           bf16x8 x[NB];
-#pragma unroll
-          for (int u = 0; u < NB; ++u)  // a partial chunk reads a stale k-step, not summed
-            x[u] = lds_rd(base + (sq_mt * KC + (u0 + u) * NQ + sq_q) * 64 + lane);
+          static_for<NB>([&](auto vc) {  // a partial chunk reads a repeated k-step, not summed
+            constexpr int u = decltype(vc)::value;
+            x[u] = lds_rd<((u0 + u) * NQ >= 4 ? 256 : 0)>(frag(mt_at, (u0 + u) * NQ + sq_q));
+          });
           lds_wait(x);
 #pragma unroll
           for (int u = 0; u < NB; ++u)
             if (FULL || (u0 + u) * NQ + sq_q < kv) ss = sumsq8(x[u], ss);
-        }
+        });
       }
     }
   };
   auto compute = [&](int c, const bf16x8(&wr)[KW]) {
-    const bf16x8* base = ring + (c % NSLOT) * SLOT;
+    const unsigned base = lds_off(ring + (c % NSLOT) * SLOT);
     const int kv = kv_of(c);
     if (kv == KC)
       compute_kv(base, wr, KC, std::true_type{});
@@ -488,6 +507,14 @@ __global__ __launch_bounds__(NW * 64) void wide_gemm_kernel(const bf16x8* __rest
 #pragma unroll
       for (int j = 0; j < 4; ++j) up[i][j] = SILU ? xch[((wg * MT + i) * 4 + j) * 64 + lane] : 0.f;
     }
+    if constexpr (EPI == EPI_RESID && NW == 16)   // (16 waves: no registers for them in the k loop)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int m = 16 * i + 4 * q + j;
+          if (m < M) res[i][j] = (float)reinterpret_cast<const bf16*>(out)[(size_t)m * ldo + g * 16 + r];
+        }
     epilogue(acc, up, [&](int i, int j) {
       if constexpr (!NORM) return 1.f;
       const int rr = 4 * q + j;

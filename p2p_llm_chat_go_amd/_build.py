@@ -131,7 +131,7 @@ def build_seqmix(force=False, jobs=8):
 # Kernels whose k loop streams through inline-asm loads (csrc/kernels/wide_gemm.hip): the
 # compiler does not know those registers are still in flight, so a spill of one would read
 # it before it lands.  Their translation units must compile with zero scratch.
-NO_SCRATCH = {"wide_gemm.hip", "tiled_gemm.hip"}
+NO_SCRATCH = {"wide_gemm.hip", "tiled_gemm.hip", "skinny_gemm.hip"}
 
 
 def check_no_scratch(src, remarks: str, obj=None):

@@ -228,7 +228,7 @@ def main(argv=None):
     ap = argparse.ArgumentParser()
     ap.add_argument("--model", default="llama3.1-8b")
     ap.add_argument("--tp", type=int, default=1, help="tune one rank's shard of a TP group")
-    ap.add_argument("--batch", default="1,2,4,8,16,48,64")
+    ap.add_argument("--batch", default="1,2,4,8,16,32,48,64")
     ap.add_argument("--save", action="store_true")
     a = ap.parse_args(argv)
     os.environ["P2P_AUTOTUNE_TABLE"] = "0"

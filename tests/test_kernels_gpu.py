@@ -157,6 +157,24 @@ def test_midm_gemm_every_epilogue(M, K):
     _every_epilogue(M, MIDM_FLAG, 1000 + M, K=K)
 
 
+@pytest.mark.parametrize("M", [16, 33, 64])
+@pytest.mark.parametrize("K", [128, 640])
+@pytest.mark.parametrize("groups", [257, 513])
+def test_midm_gemm_two_groups_and_short_rows(M, K, groups):
+    """More column groups than CUs (two to a workgroup, the last one alone), fewer chunks of 64 than
+    wavefronts and chunk counts that do not divide; bf16 inputs, fp32 sums: the reference's error is the
+    order of at most 640 fp32 sums, 640 * 2^-24 of the products' absolute sum."""
+    from p2p_llm_chat_go_amd.ops.gemm import MIDM_FLAG
+
+    torch.manual_seed(M + K + groups)
+    N = groups * 16
+    W = (torch.randn(N, K) * 0.05).to(torch.bfloat16)
+    x = torch.randn(M, K).to(torch.bfloat16)
+    out = ops.skinny_gemm(ops.tile_weight(W).to(DEV), x.to(DEV), ops.EPI_F32, norm=False, waves=MIDM_FLAG).cpu()
+    ref, bound = x.double() @ W.double().t(), x.double().abs() @ W.double().abs().t()
+    assert ((out.double() - ref).abs() <= K * 2.0 ** -24 * bound + 1e-30).all()
+
+
 @pytest.mark.parametrize("M", [2, 16, 17, 44, 64])
 @pytest.mark.parametrize("K,split", [(1024, 0), (1024, 1), (1536, 4), (2048, 3), (2048, 8),
                                      (5120, 1), (4096, 5), (4096, 16)])
