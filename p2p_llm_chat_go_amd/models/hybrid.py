@@ -383,6 +383,9 @@ class Mixer:
     # rows that read the layer input as ``w_in`` and implements ``mix`` on their product, so
     # that whoever owns the input (a layer with a gate, a ``parallel`` mixer) can run every
     # projection of the same input as one matrix product.
+    # one_input: forward() reads its input through one product alone, so it also takes rows that are not formed yet
+    # (``sm.NormedRows``)
+    one_input = False
     w_in = None
     b_in = None   # bias of the input product (activation type), or None
     wo = None
@@ -403,6 +406,7 @@ class Mixer:
 
 class GeneralDelta(Mixer):
     kind = "general_delta"
+    one_input = True
     LOW_RANK = 32
 
     @staticmethod
@@ -442,6 +446,7 @@ class GeneralDelta(Mixer):
 
 class Mamba2(Mixer):
     kind = "mamba2"
+    one_input = True
 
     def _dims(self):
         s = self.spec
@@ -473,10 +478,9 @@ class Mamba2(Mixer):
 
     def forward(self, h, b, cache, layer):
         st = cache.state[layer]
-        zx = sm.linear(h, self.w_in)
         conv = torch.empty(b.R, self.C, device=h.device, dtype=torch.float32)
         single = all(e[1] == 1 for e in b.ent_host)   # their tails move on in the convolution's launch
-        sm.mamba_conv(zx, self.inner, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, conv, roll=single)
+        zx = sm.linear_conv(h, self.w_in, self.inner, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, conv)
         y = torch.empty(b.R, self.inner, device=h.device, dtype=torch.float32)
         sm.mamba_scan(conv, zx, self.inner, self.inner + self.C, self.dt_bias, self.A_log, self.Dp,
                       st["S"], st["tail"], b.ent, b.ent_host, y, self.H, self.P, self.N, self.G, roll=not single)
@@ -490,6 +494,7 @@ class Mamba1(Mixer):
     convolution + silu; step sizes (through a rank of ``dt_rank``), B and C are projections of it;
     every channel carries ``state`` numbers with decays of their own."""
     kind = "mamba1"
+    one_input = True
 
     def _dims(self):
         s = self.spec
@@ -518,10 +523,21 @@ class Mamba1(Mixer):
     def cache_spec(self):
         return ("state", {"S": (self.N, self.I), "tail": (self.K - 1, self.I)})
 
+    def forward(self, h, b, cache, layer):
+        if not all(e[1] == 1 for e in b.ent_host):
+            return super().forward(h, b, cache, layer)
+        x = torch.empty(b.R, self.I, device=h.device, dtype=h.dtype)
+        proj = sm.linear_conv(h, self.w_in, 0, self.cw, self.cb, cache.state[layer]["tail"], b.ent, b.ent_host, b.row_ent, x)
+        mid = torch.empty(b.R, self.n_mid, device=h.device, dtype=h.dtype)
+        return sm.linear(self._scan(proj, x, b, cache, layer, mid), self.wo)
+
     def mix(self, proj, b, cache, layer, out, out_scale=1.0):
+        x = torch.empty(b.R, self.I, device=proj.device, dtype=proj.dtype)
+        sm.mamba_conv(proj, 0, self.cw, self.cb, cache.state[layer]["tail"], b.ent, b.ent_host, b.row_ent, x, roll=True)
+        return self._scan(proj, x, b, cache, layer, out, out_scale)
+
+    def _scan(self, proj, x, b, cache, layer, out, out_scale=1.0):
         st, I = cache.state[layer], self.I
-        x = torch.empty(b.R, I, device=proj.device, dtype=proj.dtype)
-        sm.mamba_conv(proj, 0, self.cw, self.cb, st["tail"], b.ent, b.ent_host, b.row_ent, x, roll=True)
         xp = sm.linear(x, self.w_x)
         sm.selective_scan(x, xp, self.rank, self.w_dt, self.dtb, self.A2, self.Dp, proj[:, I:2 * I],
                           st["S"], b.ent, b.ent_host, out)
@@ -534,6 +550,7 @@ class Lightning(Mixer):
     """Linear attention with a constant decay per head (``ops.seqmix.lightning_scan``): silu on q, k
     and v, one RMS norm over all heads with a weight per channel, a sigmoid gate per channel."""
     kind = "lightning"
+    one_input = True
 
     def _dims(self):
         s = self.spec
@@ -580,6 +597,7 @@ def _value_products(w, gated=True):
 
 class LatentAttention(Mixer):
     kind = "latent_attention"
+    one_input = True
 
     def _dims(self):
         s = self.spec
@@ -771,6 +789,7 @@ class ConvAttention(Mixer):
     the window is seen as one key and value, the means of its tokens' as the cache holds them.
     The result leaves through a sigmoid gate per channel and a biased output projection."""
     kind = "conv_attention"
+    one_input = True
 
     def _dims(self):
         s = self.spec
@@ -1252,6 +1271,7 @@ class DenseFF:
     input of the output projection, [R, n_mid]; may return a part of the result that is added
     separately) and ``w_out`` [width, n_mid]."""
     ACT = "silu"
+    one_input = True   # see Mixer
 
     def __init__(self, spec: dict, width: int):
         self.spec, self.width = spec, width
@@ -1830,26 +1850,44 @@ class HybridModel:
             return self._forward_post(b, layer_out)
         if cfg.traits.block == "streams":
             return self._forward_streams(b, layer_out)
-        x = torch.empty(b.R, cfg.width, device=self.device, dtype=torch.float32)
+        x, spare = self._residual(b)
         sm.embed_pos(w.embed, w.pos, b.ids, b.pos, x)
-        h = torch.empty(b.R, cfg.width, device=self.device, dtype=self.dtype)
+        h = rows = torch.empty(b.R, cfg.width, device=self.device, dtype=self.dtype)
         # every post-sublayer pass (norm, layer scale, residual add) also forms the next
         # sublayer's normed input from the updated rows
         sm.rmsnorm(x, w.layers[0].norm1, cfg.eps, h)
         for i, L in enumerate(w.layers):
-            after = w.layers[i + 1].norm1 if i + 1 < len(w.layers) else None
+            after = w.layers[i + 1] if i + 1 < len(w.layers) and layer_out is None else None
             m = L.mixer.forward(h, b, self.cache, i)
-            nxt = L.norm2 if L.ff is not None else after
-            sm.norm_scale_add(x, m, L.norm1b, L.ls1, cfg.eps, next_w=nxt,
-                              next_out=h if nxt is not None else None)
+            nxt = L.norm2 if L.ff is not None else w.layers[i + 1].norm1 if i + 1 < len(w.layers) else None
+            x, spare, h = self._add_norm(x, spare, h, m, L.norm1b, L.ls1, nxt, rows if nxt is not None else None,
+                                         L.ff if L.ff is not None else after and after.mixer)
             if L.ff is not None:
-                sm.norm_scale_add(x, L.ff.forward(h), L.norm2b, L.ls2, cfg.eps, next_w=after,
-                                  next_out=h if after is not None else None)
+                nxt = w.layers[i + 1].norm1 if i + 1 < len(w.layers) else None
+                x, spare, h = self._add_norm(x, spare, h, L.ff.forward(h), L.norm2b, L.ls2, nxt,
+                                             rows if nxt is not None else None, after and after.mixer)
             if layer_out is not None:
                 layer_out.append(x.clone())
         if b.n_out == 0:
             return None
         return self._logits(x, b)
+
+    def _residual(self, b):
+        """The residual rows, and for a step of few rows a second buffer for them (``sm.NormedRows``)."""
+        few = b.R <= sm.NORMED_ROWS and self.device.type == "cuda"
+        x = torch.empty(2 if few else 1, b.R, self.cfg.width, device=self.device, dtype=torch.float32)
+        return x[0], x[1] if few else None
+
+    def _add_norm(self, x, spare, h, y, w, ls, next_w, rows, reader):
+        """A sublayer's result y, normed and scaled, on top of the residual rows x (or where h, what the sublayer read, left
+        them); returns both buffers and the next sublayer's input: ``rows``, or where ``reader``, the next sublayer, takes
+        rows that its product forms, those."""
+        if isinstance(h, sm.NormedRows):
+            x, spare = h.x, h.spare
+        if reader and reader.one_input and spare is not None:
+            return x, spare, sm.NormedRows(x, spare, y, w, ls, self.cfg.eps, next_w, x if rows is None else rows)
+        sm.norm_scale_add(x, y, w, ls, self.cfg.eps, next_w=next_w, next_out=rows)
+        return x, spare, x if rows is None else rows
 
     def _logits(self, x, b: StepBatch):
         cfg, w = self.cfg, self.w
@@ -1859,11 +1897,7 @@ class HybridModel:
 
     def _head(self, hn):
         cfg, w = self.cfg, self.w
-        y = sm.linear(hn, w.head)
-        if not cfg.logit_softcap and cfg.logit_scale == 1.0:
-            return y.float()
-        return sm.softcap(y, cfg.logit_softcap, torch.empty(y.shape, device=y.device, dtype=torch.float32),
-                          scale=cfg.logit_scale)
+        return sm.logits(hn, w.head, cfg.logit_softcap or 0.0, cfg.logit_scale)
 
     def _forward_streams(self, b: StepBatch, layer_out=None):
         """x_t <- sum_s M[s, t] x_s + c_t f(N(sum_s a_s x_s)) per sublayer, N a dynamic tanh: one pointwise
@@ -1995,17 +2029,18 @@ class HybridModel:
         activation type), and the pass that norms and adds what it produced also writes them for
         the next one."""
         cfg, w = self.cfg, self.w
-        x = torch.empty(b.R, cfg.width, device=self.device, dtype=torch.float32)
+        x, spare = self._residual(b)
         # in float32 the sublayers read the residual stream itself
         h = x if self.dtype == torch.float32 else \
             torch.empty(b.R, cfg.width, device=self.device, dtype=self.dtype)
         nxt = None if h is x else h
         sm.embed_rows(w.embed, b.ids, x, nxt, scale=cfg.embed_scale)
         for i, L in enumerate(w.layers):
+            after = w.layers[i + 1].mixer if i + 1 < len(w.layers) and layer_out is None else None
             m = L.mixer.forward(h, b, self.cache, i)
-            sm.norm_scale_add(x, m, L.norm1, None, cfg.eps, next_out=nxt)
+            x, spare, h = self._add_norm(x, spare, h, m, L.norm1, None, None, nxt, L.ff if L.ff is not None else after)
             if L.ff is not None:
-                sm.norm_scale_add(x, L.ff.forward(h), L.norm2, None, cfg.eps, next_out=nxt)
+                x, spare, h = self._add_norm(x, spare, h, L.ff.forward(h), L.norm2, None, None, nxt, after)
             if layer_out is not None:
                 layer_out.append(x.clone())
         if b.n_out == 0:

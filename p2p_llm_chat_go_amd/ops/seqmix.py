@@ -51,6 +51,13 @@ _SIGS = {
                                             c_int, c_float, c_int, c_void_p],
     "p2p_sm_skinny": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                       c_void_p],
+    "p2p_sm_skinny_logits": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_int,
+                             c_void_p],
+    "p2p_sm_skinny_conv": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
+    "p2p_sm_norm_skinny": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int,
+                           c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "p2p_sm_skinny_heads": [c_void_p, ctypes.c_long, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int,
                             c_int, c_int, c_int, c_int, c_void_p],
     "p2p_sm_gdelta_chunk": [c_void_p] * 5 + [c_int, c_void_p, c_int, c_void_p, c_void_p,
@@ -345,9 +352,94 @@ def _skinny(x, w) -> bool:
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+class NormedRows:
+    """The input of a sublayer that a residual pass leaves (``norm_scale_add``: x += N(y) * w * ls, the rows h = x or
+    h = N(x) * next_w), not formed yet.  The one product that reads it forms it on the way in where a kernel does that
+    (``p2p_sm_norm_skinny``: a step of few rows), else the pass runs first.  x: the residual rows, which are in ``spare``
+    afterwards where the product formed them (its workgroups read x until the last one is done); ``x`` and ``spare``
+    then trade places.  h: the buffer for the rows, x itself in float32 without next_w."""
+
+    def __init__(self, x, spare, y, w, ls, eps, next_w, h):
+        self.x, self.spare, self.y, self.w, self.ls, self.eps, self.next_w, self.h = x, spare, y, w, ls, eps, next_w, h
+        self.formed = False
+
+    @property
+    def device(self):
+        return self.x.device
+
+    @property
+    def dtype(self):
+        return self.y.dtype
+
+    def rows(self):
+        """The rows as a tensor."""
+        if not self.formed:
+            norm_scale_add(self.x, self.y, self.w, self.ls, self.eps, next_w=self.next_w,
+                           next_out=None if self.h is self.x else self.h)
+            self.formed = True
+        return self.h
+
+    def _fits(self, w) -> bool:
+        x, y = self.x, self.y
+        M, K = x.shape
+        f32 = y.dtype == torch.float32
+        vecs = x.data_ptr() | self.spare.data_ptr() | self.w.data_ptr() | (_lib.ptr(self.ls) or 0) | \
+            (_lib.ptr(self.next_w) or 0)
+        return (not self.formed and M <= NORMED_ROWS and K <= (1024 if f32 else 2048) and y.is_cuda and y.stride(1) == 1
+                and y.stride(0) % 4 == 0 and y.data_ptr() % (16 if f32 else 8) == 0 and vecs % 16 == 0
+                and _skinny(self.h, w))
+
+    def linear(self, w, b=None, tanh_from=None, conv=None):
+        """The rows times w transposed (plus b), and behind it a convolution (``_conv_args``).  None where no kernel does
+        all that."""
+        if not self._fits(w) or (b is not None and not (b.dtype == self.dtype and b.is_cuda and b.is_contiguous())):
+            return None
+        x, y, spare = self.x, self.y, self.spare
+        (M, K), N = x.shape, w.shape[0]
+        _vec(self.w, K, "w")
+        for v in (self.ls, self.next_w):
+            if v is not None:
+                _vec(v, K, "vector")
+        if conv is not None and (conv[1].shape[1] > 4 or tanh_from is not None):
+            return None
+        out = torch.empty(M, N, device=x.device, dtype=y.dtype)
+        args = _conv_args(M, N, y.dtype, *conv) if conv is not None else (0, 0, 0) + (None,) * 5 + (0, 0)
+        _chk(lib().p2p_sm_norm_skinny(x.data_ptr(), y.data_ptr(), y.stride(0), self.w.data_ptr(), _lib.ptr(self.ls),
+                                      _lib.ptr(self.next_w), self.eps, spare.data_ptr(), None, 0, w.data_ptr(),
+                                      _lib.ptr(b), out.data_ptr(), M, N, K, N if tanh_from is None else tanh_from, *args,
+                                      _f32(y), _st(x)), "norm_skinny")
+        self.x, self.spare, self.formed, self.h = spare, x, True, None
+        return out
+
+
+# Up to so many rows a product forms its input rows itself: every workgroup does that for all of them, which costs as much
+# as the pass from 8 rows on (steps with nine such products 2048 wide, separate passes and convolutions -> formed by the
+# products, us: one row 456 -> 423, two 481 -> 451, four 522 -> 515, eight 586 -> 601, 16 731 -> 797)
+NORMED_ROWS = 4
+
+
+def _conv_args(M: int, N: int, dtype, c0: int, cw, cb, tail, ent, out):
+    """The arguments of a convolution of columns c0 .. of a product of M rows that are one token each (``mamba_conv`` with
+    roll; at most four taps)."""
+    C, taps = cw.shape
+    _rows2d(out, "out")
+    _vec(cb, C, "cb")
+    assert cw.dtype == torch.float32 and cw.is_contiguous() and out.shape == (M, C) and 0 <= c0 and c0 + C <= N
+    assert out.dtype in (torch.float32, dtype) and ent.dtype == torch.int32 and ent.is_contiguous() and ent.shape == (M, 4)
+    assert tail.dtype == torch.float32 and tail.is_contiguous() and tail.shape[1:] == (taps - 1, C)
+    return (c0, C, taps, cw.data_ptr(), cb.data_ptr(), tail.data_ptr(), ent.data_ptr(), out.data_ptr(), out.stride(0),
+            _f32(out))
+
+
 def linear(x, w, b=None, tanh_from=None):
     """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, the shapes of ``_skinny`` on a
-    kernel for few rows.  tanh_from: columns from there on pass a tanh (of the rounded result)."""
+    kernel for few rows.  tanh_from: columns from there on pass a tanh (of the rounded result).  x may be
+    ``NormedRows`` (whose only product this is)."""
+    if isinstance(x, NormedRows):
+        y = x.linear(w, b, tanh_from)
+        if y is not None:
+            return y
+        x = x.rows()
     if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
             b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
         y = F.linear(x, w, b)
@@ -359,6 +451,43 @@ def linear(x, w, b=None, tanh_from=None):
                              w.shape[0], x.shape[1], w.shape[0] if tanh_from is None else tanh_from, _f32(x),
                              _st(x)), "skinny")
     return y
+
+
+def linear_conv(x, w, c0: int, cw, cb, tail, ent, ent_host, row_ent, out):
+    """proj = ``linear(x, w)`` and out = the short convolution of its columns c0 .. (``mamba_conv``); the tails of portions of
+    one token move on.  One launch for few rows that are one token each (a step of 8 rows with four products of 10304 x
+    2048 and 6144 channels 586 -> 563 us, 16 rows 731 -> 710, the head's fp32 logits included)."""
+    single = all(e[1] == 1 for e in ent_host)
+    if single and isinstance(x, NormedRows):
+        proj = x.linear(w, conv=(c0, cw, cb, tail, ent, out))
+        if proj is not None:
+            return proj
+    if isinstance(x, NormedRows):
+        x = x.rows()
+    (M, K), N = x.shape, w.shape[0]
+    if single and 0 < M <= 16 and K <= (1024 if x.dtype == torch.float32 else 2048) and cw.shape[1] <= 4 and _skinny(x, w):
+        proj = torch.empty(M, N, device=x.device, dtype=x.dtype)
+        _chk(lib().p2p_sm_skinny_conv(x.data_ptr(), x.stride(0), w.data_ptr(), proj.data_ptr(), M, N, K,
+                                      *_conv_args(M, N, x.dtype, c0, cw, cb, tail, ent, out), _f32(x), _st(x)),
+             "skinny_conv")
+        return proj
+    proj = linear(x, w)
+    mamba_conv(proj, c0, cw, cb, tail, ent, ent_host, row_ent, out, roll=single)
+    return proj
+
+
+def logits(x, w, cap: float = 0.0, scale: float = 1.0):
+    """fp32 logits of a model's head: x times w transposed, rounded to the activation type, times ``scale`` and capped
+    (``softcap``; cap 0: not)."""
+    if x.dim() == 2 and x.shape[0] <= 16 and _skinny(x, w):
+        y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=torch.float32)
+        _chk(lib().p2p_sm_skinny_logits(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), x.shape[0], w.shape[0],
+                                        x.shape[1], cap, scale, _f32(x), _st(x)), "skinny_logits")
+        return y
+    y = linear(x, w)
+    if not cap and scale == 1.0:
+        return y.float()
+    return softcap(y, cap, torch.empty(y.shape, device=y.device, dtype=torch.float32), scale=scale)
 
 
 def heads_gated(x, w, wt, g, out, per_head: bool = False):

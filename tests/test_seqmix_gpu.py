@@ -294,6 +294,56 @@ def test_gdelta_long_portions(dt, lens, starts, H, D, decay):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(1, 1030, 1024), (2, 4096, 8), (8, 2048, 1000), (9, 40, 512), (16, 10304, 1024),
+                                   (8, 10304, 2048), (16, 2051, 1544)])
+@pytest.mark.parametrize("form", ["plain", "norm", "tanh", "conv", "conv32"])
+def test_products_form_their_rows(dt, M, N, K, form, monkeypatch):
+    """A product that forms its input rows (and convolves its columns) on the way leaves the bits of the separate passes:
+    rows, halves of the workgroup and widths that do not fill, strided y, one to four taps, slots at position 0."""
+    if dt == torch.float32 and K > 1024:
+        pytest.skip("no kernel: longer rows than registers hold")
+    g = torch.Generator().manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    x, spare, h = rnd(M, K), torch.empty(M, K, device=DEV), torch.empty(M, K, device=DEV, dtype=dt)
+    y, w, gain, ls = rnd(M, K + 8).to(dt)[:, :K], (rnd(N, K) * K ** -0.5).to(dt), rnd(K), rnd(K)
+    nw, b = (rnd(K), None) if form in ("norm", "conv32") else (None, rnd(N).to(dt))
+    taps = 1 + (M + N) % 4 if form == "conv32" else 4
+    c0, C = N // 3, N // 2
+    cw, cb, tail = rnd(C, taps), rnd(C), rnd(M + 2, taps - 1, C)
+    ent = [(r, 1, 0 if r == 1 else 5 + r, M + 1 - r) for r in range(M)]
+    entd, re = torch.tensor(ent, dtype=torch.int32, device=DEV), torch.arange(M, dtype=torch.int32, device=DEV)
+    co = torch.empty(M, C, device=DEV, dtype=torch.float32 if form == "conv32" else dt)
+    # the passes one by one
+    x1, t1, co1 = x.clone(), tail.clone(), co.clone()
+    if not sm._skinny(h, w):
+        pytest.skip("no kernel: the library's shape")
+    h1 = torch.empty_like(h)
+    sm.norm_scale_add(x1, y, gain, ls if form != "plain" else None, 1e-5, next_w=nw, next_out=h1)
+    tanh = N // 2 if form == "tanh" else None
+    want = sm.linear(h1, w, None if form.startswith("conv") else b, tanh_from=tanh)
+    monkeypatch.setattr(sm, "NORMED_ROWS", 16)
+    p = sm.NormedRows(x, spare, y, gain, ls if form != "plain" else None, 1e-5, nw, h)
+    x0 = x.clone()
+    if form.startswith("conv"):
+        sm.mamba_conv(want, c0, cw, cb, t1, entd, ent, re, co1, roll=True)
+        t2, co2 = tail.clone(), torch.empty_like(co)   # ... of rows that are there
+        assert torch.equal(sm.linear_conv(h1, w, c0, cw, cb, t2, entd, ent, re, co2), want)
+        assert torch.equal(t2, t1) and torch.equal(co2, co1)
+        got = p.linear(w, conv=(c0, cw, cb, tail, entd, co))
+        assert got is not None
+        assert torch.equal(co, co1) and torch.equal(tail, t1)
+    else:
+        got = p.linear(w, b, tanh)
+        assert got is not None
+    assert torch.equal(got, want) and torch.equal(p.x, x1) and p.x is spare and torch.equal(x, x0)
+    if not form.startswith("conv"):
+        z = (want.float() * 0.5) if tanh is None else None
+        if z is not None and b is None:
+            assert torch.equal(sm.logits(h1, w, 0.0, 0.5), z)
+            assert torch.equal(sm.logits(h1, w, 3.0, 0.5), sm.softcap(want, 3.0, torch.empty_like(z), scale=0.5))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 7, 16, 17])
 @pytest.mark.parametrize("N,K", [(1, 8), (1024, 4), (1040, 64), (1031, 1000), (1025, 2048), (33, 4096), (16, 4104)])
 @pytest.mark.parametrize("off,bias", [(0, False), (8, True), (3, True)])
