@@ -13,7 +13,7 @@
 // expert_gemm: for expert e and each of its slots s: out[s] = x[s / x_div] . W_e^T.  Rows are
 // gathered through the slot lists, so only experts with rows read their weights.  Rows of a multiple of 16
 // bytes run on the matrix cores (a 16 x 64 tile with K split over the wavefronts for decode-sized steps,
-// LDS-staged 128 x 128 or 64 x 64 tiles for prompts); odd shapes run a tiled FMA kernel.  A
+// LDS-staged tiles for prompts); odd shapes run a tiled FMA kernel.  A
 // slot's result does not depend on which other slots share its tile.
 #include "attn_tile.h"
 using namespace sm;
@@ -185,12 +185,14 @@ group_route_k(const T* __restrict__ h, int ldh, const float* __restrict__ wr, in
                  [&](int k, int e) { rows[(size_t)e * ldr + atomicAdd(&cnt[e], 1)] = r * top + k; });
 }
 
-// The same for prompts: a workgroup takes 16 rows, a wavefront each, and the experts' slot counts go up by one
+// The same, a workgroup for 16 rows, a wavefront each for the choice, and the experts' slot counts go up by one
 // atomic per workgroup and expert instead of one per slot (4096 of them on eight addresses took most of the
-// 57 us that 2048 rows of 2048 numbers needed; 20 us now, 606 rows of 1024 14 instead of 21).  Two or four rows
-// per wavefront, with the weights read once for them, measured 22 and 31 us: the chain of one row's sums
-// and choices is what is left.  A logit's sum has the order it has above.
-template <typename T>
+// 57 us that 2048 rows of 2048 numbers needed).
+// NB > 0, up to 16 NB experts: the logits of all rows on the fp32 matrix instruction, W cut among the wavefronts, 16 bytes of
+// a row per load and four of them in flight; the wavefronts' sums meet in LDS.  With a wavefront per row walking W for four
+// experts at a time (NB = 0: many experts, or rows that 16-byte loads do not fit) the chain of one row's loads and sums was
+// what was left: 2048 rows of 2048 numbers, 8 experts 18.3 -> 10.9 us.
+template <typename T, int NB>
 __global__ void __launch_bounds__(1024)
 group_route_rows_k(const T* __restrict__ h, int ldh, const float* __restrict__ wr, int R, int W, int E, int top,
                    int groups, int keep, int score, const float* __restrict__ corr, int gscore, int* __restrict__ ids,
@@ -204,29 +206,78 @@ group_route_rows_k(const T* __restrict__ h, int ldh, const float* __restrict__ w
   int* scnt = (int*)(stop + 16 * top);   // [E] slots of this workgroup, then the place of its first
   int* spick = scnt + E;                 // [16][top] expert
   int* sat = spick + 16 * top;           // [16][top] place among the workgroup's
+  __shared__ f32x4 part[NB > 0 ? 16 : 1][NB > 0 ? NB : 1][64];
   const int lane = threadIdx.x & 63, m = threadIdx.x >> 6, r = blockIdx.x * 16 + m;
   for (int e = threadIdx.x; e < E; e += 1024) scnt[e] = 0;
-  const T* x = h + (size_t)min(r, R - 1) * ldh;
-  for (int e0 = 0; e0 < E; e0 += 4) {
-    const float* w[4];
-    float d[4];
+  if constexpr (NB > 0) {
+    constexpr int EP = 16 / sizeof(T), CH = 4 * EP, U = 4;   // numbers per load, per chunk of a wavefront; chunks at once
+    const int wave = uniform(m), n16 = lane & 15, quad = lane >> 4;
+    const T* x = h + (size_t)min((int)blockIdx.x * 16 + n16, R - 1) * ldh;
+    f32x4 acc[NB];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      w[u] = wr + (size_t)min(e0 + u, E - 1) * W;
-      d[u] = 0.0f;
+    for (int b = 0; b < NB; b++) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave * CH; k0 < W; k0 += U * 16 * CH) {
+      uint4 xv[U];
+      f32x4 wv[U][NB][EP / 4];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int k = k0 + u * 16 * CH + quad * EP, kk = k < W ? k : 0;   // W is a multiple of EP; past it: struck out below
+        xv[u] = *(const uint4*)(x + kk);
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+          for (int q = 0; q < EP / 4; q++)
+            wv[u][b][q] = *(const f32x4*)(wr + (size_t)min(b * 16 + n16, E - 1) * W + kk + q * 4);
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const bool in = k0 + u * 16 * CH + quad * EP < W;
+        if (k0 + u * 16 * CH >= W) break;
+#pragma unroll
+        for (int i = 0; i < EP; i++) {
+          const float xi = in ? ldf((const T*)&xv[u], i) : 0.0f;
+#pragma unroll
+          for (int b = 0; b < NB; b++)
+            acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xi, in ? wv[u][b][i / 4][i % 4] : 0.0f, acc[b], 0, 0, 0);
+        }
+      }
     }
+#pragma unroll
+    for (int b = 0; b < NB; b++) part[wave][b][lane] = acc[b];
+    __syncthreads();
+    // row quad * 4 + i, expert b * 16 + n16 of lane quad * 16 + n16
+    for (int at = threadIdx.x; at < 16 * 16 * NB; at += 1024) {
+      const int row = at / (16 * NB), e = at % (16 * NB);
+      if (e >= E) continue;
+      float v = 0.0f;
+#pragma unroll
+      for (int w = 0; w < 16; w++) v += part[w][e / 16][row / 4 * 16 + e % 16][row % 4];
+      if (bias) v += bias[e];
+      ss[row * E + e] = score ? v : sigmoidf_(v);
+    }
+  } else {
+    const T* x = h + (size_t)min(r, R - 1) * ldh;
+    for (int e0 = 0; e0 < E; e0 += 4) {
+      const float* w[4];
+      float d[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        w[u] = wr + (size_t)min(e0 + u, E - 1) * W;
+        d[u] = 0.0f;
+      }
 #pragma unroll 4
-    for (int i = lane; i < W; i += 64) {
-      const float xv = ldf(x, i);
+      for (int i = lane; i < W; i += 64) {
+        const float xv = ldf(x, i);
 #pragma unroll
-      for (int u = 0; u < 4; u++) d[u] += xv * w[u][i];
-    }
+        for (int u = 0; u < 4; u++) d[u] += xv * w[u][i];
+      }
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      float v = wave_sum(d[u]);
-      if (lane == 0 && e0 + u < E) {
-        if (bias) v += bias[e0 + u];
-        ss[m * E + e0 + u] = score ? v : sigmoidf_(v);
+      for (int u = 0; u < 4; u++) {
+        float v = wave_sum(d[u]);
+        if (lane == 0 && e0 + u < E) {
+          if (bias) v += bias[e0 + u];
+          ss[m * E + e0 + u] = score ? v : sigmoidf_(v);
+        }
       }
     }
   }
@@ -438,10 +489,10 @@ expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
 // beyond the expert's count are skipped.  bf16: one v_mfma_f32_16x16x32_bf16 per pair of 16-byte fragments;
 // fp32: four v_mfma_f32_16x16x4_f32, component by component.
 //
-// Bound by LDS reads and the copies' latency (two or three blocks per CU).  8 experts, 4096 slots, width 2048,
-// gate and up of 1024: 70 us (490 TFLOP/s) and 40 us for the two products against 229 and 117 with register
-// staging, one step at a time; 1212 slots at width 1024: 10.7 and 8.7 us (64 x 64 tiles) against 53 and 29;
-// fp32, 1012 slots, width 1024 and 512: 44 and 24 us against 185 and 94 on vector instructions.
+// Bound by LDS reads and the copies' latency (two or three blocks per CU) and by the last round of the CUs.  8 experts,
+// 4096 slots, width 2048, gate and up of 1024: 50 us (690 TFLOP/s) and 29 us for the two products (160 rows) against 229 and
+// 117 with register staging, one step at a time; 1212 slots at width 1024: 10.7 and 8.7 us (64 x 64 tiles) against 53
+// and 29; fp32, 1012 slots, width 1024 and 512: 37 and 21 us against 185 and 94 on vector instructions.
 template <typename T, int BM, int BN>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
 expert_gemm_tile_k(const T* __restrict__ x, int ldx, int x_div, const T* __restrict__ w,
@@ -667,16 +718,28 @@ int p2p_sm_group_route(const void* h, int ldh, const float* wr, int R, int W, in
   size_t shm = (size_t)(W + 2 * E + groups + top) * 4;
   if (shm > 64 * 1024) return (int)hipErrorInvalidValue;
   const size_t many = (size_t)(16 * (2 * E + groups + 3 * top) + E) * 4;
+#define ROUTE_ROWS(NB)                                                                                          \
+  SM_DISPATCH_T(f32, hipLaunchKernelGGL((group_route_rows_k<T, NB>), dim3((R + 15) / 16), dim3(1024), many, st, \
+                                         (const T*)h, ldh, wr, R, W, E, top, groups, keep, score, corr, gscore, ids, wts, \
+                                         cnt, rows, ldr, bias, renorm, wscale))
+  // Up to 32 experts: sixteen rows' logits on the matrix instruction, unless so few rows that one per workgroup is the
+  // shorter chain (8 experts, us, one / sixteen: bf16, 1024 numbers, 100 rows 7.7 / 7.8, 200 9.7 / 7.9, 606 11.9 / 8.0; 2048
+  // numbers, 100 rows 8.4 / 9.8, 200 10.8 / 9.8, 606 17.6 / 10.0; fp32, 2048 numbers, 200 rows 10.8 / 11.5, 256 12.1 / 11.5)
+  const int ep = f32 ? 4 : 8;
+  if (R >= 200 && E <= 32 && W % ep == 0 && ldh % ep == 0 && (size_t)h % 16 == 0 && (size_t)wr % 16 == 0) {
+    if (E <= 16) ROUTE_ROWS(1);
+    else ROUTE_ROWS(2);
+    return (int)hipGetLastError();
+  }
   // Sixteen rows per workgroup take as long as one row's E sums of W products by one wavefront, whatever R is (until
   // the chip is full); one row per workgroup takes its slots' atomics, R of them, and shares a row's sums among four
   // wavefronts.  us, one / sixteen: E * W = 8192, 256 rows 10.0 / 10.9, 606 rows 18.3 / 11.1; 16384, 606 rows 19 /
   // 17; 65536, 1024 rows 40 / 54, 2048 rows 68 / 55; 262144, 2048 rows 92 / 188
   if (R >= 256 && (size_t)R * 28 >= (size_t)E * W && many <= 48 * 1024) {
-    SM_DISPATCH_T(f32, hipLaunchKernelGGL(group_route_rows_k<T>, dim3((R + 15) / 16), dim3(1024), many, st,
-                                           (const T*)h, ldh, wr, R, W, E, top, groups, keep, score, corr,
-                                           gscore, ids, wts, cnt, rows, ldr, bias, renorm, wscale));
+    ROUTE_ROWS(0);
     return (int)hipGetLastError();
   }
+#undef ROUTE_ROWS
   SM_DISPATCH_T(f32, hipLaunchKernelGGL(group_route_k<T>, dim3(R), dim3(256), shm, st,
                                          (const T*)h, ldh, wr, W, E, top, groups, keep, score, corr,
                                          gscore, ids, wts, cnt, rows, ldr, bias, renorm, wscale));
@@ -696,14 +759,32 @@ int p2p_sm_expert_gemm(const void* x, int ldx, int x_div, const void* w, const i
   const int ep = f32 ? 4 : 8;   // numbers per 16 bytes
   if (K % ep == 0 && ldx % ep == 0 && ((size_t)x & 15) == 0 && ((size_t)w & 15) == 0) {
     if (total_slots >= 64 * E) {   // prompts: tiles
-      // the larger tile needs fewer reads per product, the smaller one gives every CU a block: 160 large
-      // tiles 35 us against 27 (width 2048, 1212 slots), 432 large ones 37.6 against 43 (2400 slots)
-      const long big = (long)((total_slots + 127) / 128 + E) * ((N + 127) / 128);
 #define ET(T, BM, BN)                                                                                        \
   return launch_expert_tile<T, BM, BN>(x, ldx, x_div, w, cnt, rows, ldr, out, ldo, E, N, K, total_slots, epi, \
                                        limit, alpha, st)
-      if (f32) ET(float, 64, 64);
-      if (big >= 384) ET(bf16, 128, 128);
+      // tiles that the slots can be expected to have, half a tile wasted per expert
+      auto tiles = [&](int bm, int bn) { return (long)(total_slots / bm + (total_slots % bm + bm - 1) / bm + E / 2) * ((N + bn - 1) / bn); };
+      if (f32) {
+        // products bound: the smaller the tile, the more evenly the CUs share them (8 experts of width 1024 and 512, gate and
+        // up / down, 64 x 64 -> 32 x 64: 1012 slots 43.8 / 24.1 -> 36.9 / 20.6 us, 600 slots 40.7 / 23.2 -> 25.2 / 15.1;
+        // width 2048, 2000 slots 213 / 111 -> 188 / 98, 4096 slots 346 / 178 beside 351 / 180)
+        if (tiles(64, 64) < 2048) ET(float, 32, 64);
+        ET(float, 64, 64);
+      }
+      // Two blocks of 128 columns to a CU: the height whose rounds take the shortest time, (height + 36) in units of 0.23 us
+      // at K = 2048.  8 experts, us, 64 x 64 / 96 / 128 / 160 rows: width 2048, gate and up, 4096 slots 70 / 58 / 68 / 50
+      // (690 TFLOP/s), 2800 slots 46 / 32 / 37 / 42, 3400 slots 57 / 52 / 40 / 44, down, 4096 slots 39 / 33 / 39 / 29;
+      // width 1024, 4096 slots 25.5 / 18.8 / 23.3 / 26.0; width 4096, 4096 slots 275 / 219 / 200 / 158.  Fewer blocks leave
+      // the small tile ahead: width 2048, 1800 slots 28.7 / 28.0 / 33.9 / 39.4, 1000 slots 24.2 / 26.7, width 1024, 2800
+      // slots 17.9 / 18.7.  (One workgroup of eight wavefronts per CU that reads ahead, as the prompts' products have it,
+      // gave nothing here: 128 x 256 76 us, two rounds, where 128 x 128 had 69.)
+      if (tiles(96, 128) >= 300) {
+        auto time = [&](int bm) { return (tiles(bm, 128) + 511) / 512 * (bm + 36); };
+        const long t96 = time(96), t128 = time(128), t160 = time(160);
+        if (t96 <= t128 && t96 <= t160) ET(bf16, 96, 128);
+        if (t128 <= t160) ET(bf16, 128, 128);
+        ET(bf16, 160, 128);
+      }
       ET(bf16, 64, 64);
 #undef ET
     }

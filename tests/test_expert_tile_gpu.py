@@ -1,6 +1,6 @@
 """Routing of many rows and the tiled expert products against the PyTorch rendering of the same ops:
 experts without slots and with one, counts off the tiles' grid, row lengths that end inside a step,
-columns that end inside a tile, both tile sizes, the activations."""
+columns that end inside a tile, every tile size, the activations."""
 import pytest
 import torch
 
@@ -16,6 +16,9 @@ DEV = "cuda:0"
     (301, 200, 12, 3, 4, 2, dict()),
     (1000, 64, 70, 5, 7, 3, dict(score="softmax", group_score="max", renorm=True, scale=1.5)),
     (259, 40, 3, 1, 1, 1, dict(score="softmax", corr=True)),
+    # 17 to 32 experts, rows longer than the wavefronts' chunks at once; one row fewer than sixteen take
+    (230, 2104, 20, 4, 5, 3, dict(bias=True)), (199, 72, 8, 2, 1, 1, dict(score="top_softmax")),
+    (200, 72, 33, 2, 1, 1, dict()),
     # many experts: a row per workgroup up to R * 28 = E * W, sixteen from there on
     (300, 100, 128, 8, 8, 3, dict(renorm=True)), (365, 80, 128, 8, 8, 3, dict()), (366, 80, 128, 8, 8, 3, dict()),
     (1300, 72, 256, 8, 1, 1, dict(score="softmax"))])
@@ -44,7 +47,9 @@ def test_routing_of_many_rows(dt, R, W, E, top, groups, keep, kw):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("counts,N,K", [
     ([0, 1, 130, 400, 17], 100, 40),        # 64 x 64 tiles; K ends inside a step of either type
-    ([700, 129, 300], 5152, 72),            # 128 x 128 tiles (bf16)
+    ([700, 129, 300], 3000, 72),            # 96 x 128 tiles (bf16)
+    ([700, 129, 300], 5152, 72),            # 128 x 128 (bf16)
+    ([700, 129, 300], 7008, 72),            # 160 x 128 (bf16), 64 x 64 (fp32; the others 32 x 64)
     ([3, 0, 1], 160, 200)])                 # few slots
 @pytest.mark.parametrize("act", [None, "silu_glu", "relu2", "limit"])
 def test_expert_products(dt, counts, N, K, act):
