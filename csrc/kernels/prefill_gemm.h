@@ -4,15 +4,15 @@
 //
 // Tiles BM x BN x 64 (launch_tile has the shapes, pick_tile the choice): 512 threads = 8 waves in a 2 (M) x 4 (N)
 // grid, wave tile (BM/2) x (BN/4) of v_mfma_f32_16x16x32_bf16 accumulators; 128 x 128 and 128 x 192 on 4 waves in a
-// 2 x 2 grid (NWV below).
+// 2 x 2 grid (reads_ahead below).
 // Both operands are staged with `global_load_lds_dwordx4` (one wave-instruction
-// = one 1 KiB MFMA fragment block): the LDS image is fragment-major, so every
-// operand read is a lane-linear, conflict-free ds_read_b128 and no VGPRs or
-// VALU are spent on staging:
-//   * W is fragment-major in HBM already (ops.tile_weight): a block is 1 KiB
-//     contiguous;
-//   * X is row-major: lane l of a block fetches X[row0 + (l&15)][k0 + 8(l>>4) ..]
-//     (per-lane source address, lane-linear destination).
+// = 1 KiB), so no VGPRs or VALU are spent on staging, and read by conflict-free
+// ds_read_b128:
+//   * W is fragment-major in HBM already (ops.tile_weight): a block is one MFMA
+//     fragment, 1 KiB contiguous;
+//   * X is row-major: a block is 8 rows x 128 bytes, whole lines (a CU takes those
+//     in at 95 to 100 KB/us, the 16 rows x 64 bytes of a fragment at 58), 16-byte
+//     piece p of row R at p ^ (R & 7).
 // LDS holds two to six stages of (BM+BN) x 64 bf16 (stages_for, deep_stages_for): later
 // stages are in flight while the MFMAs consume stage kt; one barrier per
 // k-tile.  Blocks sharing a weight n-tile are consecutive after the XCD remap.
@@ -122,11 +122,18 @@ __device__ __forceinline__ void pin_scalars(const T&... v) {
   (pin_scalar(v), ...);
 }
 
-// NWV = 4 (128-row tiles): four wavefronts of 64 x BN/2 instead of eight of 64 x 32, each the only one on its SIMD.  Eight
-// in step read a half stage, waited, multiplied it, and issued the copies between.  Four read the next half stage under
-// the products of the present one, and issue their copies (a scalar address and a lane's constant offset) between the
-// products: down of llama3.1-8B at 1024 rows, 224 stages with 512 cycles of products each, 173 -> 136 us.  A fifth
-// wavefront that touched the lines of stages further ahead, so that copies find them in the L2, gave nothing.
+// Tiles that read ahead (a workgroup has the CU to itself): 128 x 128 and 128 x 192 on four wavefronts of 64 x BN/2, each
+// the only one on its SIMD, 128 x 256 on eight of 64 x 64.  Eight in step read a half stage, waited, multiplied it, and
+// issued the copies between.  These read the next half stage under the products of the present one, and issue their copies
+// (a scalar address and a lane's constant offset) between the products, into the stage whose second half every wave has in
+// registers: down of llama3.1-8B at 1024 rows, in step 173 us, ahead 136 with 128 x 128 (37 % of the time on the matrix
+// cores: the copies' issue and the meeting of the waves are the rest; LDS reads take a fifth of the cycles, no bank
+// conflicts), 118 with 128 x 256, which copies a quarter less per product.  SwiGLU 28672 x 4096, 250 rows, 128 x 256 in
+// step / ahead 85 / 68.  A fifth wavefront that touched the lines of stages further ahead gave nothing; 256 x 128
+// measured as 128 x 256.
+template <int BM, int BN, int NWV>
+constexpr bool reads_ahead() { return NWV == 4 || BM * BN == 128 * 256; }
+
 template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, int NWV = 8>
 __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
                                                           const bf16* __restrict__ X, int ldx,
@@ -134,7 +141,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
                                                           int up_off, void* __restrict__ out,
                                                           int ldo, float eps, EpiArgs ea,
                                                           SplitArgs sp) {
-  constexpr bool PIPE = NWV == 4;
+  constexpr bool PIPE = reads_ahead<BM, BN, NWV>();
   constexpr int NT = NWV * 64;
   constexpr int WN = NWV / 2;        // 2 x WN wave grid
   constexpr int FM = BM / 32;        // 16-row fragments per wave
@@ -184,13 +191,10 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
   const bf16* asrc[AI];
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
-    const int blk = w + NWV * i;  // = mi * 2 + ks
-    const int mi = blk >> 1, ks = blk & 1;
-    int row = m0 + 16 * mi + (lane & 15);
-    // PIPE: 8 rows x 128 bytes per block, 16-byte chunks of row R permuted by R & 7 (see the phased kernel)
-    if constexpr (PIPE) row = m0 + 8 * blk + (lane >> 3);
+    // 8 rows x 128 bytes per block, 16-byte chunks of row R permuted by R & 7 (see the phased kernel)
+    int row = m0 + 8 * (w + NWV * i) + (lane >> 3);
     row = row < M ? row : M - 1;
-    asrc[i] = X + (size_t)row * ldx + (PIPE ? 8 * ((lane & 7) ^ (lane >> 3)) : 32 * ks + 8 * (lane >> 4));
+    asrc[i] = X + (size_t)row * ldx + 8 * ((lane & 7) ^ (lane >> 3));
   }
   const bf16x8* bsrc[BI];
 #pragma unroll
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
       else ldsp::dma_lds16(bbase + (i - AI < HALF ? 0 : to_up) + (size_t)t * 2048, boff[i < AI ? 0 : i - AI], l);
     };
 #pragma unroll
-    for (int t = 0; t < STAGES - 1; ++t)
+    for (int t = 0; t < STAGES; ++t)
       if (t < n)
 #pragma unroll
         for (int i = 0; i < L; ++i) copy(i, t);
@@ -294,8 +298,8 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
       asm volatile("" ::: "memory");   // (the barrier alone does not order reads of LDS)
     };
     bf16x8 a0[FM], b0[FN], a1[FM], b1[FN];
-    // stages 0 .. STAGES - 2 are under way; stage 0 alone has to be there
-    wait_tiles<L, STAGES>(min(STAGES - 2, n - 1));
+    // stages 0 .. STAGES - 1 are under way; stage 0 alone has to be there
+    wait_tiles<L, STAGES + 1>(min(STAGES - 1, n - 1));
     meet();
     // the epilogue's arguments are loaded now, and lgkmcnt(0) is seen by the compiler: with a scalar load under way where
     // the loop begins it waits for all LDS reads before each product
@@ -306,23 +310,26 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
     if constexpr (SPLIT) pin_scalars(sp.splitk, sp.slab, sp.ss_slab, sp.counters, sp.gen, sp.err, sp.parallel);
     __builtin_amdgcn_s_waitcnt(0xc07f);
     read(0, 0, a0, b0);
+    // the second half of stage t is in this wave's registers before it meets the others, so from then on the stage's
+    // slot takes the next copies: a copy has STAGES - 1 stages' time
+    auto used_up = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
     int t = 0;
-    for (; t + STAGES - 1 < n; ++t) {
+    for (; t + STAGES < n; ++t) {
       read(t, 1, a1, b1);
       products(a0, b0, nothing);
-      wait_vmcnt<(STAGES - 3) * L>();   // stage t + 1 is there, for every wave once they met
+      used_up();
+      wait_vmcnt<(STAGES - 2) * L>();   // stage t + 1 is there, for every wave once they met
       meet();
       read(t + 1, 0, a0, b0);
-      // the slot of the stage that is copied held stage t - 1, whose reads every wave had used up before it met the others
       products(a1, b1, [&](int i) {
 #pragma unroll
-        for (int c = i * L / FM; c < (i + 1) * L / FM; ++c) copy(c, t + STAGES - 1);
+        for (int c = i * L / FM; c < (i + 1) * L / FM; ++c) copy(c, t + STAGES);
       });
     }
     for (; t + 1 < n; ++t) {
       read(t, 1, a1, b1);
       products(a0, b0, nothing);
-      wait_tiles<L, STAGES - 1>(min(STAGES - 3, n - 2 - t));
+      wait_tiles<L, STAGES>(min(STAGES - 2, n - 2 - t));
       meet();
       read(t + 1, 0, a0, b0);
       products(a1, b1, nothing);
@@ -344,7 +351,8 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
   #pragma unroll
         for (int j = 0; j < FN; ++j) bfr[j] = ldsp::lds_rd(sb + (bgi[j] * 2 + ks) * 64 + lane);
   #pragma unroll
-        for (int i = 0; i < FM; ++i) af[i] = ldsp::lds_rd(sa + ((wm * FM + i) * 2 + ks) * 64 + lane);
+        for (int i = 0; i < FM; ++i)
+          af[i] = ldsp::lds_rd(sa + ((wm * FM + i) * 16 + (lane & 15)) * 8 + ((4 * ks + (lane >> 4)) ^ (lane & 7)));
         ldsp::lds_wait(af, bfr);
         // keep the MFMA cluster together against the co-resident wave (guide T5)
         __builtin_amdgcn_s_setprio(1);
@@ -948,7 +956,7 @@ static int cu_count() {
   return cached[dev] > 0 ? cached[dev] : 0;
 }
 
-// Wavefronts of a tile shape: four (prefill_gemm_kernel, NWV) where a workgroup has 128 rows and a CU to itself
+// Wavefronts of a tile shape: four (reads_ahead) where a workgroup has 128 rows and a CU to itself
 template <int BM, int BN>
 constexpr int waves_for() {
   return BM == 128 && BN <= 192 ? 4 : 8;
@@ -963,11 +971,11 @@ constexpr bool splits_k() {
 // LDS stages per tile shape.  Measured on MI355X (bench/prefill_gemm_bench.py): the
 // 64-row tiles are latency-bound streams and want 3-4 stages in flight; tiles of 128 rows and more
 // on eight waves are MFMA-bound at large M, where two blocks share a CU and hide each other's
-// loads, and lose more to 1-block/CU occupancy than they gain from depth; those on four waves, one
-// to a SIMD, have the CU's LDS to themselves.
+// loads, and lose more to 1-block/CU occupancy than they gain from depth; those that read ahead have
+// the CU's LDS to themselves.
 template <int BM, int BN>
 constexpr int stages_for() {
-  if constexpr (waves_for<BM, BN>() == 4) return (160 * 1024) / ((BM + BN) * BK * 2);
+  if constexpr (reads_ahead<BM, BN, waves_for<BM, BN>()>()) return (160 * 1024) / ((BM + BN) * BK * 2);
   if constexpr (BM >= 128) return 2;
   return BN <= 128 ? 4 : 3;
 }
@@ -980,7 +988,7 @@ constexpr int stages_for() {
 // (profiles/r2_prefill_gemm_deep_stages.jsonl): deep applies from 128 rows.
 template <int BM, int BN>
 constexpr int deep_stages_for() {
-  if constexpr (BM < 128 || waves_for<BM, BN>() == 4) return stages_for<BM, BN>();
+  if constexpr (BM < 128 || reads_ahead<BM, BN, waves_for<BM, BN>()>()) return stages_for<BM, BN>();
   constexpr int stage_bytes = (BM + BN) * BK * 2;
   constexpr int most = (160 * 1024) / stage_bytes;
   return most > 6 ? 6 : (most < 2 ? 2 : most);
@@ -995,7 +1003,7 @@ int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_ti
                   int up_off, void* out, int ldo, float eps, const EpiArgs& ea, hipStream_t st,
                   int splitk, char* ws, int par) {
   constexpr int NWV = waves_for<BM, BN>();
-  constexpr size_t SHM = NWV == 4 ? (size_t)STAGES * (BM + BN) * BK * sizeof(bf16) : 0;
+  constexpr size_t SHM = reads_ahead<BM, BN, NWV>() ? (size_t)STAGES * (BM + BN) * BK * sizeof(bf16) : 0;
   const int tiles = m_tiles * n_tiles;
   auto with_lds = [](const void* k) {
     return SHM ? hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SHM) : hipSuccess;
@@ -1036,8 +1044,8 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
   const int tiles = m_tiles * n_tiles;
   const int nk = K / BK;
   const int cus = cu_count();
-  constexpr int NWV = waves_for<BM, BN>();   // four: one workgroup per CU whatever the grid
-  const bool deep_auto = (DEEP > SHALLOW || NWV == 4) && g_deep == 1 && cus > 0 && tiles <= cus;
+  constexpr bool ALONE = reads_ahead<BM, BN, waves_for<BM, BN>()>();   // one workgroup per CU whatever the grid
+  const bool deep_auto = (DEEP > SHALLOW || ALONE) && g_deep == 1 && cus > 0 && tiles <= cus;
   // too few tiles to fill 256 CUs: split K so every CU gets work (>= 4 k-tiles per slice)
   // (measured on MI355X at 8B shapes: ~400 blocks, >= 16 k-tiles per slice); the deep
   // variant keeps the grid at one block per CU instead (power-of-two slices <= CUs/tiles)
@@ -1125,12 +1133,8 @@ static bool tile_fits(int tile, int N, int epi) {
 }
 
 // The tile of a shape, 0 where N does not divide.  M <= 64
-// uses the 64-row tiles (no MFMA work or DMA on padding rows beyond one tile).  128-row tiles run on four
-// wavefronts that read ahead (prefill_gemm_kernel, NWV).  llama3.1-8B, cold weights, us, eight wavefronts in step (and
-// the tiles of 192 and 320 rows picked beside them) / now, 128, 400 and 1024 rows: o 29 / 23, 40 / 33, 58 / 50; down
-// 42 / 41, 95 / 73, 173 / 136 (890 TFLOP/s); qkv with the rows' scales and the rotation 32 / 27, 60 / 49, 91 / 66 (780).
-// What is left there is each wavefront's own chain: a wait for all wavefronts per 64 numbers of K beside 512 cycles of
-// products.
+// uses the 64-row tiles (no MFMA work or DMA on padding rows beyond one tile).  128-row tiles read ahead of their products
+// (prefill_gemm_kernel).  What is left there is a wait for all wavefronts per 64 numbers of K, and a clock of 1.9 GHz.
 static int g_tile8 = 1;  // the 192 x 256 gate_up picks below (A/B switch: p2p_prefill_tile8)
 static int pick_tile(int M, int N, int K, int epi) {
   if (N % 128) return 0;
@@ -1140,28 +1144,43 @@ static int pick_tile(int M, int N, int K, int epi) {
   // (one-m-tile 384 / 448-row tiles for 321-448 rows measured 1.1-1.3x SLOWER than the
   // 128x128 split-K / phased 256x256 picks below and were removed:
   // profiles/r3_prefill_tiles_384_448.jsonl)
-  if (N >= 16384) {
-    // SwiGLU-width projections (gate_up of llama3.1-8B, us, cold weights).  129-192 rows: one m-tile of 192 rows,
-    // 78 beside 80 with 128 x 128.  257-384 and 513-768 rows: 192 x 256 tiles waste fewer rows than the phased
-    // 256 x 256: 288 rows 106 / 112, 352 rows 107 / 108, 600 rows 195 / 204, 768 rows 198 / 208;
-    // 416 rows 193 / 115, 896 rows 278 / 217.  Not where they take a round of the CUs more (20480 x 2560, 600 rows:
-    // 131 / 73), nor up to 200 of them, where launch() cuts K as well (24576 x 4096, 300 rows: 138 / 105; 16384 x 2048:
-    // 74 beside 48 with 192 x 128)
-    if (M > 128 && M <= 192) return 7;
-    if (g_tile8 && N % 256 == 0 && ((M > 256 && M <= 384) || (M > 512 && M <= 768)) && tiles(192, 256) > 200 &&
-        (tiles(192, 256) - 1) / cus == (tiles(256, 256) - 1) / cus)
-      return 8;
-  }
-  // the phased 256x256 kernel pays from ~160 tiles (profiles/r2_prefill_gemm_phased.jsonl)
-  if (N % 256 == 0 && tiles(256, 256) >= 160) return 1;
   const long small = tiles(128, 128);
-  if (small <= cus) return 3;
+  const bool resid = epi == EPI_RESID;
+  if (small <= cus) {
+    // One round of 128 x 128 tiles, K cut where they leave CUs idle.  128 x 256 tiles copy a quarter less per product and
+    // take twice the slices: they pay where a slice keeps 2048 numbers and four slices fill the chip.  Residual, us,
+    // 128 x 128 / 128 x 256: 4096 x 14336, 300, 398, 512, 1024 rows 65 / 60, 73 / 62, 81 / 69, 135 / 118 (1020 TFLOP/s);
+    // 8192 x 28672, 256 rows 163 / 140; 4096 x 8192, 398 and 1024 rows 48 / 44, 82 / 77; 4096 x 6144, 700 rows (two
+    // slices) 60 / 56, 398 rows (four) 41 / 41; eight slices: 4096 x 14336, 256 rows 50 / 55; 4096 x 4096, 1024 rows
+    // 50 / 49.5, plain 40 / 44
+    const long wide = N % 256 == 0 ? tiles(128, 256) : 0;
+    return wide * 8 > cus && K >= 6144 && K >= (wide * 4 > cus ? 2 : 4) * 2048 && wide <= cus ? 2 : 3;
+  }
+  if (N >= 16384 && M > 128 && M <= 192) return 7;   // one row of tiles, 192 x 128: SwiGLU 28672 x 4096 62 us, 128 x 128 81
+  if (N % 256 == 0 && !(resid && K <= 3072)) {
+    // More than a round of 128 x 128: the tile whose rounds of the CUs take the shortest time.  Relative times of a round,
+    // from SwiGLU of 16384 to 36864 columns and K = 2048 and 4096 (us at 4096, phased 256 x 256 / 192 x 256 / 128 x 256 /
+    // 192 x 128; in brackets what the lines by rows before had): 28672 columns, 250 rows 126 / 95 / 68 / 91 [85], 300 rows
+    // 107 / 94 / 108 / - [100], 512 rows 113 / 174 / 119 / 145 [119], 600 rows 202 / 179 / 161 / 174 [190], 1024 rows 211 /
+    // 257 / 225 / - [213]; 22016 columns, 300 rows 104 / 130 / 98 / 85 [104], 600 rows 198 / 174 / 116 / 141 [188]; 36864
+    // columns, 300 rows 203 / 176 / 116 / 145 [194]; 12288 x 2048, 400 rows 58 / - / 32 / 44 [43], 700 rows 98 / - / 57 /
+    // 49 [79].  128 x 192, without SwiGLU: 6144 x 4096, 700 rows 46, 128 x 256 51, 192 x 128 52.  192 x 256 up to 200 tiles:
+    // launch() cuts K there as well (22016 columns above); phased: from 160 tiles (profiles/r2_prefill_gemm_phased.jsonl).
+    auto time = [&](int bm, int bn, int round) { return (tiles(bm, bn) + cus - 1) / cus * round; };
+    int best = 2;
+    long t = time(128, 256, 57);
+    auto take = [&](int tile, long other) {
+      if (other < t) t = other, best = tile;
+    };
+    take(7, time(192, 128, 44));
+    if (tile_fits(9, N, epi) && !(resid && K <= 1024)) take(9, time(128, 192, 43));
+    if (g_tile8 && tiles(192, 256) > 200) take(8, time(192, 256, 87));
+    if (tiles(256, 256) >= 160) take(1, time(256, 256, 103));
+    return best;
+  }
   // 128 x 128 takes more than one round, a workgroup per CU: a larger tile that takes one.  us, 128 x 128 / 192 x 128 /
-  // 128 x 192 / 128 x 256: normed 9216 x 4096, 448 rows 74 / 68 / 50 / 78; llama3.1-8B qkv without its rotation, 700 rows 71 / - / 49 / 78;
-  // residual 6144 x 2048, 700 rows 57 / 47 / 44 / 54; SwiGLU 12288 x 2048, 384 rows 46 / 39 / - / 43, 11264 x 2048, 300
-  // rows 40 / 38 / - / 43; where only the last fits SwiGLU 6144 x 1024, 1024 rows 30 / 35 / - / 26, 24576 x 4096, 256
-  // rows 82 / 110 / - / 79, 200 rows 76 / 111 / - / 78
-  const bool tall = tiles(192, 128) <= cus, resid = epi == EPI_RESID;
+  // 128 x 192: normed 9216 x 4096, 448 rows 74 / 68 / 50; residual 6144 x 2048, 700 rows 57 / 47 / 44
+  const bool tall = tiles(192, 128) <= cus;
   if (!(resid && K <= 1024) && tile_fits(9, N, epi) && tiles(128, 192) <= cus) return 9;
   if (tall) return 7;
   // no tile takes one.  Two workgroups on a CU hide what one waits for: the reads of the residual, the first and the last

@@ -208,7 +208,7 @@ P2P_API void p2p_prefill_phased(int on) { pgemm::g_phased = on ? 1 : 0; }
 // one block per CU (default), 2 = deep variant always.
 // Precomputed per-row rstd for normed prefill GEMMs (A/B): 1 = on (default), 0 = in-loop sums.
 P2P_API void p2p_prefill_pre_rstd(int on) { pgemm::g_pre_rstd = on ? 1 : 0; }
-// 192 x 256 tiles for SwiGLU-width projections of 257-384 and 513-768 rows (A/B): 1 = on (default)
+// 192 x 256 tiles where their rounds are the shortest (A/B): 1 = on (default)
 P2P_API void p2p_prefill_tile8(int on) { pgemm::g_tile8 = on ? 1 : 0; }
 
 P2P_API void p2p_prefill_deep(int mode) { pgemm::g_deep = (mode >= 0 && mode <= 2) ? mode : 1; }

@@ -44,6 +44,14 @@ def test_every_width_of_128_columns_has_a_tile(epi):
     assert L.p2p_prefill_tile(700, 6144, 4096, G.EPI_QKV_ROPE) == 9   # one round of 128 x 192
     assert L.p2p_prefill_tile(700, 6144, 4096, G.EPI_SILU) == 7       # ... and of 192 x 128
     assert L.p2p_prefill_tile(2048, 3072, 1024, G.EPI_RESID) == 6     # short rows: two tiles to a CU
+    # long rows: 128 x 256 in two slices of K, in four of 2048 and more, 128 x 128 where they would be shorter or eight
+    for M, N, K, tile in ((1024, 4096, 14336, 2), (398, 4096, 14336, 2), (200, 4096, 14336, 3), (700, 4096, 6144, 2),
+                          (398, 4096, 6144, 3), (1024, 4096, 4096, 3)):
+        assert L.p2p_prefill_tile(M, N, K, G.EPI_RESID) == tile, (M, N, K)
+    # SwiGLU widths: the tile whose rounds of 256 CUs are the shortest
+    for M, N, tile in ((128, 28672, 3), (150, 28672, 7), (250, 28672, 2), (300, 28672, 8), (500, 28672, 1), (700, 28672, 2),
+                       (1024, 28672, 1), (300, 22016, 7), (600, 22016, 2), (300, 36864, 2)):
+        assert L.p2p_prefill_tile(M, N, 4096, G.EPI_SILU) == tile, (M, N)
     assert L.p2p_prefill_tile(300, 100, 1024, epi) == 0 and L.p2p_prefill_tile(300, 256, 100, epi) == 0
 
 

@@ -944,10 +944,10 @@ def test_tiled_gemm(M, epi, tiled_cfg):
 
 
 @pytest.mark.parametrize("epi", ["store", "store_norm", "resid", "f32", "silu"])
-@pytest.mark.parametrize("tile,splitk,nk", [(t, 1, n) for t in (3, 9) for n in (1, 2, 3, 4, 5, 6, 11)] +
-                         [(3, 2, 9), (3, 4, 17), (3, 8, 33), (3, 3, 12)])
+@pytest.mark.parametrize("tile,splitk,nk", [(t, 1, n) for t in (2, 3, 9) for n in (1, 2, 3, 4, 5, 6, 11)] +
+                         [(3, 2, 9), (3, 4, 17), (3, 8, 33), (3, 3, 12), (2, 2, 9), (2, 4, 17), (2, 8, 33)])
 def test_tiled_gemm_read_ahead(epi, tile, splitk, nk):
-    """128-row tiles on four wavefronts: K from one stage to more than the ring holds, rows that fill a tile and that do
+    """128-row tiles that read ahead: K from one stage to more than the ring holds, rows that fill a tile and that do
     not, K slices of uneven length, against fp32 (rounding of one bf16 result: 2^-8 of the largest)."""
     from p2p_llm_chat_go_amd.ops.gemm import set_tiled_min_m, tiled_config
 
