@@ -1250,15 +1250,18 @@ def _attn_f32(q, sqh: int, sqr: int, sqm: int, pool, vbase: int, block_tables, r
               out_scale: float = 1.0, cap: float = 0.0, r1=None, r2=None, gate=None, ldg: int = 0, gpc: int = 0,
               blk=None, every: int = 0, keep: int = 0, maps: int = 1):
     """most: a bound of the keys a row sees (None: windows are not cut).  A step of fewer workgroups
-    than two per CU cuts its windows into runs of at least 128 keys (two tiles per wavefront)."""
+    than two per CU cuts its windows into runs of at least 128 keys, of 64 where those do not make more than two (8
+    heads, us, runs of 128 / 64: latents of 512, tokens at 300 and 90 43 / 22 with the kernel that takes them together, 8
+    heads of 128 on 2 17 / 15); short windows of short keys are not worth the merge (100 rows 14 / 16)."""
     U, hs = units.shape[0], 16 // latent_rows_per_wave(H // G)
     blocks, splits = U * G * maps * (-(-(H // G) // hs)), 1
     if most is not None and blocks < LATENT_SPLIT_BLOCKS:
-        splits = max(1, min(-(-most // 128), LATENT_SPLIT_BLOCKS // blocks, 64))
+        few = blocks * -(-most // 64) <= LATENT_SPLIT_BLOCKS and (most > 128 or max(D, V) > 128)
+        splits = max(1, min(-(-most // (64 if few else 128)), LATENT_SPLIT_BLOCKS // blocks, 64))
     L, part = lib(), None
     if splits > 1:
         L.p2p_sm_attn_f32_ws.restype = c_long
-        part = torch.empty(L.p2p_sm_attn_f32_ws(U, H, G, V, splits, maps), device=q.device, dtype=torch.float32)
+        part = torch.empty(L.p2p_sm_attn_f32_ws(U, H, G, D, V, splits, maps), device=q.device, dtype=torch.float32)
     _chk(L.p2p_sm_attn_f32(q.data_ptr(), sqh, sqr, sqm, pool.data_ptr(), pool.shape[1], vbase, block_tables.data_ptr(),
                            block_tables.shape[1], row_ent.data_ptr(), pos.data_ptr(), units.data_ptr(), U,
                            _lib.ptr(sink), scale, win, out.data_ptr(), soh, sor, som, H, G, D, V, page, splits,
