@@ -1,7 +1,7 @@
 """Stochastic token sampling (temperature -> top-k -> top-p -> draw) on the GPU.
 
-``sample`` runs ``sampling.hip`` (one workgroup per row, radix-select top-k,
-graph-capturable: every per-row parameter is a device tensor and the random
+``sample`` runs ``sampling.hip`` (group maxima of the whole row by many workgroups, then one workgroup per
+row over the groups that can hold the top k; graph-capturable: every per-row parameter is a device tensor and the random
 stream is a counter-based hash of (seed, position, token id)).  CPU tensors run
 ``sample_ref``, the same algorithm in PyTorch with the same hash, which is the
 numerics oracle of the kernel test.
@@ -71,6 +71,13 @@ def sample_ref(logits, temp, topk, topp, seeds, pos, out, cand_ids=None):
     return out
 
 
+def _groups(L, logits):
+    """Workspace of the group maxima (None for rows that one workgroup selects alone)."""
+    B, V = logits.shape
+    n = L.p2p_sample_groups(V)
+    return torch.empty(B, n, dtype=torch.int32, device=logits.device) if n else None
+
+
 def sample(logits: torch.Tensor, temp: torch.Tensor, topk: torch.Tensor, topp: torch.Tensor,
            seeds: torch.Tensor, pos: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """logits fp32 [B, V] -> int32 ids [B].  temp/topp fp32 [B], topk int32 [B],
@@ -84,9 +91,11 @@ def sample(logits: torch.Tensor, temp: torch.Tensor, topk: torch.Tensor, topp: t
     assert temp.dtype == torch.float32 and topp.dtype == torch.float32
     assert topk.dtype == torch.int32 and pos.dtype == torch.int32 and seeds.dtype == torch.int64
     L = _lib.lib()
+    ws = _groups(L, logits)
     _lib.check(L.p2p_sample(logits.data_ptr(), logits.stride(0), B, V, temp.data_ptr(),
                             topk.data_ptr(), topp.data_ptr(), seeds.data_ptr(), pos.data_ptr(),
-                            out.data_ptr(), _lib.stream_ptr(logits.device)), "sample")
+                            out.data_ptr(), 0 if ws is None else ws.data_ptr(),
+                            _lib.stream_ptr(logits.device)), "sample")
     return out
 
 
@@ -108,8 +117,10 @@ def topk_candidates(logits: torch.Tensor, id_off: int, cand_v: torch.Tensor,
         return cand_v, cand_id
     assert logits.dtype == torch.float32 and logits.stride(1) == 1
     L = _lib.lib()
+    ws = _groups(L, logits)
     _lib.check(L.p2p_topk_candidates(logits.data_ptr(), logits.stride(0), B, V, int(id_off),
                                      cand_v.data_ptr(), cand_id.data_ptr(),
+                                     0 if ws is None else ws.data_ptr(),
                                      _lib.stream_ptr(logits.device)), "topk_candidates")
     return cand_v, cand_id
 

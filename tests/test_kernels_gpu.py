@@ -1291,6 +1291,55 @@ def test_sample_kernel_matches_reference(V):
     assert agree >= B - 2, (agree, B)
 
 
+@pytest.mark.parametrize("V,ld", [(16256, 16256), (16257, 16260), (32000, 32001), (128256, 128256), (262144, 262144),
+                                  (262145, 262145)])
+def test_sampling_by_groups_is_the_whole_row(V, ld):
+    """Rows of 128 to 2048 groups of 128 logits are selected from their group maxima: the same candidates in the
+    same order and the same tokens, to the bit, as one workgroup over the whole row (a null workspace)."""
+    from p2p_llm_chat_go_amd.ops import _lib
+
+    L = _lib.lib()
+    assert (L.p2p_sample_groups(V) > 0) == (16256 < V <= 262144)
+    torch.manual_seed(V)
+    B = 12
+    buf = (torch.randn(B, ld) * 3).to(DEV)
+    lg = buf[:, :V]
+    lg[1] = torch.round(lg[1])           # ties everywhere
+    lg[2] = -1.5                         # one value: more logits at the bound than are ranked
+    lg[3, :300] = 9.0                    # a tie wider than k inside three groups
+    lg[4] = float("-inf")                # a masked row: 60 allowed ids, the last one among them
+    lg[4, V - 60::1] = torch.randn(60, device=DEV)
+    lg[5] = -lg[5].abs() - 1.0           # the top of the row is 0 and -0
+    lg[5, 7::101] = 0.0
+    lg[5, 9::103] = -0.0
+    lg[6, ::2] = float("nan")            # greedy (below): NaN is never chosen
+    lg[7] = float("nan")
+    lg[8] = float("-inf")
+    temp = torch.full((B,), 0.8, device=DEV)
+    temp[6:10] = 0.0
+    topk = torch.tensor([40, 128, 40, 40, 0, 64, 40, 40, 40, 40, 1, 7], dtype=torch.int32, device=DEV)
+    topp = torch.full((B,), 0.9, device=DEV)
+    seeds = torch.arange(B, dtype=torch.int64, device=DEV) * 7919 + 1
+    pos = torch.arange(B, dtype=torch.int32, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(B * max(1, L.p2p_sample_groups(V)), dtype=torch.int32, device=DEV)
+    got = []
+    for w in (0, ws.data_ptr()):
+        ids = torch.full((B,), -1, dtype=torch.int32, device=DEV)
+        _lib.check(L.p2p_sample(lg.data_ptr(), ld, B, V, temp.data_ptr(), topk.data_ptr(), topp.data_ptr(),
+                                seeds.data_ptr(), pos.data_ptr(), ids.data_ptr(), w, st), "sample")
+        cv = torch.empty(6, 128, device=DEV)
+        ci = torch.empty(6, 128, dtype=torch.int32, device=DEV)
+        _lib.check(L.p2p_topk_candidates(lg.data_ptr(), ld, 6, V, 1000, cv.data_ptr(), ci.data_ptr(), w, st),
+                   "topk_candidates")
+        got.append((ids.cpu(), cv.cpu().view(torch.int32), ci.cpu()))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    ids = got[1][0]
+    assert ids[6] == int(torch.nan_to_num(lg[6], nan=float("-inf")).argmax()) and ids[7] == 0 and ids[8] == 0
+    assert ids[9] == int(lg[9].argmax())
+
+
 @pytest.mark.parametrize("W", [2, 8])
 def test_vocab_parallel_sampling_matches_full_row(W):
     """TP sampling: per-shard top-128 candidates (p2p_topk_candidates) + the draw over the
