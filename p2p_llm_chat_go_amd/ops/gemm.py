@@ -23,7 +23,7 @@ EPI_QKV_ROPE, EPI_ARGMAX = 4, 5
 EPI_AR = 6  # TP row-parallel projection + fused all-reduce + residual (skinny_gemm_ar)
 SKINNY_MAX_M = 64
 
-# Autotuned launch codes: (N, K, epi, norm, m_tile[, "fp8"]) -> waves | (U << 8)
+# Autotuned launch codes: (N, K, epi, norm, m_tile[, "fp8"][, "rows", bucket]) -> waves | (U << 8)
 # (engine/autotune.py)
 _TUNE: dict = {}
 
@@ -111,8 +111,20 @@ def tune_key(wt, M, epi, norm):
     return key + ("fp8",) if _is_f8(wt) else key
 
 
-def set_tune(key, code: int):
+def small_m_key(key, M):
+    """Bucket of its own for 1, 2, 3-4, 5-8 and 9-16 rows, which share a 16-row tile but not a fastest
+    launch: at 1 row o_proj / down of the 8B shapes take 7.1 / 19.3 us on the skinny kernel and 9.3 / 23 us on
+    the whole-K kernel that is the fastest at 16 rows.  None above 16 rows.  Where no such size was
+    tuned the tile's own entry (the largest size tuned in it) holds."""
+    return key + ("rows", 1 << (max(M, 1) - 1).bit_length()) if M <= 16 else None
+
+
+def set_tune(key, code: int, M: int | None = None):
+    """Record a launch code for ``key``; with ``M``, for the bucket of M rows inside its tile as well."""
     _TUNE[key] = int(code)
+    fine = small_m_key(key, M) if M is not None else None
+    if fine is not None:
+        _TUNE[fine] = int(code)
 
 
 TILED_MIN_M = SKINNY_MAX_M + 1  # rows from which the tiled kernel is used (bench override)
@@ -266,7 +278,9 @@ def tiled_split_fault() -> int:
 def _code(wt, M, epi, norm, waves):
     if waves:
         return waves
-    return _TUNE.get(tune_key(wt, M, epi, norm), 0)
+    key = tune_key(wt, M, epi, norm)
+    code = _TUNE.get(small_m_key(key, M)) if M <= 16 else None
+    return _TUNE.get(key, 0) if code is None else code
 
 
 def _untuned(wt, x, epi) -> int:

@@ -65,3 +65,20 @@ def test_grouped_product_has_no_scales_of_its_own():
     assert L.p2p_grouped_gemm(*args, None, None) != 0
     args[8] = at + 2   # rows that the scales' wide loads cannot take
     assert L.p2p_grouped_gemm(*args, at, None) != 0
+
+
+def test_launch_codes_of_few_rows_keep_their_own_size():
+    """1, 2, 3-4, 5-8 and 9-16 rows share a 16-row tile but keep a code each; a size that was not tuned takes the
+    tile's (the largest tuned in it), and sizes above 16 rows have the tile's alone."""
+    w = torch.zeros(16, 8, 16, 32)
+    saved = dict(G._TUNE)
+    try:
+        G._TUNE.clear()
+        for M, code in ((1, 11), (2, 12), (16, 16), (48, 48)):
+            G.set_tune(G.tune_key(w, M, G.EPI_RESID, False), code, M)
+        got = {M: G._code(w, M, G.EPI_RESID, False, 0) for M in (1, 2, 3, 8, 9, 16, 17, 33, 48)}
+        assert got == {1: 11, 2: 12, 3: 16, 8: 16, 9: 16, 16: 16, 17: 0, 33: 48, 48: 48}
+        assert G._code(w, 1, G.EPI_RESID, False, 7) == 7 and G._code(w, 1, G.EPI_SILU, False, 0) == 0
+    finally:
+        G._TUNE.clear()
+        G._TUNE.update(saved)
