@@ -6,7 +6,7 @@
 // carries a block-table row (its sequence) and a context length; a query row
 // is either one decode token or one prefill token (causal: ctx = pos + 1).
 //
-// Grid: (chunk, kv_head, row); a chunk = 4 pages = 256 keys (16 waves x 16 keys).
+// Grid: (kv_head, row, chunk); a chunk = 4 pages = 256 keys (4 waves x 64 keys) or 16 pages (8 waves x 2 x 64).
 // GQA packing: all G = Hq / Hkv query heads of a kv head are scored against the
 // same K/V bytes in one pass (K/V read once per group, not once per q head).
 // With one chunk the block writes the final bf16 output, otherwise fp32
@@ -19,154 +19,161 @@ constexpr int PAGE = 64;
 constexpr int HD = 128;
 constexpr int CHUNK = 4 * PAGE;
 
-// Block = 16 waves = one 256-key chunk of one (row, kv head); wave w owns keys
-// [16w, 16w+16).  QK: lane = (key t = lane>>2, quarter c = lane&3) holds 32 dims of
-// K row t (four 16-B loads) and dots them with the G query heads; the four
-// quarter partials meet by two xor-shuffles.  Softmax over the wave's 16 keys by
-// xor-shuffles over the key bits.  PV: the wave's V rows go to LDS (row stride 272 B:
-// conflict-free 16-B writes and 4-B column reads) and lane owns output dims
-// 2*lane, 2*lane+1 over the 16 keys.  The 16 wave partials (m, l, o) merge
-// through LDS.  Every global load of a wave is issued before any math, so the
-// kernel pays one memory latency; the serial per-lane work is 16 keys deep.
-constexpr int WAVES = 16;
-constexpr int KPW = CHUNK / WAVES;  // keys per wave = 16
-
-template <int G>
-__global__ __launch_bounds__(WAVES * 64) void paged_attn_kernel(
+// One wave takes a page (64 keys) of a chunk at a time, all of its loads before any arithmetic, and keeps the
+// running maximum, sum and output of its pages in registers; the waves of a workgroup meet once, at the end.
+//   S^T[key][head] = K . Q^T  v_mfma_f32_16x16x32_bf16: A = 16 keys x 32 numbers from the page, B = the query heads,
+//                             padded to 16 with zeros; lane (head, key quarter) then holds the scores of
+//                             keys 16 b + 4 quarter + j
+//   O[head][number] += P . V  v_mfma_f32_4x4x1f32 of 16 blocks: a lane holds 8 numbers of one V row (quarter = which
+//                             of 4 keys, so a load is 4 whole rows of 256 B), and the quarter's probabilities
+//                             of 4 heads are the scores' registers as they are (broadcast from the quarter's first
+//                             lanes).  P stays fp32 and V is not moved: no LDS, no transposition.
+// What bounds it: the K and V bytes, 32 KB in flight per wave.  The form before it (16 waves of 16 keys, products by
+// the vector unit from LDS, a 16-way merge of 32 KB) was bound by its LDS traffic, and its order of the grid (chunks
+// first) gave XCDs 0 and 4 the chunks that every row has and 3 and 7 those that few rows have; heads come first now.
+// With the combine, per launch: 19 rows of up to 900 keys, 8 kv heads of 4 (37 MB) 27.8 -> 14.8 us; 20 rows of 200 keys
+// 11.0 -> 8.1; 1 row of 1000 12.7 -> 10.3; 64 rows of 500 (131 MB) 41.0 -> 31.8.
+// <4, 1>: a page per wave, 256-key chunks.  <8, 2>: 1024-key chunks, a quarter of the partial outputs and two pages in
+// turn per wave: 32 rows of 8000 keys 209.6 -> 199.3 us, 2 rows of 30000 55.8 -> 52.3; but at 4 rows of 1000
+// 10.9 against 17.8, so only where its workgroups are two per CU.
+template <int G, int NW, int PPW>
+__global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
     const bf16* __restrict__ q, int ldq, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
     const int* __restrict__ bt, int bt_stride, const int* __restrict__ row_bt,
     const int* __restrict__ ctx_lens, int Hkv, float scale, int n_chunks, bf16* __restrict__ out,
     int ldo, float* __restrict__ part_o, float* __restrict__ part_ml) {
-  const int c = blockIdx.x, h = blockIdx.y, r = blockIdx.z;
+  constexpr int HG = (G + 3) / 4;  // groups of 4 heads
+  const int h = blockIdx.x, r = blockIdx.y, c = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int t = lane >> 2, quarter = lane & 3;
-  // The context length, the block-table row and q are independent loads: issue them
-  // together, and issue the K/V loads before looking at ctx (keys past the context
-  // read the zero-initialised block-table tail = null page 0, always mapped), so the
-  // kernel's dependent-latency chain is row_bt -> page -> K/V, not ctx -> ... -> K/V.
+  const int n = lane & 15, qd = lane >> 4;
+  __shared__ float so[NW][G][HD];
+  __shared__ float sm[NW][G], sl[NW][G];
+
+  // independent loads together: the context length, the block-table row, q
   const int ctx = ctx_lens[r];
   const int rb = row_bt ? row_bt[r] : r;  // null: row r uses block-table row r (decode)
-
-  constexpr int VS = HD + 8;
-  __shared__ bf16x2 qs[G][HD / 2];
-  // V staging (P.V) and the wave partials of O (merge) share one region: the V rows are
-  // dead once every wave has finished its P.V (barrier below), and the union keeps the
-  // block under 80 KiB, i.e. two blocks per CU on long contexts (one block's loads in
-  // flight while the other one computes).
-  constexpr int kVsBytes = WAVES * KPW * VS * 2;
-  constexpr int kSoBytes = WAVES * G * HD * 4;
-  __shared__ __attribute__((aligned(16))) char vs_so[kVsBytes > kSoBytes ? kVsBytes : kSoBytes];
-  auto& vs = *reinterpret_cast<bf16(*)[WAVES][KPW][VS]>(vs_so);
-  auto& so = *reinterpret_cast<float(*)[WAVES][G][HD]>(vs_so);
-  __shared__ float ps[WAVES][G][KPW];
-  __shared__ float sm[WAVES][G], sl[WAVES][G];
-
-  const int key0 = c * CHUNK + w * KPW;  // first key of this wave
-
-  // 1) all global loads first: 32 dims (4 x 16 B) of K and V row `t` per lane
-  bf16x8 kr[4], vr[4];
+  bf16x8 qf[4];
   {
-    const int key = key0 + t;
-    const int pcol = min(key / PAGE, bt_stride - 1);
-    const int page = bt[(size_t)rb * bt_stride + pcol];
-    const size_t off = (((size_t)page * Hkv + h) * PAGE + (key % PAGE)) * HD + quarter * 32;
-    const bf16x8* kp = reinterpret_cast<const bf16x8*>(kc + off);
-    const bf16x8* vp = reinterpret_cast<const bf16x8*>(vc + off);
+    const bf16x2* qp = reinterpret_cast<const bf16x2*>(q + (size_t)r * ldq + (size_t)(h * G + min(n, G - 1)) * HD + 8 * qd);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) kr[i] = kp[i];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) vr[i] = vp[i];
-  }
-  const bf16x2* qrow = reinterpret_cast<const bf16x2*>(q + (size_t)r * ldq + (size_t)h * G * HD);
-  for (int i = tid; i < G * HD / 2; i += WAVES * 64) qs[i / (HD / 2)][i % (HD / 2)] = qrow[i];
-  if (c * CHUNK >= ctx) return;  // block-uniform: the whole chunk is past the context
-  const int n_valid = min(max(ctx - key0, 0), KPW);
-  const bool mine = t < n_valid;
-  __syncthreads();
-
-  float o[G][2];
-  float mg[G], lg[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    o[g][0] = o[g][1] = 0.f;
-    mg[g] = -INFINITY;
-    lg[g] = 0.f;
-  }
-  if (n_valid > 0) {
-    // 2) scores
-    float s[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) s[g] = 0.f;
-    if (mine) {
-      // bf16 dot2 (v_dot2_f32_bf16): K stays packed, 2 MACs per instruction
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const bf16x2 k2 = {kr[i][2 * j], kr[i][2 * j + 1]};
-          const int d2 = quarter * 16 + i * 4 + j;
-#pragma unroll
-          for (int g = 0; g < G; ++g) s[g] = __builtin_amdgcn_fdot2_f32_bf16(qs[g][d2], k2, s[g], false);
-        }
+        const bf16x2 x = qp[16 * s + i];
+        qf[s][2 * i] = n < G ? x[0] : (bf16)0.f;
+        qf[s][2 * i + 1] = n < G ? x[1] : (bf16)0.f;
       }
+  }
+  const int p0 = c * NW * PPW + w;  // this wave's pages: p0, p0 + NW, ...
+  int page[PPW];
 #pragma unroll
-      for (int g = 0; g < G; ++g) s[g] *= scale;
-      bf16x8* vrow = reinterpret_cast<bf16x8*>(&vs[w][t][quarter * 32]);
+  for (int t = 0; t < PPW; ++t) page[t] = bt[(size_t)rb * bt_stride + min(p0 + t * NW, bt_stride - 1)];
+  if (c * NW * PPW * PAGE >= ctx) return;  // block-uniform: the whole chunk is past the context
+
+  f32x4 acc[HG][8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) vrow[i] = vr[i];
+  for (int g = 0; g < HG; ++g)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[g][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int t = 0; t < PPW; ++t) {
+    const int nv = min(ctx - (p0 + t * NW) * PAGE, PAGE);  // keys of the page inside the context
+    if (nv <= 0) break;                                    // wave-uniform
+    // rows past the context are not read (what they hold may be anything): the last valid row stands in
+    const size_t base = ((size_t)page[t] * Hkv + h) * PAGE * HD;
+    bf16x8 kr[4][4], vr[4][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        kr[b][s] = *reinterpret_cast<const bf16x8*>(kc + base + min(16 * b + n, nv - 1) * HD + 32 * s + 8 * qd);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        vr[b][j] = *reinterpret_cast<const bf16x8*>(vc + base + min(16 * b + 4 * qd + j, nv - 1) * HD + 8 * n);
+    __builtin_amdgcn_sched_barrier(0);  // all 32 loads are on their way before the first product waits
+    f32x4 st[4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      st[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) st[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[b][s], qf[s], st[b], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        st[b][j] = 16 * b + 4 * qd + j < nv ? st[b][j] * scale : -INFINITY;
+        mx = fmaxf(mx, st[b][j]);
+      }
     }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m1 = fmaxf(m, mx), alpha = __expf(m - m1);
+    m = m1;
+    float ls = 0.f;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      s[g] += __shfl_xor(s[g], 1, 64);
-      s[g] += __shfl_xor(s[g], 2, 64);
-      float sv = mine ? s[g] : -INFINITY;
-      float m = sv;
+    for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int o2 = 4; o2 < 64; o2 <<= 1) m = fmaxf(m, __shfl_xor(m, o2, 64));
-      const float p = mine ? __expf(sv - m) : 0.f;
-      float l = p;
-#pragma unroll
-      for (int o2 = 4; o2 < 64; o2 <<= 1) l += __shfl_xor(l, o2, 64);
-      mg[g] = m;
-      lg[g] = l;  // the xor-4..32 sum runs over one lane per key (same quarter)
-      if (quarter == 0) ps[w][g][t] = p;
-    }
-    // 3) P.V over the wave's keys (same-wave LDS ops stay in order)
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll 4
-    for (int k = 0; k < n_valid; ++k) {
-      const bf16x2 vv = *reinterpret_cast<const bf16x2*>(&vs[w][k][2 * lane]);
-      const float v0 = (float)vv[0], v1 = (float)vv[1];
+      for (int j = 0; j < 4; ++j) {
+        st[b][j] = __expf(st[b][j] - m);  // -inf -> 0
+        ls += st[b][j];
+      }
+    l = fmaf(l, alpha, ls);
+    if (t > 0) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const float p = ps[w][g][k];
-        o[g][0] = fmaf(p, v0, o[g][0]);
-        o[g][1] = fmaf(p, v1, o[g][1]);
+        const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha), g));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[g >> 2][e][g & 3] *= a;
       }
     }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float v = (float)vr[b][j][e];
+          acc[0][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(st[b][j], v, acc[0][e], 2, 0, 0);
+          if constexpr (HG > 1) acc[1][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(st[b][j], v, acc[1][e], 2, 1, 0);
+        }
   }
-  __syncthreads();  // every wave's P.V has read its V rows: the region becomes `so`
+  // The four quarters hold four keys' parts of the same 8 numbers: each keeps two of them, summed.
+  const auto add32 = [](float a, float b) {  // lanes below 32: a's sum, the others b's
+    const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  };
+  const auto add16 = [](float a, float b) {  // even rows of 16 lanes: a's sum, odd ones b's
+    const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  };
+  const int d0 = 8 * n + 4 * (qd >> 1) + 2 * (qd & 1);
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    so[w][g][2 * lane] = o[g][0];
-    so[w][g][2 * lane + 1] = o[g][1];
-    if (lane == 0) {
-      sm[w][g] = mg[g];
-      sl[w][g] = lg[g];
-    }
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = add32(acc[g >> 2][e][g & 3], acc[g >> 2][e + 4][g & 3]);
+    so[w][g][d0] = add16(y[0], y[2]);
+    so[w][g][d0 + 1] = add16(y[1], y[3]);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (lane < G) {
+    sm[w][lane] = m;
+    sl[w][lane] = l;
   }
   __syncthreads();
   const int Hq = Hkv * G;
-  for (int i = tid; i < G * HD; i += WAVES * 64) {
+  for (int i = tid; i < G * HD; i += NW * 64) {
     const int g = i / HD, d = i % HD;
     float M = -INFINITY;
 #pragma unroll
-    for (int ww = 0; ww < WAVES; ++ww) M = fmaxf(M, sm[ww][g]);
+    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, sm[ww][g]);
     float num = 0.f, den = 0.f;
     if (M != -INFINITY) {
 #pragma unroll
-      for (int ww = 0; ww < WAVES; ++ww) {
+      for (int ww = 0; ww < NW; ++ww) {
         const float e = __expf(sm[ww][g] - M);
         num = fmaf(e, so[ww][g][d], num);
         den = fmaf(e, sl[ww][g], den);
@@ -196,7 +203,7 @@ constexpr int MAX_CHUNKS = 131072 / CHUNK;  // 128K-token contexts
 __global__ __launch_bounds__(HD * CG) void attn_combine_kernel(const float* __restrict__ part_o,
                                                                const float* __restrict__ part_ml,
                                                                const int* __restrict__ ctx_lens,
-                                                               int Hq, int n_chunks,
+                                                               int Hq, int n_chunks, int chunk,
                                                                bf16* __restrict__ out, int ldo) {
   __shared__ float s_e[MAX_CHUNKS];  // exp(m_c - M)
   __shared__ float s_l[MAX_CHUNKS];
@@ -204,7 +211,7 @@ __global__ __launch_bounds__(HD * CG) void attn_combine_kernel(const float* __re
   __shared__ float s_wmax[HD * CG / 64];
   const int r = blockIdx.x, hq = blockIdx.y, tid = threadIdx.x;
   const int d = tid % HD, grp = tid / HD;
-  const int nc = min(min((ctx_lens[r] + CHUNK - 1) / CHUNK, n_chunks), MAX_CHUNKS);
+  const int nc = min(min((ctx_lens[r] + chunk - 1) / chunk, n_chunks), MAX_CHUNKS);
   const size_t base = ((size_t)r * Hq + hq) * n_chunks;
   float mloc = -INFINITY;
   for (int c = tid; c < nc; c += HD * CG) {
@@ -244,9 +251,41 @@ __global__ __launch_bounds__(HD * CG) void attn_combine_kernel(const float* __re
   }
 }
 
+// The same for at most FEW chunks: a thread per output number, every load of it in flight at once.
+constexpr int FEW = 8;
+__global__ __launch_bounds__(4 * HD) void attn_combine_few_kernel(const float* __restrict__ part_o,
+                                                                  const float* __restrict__ part_ml,
+                                                                  const int* __restrict__ ctx_lens,
+                                                                  int Hq, int n_chunks, int chunk,
+                                                                  bf16* __restrict__ out, int ldo) {
+  const int r = blockIdx.x, hq = blockIdx.y * 4 + threadIdx.x / HD, d = threadIdx.x % HD;
+  if (hq >= Hq) return;
+  const int ctx = ctx_lens[r];
+  const size_t base = ((size_t)r * Hq + hq) * n_chunks;
+  float o[FEW], m[FEW], l[FEW];
+#pragma unroll
+  for (int c = 0; c < FEW; ++c) {
+    const size_t i = base + min(c, n_chunks - 1);
+    o[c] = part_o[i * HD + d];
+    m[c] = part_ml[2 * i];
+    l[c] = part_ml[2 * i + 1];
+  }
+  const int nc = min((ctx + chunk - 1) / chunk, n_chunks);
+  float M = -INFINITY, num = 0.f, den = 0.f;
+#pragma unroll
+  for (int c = 0; c < FEW; ++c) M = c < nc ? fmaxf(M, m[c]) : M;
+#pragma unroll
+  for (int c = 0; c < FEW; ++c) {
+    // chunks past the context were not written: not read into the sums either
+    const float e = c < nc && m[c] != -INFINITY ? __expf(m[c] - M) : 0.f;
+    num = fmaf(e, c < nc ? o[c] : 0.f, num);
+    den = fmaf(e, c < nc ? l[c] : 0.f, den);
+  }
+  out[(size_t)r * ldo + (size_t)hq * HD + d] = f2bf(den > 0.f ? num / den : 0.f);
+}
+
 // ---- single-chunk decode attention on MFMA (contexts <= 256 keys: chat decode) ----
-// The 16-wave kernel above spends its time in a serial per-lane P.V loop over LDS and a
-// 16-way cross-wave merge; here 4 waves x 64 keys (= one KV page per wave, so one
+// Opt-in, P in bf16 and V through LDS: 4 waves x 64 keys (= one KV page per wave, so one
 // block-table load per wave) run both products on v_mfma_f32_16x16x32_bf16 with the
 // query heads on the MFMA's N axis (G <= 16, padded with zero rows):
 //   S^T[key][head] = K . Q^T   (A = 16 keys x 32 dims straight from the page, 16 B per
@@ -397,40 +436,55 @@ __global__ __launch_bounds__(MW * 64) void paged_attn_mfma_kernel(
   }
 }
 
-// Opt-in (p2p_paged_attention_mfma(1)): measured on MI355X it is 7.7-7.9 us per launch
-// at 44-256 keys vs 6.3-8.1 us for the 16-wave kernel (profiles/r2_decode_attn_mfma.jsonl):
-// both are bound by the block-table -> K/V load chain, not by the arithmetic.
+// Opt-in (p2p_paged_attention_mfma(1)): 7.7-7.9 us per launch at 44-256 keys, no faster than fp32 probabilities
+// (profiles/r2_decode_attn_mfma.jsonl): bound by the block-table -> K/V load chain, not by the arithmetic.
 static int g_attn_mfma = 0;
+
+template <int G, int NW, int PPW>
+int launch_pages(const void* q, int ldq, const void* kc, const void* vc, const int* bt, int bt_stride,
+                 const int* row_bt, const int* ctx, int R, int Hkv, float scale, int max_ctx, void* out,
+                 int ldo, float* part_o, float* part_ml, hipStream_t st) {
+  constexpr int chunk = NW * PPW * PAGE;
+  const int n_chunks = (max_ctx + chunk - 1) / chunk;
+  hipLaunchKernelGGL((paged_attn_kernel<G, NW, PPW>), dim3(Hkv, R, n_chunks), dim3(NW * 64), 0, st,
+                     (const bf16*)q, ldq, (const bf16*)kc, (const bf16*)vc, bt, bt_stride, row_bt,
+                     ctx, Hkv, scale, n_chunks, (bf16*)out, ldo, part_o, part_ml);
+  int e = (int)hipGetLastError();
+  if (e || n_chunks == 1) return e;
+  if (n_chunks <= FEW)
+    hipLaunchKernelGGL(attn_combine_few_kernel, dim3(R, (Hkv * G + 3) / 4), dim3(4 * HD), 0, st, part_o, part_ml,
+                       ctx, Hkv * G, n_chunks, chunk, (bf16*)out, ldo);
+  else
+    hipLaunchKernelGGL(attn_combine_kernel, dim3(R, Hkv * G), dim3(HD * CG), 0, st, part_o, part_ml, ctx,
+                     Hkv * G, n_chunks, chunk, (bf16*)out, ldo);
+  return (int)hipGetLastError();
+}
 
 template <int G>
 int launch_attn(const void* q, int ldq, const void* kc, const void* vc, const int* bt,
                 int bt_stride, const int* row_bt, const int* ctx, int R, int Hkv, float scale,
-                int n_chunks, void* out, int ldo, float* part_o, float* part_ml, hipStream_t st) {
-  if (n_chunks == 1 && g_attn_mfma) {
+                int max_ctx, void* out, int ldo, float* part_o, float* part_ml, hipStream_t st) {
+  if (max_ctx <= CHUNK && g_attn_mfma) {
     hipLaunchKernelGGL((paged_attn_mfma_kernel<G>), dim3(Hkv, R), dim3(MW * 64), 0, st,
                        (const bf16*)q, ldq, (const bf16*)kc, (const bf16*)vc, bt, bt_stride, row_bt,
                        ctx, Hkv, scale, (bf16*)out, ldo);
     return (int)hipGetLastError();
   }
-  hipLaunchKernelGGL((paged_attn_kernel<G>), dim3(n_chunks, Hkv, R), dim3(WAVES * 64), 0, st,
-                     (const bf16*)q, ldq, (const bf16*)kc, (const bf16*)vc, bt, bt_stride, row_bt,
-                     ctx, Hkv, scale, n_chunks, (bf16*)out, ldo, part_o, part_ml);
-  int e = (int)hipGetLastError();
-  if (e || n_chunks == 1) return e;
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(R, Hkv * G), dim3(HD * CG), 0, st, part_o, part_ml, ctx,
-                     Hkv * G, n_chunks, (bf16*)out, ldo);
-  return (int)hipGetLastError();
+  // 1024-key chunks where they give 512 workgroups and more (measured at the kernel)
+  if (max_ctx >= 1024 && (long long)R * Hkv * ((max_ctx + 1023) / 1024) >= 512)
+    return launch_pages<G, 8, 2>(q, ldq, kc, vc, bt, bt_stride, row_bt, ctx, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, st);
+  return launch_pages<G, 4, 1>(q, ldq, kc, vc, bt, bt_stride, row_bt, ctx, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, st);
 }
 
 }  // namespace
 
-// 1: contexts <= 256 keys run the 4-wave MFMA kernel; 0 (default): the 16-wave kernel.
+// 1: contexts <= 256 keys run the kernel with bf16 probabilities; 0 (default): paged_attn_kernel.
 P2P_API void p2p_paged_attention_mfma(int on) { g_attn_mfma = on; }
 
 // row_bt null = identity (decode batches: row r is sequence r), one dependent load less
 // on the kernel's critical path (row_bt -> page -> K/V becomes page -> K/V).
-// max_ctx bounds the number of 256-key chunks (grid.x); rows whose context is
-// shorter exit early.  part_o / part_ml: workspace of R*Hq*n_chunks*(128 | 2) floats,
+// max_ctx bounds the number of chunks (grid.z); workgroups past a row's context
+// exit early.  part_o / part_ml: workspace of R*Hq*n_chunks*(128 | 2) floats,
 // unused when max_ctx <= 256.
 P2P_API int p2p_paged_attention(const void* q, int ldq, const void* k_cache, const void* v_cache,
                                 const int* block_tables, int bt_stride, const int* row_bt,
@@ -442,10 +496,10 @@ P2P_API int p2p_paged_attention(const void* q, int ldq, const void* k_cache, con
   if (n_chunks > 1 && (!part_o || !part_ml)) return (int)hipErrorInvalidValue;
   if (n_chunks > MAX_CHUNKS) return (int)hipErrorInvalidValue;
   switch (Hq / Hkv) {
-    case 1: return launch_attn<1>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, n_chunks, out, ldo, part_o, part_ml, stream);
-    case 2: return launch_attn<2>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, n_chunks, out, ldo, part_o, part_ml, stream);
-    case 4: return launch_attn<4>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, n_chunks, out, ldo, part_o, part_ml, stream);
-    case 8: return launch_attn<8>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, n_chunks, out, ldo, part_o, part_ml, stream);
+    case 1: return launch_attn<1>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, stream);
+    case 2: return launch_attn<2>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, stream);
+    case 4: return launch_attn<4>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, stream);
+    case 8: return launch_attn<8>(q, ldq, k_cache, v_cache, block_tables, bt_stride, row_bt, ctx_lens, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, stream);
   }
   return (int)hipErrorInvalidValue;
 }

@@ -325,8 +325,8 @@ def _make_cache(P, Hkv, seed=0):
 @pytest.mark.parametrize("ctxs", [[1], [63, 64, 65], [256, 200, 129, 17], [300, 7], [1000, 257, 1]])
 @pytest.mark.parametrize("mfma", [False, True])
 def test_paged_attention(G, ctxs, mfma):
-    """Contexts <= 256: the 16-wave kernel or (mfma) the 4-wave MFMA kernel; longer
-    contexts the split-K kernel + combine."""
+    """Contexts <= 256: one chunk, with (mfma) bf16 probabilities; longer contexts several chunks and
+    their combine."""
     from p2p_llm_chat_go_amd.ops import _lib
 
     _lib.lib().p2p_paged_attention_mfma(int(mfma))
@@ -355,6 +355,36 @@ def _paged_attention_case(G, ctxs):
                               ctx.to(DEV), Hq, Hkv, max_ctx)
     torch.cuda.synchronize()
     assert _rel(out.cpu(), ref) < 1e-2
+
+
+@pytest.mark.parametrize("R,Hkv,G,max_ctx", [(64, 8, 2, 1024), (43, 8, 1, 1100), (8, 8, 4, 9000), (2, 1, 8, 2305),
+                                             (3, 3, 4, 2048), (17, 8, 4, 256)])
+def test_paged_attention_chunks(R, Hkv, G, max_ctx):
+    """Both chunk lengths (512 workgroups and more of 1024 keys: the long one), one chunk, up to 8 and more of them;
+    contexts that end in every part of a page; whatever lies past a context (the rest of its last page, the null
+    page) is NaN; q in rows of 4-byte alignment.  The result is rounded once to bf16 (relative 2^-9 at most) and
+    everything before it is fp32."""
+    g = torch.Generator().manual_seed(R + max_ctx)
+    k, v = _make_cache(1 + 40 + R, Hkv, seed=G)
+    ctx = torch.randint(1, max_ctx + 1, (R,), generator=g).int()
+    ctx[0], ctx[-1] = max_ctx, 1
+    npg = (max_ctx + 63) // 64
+    bt = torch.zeros(R, npg, dtype=torch.int32)
+    k[0], v[0] = float("nan"), float("nan")
+    for r in range(R):  # shared pages, the last one the row's own
+        n = (int(ctx[r]) + 63) // 64
+        bt[r, :n] = torch.randint(1, 41, (n,), generator=g).int()
+        bt[r, n - 1] = 41 + r
+        k[41 + r, :, (int(ctx[r]) - 1) % 64 + 1:] = float("nan")
+        v[41 + r, :, (int(ctx[r]) - 1) % 64 + 1:] = float("nan")
+    Hq = Hkv * G
+    q = torch.randn(R, Hq * 128 + 2, generator=g).to(torch.bfloat16)
+    ref = A.paged_attention_ref(q[:, 2:].contiguous(), k, v, bt, None, ctx, Hq, Hkv, 1 / math.sqrt(128),
+                                torch.empty(R, Hq * 128))
+    out = ops.paged_attention(q.to(DEV)[:, 2:], k.to(DEV), v.to(DEV), bt.to(DEV), None, ctx.to(DEV), Hq, Hkv, max_ctx)
+    assert float((out.float().cpu() - ref).norm() / ref.norm()) < 2 ** -9
+    far = (out.float().cpu() - ref).abs() - ref.abs() * 2 ** -8
+    assert float(far.max()) < 1e-5
 
 
 def test_paged_attention_spike_forces_rescale():
