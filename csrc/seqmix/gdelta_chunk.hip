@@ -19,9 +19,13 @@
 // A weight of zero stands for "not before this token" in these products, and 0 * inf is nan: a chunk and head whose
 // inputs are not all finite is walked token by token instead, so that tokens before such an input are what they were.
 //
-// A chunk and head are about 700 matrix instructions per wavefront.  The walk of gdelta_scan_k (once for L and T, once
+// A chunk and head are about 600 matrix instructions per wavefront.  The walk of gdelta_scan_k (once for L and T, once
 // for the outputs) took 2 x 205 us for 2048 tokens and 32 heads of 64, and the chain 654 us of 32 dependent products on
-// 32 workgroups with scalar sums; the three kernels here take 164, 36 and 20 us.
+// 32 workgroups with scalar sums; the three kernels here take 84, 31 and 21 us.  The first is bound by its workgroups' chains of
+// loads, products and barriers (the products alone: 40 us).  It took 168 with six tables in LDS (104 KB: one
+// workgroup per CU), 108 with four (two of them take the places of U and R in turn: 77 KB, two workgroups), 104 with a
+// table of weights per wavefront instead of 16 rows of all four, 84 with no load behind a branch and one
+// division in 64 bits instead of sixteen.
 #include "common.h"
 using namespace sm;
 
@@ -47,27 +51,15 @@ struct GdeltaArgs {
   float eps;
 };
 
-// T, L, Q and O of a chunk and head by its tokens in order: a thread takes 16 rows of a column of T and of L
+// T, L, Q and O of a chunk and head by its tokens in order, WT of them staged at a time: a thread takes 16 rows of a
+// column of T and of L
 template <typename T>
 __device__ __forceinline__ void walk_chunk(const GdeltaArgs& p, const Entry& en, int c, int h, float* smem) {
-  float *sr = smem, *sk = sr + GC * GLD, *su = sk + GC * GLD, *sa = su + GC * GLD, *sw = sa + GC * GLD, *sv = sw + GC * GLD;
+  constexpr int WT = 32;   // six rows per token: what the four tables' LDS holds
+  float *sr = smem, *sk = sr + WT * GLD, *su = sk + WT * GLD, *sa = su + WT * GLD, *sw = sa + WT * GLD, *sv = sw + WT * GLD;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, D = p.D;
   const int vc = wave * 16 + (lane & 15), i0 = (lane >> 4) * 16;
   const int col = h * D + min(lane, D - 1);
-  for (int t = wave; t < en.n; t += 4) {   // a wavefront's own places below: no wait needed in between
-    const size_t row = (size_t)(en.row0 + t);
-    const int at = t * GLD + lane;
-    const bool in = lane < D;
-    const float k = in ? ldf((const T*)p.k, row * p.ld + col) : 0.0f;
-    const float u = k * (1.0f / sqrtf(wave_sum(k * k) + 1e-6f));
-    sr[at] = in ? ldf((const T*)p.r, row * p.ld + col) : 0.0f;
-    sk[at] = k;
-    su[at] = u;
-    sa[at] = in ? sigmoidf_(ldf((const T*)p.a, row * p.ld + col) + p.ab[col]) * u : 0.0f;
-    sw[at] = in ? expf(-GD_DECAY_SCALE * sigmoidf_(ldf((const T*)p.lo, row * p.ldlo + col) + p.w0[col])) : 1.0f;
-    sv[at] = in ? ldf((const T*)p.v, row * p.ld + col) : 0.0f;
-  }
-  __syncthreads();
   float S[16], M[16];
 #pragma unroll
   for (int q = 0; q < 16; q++) S[q] = 0.0f, M[q] = i0 + q == vc ? 1.0f : 0.0f;
@@ -76,30 +68,48 @@ __device__ __forceinline__ void walk_chunk(const GdeltaArgs& p, const Entry& en,
     return x + __shfl_xor(x, 32, 64);
   };
   const size_t base = ((size_t)c * p.H + h) * GC * GC;
-  for (int t = 0; t < en.n; t++) {
-    const int at = t * GLD + i0;
-    float ds = 0.0f, dm = 0.0f, os = 0.0f, om = 0.0f;
+  for (int b0 = 0; b0 < en.n; b0 += WT) {
+    const int nb = min(WT, en.n - b0);
+    for (int t = wave; t < nb; t += 4) {
+      const size_t row = (size_t)(en.row0 + b0 + t);
+      const int at = t * GLD + lane;
+      const bool in = lane < D;
+      const float k = in ? ldf((const T*)p.k, row * p.ld + col) : 0.0f;
+      const float u = k * (1.0f / sqrtf(wave_sum(k * k) + 1e-6f));
+      sr[at] = in ? ldf((const T*)p.r, row * p.ld + col) : 0.0f;
+      sk[at] = k;
+      su[at] = u;
+      sa[at] = in ? sigmoidf_(ldf((const T*)p.a, row * p.ld + col) + p.ab[col]) * u : 0.0f;
+      sw[at] = in ? expf(-GD_DECAY_SCALE * sigmoidf_(ldf((const T*)p.lo, row * p.ldlo + col) + p.w0[col])) : 1.0f;
+      sv[at] = in ? ldf((const T*)p.v, row * p.ld + col) : 0.0f;
+    }
+    __syncthreads();
+    for (int t = 0; t < nb; t++) {
+      const int at = t * GLD + i0;
+      float ds = 0.0f, dm = 0.0f, os = 0.0f, om = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      ds += su[at + q] * S[q];
-      dm += su[at + q] * M[q];
-    }
-    ds = over_rows(ds);
-    dm = over_rows(dm);
-    const float v = sv[t * GLD + vc];
+      for (int q = 0; q < 16; q++) {
+        ds += su[at + q] * S[q];
+        dm += su[at + q] * M[q];
+      }
+      ds = over_rows(ds);
+      dm = over_rows(dm);
+      const float v = sv[t * GLD + vc];
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      S[q] = sw[at + q] * S[q] - sa[at + q] * ds + sk[at + q] * v;
-      M[q] = sw[at + q] * M[q] - sa[at + q] * dm;
-      os += S[q] * sr[at + q];
-      om += M[q] * sr[at + q];
+      for (int q = 0; q < 16; q++) {
+        S[q] = sw[at + q] * S[q] - sa[at + q] * ds + sk[at + q] * v;
+        M[q] = sw[at + q] * M[q] - sa[at + q] * dm;
+        os += S[q] * sr[at + q];
+        om += M[q] * sr[at + q];
+      }
+      os = over_rows(os);
+      om = over_rows(om);
+      if (i0 == 0) {
+        p.oo[base + (b0 + t) * GC + vc] = os;
+        p.qq[base + (b0 + t) * GC + vc] = om;
+      }
     }
-    os = over_rows(os);
-    om = over_rows(om);
-    if (i0 == 0) {
-      p.oo[base + t * GC + vc] = os;
-      p.qq[base + t * GC + vc] = om;
-    }
+    __syncthreads();   // the tokens have been used
   }
 #pragma unroll
   for (int q = 0; q < 16; q++) {
@@ -109,14 +119,12 @@ __device__ __forceinline__ void walk_chunk(const GdeltaArgs& p, const Entry& en,
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
+__global__ void __launch_bounds__(256, 2) gdelta_chunk_k(GdeltaArgs p) {
   extern __shared__ __align__(16) float smem[];
-  float* sU = smem;                  // u e_(t-1), later the weights of v_s in p_t
-  float* sR = sU + GC * GLD;         // r e_t,     later the weights of p_s in o_t
+  float* sU = smem;                  // u e_(t-1), then the weights of v_s in p_t, then those of v_s in o_t
+  float* sR = sU + GC * GLD;         // r e_t,     then the weights of p_s in p_t, then those of p_s in o_t
   float* sK = sR + GC * GLD;         // k / e_s
   float* sA = sK + GC * GLD;         // a u / e_s
-  float* sL = sA + GC * GLD;         // weights of p_s in p_t
-  float* sB = sL + GC * GLD;         // weights of v_s in o_t
   __shared__ double sTot[4][GC];
   __shared__ float sMid[GC], sEnd[GC];
   __shared__ __align__(16) float sD[4][16][20];   // inverses of the blocks on the diagonal
@@ -124,28 +132,44 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
   const Entry en = load_entry(p.vent, c);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, quad = lane >> 4;
   float odd = 0.0f;   // becomes nan with an input that is not finite
+  // values as operands: token 16 b + quad * 4 + e, this wavefront's 16 columns
+  const int vc = wave * 16 + n16;
+  f32x4 V[4];
   // a lane's channel of the wavefront's 16 tokens
   {
     const int col = h * D + min(lane, D - 1);
     const bool in = lane < D;
     const float w0 = p.w0[col], ab = p.ab[col];
+    // every load first and none behind a branch (which would wait for those before it)
     float kv[16], rv[16], av[16], w[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const size_t row = (size_t)(en.row0 + min(wave * 16 + q, en.n - 1));
+      kv[q] = ldf((const T*)p.k, row * p.ld + col);
+      rv[q] = ldf((const T*)p.r, row * p.ld + col);
+      av[q] = ldf((const T*)p.a, row * p.ld + col);
+      w[q] = ldf((const T*)p.lo, row * p.ldlo + col);
+    }
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        V[b][e] = ldf((const T*)p.v, (size_t)(en.row0 + min(b * 16 + quad * 4 + e, en.n - 1)) * p.ld + h * D + min(vc, D - 1));
     double all = 1.0;
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int t = wave * 16 + q;
-      const size_t row = (size_t)(en.row0 + min(t, en.n - 1));
-      const bool have = in && t < en.n;
-      kv[q] = have ? ldf((const T*)p.k, row * p.ld + col) : 0.0f;
-      rv[q] = have ? ldf((const T*)p.r, row * p.ld + col) : 0.0f;
-      av[q] = sigmoidf_(ldf((const T*)p.a, row * p.ld + col) + ab);
-      w[q] = have ? expf(-GD_DECAY_SCALE * sigmoidf_(ldf((const T*)p.lo, row * p.ldlo + col) + w0)) : 1.0f;
+      const bool have = in && wave * 16 + q < en.n;
+      kv[q] = have ? kv[q] : 0.0f;
+      rv[q] = have ? rv[q] : 0.0f;
+      av[q] = sigmoidf_(av[q] + ab);
+      w[q] = have ? expf(-GD_DECAY_SCALE * sigmoidf_(w[q] + w0)) : 1.0f;
       all *= w[q];
     }
     sTot[wave][lane] = all;
     __syncthreads();
     const double t0 = sTot[0][lane], t1 = sTot[1][lane], t2 = sTot[2][lane], t3 = sTot[3][lane];
     double up = wave == 0 ? 1.0 / (t0 * t1) : wave == 1 ? 1.0 / t1 : wave == 2 ? 1.0 : t2;   // before this token
+    double down = 1.0 / (up * all);                                                          // after the last one
     if (wave == 0) {
       sMid[lane] = (float)(t0 * t1);
       sEnd[lane] = (float)(t2 * t3);   // to the chunk's end, from the middle
@@ -156,56 +180,55 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
       const float u = kv[q] * (1.0f / sqrtf(wave_sum(kv[q] * kv[q]) + 1e-6f));
       sU[at] = (float)(u * up);
       up *= w[q];
-      const double down = 1.0 / up;
-      const float kd = (float)(kv[q] * down), ad = (float)((double)(av[q] * u) * down);
       sR[at] = (float)(rv[q] * up);
+      av[q] *= u;
+    }
+#pragma unroll
+    for (int q = 15; q >= 0; q--) {   // one division for the sixteen
+      const int at = (wave * 16 + q) * GLD + lane;
+      const float kd = (float)(kv[q] * down), ad = (float)((double)av[q] * down);
+      down *= w[q];
       sK[at] = kd;
       sA[at] = ad;
       odd += 0.0f * kd + 0.0f * ad;
     }
   }
-  // values as operands: token 16 b + quad * 4 + e, this wavefront's 16 columns
-  const int vc = wave * 16 + n16;
-  f32x4 V[4];
 #pragma unroll
   for (int b = 0; b < 4; b++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int t = b * 16 + quad * 4 + e;
-      V[b][e] = (t < en.n && vc < D) ? ldf((const T*)p.v, (size_t)(en.row0 + t) * p.ld + h * D + vc) : 0.0f;
+      V[b][e] = b * 16 + quad * 4 + e < en.n && vc < D ? V[b][e] : 0.0f;
       odd += 0.0f * V[b][e];
     }
   if (__syncthreads_or(odd != 0.0f)) {
     walk_chunk<T>(p, en, c, h, smem);
     return;
   }
-  // the four tables of weights: this wavefront's 16 rows t, s <= t
-  f32x4 akk[4], auu[4], bk[4], bu[4];
+  // the four tables of weights, one per wavefront, its blocks of rows t and s <= t (by rows, the last wavefront had four
+  // times the first one's products): U.K, U.A, R.K, R.A
+  f32x4 tab[10];   // block (b, j) at b (b + 1) / 2 + j
 #pragma unroll
-  for (int j = 0; j < 4; j++) akk[j] = auu[j] = bk[j] = bu[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 10; i++) tab[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  {
+    const float *sx = wave & 2 ? sR : sU, *sy = wave & 1 ? sA : sK;
 #pragma unroll
-  for (int kk = 0; kk < 4; kk++) {
-    const int at = kk * 16 + quad * 4;
-    const f32x4 u = *(const f32x4*)(sU + (wave * 16 + n16) * GLD + at);
-    const f32x4 r = *(const f32x4*)(sR + (wave * 16 + n16) * GLD + at);
+    for (int kk = 0; kk < 4; kk++) {
+      f32x4 x[4], y[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-      if (j <= wave) {
-        const f32x4 kd = *(const f32x4*)(sK + (j * 16 + n16) * GLD + at);
-        const f32x4 ad = *(const f32x4*)(sA + (j * 16 + n16) * GLD + at);
-        f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, p2 = p0, p3 = p0;   // sums of 16
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          p0 = MFMA4(u[e], kd[e], p0);
-          p1 = MFMA4(u[e], ad[e], p1);
-          p2 = MFMA4(r[e], kd[e], p2);
-          p3 = MFMA4(r[e], ad[e], p3);
-        }
-        akk[j] += p0;
-        auu[j] += p1;
-        bk[j] += p2;
-        bu[j] += p3;
+      for (int j = 0; j < 4; j++) {
+        x[j] = *(const f32x4*)(sx + (j * 16 + n16) * GLD + kk * 16 + quad * 4);
+        y[j] = *(const f32x4*)(sy + (j * 16 + n16) * GLD + kk * 16 + quad * 4);
       }
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int j = 0; j <= b; j++) {
+          f32x4 p0 = {0.f, 0.f, 0.f, 0.f};   // sums of 16
+#pragma unroll
+          for (int e = 0; e < 4; e++) p0 = MFMA4(x[b][e], y[j][e], p0);
+          tab[b * (b + 1) / 2 + j] += p0;
+        }
+    }
   }
   // G starts as U, Q as R: this wavefront's 16 columns
   f32x4 G[4], Q[4];
@@ -217,19 +240,22 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
       G[b][e] = sU[at];
       Q[b][e] = sR[at];
     }
+  // two tables in LDS at a time, the other two in registers until these have been used
+  auto put = [&](int half) {
+    if (wave >> 1 != half) return;
+    float* dst = wave & 1 ? sR : sU;
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int j = 0; j <= b; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int t = b * 16 + quad * 4 + e, s = j * 16 + n16;
+          dst[t * GLD + s] = s < t + half ? tab[b * (b + 1) / 2 + j][e] : 0.0f;
+        }
+  };
   __syncthreads();   // U and R have been read
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-    if (j <= wave) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int t = wave * 16 + quad * 4 + e, s = j * 16 + n16, at = t * GLD + s;
-        sU[at] = s < t ? akk[j][e] : 0.0f;
-        sL[at] = s < t ? auu[j][e] : 0.0f;
-        sB[at] = s <= t ? bk[j][e] : 0.0f;
-        sR[at] = s <= t ? bu[j][e] : 0.0f;
-      }
-    }
+  put(0);   // U.K and U.A
   __syncthreads();
   // the inverse of this wavefront's block on the diagonal, a column per lane
   {
@@ -238,7 +264,7 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
     for (int i = 0; i < 16; i++) {
       float v = i == n16 ? 1.0f : 0.0f;
 #pragma unroll
-      for (int q = 0; q < i; q++) v = fmaf(-sL[(wave * 16 + i) * GLD + wave * 16 + q], x[q], v);
+      for (int q = 0; q < i; q++) v = fmaf(-sR[(wave * 16 + i) * GLD + wave * 16 + q], x[q], v);
       x[i] = v;
     }
     if (quad == 0) {
@@ -263,7 +289,7 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
   for (int b = 0; b < 4; b++) {
 #pragma unroll
     for (int j = 0; j < b; j++) {
-      const f32x4 f = *(const f32x4*)(sL + (b * 16 + n16) * GLD + j * 16 + quad * 4);
+      const f32x4 f = *(const f32x4*)(sR + (b * 16 + n16) * GLD + j * 16 + quad * 4);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         G[b] = MFMA4(-f[e], G[j][e], G[b]);
@@ -282,6 +308,9 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
   }
   const size_t base = ((size_t)c * p.H + h) * GC * GC;
   const float emid = sMid[vc];
+  __syncthreads();   // the system has been solved
+  put(1);   // R.K and R.A
+  __syncthreads();
   // outputs: Q and O
 #pragma unroll
   for (int b = 0; b < 4; b++) {
@@ -289,7 +318,7 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
 #pragma unroll
     for (int j = 0; j <= b; j++) {
       const f32x4 fu = *(const f32x4*)(sR + (b * 16 + n16) * GLD + j * 16 + quad * 4);
-      const f32x4 fk = *(const f32x4*)(sB + (b * 16 + n16) * GLD + j * 16 + quad * 4);
+      const f32x4 fk = *(const f32x4*)(sU + (b * 16 + n16) * GLD + j * 16 + quad * 4);
       f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, p2 = p0;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
@@ -336,7 +365,8 @@ __global__ void __launch_bounds__(256) gdelta_chunk_k(GdeltaArgs p) {
 }
 
 // S <- T S + L over each portion's chunks, 16 columns of a head per workgroup, a wavefront per 16 rows; the state before
-// a chunk replaces its L.  What a chunk needs from memory does not depend on the state: it is read a chunk ahead.
+// a chunk replaces its L.  What a chunk needs from memory does not depend on the state: it is read three chunks
+// ahead (one: 36 us for 32 chunks and heads, every chunk a wait for memory; three: 31).
 __global__ void __launch_bounds__(256) gdelta_chain_k(GdeltaArgs p) {
   __shared__ float sS[2][GC][17];
   const int c0 = p.cent[4 * blockIdx.z], nc = p.cent[4 * blockIdx.z + 1], start = p.cent[4 * blockIdx.z + 2],
@@ -352,35 +382,38 @@ __global__ void __launch_bounds__(256) gdelta_chain_k(GdeltaArgs p) {
   const size_t step = (size_t)p.H * GC * GC;
   const float* tp = p.trn + (size_t)c0 * step + (size_t)h * GC * GC + (wave * 16 + n16) * GC + quad * 4;
   float* lp = p.loc + (size_t)c0 * step + (size_t)h * GC * GC + row * GC + col;
-  f32x4 T[4], L;
+  f32x4 T[3][4], L[3];
   auto load = [&](int c, f32x4 (&t)[4], f32x4& l) {
+    c = min(c, nc - 1);   // (beyond the end: not used)
 #pragma unroll
     for (int b = 0; b < 4; b++) t[b] = *(const f32x4*)(tp + c * step + b * 16);
 #pragma unroll
     for (int e = 0; e < 4; e++) l[e] = lp[c * step + e * GC];
   };
-  load(0, T, L);
-  for (int c = 0; c < nc; c++) {
-    f32x4 Tn[4], Ln;
-    if (c + 1 < nc) load(c + 1, Tn, Ln);
-    float(*S)[17] = sS[c & 1];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      S[row + e][n16] = cur[e];
-      lp[c * step + e * GC] = cur[e];
+  for (int u = 0; u < 3; u++) load(u, T[u], L[u]);
+  for (int k = 0; k < nc; k += 3) {
+#pragma unroll
+    for (int u = 0; u < 3; u++) {
+      const int c = k + u;
+      if (c >= nc) break;
+      float(*S)[17] = sS[c & 1];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        S[row + e][n16] = cur[e];
+        lp[c * step + e * GC] = cur[e];
+      }
+      __syncthreads();
+      f32x4 a[4];
+      a[0] = L[u];
+      a[1] = a[2] = a[3] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) a[b] = MFMA4(T[u][b][e], S[b * 16 + quad * 4 + e][n16], a[b]);
+      cur = (a[0] + a[1]) + (a[2] + a[3]);
+      load(c + 3, T[u], L[u]);
     }
-    __syncthreads();
-    f32x4 a[4];
-    a[0] = L;
-    a[1] = a[2] = a[3] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) a[b] = MFMA4(T[b][e], S[b * 16 + quad * 4 + e][n16], a[b]);
-    cur = (a[0] + a[1]) + (a[2] + a[3]);
-#pragma unroll
-    for (int b = 0; b < 4; b++) T[b] = Tn[b];
-    L = Ln;
   }
 #pragma unroll
   for (int e = 0; e < 4; e++)
@@ -458,7 +491,7 @@ int p2p_sm_gdelta_chunk(const void* r, const void* k, const void* v, const void*
   const size_t sz = (size_t)NV * H * GC * GC;
   const GdeltaArgs p = {r, k, v, g, a, ld, lo, ldlo, w0, ab, normw, state, tmp, tmp + sz, tmp + 2 * sz, tmp + 3 * sz,
                         vent, cent, out, ldo, H, D, eps};
-  constexpr int shm = 6 * GC * GLD * 4;
+  constexpr int shm = 4 * GC * GLD * 4;
   static const hipError_t attr = [] {
     const hipError_t e = hipFuncSetAttribute((const void*)gdelta_chunk_k<float>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, shm);
