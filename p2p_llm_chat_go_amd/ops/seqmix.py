@@ -69,7 +69,7 @@ _SIGS = {
                                                     c_void_p, c_int, c_void_p, c_int, c_int, c_int,
                                                     c_float, c_int, c_void_p],
     "p2p_sm_mamba_scan_chunked": [c_void_p, c_int, c_void_p, c_int, c_int, c_void_p,
-                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int,
                                   c_int, c_void_p],
     "p2p_sm_mamba_conv": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -1122,10 +1122,12 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
         NV = vent.shape[0]
         tmp = torch.empty(NV, H, N, P, device=zx.device, dtype=torch.float32)
         decay = torch.empty(NV, H, device=zx.device, dtype=torch.float32)
+        # heads that share B and C share their products (a group's 64 x 64 per chunk)
+        cb = torch.empty(NV, G, 64, 64, device=zx.device, dtype=torch.float32) if H > G else None
         _chk(lib().p2p_sm_mamba_scan_chunked(
             conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), dtoff, dt_bias.data_ptr(),
             A_log.data_ptr(), Dp.data_ptr(), state.data_ptr(), tmp.data_ptr(), decay.data_ptr(),
-            vent.data_ptr(), NV, cent.data_ptr(), cent.shape[0], y.data_ptr(), H, P, N, G, _f32(zx),
+            _lib.ptr(cb), vent.data_ptr(), NV, cent.data_ptr(), cent.shape[0], y.data_ptr(), H, P, N, G, _f32(zx),
             _st(zx)), "mamba_scan_chunked")
     if walk is not None:
         _chk(lib().p2p_sm_mamba_scan(conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), xoff, dtoff,

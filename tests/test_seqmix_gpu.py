@@ -269,6 +269,31 @@ def test_mamba_long_portions(lens, starts, H, P, N, G, steep):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,P,N,G", [(8, 64, 128, 2), (6, 32, 16, 3), (4, 100, 44, 1), (2, 64, 30, 1), (2, 200, 8, 1)])
+def test_mamba_groups_share_their_products(dt, H, P, N, G):
+    """Heads of a group take the products of B and C from one workgroup, and z and y four numbers at a time where rows
+    allow it: to the bit what every head forms by itself (a group each, with the same B and C) and what odd rows give."""
+    g = torch.Generator().manual_seed(H + P + N)
+    inner, lens = H * P, [150, 64, 33]
+    ent_h, ent, _row_ent, R = _ents(lens, [0, 5, 0], [2, 1, 0])
+    x, bc = torch.randn(R, inner, generator=g), torch.randn(2, R, G, N, generator=g)
+    zx = torch.randn(R, 2 * inner + 2 * H * N + H, generator=g).to(dt).to(DEV)
+    dtb, Al, Dp = (torch.randn(H, generator=g).to(DEV) for _ in range(3))
+    S0 = torch.randn(4, H, N, P, generator=g)
+    res = []
+    for groups, pad in ((G, 0), (H, 0), (G, 1)):
+        B, C = (b.repeat_interleave(groups // G, 1).reshape(R, groups * N) for b in bc)
+        conv = torch.cat([x, B, C], 1).to(DEV)
+        z = torch.nn.functional.pad(zx, (0, pad))
+        S, T = S0.to(DEV), torch.zeros(4, 3, conv.shape[1], device=DEV)
+        y = sm.mamba_scan(conv, z, inner, zx.shape[1] - H, dtb, Al, Dp, S, T, ent.to(DEV), ent_h,
+                          torch.empty(R, inner, device=DEV), H, P, N, groups)
+        res.append((y, S))
+    for y, S in res[1:]:
+        assert torch.equal(y, res[0][0]) and torch.equal(S, res[0][1])
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("lens,starts", [([130, 64, 1], [0, 7, 3]), ([65], [0]), ([33, 200], [5, 0])])
 @pytest.mark.parametrize("H,D", [(4, 64), (2, 33), (1, 5)])
 @pytest.mark.parametrize("decay", [-20.0, 0.0, 20.0])
