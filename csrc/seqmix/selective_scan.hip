@@ -34,12 +34,15 @@ struct SelArgs {
 #define SEL_U 4   // tokens whose inputs are loaded together
 
 // mode 0: portions from their slots' states, states written back; 1: a chunk from zero, end state to
-// `state[slot]`, sum of dt to dtsum; 2: a chunk from state[slot], outputs only
-template <typename T, int NS>
-__global__ void __launch_bounds__(1024)
-selective_scan_k(SelArgs a, int SN, int CW) {
+// `state[slot]`, sum of dt to dtsum; 2: a chunk from state[slot], outputs only.  ONE: a wavefront has all states (SN = 1)
+// What bounds it: the vector unit, 16 exponentials and 48 products per channel and token at 16 states.  2644 rows of 4096
+// channels in chunks of 64: 45 us (mode 1) and 56 (mode 2).  With the mode and SN known only at run time, z behind
+// a branch, and a stretch's inputs loaded when it began, each stretch waited for memory: 61 us each.
+template <typename T, int NS, int mode, bool ONE>
+__global__ void __launch_bounds__(ONE ? 256 : 1024)
+selective_scan_k(SelArgs a, int sn_all, int CW) {
   extern __shared__ __align__(16) float smem[];
-  const int I = a.I, N = a.N, CT = a.CT, mode = a.mode;
+  const int I = a.I, N = a.N, CT = a.CT, SN = ONE ? 1 : sn_all;
   const Entry en = load_entry(a.ent, blockIdx.y);
   if (en.n <= 0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -66,6 +69,17 @@ selective_scan_k(SelArgs a, int SN, int CW) {
   for (int q = 0; q < NS; q++) if (n0 + q >= N) S[q] = 0.0f;
   const float bias = a.dtb[cc], Dc = a.Dp[cc];
   float dts = 0.0f;
+  float xn[SEL_U], dn[SEL_U], zn[SEL_U];   // the next stretch's inputs
+  auto load = [&](int t) {
+#pragma unroll
+    for (int u = 0; u < SEL_U; u++) {
+      const size_t row = (size_t)(en.row0 + min(t + u, en.n - 1));
+      xn[u] = ldf(x, row * a.ldx + cc);
+      dn[u] = ldf(dt, row * a.lddt + cc);
+      zn[u] = mode != 1 && ONE ? ldf(z, row * a.ldz + cc) : 0.0f;
+    }
+  };
+  if (ONE) load(0);   // (sixteen wavefronts of 32 states have no registers to spare)
   for (int t0 = 0; t0 < en.n; t0 += CT) {
     const int ct = min(CT, en.n - t0);
     __syncthreads();
@@ -78,13 +92,10 @@ selective_scan_k(SelArgs a, int SN, int CW) {
     __syncthreads();
     for (int t1 = 0; t1 < ct; t1 += SEL_U) {
       float xv[SEL_U], dv[SEL_U], zv[SEL_U];
+      if (!ONE) load(t0 + t1);
 #pragma unroll
-      for (int u = 0; u < SEL_U; u++) {
-        const size_t row = (size_t)(en.row0 + t0 + min(t1 + u, ct - 1));
-        xv[u] = ldf(x, row * a.ldx + cc);
-        dv[u] = ldf(dt, row * a.lddt + cc);
-        zv[u] = mode != 1 && sn == 0 ? ldf(z, row * a.ldz + cc) : 0.0f;
-      }
+      for (int u = 0; u < SEL_U; u++) xv[u] = xn[u], dv[u] = dn[u], zv[u] = zn[u];
+      if (ONE) load(t0 + t1 + SEL_U);
 #pragma unroll
       for (int u = 0; u < SEL_U; u++) {
         const int t = t1 + u;
@@ -111,13 +122,13 @@ selective_scan_k(SelArgs a, int SN, int CW) {
         }
         if (mode != 1) {
           acc += acc1;
-          if (sn == 0) acc = (acc + Dc * xv[u]) * (SN == 1 ? silu_(zv[u]) : 1.0f);
-          if (SN > 1) sy[(t * SN + sn) * CW * 64 + cw * 64 + lane] = acc;
+          if (sn == 0) acc = (acc + Dc * xv[u]) * (ONE ? silu_(zv[u]) : 1.0f);
+          if (!ONE) sy[(t * SN + sn) * CW * 64 + cw * 64 + lane] = acc;
           else if (act) stf(y, (size_t)(en.row0 + t0 + t) * a.ldy + c, acc);
         }
       }
     }
-    if (SN > 1 && mode != 1) {
+    if (!ONE && mode != 1) {
       __syncthreads();
       const int W = CW * 64;
       for (int idx = threadIdx.x; idx < ct * W; idx += blockDim.x) {
@@ -243,19 +254,23 @@ static int launch_sel(SelArgs a, int E, int f32, hipStream_t st) {
   if (N < 1 || SN > 16 || a.I < 1) return (int)hipErrorInvalidValue;
   const int CW = SN >= 4 ? 1 : 4 / SN;
   const int NP = SN * ns;
-  int CT = 32;
+  int CT = 64;   // (a chunk's tokens in one go)
   auto lds = [&](int ct) { return (size_t)ct * (2 * NP + (SN > 1 ? SN * CW * 64 : 0)) * 4; };
   while (CT > SEL_U && lds(CT) > 32 * 1024) CT /= 2;
   if (lds(CT) > 64 * 1024) return (int)hipErrorInvalidValue;
   a.CT = CT;
   dim3 grid((a.I + CW * 64 - 1) / (CW * 64), E), block(64 * SN * CW);
-#define SEL(NS) \
-  SM_DISPATCH_T(f32, hipLaunchKernelGGL((selective_scan_k<T, NS>), grid, block, lds(CT), st, a, SN, CW))
-  if (ns == 4) SEL(4);
-  else if (ns == 8) SEL(8);
-  else if (ns == 16) SEL(16);
-  else if (ns == 24) SEL(24);
-  else SEL(32);
+#define SEL(NS, ONE)                                                                               \
+  SM_DISPATCH_T(f32, hipLaunchKernelGGL((a.mode == 0   ? selective_scan_k<T, NS, 0, ONE>           \
+                                         : a.mode == 1 ? selective_scan_k<T, NS, 1, ONE>           \
+                                                       : selective_scan_k<T, NS, 2, ONE>),         \
+                                        grid, block, lds(CT), st, a, SN, CW))
+  if (ns == 4) SEL(4, true);
+  else if (ns == 8) SEL(8, true);
+  else if (ns == 16) SEL(16, true);
+  else if (ns == 24) SEL(24, true);
+  else if (SN == 1) SEL(32, true);
+  else SEL(32, false);
 #undef SEL
   return (int)hipGetLastError();
 }
