@@ -10,6 +10,9 @@
 // `pw` [H, 65] holds the powers lam^0 .. lam^64 of every head, so no power is formed here.
 // One workgroup of four wavefronts per (chunk, head).  Sizes are padded to multiples of 16 with
 // zeros in LDS; rows are laid out so that the lanes of a fragment read hit different banks.
+// What bounds it: a workgroup's chain of loads and products (the output pass's products alone take 20 us), two
+// workgroups per CU.  2644 rows, 16 heads of 128 x 128: 36, 19 and 69 us; with one load in flight per thread while staging and the
+// state's rows loaded as they are used 41, 19 and 83.
 #include "common.h"
 using namespace sm;
 
@@ -26,29 +29,57 @@ __device__ __forceinline__ float lsilu(float x) {
 static __host__ __device__ __forceinline__ int ld_rows(int n) { return n + ((4 - n) & 63); }
 static __host__ __device__ __forceinline__ int ld_cols(int n) { return n + ((16 - n) & 63); }
 
+// Rows on their way to LDS, four numbers per load and eight loads of a thread in flight (none behind a branch, which would
+// wait for those before it): numbers 4 * (base + 256 i + thread) of the rows padded to 4 * w4
+template <typename T>
+struct Batch {
+  static constexpr int U = 8, N = 256 * U;
+  uint2 lo[U], hi[U];   // (bf16: lo alone)
+  __device__ __forceinline__ void load(const T* __restrict__ src, size_t ld, int n, int width, int w4, int base) {
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const int idx = base + i * 256 + threadIdx.x, t = idx / w4, c = (idx % w4) * 4;
+      const T* p = src + (size_t)min(t, n - 1) * ld + min(c, width - 4);
+      if constexpr (sizeof(T) == 2) {
+        lo[i] = *(const uint2*)p;
+      } else {
+        const uint4 u = *(const uint4*)p;
+        lo[i] = make_uint2(u.x, u.y);
+        hi[i] = make_uint2(u.z, u.w);
+      }
+    }
+  }
+  template <typename F>
+  __device__ __forceinline__ void store(float* dst, int ldd, int n, int width, int w4, int base, F scale) const {
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const int idx = base + i * 256 + threadIdx.x, t = idx / w4, c = (idx % w4) * 4;
+      if (idx >= LC * w4) break;
+      float4 v;
+      if constexpr (sizeof(T) == 2) {
+        v.x = __uint_as_float(lo[i].x << 16); v.y = __uint_as_float(lo[i].x & 0xffff0000u);
+        v.z = __uint_as_float(lo[i].y << 16); v.w = __uint_as_float(lo[i].y & 0xffff0000u);
+      } else {
+        v = make_float4(__uint_as_float(lo[i].x), __uint_as_float(lo[i].y), __uint_as_float(hi[i].x), __uint_as_float(hi[i].y));
+      }
+      const float m = scale(min(t, n - 1));
+      v.x = lsilu(v.x) * m; v.y = lsilu(v.y) * m; v.z = lsilu(v.z) * m; v.w = lsilu(v.w) * m;
+      *(float4*)(dst + t * ldd + c) = t < n && c < width ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+};
+
 // n rows of `width` numbers of src (row stride ld) -> dst [LC][ldd] through silu, times scale(t);
-// zeros up to `pad` columns and in rows n .. LC-1
+// zeros up to `pad` columns and in rows n .. LC-1.  The numbers below `base` are there already
 template <typename T, typename F>
 __device__ __forceinline__ void stage(const T* __restrict__ src, size_t ld, int n, int width, int pad,
-                                      float* dst, int ldd, bool vec, F scale) {
-  if (vec) {   // four numbers per load
-    const int w4 = pad / 4;
-    for (int idx = threadIdx.x; idx < LC * w4; idx += 256) {
-      const int t = idx / w4, c = (idx % w4) * 4;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (t < n && c < width) {
-        const T* p = src + (size_t)t * ld + c;
-        if constexpr (sizeof(T) == 2) {
-          const uint2 u = *(const uint2*)p;
-          v.x = __uint_as_float(u.x << 16); v.y = __uint_as_float(u.x & 0xffff0000u);
-          v.z = __uint_as_float(u.y << 16); v.w = __uint_as_float(u.y & 0xffff0000u);
-        } else {
-          v = *(const float4*)p;
-        }
-        const float m = scale(t);
-        v.x = lsilu(v.x) * m; v.y = lsilu(v.y) * m; v.z = lsilu(v.z) * m; v.w = lsilu(v.w) * m;
-      }
-      *(float4*)(dst + t * ldd + c) = v;
+                                      float* dst, int ldd, bool vec, F scale, int base = 0) {
+  if (vec) {
+#pragma unroll 1
+    for (; base < LC * (pad / 4); base += Batch<T>::N) {
+      Batch<T> b;
+      b.load(src, ld, n, width, pad / 4, base);
+      b.store(dst, ldd, n, width, pad / 4, base, scale);
     }
     return;
   }
@@ -72,8 +103,20 @@ lightning_local_k(const T* __restrict__ proj, int ldp, const float* __restrict__
   const T* row = proj + (size_t)en.row0 * ldp;
   const float* p = pw + (size_t)h * (LC + 1);
   const int n = en.n;
-  stage(row + (size_t)H * D + h * D, (size_t)ldp, n, D, DP, sK, LDK, vec, [&](int t) { return p[n - 1 - t]; });
-  stage(row + (size_t)2 * H * D + h * V, (size_t)ldp, n, V, VP, sV, LDV, vec, [](int) { return 1.0f; });
+  const T *K = row + (size_t)H * D + h * D, *Vp = row + (size_t)2 * H * D + h * V;
+  auto power = [&](int t) { return p[n - 1 - t]; };
+  auto one = [](int) { return 1.0f; };
+  int base = 0;
+  if (vec) {   // both in one wait for memory, as far as a batch goes
+    Batch<T> k, v;
+    k.load(K, (size_t)ldp, n, D, DP / 4, 0);
+    v.load(Vp, (size_t)ldp, n, V, VP / 4, 0);
+    k.store(sK, LDK, n, D, DP / 4, 0, power);
+    v.store(sV, LDV, n, V, VP / 4, 0, one);
+    base = Batch<T>::N;
+  }
+  stage(K, (size_t)ldp, n, D, DP, sK, LDK, vec, power, base);
+  stage(Vp, (size_t)ldp, n, V, VP, sV, LDV, vec, one, base);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
   const int steps = (n + 3) / 4;
@@ -82,6 +125,7 @@ lightning_local_k(const T* __restrict__ proj, int ldp, const float* __restrict__
     f32x4 acc[NVT];
 #pragma unroll
     for (int j = 0; j < NVT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
     for (int s = 0; s < steps; s++) {
       const float a = sK[(4 * s + k4) * LDK + dt * 16 + i16];
 #pragma unroll
@@ -146,11 +190,37 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
   const T* row = proj + (size_t)en.row0 * ldp;
   const float* p = pw + (size_t)h * (LC + 1);
   auto one = [](int) { return 1.0f; };
-  stage(row + (size_t)h * D, (size_t)ldp, n, D, DP, sQ, LDQ, vec, one);
-  stage(row + (size_t)H * D + h * D, (size_t)ldp, n, D, DP, sK, LDQ, vec, one);
-  __syncthreads();
+  const T *Qp = row + (size_t)h * D, *Kp = Qp + (size_t)H * D, *Vp = row + (size_t)2 * H * D + h * V;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
   const int r0 = wave * 16;                                  // this wavefront's 16 tokens
+  // the state's rows, four blocks of four ahead of their products
+  const float* S = cs + ((size_t)c * H + h) * D * V;
+  constexpr int AHEAD = 4;
+  float st[AHEAD][NVT];
+  auto rows_of = [&](int s, float (&b)[NVT]) {
+    const float* Sr = S + (size_t)min(4 * s + k4, D - 1) * V;
+#pragma unroll
+    for (int j = 0; j < NVT; j++) b[j] = Sr[min(j * 16 + i16, V - 1)];
+  };
+  Batch<T> vb;                                               // the values, until the keys' place is free
+  int base = 0;
+  if (vec) {
+    Batch<T> qb, kb;
+    qb.load(Qp, (size_t)ldp, n, D, DP / 4, 0);
+    kb.load(Kp, (size_t)ldp, n, D, DP / 4, 0);
+    vb.load(Vp, (size_t)ldp, n, V, VP / 4, 0);
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) rows_of(u, st[u]);
+    qb.store(sQ, LDQ, n, D, DP / 4, 0, one);
+    kb.store(sK, LDQ, n, D, DP / 4, 0, one);
+    base = Batch<T>::N;
+  } else {
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) rows_of(u, st[u]);
+  }
+  stage(Qp, (size_t)ldp, n, D, DP, sQ, LDQ, vec, one, base);
+  stage(Kp, (size_t)ldp, n, D, DP, sK, LDQ, vec, one, base);
+  __syncthreads();
   // weights lam^(t-s) q_t . k_s, s <= t
   f32x4 w[LC / 16];
 #pragma unroll
@@ -160,6 +230,7 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
 #pragma unroll
   for (int j = 0; j < NVT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (r0 < n) {
+#pragma unroll 4
     for (int s = 0; s < DP / 4; s++) {
       const float a = sQ[(r0 + i16) * LDQ + 4 * s + k4];
 #pragma unroll
@@ -167,17 +238,15 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
         if (j <= wave)
           w[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sK[(j * 16 + i16) * LDQ + 4 * s + k4], w[j], 0, 0, 0);
     }
-    const float* S = cs + ((size_t)c * H + h) * D * V;
-#pragma unroll 2
-    for (int s = 0; s < DP / 4; s++) {
-      const float a = sQ[(r0 + i16) * LDQ + 4 * s + k4];     // zero beyond D
-      const float* Sr = S + (size_t)min(4 * s + k4, D - 1) * V;
-      float b[NVT];
+    for (int s0 = 0; s0 < DP / 4; s0 += AHEAD) {             // (DP is a multiple of 16)
 #pragma unroll
-      for (int j = 0; j < NVT; j++) b[j] = Sr[min(j * 16 + i16, V - 1)];
+      for (int u = 0; u < AHEAD; u++) {
+        const float a = sQ[(r0 + i16) * LDQ + 4 * (s0 + u) + k4];   // zero beyond D
 #pragma unroll
-      for (int j = 0; j < NVT; j++)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[j], acc[j], 0, 0, 0);
+        for (int j = 0; j < NVT; j++)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, st[u][j], acc[j], 0, 0, 0);
+        rows_of(s0 + u + AHEAD, st[u]);
+      }
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -187,7 +256,8 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
     }
   }
   __syncthreads();   // queries and keys have been read
-  stage(row + (size_t)2 * H * D + h * V, (size_t)ldp, n, V, VP, sV, LDV, vec, one);
+  if (vec) vb.store(sV, LDV, n, V, VP / 4, 0, one);
+  stage(Vp, (size_t)ldp, n, V, VP, sV, LDV, vec, one, base);
 #pragma unroll
   for (int j = 0; j < LC / 16; j++)
 #pragma unroll
@@ -197,6 +267,7 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
     }
   __syncthreads();
   if (r0 >= n) return;
+#pragma unroll 4
   for (int s = 0; s < (wave + 1) * 4; s++) {
     const float a = sP[(r0 + i16) * LDP + 4 * s + k4];
 #pragma unroll
