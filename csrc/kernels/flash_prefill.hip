@@ -16,7 +16,10 @@
 // O(T^2): here each K/V tile is read once per 16 query tokens x G heads.
 // Behavioural parity: the reference delegates prompt processing to an external
 // Ollama server (`web/streamlit_app.py:89-101`), see SURVEY.md §2B.2 B2.3.
+#include <type_traits>
+
 #include "common.h"
+#include "lds_pipe.h"
 
 namespace {
 
@@ -192,30 +195,29 @@ int launch(const bf16* q, int ldq, const bf16* kc, const bf16* vc, const int* bt
 }
 
 // ---------------------------------------------------------------------------------
-// v2: 256 query rows per workgroup (8 waves x 32 rows), one 64-key page per K/V tile,
+// v2: 128 or 256 query rows per workgroup (NW = 4 or 8 waves x 32 rows), one 64-key page per K/V tile,
 // v_mfma_f32_32x32x16_bf16 throughout.
 //
-// A workgroup = one KV head x QT = 256/G consecutive tokens of one sequence; wave w
-// owns q head kvh*G + w/(8/G) and 32 of the tokens, so every K/V page staged in LDS
-// feeds 256 (token, head) rows -- 16x the reuse of v1 (16 tokens x G heads).
+// A workgroup = one KV head x QT = 32 NW / G consecutive tokens of one sequence; wave w
+// owns q head kvh*G + w/(NW/G) and 32 of the tokens, so every K/V page staged in LDS
+// feeds 128 or 256 (token, head) rows -- 8x or 16x the reuse of v1 (16 tokens x G heads).
 // Per 64-key tile and wave, both products keep the query row on the lane:
 //   S^T[32 keys x 32 rows] = K . Q^T   (per 32-key half: 8 MFMAs over d = 128)
 //   O^T[128 d  x 32 rows] += V^T . P^T (4 d-blocks x 2 halves x 2 k-steps = 16 MFMAs)
 // so the online-softmax statistics and the O rescale are per lane (no cross-lane
 // moves but one xor-32 for the row max / sum).  The S^T accumulator registers are
-// directly the P^T B operand (cdna_hip_programming.md §3 "An accumulator tile as the
-// next MFMA's operand"): register 8s+j of lane half h holds S^T row
+// directly the P^T B operand: register 8s+j of lane half h holds S^T row
 // 16s + 8(j>>2) + 4h + (j&3); the K rows are loaded permuted (row rho <- key
 // kappa(rho)) so that this row is key 16s + 8h + j, i.e. the eight keys a lane
-// contributes to one k-step are CONSECUTIVE -- the V^T A-fragment is then a single
-// 16-byte LDS read of a [d][key] image.  K is staged row-major [key][d] (272-B rows:
-// conflict-free b128 reads), V transposed to [d][key] (144-B rows) while staging.
-// The next page's global loads are issued right after the barrier and land in
-// registers while the MFMAs run (one barrier per tile, two LDS stages).
-constexpr int KLD2 = HD + 8;  // K image row stride (bf16)
-constexpr int VLD2 = 64 + 8;  // V^T image row stride (bf16)
-constexpr int KS_ELEMS = 64 * KLD2, VS_ELEMS = HD * VLD2;
-
+// contributes to one k-step are CONSECUTIVE.  Rows of 256 bytes in LDS, 16-byte piece p of row r at
+// p ^ (r & 15) (K: 16 rows x a piece per read) and p ^ 4 (r & 3) (V: 4 rows x 64 bytes): no bank conflicts.
+// What bounds it: a wavefront's chain per page (scores, maximum, exponentials, second product), with one or two
+// wavefronts per SIMD to fill it.  So the page's K and V come by LDS DMA (no registers, no stores), V is read
+// transposed (ds_read_b64_tr_b16) from the rows as they are, and a page's exponentials run between the products of the
+// page before with V (K is a page ahead of V for that; two stages of each).
+// One prompt, 32 heads on 8, per layer: 128 rows (16-token tiles) 9.1 -> 8.2 us with 4 waves, 256 14.5 -> 10.7, 512 25.5 ->
+// 16.0, 700 34.6 -> 20.9; 1024 (8 waves, K and V through registers, V transposed by 2-byte stores) 38.6 -> 28.5, 2048
+// 68 -> 55, 4096 162 -> 168 (8 waves 163).
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ int kperm(int rho) {  // S^T row rho -> key within the 32-key half
@@ -223,14 +225,15 @@ __device__ __forceinline__ int kperm(int rho) {  // S^T row rho -> key within th
   return 16 * s + 8 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
 }
 
-template <int G>
-__global__ __launch_bounds__(512) void flash_prefill2_kernel(
+template <int G, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void flash_prefill2_kernel(
     const bf16* __restrict__ q, int ldq, const bf16* __restrict__ kc,
     const bf16* __restrict__ vc, const int* __restrict__ bt, int bt_stride,
     const Tile* __restrict__ tiles, int n_tiles, int Hkv, float scale_log2,
     bf16* __restrict__ out, int ldo) {
-  constexpr int WPH = 8 / G;  // waves per q head
-  __shared__ __attribute__((aligned(16))) bf16 lds[2 * (KS_ELEMS + VS_ELEMS)];
+  constexpr int WPH = NW / G;  // waves per q head
+  constexpr int PG = PAGE * HD;                                  // numbers of a page's K (V)
+  __shared__ __attribute__((aligned(16))) bf16 lds[4 * PG];      // K, K, V, V
 
   // heads outermost, heaviest (latest) tiles first; one head's tiles share an XCD's L2
   const int nb = n_tiles * Hkv;
@@ -238,13 +241,39 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(
   const int kvh = b / n_tiles, ti = n_tiles - 1 - b % n_tiles;
   const Tile T = tiles[ti];
   if (T.n <= 0) return;  // padding tile of a graph-captured prefill (fixed grid)
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r32 = lane & 31, hh = lane >> 5;
   const int h = kvh * G + w / WPH;
   const int t = (w % WPH) * 32 + r32;      // token of this lane's query row
   const int tok = t < T.n ? t : T.n - 1;
   const int my_pos = T.pos0 + tok;
   const int row = T.row0 + tok;
+
+  const int last = T.pos0 + T.n - 1;
+  const int n_kt = last / PAGE + 1;
+  const int* btr = bt + (size_t)T.seq * bt_stride;
+  const size_t head_off = (size_t)kvh * PG;
+  const size_t page_sz = (size_t)Hkv * PG;
+
+  // copies: an instruction takes four rows; this wave's are rows 4 (w + NW i) + lane / 16.  Rows past the last key
+  // (whatever they hold) are that key's again
+  constexpr int CP = 16 / NW;
+  const unsigned l0 = __builtin_amdgcn_readfirstlane(ldsp::lds_off(lds)) + w * 1024;
+  const int cr = 4 * w + (lane >> 4), cp = lane & 15;
+  auto copy = [&](const bf16* pool, int kt, int page, unsigned dst, bool is_v) {
+    const void* base = pool + (size_t)page * page_sz + head_off;
+    const int lim = last - kt * PAGE;
+#pragma unroll
+    for (int i = 0; i < CP; ++i) {
+      const int r = cr + 4 * NW * i;
+      ldsp::dma_lds16(base, min(r, lim) * (HD * 2) + ((cp ^ (is_v ? 4 * (r & 3) : r & 15)) << 4), dst + i * NW * 1024);
+    }
+  };
+  auto copy_k = [&](int kt, int page) { copy(kc, kt, page, l0 + (kt & 1) * (PG * 2), false); };
+  auto copy_v = [&](int kt, int page) { copy(vc, kt, page, l0 + (2 + (kt & 1)) * (PG * 2), true); };
+  auto page_of = [&](int kt) { return btr[min(kt, n_kt - 1)]; };
+  int p0 = page_of(0), p1 = page_of(1);    // pages kt and kt + 1
+  copy_k(0, p0);
 
   // Q^T B fragments: k-step s covers d = 16s .. 16s+15, lane half hh holds 8hh .. 8hh+7
   bf16x8 qf[8];
@@ -260,64 +289,79 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(
     for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
   float m = -INFINITY, l = 0.f;
 
-  const int last = T.pos0 + T.n - 1;
-  const int n_kt = last / PAGE + 1;
-  const int* btr = bt + (size_t)T.seq * bt_stride;
-  const size_t head_off = (size_t)kvh * PAGE * HD;
-  const size_t page_sz = (size_t)Hkv * PAGE * HD;
-  const int krow = kperm(r32);
-
-  // K/V of a page travel global -> registers -> LDS.  Two register sets, so a page's
-  // loads are issued two tiles before it is staged: a fetch has two tiles of MFMA work
-  // (~2 us at 8 waves) to land instead of one, which left the loop waiting on L2/HBM.
-  bf16x8 kA[2], vA[2], kB[2], vB[2];
-  auto fetch = [&](int kt, bf16x8 (&kr)[2], bf16x8 (&vr)[2]) {
-    const size_t base = (size_t)btr[kt] * page_sz + head_off;
-    const bf16x8* kp = reinterpret_cast<const bf16x8*>(kc + base);
-    const bf16x8* vp = reinterpret_cast<const bf16x8*>(vc + base);
-  // K: chunk c = key (c >> 4), dims 8 (c & 15)..+7 (row-major image, b128 stores).
-  // V: chunk c = key (c & 63), dims 8 (c >> 6)..+7 -- the 64 lanes of a wave hold the 64
-  // keys of ONE 8-dim column block, so each of the eight transposed b16 stores writes 128
-  // contiguous bytes of one V^T row (bank-conflict free; with a lane per dim chunk instead
-  // they hit 2 banks, 8-16 way conflicts that cost more than the tile's MFMAs).
+  // K rows kperm(r32) and 32 further; V: lane L of 16 names row L / 4 of four and 4 of 16 numbers, see read_v
+  const int krow = kperm(r32), L = lane & 15;
+  const bf16* kl = lds + krow * HD;
+  const bf16* vl = lds + 2 * PG + (8 * hh + (L >> 2)) * HD + 4 * (L & 1);
+  const int vp = 2 * ((lane >> 4) & 1) + ((L >> 1) & 1);
+  auto read_k = [&](int st, int kh, int s) {
+    return *reinterpret_cast<const bf16x8*>(kl + st * PG + 32 * kh * HD + (((2 * s + hh) ^ (krow & 15)) << 3));
+  };
+  // V^T of numbers 32 db + r32, keys 32 kh + 16 s2 + 8 hh + 0 .. 7
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* lds4_t;
+  auto read_v = [&](int st, int db, int kh, int s2) {
+    const bf16* p = vl + st * PG + (32 * kh + 16 * s2) * HD + ((((db ^ (L >> 2)) << 2) | vp) << 3);
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)p);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(p + 4 * HD));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  f32x16_t sc[2];
+  bf16x8 pf[2][2];   // P^T of the page before
+  // O^T += V^T . P^T of page `of`, in eight pairs of products; LDS reads go out a pair ahead of the products that take
+  // them, and between the pairs runs `work`
+  auto second_product = [&](int of, auto&& work) {
+    const int st = of & 1;
+    bf16x8 vf[2][2];
+    auto read_v2 = [&](int j) {   // half j & 1 of the keys, numbers 32 (j / 2) ..
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int c = tid + 512 * i;
-      kr[i] = kp[c];
-      vr[i] = vp[(c & 63) * (HD / 8) + (c >> 6)];
+      for (int i = 0; i < 2; ++i) vf[j & 1][i] = read_v(st, j >> 1, j & 1, i);
+    };
+    read_v2(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j < 7) read_v2(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        o[j >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[j & 1][i], pf[j & 1][i], o[j >> 1], 0, 0, 0);
+      work(j);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto stash = [&](int st, const bf16x8 (&kr)[2], const bf16x8 (&vr)[2]) {
-    bf16* Ks = lds + st * (KS_ELEMS + VS_ELEMS);
-    bf16* Vt = Ks + KS_ELEMS;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int c = tid + 512 * i;
-      *reinterpret_cast<bf16x8*>(&Ks[(c >> 4) * KLD2 + (c & 15) * 8]) = kr[i];
-      const int key = c & 63, d0 = (c >> 6) * 8;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) Vt[(d0 + j) * VLD2 + key] = vr[i][j];
-    }
-  };
-  auto tile = [&](int kt, int st) {
-    const bf16* Ks = lds + st * (KS_ELEMS + VS_ELEMS);
-    const bf16* Vt = Ks + KS_ELEMS;
 
+  for (int kt = 0; kt < n_kt; ++kt) {
+    // K of this page and V of the one before have landed; every wave is past the last page's K and the V before it
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    copy_v(kt, p0);
+    if (kt + 1 < n_kt) copy_k(kt + 1, p1);
+    p0 = p1;
+    p1 = page_of(kt + 2);
     // ---- S^T = K . Q^T, two 32-key halves ----
-    f32x16_t sc[2];
+    {
+      bf16x8 kf[2][2];
+      auto read_k2 = [&](int s) {
 #pragma unroll
-    for (int kh = 0; kh < 2; ++kh) {
+        for (int kh = 0; kh < 2; ++kh) kf[s & 1][kh] = read_k(kt & 1, kh, s);
+      };
+      read_k2(0);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sc[kh][i] = 0.f;
-      const bf16* kp = Ks + (32 * kh + krow) * KLD2 + 8 * hh;
+      for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
-        sc[kh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            *reinterpret_cast<const bf16x8*>(kp + 16 * s), qf[s], sc[kh], 0, 0, 0);
+        for (int i = 0; i < 16; ++i) sc[kh][i] = 0.f;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        if (s < 7) read_k2(s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh)
+          sc[kh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s & 1][kh], qf[s], sc[kh], 0, 0, 0);
+      }
     }
     // ---- online softmax for this lane's query row (keys of reg rr: 16(rr>>3)+8hh+(rr&7)) ----
     // m is the running max of the RAW scores; p = exp2(s * c - m * c) is one FMA + exp.
-    // Deferred rescale (cdna_hip_programming.md T13): O and l are rescaled only when some
+    // Deferred rescale: O and l are rescaled only when some
     // row's max grew by more than RESCALE_THR (log2 units) -- wave-uniform decision, each
     // lane with its own factor -- so most tiles skip the 64-register multiply; the
     // unrescaled p stay <= 2^RESCALE_THR, exact in fp32 and safe in bf16.
@@ -340,53 +384,44 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) mx = fmaxf(mx, sc[kh][rr]);
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (__any((mx - m) * scale_log2 > RESCALE_THR)) {
+    const bool rescale = __any((mx - m) * scale_log2 > RESCALE_THR);
+    float alpha = 1.f;
+    if (rescale) {
       const float mn = fmaxf(m, mx);
-      const float alpha = exp2f((m - mn) * scale_log2);
+      alpha = exp2f((m - mn) * scale_log2);
       m = mn;
       l *= alpha;
-#pragma unroll
-      for (int db = 0; db < 4; ++db) o[db] *= alpha;
     }
     const float mc = m * scale_log2;
     float ps = 0.f;
-    bf16x8 pf[2][2];
+    bf16x8 pn[2][2];
+    auto exps = [&](int j) {
 #pragma unroll
-    for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-      for (int rr = 0; rr < 16; ++rr) {
+      for (int e = 0; e < 4; ++e) {
+        const int kh = j >> 2, rr = (j & 3) * 4 + e;
         // raw v_exp_f32 (arguments <= RESCALE_THR; underflow to 0 is what we want)
         const float p = __builtin_amdgcn_exp2f(fmaf(sc[kh][rr], scale_log2, -mc));
         ps += p;
-        pf[kh][rr >> 3][rr & 7] = f2bf(p);
+        pn[kh][rr >> 3][rr & 7] = f2bf(p);
       }
-    l += ps;
-    // ---- O^T += V^T . P^T ----
+    };
+    if (kt > 0) {
+      second_product(kt - 1, exps);
+    } else {
 #pragma unroll
-    for (int db = 0; db < 4; ++db) {
-      const bf16* vp = Vt + (32 * db + r32) * VLD2 + 8 * hh;
-#pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              *reinterpret_cast<const bf16x8*>(vp + 32 * kh + 16 * s2), pf[kh][s2], o[db], 0, 0, 0);
+      for (int j = 0; j < 8; ++j) exps(j);
     }
-  };
-
-  fetch(0, kA, vA);
-  if (n_kt > 1) fetch(1, kB, vB);
-  for (int kt = 0; kt < n_kt; kt += 2) {
-    stash(0, kA, vA);
-    __syncthreads();  // stage 0 complete; every wave is past tile kt-1 (WAR on stage 1)
-    if (kt + 2 < n_kt) fetch(kt + 2, kA, vA);
-    tile(kt, 0);
-    if (kt + 1 >= n_kt) break;
-    stash(1, kB, vB);
-    __syncthreads();
-    if (kt + 3 < n_kt) fetch(kt + 3, kB, vB);
-    tile(kt + 1, 1);
+    l += ps;
+    if (rescale) {   // (O has the page before by now, which the old maximum scaled)
+#pragma unroll
+      for (int db = 0; db < 4; ++db) o[db] *= alpha;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pf[i >> 1][i & 1] = pn[i >> 1][i & 1];
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  second_product(n_kt - 1, [](int) {});
 
   l += __shfl_xor(l, 32, 64);
   if (t < T.n) {
@@ -404,19 +439,19 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(
   }
 }
 
-template <int G>
+template <int G, int NW>
 int launch2(const bf16* q, int ldq, const bf16* kc, const bf16* vc, const int* bt, int bt_stride,
             const Tile* tiles, int n_tiles, int Hkv, float scale, bf16* out, int ldo,
             hipStream_t st) {
   const float sl2 = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL(flash_prefill2_kernel<G>, dim3(n_tiles * Hkv), dim3(512), 0, st, q, ldq, kc,
+  hipLaunchKernelGGL((flash_prefill2_kernel<G, NW>), dim3(n_tiles * Hkv), dim3(64 * NW), 0, st, q, ldq, kc,
                      vc, bt, bt_stride, tiles, n_tiles, Hkv, sl2, out, ldo);
   P2P_CHECK_LAUNCH();
 }
 
 }  // namespace
 
-// v2 entry: tiles of at most 256 / (Hq/Hkv) tokens (p2p_flash_prefill_tile), otherwise as
+// v2 entry: tiles of at most `tile` tokens, 256 / (Hq/Hkv) (p2p_flash_prefill_tile) or fewer, otherwise as
 // p2p_flash_prefill.  K/V pages must be whole 64-key pages of the block table.
 P2P_API int p2p_flash_prefill_tile(int Hq, int Hkv) {
   if (Hkv <= 0 || Hq % Hkv) return 0;
@@ -427,8 +462,8 @@ P2P_API int p2p_flash_prefill_tile(int Hq, int Hkv) {
 P2P_API int p2p_flash_prefill2(const void* q, int ldq, const void* kc, const void* vc,
                                const int* bt, int bt_stride, const int* tiles, int n_tiles,
                                int Hq, int Hkv, int head_dim, float scale, void* out, int ldo,
-                               void* stream) {
-  if (head_dim != HD || Hkv <= 0 || Hq % Hkv) return 1;
+                               int tile, void* stream) {
+  if (head_dim != HD || Hkv <= 0 || Hq % Hkv || tile < 1 || tile > p2p_flash_prefill_tile(Hq, Hkv)) return 1;
   if (n_tiles <= 0) return 0;
   auto Q = (const bf16*)q;
   auto K = (const bf16*)kc;
@@ -436,13 +471,16 @@ P2P_API int p2p_flash_prefill2(const void* q, int ldq, const void* kc, const voi
   auto T = (const Tile*)tiles;
   auto O = (bf16*)out;
   auto st = (hipStream_t)stream;
+  const bool narrow = tile * (Hq / Hkv) <= 128;   // four waves hold the tile
+#define FLASH2(G, NW) launch2<G, NW>(Q, ldq, K, V, bt, bt_stride, T, n_tiles, Hkv, scale, O, ldo, st)
   switch (Hq / Hkv) {
-    case 1: return launch2<1>(Q, ldq, K, V, bt, bt_stride, T, n_tiles, Hkv, scale, O, ldo, st);
-    case 2: return launch2<2>(Q, ldq, K, V, bt, bt_stride, T, n_tiles, Hkv, scale, O, ldo, st);
-    case 4: return launch2<4>(Q, ldq, K, V, bt, bt_stride, T, n_tiles, Hkv, scale, O, ldo, st);
-    case 8: return launch2<8>(Q, ldq, K, V, bt, bt_stride, T, n_tiles, Hkv, scale, O, ldo, st);
+    case 1: return narrow ? FLASH2(1, 4) : FLASH2(1, 8);
+    case 2: return narrow ? FLASH2(2, 4) : FLASH2(2, 8);
+    case 4: return narrow ? FLASH2(4, 4) : FLASH2(4, 8);
+    case 8: return FLASH2(8, 8);
     default: return 2;
   }
+#undef FLASH2
 }
 
 // tiles: int32 [n_tiles, 4] = (first row, n tokens <= 16, sequence, first position);

@@ -39,7 +39,7 @@ _SIGS = {
     "p2p_flash_prefill": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
                           c_int, c_int, c_int, c_float, c_void_p, c_int, c_void_p],
     "p2p_flash_prefill2": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
-                           c_int, c_int, c_int, c_float, c_void_p, c_int, c_void_p],
+                           c_int, c_int, c_int, c_float, c_void_p, c_int, c_int, c_void_p],
     "p2p_flash_prefill_tile": [c_int, c_int],
     "p2p_tall_silu": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float,
                       c_void_p],

@@ -273,24 +273,29 @@ def attn_oproj_heads(q, k_cache, v_cache, block_tables, row_bt, ctx_lens, n_head
 
 
 QTILE = 16
-# v2 flash prefill (256 query rows per workgroup, 32x32x16 MFMA); P2P_FLASH_V2=0 selects v1
+# v2 flash prefill (128 or 256 query rows per workgroup, 32x32x16 MFMA); P2P_FLASH_V2=0 selects v1
 FLASH_V2 = os.environ.get("P2P_FLASH_V2", "1") != "0"
 
 
-# v2 pays from about this many (query tile, kv head) workgroups; below it the 16-token
-# v1 tiles spread a short prompt over more CUs (profiles/r2_flash_prefill_v2.jsonl:
-# T=512 v1 27 us vs v2 40 us; T=2048 v2 138 us vs v1 236 us)
-FLASH_V2_MIN_BLOCKS = 128  # v1 wins up to T=512 at 8 KV heads, v2 from ~1K (profiles/r2_flash_prefill_v2_conflict_free.jsonl)
+# v2 tiles of 128 query rows (4 waves) pay from about this many rows, below it the 16-token v1 tiles spread a short
+# prompt over more CUs (one prompt, 32 heads on 8, v1 / v2 us: 64 rows 6.2 / 7.1, 100 7.8 / 8.2, 128 9.1 / 8.2, 256 14.5 /
+# 10.7, 1024 49.8 / 28.5).  With 8 query heads per kv head a tile of 32 tokens takes 8 waves, which pay from about
+# FLASH_V2_MIN_BLOCKS (query tile, kv head) workgroups (512 rows 25.5 / 23.1).
+FLASH_V2_MIN_ROWS = 128
+FLASH_V2_MIN_BLOCKS = 128
 
 
 def flash_tile(n_heads: int, n_kv: int, rows: int | None = None) -> int:
-    """Tokens per query tile for a prefill chunk of ``rows`` tokens: v2 (256 / (Hq/Hkv))
-    when it yields enough workgroups, else v1 (16)."""
+    """Tokens per query tile: the widest that v2 takes (256 / (Hq/Hkv)), or for a prefill chunk of ``rows`` tokens v2's
+    128 query rows (8 heads per kv head: 256) where they pay, else v1's 16 tokens."""
     G = n_heads // n_kv
     if FLASH_V2 and G in (1, 2, 4, 8):
-        t = 256 // G
-        if rows is None or -(-rows // t) * n_kv >= FLASH_V2_MIN_BLOCKS:
-            return t
+        if rows is None:
+            return 256 // G
+        if G < 8 and rows >= FLASH_V2_MIN_ROWS:
+            return 128 // G
+        if G == 8 and -(-rows // (256 // G)) * n_kv >= FLASH_V2_MIN_BLOCKS:
+            return 256 // G
     return QTILE
 
 
@@ -345,12 +350,12 @@ def flash_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         return paged_attention_ref(q, k_cache, v_cache, block_tables, row_bt, ctx, n_heads, n_kv,
                                    scale, out)
     L = _lib.lib()
-    fn = L.p2p_flash_prefill2 if qtile > QTILE else L.p2p_flash_prefill
+    fn, wide = (L.p2p_flash_prefill2, (qtile,)) if qtile > QTILE else (L.p2p_flash_prefill, ())
     _lib.check(fn(q.data_ptr(), q.stride(0), k_cache.data_ptr(),
                                    v_cache.data_ptr(), block_tables.data_ptr(),
                                    block_tables.stride(0), tiles.data_ptr(), tiles.shape[0],
                                    n_heads, n_kv, HEAD_DIM, float(scale), out.data_ptr(),
-                                   out.stride(0), _lib.stream_ptr(q.device)), "flash_prefill")
+                                   out.stride(0), *wide, _lib.stream_ptr(q.device)), "flash_prefill")
     return out
 
 

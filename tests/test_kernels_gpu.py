@@ -572,6 +572,35 @@ def test_flash_prefill(G, lens, v2, monkeypatch):
     assert _rel(out.cpu(), row.cpu()) < 1e-2
 
 
+@pytest.mark.parametrize("G,width", [(1, 128), (2, 64), (4, 32), (4, 64), (8, 32), (4, 17)])
+@pytest.mark.parametrize("lens", [[(0, 1)], [(0, 64), (64, 65)], [(191, 2), (0, 130), (500, 33)]])
+def test_flash_prefill_widths(G, width, lens):
+    """Four and eight waves per tile, last tiles of every height, contexts that end in every part of a page and one to
+    several pages; what lies past a context (the rest of its last page) is NaN and must not be read.  P is rounded
+    to bf16 and so is the result: twice 2^-9 and their sums' fp32 rounding."""
+    g = torch.Generator().manual_seed(G + width)
+    Hkv, B = 2, len(lens)
+    Hq = Hkv * G
+    npg = (max(s + n for s, n in lens) + 63) // 64
+    k, v = _make_cache(1 + B * npg, Hkv, seed=G)
+    bt = (torch.randperm(B * npg, generator=g) + 1).view(B, npg).to(torch.int32)
+    seq, pos = [], []
+    for b, (s0, n) in enumerate(lens):
+        seq += [b] * n
+        pos += list(range(s0, s0 + n))
+        end = s0 + n
+        last = int(bt[b, (end - 1) // 64])
+        k[last, :, (end - 1) % 64 + 1:] = float("nan")
+        v[last, :, (end - 1) % 64 + 1:] = float("nan")
+    R = len(seq)
+    q = torch.randn(R, Hq * 128, generator=g).to(torch.bfloat16)
+    ref = A.paged_attention_ref(q, k, v, bt, torch.tensor(seq, dtype=torch.int32), torch.tensor(pos, dtype=torch.int32) + 1,
+                                Hq, Hkv, 1 / math.sqrt(128), torch.empty(R, Hq * 128))
+    tiles = ops.prefill_tiles(seq, pos, width)
+    out = ops.flash_prefill(q.to(DEV), k.to(DEV), v.to(DEV), bt.to(DEV), tiles.to(DEV), Hq, Hkv, qtile=width)
+    assert float((out.float().cpu() - ref).norm() / ref.norm()) < 2 ** -8
+
+
 # ------------------------------------------------------------ rope + cache
 def test_rope_cache():
     from p2p_llm_chat_go_amd.models.config import LLAMA31_8B, rope_table
