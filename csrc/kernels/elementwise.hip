@@ -190,6 +190,27 @@ P2P_API int p2p_advance(int* ids, unsigned long long* keys, int* pos, int* ctx, 
   return (int)hipGetLastError();
 }
 
+// What the host reads behind decode steps, in one launch instead of three copies and waits (tokens, the hand-offs' fault
+// word, the split-K fault word: 35 us behind a step, 12 now): out is page-locked host memory
+__global__ __launch_bounds__(256) void step_report_kernel(const int* __restrict__ hist, int ldh, int n, int k,
+                                                          const int* __restrict__ err, const int* __restrict__ fault,
+                                                          int* __restrict__ out) {
+  for (int i = threadIdx.x; i < n * k; i += 256) out[i] = hist[(size_t)(i / k) * ldh + i % k];
+  if (threadIdx.x == 0) {
+    out[n * k] = *err;
+    out[n * k + 1] = fault ? *fault : 0;
+  }
+}
+
+extern "C" int* p2p_split_fault_word_ptr(hipStream_t st);
+
+P2P_API int p2p_step_report(const int* hist, int ldh, int n, int k, const int* err, int* out, hipStream_t st) {
+  if (n <= 0 || k <= 0 || ldh < k) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(step_report_kernel, dim3(1), dim3(256), 0, st, hist, ldh, n, k, err, p2p_split_fault_word_ptr(st),
+                     out);
+  return (int)hipGetLastError();
+}
+
 // Row-major X [M, K] -> fragment-major Xf: 16-row m-tiles, each K/32 MFMA A fragments of
 // 1 KiB (lane l of fragment (mt, s) holds X[16 mt + (l & 15)][32 s + 8 (l >> 4) .. + 7]);
 // rows past M are zero.  One thread per 16-byte chunk.

@@ -338,9 +338,7 @@ class Engine:
         last = [0] * B
         for j, r in enumerate(rows):  # rows are grouped by sequence, in order
             last[r[0]] = j
-        g.load(g.host_meta(rows, block_tables, last))
-        if sampled:
-            g.samp.load(list(sampling))
+        g.load(g.host_meta(rows, block_tables, last), list(sampling) if sampled else None)
         g.replay()
         return g.first[:B]
 
@@ -365,13 +363,14 @@ class Engine:
             params = []
         g = self.decode_graph(max(len(last_ids), batch_bucket or 1), ctx, greedy=greedy)
         st = g.state
-        st.load(last_ids, pos, block_tables)
+        st.load(last_ids, pos, block_tables, None if greedy else params)
         if greedy:
             g.replay(k)
         else:
-            g.step_sampled(params, k)
-        hist = st.hist[:len(last_ids), :k].cpu().tolist()
-        self.model.check_faults(st.ws)
+            g.replay_sampled(k)
+        hist, fault = st.report(len(last_ids), k)
+        if fault or self.model.comm is not None:   # (a group agrees on its faults at every step)
+            self.model.check_faults(st.ws)
         return hist
 
     # ------------------------------------------------------------- generate

@@ -33,11 +33,12 @@ class DecodeState:
         self.max_pages = max_pages
         self.max_steps = max_steps
         self.max_ctx = max_ctx
-        # ids | pos | ctx | slots | block tables | step: views of ONE device buffer, so `load`
-        # refreshes a batch's whole state with one host->device copy
+        # ids | pos | ctx | slots | block tables | step | sampling parameters: views of ONE device buffer, so
+        # `load` refreshes a batch's whole state with one host->device copy
         n = B * (4 + max_pages)
-        state = torch.zeros(n + 1, device=dev, dtype=i32)
-        self.meta, self.step = state[:n], state[n:]
+        at = (n + 2) // 2 * 2
+        state = torch.zeros(at + SamplerSlots.words(B), device=dev, dtype=i32)
+        self.meta, self.step = state[:n], state[n:n + 1]
         self.image = HostImage(state)
         self.ids, self.pos, self.ctx, self.slots = (self.meta[k * B:(k + 1) * B] for k in range(4))
         self.bt = self.meta[4 * B:].view(B, max_pages)
@@ -45,7 +46,8 @@ class DecodeState:
         self.row_bt = torch.arange(B, device=dev, dtype=i32)
         self.hist = torch.zeros(B, max_steps, device=dev, dtype=i32)
         self.ws = model.new_workspace(B, max_ctx)
-        self.samp = SamplerSlots(B, dev)  # sampled graphs read these (ops.sample)
+        self.samp = SamplerSlots(B, dev, self.image, at)  # sampled graphs read these (ops.sample)
+        self._report = None
         if model.tp > 1:  # vocab-parallel sampling: per-shard top-128 candidates, gathered
             W = model.tp
             self.cand_v = torch.empty(B, 128, device=dev, dtype=torch.float32)
@@ -62,13 +64,14 @@ class DecodeState:
         self.step.zero_()
         self.ws.keys.zero_()
 
-    def load(self, ids, pos, block_tables):
-        """ids/pos: int lists (n <= B); block_tables: list of page lists."""
+    def load(self, ids, pos, block_tables, params: list | None = None):
+        """ids/pos: int lists (n <= B); block_tables: list of page lists; params: the rows' SamplingParams, in
+        the same copy (None: the device's stay)."""
         n = len(ids)
         B, P = self.B, self.max_pages
         assert n <= B
         self.ws.keys.zero_()
-        host = self.image.fill()   # rows >= n: dummies (page 0, position 0)
+        host = self.image.fill()[:self.samp.at]   # rows >= n: dummies (page 0, position 0)
         host[:] = 0
         bt = host[4 * B:4 * B + B * P].reshape(B, P)
         for b, pages in enumerate(block_tables):
@@ -78,7 +81,24 @@ class DecodeState:
         host[:n] = ids
         host[2 * B:3 * B] = p + 1
         host[3 * B:4 * B] = bt[np.arange(B), p // PAGE] * PAGE + p % PAGE
-        self.image.send()
+        if params is None:
+            self.image.send(0, self.samp.at)
+        else:
+            self.samp.fill(params)
+            self.image.send()
+
+    def report(self, n: int, k: int) -> tuple:
+        """(the k newest-loaded steps' tokens of the first n rows as lists, a kernel's bounded wait timed out).  The
+        host waits once: tokens and fault words come in one launch that writes to page-locked memory."""
+        k = min(k, self.max_steps)
+        if not self.hist.is_cuda:
+            return self.hist[:n, :k].tolist(), False
+        if self._report is None:
+            self._report = torch.zeros(self.B * self.max_steps + 2, dtype=torch.int32, pin_memory=True)
+        ops.step_report(self.hist, n, k, self.ws.err, self._report)
+        torch.cuda.current_stream(self.hist.device).synchronize()
+        r = self._report.numpy()
+        return r[:n * k].reshape(n, k).tolist(), bool(r[n * k] or r[n * k + 1])
 
     def body_logits(self):
         """Forward only (sampling mode): logits of every row in ws.logits."""
@@ -253,8 +273,12 @@ class DecodeGraph:
         """n decode steps with per-row SamplingParams (temperature <= 0 rows stay greedy):
         the parameters are loaded into device slots, then each
         step is one replay -- forward, ops.sample and advance are all in the graph."""
-        assert not self.greedy
         self.state.samp.load(params)
+        self.replay_sampled(n)
+
+    def replay_sampled(self, n: int = 1):
+        """step_sampled with the parameters that the state holds."""
+        assert not self.greedy
         for _ in range(n):
             if self.graph is not None:
                 self.graph.replay()
@@ -302,8 +326,9 @@ class PrefillGraph:
         for name, n in sizes:
             self.offsets[name] = (o, n)
             o += n
-        self.meta = torch.zeros(o, device=dev, dtype=torch.int32)
-        self.image = HostImage(self.meta)
+        at = (o + 1) // 2 * 2   # (a sampled graph's parameters behind it, for one copy)
+        self.image = HostImage(torch.zeros(at + (0 if greedy else SamplerSlots.words(S)), device=dev, dtype=torch.int32))
+        self.meta = self.image.dev[:o]
         v = {name: self.meta[a:a + n] for name, (a, n) in self.offsets.items()}
         self.bt = v["bt"].view(S + 1, max_pages)
         self.seq, self.pos, self.ids, self.slots, self.ctx = (v[k] for k in ("seq", "pos", "ids",
@@ -314,7 +339,7 @@ class PrefillGraph:
         self.first = torch.zeros(S, device=dev, dtype=torch.int32)
         self.samp = None
         if not greedy:  # per-sequence sampling parameters, read by the captured ops.sample
-            self.samp = SamplerSlots(S, dev)
+            self.samp = SamplerSlots(S, dev, self.image, at)
             if model.tp > 1:  # vocab-parallel draw: top-128 per shard, one all-gather
                 W = model.tp
                 self.cand_v = torch.empty(S, 128, device=dev, dtype=torch.float32)
@@ -367,9 +392,15 @@ class PrefillGraph:
         v["tiles"][:4 * len(tl)] = np.asarray(tl, dtype=np.int32).reshape(-1)
         return torch.from_numpy(host)
 
-    def load(self, host: torch.Tensor):
-        self.image.fill()[:] = host.numpy()
-        self.image.send()
+    def load(self, host: torch.Tensor, params: list | None = None):
+        """The chunk's image and, for a sampled graph, its sequences' SamplingParams (None: the device's stay)."""
+        n = self.meta.shape[0]
+        self.image.fill()[:n] = host.numpy()
+        if params is None:
+            self.image.send(0, n)
+        else:
+            self.samp.fill(params)
+            self.image.send()
 
     # ------------------------------------------------------------------ device side
     def body(self):

@@ -69,8 +69,9 @@ class HostImage:
             self.busy = False
         return self.host.numpy()
 
-    def send(self):
-        self.dev.copy_(self.host, non_blocking=True)
+    def send(self, lo: int = 0, hi: int | None = None):
+        """Queue the copy of words lo .. hi - 1 (None: all)."""
+        self.dev[lo:hi].copy_(self.host[lo:hi], non_blocking=True)
         if self.sent is not None:
             self.sent.record(torch.cuda.current_stream(self.dev.device))
             self.busy = True
@@ -82,26 +83,36 @@ _PADDING = (0.0, 40, 0.9, 0)   # a row no sequence has: greedy, and the same in 
 class SamplerSlots:
     """Per-row sampling parameters of a decode batch as device tensors, read by the
     graph-captured ``ops.sample`` launch (so a sampled decode step replays like a
-    greedy one): views of one buffer, which ``load`` fills with one copy (each time: the native loop writes them too)."""
+    greedy one): views of one buffer, which ``load`` fills with one copy (each time: the native loop writes them too).
+    With ``image`` they are its words from ``at`` (even) on, and ``fill`` leaves the copy to the owner, who sends
+    them with its own words."""
 
-    def __init__(self, B: int, device):
-        self.B = B
+    def __init__(self, B: int, device, image: HostImage | None = None, at: int = 0):
+        self.B, self.at = B, at
+        self.image = HostImage(torch.zeros(self.words(B), device=device, dtype=torch.int32)) if image is None else image
         o = (3 * B + 1) // 2 * 2   # the seeds' 64-bit words after three 32-bit ones per row
-        self.buf = torch.zeros(o + 2 * B, device=device, dtype=torch.int32)
-        self.image = HostImage(self.buf)
+        self.buf = self.image.dev[at:at + self.words(B)]
         (self.temp, self.topk, self.topp, self.seeds), self.parts = (
             (v[:B].view(torch.float32), v[B:2 * B], v[2 * B:3 * B].view(torch.float32), v[o:].view(torch.int64))
-            for v in (self.buf, self.image.host))
+            for v in (self.buf, self.image.host[at:at + self.words(B)]))
         self.load([])
 
-    def load(self, params: list):
+    @staticmethod
+    def words(B: int) -> int:
+        return (3 * B + 1) // 2 * 2 + 2 * B
+
+    def fill(self, params: list):
+        """The rows' parameters into the image, which ``image.fill`` has freed."""
         params = params[:self.B]
         rows = [(p.temperature, p.top_k, p.top_p, p.resolved_seed()) for p in params]
         rows += [_PADDING] * (self.B - len(rows))
-        self.image.fill()
         for view, col in zip(self.parts, zip(*rows)):
             view.numpy()[:] = col
-        self.image.send()
+
+    def load(self, params: list):
+        self.image.fill()
+        self.fill(params)
+        self.image.send(self.at, self.at + self.words(self.B))
 
 
 def sample(logits: torch.Tensor, params: list, pos) -> torch.Tensor:

@@ -80,3 +80,13 @@ def advance(ids, pos, ctx, slots, block_tables, hist, step, keys=None):
                              block_tables.data_ptr(), block_tables.stride(0),
                              _lib.ptr(hist), 0 if hist is None else hist.stride(0),
                              step.data_ptr(), B, _lib.stream_ptr(ids.device)), "advance")
+
+
+def step_report(hist, n: int, k: int, err, out):
+    """hist[:n, :k] (int32), err[0] and the device's split-K fault word into ``out`` (page-locked int32, n * k + 2 words),
+    written by the launch itself: readable once the stream has been waited for."""
+    assert hist.dtype == err.dtype == out.dtype == torch.int32 and hist.stride(1) == 1
+    assert out.is_pinned() and out.is_contiguous() and out.numel() >= n * k + 2
+    assert 0 < n <= hist.shape[0] and 0 < k <= hist.shape[1]
+    _lib.check(_lib.lib().p2p_step_report(hist.data_ptr(), hist.stride(0), n, k, err.data_ptr(), out.data_ptr(),
+                                          _lib.stream_ptr(hist.device)), "step_report")

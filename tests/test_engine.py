@@ -159,6 +159,32 @@ def test_sampled_decode_graph_gpu():
     assert a != ref
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("greedy", [True, False])
+def test_decode_steps_read_back_once_gpu(greedy):
+    """decode_steps loads a batch's state and sampling parameters with one copy and reads tokens and fault words from one
+    launch: the tokens of the state's history, other parameters at the next call, and a fault still raises."""
+    from p2p_llm_chat_go_amd.engine.sampling import SamplingParams
+
+    cfg = TINY_LLAMA.replace(n_layers=2)
+    eng = Engine(cfg, weights=EngineWeights.random(cfg, "cuda", seed=9), device="cuda", kv_pages=32, max_batch=4)
+    prompts = [[1, 2, 3, 4, 5], [7] * 40, [3, 9]]
+    pages = [eng.kv.allocator.alloc(2) for _ in prompts]
+    first = eng.prefill(prompts, pages).cpu().tolist()
+    at = [len(p) for p in prompts]
+    seen = []
+    for seeds in ((5, 6, 7), (8, 9, 10), (5, 6, 7)):
+        params = None if greedy else [SamplingParams(temperature=1.3, top_k=64, top_p=0.95, seed=s) for s in seeds]
+        seen.append(eng.decode_steps(first, at, pages, 128, 5, params=params))
+        st = eng.decode_graph(3, 128, greedy=greedy).state
+        assert seen[-1] == st.hist[:3, :5].cpu().tolist()
+    assert seen[0] == seen[2] and (seen[0] == seen[1]) == greedy
+    st.ws.err.fill_(1)
+    with pytest.raises(RuntimeError):
+        eng.decode_steps(first, at, pages, 128, 1, params=params)
+    assert int(st.ws.err) == 0
+
+
 def test_fp8_quantize_roundtrip_cpu():
     from p2p_llm_chat_go_amd import ops
 
