@@ -216,8 +216,8 @@ int launch(const bf16* q, int ldq, const bf16* kc, const bf16* vc, const int* bt
 // transposed (ds_read_b64_tr_b16) from the rows as they are, and a page's exponentials run between the products of the
 // page before with V (K is a page ahead of V for that; two stages of each).
 // One prompt, 32 heads on 8, per layer: 128 rows (16-token tiles) 9.1 -> 8.2 us with 4 waves, 256 14.5 -> 10.7, 512 25.5 ->
-// 16.0, 700 34.6 -> 20.9; 1024 (8 waves, K and V through registers, V transposed by 2-byte stores) 38.6 -> 28.5, 2048
-// 68 -> 55, 4096 162 -> 168 (8 waves 163).
+// 16.0, 700 34.6 -> 20.9; 1024 (8 waves, K and V through registers, V transposed by 2-byte stores) 39 -> 28.5, 2048
+// 69 -> 55.  With 8 waves 1024 39 -> 38, 4096 149 -> 148, 8192 554 -> 557 (4 waves 156 and 564).  Same results to the bit.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ int kperm(int rho) {  // S^T row rho -> key within the 32-key half

@@ -314,7 +314,7 @@ class PrefillGraph:
         self.rows, self.n_seq, self.max_pages, self.max_ctx = rows, n_seq, max_pages, max_ctx
         self.n_out = n_seq
         self.greedy = greedy
-        self.qtile = ops.flash_tile(model.nq, model.nkv, rows)
+        self.qtile = ops.flash_tile(model.nq, model.nkv, rows, model.cfg.is_moe)
         # tiles never straddle sequences: <= rows / qtile + one partial tile per sequence
         # (the dummy sequence included) + one per wrap of the dummy rows' positions
         self.max_tiles = -(-rows // self.qtile) + n_seq + 1 + rows // (max_pages * PAGE) + 1

@@ -82,3 +82,19 @@ def test_launch_codes_of_few_rows_keep_their_own_size():
     finally:
         G._TUNE.clear()
         G._TUNE.update(saved)
+
+
+@pytest.mark.parametrize("nq,nkv", [(32, 32), (32, 16), (32, 8), (64, 8), (4, 1), (24, 8)])
+def test_query_tiles_by_rows(nq, nkv):
+    """v2 tiles of 128 query rows from 128 rows on, of 256 from 512 workgroups on (8 heads per kv head and models with a
+    router: 128); other head groups 16 tokens."""
+    from p2p_llm_chat_go_amd.ops import attention as A
+
+    G = nq // nkv
+    for rows in (1, 127, 128, 500, 1024, 2049, 40000):
+        blocks = -(-rows // (256 // G)) * nkv
+        many = blocks >= 128
+        wide = blocks >= (128 if G == 8 else 512)
+        want = 16 if G == 3 else 256 // G if wide else 128 // G if G < 8 and rows >= 128 else 16
+        assert A.flash_tile(nq, nkv, rows) == want
+        assert A.flash_tile(nq, nkv, rows, routed=True) == (256 // G if G != 3 and many else 16)

@@ -151,7 +151,7 @@ def test_skinny_two_groups_per_block(M, w, u):
 @pytest.mark.parametrize("K", [1024, 1536])
 def test_midm_gemm_every_epilogue(M, K):
     """The mid-M LDS-DMA kernel (launch-code bit ops.gemm.MIDM_FLAG: one column group per
-    workgroup, whole K, 4-wave k-split) on every epilogue vs fp32 references."""
+    workgroup, whole K, 8-wave k-split) on every epilogue vs fp32 references."""
     from p2p_llm_chat_go_amd.ops.gemm import MIDM_FLAG
 
     _every_epilogue(M, MIDM_FLAG, 1000 + M, K=K)
