@@ -88,11 +88,11 @@ class DecodeState:
             self.image.send()
 
     def report(self, n: int, k: int) -> tuple:
-        """(the k newest-loaded steps' tokens of the first n rows as lists, a kernel's bounded wait timed out).  The
+        """(the k steps' tokens of the first n rows as lists, a kernel's bounded wait may have timed out).  The
         host waits once: tokens and fault words come in one launch that writes to page-locked memory."""
         k = min(k, self.max_steps)
-        if not self.hist.is_cuda:
-            return self.hist[:n, :k].tolist(), False
+        if not self.hist.is_cuda or n * k == 0:   # (a group's rank may have no rows: check_faults reads the words)
+            return self.hist[:n, :k].tolist(), self.hist.is_cuda
         if self._report is None:
             self._report = torch.zeros(self.B * self.max_steps + 2, dtype=torch.int32, pin_memory=True)
         ops.step_report(self.hist, n, k, self.ws.err, self._report)
@@ -314,7 +314,8 @@ class PrefillGraph:
         self.rows, self.n_seq, self.max_pages, self.max_ctx = rows, n_seq, max_pages, max_ctx
         self.n_out = n_seq
         self.greedy = greedy
-        self.qtile = ops.flash_tile(model.nq, model.nkv, rows, model.cfg.is_moe)
+        routed = getattr(getattr(model, "cfg", None), "is_moe", False)
+        self.qtile = ops.flash_tile(model.nq, model.nkv, rows, routed)
         # tiles never straddle sequences: <= rows / qtile + one partial tile per sequence
         # (the dummy sequence included) + one per wrap of the dummy rows' positions
         self.max_tiles = -(-rows // self.qtile) + n_seq + 1 + rows // (max_pages * PAGE) + 1

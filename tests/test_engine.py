@@ -179,6 +179,8 @@ def test_decode_steps_read_back_once_gpu(greedy):
         st = eng.decode_graph(3, 128, greedy=greedy).state
         assert seen[-1] == st.hist[:3, :5].cpu().tolist()
     assert seen[0] == seen[2] and (seen[0] == seen[1]) == greedy
+    # a rank of a group may have no rows of its own
+    assert eng.decode_steps([], [], [], 128, 2, params=None if greedy else [], greedy=greedy) == []
     st.ws.err.fill_(1)
     with pytest.raises(RuntimeError):
         eng.decode_steps(first, at, pages, 128, 1, params=params)
