@@ -278,10 +278,10 @@ FLASH_V2 = os.environ.get("P2P_FLASH_V2", "1") != "0"
 
 
 # v2 tiles of 128 query rows (4 waves) pay from about this many rows, below it the 16-token v1 tiles spread a short
-# prompt over more CUs (one prompt, 32 heads on 8, v1 / v2 us: 64 rows 6.2 / 7.1, 100 7.8 / 8.2, 128 9.1 / 8.2, 256 14.5 /
-# 10.7, 1024 49.8 / 28.5) and up to where tiles of 256 take two rounds of the CUs and more (FLASH_V2_WIDE_BLOCKS: tiles of
+# prompt over more CUs (one prompt, 32 heads on 8, v1 / v2 us: 64 rows 6.0 / 7.0, 100 7.1 / 8.2, 128 8.1 / 8.2, 256 11.7 /
+# 10.7, 1000 40 / 28) and up to where tiles of 256 take two rounds of the CUs and more (FLASH_V2_WIDE_BLOCKS: tiles of
 # 128 / 256, 2048 rows 55 / 67, 3072 98 / 100, 4096 156 / 148, 8192 564 / 557).  With 8 query heads per kv head a tile of 32 tokens takes 8 waves, which pay from about
-# FLASH_V2_MIN_BLOCKS (query tile, kv head) workgroups (512 rows 25.5 / 23.1).
+# FLASH_V2_MIN_BLOCKS (query tile, kv head) workgroups (512 rows 19.5 / 22.9, 1024 41 / 38).
 FLASH_V2_MIN_ROWS = 128
 FLASH_V2_MIN_BLOCKS = 128
 FLASH_V2_WIDE_BLOCKS = 512
@@ -291,7 +291,7 @@ def flash_tile(n_heads: int, n_kv: int, rows: int | None = None, routed: bool = 
     """Tokens per query tile: the widest that v2 takes (256 / (Hq/Hkv)), or for a prefill chunk of ``rows`` tokens v2's
     128 or 256 query rows (8 heads per kv head: 256) where they pay, else v1's 16 tokens.  routed: the model has a router,
     whose choice between two nearly equal experts turns on the last bits of its input and moves a row's logits by 10 %
-    and more: it keeps v1 up to FLASH_V2_MIN_BLOCKS (700 rows 34.6 against 20.9 us a layer of 900), so that
+    and more: it keeps v1 up to FLASH_V2_MIN_BLOCKS (700 rows 29 against 21 us of a layer's 900), so that
     prompts are routed as they always were."""
     G = n_heads // n_kv
     if FLASH_V2 and G in (1, 2, 4, 8):

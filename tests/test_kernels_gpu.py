@@ -572,10 +572,10 @@ def test_flash_prefill(G, lens, v2, monkeypatch):
     assert _rel(out.cpu(), row.cpu()) < 1e-2
 
 
-@pytest.mark.parametrize("G,width", [(1, 128), (2, 64), (4, 32), (4, 64), (8, 32), (4, 17)])
-@pytest.mark.parametrize("lens", [[(0, 1)], [(0, 64), (64, 65)], [(191, 2), (0, 130), (500, 33)]])
+@pytest.mark.parametrize("G,width", [(1, 128), (2, 64), (4, 32), (4, 64), (8, 32), (4, 17), (1, 16), (2, 16), (4, 16), (8, 16)])
+@pytest.mark.parametrize("lens", [[(0, 1)], [(0, 64), (64, 65)], [(191, 2), (0, 130), (500, 33)], [(0, 31), (32, 1), (40, 60)]])
 def test_flash_prefill_widths(G, width, lens):
-    """Four and eight waves per tile, last tiles of every height, contexts that end in every part of a page and one to
+    """Tiles of 16 tokens and of four and eight waves, last tiles of every height, contexts that end in every part of a page and one to
     several pages; what lies past a context (the rest of its last page) is NaN and must not be read.  P is rounded
     to bf16 and so is the result: twice 2^-9 and their sums' fp32 rounding."""
     g = torch.Generator().manual_seed(G + width)
