@@ -191,7 +191,8 @@ P2P_API int p2p_advance(int* ids, unsigned long long* keys, int* pos, int* ctx, 
 }
 
 // What the host reads behind decode steps, in one launch instead of three copies and waits (tokens, the hand-offs' fault
-// word, the split-K fault word: 35 us behind a step, 12 now): out is page-locked host memory
+// word, the split-K fault word; a step of 8 layers, with its inputs in one copy as well, 880 -> 848 us): out is
+// page-locked host memory
 __global__ __launch_bounds__(256) void step_report_kernel(const int* __restrict__ hist, int ldh, int n, int k,
                                                           const int* __restrict__ err, const int* __restrict__ fault,
                                                           int* __restrict__ out) {
