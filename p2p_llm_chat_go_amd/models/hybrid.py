@@ -1884,7 +1884,7 @@ class HybridModel:
         rows that its product forms, those."""
         if isinstance(h, sm.NormedRows):
             x, spare = h.x, h.spare
-        if reader and reader.one_input and spare is not None:
+        if spare is not None and getattr(reader, "one_input", False):
             return x, spare, sm.NormedRows(x, spare, y, w, ls, self.cfg.eps, next_w, x if rows is None else rows)
         sm.norm_scale_add(x, y, w, ls, self.cfg.eps, next_w=next_w, next_out=rows)
         return x, spare, x if rows is None else rows
