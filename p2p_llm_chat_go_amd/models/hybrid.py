@@ -355,6 +355,18 @@ class StepBatch:
 
 
 # ---------------------------------------------------------------------------- mixers
+def takes_unformed(part) -> bool:
+    """Whether ``part.forward`` takes rows that are not formed yet (``sm.NormedRows``).  ``one_input = True`` promises it
+    for the forward() that the class declaring it has; a class below it with a forward() of its own reads a tensor, unless
+    it declares it too."""
+    for c in type(part).__mro__:
+        if "one_input" in vars(c):
+            return bool(c.one_input)
+        if "forward" in vars(c):
+            break
+    return False
+
+
 class Mixer:
     """One sequence mixer: weights + forward on a step.  ``cache_spec`` tells the sequence
     cache what the layer keeps between steps."""
@@ -383,8 +395,8 @@ class Mixer:
     # rows that read the layer input as ``w_in`` and implements ``mix`` on their product, so
     # that whoever owns the input (a layer with a gate, a ``parallel`` mixer) can run every
     # projection of the same input as one matrix product.
-    # one_input: forward() reads its input through one product alone, so it also takes rows that are not formed yet
-    # (``sm.NormedRows``)
+    # one_input: this class's forward() reads its input through one product alone, so it also takes rows that are not
+    # formed yet (see ``takes_unformed``)
     one_input = False
     w_in = None
     b_in = None   # bias of the input product (activation type), or None
@@ -1271,7 +1283,7 @@ class DenseFF:
     input of the output projection, [R, n_mid]; may return a part of the result that is added
     separately) and ``w_out`` [width, n_mid]."""
     ACT = "silu"
-    one_input = True   # see Mixer
+    one_input = True   # see ``takes_unformed``
 
     def __init__(self, spec: dict, width: int):
         self.spec, self.width = spec, width
@@ -1884,7 +1896,7 @@ class HybridModel:
         rows that its product forms, those."""
         if isinstance(h, sm.NormedRows):
             x, spare = h.x, h.spare
-        if spare is not None and getattr(reader, "one_input", False):
+        if spare is not None and takes_unformed(reader):
             return x, spare, sm.NormedRows(x, spare, y, w, ls, self.cfg.eps, next_w, x if rows is None else rows)
         sm.norm_scale_add(x, y, w, ls, self.cfg.eps, next_w=next_w, next_out=rows)
         return x, spare, x if rows is None else rows

@@ -95,3 +95,34 @@ def test_a_feed_forward_of_an_author(dev, design, monkeypatch):
                         lambda h, t, p, _: h @ t[p + "m"].T + h)
     t = mod.toks(sum(CUTS), cfg.vocab, 4)
     mod.close(_run(mod, mod.engine(cfg, sd, dev), t, CUTS), O.forward(c, sd, t))
+
+
+@pytest.mark.parametrize("dev", DEVICES)
+@pytest.mark.parametrize("design", ["Regesun", "Rasepel"])
+def test_parts_below_a_registered_one(dev, design, monkeypatch):
+    """A class below a registered one whose forward() is its own reads a tensor, in steps of any number of rows; one that
+    keeps the forward() it inherits, or says so itself, takes rows that are not formed."""
+    seen = []
+
+    def reading(base, **more):
+        def forward(self, h, *a):
+            seen.append((h.shape[0], type(h)))
+            return base.forward(self, h * 1.0, *a)
+        return type("Reading" + base.__name__, (base,), dict(more, forward=forward))
+
+    first, second = (Hy.GeneralDelta, Hy.Mamba2) if design == "Regesun" else (Hy.Lightning, Hy.Mamba1)
+    for base in (first, second):
+        monkeypatch.setitem(Hy.MIXERS, base.kind, reading(base))
+    monkeypatch.setitem(Hy.FEEDFORWARDS, "dense", reading(Hy.DenseFF))
+    _few_rows_everywhere(monkeypatch)
+    layers = [dict(Re.GD, mlp=Re.LA["mlp"]), Re.MB, Re.GD] if design == "Regesun" else [Ra.layer(Ra.LG, Ra.FF), Ra.MB, Ra.LG]
+    mod, O, c, cfg, sd = _build(design, monkeypatch, layers)
+    t = mod.toks(sum(CUTS), cfg.vocab, 5)
+    mod.close(_run(mod, mod.engine(cfg, sd, dev), t, CUTS), O.forward(c, sd, t))
+    assert {n for n, _ in seen} == set(CUTS) and {k for _, k in seen} == {torch.Tensor}
+
+    part = lambda cls: Hy.takes_unformed(object.__new__(cls))
+    for base in (first, second, Hy.DenseFF, Hy.LatentAttention, Hy.ConvAttention):
+        assert part(base) and part(type("Kept", (base,), {})) and part(reading(base, one_input=True))
+        assert not part(reading(base)) and not part(type("Below", (reading(base),), {}))
+    assert part(Hy.GeluFF) and not part(Hy.WindowAttention) and not part(Hy.MoEFF) and not part(Hy.Parallel)
