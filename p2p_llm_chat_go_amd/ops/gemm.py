@@ -120,11 +120,14 @@ def small_m_key(key, M):
 
 
 def set_tune(key, code: int, M: int | None = None):
-    """Record a launch code for ``key``; with ``M``, for the bucket of M rows inside its tile as well."""
+    """Record a launch code for ``key``: with ``M`` for the tile and for the bucket of M rows inside it, without for all
+    rows of the tile, whatever its buckets held."""
     _TUNE[key] = int(code)
-    fine = small_m_key(key, M) if M is not None else None
-    if fine is not None:
-        _TUNE[fine] = int(code)
+    if M is None:
+        for b in (1, 2, 4, 8, 16):
+            _TUNE.pop(small_m_key(key, b), None)
+    elif M <= 16:
+        _TUNE[small_m_key(key, M)] = int(code)
 
 
 TILED_MIN_M = SKINNY_MAX_M + 1  # rows from which the tiled kernel is used (bench override)

@@ -84,6 +84,26 @@ def test_launch_codes_of_few_rows_keep_their_own_size():
         G._TUNE.update(saved)
 
 
+def test_a_launch_code_without_rows_holds_for_all_of_its_tile():
+    """set_tune(key, code), as a program sets a code of its own, is what every size of the tile runs on, also where the
+    tuner has recorded sizes before; other shapes keep theirs."""
+    w, other = torch.zeros(16, 8, 16, 32), torch.zeros(8, 8, 16, 32)
+    saved = dict(G._TUNE)
+    try:
+        G._TUNE.clear()
+        for v in (w, other):
+            for M in (1, 2, 4, 8, 16, 48):
+                G.set_tune(G.tune_key(v, M, G.EPI_RESID, False), M, M)
+        G.set_tune(G.tune_key(w, 1, G.EPI_RESID, False), 77)
+        assert [G._code(w, M, G.EPI_RESID, False, 0) for M in (1, 2, 3, 8, 9, 16, 48)] == [77] * 6 + [48]
+        assert [G._code(other, M, G.EPI_RESID, False, 0) for M in (1, 2, 3, 8, 9, 16)] == [1, 2, 4, 8, 16, 16]
+        G.set_tune(G.tune_key(w, 2, G.EPI_RESID, False), 5, 2)
+        assert [G._code(w, M, G.EPI_RESID, False, 0) for M in (1, 2, 3)] == [5, 5, 5]
+    finally:
+        G._TUNE.clear()
+        G._TUNE.update(saved)
+
+
 @pytest.mark.parametrize("nq,nkv", [(32, 32), (32, 16), (32, 8), (64, 8), (4, 1), (24, 8)])
 def test_query_tiles_by_rows(nq, nkv):
     """v2 tiles of 128 query rows from 128 rows on, of 256 from 512 workgroups on (8 heads per kv head and models with a
