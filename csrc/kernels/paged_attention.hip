@@ -80,7 +80,8 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
   for (int t = 0; t < PPW; ++t) {
     const int nv = min(ctx - (p0 + t * NW) * PAGE, PAGE);  // keys of the page inside the context
     if (nv <= 0) break;                                    // wave-uniform
-    // rows past the context are not read (what they hold may be anything): the last valid row stands in
+    // rows past the context are not read (what they hold may be anything): the last valid row stands in, as a key struck
+    // out below, as a value set to zero (its own weight is its key's: 0 * inf would be nan)
     const size_t base = ((size_t)page[t] * Hkv + h) * PAGE * HD;
     bf16x8 kr[4][4], vr[4][4];
 #pragma unroll
@@ -120,6 +121,13 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
         ls += st[b][j];
       }
     l = fmaf(l, alpha, ls);
+    if (nv < PAGE) {  // wave-uniform
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (16 * b + 4 * qd + j >= nv) vr[b][j] = bf16x8{};
+    }
     if (t > 0) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {

@@ -357,6 +357,33 @@ def _paged_attention_case(G, ctxs):
     assert _rel(out.cpu(), ref) < 1e-2
 
 
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+@pytest.mark.parametrize("max_ctx", [256, 900, 1100])     # one chunk, chunks of 256 keys, of 1024
+def test_paged_attention_keeps_an_infinite_value(G, max_ctx):
+    """The last token's value is infinite in one number: the rows that see it are infinite there, of the value's sign,
+    and elsewhere what they were, wherever in its page the context ends."""
+    R, Hkv = (64, 8) if max_ctx == 1100 else (7, 3)
+    g = torch.Generator().manual_seed(G + max_ctx)
+    k, v = _make_cache(1 + 18 * R, Hkv, seed=G)
+    ctx = torch.randint(1, max_ctx + 1, (R,), generator=g).int()
+    ctx[:7] = torch.tensor([max_ctx, 1, 2, 63, 64, 65, 130])
+    npg = (max_ctx + 63) // 64
+    bt = (torch.randperm(18 * R, generator=g)[:npg * R] + 1).view(R, npg).to(torch.int32)
+    Hq = Hkv * G
+    q = torch.randn(R, Hq * 128, generator=g).to(torch.bfloat16)
+    run = lambda: ops.paged_attention(q.to(DEV), k.to(DEV), v.to(DEV), bt.to(DEV), None, ctx.to(DEV), Hq, Hkv,
+                                      max_ctx).float().cpu().view(R, Hkv, G, 128)
+    want = run()
+    sign = torch.where(torch.arange(R) % 2 == 0, 1.0, -1.0)
+    for r in range(R):
+        last = int(ctx[r]) - 1
+        v[bt[r, last // 64].long(), :, last % 64, 5] = sign[r] * float("inf")
+    got = run()
+    assert torch.equal(got[..., 5], (sign * float("inf"))[:, None, None].expand(R, Hkv, G))
+    got[..., 5] = want[..., 5]
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("R,Hkv,G,max_ctx", [(64, 8, 2, 1024), (43, 8, 1, 1100), (8, 8, 4, 9000), (2, 1, 8, 2305),
                                              (3, 3, 4, 2048), (17, 8, 4, 256)])
 def test_paged_attention_chunks(R, Hkv, G, max_ctx):
