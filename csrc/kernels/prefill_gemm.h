@@ -1157,6 +1157,14 @@ static int pick_tile(int M, int N, int K, int epi) {
     return wide * 8 > cus && K >= 6144 && K >= (wide * 4 > cus ? 2 : 4) * 2048 && wide <= cus ? 2 : 3;
   }
   if (N >= 16384 && M > 128 && M <= 192) return 7;   // one row of tiles, 192 x 128: SwiGLU 28672 x 4096 62 us, 128 x 128 81
+  // A residual product with a short K that gives 160 tiles of 256 x 256 and more waits for its residual and its first and last
+  // stages: pairs of workgroups per CU hide that, but where the larger tiles' last round fills the CUs and K gives them time.
+  // us, pairs / 128 x 256 / phased 256 x 256: 8192 x 1024, 2048 rows 59 / 68 / 62, 8192 x 3072, 2048 rows 115 / 117 / 110,
+  // 1500 rows 93 / 106 / 104, 6144 x 2048, 4096 rows 124 / 131 / 160
+  if (resid && K <= 3072 && N % 256 == 0 && tiles(256, 256) >= 160) {
+    const long last = tiles(256, 256) % cus;
+    return K >= 2560 && (last == 0 || last * 6 > cus * 5) ? 1 : 6;
+  }
   if (N % 256 == 0 && !(resid && K <= 3072)) {
     // More than a round of 128 x 128: the tile whose rounds of the CUs take the shortest time.  Relative times of a round,
     // from SwiGLU of 16384 to 36864 columns and K = 2048 and 4096 (us at 4096, phased 256 x 256 / 192 x 256 / 128 x 256 /

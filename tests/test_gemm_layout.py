@@ -118,3 +118,13 @@ def test_query_tiles_by_rows(nq, nkv):
         want = 16 if G == 3 else 256 // G if wide else 128 // G if G < 8 and rows >= 128 else 16
         assert A.flash_tile(nq, nkv, rows) == want
         assert A.flash_tile(nq, nkv, rows, routed=True) == (256 // G if G != 3 and many else 16)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    # fewer than 160 tiles of 256 x 256: pairs up to 512 of 128 x 128, 128 x 256 beyond; pairs again ..
+    (1024, 8192, 1024, 6), (1536, 6144, 1024, 2), (1280, 8192, 1024, 6), (2048, 8192, 1024, 6), (4096, 6144, 2048, 6), (2560, 4096, 3072, 6),
+    # .. phased where K is long enough and its last round fills five of six CUs
+    (2048, 8192, 2560, 1), (2048, 8192, 2496, 6), (1500, 8192, 3072, 6), (2800, 5120, 2560, 1), (4096, 6144, 3072, 6),
+    (2048, 8192, 3136, 1)])
+def test_tiles_of_residual_products_with_a_short_k(M, N, K, tile):
+    assert _lib.lib().p2p_prefill_tile(M, N, K, G.EPI_RESID) == tile
