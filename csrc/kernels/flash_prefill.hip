@@ -34,13 +34,13 @@ struct Tile {
   int row0, n, seq, pos0;
 };
 
-template <int G>
+template <int G, int NST>   // stages
 __global__ __launch_bounds__(64 * G) void flash_prefill_kernel(
     const bf16* __restrict__ q, int ldq, const bf16* __restrict__ kc,
     const bf16* __restrict__ vc, const int* __restrict__ bt, int bt_stride,
     const Tile* __restrict__ tiles, int n_tiles, int Hkv, float scale_log2,
     bf16* __restrict__ out, int ldo) {
-  constexpr int NST = 3, TE = KT * HD;                      // stages; numbers of a tile's K (V)
+  constexpr int TE = KT * HD, AHEAD = NST - 1;              // numbers of a tile's K (V); tiles copied ahead
   __shared__ __attribute__((aligned(16))) bf16 lds[NST * 2 * TE];   // K, V of every stage
 
   const int nb = n_tiles * Hkv;
@@ -76,8 +76,8 @@ __global__ __launch_bounds__(64 * G) void flash_prefill_kernel(
   };
   auto page_of = [&](int kt) { return btr[min(kt, n_kt - 1) * KT / PAGE]; };
   copy(0, page_of(0), 0);
-  if (n_kt > 1) copy(1, page_of(1), 1);
-  int p2 = page_of(2);
+  if (AHEAD > 1 && n_kt > 1) copy(1, page_of(1), 1);
+  int pa = page_of(AHEAD);
 
   // Q^T B-operand fragments: token col, d = 32s + 8g + j
   const int tok = col < T.n ? col : T.n - 1;
@@ -99,19 +99,19 @@ __global__ __launch_bounds__(64 * G) void flash_prefill_kernel(
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) s16x4* lds4_t;
   const int vrow = 4 * g + (col >> 2), vx = 2 * (vrow & 7);       // (16 rows further: the same permutation)
-  int st = 0, st2 = 2;                                       // stages of tile kt and kt + 2
+  int st = 0, sa = AHEAD;                                    // stages of tile kt and kt + AHEAD
   for (int kt = 0; kt < n_kt; ++kt) {
-    // this wave's copies of the tile have landed, then every wave's; the stage after next is used up
-    // (its own reads of the tile before are done, too)
-    if (kt + 1 < n_kt) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * CP) : "memory");
+    // this wave's copies of the tile have landed, then every wave's; the stage of the tile before is used up
+    // (its own reads of it are done, too)
+    if (AHEAD > 1 && kt + 1 < n_kt) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * CP) : "memory");
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (kt + 2 < n_kt) copy(kt + 2, p2, st2);
-    p2 = page_of(kt + 3);
+    if (kt + AHEAD < n_kt) copy(kt + AHEAD, pa, sa);
+    pa = page_of(kt + AHEAD + 1);
     const bf16* Ks = lds + st * 2 * TE;
     const bf16* Vs = Ks + TE;
-    st2 = st;
+    sa = st;
     st = st == NST - 1 ? 0 : st + 1;
 
     // S^T = K Q^T : two 16-key row tiles
@@ -195,7 +195,17 @@ int launch(const bf16* q, int ldq, const bf16* kc, const bf16* vc, const int* bt
            const Tile* tiles, int n_tiles, int Hkv, float scale, bf16* out, int ldo,
            hipStream_t st) {
   const float sl2 = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL(flash_prefill_kernel<G>, dim3(n_tiles * Hkv), dim3(64 * G), 0, st, q, ldq,
+  // Three stages are 48 KB: three workgroups to a CU.  Where those are one or two waves each and there are more of them, two
+  // stages hide as much by the other two workgroups that then fit: 32 heads on 32, 32 prompts of 8 on 900 earlier tokens,
+  // 1024 workgroups, 99 us with three, 82 with two; 32 on 16, 20 prompts of 44, 960 workgroups, 9.0 and 6.6.
+  if constexpr (G <= 2) {
+    if ((long)n_tiles * Hkv > 768) {
+      hipLaunchKernelGGL((flash_prefill_kernel<G, 2>), dim3(n_tiles * Hkv), dim3(64 * G), 0, st, q, ldq,
+                         kc, vc, bt, bt_stride, tiles, n_tiles, Hkv, sl2, out, ldo);
+      P2P_CHECK_LAUNCH();
+    }
+  }
+  hipLaunchKernelGGL((flash_prefill_kernel<G, 3>), dim3(n_tiles * Hkv), dim3(64 * G), 0, st, q, ldq,
                      kc, vc, bt, bt_stride, tiles, n_tiles, Hkv, sl2, out, ldo);
   P2P_CHECK_LAUNCH();
 }

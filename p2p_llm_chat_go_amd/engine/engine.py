@@ -286,7 +286,8 @@ class Engine:
             greedy = all_logits is None and not sampled
             tiles_h = qtile = None
             if self.flash_prefill_min and R >= self.flash_prefill_min:
-                qtile = ops.flash_tile(self.model.nq, self.model.nkv, R, self.cfg.is_moe)
+                qtile = ops.flash_tile(self.model.nq, self.model.nkv, R, self.cfg.is_moe,
+                                       chunk[-1][0] - chunk[0][0] + 1, int(pos.max()) + 1)
                 tiles_h = ops.prefill_tiles(seq.tolist(), pos.tolist(), qtile)
             # every host-built input of the chunk (block tables, row metadata, output rows,
             # flash tiles, result scatter) in ONE host->device copy: each separate copy of

@@ -315,7 +315,8 @@ class PrefillGraph:
         self.n_out = n_seq
         self.greedy = greedy
         routed = getattr(getattr(model, "cfg", None), "is_moe", False)
-        self.qtile = ops.flash_tile(model.nq, model.nkv, rows, routed)
+        # (the contexts of a bucket reach about three quarters of it)
+        self.qtile = ops.flash_tile(model.nq, model.nkv, rows, routed, n_seq, max_ctx * 3 // 4)
         # tiles never straddle sequences: <= rows / qtile + one partial tile per sequence
         # (the dummy sequence included) + one per wrap of the dummy rows' positions
         self.max_tiles = -(-rows // self.qtile) + n_seq + 1 + rows // (max_pages * PAGE) + 1

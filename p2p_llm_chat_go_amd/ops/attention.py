@@ -287,12 +287,20 @@ FLASH_V2_MIN_BLOCKS = 128
 FLASH_V2_WIDE_BLOCKS = 512
 
 
-def flash_tile(n_heads: int, n_kv: int, rows: int | None = None, routed: bool = False) -> int:
+def flash_tile(n_heads: int, n_kv: int, rows: int | None = None, routed: bool = False, seqs: int = 1,
+               ctx: int | None = None) -> int:
     """Tokens per query tile: the widest that v2 takes (256 / (Hq/Hkv)), or for a prefill chunk of ``rows`` tokens v2's
-    128 or 256 query rows (8 heads per kv head: 256) where they pay, else v1's 16 tokens.  routed: the model has a router,
-    whose choice between two nearly equal experts turns on the last bits of its input and moves a row's logits by 10 %
-    and more: it keeps v1 up to FLASH_V2_MIN_BLOCKS (700 rows 29 against 21 us of a layer's 900), so that
-    prompts are routed as they always were."""
+    128 or 256 query rows (8 heads per kv head: 256) where they pay, else v1's 16 tokens.
+
+    seqs, ctx: sequences that share the rows, and the longest context (None: unknown, taken as long).  A tile of 128 query
+    rows stages the keys for 8 wavefronts; with few keys, or few of its rows filled, the 16-token tiles end sooner (32
+    heads on 8, us, 16 tokens -> 128 rows: 20 prompts of 44 tokens 6.9 -> 9.7, 8 of 33 4.9 -> 6.8, 64 of 8 on 200 earlier
+    tokens 14.2 -> 16.3; but 32 heads on 32, 8 prompts of 128 on 128 earlier, 27 -> 14).  So they stay for contexts up to 192
+    while workgroups x context is 65536 at most, and for prompts of at most 16 tokens from 384 workgroups on.
+
+    routed: the model has a router.  Its choice between two nearly equal experts turns on the last bits of its input, and a
+    row that goes to the other one moves its logits by 10 % and more; such a model keeps v1 up to FLASH_V2_MIN_BLOCKS (700
+    rows 29 against 21 us of a layer's 900)."""
     G = n_heads // n_kv
     if FLASH_V2 and G in (1, 2, 4, 8):
         if rows is None:
@@ -301,6 +309,10 @@ def flash_tile(n_heads: int, n_kv: int, rows: int | None = None, routed: bool = 
         if blocks >= (FLASH_V2_MIN_BLOCKS if G == 8 or routed else FLASH_V2_WIDE_BLOCKS):
             return 256 // G
         if G < 8 and not routed and rows >= FLASH_V2_MIN_ROWS:
+            each = -(-rows // seqs)
+            small = seqs * -(-each // QTILE) * n_kv     # workgroups of 16-token tiles
+            if ctx is not None and ((ctx <= 192 and small * ctx <= 65536) or (each <= QTILE and small >= 384)):
+                return QTILE
             return 128 // G
     return QTILE
 

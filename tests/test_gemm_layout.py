@@ -120,6 +120,57 @@ def test_query_tiles_by_rows(nq, nkv):
         assert A.flash_tile(nq, nkv, rows, routed=True) == (256 // G if G != 3 and many else 16)
 
 
+@pytest.mark.parametrize("nq,nkv,rows,dense,routed", [
+    # query heads, key/value heads, rows of a chunk -> tokens per query tile, of a model without and with a router
+    (32, 8, 1, 16, 16), (32, 8, 127, 16, 16), (32, 8, 128, 32, 16), (32, 8, 700, 32, 16), (32, 8, 960, 32, 16),
+    (32, 8, 961, 32, 64), (32, 8, 4032, 32, 64), (32, 8, 4033, 64, 64), (32, 8, 8192, 64, 64),
+    (32, 32, 127, 16, 16), (32, 32, 128, 128, 16), (32, 32, 768, 128, 16), (32, 32, 769, 128, 256), (32, 32, 3840, 128, 256),
+    (32, 32, 3841, 256, 256), (32, 16, 128, 64, 16), (32, 16, 896, 64, 16), (32, 16, 897, 64, 128), (32, 16, 3969, 128, 128),
+    (64, 8, 128, 16, 16), (64, 8, 480, 16, 16), (64, 8, 481, 32, 32), (64, 8, 4096, 32, 32), (4, 1, 4096, 32, 16),
+    (24, 8, 100, 16, 16), (24, 8, 4096, 16, 16)])
+def test_query_tiles_that_kernels_take(nq, nkv, rows, dense, routed):
+    """The tile of a prompt's attention on both sides of every line, and what its kernels need: 256 rows of (token, query
+    head) at most, 1, 2, 4 or 8 query heads per key/value head above 16 tokens, and room in a captured chunk."""
+    from types import SimpleNamespace
+
+    from p2p_llm_chat_go_amd import ops
+    from p2p_llm_chat_go_amd.engine.graph import PrefillGraph
+    from p2p_llm_chat_go_amd.ops import attention as A
+
+    G = nq // nkv
+    for want, r in ((dense, False), (routed, True)):
+        tile = A.flash_tile(nq, nkv, rows, r)
+        assert tile == want
+        assert tile == A.QTILE or (G in (1, 2, 4, 8) and A.QTILE < tile <= ops.kernel_lib().p2p_flash_prefill_tile(nq, nkv)
+                                   and tile * G <= 256)
+        # a captured chunk of these rows, filled or with dummy rows behind its sequences
+        model = SimpleNamespace(device=torch.device("cpu"), nq=nq, nkv=nkv, tp=1, cfg=SimpleNamespace(is_moe=r))
+        pages = -(-rows // A.PAGE)
+        g = PrefillGraph(model, None, rows, 3, pages, pages * A.PAGE)
+        for lens in ([rows], [max(1, rows // 3), rows // 2], [1, 1, 1]):
+            chunk = [(b, t, 5) for b, n in enumerate(lens) for t in range(n)][:rows]
+            at, n = g.offsets["tiles"]
+            tiles = g.host_meta(chunk, [list(range(1, pages + 1))] * 3, [0])[at:at + n].view(-1, 4)
+            assert g.qtile == A.flash_tile(nq, nkv, rows, r, 3, pages * A.PAGE * 3 // 4)
+            assert int(tiles[:, 1].max()) <= g.qtile and int(tiles[:, 1].sum()) == rows
+
+
+@pytest.mark.parametrize("nq,nkv,seqs,each,past,tile", [
+    # 16-token tiles: short contexts while workgroups x context is 65536 at most (here 512 x 128, 512 x 144) ..
+    (32, 8, 20, 44, 0, 16), (32, 8, 8, 33, 0, 16), (32, 8, 1, 192, 0, 16), (32, 8, 1, 193, 0, 32), (32, 32, 2, 128, 0, 16),
+    (32, 32, 2, 128, 16, 128), (32, 32, 8, 128, 128, 128),
+    # .. and prompts of a tile from 384 workgroups on
+    (32, 8, 48, 16, 4000, 16), (32, 8, 47, 16, 4000, 32), (32, 8, 48, 17, 4000, 32), (32, 8, 128, 1, 900, 16),
+    # as before: many rows, 8 heads to one
+    (32, 8, 256, 17, 0, 64), (64, 8, 60, 8, 0, 16), (64, 8, 61, 8, 0, 32)])
+def test_query_tiles_of_short_prompts(nq, nkv, seqs, each, past, tile):
+    """The tile by the sequences of a chunk and its longest context; without them as for one long sequence."""
+    from p2p_llm_chat_go_amd.ops import attention as A
+
+    assert A.flash_tile(nq, nkv, seqs * each, False, seqs, past + each) == tile
+    assert A.flash_tile(nq, nkv, seqs * each, True, seqs, past + each) == A.flash_tile(nq, nkv, seqs * each, True)
+
+
 @pytest.mark.parametrize("M,N,K,tile", [
     # fewer than 160 tiles of 256 x 256: pairs up to 512 of 128 x 128, 128 x 256 beyond; pairs again ..
     (1024, 8192, 1024, 6), (1536, 6144, 1024, 2), (1280, 8192, 1024, 6), (2048, 8192, 1024, 6), (4096, 6144, 2048, 6), (2560, 4096, 3072, 6),

@@ -630,6 +630,26 @@ def test_flash_prefill_widths(G, width, lens):
 
 # ------------------------------------------------------------ rope + cache
 def test_rope_cache():
+@pytest.mark.parametrize("G,Hkv,seqs", [(1, 16, 48), (1, 16, 49), (2, 8, 96), (2, 8, 97)])
+def test_flash_prefill_of_many_workgroups(G, Hkv, seqs):
+    """768 workgroups of the 16-token kernel and more, with which it keeps fewer tiles of keys in flight: contexts of one to
+    five tiles of 32 keys, ends in every part of one.  P is rounded to bf16 and so is the result: twice 2^-9."""
+    g = torch.Generator().manual_seed(G + seqs)
+    lens = [(b * 29 % 150, 1 + b % 11) for b in range(seqs)]
+    Hq, npg = Hkv * G, 3
+    k, v = _make_cache(1 + seqs * npg, Hkv, seed=G)
+    bt = (torch.randperm(seqs * npg, generator=g) + 1).view(seqs, npg).to(torch.int32)
+    seq = [b for b, (_, n) in enumerate(lens) for _ in range(n)]
+    pos = [s + i for s, n in lens for i in range(n)]
+    q = torch.randn(len(seq), Hq * 128, generator=g).to(torch.bfloat16)
+    ref = A.paged_attention_ref(q, k, v, bt, torch.tensor(seq, dtype=torch.int32), torch.tensor(pos, dtype=torch.int32) + 1,
+                                Hq, Hkv, 1 / math.sqrt(128), torch.empty(len(seq), Hq * 128))
+    tiles = ops.prefill_tiles(seq, pos, A.QTILE)
+    assert (len(tiles) * Hkv > 768) == (seqs % 2 == 1)
+    out = ops.flash_prefill(q.to(DEV), k.to(DEV), v.to(DEV), bt.to(DEV), tiles.to(DEV), Hq, Hkv, qtile=A.QTILE)
+    assert float((out.float().cpu() - ref).norm() / ref.norm()) < 2 ** -8
+
+
     from p2p_llm_chat_go_amd.models.config import LLAMA31_8B, rope_table
 
     Hq, Hkv, T = 8, 2, 37
