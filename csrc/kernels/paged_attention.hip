@@ -43,6 +43,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
     const int* __restrict__ ctx_lens, int Hkv, float scale, int n_chunks, bf16* __restrict__ out,
     int ldo, float* __restrict__ part_o, float* __restrict__ part_ml) {
   constexpr int HG = (G + 3) / 4;  // groups of 4 heads
+  constexpr bool ONE = G == 1;
   const int h = blockIdx.x, r = blockIdx.y, c = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int n = lane & 15, qd = lane >> 4;
@@ -60,8 +61,8 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const bf16x2 x = qp[16 * s + i];
-        qf[s][2 * i] = n < G ? x[0] : (bf16)0.f;
-        qf[s][2 * i + 1] = n < G ? x[1] : (bf16)0.f;
+        qf[s][2 * i] = ONE || n < G ? x[0] : (bf16)0.f;
+        qf[s][2 * i + 1] = ONE || n < G ? x[1] : (bf16)0.f;
       }
   }
   const int p0 = c * NW * PPW + w;  // this wave's pages: p0, p0 + NW, ...
@@ -143,6 +144,10 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float v = (float)vr[b][j][e];
+          if constexpr (ONE) {
+            acc[0][e][0] = fmaf(st[b][j], v, acc[0][e][0]);
+            continue;
+          }
           acc[0][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(st[b][j], v, acc[0][e], 2, 0, 0);
           if constexpr (HG > 1) acc[1][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(st[b][j], v, acc[1][e], 2, 1, 0);
         }
@@ -478,8 +483,10 @@ int launch_attn(const void* q, int ldq, const void* kc, const void* vc, const in
                        ctx, Hkv, scale, (bf16*)out, ldo);
     return (int)hipGetLastError();
   }
-  // 1024-key chunks where they give 512 workgroups and more (measured at the kernel)
-  if (max_ctx >= 1024 && (long long)R * Hkv * ((max_ctx + 1023) / 1024) >= 512)
+  // 1024-key chunks where they give 512 workgroups and more (measured at the kernel); up to 4 heads 640: 512 end as one
+  // round of which contexts below their bucket leave CUs idle (8 kv heads of 4, 8 rows of 5120 keys in a bucket of 8192:
+  // 31.3 us with 256-key chunks, 39.5 with these; one head, 8 rows 30.0 / 35.5; 8 heads gain there: 1.5 times slower)
+  if (max_ctx >= 1024 && (long long)R * Hkv * ((max_ctx + 1023) / 1024) >= (G == 8 ? 512 : 640))
     return launch_pages<G, 8, 2>(q, ldq, kc, vc, bt, bt_stride, row_bt, ctx, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, st);
   return launch_pages<G, 4, 1>(q, ldq, kc, vc, bt, bt_stride, row_bt, ctx, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, st);
 }
