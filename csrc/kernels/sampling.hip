@@ -282,7 +282,12 @@ __global__ __launch_bounds__(THREADS) void sample_kernel(
         const unsigned u = s_ck[min(c, nc - 1)];
         const int i = s_ci[min(c, nc - 1)];
         int n = 0;
-        for (int q = tid & 3; q < nc; q += 4) n += s_ck[q] > u || (s_ck[q] == u && s_ci[q] < i);
+#pragma unroll 8
+        for (int q = tid & 3; q < nc; q += 4) {  // both reads of every turn go out ahead of their comparison
+          const unsigned uq = s_ck[q];
+          const int iq = s_ci[q];
+          n += (uq > u) | ((uq == u) & (iq < i));
+        }
         n += __shfl_xor(n, 1, 64);
         n += __shfl_xor(n, 2, 64);
         if ((tid & 3) == 0 && c < nc && n < k) { s_tmk[n] = u; s_ci[RANKED + n] = i; }
@@ -295,9 +300,11 @@ __global__ __launch_bounds__(THREADS) void sample_kernel(
         const float v = key_float(s_tmk[cc]);
         const unsigned u = ord_key(v + 0.f);
         int n = 0;
+#pragma unroll 8
         for (int q = tid & 3; q < k; q += 4) {
           const unsigned uq = ord_key(key_float(s_tmk[q]) + 0.f);
-          n += uq > u || (uq == u && s_ci[RANKED + q] < i);
+          const int iq = s_ci[RANKED + q];
+          n += (uq > u) | ((uq == u) & (iq < i));
         }
         n += __shfl_xor(n, 1, 64);
         n += __shfl_xor(n, 2, 64);
@@ -549,6 +556,10 @@ P2P_API int p2p_sample_groups(int V) {
 static int row_groups(const float* logits, int ld, int B, int V, const float* temp, unsigned* ws, int* ng,
                       hipStream_t st) {
   *ng = ws ? p2p_sample_groups(V) : 0;
+  // Below 192 groups any k = 128 finds logits in most of them, and the launch of kernel a is not won back (16384 logits,
+  // k = 128, one workgroup per row / two launches: 18.4 / 26.4 us); nor is it for many rows of a small vocabulary, which
+  // fill the CUs by themselves (32000 logits, 256 rows, k = 128 23.6 / 28.2, greedy 8.6 / 11.9).
+  if (*ng < 192 || (B > 64 && V < 49152)) *ng = 0;
   if (*ng == 0) return 0;
   const int wgs = (*ng + 4 * GPW - 1) / (4 * GPW);
   for (int r = 0; r < B; r += 65535)  // grid.y

@@ -1399,6 +1399,30 @@ def test_sample_kernel_matches_reference(V):
     assert agree >= B - 2, (agree, B)
 
 
+@pytest.mark.parametrize("B,V", [(3, 16384), (3, 24448), (3, 24449), (64, 32000), (65, 32000), (65, 49151), (65, 49152)])
+def test_sampling_of_few_groups_and_many_rows(B, V):
+    """Rows with a workspace, on both sides of where the group maxima are formed: the tokens of one workgroup per row."""
+    from p2p_llm_chat_go_amd.ops import _lib
+
+    L = _lib.lib()
+    torch.manual_seed(B + V)
+    lg = (torch.randn(B, V) * 3).to(DEV)
+    lg[1] = torch.round(lg[1])
+    temp = torch.where(torch.arange(B) % 3 == 2, 0.0, 0.8).to(DEV)
+    topk = torch.tensor([40, 0, 1, 128] * B, dtype=torch.int32)[:B].to(DEV)
+    topp, seeds = torch.full((B,), 0.9, device=DEV), torch.arange(B, dtype=torch.int64, device=DEV) * 7919 + 1
+    pos = torch.arange(B, dtype=torch.int32, device=DEV)
+    ws = torch.empty(B * L.p2p_sample_groups(V), dtype=torch.int32, device=DEV)
+    got = []
+    for w in (ws.data_ptr(), None):
+        ids = torch.full((B,), -1, dtype=torch.int32, device=DEV)
+        assert L.p2p_sample(lg.data_ptr(), V, B, V, temp.data_ptr(), topk.data_ptr(), topp.data_ptr(), seeds.data_ptr(),
+                            pos.data_ptr(), ids.data_ptr(), w, torch.cuda.current_stream().cuda_stream) == 0
+        got.append(ids.cpu())
+    assert torch.equal(*got) and bool((got[0] >= 0).all())
+    assert torch.equal(got[0][2::3].long(), lg[2::3].argmax(1).cpu())
+
+
 @pytest.mark.parametrize("V,ld", [(16256, 16256), (16257, 16260), (32000, 32001), (128256, 128256), (262144, 262144),
                                   (262145, 262145)])
 def test_sampling_by_groups_is_the_whole_row(V, ld):
