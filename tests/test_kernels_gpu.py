@@ -630,8 +630,6 @@ def test_flash_prefill_widths(G, width, lens):
     assert float((out.float().cpu() - ref).norm() / ref.norm()) < 2 ** -8
 
 
-# ------------------------------------------------------------ rope + cache
-def test_rope_cache():
 @pytest.mark.parametrize("G,Hkv,seqs", [(1, 16, 48), (1, 16, 49), (2, 8, 96), (2, 8, 97)])
 def test_flash_prefill_of_many_workgroups(G, Hkv, seqs):
     """768 workgroups of the 16-token kernel and more, with which it keeps fewer tiles of keys in flight: contexts of one to
@@ -652,6 +650,8 @@ def test_flash_prefill_of_many_workgroups(G, Hkv, seqs):
     assert float((out.float().cpu() - ref).norm() / ref.norm()) < 2 ** -8
 
 
+# ------------------------------------------------------------ rope + cache
+def test_rope_cache():
     from p2p_llm_chat_go_amd.models.config import LLAMA31_8B, rope_table
 
     Hq, Hkv, T = 8, 2, 37
