@@ -8,10 +8,11 @@
 //                                         are one k index of four products
 //   O[16 pairs x V]        += P . V       a lane's four weights are the k indices of four products, its
 //                                         16 bytes of a value row the column of four output tiles
-// so neither operand goes through LDS.  Up to 128 numbers per key and value the four wavefronts take every fourth tile each,
-// with a softmax of its own, and are merged in LDS at the end (attn_f32_k); longer ones they take together, a quarter of the
-// channels each (attn_f32_wide_k): a tile of 512 numbers is 8192 cycles of products, which one wavefront would walk through
-// alone behind its tile's loads.  The next tile's keys and this one's values are asked for ahead of the products.
+// so neither operand goes through LDS.  The four wavefronts take every fourth tile each, with a softmax of its own, and are
+// merged in LDS at the end (attn_f32_k), or take longer keys and values together, a quarter of the channels each
+// (attn_f32_wide_k): a tile of 512 numbers is 8192 cycles of products, which one wavefront would walk through alone
+// behind its tile's loads.  Where registers hold them, the next tile's keys and this one's values are asked for ahead of the
+// products.  form_of() has the choice.
 //
 // Bound by a tile's loads (a key load touches 16 half lines) and its products, which overlap only across the two workgroups
 // of a CU.  8 heads, us, a wavefront per tile without loads ahead / now: latents of 512, prompts of 389 and 117 rows 101 / 64
@@ -189,10 +190,11 @@ __device__ __forceinline__ void pairs_alone(const AttnF32Args& a, const Work& w,
   }
 }
 
-// Keys and values of up to 128 numbers: a wavefront takes every fourth tile of 16 keys on its own
-// (loads that the compiler can count: no branch around one, or it waits for younger ones too)
+// A wavefront takes every fourth tile of 16 keys on its own.  NK > 0, keys and values of up to 128 numbers: the next tile's
+// keys and this one's values are asked for ahead (loads that the compiler can count: no branch around one, or it waits for
+// younger ones too); 0: as they are used, with registers for more wavefronts or longer rows
 template <int NB, int NK>  // value channels in blocks of 64, key channels in steps of 16
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, NK ? 2 : 1)
 attn_f32_k(AttnF32Args a) {
   constexpr int VP = NB * 64;
   extern __shared__ __align__(16) float smem[];   // queries [16][LDQ], at the end sums [16][VP]
@@ -201,7 +203,7 @@ attn_f32_k(AttnF32Args a) {
   const int tid = threadIdx.x, lane = tid & 63, n16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const Work w = find_work(a);
-  const int D = a.D, V = a.V, DP = NK * 16, LDQ = DP + 4;
+  const int D = a.D, V = a.V, DP = NK ? NK * 16 : (D + 15) & ~15, LDQ = DP + 4;
   const int koff = w.gk * D, voff = a.vbase + w.g * V;
   const Pair pr = find_pair(a, w, n16);
   for (int i = tid; i < 16 * (DP / 4); i += 256) {
@@ -219,38 +221,48 @@ attn_f32_k(AttnF32Args a) {
 
   // The next tile's keys are asked for when this one's are used up, a tile's values before its scores: what a wavefront
   // waits for came out behind the products of the one or the other
-  f32x4 kv[NK];
+  f32x4 kv[NK ? NK : 1];
   auto ask = [&](const float* row) {   // beyond D: the key's start, which meets zeros
 #pragma unroll
     for (int i = 0; i < NK; i++) kv[i] = *(const f32x4*)(row + koff + (i * 16 + quad * 4 < D ? i * 16 + quad * 4 : 0));
   };
-  const float* krow = key_row(a, w, (w.t_lo + wave) * 16 + n16);
-  ask(krow);
+  const float* krow = NK || w.t_lo + wave < w.t_hi ? key_row(a, w, (w.t_lo + wave) * 16 + n16) : nullptr;
+  if (NK) ask(krow);
   for (int ti = w.t_lo + wave; ti < w.t_hi; ti += 4) {
     const int u0 = ti * 16;
-    const float* nxt = key_row(a, w, u0 + 64 + n16);
+    const float* nxt = NK || ti + 4 < w.t_hi ? key_row(a, w, u0 + 64 + n16) : nullptr;
     // the values of keys quad * 4 + e
+    const float* vrow[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) vrow[e] = (const float*)__shfl((unsigned long long)krow, quad * 4 + e, 64) + voff;
+    auto value = [&](int e, int b) {   // columns beyond V are not written
+      const int c = b * 64 + n16 * 4;
+      return *(const f32x4*)(vrow[e] + (c < V ? c : 0));
+    };
     f32x4 vv[4][NB];
+    if constexpr (NK > 0) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float* vrow = (const float*)__shfl((unsigned long long)krow, quad * 4 + e, 64) + voff;
+      for (int e = 0; e < 4; e++)
 #pragma unroll
-      for (int b = 0; b < NB; b++) {   // columns beyond V are not written
-        const int c = b * 64 + n16 * 4;
-        vv[e][b] = *(const f32x4*)(vrow + (c < V ? c : 0));
-      }
+        for (int b = 0; b < NB; b++) vv[e][b] = value(e, b);
     }
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
     const float* qp = smem + n16 * LDQ + quad * 4;
+    auto product = [&](const f32x4& k, const f32x4& q) {
+      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[0], q[0], s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[1], q[1], s1, 0, 0, 0);
+      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[2], q[2], s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[3], q[3], s1, 0, 0, 0);
+    };
+    if constexpr (NK > 0) {
 #pragma unroll
-    for (int i = 0; i < NK; i++) {
-      const f32x4 qv = *(const f32x4*)(qp + i * 16);   // zero beyond D
-      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i][0], qv[0], s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i][1], qv[1], s1, 0, 0, 0);
-      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i][2], qv[2], s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i][3], qv[3], s1, 0, 0, 0);
+      for (int i = 0; i < NK; i++) product(kv[i], *(const f32x4*)(qp + i * 16));   // (queries: zero beyond D)
+      ask(nxt);
+    } else {
+#pragma unroll 8
+      for (int c = 0; c < DP; c += 16)
+        product(*(const f32x4*)(krow + koff + (c + quad * 4 < D ? c + quad * 4 : 0)), *(const f32x4*)(qp + c));
     }
-    ask(nxt);
     float sv[4];
     const float tmax = scores_of(a, w, pr, u0 + quad * 4, s0 + s1, sv);
     weights_of(sv, tmax, m_run, l_part, acc, quad);
@@ -259,8 +271,11 @@ attn_f32_k(AttnF32Args a) {
 #pragma unroll
       for (int b = 0; b < NB; b++)
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+        for (int t = 0; t < 4; t++) {
+          if constexpr (NK == 0)
+            if (t == 0) vv[e][b] = value(e, b);
           acc[b * 4 + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[e], vv[e][b][t], acc[b * 4 + t], 0, 0, 0);
+        }
     krow = nxt;
   }
   // the wavefronts' sums under their common maximum, one after the other; the sink (of the first run) is a fifth
@@ -469,9 +484,26 @@ __global__ void __launch_bounds__(128) attn_f32_merge_k(AttnF32Args a, int VP) {
   }
 }
 
-static int value_blocks(int D, int V) {   // from four on (keys above 128 numbers too) attn_f32_wide_k
-  const int n = D > 128 && V <= 256 ? 4 : (V + 63) / 64;
-  return n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : 8;
+// The kernel of a shape: attn_f32_k without loads ahead, with them, or attn_f32_wide_k.  us, waves / ahead / wide:
+// * up to 128 numbers: ahead.  8 heads of 128 on 2, 400 and 400 rows 29 / 22 / 49, one token at 500 15.3 / 13.3 / 15.6;
+// * longer values: wide while there are few workgroups, which then share a tile's loads and products; with many they hide
+//   each other's waits, and waves that meet at no barrier are ahead.  Latents of 256, 8 heads, a token at 500 18.9 / - / 16.9, 333
+//   rows behind 500 57.8 / - / 54.9 (167 workgroups), 1000 rows 115 / - / 134 (500); of 192, 4 heads, 333 rows 26.6 / - /
+//   24.8 (84), 1000 rows 77 / - / 87 (250); 16 heads on one with keys of 64 and values of 256, 32 tokens at 90 17.5 / - / 15.6
+//   (32), 100 rows behind 500 30 / - / 35 (100), 512 rows 45 / - / 71;
+// * keys above 128 alone: waves.  8 heads of 192 and 128 on 2, 1000 rows 93 / - / 151;
+// * more than 256: wide (what waves would hold does not fit their registers), but for keys alone with many workgroups: 8 heads
+//   of 384 and 128 on 2, one token 12.2 / - / 8.1, 1000 rows 178 / - / 203.
+enum Form { WAVES, AHEAD, WIDE };
+static Form form_of(int D, int V, long groups) {
+  if (D > 256 || V > 256) return V <= 256 && groups >= 128 ? WAVES : WIDE;
+  if (V > 128) return groups < (D > 192 ? 256 : D > 128 ? 128 : 64) ? WIDE : WAVES;
+  return D > 128 ? WAVES : AHEAD;
+}
+// value channels of that kernel in blocks of 64
+static int value_blocks(int V, Form form) {
+  const int n = (V + 63) / 64;
+  return form == WIDE ? n <= 4 ? 4 : 8 : n <= 2 ? n : 4;
 }
 static int head_slots(int HG) {
   int hs = 1;
@@ -480,18 +512,25 @@ static int head_slots(int HG) {
 }
 
 template <int NB>
-static int launch_f32(const AttnF32Args& a, dim3 grid, hipStream_t st) {
-  if constexpr (NB >= 4) {
-    if (a.D <= 256) hipLaunchKernelGGL((attn_f32_wide_k<NB, 4>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((attn_f32_wide_k<NB, 8>), grid, dim3(256), 0, st, a);
-  } else {
-    const int steps = a.D <= 64 ? 4 : 8;
-    const size_t queries = (size_t)16 * (steps * 16 + 4) * 4, sums = (size_t)16 * NB * 64 * 4;
-    const size_t shm = queries > sums ? queries : sums;
-    if (steps == 4) hipLaunchKernelGGL((attn_f32_k<NB, 4>), grid, dim3(256), shm, st, a);
-    else hipLaunchKernelGGL((attn_f32_k<NB, 8>), grid, dim3(256), shm, st, a);
+static void launch_waves(const AttnF32Args& a, bool ahead, dim3 grid, hipStream_t st) {
+  const int steps = !ahead ? (a.D + 15) / 16 : a.D <= 16 ? 1 : a.D <= 32 ? 2 : a.D <= 64 ? 4 : 8;
+  const size_t queries = (size_t)16 * (steps * 16 + 4) * 4, sums = (size_t)16 * NB * 64 * 4;
+  const size_t shm = queries > sums ? queries : sums;
+  if constexpr (NB <= 2) {
+    if (ahead) {
+      if (steps == 1) hipLaunchKernelGGL((attn_f32_k<NB, 1>), grid, dim3(256), shm, st, a);
+      else if (steps == 2) hipLaunchKernelGGL((attn_f32_k<NB, 2>), grid, dim3(256), shm, st, a);
+      else if (steps == 4) hipLaunchKernelGGL((attn_f32_k<NB, 4>), grid, dim3(256), shm, st, a);
+      else hipLaunchKernelGGL((attn_f32_k<NB, 8>), grid, dim3(256), shm, st, a);
+      return;
+    }
   }
-  return (int)hipGetLastError();
+  hipLaunchKernelGGL((attn_f32_k<NB, 0>), grid, dim3(256), shm, st, a);
+}
+template <int NB>
+static void launch_wide(const AttnF32Args& a, dim3 grid, hipStream_t st) {
+  if (a.D <= 256) hipLaunchKernelGGL((attn_f32_wide_k<NB, 4>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((attn_f32_wide_k<NB, 8>), grid, dim3(256), 0, st, a);
 }
 
 extern "C" {
@@ -503,7 +542,8 @@ int p2p_sm_attn_f32_ok(int D, int V) { return D >= 4 && V >= 4 && D % 4 == 0 && 
 long p2p_sm_attn_f32_ws(int U, int H, int G, int D, int V, int splits, int maps) {
   if (splits <= 1 || G < 1 || H % G) return 0;
   const int HG = H / G, HS = head_slots(HG);
-  return (long)U * G * maps * ((HG + HS - 1) / HS) * splits * 16 * (value_blocks(D, V) * 64 + 2);
+  const long groups = (long)U * G * maps * ((HG + HS - 1) / HS) * splits;
+  return groups * 16 * (value_blocks(V, form_of(D, V, groups)) * 64 + 2);
 }
 
 // units: row groups of at most 16 / HS rows, HS the power of two >= min(H / G, 16)
@@ -523,10 +563,14 @@ int p2p_sm_attn_f32(const float* q, long sqh, long sqr, long sqm, const float* p
                          out, soh, sor, som, U, H, G, D, V, page, HS, splits, part, out_scale, cap, r1, r2, gate, ldg,
                          gate_pc, blk, P, keep, maps};
   const dim3 grid(U, G * maps * ((HG + HS - 1) / HS), splits);
-  const int nb = value_blocks(D, V);
-  const int err = nb == 1 ? launch_f32<1>(a, grid, st) : nb == 2 ? launch_f32<2>(a, grid, st)
-                : nb == 4 ? launch_f32<4>(a, grid, st) : launch_f32<8>(a, grid, st);
-  if (err || splits == 1) return err;
+  const Form form = form_of(D, V, (long)grid.x * grid.y * grid.z);
+  const int nb = value_blocks(V, form);
+  if (form == WIDE) nb == 4 ? launch_wide<4>(a, grid, st) : launch_wide<8>(a, grid, st);
+  else if (nb == 4) launch_waves<4>(a, false, grid, st);
+  else if (nb == 2) launch_waves<2>(a, form == AHEAD, grid, st);
+  else launch_waves<1>(a, form == AHEAD, grid, st);
+  if (const int err = (int)hipGetLastError()) return err;
+  if (splits == 1) return 0;
   hipLaunchKernelGGL(attn_f32_merge_k, dim3(grid.x, grid.y, 16), dim3(128), 0, st, a, nb * 64);
   return (int)hipGetLastError();
 }

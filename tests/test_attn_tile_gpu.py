@@ -88,6 +88,15 @@ def test_window_attention_tiles_of_one_narrow_side(step, H, G, D, V, form):
     test_window_attention_tiles(step, H, G, D, V, form, torch.bfloat16)
 
 
+@pytest.mark.parametrize("step", sorted(STEPS))    # few and many workgroups: either side of the lines between the kernels
+@pytest.mark.parametrize("H,G,D,V", [(8, 2, 192, 128), (8, 2, 132, 40), (16, 16, 260, 72), (16, 8, 512, 256), (16, 16, 200, 136),
+                                     (8, 2, 64, 512), (16, 16, 200, 260)])
+@pytest.mark.parametrize("form", ["window", "sink", "blocks"])
+def test_window_attention_of_long_rows(step, H, G, D, V, form):
+    """fp32 keys or values of more than 128 numbers: a wavefront per tile, or all four on it."""
+    test_window_attention_tiles(step, H, G, D, V, form, torch.float32)
+
+
 def test_group_size():
     one = [(i, 1, 5, i) for i in range(8)]
     assert sm.attn_unit_rows(4, one) == 4                     # decoded tokens
