@@ -722,11 +722,17 @@ int p2p_sm_group_route(const void* h, int ldh, const float* wr, int R, int W, in
   SM_DISPATCH_T(f32, hipLaunchKernelGGL((group_route_rows_k<T, NB>), dim3((R + 15) / 16), dim3(1024), many, st, \
                                          (const T*)h, ldh, wr, R, W, E, top, groups, keep, score, corr, gscore, ids, wts, \
                                          cnt, rows, ldr, bias, renorm, wscale))
-  // Up to 32 experts: sixteen rows' logits on the matrix instruction, unless so few rows that one per workgroup is the
-  // shorter chain (8 experts, us, one / sixteen: bf16, 1024 numbers, 100 rows 7.7 / 7.8, 200 9.7 / 7.9, 606 11.9 / 8.0; 2048
-  // numbers, 100 rows 8.4 / 9.8, 200 10.8 / 9.8, 606 17.6 / 10.0; fp32, 2048 numbers, 200 rows 10.8 / 11.5, 256 12.1 / 11.5)
+  // Up to 32 experts: sixteen rows' logits on the matrix instruction, from as many rows on as make one row per workgroup (below)
+  // the longer chain.  A workgroup's products grow with the numbers of a row, in fp32 and above 16 experts (two products per
+  // step) faster than one row's share.  us, one / sixteen: bf16, 8 experts, 1024 numbers, 100 rows 9.0 / 9.3, 200 11.2 / 9.4,
+  // 700 13.5 / 9.6; 2048, 150 rows 11.1 / 11.3, 200 12.2 / 11.3, 2048 rows 19.9 / 12.3; 4096, 200 14.6 / 15.3, 256 15.8 / 15.3;
+  // 32 experts, 2048, 200 13.2 / 16.6, 400 16.5 / 17.0, 700 21.0 / 16.8; fp32, 8 experts, 2048, 200 12.4 / 13.0, 300 14.7 /
+  // 13.0; 4096, 300 17.1 / 18.7, 400 19.6 / 18.7; 32 experts, 2048, 400 16.1 / 18.3, 700 21.0 / 18.5.
+  // The logits' sums have another order then (fp32 both): experts whose scores are as close as fp32 rounding of W products
+  // may be chosen otherwise in a step of so many rows than in a smaller one.
   const int ep = f32 ? 4 : 8;
-  if (R >= 200 && E <= 32 && W % ep == 0 && ldh % ep == 0 && (size_t)h % 16 == 0 && (size_t)wr % 16 == 0) {
+  const int from = max(200, E <= 16 ? f32 ? 90 + W / 12 : 120 + W / 26 : f32 ? 240 + W / 8 : 190 + W / 10);
+  if (R >= from && E <= 32 && W % ep == 0 && ldh % ep == 0 && (size_t)h % 16 == 0 && (size_t)wr % 16 == 0) {
     if (E <= 16) ROUTE_ROWS(1);
     else ROUTE_ROWS(2);
     return (int)hipGetLastError();

@@ -21,7 +21,9 @@ DEV = "cuda:0"
     (200, 72, 33, 2, 1, 1, dict()),
     # many experts: a row per workgroup up to R * 28 = E * W, sixteen from there on
     (300, 100, 128, 8, 8, 3, dict(renorm=True)), (365, 80, 128, 8, 8, 3, dict()), (366, 80, 128, 8, 8, 3, dict()),
-    (1300, 72, 256, 8, 1, 1, dict(score="softmax"))])
+    (1300, 72, 256, 8, 1, 1, dict(score="softmax")),
+    # 17 to 32 experts and long rows from 400 (bf16) and 503 rows (fp32) on
+    (520, 2104, 20, 4, 5, 3, dict(bias=True)), (502, 2104, 20, 4, 5, 3, dict(bias=True))])
 def test_routing_of_many_rows(dt, R, W, E, top, groups, keep, kw):
     g = torch.Generator().manual_seed(2)
     h, wr = torch.randn(R, W, generator=g).to(dt), torch.randn(E, W, generator=g) / W ** 0.5
@@ -42,6 +44,37 @@ def test_routing_of_many_rows(dt, R, W, E, top, groups, keep, kw):
     # every slot is in its expert's list, once
     for e in range(E):
         assert sorted(r2[e, :int(c2[e])].tolist()) == (i2.reshape(-1) == e).nonzero()[:, 0].tolist()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W,E,top,at", [(2048, 8, 2, (200, 260)), (1024, 20, 3, (292, 368)), (72, 5, 1, (200, 200))])
+def test_routing_below_and_above_the_row_threshold(dt, W, E, top, at):
+    """From a number of rows on (at: bf16, fp32) a router's logits are summed in another order: both within fp32 rounding of
+    64 bits, and the same experts wherever no two scores are closer than that."""
+    R = at[dt == torch.float32]
+    g = torch.Generator().manual_seed(W)
+    h, wr = torch.randn(R, W, generator=g).to(dt), torch.randn(E, W, generator=g) / W ** 0.5
+    h[:7] = 0.0
+    h[:7, :E] = 1.0
+    wr[:, :E] = wr[0, :E]                                     # rows 0 .. 6: sums of E products, all experts tied
+    z = h.double() @ wr.double().t()
+    bound = W * 2.0 ** -24 * (h.double().abs() @ wr.double().abs().t())   # W fp32 products and sums, in any order
+    score = torch.sigmoid(z)
+    # the sigmoid carries a quarter of a logit's error on at most, and adds its own few roundings
+    off = bound / 4 + 8 * 2.0 ** -24
+    ranked, order = score.sort(1, descending=True)
+    clear = ranked[:, top - 1] - ranked[:, top] > 2 * off.amax(1)
+    inside = (ranked[:, :top - 1] - ranked[:, 1:top] > 2 * off.amax(1, keepdim=True)).all(1)
+    assert clear[7:].float().mean() > 0.95 and not clear[:7].any()
+    for rows in (R - 1, R):
+        ids, wts = torch.empty(rows, top, dtype=torch.int32, device=DEV), torch.empty(rows, top, device=DEV)
+        cnt, lists = torch.empty(E, dtype=torch.int32, device=DEV), torch.empty(E, rows * top, dtype=torch.int32, device=DEV)
+        sm.group_route(h[:rows].to(DEV), wr.to(DEV), top, 1, 1, ids, wts, cnt, lists)
+        ids, wts = ids.cpu().long(), wts.cpu().double()
+        assert ((wts - score[:rows].gather(1, ids)).abs() <= off[:rows].gather(1, ids)).all()
+        assert torch.equal(ids[clear[:rows]].sort(1)[0], order[:rows, :top][clear[:rows]].sort(1)[0])
+        both = (clear & inside)[:rows]
+        assert torch.equal(ids[both], order[:rows, :top][both])
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
