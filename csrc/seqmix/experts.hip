@@ -597,6 +597,71 @@ expert_gemm_tile_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
   }
 }
 
+// The height of a prompt's expert tiles.  Tokens are taken to be routed at random: an expert has slots / E rows, give or take
+// the root of that.  Fitted to sweeps of 540 to 8192 slots over 4, 8, 16, 32 and 64 experts of width 768 to 4096, evenly
+// routed and skewed by a factor of 20; times below in us, all on one card.
+struct TileHeight {
+  int E, N, K, slots;
+  double mean() const { return (double)slots / E; }
+  int of(double n, int bm) const { return (int)ceil((n < 1 ? 1 : n) / bm); }
+  // row tiles of all experts, when one has `dev` standard deviations more rows than the mean, and in the mean
+  int most(int bm, double dev) const { return E * of(mean() + dev * sqrt(mean()), bm); }
+  double middle(int bm, double dev) const {
+    const double d = dev * sqrt(mean());
+    return E * (of(mean() - d, bm) + 2 * of(mean(), bm) + of(mean() + d, bm)) / 4.0;
+  }
+
+  // Products bound, so a CU's time is the tiles it is given, never less than two deep (a lone block waits for memory):
+  // 117 : 215 for a tile of 32 and of 64 rows.  The small tile fills the chip sooner (8 experts, gate and up, 64 -> 32 rows:
+  // width 1024, 600 slots 40 -> 26, 1600 slots 62 -> 48; width 2048, 1800 slots 212 -> 183), the large one
+  // needs 0.92 of the time per row where both do (width 2048, 700 slots 87 with 32 rows, 76 with 64, 4096 slots 356 and
+  // 350).  Of 424 sizes 48 end above the faster one by more than 5 %, 1.09 at most with 8
+  // experts of equal width, 1.25 with 32.
+  double units(int bm) const {
+    const int cols = (N + 63) / 64, pm = (((slots + bm - 1) / bm + E + 7) & ~7) / 8;
+    // Two row tiles to an XCD at most: known exactly.  Blocks without a tile leave at once, and the hardware deals blocks to
+    // its four shader engines in turn, so with pm row tiles launched the ones that exist count up to the next multiple of
+    // gcd(pm, 4) (1024 columns x 64 on 4 experts: 512 blocks on half of the CUs, 161 us for 87).
+    const int g = pm % 4 == 0 ? 4 : pm % 2 == 0 ? 2 : 1;
+    const int pr = ((most(bm, 2) + 7) / 8 + g - 1) / g * g;
+    if (pr <= 2 && cols * pr <= 64) return 2;
+    const double x = middle(bm, 1.3) * cols / 256;
+    return x >= 5 ? x + 0.4 : x + 0.3 <= 2 ? 2 : ceil(x + 0.3);
+  }
+  int f32() const { return 117 * units(32) < 215 * units(64) ? 32 : 64; }
+
+  // us of a bf16 tile's rounds, or of reading each row tile's weights once through the caches at 8 TB/s
+  double time(int bm, double tiles) const {
+    const int cols = bm == 64 ? (N + 63) / 64 : (N + 127) / 128;
+    const int n = (int)ceil(ceil(tiles / 8) * cols / 32);   // blocks to a CU: row tiles are dealt to 8 XCDs of 32 CUs
+    static const float small[9] = {0, 10.3f, 11, 14, 18, 25.5f, 27, 30, 32.5f};
+    const double k = K / 1024.0;
+    const double work = bm == 64 ? (n <= 8 ? small[n] : 4.0 * n + 1) * k
+                                 : (bm + 36) * 0.115 * (1.08 * (n / 2) + 0.92 * (n % 2)) * k;   // two blocks share a CU
+    const double read = ceil(tiles) * N * K * 2 / 8e6;
+    return work > read ? work : read;
+  }
+  // 64 x 64, or 128 x 128 once that gives one and a half blocks to a CU; 96 or 160 rows (or the other of the two) only where
+  // they win by a twentieth with two standard deviations more rows than the mean, so that one crowded expert does not cost a
+  // round.  8 experts, 64 / 96 / 128 / 160 rows: width 2048, gate and up, 4096 slots 67 / 54 / 65 / 45 (760 TFLOP/s), 2800
+  // slots 51 / 53 / 39 / 43, 1800 slots 44 / 29 / 36 / 40, 1012 slots 25 / 28 / 34 / 35; width 1024, 4096 slots 25.9 / 18.6 /
+  // 22.8 / 25.8.  With 8
+  // experts of equal width 4 of 136 sizes end above the pick of those two by more than 3 % (1.12), elsewhere 32 of 424 (1.36:
+  // 4 experts of width 4096, 1200 slots).  (One workgroup of eight wavefronts per CU that
+  // reads ahead, as the prompts' products have it, gave nothing here: 128 x 256 76 us, two rounds, where 128 x 128 had 69.)
+  int bf16() const {
+    const int old = (long)((slots + 127) / 128 + E) * ((N + 127) / 128) >= 384 ? 128 : 64;
+    int best = 64;
+    double t = time(64, most(64, 2));
+    for (int bm : {96, 128, 160}) {
+      const double u = time(bm, most(bm, 2));
+      if (u < t) best = bm, t = u;
+    }
+    const double mid = middle(old, 1);
+    return t < 0.95 * time(old, ceil(mid < 1 ? 1 : mid)) ? best : old;
+  }
+};
+
 template <typename T, int BM, int BN>
 static int launch_expert_tile(const void* x, int ldx, int x_div, const void* w, const int* cnt, const int* rows, int ldr,
                               void* out, int ldo, int E, int N, int K, int slots, int epi, float limit, float alpha,
@@ -755,6 +820,13 @@ int p2p_sm_group_route(const void* h, int ldh, const float* wr, int R, int W, in
 // total_slots: slots over all experts (rows * top; every slot is in exactly one list).
 // epi = 1: w holds gate / up rows interleaved in groups of 16 (N = 2F rows, a multiple of 32)
 // and out [slots, F] receives the experts' activation instead of the raw products.
+// rows of a prompt's expert tiles (0: few slots, no tiles)
+int p2p_sm_expert_tile(int E, int N, int K, int total_slots, int f32) {
+  if (E < 1 || N < 1 || K < 1 || total_slots < 64 * E) return 0;
+  const TileHeight pick{E, N, K, total_slots};
+  return f32 ? pick.f32() : pick.bf16();
+}
+
 int p2p_sm_expert_gemm(const void* x, int ldx, int x_div, const void* w, const int* cnt,
                        const int* rows, int ldr, void* out, int ldo, int E, int N, int K,
                        int total_slots, int epi, float limit, float alpha, int f32,
@@ -768,30 +840,17 @@ int p2p_sm_expert_gemm(const void* x, int ldx, int x_div, const void* w, const i
 #define ET(T, BM, BN)                                                                                        \
   return launch_expert_tile<T, BM, BN>(x, ldx, x_div, w, cnt, rows, ldr, out, ldo, E, N, K, total_slots, epi, \
                                        limit, alpha, st)
-      // tiles that the slots can be expected to have, half a tile wasted per expert
-      auto tiles = [&](int bm, int bn) { return (long)(total_slots / bm + (total_slots % bm + bm - 1) / bm + E / 2) * ((N + bn - 1) / bn); };
+      const TileHeight pick{E, N, K, total_slots};
       if (f32) {
-        // products bound: the smaller the tile, the more evenly the CUs share them (8 experts of width 1024 and 512, gate and
-        // up / down, 64 x 64 -> 32 x 64: 1012 slots 43.8 / 24.1 -> 36.9 / 20.6 us, 600 slots 40.7 / 23.2 -> 25.2 / 15.1;
-        // width 2048, 2000 slots 213 / 111 -> 188 / 98, 4096 slots 346 / 178 beside 351 / 180)
-        if (tiles(64, 64) < 2048) ET(float, 32, 64);
+        if (pick.f32() == 32) ET(float, 32, 64);
         ET(float, 64, 64);
       }
-      // Two blocks of 128 columns to a CU: the height whose rounds take the shortest time, (height + 36) in units of 0.23 us
-      // at K = 2048.  8 experts, us, 64 x 64 / 96 / 128 / 160 rows: width 2048, gate and up, 4096 slots 70 / 58 / 68 / 50
-      // (690 TFLOP/s), 2800 slots 46 / 32 / 37 / 42, 3400 slots 57 / 52 / 40 / 44, down, 4096 slots 39 / 33 / 39 / 29;
-      // width 1024, 4096 slots 25.5 / 18.8 / 23.3 / 26.0; width 4096, 4096 slots 275 / 219 / 200 / 158.  Fewer blocks leave
-      // the small tile ahead: width 2048, 1800 slots 28.7 / 28.0 / 33.9 / 39.4, 1000 slots 24.2 / 26.7, width 1024, 2800
-      // slots 17.9 / 18.7.  (One workgroup of eight wavefronts per CU that reads ahead, as the prompts' products have it,
-      // gave nothing here: 128 x 256 76 us, two rounds, where 128 x 128 had 69.)
-      if (tiles(96, 128) >= 300) {
-        auto time = [&](int bm) { return (tiles(bm, 128) + 511) / 512 * (bm + 36); };
-        const long t96 = time(96), t128 = time(128), t160 = time(160);
-        if (t96 <= t128 && t96 <= t160) ET(bf16, 96, 128);
-        if (t128 <= t160) ET(bf16, 128, 128);
-        ET(bf16, 160, 128);
+      switch (pick.bf16()) {
+        case 64: ET(bf16, 64, 64);
+        case 96: ET(bf16, 96, 128);
+        case 128: ET(bf16, 128, 128);
+        default: ET(bf16, 160, 128);
       }
-      ET(bf16, 64, 64);
 #undef ET
     }
     int tmp = (((total_slots + 15) / 16 + E) + 7) & ~7;

@@ -185,6 +185,7 @@ _SIGS = {
     "p2p_sm_expert_gemm": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                            c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int,
                            c_void_p],
+    "p2p_sm_expert_tile": [c_int] * 5,
     "p2p_sm_expert_combine": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                               c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
 }

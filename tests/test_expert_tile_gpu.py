@@ -81,11 +81,17 @@ def test_routing_below_and_above_the_row_threshold(dt, W, E, top, at):
 @pytest.mark.parametrize("counts,N,K", [
     ([0, 1, 130, 400, 17], 100, 40),        # 64 x 64 tiles; K ends inside a step of either type
     ([700, 129, 300], 3000, 72),            # 96 x 128 tiles (bf16)
-    ([700, 129, 300], 5152, 72),            # 128 x 128 (bf16)
-    ([700, 129, 300], 7008, 72),            # 160 x 128 (bf16), 64 x 64 (fp32; the others 32 x 64)
-    ([3, 0, 1], 160, 200)])                 # few slots
+    ([700, 129, 300], 5152, 72),            # 64 x 64 (fp32; the ones before 32 x 64)
+    ([700, 129, 300], 7008, 72),
+    ([3, 0, 1], 160, 200),                  # few slots
+    ([0, 1, 129, 170, 100], 5152, 72),      # 128 x 128 (bf16)
+    ([321, 1, 158, 0, 170], 5152, 72)])     # 160 x 128 (bf16)
 @pytest.mark.parametrize("act", [None, "silu_glu", "relu2", "limit"])
 def test_expert_products(dt, counts, N, K, act):
+    tiles = {(548, 100): (64, 32), (1129, 3000): (96, 32), (1129, 5152): (96, 64), (1129, 7008): (96, 64), (4, 160): (0, 0),
+             (400, 5152): (128, 32), (650, 5152): (160, 32)}
+    assert sm.lib().p2p_sm_expert_tile(len(counts), N, K, sum(counts), dt == torch.float32) == \
+        tiles[sum(counts), N][dt == torch.float32]
     if act in ("silu_glu", "limit"):
         N = N // 32 * 32
     g = torch.Generator().manual_seed(4)
