@@ -1121,14 +1121,14 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
     if least > 0:
         vent, cent, walk = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, zx.device)
         NV = vent.shape[0]
-        tmp = torch.empty(NV, H, N, P, device=zx.device, dtype=torch.float32)
-        decay = torch.empty(NV, H, device=zx.device, dtype=torch.float32)
-        # heads that share B and C share their products (a group's 64 x 64 per chunk)
-        cb = torch.empty(NV, G, 64, 64, device=zx.device, dtype=torch.float32) if H > G else None
+        # one buffer: the products of B and C that heads share (a group's 64 x 64 per chunk), the portions' states, their decays
+        shared, states = NV * G * 64 * 64 if H > G else 0, NV * H * N * P
+        ws = torch.empty(shared + states + NV * H, device=zx.device, dtype=torch.float32)
+        at = ws.data_ptr()
         _chk(lib().p2p_sm_mamba_scan_chunked(
             conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), dtoff, dt_bias.data_ptr(),
-            A_log.data_ptr(), Dp.data_ptr(), state.data_ptr(), tmp.data_ptr(), decay.data_ptr(),
-            _lib.ptr(cb), vent.data_ptr(), NV, cent.data_ptr(), cent.shape[0], y.data_ptr(), H, P, N, G, _f32(zx),
+            A_log.data_ptr(), Dp.data_ptr(), state.data_ptr(), at + 4 * shared, at + 4 * (shared + states),
+            at if shared else None, vent.data_ptr(), NV, cent.data_ptr(), cent.shape[0], y.data_ptr(), H, P, N, G, _f32(zx),
             _st(zx)), "mamba_scan_chunked")
     if walk is not None:
         _chk(lib().p2p_sm_mamba_scan(conv.data_ptr(), C, zx.data_ptr(), zx.stride(0), xoff, dtoff,
