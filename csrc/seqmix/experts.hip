@@ -645,7 +645,7 @@ struct TileHeight {
   // they win by a twentieth with two standard deviations more rows than the mean, so that one crowded expert does not cost a
   // round.  8 experts, 64 / 96 / 128 / 160 rows: width 2048, gate and up, 4096 slots 67 / 54 / 65 / 45 (760 TFLOP/s), 2800
   // slots 51 / 53 / 39 / 43, 1800 slots 44 / 29 / 36 / 40, 1012 slots 25 / 28 / 34 / 35; width 1024, 4096 slots 25.9 / 18.6 /
-  // 22.8 / 25.8.  With 8
+  // 22.8 / 25.8; width 4096, down, 900 slots 48 / 62 / 38 / 39.  With 8
   // experts of equal width 4 of 136 sizes end above the pick of those two by more than 3 % (1.12), elsewhere 32 of 424 (1.36:
   // 4 experts of width 4096, 1200 slots).  (One workgroup of eight wavefronts per CU that
   // reads ahead, as the prompts' products have it, gave nothing here: 128 x 256 76 us, two rounds, where 128 x 128 had 69.)
