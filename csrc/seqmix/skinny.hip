@@ -189,8 +189,7 @@ __global__ void __launch_bounds__(512) walk_k(SkinnyArgs a) {
 
 // A row pass as the way into a product (norm_scale_add_k in norms.hip has the sums, in the same order):
 //   xo = x + y / sqrt(mean(y^2) + eps) * w * ls,   h = xo, or with w2 xo / sqrt(mean(xo^2) + eps) * w2
-// Every workgroup forms all rows of h for itself; one writes xo (not over x, which others may still read) and, where
-// another product reads it, h.
+// Every workgroup forms all rows of h for itself; one writes xo (not over x, which others may still read).
 struct PreArgs {
   const float* x;
   const void* y;
@@ -198,8 +197,6 @@ struct PreArgs {
   const float *w, *ls, *w2;
   float eps;
   float* xo;
-  void* h;     // or null
-  int ldh;
 };
 
 // A short causal convolution + bias + silu behind a product whose rows are one token each (mamba_conv_k in mamba.hip):
@@ -417,10 +414,7 @@ __global__ void __launch_bounds__(512) norm_walk_k(SkinnyArgs a, PreArgs pre, Co
       }
 #pragma unroll
       for (int k = 0; k < NC; k++)
-        if (place(k) < n) {
-          stv<4>(sh + m * LD, place(k), x[b][k]);
-          if (pre.h && blockIdx.x == 0) stv<4>((T*)pre.h + (size_t)m * pre.ldh, place(k), x[b][k]);
-        }
+        if (place(k) < n) stv<4>(sh + m * LD, place(k), x[b][k]);
     }
     meet();   // (also: the next rows' sums take the place of these)
   }
@@ -538,19 +532,21 @@ static int launch_normed(const SkinnyArgs& a, const PreArgs& pre, const ConvArgs
 extern "C" {
 
 // p2p_sm_skinny on rows that a residual pass leaves (PreArgs; x, xo fp32 [M, K] packed), with an optional convolution
-// behind columns c0 .. c0 + C - 1 (cw null: none).  K is a multiple of 4 of at most 2048 numbers in bf16, 1024 in fp32.
+// behind columns c0 .. c0 + C - 1 (cw null: none).  K is a multiple of 4 (fp32) or 8 (bf16) of at most 1024 numbers in
+// fp32, 2048 in bf16.  Up to 16 rows; models send 4 at most (NORMED_ROWS in ops/seqmix.py), more than that, whose rows a
+// workgroup forms in several goes, are the tests' alone.
 int p2p_sm_norm_skinny(const float* x, const void* y, int ldy, const float* nw, const float* ls, const float* w2,
-                       float eps, float* xo, void* h, int ldh, const void* w, const void* bias, void* out, int M, int N,
-                       int K, int tanh_from, int c0, int C, int taps, const float* cw, const float* cb, float* tail,
+                       float eps, float* xo, const void* w, const void* bias, void* out, int M, int N, int K,
+                       int tanh_from, int c0, int C, int taps, const float* cw, const float* cb, float* tail,
                        const int* ent, void* conv, int ldo, int conv_f32, int f32, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   const int ep = f32 ? 4 : 8;
-  if (M > 16 || K < ep || K % ep || K > (f32 ? 1024 : 2048) || (size_t)w % 16 || ldy % 4 || ldh % 4 || xo == x ||
-      (((size_t)x | (size_t)xo | (size_t)nw | (size_t)ls | (size_t)w2) % 16) || (((size_t)y | (size_t)h) % (f32 ? 16 : 8)) ||
+  if (M > 16 || K < ep || K % ep || K > (f32 ? 1024 : 2048) || (size_t)w % 16 || ldy % 4 || xo == x ||
+      (((size_t)x | (size_t)xo | (size_t)nw | (size_t)ls | (size_t)w2) % 16) || (size_t)y % (f32 ? 16 : 8) ||
       (cw && (taps < 1 || taps > 4 || c0 < 0 || c0 + C > N || tanh_from < N)))
     return (int)hipErrorInvalidValue;
   const SkinnyArgs a = {nullptr, w, bias, out, 0, M, N, K, N, 0, 0, 0, tanh_from, nullptr, 0, 0, 0, 0.0f, 1.0f};
-  const PreArgs pre = {x, y, ldy, nw, ls, w2, eps, xo, h, ldh};
+  const PreArgs pre = {x, y, ldy, nw, ls, w2, eps, xo};
   const ConvArgs cv = {c0, C, taps, cw, cb, tail, ent, conv, ldo, conv_f32};
   if (cw) SM_DISPATCH_T(f32, return (launch_normed<T, false, true>(a, pre, cv, st)));
   if (tanh_from < N) SM_DISPATCH_T(f32, return (launch_normed<T, true, false>(a, pre, cv, st)));

@@ -55,7 +55,7 @@ _SIGS = {
                              c_void_p],
     "p2p_sm_skinny_conv": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                            c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
-    "p2p_sm_norm_skinny": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int,
+    "p2p_sm_norm_skinny": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p,
                            c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                            c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "p2p_sm_skinny_heads": [c_void_p, ctypes.c_long, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int,
@@ -406,7 +406,7 @@ class NormedRows:
         out = torch.empty(M, N, device=x.device, dtype=y.dtype)
         args = _conv_args(M, N, y.dtype, *conv) if conv is not None else (0, 0, 0) + (None,) * 5 + (0, 0)
         _chk(lib().p2p_sm_norm_skinny(x.data_ptr(), y.data_ptr(), y.stride(0), self.w.data_ptr(), _lib.ptr(self.ls),
-                                      _lib.ptr(self.next_w), self.eps, spare.data_ptr(), None, 0, w.data_ptr(),
+                                      _lib.ptr(self.next_w), self.eps, spare.data_ptr(), w.data_ptr(),
                                       _lib.ptr(b), out.data_ptr(), M, N, K, N if tanh_from is None else tanh_from, *args,
                                       _f32(y), _st(x)), "norm_skinny")
         self.x, self.spare, self.formed, self.h = spare, x, True, None
