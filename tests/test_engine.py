@@ -187,6 +187,33 @@ def test_decode_steps_read_back_once_gpu(greedy):
     assert int(st.ws.err) == 0
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("greedy", [True, False])
+def test_decode_steps_see_the_split_fault_word_gpu(greedy):
+    """A K slice that gave up sets the kernels' split-K fault word, not the workspace's: the step's report carries it too.
+    Set here by the host between two calls; the call raises, the word is cleared and the next call answers."""
+    import ctypes
+
+    from p2p_llm_chat_go_amd.engine.sampling import SamplingParams
+    from p2p_llm_chat_go_amd.ops.gemm import split_fault_word, tiled_split_fault
+
+    cfg = TINY_LLAMA.replace(n_layers=2)
+    eng = Engine(cfg, weights=EngineWeights.random(cfg, "cuda", seed=9), device="cuda", kv_pages=32, max_batch=4)
+    prompts = [[1, 2, 3, 4, 5], [7] * 40]
+    pages = [eng.kv.allocator.alloc(2) for _ in prompts]
+    first = eng.prefill(prompts, pages).cpu().tolist()
+    params = None if greedy else [SamplingParams(temperature=1.3, top_k=64, top_p=0.95, seed=s) for s in (5, 6)]
+    step = lambda: eng.decode_steps(first, [len(p) for p in prompts], pages, 128, 3, params=params)
+    want = step()
+    word, one = split_fault_word(eng.device), torch.ones(1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipMemcpy(ctypes.c_void_p(word), ctypes.c_void_p(one.data_ptr()), ctypes.c_size_t(4), 3) == 0
+    with pytest.raises(RuntimeError, match="split-K"):
+        step()
+    assert tiled_split_fault() == 0 and step() == want
+
+
 def test_fp8_quantize_roundtrip_cpu():
     from p2p_llm_chat_go_amd import ops
 
