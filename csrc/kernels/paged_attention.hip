@@ -45,7 +45,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
   constexpr int HG = (G + 3) / 4;  // groups of 4 heads
   constexpr bool ONE = G == 1;
   const int h = blockIdx.x, r = blockIdx.y, c = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, qd = lane >> 4;
   __shared__ float so[NW][G][HD];
   __shared__ float sm[NW][G], sl[NW][G];
@@ -81,20 +81,24 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
   for (int t = 0; t < PPW; ++t) {
     const int nv = min(ctx - (p0 + t * NW) * PAGE, PAGE);  // keys of the page inside the context
     if (nv <= 0) break;                                    // wave-uniform
-    // rows past the context are not read (what they hold may be anything): the last valid row stands in, as a key struck
-    // out below, as a value set to zero (its own weight is its key's: 0 * inf would be nan)
-    const size_t base = ((size_t)page[t] * Hkv + h) * PAGE * HD;
+    // rows past the context are not read (what they hold may be anything): they are beyond the buffers' end, zero for both
+    // products (the last valid row in their place would make 0 * inf of its infinite values)
+    const size_t base = ((size_t)__builtin_amdgcn_readfirstlane(page[t]) * Hkv + h) * PAGE * HD;
+    const int bytes = nv * HD * (int)sizeof(bf16);
+    const __amdgpu_buffer_rsrc_t keys = __builtin_amdgcn_make_buffer_rsrc((void*)(kc + base), 0, bytes, 0x00027000);
+    const __amdgpu_buffer_rsrc_t values = __builtin_amdgcn_make_buffer_rsrc((void*)(vc + base), 0, bytes, 0x00027000);
+    auto load = [](const __amdgpu_buffer_rsrc_t& rows, int at) {
+      return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rows, at * (int)sizeof(bf16), 0, 0));
+    };
     bf16x8 kr[4][4], vr[4][4];
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
-        kr[b][s] = *reinterpret_cast<const bf16x8*>(kc + base + min(16 * b + n, nv - 1) * HD + 32 * s + 8 * qd);
+      for (int s = 0; s < 4; ++s) kr[b][s] = load(keys, (16 * b + n) * HD + 32 * s + 8 * qd);
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        vr[b][j] = *reinterpret_cast<const bf16x8*>(vc + base + min(16 * b + 4 * qd + j, nv - 1) * HD + 8 * n);
+      for (int j = 0; j < 4; ++j) vr[b][j] = load(values, (16 * b + 4 * qd + j) * HD + 8 * n);
     __builtin_amdgcn_sched_barrier(0);  // all 32 loads are on their way before the first product waits
     f32x4 st[4];
     float mx = -INFINITY;
@@ -122,13 +126,6 @@ __global__ __launch_bounds__(NW * 64) void paged_attn_kernel(
         ls += st[b][j];
       }
     l = fmaf(l, alpha, ls);
-    if (nv < PAGE) {  // wave-uniform
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (16 * b + 4 * qd + j >= nv) vr[b][j] = bf16x8{};
-    }
     if (t > 0) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -483,10 +480,11 @@ int launch_attn(const void* q, int ldq, const void* kc, const void* vc, const in
                        ctx, Hkv, scale, (bf16*)out, ldo);
     return (int)hipGetLastError();
   }
-  // 1024-key chunks where they give 512 workgroups and more (measured at the kernel); up to 4 heads 640: 512 end as one
-  // round of which contexts below their bucket leave CUs idle (8 kv heads of 4, 8 rows of 5120 keys in a bucket of 8192:
-  // 31.3 us with 256-key chunks, 39.5 with these; one head, 8 rows 30.0 / 35.5; 8 heads gain there: 1.5 times slower)
-  if (max_ctx >= 1024 && (long long)R * Hkv * ((max_ctx + 1023) / 1024) >= (G == 8 ? 512 : 640))
+  // 1024-key chunks where they give 512 workgroups and more (measured at the kernel); 640 where up to 4 heads to a kv head
+  // and several chunks meet: 512 end as one round of which contexts below their bucket leave CUs idle (8 kv heads of 4, 8
+  // rows of 5120 keys in a bucket of 8192: 31.3 us with 256-key chunks, 39.5 with these; one head, 8 rows 30.0 / 35.5)
+  const long long groups = max_ctx < 1024 ? 0 : (long long)R * Hkv * ((max_ctx + 1023) / 1024);
+  if (groups >= (G == 8 || max_ctx == 1024 ? 512 : 640))
     return launch_pages<G, 8, 2>(q, ldq, kc, vc, bt, bt_stride, row_bt, ctx, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, st);
   return launch_pages<G, 4, 1>(q, ldq, kc, vc, bt, bt_stride, row_bt, ctx, R, Hkv, scale, max_ctx, out, ldo, part_o, part_ml, st);
 }

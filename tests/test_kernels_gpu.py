@@ -385,11 +385,12 @@ def test_paged_attention_keeps_an_infinite_value(G, max_ctx):
 
 
 @pytest.mark.parametrize("R,Hkv,G,max_ctx", [(64, 8, 2, 1024), (43, 8, 1, 1100), (8, 8, 4, 9000), (2, 1, 8, 2305),
-                                             (3, 3, 4, 2048), (17, 8, 4, 256), (79, 8, 2, 1024), (80, 8, 2, 1024),
-                                             (9, 8, 4, 9000), (79, 8, 1, 1024), (80, 8, 1, 1024), (63, 1, 8, 8192),
+                                             (3, 3, 4, 2048), (17, 8, 4, 256), (63, 8, 2, 1024), (39, 8, 2, 2048), (40, 8, 2, 2048),
+                                             (9, 8, 4, 9000), (64, 8, 1, 1024), (39, 8, 1, 1100), (63, 1, 8, 8192),
                                              (64, 1, 8, 8192)])
 def test_paged_attention_chunks(R, Hkv, G, max_ctx):
-    """Both chunk lengths (640 workgroups and more of 1024 keys, 512 with 8 heads to a kv head: the long one), one chunk, up to 8 and more of them;
+    """Both chunk lengths (512 workgroups and more of 1024 keys, or 640 where several chunks meet and up to 4 heads are to a
+    kv head: the long one), one chunk, up to 8 and more of them;
     contexts that end in every part of a page; whatever lies past a context (the rest of its last page, the null
     page) is NaN; q in rows of 4-byte alignment.  The result is rounded once to bf16 (relative 2^-9 at most) and
     everything before it is fp32."""
