@@ -4,15 +4,15 @@
 // hash of (seed, position, token id), so a replayed graph draws fresh numbers
 // every step without host state).
 //
-// A row of a real vocabulary (16384 to 262144 logits) takes two launches: one workgroup per row reads
-// 513 KB twice and sorts in 28 barriers, 33 us at 128256 logits whatever the batch (up to the CUs), and that
-// chain, not memory, is what bounds it.  So
+// A row of a real vocabulary (24449 to 262144 logits; row_groups() has the exceptions) takes two launches: one workgroup
+// per row reads 513 KB twice and selects and sorts between 28 barriers, 28 us at 128256 logits whatever the batch (up to
+// the CUs; back to back, 33 behind another kernel), and that chain, not memory, is what bounds it.  So
 //   a. row_groups_kernel leaves the largest key of every 128 neighbouring logits, by as many workgroups as
 //      the rows have (one read of the logits: 4.7 us for a row, launch and all, 6.1 for 32);
 //   b. sample_kernel takes a bound from those maxima that at least k logits reach, reads only the groups that
 //      reach it (about 45 of 1002 at k = 40) and ranks what it finds by counting: no histogram, no sort.
 // Both sides give the same candidates in the same order, so the same tokens.  Back to back, k = 40: 128256 logits
-// 28.0 -> 13.5 us for 1 row and 28.4 -> 15.7 for 32, 32000 logits 19.6 -> 13.2; what is left is
+// 27.7 -> 11.8 us for 1 row and 35.3 -> 18.1 for 64, 32000 logits 18.9 -> 11.9, 128256 with k = 128 28.5 -> 17.7; what is left is
 // two launches' ends and the chain of the second (maxima, bound, groups, ranks, draw).
 // Other rows (small vocabularies, gathered shards, and rows with more than 1024 logits at the bound: ties)
 // are selected by one workgroup (1024 threads = 16 waves, the row stays L2-resident across passes):
@@ -556,10 +556,11 @@ P2P_API int p2p_sample_groups(int V) {
 static int row_groups(const float* logits, int ld, int B, int V, const float* temp, unsigned* ws, int* ng,
                       hipStream_t st) {
   *ng = ws ? p2p_sample_groups(V) : 0;
-  // Below 192 groups any k = 128 finds logits in most of them, and the launch of kernel a is not won back (16384 logits,
-  // k = 128, one workgroup per row / two launches: 18.4 / 26.4 us); nor is it for many rows of a small vocabulary, which
-  // fill the CUs by themselves (32000 logits, 256 rows, k = 128 23.6 / 28.2, greedy 8.6 / 11.9).
-  if (*ng < 192 || (B > 64 && V < 49152)) *ng = 0;
+  // Below 192 groups k = 128 finds logits in most of them, and the launch of kernel a is not won back (16384 logits, one
+  // workgroup per row / two launches: k = 128 18.2 / 26.4 us, but k = 40 17.6 / 11.7).  For many rows, which fill the CUs by
+  // themselves, both are level at the worst k (32000 logits, 256 rows: k = 128 23.6 / 24.0, 40 23.1 / 18.5, 1 22.5 / 15.7;
+  // greedy rows 8.6 / 11.8, which only come beside sampled ones: a step of greedy rows takes its argmax).
+  if (*ng < 192) *ng = 0;
   if (*ng == 0) return 0;
   const int wgs = (*ng + 4 * GPW - 1) / (4 * GPW);
   for (int r = 0; r < B; r += 65535)  // grid.y
