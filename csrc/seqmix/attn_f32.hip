@@ -486,18 +486,19 @@ __global__ void __launch_bounds__(128) attn_f32_merge_k(AttnF32Args a, int VP) {
 
 // The kernel of a shape: attn_f32_k without loads ahead, with them, or attn_f32_wide_k.  us, waves / ahead / wide:
 // * up to 128 numbers: ahead.  8 heads of 128 on 2, 400 and 400 rows 29 / 22 / 49, one token at 500 15.3 / 13.3 / 15.6;
-// * longer values: wide while there are few workgroups, which then share a tile's loads and products; with many they hide
-//   each other's waits, and waves that meet at no barrier are ahead.  Latents of 256, 8 heads, a token at 500 18.9 / - / 16.9, 333
-//   rows behind 500 57.8 / - / 54.9 (167 workgroups), 1000 rows 115 / - / 134 (500); of 192, 4 heads, 333 rows 26.6 / - /
-//   24.8 (84), 1000 rows 77 / - / 87 (250); 16 heads on one with keys of 64 and values of 256, 32 tokens at 90 17.5 / - / 15.6
-//   (32), 100 rows behind 500 30 / - / 35 (100), 512 rows 45 / - / 71;
-// * keys above 128 alone: waves.  8 heads of 192 and 128 on 2, 1000 rows 93 / - / 151;
+// * longer values: wide while there are few groups of rows, whose workgroups share a tile's loads and products; with many
+//   they hide each other's waits, and waves that meet at no barrier are ahead.  Groups (before windows are cut into runs),
+//   wide / waves: 16 heads, latents of 256, 210 (160 keys) 30 / 36, 320 31 / 35 (564 keys: 92 / 82), 333 (423) 59 / 56, 512 (600) 85 / 78;
+//   4 heads of 136 and 200 on 2, 54 (160) 18.6 / 20.4, 84 27 / 29, 200 level, 250 (1500) 122 / 114; 16 on one with keys of 64
+//   and values of 256, 40 (130) 16.8 / 18.7, 100 (190) 22.7 / 23.6, (600) 14 % less, 333 (333) 46 / 34;
+// * keys above 128 alone: waves.  8 heads of 192 and 128 on 2, 1000 rows 151 / 98, 32 tokens at 500 22.0 / 19.7, at 90 17.2 /
+//   14.1, with one key each 7.8 / 9.6;
 // * more than 256: wide (what waves would hold does not fit their registers), but for keys alone with many workgroups: 8 heads
-//   of 384 and 128 on 2, one token 12.2 / - / 8.1, 1000 rows 178 / - / 203.
+//   of 384 and 128 on 2, one token 8.1 / 12.2, 1000 rows 203 / 178.
 enum Form { WAVES, AHEAD, WIDE };
-static Form form_of(int D, int V, long groups) {
-  if (D > 256 || V > 256) return V <= 256 && groups >= 128 ? WAVES : WIDE;
-  if (V > 128) return groups < (D > 192 ? 256 : D > 128 ? 128 : 64) ? WIDE : WAVES;
+static Form form_of(int D, int V, long groups, int splits) {
+  if (D > 256 || V > 256) return V <= 256 && groups * splits >= 128 ? WAVES : WIDE;
+  if (V > 128) return groups <= (D > 192 ? 256 : D > 128 ? 127 : 95) ? WIDE : WAVES;
   return D > 128 ? WAVES : AHEAD;
 }
 // value channels of that kernel in blocks of 64
@@ -542,8 +543,8 @@ int p2p_sm_attn_f32_ok(int D, int V) { return D >= 4 && V >= 4 && D % 4 == 0 && 
 long p2p_sm_attn_f32_ws(int U, int H, int G, int D, int V, int splits, int maps) {
   if (splits <= 1 || G < 1 || H % G) return 0;
   const int HG = H / G, HS = head_slots(HG);
-  const long groups = (long)U * G * maps * ((HG + HS - 1) / HS) * splits;
-  return groups * 16 * (value_blocks(V, form_of(D, V, groups)) * 64 + 2);
+  const long groups = (long)U * G * maps * ((HG + HS - 1) / HS);
+  return groups * splits * 16 * (value_blocks(V, form_of(D, V, groups, splits)) * 64 + 2);
 }
 
 // units: row groups of at most 16 / HS rows, HS the power of two >= min(H / G, 16)
@@ -563,7 +564,7 @@ int p2p_sm_attn_f32(const float* q, long sqh, long sqr, long sqm, const float* p
                          out, soh, sor, som, U, H, G, D, V, page, HS, splits, part, out_scale, cap, r1, r2, gate, ldg,
                          gate_pc, blk, P, keep, maps};
   const dim3 grid(U, G * maps * ((HG + HS - 1) / HS), splits);
-  const Form form = form_of(D, V, (long)grid.x * grid.y * grid.z);
+  const Form form = form_of(D, V, (long)grid.x * grid.y, splits);
   const int nb = value_blocks(V, form);
   if (form == WIDE) nb == 4 ? launch_wide<4>(a, grid, st) : launch_wide<8>(a, grid, st);
   else if (nb == 4) launch_waves<4>(a, false, grid, st);

@@ -1257,12 +1257,13 @@ def _attn_f32(q, sqh: int, sqr: int, sqm: int, pool, vbase: int, block_tables, r
     than one with keys and values of up to 128 numbers (8 heads, us, runs of 128 / 64: latents of 512, tokens at 300 and 90
     43 / 22 with the kernel that takes them together, 8 heads of 128 on 2 17 / 15, 100 rows of those behind 500, 50
     workgroups, 17.7 / 19.8).  Windows of 128 keys and less are not worth the merge up to 256 numbers (100 rows of 128 14 /
-    16; 16 heads, three prompts of 70, latents of 256 21 / 31, values of 256 on one 17 / 27)."""
+    16; 16 heads, three prompts of 70, latents of 256 21 / 31, values of 256 on one 17 / 27), but for few rows with long
+    values, whose workgroups share a tile (8 tokens at 90, latents of 256 17.0 / 15.2)."""
     U, hs = units.shape[0], 16 // latent_rows_per_wave(H // G)
     blocks, splits = U * G * maps * (-(-(H // G) // hs)), 1
     if most is not None and blocks < LATENT_SPLIT_BLOCKS:
         few = blocks * -(-most // 64) <= (LATENT_SPLIT_BLOCKS if max(D, V) > 128 else LATENT_SPLIT_BLOCKS // 2) and (
-            most > 128 or max(D, V) > 256)
+            most > 128 or max(D, V) > 256 or (V > 128 and blocks <= 64))
         splits = max(1, min(-(-most // (64 if few else 128)), LATENT_SPLIT_BLOCKS // blocks, 64))
     L, part = lib(), None
     if splits > 1:
