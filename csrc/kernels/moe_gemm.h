@@ -17,7 +17,8 @@
 // 128 x 128 tiles with one launch dimension per expert / this: 65 rows 366 / 318 and 220 / 156, 400 rows 1180 / 367 and
 // 583 / 187, 700 rows 678 / 425 and 541 / 226 (a model's uneven routing: 500 and 245 now), 1024 rows 1223 / 640 and
 // 630 / 315; 59 to 400 rows per expert 772 / 616 and 539 / 524.  Up to about 200 rows the weight stream (5.9 TB/s) is the
-// bound, above that what a CU takes in, rows from the L2 and weights together, at some 40 KB/us.  Half a stage read ahead
+// bound.  Above that a CU takes in some 40 KB/us, rows from the L2 and weights together, which is not what its copies reach
+// (95 to 100 KB/us in whole lines, and these are whole lines): what it waits for is not established.  Half a stage read ahead
 // of its products measured the same, two stages in flight for rows and weights alike (every wavefront copying both) 5 to 40 % slower; copies issued before the reads
 // instead of between the products 2 to 5 % slower from 400 rows on, but for tiles of more than 256 rows (down 365
 // against 323 us at 1024 rows).
