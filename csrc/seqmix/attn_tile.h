@@ -30,6 +30,12 @@ __device__ __forceinline__ void copy_lds16_at(const void* g, int at, unsigned l)
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(g), "v"(at), "s"(l)
                : "memory", "m0");
 }
+// The same to LDS byte address l + ON + 16 * i
+template <int ON>
+__device__ __forceinline__ void copy_lds16_on(const void* g, int at, unsigned l) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(g), "v"(at), "s"(l), "n"(ON)
+               : "memory", "m0", "scc");
+}
 #pragma clang diagnostic pop
 
 __device__ __forceinline__ unsigned lds_address(const void* p) {

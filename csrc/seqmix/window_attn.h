@@ -32,6 +32,23 @@ inline int window_pad32(int n) {   // 32-channel steps the kernels are instantia
   return s <= 1 ? 1 : s <= 2 ? 2 : s <= 4 ? 4 : 8;
 }
 
+// What prompt_attn_k takes beside it (prompt_attn.hip)
+struct PromptArgs {
+  WindowArgs w;
+  int qhs;                        // between the queries of two heads
+  const sm::bf16* qrot;           // [rows, H * Rd] rotated query parts
+  int ldqr;
+  const sm::bf16* kv;             // keys and values formed for the step
+  int ldkv;
+  const int* kbase;
+  int kstride;
+  int ldr, rot0, Rd;              // rows of the pool, where the rotated key part stands in them, its channels
+  int gate_wide, out_wide;        // four numbers at once
+};
+// (row, head) pairs of its workgroups
+#define PROMPT_PAIRS 64
+int prompt_attn_paged(const WindowArgs& w, hipStream_t st);
+
 // (row, head) pairs of a workgroup of window_attn_tile_k
 #define WINDOW_TILE_PAIRS 64
 int window_attn_tile(const WindowArgs& a, int maps, hipStream_t st);

@@ -23,7 +23,8 @@
 // What bounds it: with plain scores the LDS reads (a wavefront reads the whole tile for 16 pairs) and
 // the copies, then the exponentials; with capped and penalised scores the exponentials and logarithms.
 // 2048 rows, 16 heads on 4, D = V = 128: 56 us (300 TFLOP/s) against 276 us for window_attn_mfma_k; a window of 256 20
-// against 58; 32 heads on 8, D = V = 64: 62 against 264.
+// against 58; 32 heads on 8, D = V = 64: 62 against 264.  (Such windows alone are prompt_attn_k's now, 42 us; blocks, kept
+// tokens, two maps and other sizes are this kernel's.)
 //
 // Grid: one dimension, (row group, key/value head, head block) with the last row groups first (they
 // see the most keys), key/value heads innermost so that an XCD's workgroups share few heads; y:
@@ -499,7 +500,9 @@ static int launch_keys(const WindowArgs& a, int maps, hipStream_t st) {
   if (maps == 2) return launch_tile<NK, NV2, KEYS_KEPT, 2>(a, st);
   if (a.blk) return launch_tile<NK, NV2, KEYS_BLOCKS, 1>(a, st);
   if (a.keep) return launch_tile<NK, NV2, KEYS_KEPT, 1>(a, st);
-  return launch_tile<NK, NV2, KEYS_WINDOW, 1>(a, st);
+  // windows alone, with keys and values of 33 to 128 numbers: prompt_attn.hip (its figures)
+  if constexpr (NK >= 2 && NK <= 4 && NV2 >= 2 && NV2 <= 4) return prompt_attn_paged(a, st);
+  else return launch_tile<NK, NV2, KEYS_WINDOW, 1>(a, st);
 }
 
 template <int NK>

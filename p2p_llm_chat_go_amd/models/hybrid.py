@@ -353,6 +353,25 @@ class StepBatch:
             rows = self._units[key] = sm.attn_unit_rows(rows_per_wave, self.ent_host, latent)
         return self.units(rows), rows
 
+    def formed_keys(self, win: int):
+        """(pool rows of the keys that this step's rows see, entry by entry; per entry what turns a position into its place
+        among them) for latent attention that forms its keys."""
+        if all(e[2] == 0 for e in self.ent_host):
+            return self.cache_rows, self.ent[:, 0]
+        got = self._units.get(("keys", win))
+        if got is None:
+            at, base, n = [], [], 0
+            for e, (_row0, rows, start, _slot) in enumerate(self.ent_host):
+                lo = max(0, start - win + 1)
+                j = torch.arange(lo, start + rows, dtype=torch.int32)
+                at.append(e * self.meta["maxp"] * PAGE + j)
+                base.append(n - lo)
+                n += start + rows - lo
+            at = torch.cat(at + [torch.tensor(base, dtype=torch.int32)]).to(self.ids.device)
+            at, base = at[:n], at[n:]
+            got = self._units[("keys", win)] = (self.block_tables.view(-1)[at // PAGE] * PAGE + at % PAGE, base)
+        return got
+
 
 # ---------------------------------------------------------------------------- mixers
 def takes_unformed(part) -> bool:
@@ -629,10 +648,11 @@ class LatentAttention(Mixer):
         # one projection for everything that reads the layer input: q | latent | gate
         self.w_in = torch.cat([get("q"), get("dkv"), get("g")], 0).to(dev, dtype).contiguous()
         self.cnorm = _vec(get("dkv.norm"), dev)
-        # keys and values are never formed: the query is carried into latent space with
-        # W_uk (per head [D, rank]) and the attended latent leaves through W_uv^T
-        self.uk = get("uk").to(dev, dtype).view(H, D, r).contiguous()
-        self.uv, self.uvt = _value_products(get("uv").to(dev, dtype).view(H, V, r))
+        # a step's keys and values are not formed: the query is carried into latent space with
+        # W_uk (per head [D, rank]) and the attended latent leaves through W_uv^T; a prompt's are formed by one product
+        self.ukv = torch.cat([get("uk"), get("uv")], 0).to(dev, dtype).contiguous()
+        self.uk = self.ukv[:H * D].view(H, D, r)
+        self.uv, self.uvt = _value_products(self.ukv[H * D:].view(H, V, r))
         self.sink = _vec(get("sink"), dev)
         self.wo = get("o").to(dev, dtype).contiguous()
 
@@ -644,13 +664,19 @@ class LatentAttention(Mixer):
         pool = cache.paged[layer]
         proj = sm.linear(h, self.w_in)
         sm.rmsnorm(proj[:, H * D:H * D + r], self.cnorm, self.eps, pool, out_rows=b.cache_rows)
+        gated = torch.empty(b.R, H * V, device=h.device, dtype=h.dtype)
+        if sm.formed_ok(proj, pool, D, 0, V, r) and sm.latent_forms(b.ent_host, self.win):
+            rows, kbase = b.formed_keys(self.win)
+            kv = sm.linear(pool.index_select(0, rows), self.ukv)
+            sm.formed_attn(proj, D, None, kv, kbase, pool, r, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
+                           gated, PAGE, H, D, V, b.units(sm.FORMED_PAIRS), gate=proj[:, H * D + r:], gate_channels=True)
+            return sm.linear(gated, self.wo)
         qa = torch.bmm(proj[:, :H * D].view(b.R, H, D).transpose(0, 1), self.uk)   # [H, R, rank]
         ol = torch.empty_like(qa)
         units, rows = b.attn_units(sm.latent_rows_per_wave(H), sm.latent_mfma_ok(qa, pool) and pool.shape[1] > 32,
                                    pool.shape[1])
         sm.latent_attn(qa, pool, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
                        ol, PAGE, units=units, unit_rows=rows, max_keys=b.max_keys)
-        gated = torch.empty(b.R, H * V, device=h.device, dtype=h.dtype)
         sm.heads_gated(ol, self.uv, self.uvt, proj[:, H * D + r:], gated)
         return sm.linear(gated, self.wo)
 
@@ -990,8 +1016,9 @@ class RopeLatentAttention(Mixer):
         self.cnorm = _vec(get("dkv.norm"), dev)
         if self.QUERY_LATENT:
             self.qnorm, self.uq = _vec(get("dq.norm"), dev), get("uq").to(dev, dtype).contiguous()
-        self.uk = get("uk").to(dev, dtype).view(H, D, r).contiguous()
-        self.uv, self.uvt = _value_products(get("uv").to(dev, dtype).view(H, V, r), self.HEAD_GATE)
+        self.ukv = torch.cat([get("uk"), get("uv")], 0).to(dev, dtype).contiguous()
+        self.uk = self.ukv[:H * D].view(H, D, r)
+        self.uv, self.uvt = _value_products(self.ukv[H * D:].view(H, V, r), self.HEAD_GATE)
         self.inv_freq = sm.rope_inv_freq(self.rot_base, self.rot_dims, dev, self.rot_scaling)
         self.rot_mag = sm.rope_magnitude(self.rot_scaling)
         self.wo = get("o").to(dev, dtype).contiguous()
@@ -1014,8 +1041,19 @@ class RopeLatentAttention(Mixer):
             sm.latent_prep(proj[:, qr:], 0, r, Rd, None, self.cnorm, self.inv_freq, b.pos, b.cache_rows,
                            pool, self.eps, None, rm=self.rot_mag)
         nrot2 = self.rot_dims
-        qa = torch.empty(H, R, r + Rd, device=dev, dtype=dt)
         q3 = q.unflatten(1, (H, D + Rd))
+        if sm.formed_ok(q, pool, D, Rd, V, r) and sm.latent_forms(b.ent_host, self.win):
+            qrot = torch.empty(R, H * Rd, device=dev, dtype=dt)
+            sm.rope_rows(q[:, D:], H, D + Rd, self.inv_freq, b.pos, qrot, Rd, rm=self.rot_mag)
+            if nrot2 < Rd:
+                qrot.unflatten(1, (H, Rd))[:, :, nrot2:] = q3[:, :, D + nrot2:]
+            rows, kbase = b.formed_keys(self.win)
+            kv = sm.linear(pool.index_select(0, rows)[:, :r], self.ukv)
+            sm.formed_attn(q, D + Rd, qrot, kv, kbase, pool, r, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, out,
+                           PAGE, H, D, V, b.units(sm.FORMED_PAIRS), out_scale=out_scale,
+                           gate=proj[:, qr + r + Rd:] if self.HEAD_GATE else None)
+            return out
+        qa = torch.empty(H, R, r + Rd, device=dev, dtype=dt)
         torch.bmm(q3[:, :, :D].transpose(0, 1), self.uk, out=qa[:, :, :r])
         sm.rope_rows(q[:, D:], H, D + Rd, self.inv_freq, b.pos, qa[0, :, r:], qa.stride(0),
                      rm=self.rot_mag)

@@ -106,6 +106,9 @@ _SIGS = {
     "p2p_sm_latent_attn_mfma": [c_void_p, c_long, c_long, c_void_p, c_void_p, c_int, c_void_p,
                                 c_void_p, c_void_p, c_int, c_void_p, c_float, c_int, c_void_p,
                                 c_long, c_long, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
+    "p2p_sm_formed_attn": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int,
+                           c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_float, c_int, c_void_p,
+                           c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_int, c_int, c_void_p],
     "p2p_sm_attn_f32": [c_void_p, c_long, c_long, c_long, c_void_p, c_int, c_int, c_void_p, c_int,
                         c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_float, c_int, c_void_p,
                         c_long, c_long, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
@@ -1302,6 +1305,18 @@ def _key_runs(blocks: int, most: int, tile: int, few: int = 128) -> int:
     return max(1, min(-(-most // run), LATENT_SPLIT_BLOCKS // blocks, 64))
 
 
+def _prompt_runs(blocks: int, most: int, each: float) -> int:
+    """Runs of keys for prompts whose keys and values have up to 128 numbers: the number for which a run's tiles of 64 keys
+    (``each`` us where a workgroup waits for its own) and the merge (3.5 us, and 0.03 for each run of a workgroup) take the
+    least.  Through prompt_attn_k, 16 heads of 128 on 4, us, whole windows / cut in 2 / 4 / 8: 389 rows 11.9 / 21.3 / 23.4 / -, 1024 rows 21.8 / 41.3 / 42.0 / -, 64 rows behind
+    512 14.7 / 14.5 / 13.0 / 13.2, behind 3000 51 / 33 / 21.8 / 17.7, 256 rows behind 1024 24.9 / 23.9 / 20.8 / 23.9, 512 rows
+    behind 3000 57.5 / 47.9 / 40.4 / 44.5; through window_attn_tile_k, with blocks behind a window of 1024, 389 rows 17.6 / 22.1 /
+    22.3 / -, 1024 rows 33.2 / 45.8 / 42.3 / -, 64 rows behind 512 21.8 / 16.3 / 13.7 / 13.2."""
+    tiles = -(-most // 64)
+    cost = lambda s: each * -(-tiles // s) + (3.5 + 0.03 * blocks * s if s > 1 else 0.0)
+    return min(range(1, min(tiles, 64) + 1), key=cost) if tiles > 1 else 1
+
+
 def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: int, out,
                 page: int, units=None, max_keys=None, unit_rows=None):
     """Windowed attention over cached latents with a softmax sink.
@@ -1380,6 +1395,87 @@ def latent_attn(qa, cache, block_tables, row_ent, pos, sink, scale: float, win: 
                                   row_ent.data_ptr(), pos.data_ptr(), _lib.ptr(sink), scale,
                                   win, out.data_ptr(), out.stride(0), out.stride(1), R, H, rank,
                                   page, _f32(qa), _st(qa)), "latent_attn")
+    return out
+
+
+FORMED_PAIRS = 64   # rows of one head that a workgroup of the formed kernel takes
+
+
+def latent_forms(ent_host: list, win: int) -> bool:
+    """Whether a step's latent attention forms keys and values (``formed_attn``): for portions of together 32 rows and more whose
+    windows hold up to six keys per row.  Steps of single tokens never do, so that a captured one keeps to its kernels.  A whole
+    layer's attention with its products, in latent space / formed, us (latents of 512 and a window of 1024, of 448 with a rotated
+    part; 16 heads of 128, the latter also 8): 16 rows 38 / 37, 51 / 46, 40 / 37, 32 rows 50 / 40, 66 / 52, 55 / 43, 256 rows
+    85 / 58, 95 / 65, 85 / 53, 2048 rows 181 / 90, 259 / 118; 256 rows behind 1024 100 / 75, 112 / 85, 95 / 77; 512 rows behind 3072
+    110 / 78, 174 / 136, 122 / 121."""
+    rows = sum(e[1] for e in ent_host)
+    keys = sum(min(e[2], win - 1) + e[1] for e in ent_host)
+    return rows >= 32 and max(e[1] for e in ent_host) > 1 and keys <= 6 * rows
+
+
+def formed_ok(q, pool, D: int, Rd: int, V: int, rank: int) -> bool:
+    """The kernel of formed keys and values serves bf16 with keys and values of up to 128 numbers and rotated parts of up to
+    64, all multiples of 8, on 16-byte aligned rows.  P2P_LATENT_MFMA=0 switches it off."""
+    return (q.is_cuda and q.dtype == torch.bfloat16 and 8 <= D <= 128 and D % 8 == 0 and 8 <= V <= 128 and V % 8 == 0
+            and 0 <= Rd <= 64 and Rd % 8 == 0 and rank % 8 == 0 and q.stride(1) == 1 and q.stride(0) % 8 == 0
+            and q.data_ptr() % 16 == 0 and pool.data_ptr() % 16 == 0 and pool.shape[1] % 8 == 0
+            and os.environ.get("P2P_LATENT_MFMA", "1") != "0")
+
+
+def formed_attn(q, qhs: int, qrot, kv, kbase, pool, rank: int, block_tables, row_ent, pos, sink, scale: float, win: int, out,
+                page: int, H: int, D: int, V: int, units, out_scale: float = 1.0, gate=None, gate_channels: bool = False):
+    """Windowed attention of a prompt's rows over keys and values formed from latents.
+
+    q [R, ..]: head h's D numbers at column h * qhs; qrot [R, H * Rd] the rotated query parts, or None.  kv [tokens, H * (D + V)]:
+    all heads' keys, then their values; key j of entry e is row kbase[e] + j (kbase int32, any stride).  pool: the layer's cache,
+    whose rows hold Rd numbers of rotated key behind ``rank``.  out [R, H * V] = sum_j p_j v_j * out_scale with p = softmax over
+    {sink_h} U {scale * (q . k_j + qrot . rot_j) : 0 <= pos - j < win} (sink None: without it), times a sigmoid gate per head or
+    channel (``window_attn``).  units: ``make_units(entries, FORMED_PAIRS)`` on the device."""
+    R = q.shape[0]
+    Rd = 0 if qrot is None else qrot.shape[1] // H
+    if not q.is_cuda:
+        bt = block_tables.long()
+        for r in range(R):
+            e, p = int(row_ent[r]), int(pos[r])
+            j = torch.arange(max(0, p - win + 1), p + 1)
+            row = kv[int(kbase[e]) + j].float()
+            qh = torch.as_strided(q, (H, D), (qhs, 1), q.storage_offset() + r * q.stride(0)).float()
+            s = torch.einsum("hd,nhd->hn", qh, row[:, :H * D].view(-1, H, D))
+            if Rd:
+                rot = pool[bt[e][j // page] * page + j % page, rank:].float()
+                s = s + qrot[r].view(H, Rd).float() @ rot.T
+            s = s * scale
+            m = s.max(-1).values if sink is None else torch.maximum(s.max(-1).values, sink)
+            w = torch.exp(s - m[:, None])
+            den = w.sum(-1) if sink is None else w.sum(-1) + torch.exp(sink - m)
+            o = torch.einsum("hn,nhv->hv", w / den[:, None], row[:, H * D:].view(-1, H, V)) * out_scale
+            if gate is not None:
+                o = o * torch.sigmoid(gate[r, :H * V].float().view(H, V) if gate_channels else gate[r, :H].float()[:, None])
+            out[r] = o.reshape(H * V).to(out.dtype)
+        return out
+    _rows2d(q, "q")
+    _rows2d(out, "out")
+    assert out.shape == (R, H * V) and q.shape[1] >= (H - 1) * qhs + D and q.dtype == kv.dtype == pool.dtype == out.dtype
+    assert kv.dim() == 2 and kv.stride(1) == 1 and kv.shape[1] == H * (D + V) and kv.data_ptr() % 16 == 0
+    assert pool.dim() == 2 and pool.is_contiguous() and pool.shape[1] == rank + Rd
+    assert kbase.dtype == torch.int32 and kbase.dim() == 1 and kbase.numel() == block_tables.shape[0]
+    assert block_tables.dtype == torch.int32 and block_tables.is_contiguous()
+    assert row_ent.dtype == torch.int32 and pos.dtype == torch.int32
+    assert units.dtype == torch.int32 and units.is_contiguous() and units.shape[1] == 2
+    if Rd:
+        _rows2d(qrot, "qrot")
+        assert qrot.shape[0] == R and qrot.dtype == q.dtype and qrot.data_ptr() % 16 == 0
+    if sink is not None:
+        _vec(sink, H, "sink")
+    if gate is not None:
+        _rows2d(gate, "gate")
+        assert gate.shape[0] >= R and gate.shape[1] >= (H * V if gate_channels else H) and gate.dtype == q.dtype
+    _chk(lib().p2p_sm_formed_attn(q.data_ptr(), q.stride(0), qhs, _lib.ptr(qrot), qrot.stride(0) if Rd else 0, kv.data_ptr(),
+                                  kv.stride(0), kbase.data_ptr(), kbase.stride(0), pool.data_ptr(), pool.shape[1], rank, Rd,
+                                  block_tables.data_ptr(), block_tables.shape[1], row_ent.data_ptr(), pos.data_ptr(),
+                                  units.data_ptr(), units.shape[0], _lib.ptr(sink), scale, win, out.data_ptr(), out.stride(0),
+                                  H, D, V, page, out_scale, _lib.ptr(gate), 0 if gate is None else gate.stride(0),
+                                  1 if gate_channels else 0, _st(q)), "formed_attn")
     return out
 
 
@@ -1919,7 +2015,10 @@ def window_attn(q, pool, block_tables, row_ent, pos, sink, scale: float, win: in
         splits = 1
         if max_keys is not None and blocks < LATENT_SPLIT_BLOCKS:
             most = min(max_keys, win + keep) + (max(0, max_keys - win) // every if blk is not None else 0)
-            splits = _key_runs(blocks, most, tile)
+            if tile and M == 1 and 32 < D <= 128 and 32 < V <= 128:
+                splits = _prompt_runs(blocks, most, 0.95 if blk is None and not keep else 1.4)
+            else:
+                splits = _key_runs(blocks, most, tile)
         part = None
         if splits > 1:
             L = lib()
