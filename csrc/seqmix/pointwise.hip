@@ -104,7 +104,22 @@ __global__ void softcap_k(const T* __restrict__ y, int ld, float* __restrict__ o
   out[(size_t)r * n + c] = cap > 0.0f ? cap * tanhf(z / cap) : z;
 }
 
+// Words between page-locked host memory and device memory, past the caches (a captured step's first and last kernel: its
+// metadata in, its tokens out)
+__global__ void copy_words_k(const int* src, int* dst, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int v = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(dst + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 extern "C" {
+
+int p2p_sm_copy_words(const int* src, int* dst, int n, hipStream_t st) {
+  if (n <= 0) return 0;
+  hipLaunchKernelGGL(copy_words_k, dim3((n + 255) / 256), dim3(256), 0, st, src, dst, n);
+  return (int)hipGetLastError();
+}
 
 int p2p_sm_glu_act(const void* gu, int ld, void* out, int ldo, int R, int F, int act, int f32,
                    hipStream_t st) {

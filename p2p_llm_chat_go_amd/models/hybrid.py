@@ -311,8 +311,8 @@ class StepBatch:
         self.flat, self.meta = flat, meta
         self.R, self.E = meta["R"], meta["E"]
         self.ent_host, self.n_out, self.max_pos = meta["ent_host"], meta["n_out"], meta["max_pos"]
-        # most keys any row of this step can see; a batch that is reloaded for a captured
-        # graph reports the whole width of its block tables instead
+        # most keys any row of this step can see; the batch of a captured graph
+        # reports the whole width of its block tables instead
         self.max_keys = meta["max_pos"] + 1
         cut, o = [], 0
         for n in meta["sizes"]:
@@ -323,16 +323,6 @@ class StepBatch:
         self.out_rows = cut[5][:self.n_out]
         self.block_tables = cut[6].view(meta["E"], meta["maxp"])
         self._units = {}
-
-    def reload(self, entries: list, want: list):
-        """Same shape of step (rows, entries, wanted rows, table width), new contents, written
-        into the device tensors this batch already has (a captured graph reads them)."""
-        host, meta = self.build_host(entries, want, self.meta["maxp"])
-        if meta["sizes"] != self.meta["sizes"] or meta["maxp"] != self.meta["maxp"]:
-            raise ValueError("a reloaded step must have the shape of the captured one")
-        self.flat.copy_(host, non_blocking=True)
-        self.ent_host, self.max_pos = meta["ent_host"], meta["max_pos"]
-        self.meta = meta
 
     def units(self, rows_per_wave: int):
         """Row groups for the matrix-core attention kernel (``ops.seqmix.make_units``)."""

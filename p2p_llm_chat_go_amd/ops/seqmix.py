@@ -114,6 +114,7 @@ _SIGS = {
                         c_long, c_long, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                         c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                         c_int, c_int, c_int, c_void_p],
+    "p2p_sm_copy_words": [c_void_p, c_void_p, c_int, c_void_p],
     "p2p_sm_tanh": [c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "p2p_sm_sigmoid_gate": [c_void_p, c_long, c_long, c_void_p, c_int, c_void_p, c_int, c_int,
                             c_int, c_int, c_int, c_int, c_void_p],
@@ -268,6 +269,15 @@ def _vec(t, n, name):
 
 def _rms(x, eps):
     return x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+
+
+def copy_words(src, dst):
+    """dst = src, contiguous int32 of which one is in page-locked host memory, by a kernel of the device's current stream: a
+    node of a captured step, where a copy would be a submission of its own before it and a wait of its own behind it."""
+    assert src.dtype == dst.dtype == torch.int32 and src.is_contiguous() and dst.is_contiguous() and src.numel() == dst.numel()
+    assert src.is_cuda != dst.is_cuda and (dst if src.is_cuda else src).is_pinned()
+    _chk(lib().p2p_sm_copy_words(src.data_ptr(), dst.data_ptr(), src.numel(), _st(src if src.is_cuda else dst)), "copy_words")
+    return dst
 
 
 # ------------------------------------------------------------------ embedding / norms
