@@ -3,6 +3,7 @@
 //   g = min(gate, limit), u = clamp(up, -limit, limit), y = g * sigmoid(1.702 g) * (u + 1),
 // the silu-gated one, silu(gate) * up, and the tanh cap of the logits.
 #include "common.h"
+#include "unit_act.h"
 using namespace sm;
 
 template <typename T>
@@ -55,12 +56,6 @@ __global__ void ff_act4_k(const T* __restrict__ gu, int ld, T* __restrict__ out,
                     (u + 1.0f));
   }
   *(V4*)(out + (size_t)r * ldo + c) = o;
-}
-
-// tanh form of gelu: 0.5 z (1 + tanh(y)), y = sqrt(2/pi) (z + 0.044715 z^3), evaluated as
-// z * sigmoid(2 y), which is the same function (1 + tanh(y) = 2 sigmoid(2 y))
-__device__ __forceinline__ float gelu_tanhf_(float z) {
-  return z * sigmoidf_(1.5957691216057308f * (z + 0.044715f * z * z * z));
 }
 
 // [gate | up] -> act(gate) * up; act: 0 silu, 1 gelu (tanh form).  Bound by memory and by the number of wavefronts:

@@ -1,0 +1,303 @@
+// Products of prompts: out[M, N] = x[M, K] . w[N, K]^T (+ bias), bf16 with fp32 sums, both operands row-major as the models hold
+// them, and what follows the product in its epilogue: a tanh of the columns from tanh_from on (of the rounded result), or the
+// gated unit of a feed-forward, whose gate rows and up rows of w a tile takes together (the result is rounded once, after it).
+//
+// A workgroup owns BM rows x BN columns; WM x WN wavefronts of 16 FM x 16 FN each, WK groups of them that take every WK-th 64
+// numbers of K and meet in LDS at the end.  Both operands go to LDS by copies of 8 rows x 128 bytes (whole lines: a CU takes those
+// in at 95 KB/us, 16 rows x 64 bytes at 58), 16-byte piece p of a row at p ^ its key, ST stages deep; the next half stage is read
+// under the products of the present one, and the copies are issued between products, into the slot that every wavefront has in
+// registers.  W is the product's left operand, its rows dealt so that a lane ends with neighbouring columns of one row of out.
+//
+// What bounds it: below some 1000 rows the copies into LDS (64 x 64: 16 KB for 128 cycles of the matrix cores) and the few
+// workgroups, which is why K is cut inside a workgroup (2048 x 8192, 20 rows: 128 workgroups of 32 x 16 with four groups 11.7 us,
+// 32 x 32 16.7) and eight wavefronts pay where four leave each SIMD one (128 x 128, 2048 x 8192, 2048 rows: 92 us, eight 80);
+// above, LDS: 256 x 256 reads and writes it for as many cycles as the matrix cores take (16384 x 2048, 2048 rows 115 us, 1190
+// TFLOP/s).  10304 x 2048: 48, 300, 1024, 2048 rows 12.6, 24.5, 49.7, 90 us (the library's 15.0, 25.5, 51, 100).
+#include <algorithm>
+
+#include "attn_tile.h"
+#include "unit_act.h"
+using namespace sm;
+
+struct GemmArgs {
+  const bf16* x;
+  const int* rows;      // which rows of x (null: 0 .. M - 1)
+  int ldx;
+  const bf16 *w, *bias;
+  bf16* out;
+  int ldo, M, N, K;     // N: columns of out (a gated unit's w has 2 N rows)
+  int tanh_from;
+  int act;              // gated units: see unit_act
+  float limit, alpha;
+  int m_tiles, n_tiles, wide;
+};
+
+// at most `pending` stages of L copies each under way
+template <int L>
+__device__ __forceinline__ void wait_stages(int pending) {
+  switch (pending) {
+    case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+    case 1: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory"); break;
+    case 2: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * L) : "memory"); break;
+    default: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * L) : "memory"); break;
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int ST, bool ACT>
+__global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
+  constexpr int FM = BM / (16 * WM), FN = BN / (16 * WN), WPK = WM * WN;
+  constexpr int AI = BM / 8 / WPK, BI = BN / 8 / WPK, L = AI + BI;   // copies of a wavefront per stage
+  constexpr int KG = (BM + BN) * 128, STAGE = WK * KG;               // bytes
+  constexpr int RUN = (ACT ? 2 : 4) * FN;                            // neighbouring columns of a lane
+  static_assert(AI * 8 * WPK == BM && BI * 8 * WPK == BN && FM * 16 * WM == BM && FN * 16 * WN == BN, "tile");
+  static_assert(!ACT || FN % 2 == 0, "gate and up");
+  static_assert(3 * L < 64 && ST >= 2 && ST <= 5, "counted copies");
+  extern __shared__ __align__(16) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), i16 = lane & 15, k4 = lane >> 4;
+  const int kg = wave / WPK, wk = wave % WPK, wm = wk / WN, wn = wk % WN;
+  // an XCD's workgroups are neighbours in a list that walks bands of rows, columns outside
+  constexpr int GM = 1024 / BM;
+  const int nb = a.m_tiles * a.n_tiles, per = nb / 8, over = nb % 8, xcd = blockIdx.x % 8;
+  const int tile = (xcd < over ? xcd * (per + 1) : over * (per + 1) + (xcd - over) * per) + blockIdx.x / 8;
+  const int band = tile / (GM * a.n_tiles), first = band * GM, gm = min(a.m_tiles - first, GM), in = tile - band * GM * a.n_tiles;
+  const int m0 = (first + in % gm) * BM, n0 = in / gm * (ACT ? BN / 2 : BN);
+  const int nk = a.K / 64, n = (nk + WK - 1) / WK;
+
+  // copies: an address of the wavefront's per stage, a lane's offset that stays
+  const char* xs = (const char*)(a.x + (a.rows ? 0 : (size_t)m0 * a.ldx));
+  const char* ws = (const char*)(a.w + (size_t)n0 * a.K);
+  const int p8 = lane & 7, r8 = lane >> 3;
+  int at[L];
+#pragma unroll
+  for (int i = 0; i < AI; i++) {
+    const int r = 8 * (wk + WPK * i) + r8;
+    const int m = min(m0 + r, a.M - 1);
+    at[i] = (a.rows ? a.rows[m] : m - m0) * a.ldx * 2 + ((p8 ^ (r & 7)) << 4);
+  }
+  auto w_key = [](int r) { return (r & 3) | ((r / RUN) & 1) << 2; };   // r: row among those of a wavefront
+#pragma unroll
+  for (int i = 0; i < BI; i++) {
+    const int r = 8 * (wk + WPK * i) + r8, rw = r % (16 * FN);
+    int row = ACT ? r / (16 * FN) * (8 * FN) + rw % (8 * FN) : r;
+    row = min(n0 + row, a.N - 1) - n0 + (ACT && rw >= 8 * FN ? a.N : 0);
+    at[AI + i] = row * a.K * 2 + ((p8 ^ w_key(rw)) << 4);
+  }
+  const unsigned lds0 = lds_address(lds) + kg * KG + wk * 1024;
+  auto copy = [&](int i, int t) {   // the i-th of this wavefront's copies of stage t
+    const unsigned to = lds0 + (t % ST) * STAGE + (i < AI ? i * (WPK * 1024) : BM * 128 + (i - AI) * (WPK * 1024));
+    const int kt = WK == 1 ? t : min(t * WK + kg, nk - 1);
+    copy_lds16_at((i < AI ? xs : ws) + (size_t)kt * 128, at[i], to);
+  };
+#pragma unroll
+  for (int t = 0; t < ST; t++)
+    if (t < n)
+#pragma unroll
+      for (int i = 0; i < L; i++) copy(i, t);
+
+  // this lane's rows in a stage
+  const char* base = lds + kg * KG;
+  const int xr = wm * FM * 16 + i16, xk = i16 & 7;
+  const int wr = (i16 >> 2) * RUN + (i16 & 3), wkey = (i16 & 3) | ((i16 >> 2) & 1) << 2;
+  auto read = [&](int t, int ks, bf16x8(&xf)[FM], bf16x8(&wf)[FN]) {
+    const char* s = base + (t % ST) * STAGE;
+#pragma unroll
+    for (int j = 0; j < FN; j++) {
+      const int r = wn * 16 * FN + (ACT && j >= FN / 2 ? 8 * FN + (j - FN / 2) * 4 : j * 4) + wr;
+      wf[j] = *(const bf16x8*)(s + BM * 128 + r * 128 + (((4 * ks + k4) ^ wkey) << 4));
+    }
+#pragma unroll
+    for (int i = 0; i < FM; i++) xf[i] = *(const bf16x8*)(s + (xr + i * 16) * 128 + (((4 * ks + k4) ^ xk) << 4));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; i++)
+#pragma unroll
+    for (int j = 0; j < FN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto products = [&](const bf16x8(&xf)[FM], const bf16x8(&wf)[FN], auto&& between) {
+#pragma unroll
+    for (int i = 0; i < FM; i++) {
+#pragma unroll
+      for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      between(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto nothing = [](int) {};
+  auto meet = [] {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto used_up = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+  bf16x8 x0[FM], w0[FN], x1[FM], w1[FN];
+  wait_stages<L>(min(ST - 1, n - 1));
+  meet();
+  __builtin_amdgcn_s_waitcnt(0xc07f);   // (seen by the compiler: no scalar load is under way where the loop begins)
+  read(0, 0, x0, w0);
+  int t = 0;
+  for (; t + ST < n; t++) {
+    read(t, 1, x1, w1);
+    products(x0, w0, nothing);
+    used_up();
+    wait_stages<L>(ST - 2);   // stage t + 1 is there, for every wavefront once they met
+    meet();
+    read(t + 1, 0, x0, w0);
+    products(x1, w1, [&](int i) {
+#pragma unroll
+      for (int c = i * L / FM; c < (i + 1) * L / FM; c++) copy(c, t + ST);
+    });
+  }
+  for (; t + 1 < n; t++) {
+    read(t, 1, x1, w1);
+    products(x0, w0, nothing);
+    wait_stages<L>(min(ST - 2, n - 2 - t));
+    meet();
+    read(t + 1, 0, x0, w0);
+    products(x1, w1, nothing);
+  }
+  if (WK == 1 || t * WK + kg < nk) {
+    read(t, 1, x1, w1);
+    products(x0, w0, nothing);
+    products(x1, w1, nothing);
+  }
+  if constexpr (WK > 1) {   // the groups' sums, in their order
+    used_up();
+    __syncthreads();
+    f32x4* sx = (f32x4*)lds;
+    if (kg > 0)
+#pragma unroll
+      for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) sx[(((kg - 1) * WPK + wk) * FM * FN + i * FN + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 0; g < WK - 1; g++)
+#pragma unroll
+      for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[i][j] += sx[((g * WPK + wk) * FM * FN + i * FN + j) * 64 + lane];
+  }
+  // this lane's columns c0 .. c0 + RUN - 1 of FM rows
+  const int c0 = n0 + wn * 4 * RUN + k4 * RUN;
+  if (c0 >= a.N) return;
+  const bool whole = c0 + RUN <= a.N;
+  float bias[RUN];
+  if (!ACT && a.bias) {
+#pragma unroll
+    for (int e = 0; e < RUN; e++) bias[e] = __bfloat162float(a.bias[min(c0 + e, a.N - 1)]);
+  }
+#pragma unroll
+  for (int i = 0; i < FM; i++) {
+    const int m = m0 + wm * FM * 16 + i * 16 + i16;
+    if (m >= a.M) continue;
+    alignas(16) bf16 o[RUN];
+#pragma unroll
+    for (int e = 0; e < RUN; e++) {
+      float v = acc[i][e / 4][e % 4];
+      if constexpr (ACT) v = unit_act(a.act, v, acc[i][FN / 2 + e / 4][e % 4], a.limit, a.alpha);
+      else if (a.bias) v += bias[e];
+      o[e] = __float2bfloat16(v);
+      if (!ACT && c0 + e >= a.tanh_from) o[e] = __float2bfloat16(tanhf(__bfloat162float(o[e])));
+    }
+    bf16* to = a.out + (size_t)m * a.ldo + c0;
+    if (whole && a.wide) {
+      if constexpr (RUN % 8 == 0) {
+        if (a.wide > 1) {
+#pragma unroll
+          for (int e = 0; e < RUN; e += 8) *(uint4*)(to + e) = *(const uint4*)(o + e);
+          continue;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < RUN; e += 4) *(uint2*)(to + e) = *(const uint2*)(o + e);
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < RUN; e++)
+      if (c0 + e < a.N) to[e] = o[e];
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int ST>
+static int launch_gemm(GemmArgs a, hipStream_t st) {
+  a.m_tiles = (a.M + BM - 1) / BM;
+  const int cols = a.act >= 0 ? BN / 2 : BN;
+  a.n_tiles = (a.N + cols - 1) / cols;
+  constexpr size_t stages = (size_t)ST * WK * (BM + BN) * 128, sums = (size_t)(WK - 1) * BM * BN * 4, shm = stages > sums ? stages : sums;
+  constexpr bool UNITS = BN / (16 * WN) % 2 == 0;   // takes gate and up
+  if (a.act >= 0 && !UNITS) return (int)hipErrorInvalidValue;
+  const void* const f[] = {(const void*)prompt_gemm_k<BM, BN, WM, WN, WK, ST, false>,
+                           (const void*)prompt_gemm_k<BM, BN, WM, WN, WK, ST, UNITS>};
+  static const hipError_t attr = [&] {
+    for (const void* k : f)
+      if (const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm)) return e;
+    return hipSuccess;
+  }();
+  if (attr != hipSuccess) return (int)attr;
+  void* args[] = {&a};
+  return (int)hipLaunchKernel(f[a.act >= 0], dim3(a.m_tiles * a.n_tiles), dim3(64 * WM * WN * WK), args, shm, st);
+}
+
+// The tiles, and what a product takes on them: us(q) = start + (q - 1) round + K / 64 (q == 1 ? alone : max(alone, each q)) for
+// q workgroups per CU.  Fitted to products of 192 to 16384 columns, K 128 to 8192 and 20 to 2644 rows (5 % off at the tiles that
+// win; what the rule takes is 0.8 % above the best tile on average, 15 % at worst), weights not in the caches.
+struct Tile {
+  int bm, bn;
+  bool units;   // a wavefront's columns are an even number of 16
+  float start, round, alone, each;
+};
+static const Tile TILES[] = {
+    {32, 16, false, 2.9f, 1.5f, 0.068f, 0.074f},    {32, 32, true, 3.5f, 1.9f, 0.091f, 0.100f},
+    {32, 64, true, 3.3f, 1.9f, 0.151f, 0.160f},     {64, 32, true, 3.4f, 2.0f, 0.133f, 0.144f},
+    {64, 64, true, 3.3f, 1.9f, 0.199f, 0.210f},     {64, 64, true, 3.0f, 0.8f, 0.241f, 0.190f},
+    {128, 64, true, 3.3f, 2.4f, 0.291f, 0.294f},    {128, 128, true, 4.0f, 4.0f, 0.453f, 0.456f},
+    {192, 128, true, 5.0f, 4.9f, 0.599f, 0.622f},   {256, 128, true, 7.0f, 3.7f, 0.658f, 0.783f},
+    {192, 256, true, 7.9f, 0.0f, 1.082f, 1.304f},   {256, 256, true, 9.3f, 7.8f, 1.278f, 1.447f},
+    {192, 192, false, 11.2f, 6.3f, 0.684f, 0.864f}, {256, 192, false, 12.1f, 0.0f, 1.039f, 1.413f}};
+static int pick_tile(int M, int N, int K, bool units) {   // N: rows of w
+  int best = 0;
+  float least = 0.0f;
+  for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); i++) {
+    const Tile& t = TILES[i];
+    if (units && !t.units) continue;
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), q = (tiles + 255) / 256;
+    const float us = t.start + (q - 1) * t.round + K / 64 * (q == 1 ? t.alone : std::max(t.alone, t.each * q));
+    if (!best || us < least) best = i + 1, least = us;
+  }
+  return best;
+}
+
+extern "C" {
+
+// x: M rows, or with `rows` those of `span` numbers that it names; act < 0: no gated unit; tile: 0 by the rule
+int p2p_sm_prompt_gemm(const void* x, const int* rows, long span, int ldx, const void* w, const void* bias, void* out, int ldo, int M,
+                       int N, int K, int tanh_from, int act, float limit, float alpha, int tile, hipStream_t st) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K < 64 || K % 64 || ldx < 0 || ldx % 8 || (size_t)x % 16 || (size_t)w % 16 || act > 2 || tile < 0 || tile > (int)(sizeof(TILES) / sizeof(TILES[0])) ||
+      (rows ? span * 2 : (long)ldx * 512) >= 1l << 31 || (long)K * 2 * (act >= 0 ? N + 256l : 256l) >= 1l << 31)
+    return (int)hipErrorInvalidValue;
+  const int wide = ldo % 8 == 0 && (size_t)out % 16 == 0 ? 2 : ldo % 4 == 0 && (size_t)out % 8 == 0 ? 1 : 0;
+  const GemmArgs a = {(const bf16*)x, rows, ldx, (const bf16*)w, (const bf16*)bias, (bf16*)out, ldo, M, N, K, tanh_from,
+                      act, limit, alpha, 0, 0, wide};
+  switch (tile ? tile : pick_tile(M, act >= 0 ? 2 * N : N, K, act >= 0)) {
+    case 1: return launch_gemm<32, 16, 1, 1, 4, 4>(a, st);
+    case 2: return launch_gemm<32, 32, 1, 1, 4, 4>(a, st);
+    case 3: return launch_gemm<32, 64, 1, 2, 2, 4>(a, st);
+    case 4: return launch_gemm<64, 32, 2, 1, 4, 3>(a, st);
+    case 5: return launch_gemm<64, 64, 2, 2, 2, 3>(a, st);
+    case 6: return launch_gemm<64, 64, 2, 2, 1, 4>(a, st);
+    case 7: return launch_gemm<128, 64, 4, 2, 1, 4>(a, st);
+    case 8: return launch_gemm<128, 128, 2, 4, 1, 4>(a, st);
+    case 9: return launch_gemm<192, 128, 2, 4, 1, 3>(a, st);
+    case 10: return launch_gemm<256, 128, 4, 2, 1, 3>(a, st);
+    case 11: return launch_gemm<192, 256, 2, 4, 1, 2>(a, st);
+    case 12: return launch_gemm<256, 256, 2, 4, 1, 2>(a, st);
+    case 13: return launch_gemm<192, 192, 2, 4, 1, 3>(a, st);
+    case 14: return launch_gemm<256, 192, 2, 4, 1, 2>(a, st);
+  }
+  return (int)hipErrorInvalidValue;
+}
+
+}  // extern "C"

@@ -535,7 +535,8 @@ class Mamba1(Mixer):
         self.w_in = get("in").to(dev, dtype).contiguous()
         self.cw, self.cb = _vec(get("conv"), dev), _vec(get("conv.b"), dev)
         self.w_x = get("x").to(dev, dtype).contiguous()
-        self.w_dt = get("dt").to(dev, dtype).t().contiguous()                     # [rank, I]
+        self.w_dt_rows = get("dt").to(dev, dtype).contiguous()                    # [I, rank], prompts read these
+        self.w_dt = self.w_dt_rows.t().contiguous()                               # [rank, I]
         self.dtb, self.Dp = _vec(get("dt.b"), dev), _vec(get("D"), dev)
         # A = -exp(A_log) as a base-2 exponent, states by rows
         self.A2 = (-torch.exp(get("A_log").double()) * sm.LOG2E).t().float().contiguous().to(dev)
@@ -561,7 +562,7 @@ class Mamba1(Mixer):
         st, I = cache.state[layer], self.I
         xp = sm.linear(x, self.w_x)
         sm.selective_scan(x, xp, self.rank, self.w_dt, self.dtb, self.A2, self.Dp, proj[:, I:2 * I],
-                          st["S"], b.ent, b.ent_host, out)
+                          st["S"], b.ent, b.ent_host, out, wdt_rows=self.w_dt_rows)
         if out_scale != 1.0:
             out.mul_(out_scale)
         return out
@@ -657,7 +658,7 @@ class LatentAttention(Mixer):
         gated = torch.empty(b.R, H * V, device=h.device, dtype=h.dtype)
         if sm.formed_ok(proj, pool, D, 0, V, r) and sm.latent_forms(b.ent_host, self.win):
             rows, kbase = b.formed_keys(self.win)
-            kv = sm.linear(pool.index_select(0, rows), self.ukv)
+            kv = sm.linear(pool, self.ukv, rows=rows)
             sm.formed_attn(proj, D, None, kv, kbase, pool, r, b.block_tables, b.row_ent, b.pos, self.sink, self.scale, self.win,
                            gated, PAGE, H, D, V, b.units(sm.FORMED_PAIRS), gate=proj[:, H * D + r:], gate_channels=True)
             return sm.linear(gated, self.wo)
@@ -1038,7 +1039,7 @@ class RopeLatentAttention(Mixer):
             if nrot2 < Rd:
                 qrot.unflatten(1, (H, Rd))[:, :, nrot2:] = q3[:, :, D + nrot2:]
             rows, kbase = b.formed_keys(self.win)
-            kv = sm.linear(pool.index_select(0, rows)[:, :r], self.ukv)
+            kv = sm.linear(pool[:, :r], self.ukv, rows=rows)
             sm.formed_attn(q, D + Rd, qrot, kv, kbase, pool, r, b.block_tables, b.row_ent, b.pos, None, self.scale, self.win, out,
                            PAGE, H, D, V, b.units(sm.FORMED_PAIRS), out_scale=out_scale,
                            gate=proj[:, qr + r + Rd:] if self.HEAD_GATE else None)
@@ -1305,6 +1306,8 @@ class DenseFF:
     """Gated feed-forward W_down(act(W_gate h) * W_up h): silu-gated, or with a ``limit`` in its
     config the clamped unit of ``ops.seqmix.ff_act``.
 
+    ``fill`` without a product forms it itself (``ops.seqmix.linear_unit``).
+
     Every feed-forward offers two ways in: ``forward(h)``, or for a layer that runs the
     projections of its input and the output projections of its sublayers as one product each:
     ``w_in`` (rows that read the layer input, or None), ``fill(proj, h, mid)`` (writes the
@@ -1327,7 +1330,9 @@ class DenseFF:
         self.w_down = self.w_out = get("down").to(dev, dtype).contiguous()
 
     def fill(self, gu, h, mid):
-        if self.limit is None:
+        if gu is None:   # (the product is formed here)
+            sm.linear_unit(h, self.w_gu, mid, self.ACT, self.limit)
+        elif self.limit is None:
             sm.glu_act(gu, mid, self.ACT)
         else:
             sm.ff_act(gu, mid, self.limit)
@@ -1340,7 +1345,11 @@ class DenseFF:
         return sm.linear(act, self.w_down)
 
     def forward(self, h):
-        return self.forward_proj(sm.linear(h, self.w_gu))
+        if isinstance(h, sm.NormedRows):
+            return self.forward_proj(sm.linear(h, self.w_gu))
+        act = torch.empty(h.shape[0], self.F, device=h.device, dtype=h.dtype)
+        self.fill(None, h, act)
+        return sm.linear(act, self.w_down)
 
 
 class MoEFF:
@@ -1563,7 +1572,7 @@ class TopMoEFF:
     def fill_routed(self, proj, h, mid, cnt=None):
         """``fill`` for a layer whose residual pass sums the routed experts itself."""
         if self.Fs:
-            sm.glu_act(proj, mid, "silu")
+            sm.linear_unit(h, self.w_in, mid) if proj is None else sm.glu_act(proj, mid, "silu")
         return self.routed(h, cnt)
 
     def fill(self, proj, h, mid):
@@ -1575,7 +1584,7 @@ class TopMoEFF:
         y = sm.expert_combine(y, wts, torch.empty(h.shape[0], self.width, device=h.device, dtype=h.dtype))
         if self.Fs:
             mid = torch.empty(h.shape[0], self.Fs, device=h.device, dtype=h.dtype)
-            sm.glu_act(sm.linear(h, self.w_in), mid, "silu")
+            sm.linear_unit(h, self.w_in, mid)
             y = y + sm.linear(mid, self.w_out)
         return y
 
@@ -1962,11 +1971,8 @@ class HybridModel:
             if q == 1:
                 y = L.mixer.forward(h, b, self.cache, i)
             elif moe[i]:
-                mid = proj = None
-                if L.ff.n_mid:
-                    proj = sm.linear(h, L.ff.w_in)
-                    mid = torch.empty(R, L.ff.n_mid, device=dev, dtype=self.dtype)
-                routed = L.ff.fill_routed(proj, h, mid, cnts[sum(moe[:i]), :L.ff.E])
+                mid = torch.empty(R, L.ff.n_mid, device=dev, dtype=self.dtype) if L.ff.n_mid else None
+                routed = L.ff.fill_routed(None, h, mid, cnts[sum(moe[:i]), :L.ff.E])
                 y = sm.linear(mid, L.ff.w_out) if mid is not None else None
             else:
                 y = L.ff.forward(h)
@@ -2020,7 +2026,8 @@ class HybridModel:
             L.mixer.mix(sm.linear(h1, L.mixer.w_in, L.mixer.b_in), b, self.cache, k, mid[:, :mm])
             extra = routed = None
             if L.ff is not None:
-                proj = sm.linear(h2, L.ff.w_in) if L.ff.w_in is not None else None
+                own = moe[k] or isinstance(L.ff, DenseFF) or L.ff.w_in is None   # (forms the product of its gated unit itself)
+                proj = None if own else sm.linear(h2, L.ff.w_in)
                 if moe[k]:
                     routed = L.ff.fill_routed(proj, h2, mid[:, mm:], cnts[sum(moe[:k]), :L.ff.E])
                 else:

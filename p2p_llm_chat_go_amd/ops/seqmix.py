@@ -51,6 +51,8 @@ _SIGS = {
                                             c_int, c_float, c_int, c_void_p],
     "p2p_sm_skinny": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                       c_void_p],
+    "p2p_sm_prompt_gemm": [c_void_p, c_void_p, c_long, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
+                           c_int, c_float, c_float, c_int, c_void_p],
     "p2p_sm_skinny_logits": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_int,
                              c_void_p],
     "p2p_sm_skinny_conv": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
@@ -445,10 +447,47 @@ def _conv_args(M: int, N: int, dtype, c0: int, cw, cb, tail, ent, out):
             _f32(out))
 
 
-def linear(x, w, b=None, tanh_from=None):
-    """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, the shapes of ``_skinny`` on a
-    kernel for few rows.  tanh_from: columns from there on pass a tanh (of the rounded result).  x may be
-    ``NormedRows`` (whose only product this is)."""
+def _prompt_gemm_ok(x, w, b=None) -> bool:
+    """Products that ``csrc/seqmix/prompt_gemm.hip`` takes: bf16, K in steps of 64, rows that 16-byte copies can read."""
+    if x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda \
+            or x.device != w.device or x.requires_grad or w.requires_grad:
+        return False
+    (M, K), ld = x.shape, x.stride(0)
+    return (M > 0 and K >= 64 and K % 64 == 0 and w.shape[1] == K and w.is_contiguous() and x.stride(1) == 1 and ld >= K
+            and ld % 8 == 0 and ld < 1 << 22 and K * (w.shape[0] + 256) < 1 << 30
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (b is None or b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and not b.requires_grad))
+
+
+def _prompt_gemm(x, w, b, out, tanh_from=None, act: int = -1, limit: float = 0.0, alpha: float = 0.0, rows=None, tile: int = 0):
+    M, N = out.shape
+    _chk(lib().p2p_sm_prompt_gemm(x.data_ptr(), _lib.ptr(rows), (x.shape[0] - 1) * x.stride(0) + x.shape[1], x.stride(0),
+                                  w.data_ptr(), _lib.ptr(b), out.data_ptr(), out.stride(0), M, N, x.shape[1],
+                                  N if tanh_from is None else tanh_from, act, limit, alpha, tile, _st(x)), "prompt_gemm")
+    return out
+
+
+def _library_tiles(M: int, N: int, K: int) -> bool:
+    """One round of the CUs of whole 256 x 256 tiles, at least three quarters full: the library's kernel for those is the
+    faster one (library / ``prompt_gemm``, us, K = 2048: 8192 columns, 1500 rows 45 / 50, 2048 rows 53 / 60; 16384 columns, 700
+    rows 46 / 51, 1024 rows 57 / 59; a half-full round, 8192 columns of 1024 rows, 37 / 33; more than a round, 2644 rows, 104 / 90)."""
+    return N % 256 == 0 and K >= 1024 and 192 <= (M + 255) // 256 * (N // 256) <= 256
+
+
+def linear(x, w, b=None, tanh_from=None, rows=None):
+    """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, on kernels of few rows (``_skinny``) and of more
+    (``_prompt_gemm_ok``).  tanh_from: columns from there on pass a tanh (of the rounded result).  rows: int32, which rows of
+    x (default: all).  x may be ``NormedRows`` (whose only product this is).
+
+    Why not the library's above 16 rows: a call of it costs 21 us of host time, this one 6, and prompts of a few hundred rows
+    wait for the host; and it is slower itself, by 16 % on average over 192 to 16384 columns, K 128 to 8192 and 20 to 2644
+    rows (10304 x 2048, 2048 rows 100 -> 90 us, 8192 x 2048, 2644 rows 104 -> 90, 2048 x 8192, 300 rows 33 -> 31, 2048 x 2048,
+    48 rows 8.6 -> 5.1; but see ``_library_tiles``)."""
+    if rows is not None:
+        if (x.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and rows.shape[0] > 16 and b is None
+                and tanh_from is None and x.shape[0] * x.stride(0) < 1 << 30 and _prompt_gemm_ok(x, w)):
+            return _prompt_gemm(x, w, None, torch.empty(rows.shape[0], w.shape[0], device=x.device, dtype=x.dtype), rows=rows)
+        x = x.index_select(0, rows)
     if isinstance(x, NormedRows):
         y = x.linear(w, b, tanh_from)
         if y is not None:
@@ -456,6 +495,9 @@ def linear(x, w, b=None, tanh_from=None):
         x = x.rows()
     if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
             b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
+        if x.dim() == 2 and x.shape[0] > 16 and _prompt_gemm_ok(x, w, b) and not (
+                tanh_from is None and _library_tiles(x.shape[0], w.shape[0], x.shape[1])):
+            return _prompt_gemm(x, w, b, torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype), tanh_from)
         y = F.linear(x, w, b)
         if tanh_from is not None:
             tanh_(y[:, tanh_from:])
@@ -465,6 +507,19 @@ def linear(x, w, b=None, tanh_from=None):
                              w.shape[0], x.shape[1], w.shape[0] if tanh_from is None else tanh_from, _f32(x),
                              _st(x)), "skinny")
     return y
+
+
+def linear_unit(x, w, out, act: str = "silu", limit: float | None = None):
+    """out [M, F] = the gated unit of x times w [gate | up, 2 F rows] transposed: ``glu_act``, or with a limit ``ff_act``, in the
+    product's epilogue where a kernel does that (2048 rows of 2048, product and pass -> one launch, us: 2 x 8192 columns 128 ->
+    116, 2 x 4096 64 -> 60)."""
+    M, F_ = out.shape
+    if M > 16 and _prompt_gemm_ok(x, w) and x.shape[0] == M and w.shape[0] == 2 * F_ and out.dtype == x.dtype and \
+            out.device == x.device and out.stride(1) == 1:
+        code = GLU_ACTS[act] if limit is None else 2
+        return _prompt_gemm(x, w, None, out, act=code, limit=0.0 if limit is None else limit, alpha=FF_ALPHA)
+    gu = linear(x, w)
+    return glu_act(gu, out, act) if limit is None else ff_act(gu, out, limit)
 
 
 def linear_conv(x, w, c0: int, cw, cb, tail, ent, ent_host, row_ent, out):
@@ -830,7 +885,10 @@ def sigmoid_gate(o, g, out, H: int, V: int, per_head: bool = False):
     return out
 
 
-def ff_act(gu, out, limit: float, alpha: float = 1.702):
+FF_ALPHA = 1.702
+
+
+def ff_act(gu, out, limit: float, alpha: float = FF_ALPHA):
     """[gate | up] -> min(gate, limit) * sigmoid(alpha * .) * (clamp(up, +-limit) + 1)."""
     R, F = out.shape
     if not gu.is_cuda:
@@ -1159,11 +1217,11 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
 LOG2E = math.log2(math.e)
 
 
-def selective_scan(x, xp, rank: int, wdt, dt_bias, A2, Dp, z, state, ent, ent_host, y):
+def selective_scan(x, xp, rank: int, wdt, dt_bias, A2, Dp, z, state, ent, ent_host, y, wdt_rows=None):
     """Selective state-space scan of the first Mamba, I channels with N states of their own.
     x [R, I] the convolved inputs, xp = [low-rank step sizes (rank) | B (N) | C (N)] per row, z [R, I]
     the gate, all activation typed.  dt = softplus(wdt^T low + dt_bias) with wdt [rank, I]
-    (activation type); A2 fp32 [N, I] = A * log2(e);
+    (activation type; wdt_rows: the same as [I, rank], which portions' product reads); A2 fp32 [N, I] = A * log2(e);
         S[n, c] <- exp(dt_c A[n, c]) S[n, c] + dt_c x_c B_n,   y_c = (sum_n S[n, c] C_n + D_c x_c) silu(z_c).
     state fp32 [slots, N, I]; y [R, I] activation type.  A step of single tokens runs one fused
     kernel per row (projection of dt included); portions project dt with one product first, and
@@ -1204,7 +1262,7 @@ def selective_scan(x, xp, rank: int, wdt, dt_bias, A2, Dp, z, state, ent, ent_ho
             z.stride(0), state.data_ptr(), ent.data_ptr(), E, y.data_ptr(), y.stride(0), I, N,
             _f32(y), _st(y)), "selective_step")
         return y
-    dt = torch.mm(xp[:, :rank], wdt)
+    dt = torch.mm(xp[:, :rank], wdt) if wdt_rows is None else linear(xp[:, :rank], wdt_rows)
     vent = cent = tmp = dtsum = None
     NV = 0
     if _chunked(ent_host):

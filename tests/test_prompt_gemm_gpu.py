@@ -1,0 +1,88 @@
+"""Products of prompts (``ops.seqmix.linear`` above 16 rows, ``linear_unit``) against 64-bit products."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from p2p_llm_chat_go_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TILES = 14
+
+
+def _case(M, N, K, ld=None, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + M * 7 + N)
+    x = torch.randn(M, ld or K, generator=g, device=DEV).bfloat16()[:, :K]
+    return x, (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+
+
+def _close(got, ref):
+    # one rounding to bf16 (2^-9 of the value at most) of fp32 sums of K products: K 2^-24 of the products' magnitude, which
+    # rows ~ N(0, 1) and weights ~ N(0, 1/K) keep below sqrt(K) 2^-24 * 4 of the results' size
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * 4 * got.shape[1] ** 0.5 + 1e-3 * ref.abs().mean()
+    assert bool(((got.double() - ref).abs() <= bound).all())
+
+
+# rows and columns at the edges of every tile (32 to 256), one 64 of K, fewer stages than a tile keeps, groups of K left over
+@pytest.mark.parametrize("tile", range(TILES + 1))
+@pytest.mark.parametrize("M,N,K,ld", [(1, 8, 64, 64), (31, 100, 128, 136), (33, 33, 192, 192), (257, 264, 448, 456),
+                                      (200, 77, 1088, 1088), (513, 520, 320, 320)])
+def test_tiles(tile, M, N, K, ld):
+    x, w = _case(M, N, K, ld)
+    b = torch.randn(N, device=DEV).bfloat16()
+    for shift in (0, 3, 4):   # 16-byte, 2-byte and 8-byte places of the rows
+        whole = torch.full((M + 2, N + 16), 9.0, device=DEV, dtype=torch.bfloat16)
+        out = whole[1:M + 1, shift:shift + N]
+        sm._prompt_gemm(x, w, b, out, tanh_from=N - 5, tile=tile)
+        ref = x.double() @ w.double().t() + b.double()
+        _close(out[:, :N - 5], ref[:, :N - 5])
+        tail = torch.tanh(ref[:, N - 5:])   # of the rounded result: 2^-9 of it, then a rounding
+        assert (out[:, N - 5:].double() - tail).abs().max() <= 2.0 ** -7 * 4
+        out.fill_(9.0)
+        assert bool((whole == 9.0).all())   # nothing beside it was written
+
+
+@pytest.mark.parametrize("tile", [0] + list(range(2, TILES - 1)))
+@pytest.mark.parametrize("act,limit", [("silu", None), ("gelu_tanh", None), ("silu", 1.0)])
+def test_units(tile, act, limit):
+    M, n, K = 131, 330, 256
+    x, w = _case(M, 2 * n, K)
+    ref = x.double() @ (3 * w).double().t()
+    g, u = ref[:, :n], ref[:, n:]
+    if limit is not None:
+        g = g.clamp(max=limit)
+        want = g * torch.sigmoid(1.702 * g) * (u.clamp(-limit, limit) + 1)
+    else:
+        want = (F.silu(g) if act == "silu" else F.gelu(g, approximate="tanh")) * u
+    out = torch.empty(M, n, device=DEV, dtype=torch.bfloat16)
+    sm._prompt_gemm(x, 3 * w, None, out, act=sm.GLU_ACTS[act] if limit is None else 2, limit=limit or 0.0, alpha=sm.FF_ALPHA,
+                    tile=tile)
+    assert ((out.double() - want).norm() / want.norm()).item() < 2.0 ** -8
+    got = sm.linear_unit(x, 3 * w, torch.empty_like(out), act, limit)
+    assert ((got.double() - want).norm() / want.norm()).item() < 2.0 ** -8
+
+
+def test_rows_and_other_rows():
+    x, w = _case(300, 96, 128, 160)
+    rows = torch.randint(0, 300, (45,), device=DEV, dtype=torch.int32)
+    assert torch.equal(sm.linear(x, w, rows=rows), sm.linear(x[rows.long()].contiguous(), w))
+    y = sm.linear(x, w)
+    x[7], x[299, 3] = float("inf"), float("nan")   # a row's values reach no other row
+    z = sm.linear(x, w)
+    keep = [i for i in range(300) if i not in (7, 299)]
+    assert torch.equal(z[keep], y[keep]) and not bool(torch.isfinite(z[7]).any())
+
+
+def test_other_forms_stay_with_the_library():
+    x, w = _case(40, 64, 96)                                  # K not in steps of 64
+    assert torch.equal(sm.linear(x, w), F.linear(x, w))
+    x, w = _case(40, 64, 128, 132)                            # rows that 16-byte copies cannot read
+    assert torch.equal(sm.linear(x, w), F.linear(x, w))
+    x, w = _case(40, 64, 128)
+    for a, b in ((x[:1].expand(40, 128), w), (x, w.t().contiguous().t()), (x.t().contiguous().t(), w), (x[None], w)):
+        assert not sm._prompt_gemm_ok(a, b)
+        assert torch.equal(sm.linear(a, b), F.linear(a, b))
+    w.requires_grad_(True)                                    # whose gradient somebody wants
+    sm.linear(x, w).sum().backward()
+    assert w.grad is not None
+    assert sm.linear(x[:0], w.detach()).shape == (0, 64)
