@@ -10,9 +10,13 @@
 //
 // What bounds it: below some 1000 rows the copies into LDS (64 x 64: 16 KB for 128 cycles of the matrix cores) and the few
 // workgroups, which is why K is cut inside a workgroup (2048 x 8192, 20 rows: 128 workgroups of 32 x 16 with four groups 11.7 us,
-// 32 x 32 16.7) and eight wavefronts pay where four leave each SIMD one (128 x 128, 2048 x 8192, 2048 rows: 92 us, eight 80);
-// above, LDS: 256 x 256 reads and writes it for as many cycles as the matrix cores take (16384 x 2048, 2048 rows 115 us, 1190
-// TFLOP/s).  10304 x 2048: 48, 300, 1024, 2048 rows 12.6, 24.5, 49.7, 90 us (the library's 15.0, 25.5, 51, 100).
+// 32 x 32 16.7) and eight wavefronts pay where four leave each SIMD one (128 x 128, 2048 x 8192, 2048 rows: 92 us, eight 79);
+// above, LDS: 256 x 256 reads and writes it for as many cycles as the matrix cores take (16384 x 2048, 2048 rows 111 us, 1240
+// TFLOP/s; on four wavefronts of 128 x 128, which read a third less, a stage takes 1.42 us for 1.61, but start and end of a tile
+// 20 us more).  The code behind the products is run once per tile and comes from memory, so it is kept short: with tanhf() and
+// the stores of single numbers unrolled in it, 128 x 128 took 79 us where it takes 67, 256 x 256 60 us where 56.
+// us, the library's -> this: 10304 x 2048, 48, 300, 1024, 2048 rows 15.0 -> 12.6, 25.5 -> 20.2, 51 -> 48, 100 -> 84; 2048 x 8192,
+// 300 and 2048 rows 32 -> 32, 82 -> 65; 2048 x 2048, 48 and 2048 rows 8.6 -> 5.0, 21.5 -> 18.9.
 #include <algorithm>
 
 #include "attn_tile.h"
@@ -98,15 +102,21 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
   const char* base = lds + kg * KG;
   const int xr = wm * FM * 16 + i16, xk = i16 & 7;
   const int wr = (i16 >> 2) * RUN + (i16 & 3), wkey = (i16 & 3) | ((i16 >> 2) & 1) << 2;
-  auto read = [&](int t, int ks, bf16x8(&xf)[FM], bf16x8(&wf)[FN]) {
+  // Tiles of more products read them one fragment row at a time under the products of the one before (256 x 256, 10304 x 2048,
+  // 1500 rows: all at once 60 us, a row at a time 55; 64 x 64, 2048 x 8192, 20 rows 31.6 and 34)
+  constexpr bool SPREAD = FM * FN >= 8;
+  auto read1 = [&](int t, int ks, int i, bf16x8(&xf)[FM], bf16x8(&wf)[FN]) {   // the i-th of FM parts
     const char* s = base + (t % ST) * STAGE;
 #pragma unroll
-    for (int j = 0; j < FN; j++) {
+    for (int j = i * FN / FM; j < (i + 1) * FN / FM; j++) {
       const int r = wn * 16 * FN + (ACT && j >= FN / 2 ? 8 * FN + (j - FN / 2) * 4 : j * 4) + wr;
       wf[j] = *(const bf16x8*)(s + BM * 128 + r * 128 + (((4 * ks + k4) ^ wkey) << 4));
     }
+    xf[i] = *(const bf16x8*)(s + (xr + i * 16) * 128 + (((4 * ks + k4) ^ xk) << 4));
+  };
+  auto read = [&](int t, int ks, bf16x8(&xf)[FM], bf16x8(&wf)[FN]) {
 #pragma unroll
-    for (int i = 0; i < FM; i++) xf[i] = *(const bf16x8*)(s + (xr + i * 16) * 128 + (((4 * ks + k4) ^ xk) << 4));
+    for (int i = 0; i < FM; i++) read1(t, ks, i, xf, wf);
     __builtin_amdgcn_sched_barrier(0);
   };
   f32x4 acc[FM][FN];
@@ -137,13 +147,16 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
   read(0, 0, x0, w0);
   int t = 0;
   for (; t + ST < n; t++) {
-    read(t, 1, x1, w1);
-    products(x0, w0, nothing);
+    if constexpr (!SPREAD) read(t, 1, x1, w1);
+    products(x0, w0, [&](int i) {
+      if constexpr (SPREAD) read1(t, 1, i, x1, w1);
+    });
     used_up();
     wait_stages<L>(ST - 2);   // stage t + 1 is there, for every wavefront once they met
     meet();
-    read(t + 1, 0, x0, w0);
+    if constexpr (!SPREAD) read(t + 1, 0, x0, w0);
     products(x1, w1, [&](int i) {
+      if constexpr (SPREAD) read1(t + 1, 0, i, x0, w0);
 #pragma unroll
       for (int c = i * L / FM; c < (i + 1) * L / FM; c++) copy(c, t + ST);
     });
@@ -179,19 +192,17 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < FN; j++) acc[i][j] += sx[((g * WPK + wk) * FM * FN + i * FN + j) * 64 + lane];
   }
-  // this lane's columns c0 .. c0 + RUN - 1 of FM rows
-  const int c0 = n0 + wn * 4 * RUN + k4 * RUN;
-  if (c0 >= a.N) return;
-  const bool whole = c0 + RUN <= a.N;
+  // this lane's columns c0 .. c0 + RUN - 1 of FM rows.  (Little code: a tile runs through it once, from memory)
+  const int cw = n0 + wn * 4 * RUN, c0 = cw + k4 * RUN;
   float bias[RUN];
   if (!ACT && a.bias) {
 #pragma unroll
     for (int e = 0; e < RUN; e++) bias[e] = __bfloat162float(a.bias[min(c0 + e, a.N - 1)]);
   }
+  const bool tanhs = !ACT && cw + 4 * RUN > a.tanh_from;
+  if (!a.wide) __syncthreads();   // (LDS is used again)
 #pragma unroll
   for (int i = 0; i < FM; i++) {
-    const int m = m0 + wm * FM * 16 + i * 16 + i16;
-    if (m >= a.M) continue;
     alignas(16) bf16 o[RUN];
 #pragma unroll
     for (int e = 0; e < RUN; e++) {
@@ -199,24 +210,41 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
       if constexpr (ACT) v = unit_act(a.act, v, acc[i][FN / 2 + e / 4][e % 4], a.limit, a.alpha);
       else if (a.bias) v += bias[e];
       o[e] = __float2bfloat16(v);
-      if (!ACT && c0 + e >= a.tanh_from) o[e] = __float2bfloat16(tanhf(__bfloat162float(o[e])));
     }
-    bf16* to = a.out + (size_t)m * a.ldo + c0;
-    if (whole && a.wide) {
-      if constexpr (RUN % 8 == 0) {
-        if (a.wide > 1) {
+    if (tanhs) {
 #pragma unroll
-          for (int e = 0; e < RUN; e += 8) *(uint4*)(to + e) = *(const uint4*)(o + e);
-          continue;
-        }
+      for (int e = 0; e < RUN; e++)
+        if (c0 + e >= a.tanh_from) o[e] = __float2bfloat16(tanh_(__bfloat162float(o[e])));
+    }
+    const int m1 = m0 + wm * FM * 16 + i * 16, m = m1 + i16;
+    if (a.wide) {
+      bf16* to = a.out + (size_t)m * a.ldo + c0;
+      constexpr int V = RUN % 8 == 0 ? 8 : 4;
+      if (a.wide >= V) {
+#pragma unroll
+        for (int e = 0; e < RUN; e += V)
+          if (m < a.M && c0 + e < a.N) {
+            if constexpr (V == 8) *(uint4*)(to + e) = *(const uint4*)(o + e);
+            else *(uint2*)(to + e) = *(const uint2*)(o + e);
+          }
+      } else {
+#pragma unroll
+        for (int e = 0; e < RUN; e += 4)
+          if (m < a.M && c0 + e < a.N) *(uint2*)(to + e) = *(const uint2*)(o + e);
       }
-#pragma unroll
-      for (int e = 0; e < RUN; e += 4) *(uint2*)(to + e) = *(const uint2*)(o + e);
       continue;
     }
+    // rows or columns that wide stores do not fit: one number at a time, from the wavefront's own place in LDS
+    bf16* const so = (bf16*)lds + wk * (64 * RUN);
 #pragma unroll
-    for (int e = 0; e < RUN; e++)
-      if (c0 + e < a.N) to[e] = o[e];
+    for (int e = 0; e < RUN; e++) so[(k4 * RUN + e) * 16 + i16] = o[e];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll 1
+    for (int q = lane; q < 64 * RUN; q += 64) {
+      const int r = m1 + q / (4 * RUN), c = cw + q % (4 * RUN);
+      if (r < a.M && c < a.N) a.out[(size_t)r * a.ldo + c] = so[q % (4 * RUN) * 16 + q / (4 * RUN)];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
 }
 
@@ -241,21 +269,21 @@ static int launch_gemm(GemmArgs a, hipStream_t st) {
 }
 
 // The tiles, and what a product takes on them: us(q) = start + (q - 1) round + K / 64 (q == 1 ? alone : max(alone, each q)) for
-// q workgroups per CU.  Fitted to products of 192 to 16384 columns, K 128 to 8192 and 20 to 2644 rows (5 % off at the tiles that
-// win; what the rule takes is 0.8 % above the best tile on average, 15 % at worst), weights not in the caches.
+// q workgroups per CU.  Fitted to products of 192 to 16384 columns, K 128 to 8192 and 20 to 2644 rows (4 % off at the tiles that
+// win; what the rule takes is 0.3 % above the best tile on average, 15 % at worst), weights not in the caches.
 struct Tile {
   int bm, bn;
   bool units;   // a wavefront's columns are an even number of 16
   float start, round, alone, each;
 };
 static const Tile TILES[] = {
-    {32, 16, false, 2.9f, 1.5f, 0.068f, 0.074f},    {32, 32, true, 3.5f, 1.9f, 0.091f, 0.100f},
-    {32, 64, true, 3.3f, 1.9f, 0.151f, 0.160f},     {64, 32, true, 3.4f, 2.0f, 0.133f, 0.144f},
-    {64, 64, true, 3.3f, 1.9f, 0.199f, 0.210f},     {64, 64, true, 3.0f, 0.8f, 0.241f, 0.190f},
-    {128, 64, true, 3.3f, 2.4f, 0.291f, 0.294f},    {128, 128, true, 4.0f, 4.0f, 0.453f, 0.456f},
-    {192, 128, true, 5.0f, 4.9f, 0.599f, 0.622f},   {256, 128, true, 7.0f, 3.7f, 0.658f, 0.783f},
-    {192, 256, true, 7.9f, 0.0f, 1.082f, 1.304f},   {256, 256, true, 9.3f, 7.8f, 1.278f, 1.447f},
-    {192, 192, false, 11.2f, 6.3f, 0.684f, 0.864f}, {256, 192, false, 12.1f, 0.0f, 1.039f, 1.413f}};
+    {32, 16, false, 2.8f, 1.2f, 0.067f, 0.082f},   {32, 32, true, 3.3f, 1.4f, 0.090f, 0.115f},
+    {32, 64, true, 3.0f, 1.5f, 0.155f, 0.164f},    {64, 32, true, 3.2f, 1.7f, 0.136f, 0.147f},
+    {64, 64, true, 3.2f, 1.6f, 0.192f, 0.222f},    {64, 64, true, 2.7f, 0.7f, 0.243f, 0.189f},
+    {128, 64, true, 3.0f, 2.1f, 0.289f, 0.286f},   {128, 128, true, 3.6f, 3.1f, 0.449f, 0.452f},
+    {192, 128, true, 5.2f, 2.9f, 0.580f, 0.636f},  {256, 128, true, 7.4f, 3.3f, 0.681f, 0.803f},
+    {192, 256, true, 6.9f, 0.0f, 1.055f, 1.264f},  {256, 256, true, 7.9f, 0.0f, 1.278f, 1.498f},
+    {192, 192, false, 9.9f, 6.3f, 0.686f, 0.833f}, {256, 192, false, 9.7f, 5.7f, 0.974f, 1.198f}};
 static int pick_tile(int M, int N, int K, bool units) {   // N: rows of w
   int best = 0;
   float least = 0.0f;
@@ -275,10 +303,11 @@ extern "C" {
 int p2p_sm_prompt_gemm(const void* x, const int* rows, long span, int ldx, const void* w, const void* bias, void* out, int ldo, int M,
                        int N, int K, int tanh_from, int act, float limit, float alpha, int tile, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
-  if (K < 64 || K % 64 || ldx < 0 || ldx % 8 || (size_t)x % 16 || (size_t)w % 16 || act > 2 || tile < 0 || tile > (int)(sizeof(TILES) / sizeof(TILES[0])) ||
+  if (K < 64 || K % 64 || ldx < 0 || ldx % 8 || (size_t)x % 16 || (size_t)w % 16 || act > 2 || tile < 0 || tile > 16 ||
       (rows ? span * 2 : (long)ldx * 512) >= 1l << 31 || (long)K * 2 * (act >= 0 ? N + 256l : 256l) >= 1l << 31)
     return (int)hipErrorInvalidValue;
-  const int wide = ldo % 8 == 0 && (size_t)out % 16 == 0 ? 2 : ldo % 4 == 0 && (size_t)out % 8 == 0 ? 1 : 0;
+  // neighbours that a store takes at once
+  const int wide = ldo % 8 == 0 && N % 8 == 0 && (size_t)out % 16 == 0 ? 8 : ldo % 4 == 0 && N % 4 == 0 && (size_t)out % 8 == 0 ? 4 : 0;
   const GemmArgs a = {(const bf16*)x, rows, ldx, (const bf16*)w, (const bf16*)bias, (bf16*)out, ldo, M, N, K, tanh_from,
                       act, limit, alpha, 0, 0, wide};
   switch (tile ? tile : pick_tile(M, act >= 0 ? 2 * N : N, K, act >= 0)) {

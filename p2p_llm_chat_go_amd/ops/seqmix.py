@@ -467,22 +467,15 @@ def _prompt_gemm(x, w, b, out, tanh_from=None, act: int = -1, limit: float = 0.0
     return out
 
 
-def _library_tiles(M: int, N: int, K: int) -> bool:
-    """One round of the CUs of whole 256 x 256 tiles, at least three quarters full: the library's kernel for those is the
-    faster one (library / ``prompt_gemm``, us, K = 2048: 8192 columns, 1500 rows 45 / 50, 2048 rows 53 / 60; 16384 columns, 700
-    rows 46 / 51, 1024 rows 57 / 59; a half-full round, 8192 columns of 1024 rows, 37 / 33; more than a round, 2644 rows, 104 / 90)."""
-    return N % 256 == 0 and K >= 1024 and 192 <= (M + 255) // 256 * (N // 256) <= 256
-
-
 def linear(x, w, b=None, tanh_from=None, rows=None):
     """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, on kernels of few rows (``_skinny``) and of more
     (``_prompt_gemm_ok``).  tanh_from: columns from there on pass a tanh (of the rounded result).  rows: int32, which rows of
     x (default: all).  x may be ``NormedRows`` (whose only product this is).
 
     Why not the library's above 16 rows: a call of it costs 21 us of host time, this one 6, and prompts of a few hundred rows
-    wait for the host; and it is slower itself, by 16 % on average over 192 to 16384 columns, K 128 to 8192 and 20 to 2644
-    rows (10304 x 2048, 2048 rows 100 -> 90 us, 8192 x 2048, 2644 rows 104 -> 90, 2048 x 8192, 300 rows 33 -> 31, 2048 x 2048,
-    48 rows 8.6 -> 5.1; but see ``_library_tiles``)."""
+    wait for the host; and it is slower itself, by 20 % on average over 192 to 16384 columns, K 128 to 8192 and 20 to 2644
+    rows (10304 x 2048, 2048 rows 100 -> 84 us, 2048 x 8192, 2048 rows 82 -> 65, 2048 x 2048, 48 rows 8.6 -> 5.0; one of the few
+    the other way: 8192 x 2048, 1300 rows 43.5 -> 46)."""
     if rows is not None:
         if (x.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and rows.shape[0] > 16 and b is None
                 and tanh_from is None and x.shape[0] * x.stride(0) < 1 << 30 and _prompt_gemm_ok(x, w)):
@@ -495,8 +488,7 @@ def linear(x, w, b=None, tanh_from=None, rows=None):
         x = x.rows()
     if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
             b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
-        if x.dim() == 2 and x.shape[0] > 16 and _prompt_gemm_ok(x, w, b) and not (
-                tanh_from is None and _library_tiles(x.shape[0], w.shape[0], x.shape[1])):
+        if x.dim() == 2 and x.shape[0] > 16 and _prompt_gemm_ok(x, w, b):
             return _prompt_gemm(x, w, b, torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype), tanh_from)
         y = F.linear(x, w, b)
         if tanh_from is not None:
@@ -512,7 +504,7 @@ def linear(x, w, b=None, tanh_from=None, rows=None):
 def linear_unit(x, w, out, act: str = "silu", limit: float | None = None):
     """out [M, F] = the gated unit of x times w [gate | up, 2 F rows] transposed: ``glu_act``, or with a limit ``ff_act``, in the
     product's epilogue where a kernel does that (2048 rows of 2048, product and pass -> one launch, us: 2 x 8192 columns 128 ->
-    116, 2 x 4096 64 -> 60)."""
+    113, 2 x 4096 64 -> 57)."""
     M, F_ = out.shape
     if M > 16 and _prompt_gemm_ok(x, w) and x.shape[0] == M and w.shape[0] == 2 * F_ and out.dtype == x.dtype and \
             out.device == x.device and out.stride(1) == 1:
