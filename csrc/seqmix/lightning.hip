@@ -8,17 +8,19 @@
 //                at position 0); the last one is the slot's new state
 //   output pass  o_t = lam^(t+1) S^T q_t + sum_{s <= t} lam^(t-s) (q_t . k_s) v_s
 // `pw` [H, 65] holds the powers lam^0 .. lam^64 of every head, so no power is formed here.
-// One workgroup of four wavefronts per (chunk, head).  Sizes are padded to multiples of 16 with
+// One workgroup of eight wavefronts per (chunk, head).  Sizes are padded to multiples of 16 with
 // zeros in LDS; rows are laid out so that the lanes of a fragment read hit different banks.
-// What bounds it: a workgroup's chain of loads and products (the output pass's products alone take 20 us), two
-// workgroups per CU.  2644 rows, 16 heads of 128 x 128: 36, 19 and 69 us; with one load in flight per thread while staging and the
-// state's rows loaded as they are used 41, 19 and 83.
+// What bounds it: a workgroup's chain of loads and products (the output pass's products alone take 15 us), two
+// workgroups per CU, which LDS allows; so each has eight wavefronts, a pair of which share 16 tokens (or rows of the state) and
+// take half of the columns each.  2644 rows, 16 heads of 128 x 128: 31, 19 and 50 us; on four wavefronts 38, 19 and 72, with one
+// load in flight per thread while staging and the state's rows loaded as they are used 41, 19 and 83.
 #include "common.h"
 using namespace sm;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define LC 64   // tokens of a chunk
+#define LT 512  // threads of a workgroup: eight wavefronts
 
 __device__ __forceinline__ float lsilu(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
@@ -29,16 +31,16 @@ __device__ __forceinline__ float lsilu(float x) {
 static __host__ __device__ __forceinline__ int ld_rows(int n) { return n + ((4 - n) & 63); }
 static __host__ __device__ __forceinline__ int ld_cols(int n) { return n + ((16 - n) & 63); }
 
-// Rows on their way to LDS, four numbers per load and eight loads of a thread in flight (none behind a branch, which would
-// wait for those before it): numbers 4 * (base + 256 i + thread) of the rows padded to 4 * w4
+// Rows on their way to LDS, four numbers per load and four loads of a thread in flight (none behind a branch, which would
+// wait for those before it): numbers 4 * (base + LT i + thread) of the rows padded to 4 * w4
 template <typename T>
 struct Batch {
-  static constexpr int U = 8, N = 256 * U;
+  static constexpr int U = 4, N = LT * U;
   uint2 lo[U], hi[U];   // (bf16: lo alone)
   __device__ __forceinline__ void load(const T* __restrict__ src, size_t ld, int n, int width, int w4, int base) {
 #pragma unroll
     for (int i = 0; i < U; i++) {
-      const int idx = base + i * 256 + threadIdx.x, t = idx / w4, c = (idx % w4) * 4;
+      const int idx = base + i * LT + threadIdx.x, t = idx / w4, c = (idx % w4) * 4;
       const T* p = src + (size_t)min(t, n - 1) * ld + min(c, width - 4);
       if constexpr (sizeof(T) == 2) {
         lo[i] = *(const uint2*)p;
@@ -53,7 +55,7 @@ struct Batch {
   __device__ __forceinline__ void store(float* dst, int ldd, int n, int width, int w4, int base, F scale) const {
 #pragma unroll
     for (int i = 0; i < U; i++) {
-      const int idx = base + i * 256 + threadIdx.x, t = idx / w4, c = (idx % w4) * 4;
+      const int idx = base + i * LT + threadIdx.x, t = idx / w4, c = (idx % w4) * 4;
       if (idx >= LC * w4) break;
       float4 v;
       if constexpr (sizeof(T) == 2) {
@@ -83,14 +85,14 @@ __device__ __forceinline__ void stage(const T* __restrict__ src, size_t ld, int 
     }
     return;
   }
-  for (int idx = threadIdx.x; idx < LC * pad; idx += 256) {
+  for (int idx = threadIdx.x; idx < LC * pad; idx += LT) {
     const int t = idx / pad, c = idx % pad;
     dst[t * ldd + c] = (t < n && c < width) ? lsilu(ldf(src, (size_t)t * ld + c)) * scale(t) : 0.0f;
   }
 }
 
 template <typename T, int NVT>   // value size padded to NVT * 16
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(LT)
 lightning_local_k(const T* __restrict__ proj, int ldp, const float* __restrict__ pw,
                   const int* __restrict__ vent, float* __restrict__ cs, int H, int D, int V,
                   int vec) {
@@ -119,24 +121,26 @@ lightning_local_k(const T* __restrict__ proj, int ldp, const float* __restrict__
   stage(Vp, (size_t)ldp, n, V, VP, sV, LDV, vec, one, base);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+  constexpr int NVH = NVT / 2;                               // a wavefront takes 16 rows of the state, half of the columns
+  const int j0 = (wave & 1) * NVH;
   const int steps = (n + 3) / 4;
   float* out = cs + ((size_t)c * H + h) * D * V;
-  for (int dt = wave; dt * 16 < DP; dt += 4) {
-    f32x4 acc[NVT];
+  for (int dt = wave >> 1; dt * 16 < DP; dt += 4) {
+    f32x4 acc[NVH];
 #pragma unroll
-    for (int j = 0; j < NVT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NVH; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int s = 0; s < steps; s++) {
       const float a = sK[(4 * s + k4) * LDK + dt * 16 + i16];
 #pragma unroll
-      for (int j = 0; j < NVT; j++)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sV[(4 * s + k4) * LDV + j * 16 + i16], acc[j], 0, 0, 0);
+      for (int j = 0; j < NVH; j++)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sV[(4 * s + k4) * LDV + (j0 + j) * 16 + i16], acc[j], 0, 0, 0);
     }
 #pragma unroll
-    for (int j = 0; j < NVT; j++)
+    for (int j = 0; j < NVH; j++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int d = dt * 16 + k4 * 4 + r, v = j * 16 + i16;
+        const int d = dt * 16 + k4 * 4 + r, v = (j0 + j) * 16 + i16;
         if (d < D && v < V) out[(size_t)d * V + v] = acc[j][r];
       }
   }
@@ -174,7 +178,7 @@ lightning_chain_k(float* __restrict__ cs, const float* __restrict__ pw, const in
 }
 
 template <typename T, int NVT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(LT)
 lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ pw,
                 const int* __restrict__ vent, const float* __restrict__ cs, float* __restrict__ out,
                 int ldo, int H, int D, int V, int vec) {
@@ -192,15 +196,18 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
   auto one = [](int) { return 1.0f; };
   const T *Qp = row + (size_t)h * D, *Kp = Qp + (size_t)H * D, *Vp = row + (size_t)2 * H * D + h * V;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
-  const int r0 = wave * 16;                                  // this wavefront's 16 tokens
+  // this wavefront's 16 tokens and its half of the columns (and of the weights' blocks); the longest and the shortest rows of
+  // weights share a SIMD
+  constexpr int NVH = NVT / 2;
+  const int half = wave >> 2, rb = half ? 7 - wave : wave, r0 = rb * 16, j0 = half * NVH;
   // the state's rows, four blocks of four ahead of their products
   const float* S = cs + ((size_t)c * H + h) * D * V;
   constexpr int AHEAD = 4;
-  float st[AHEAD][NVT];
-  auto rows_of = [&](int s, float (&b)[NVT]) {
+  float st[AHEAD][NVH];
+  auto rows_of = [&](int s, float (&b)[NVH]) {
     const float* Sr = S + (size_t)min(4 * s + k4, D - 1) * V;
 #pragma unroll
-    for (int j = 0; j < NVT; j++) b[j] = Sr[min(j * 16 + i16, V - 1)];
+    for (int j = 0; j < NVH; j++) b[j] = Sr[min((j0 + j) * 16 + i16, V - 1)];
   };
   Batch<T> vb;                                               // the values, until the keys' place is free
   int base = 0;
@@ -221,29 +228,29 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
   stage(Qp, (size_t)ldp, n, D, DP, sQ, LDQ, vec, one, base);
   stage(Kp, (size_t)ldp, n, D, DP, sK, LDQ, vec, one, base);
   __syncthreads();
-  // weights lam^(t-s) q_t . k_s, s <= t
-  f32x4 w[LC / 16];
+  // weights lam^(t-s) q_t . k_s, s <= t, of blocks 2 j + half
+  f32x4 w[LC / 32];
 #pragma unroll
-  for (int j = 0; j < LC / 16; j++) w[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < LC / 32; j++) w[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // from the state before the chunk: S^T q, lam^(t+1) comes after the sum
-  f32x4 acc[NVT];
+  f32x4 acc[NVH];
 #pragma unroll
-  for (int j = 0; j < NVT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < NVH; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (r0 < n) {
 #pragma unroll 4
     for (int s = 0; s < DP / 4; s++) {
       const float a = sQ[(r0 + i16) * LDQ + 4 * s + k4];
 #pragma unroll
-      for (int j = 0; j < LC / 16; j++)
-        if (j <= wave)
-          w[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sK[(j * 16 + i16) * LDQ + 4 * s + k4], w[j], 0, 0, 0);
+      for (int j = 0; j < LC / 32; j++)
+        if (2 * j + half <= rb)
+          w[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sK[((2 * j + half) * 16 + i16) * LDQ + 4 * s + k4], w[j], 0, 0, 0);
     }
     for (int s0 = 0; s0 < DP / 4; s0 += AHEAD) {             // (DP is a multiple of 16)
 #pragma unroll
       for (int u = 0; u < AHEAD; u++) {
         const float a = sQ[(r0 + i16) * LDQ + 4 * (s0 + u) + k4];   // zero beyond D
 #pragma unroll
-        for (int j = 0; j < NVT; j++)
+        for (int j = 0; j < NVH; j++)
           acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, st[u][j], acc[j], 0, 0, 0);
         rows_of(s0 + u + AHEAD, st[u]);
       }
@@ -252,27 +259,27 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
     for (int r = 0; r < 4; r++) {
       const float m = p[r0 + k4 * 4 + r + 1];
 #pragma unroll
-      for (int j = 0; j < NVT; j++) acc[j][r] *= m;
+      for (int j = 0; j < NVH; j++) acc[j][r] *= m;
     }
   }
   __syncthreads();   // queries and keys have been read
   if (vec) vb.store(sV, LDV, n, V, VP / 4, 0, one);
   stage(Vp, (size_t)ldp, n, V, VP, sV, LDV, vec, one, base);
 #pragma unroll
-  for (int j = 0; j < LC / 16; j++)
+  for (int j = 0; j < LC / 32; j++)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int t = r0 + k4 * 4 + r, s = j * 16 + i16;
+      const int t = r0 + k4 * 4 + r, s = (2 * j + half) * 16 + i16;
       sP[t * LDP + s] = s <= t ? w[j][r] * p[t - s] : 0.0f;
     }
   __syncthreads();
   if (r0 >= n) return;
 #pragma unroll 4
-  for (int s = 0; s < (wave + 1) * 4; s++) {
+  for (int s = 0; s < (rb + 1) * 4; s++) {
     const float a = sP[(r0 + i16) * LDP + 4 * s + k4];
 #pragma unroll
-    for (int j = 0; j < NVT; j++)
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sV[(4 * s + k4) * LDV + j * 16 + i16], acc[j], 0, 0, 0);
+    for (int j = 0; j < NVH; j++)
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sV[(4 * s + k4) * LDV + (j0 + j) * 16 + i16], acc[j], 0, 0, 0);
   }
 #pragma unroll
   for (int r = 0; r < 4; r++) {
@@ -280,8 +287,8 @@ lightning_out_k(const T* __restrict__ proj, int ldp, const float* __restrict__ p
     if (t >= n) continue;
     float* o = out + (size_t)(en.row0 + t) * ldo + (size_t)h * V;
 #pragma unroll
-    for (int j = 0; j < NVT; j++) {
-      const int v = j * 16 + i16;
+    for (int j = 0; j < NVH; j++) {
+      const int v = (j0 + j) * 16 + i16;
       if (v < V) o[v] = acc[j][r];
     }
   }
@@ -306,11 +313,11 @@ static int launch_light(const T* proj, int ldp, const float* pw, float* state, c
   }();
   if (attr != hipSuccess) return (int)attr;
   dim3 grid(NV, H);
-  hipLaunchKernelGGL((lightning_local_k<T, NVT>), grid, dim3(256), shm1, st, proj, ldp, pw, vent, cs, H,
+  hipLaunchKernelGGL((lightning_local_k<T, NVT>), grid, dim3(LT), shm1, st, proj, ldp, pw, vent, cs, H,
                      D, V, vec);
   hipLaunchKernelGGL(lightning_chain_k, dim3((D * V + 255) / 256, H, E), dim3(256), 0, st, cs, pw, vent,
                      state, cent, H, D * V);
-  hipLaunchKernelGGL((lightning_out_k<T, NVT>), grid, dim3(256), shm2, st, proj, ldp, pw, vent, cs, out,
+  hipLaunchKernelGGL((lightning_out_k<T, NVT>), grid, dim3(LT), shm2, st, proj, ldp, pw, vent, cs, out,
                      ldo, H, D, V, vec);
   return (int)hipGetLastError();
 }
