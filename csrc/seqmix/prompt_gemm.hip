@@ -146,28 +146,46 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
   __builtin_amdgcn_s_waitcnt(0xc07f);   // (seen by the compiler: no scalar load is under way where the loop begins)
   read(0, 0, x0, w0);
   int t = 0;
-  for (; t + ST < n; t++) {
+  auto half0 = [&](int t) {
     if constexpr (!SPREAD) read(t, 1, x1, w1);
     products(x0, w0, [&](int i) {
       if constexpr (SPREAD) read1(t, 1, i, x1, w1);
     });
     used_up();
-    wait_stages<L>(ST - 2);   // stage t + 1 is there, for every wavefront once they met
-    meet();
+  };
+  auto half1 = [&](int t, bool more) {
     if constexpr (!SPREAD) read(t + 1, 0, x0, w0);
     products(x1, w1, [&](int i) {
       if constexpr (SPREAD) read1(t + 1, 0, i, x0, w0);
+      if (more) {
 #pragma unroll
-      for (int c = i * L / FM; c < (i + 1) * L / FM; c++) copy(c, t + ST);
+        for (int c = i * L / FM; c < (i + 1) * L / FM; c++) copy(c, t + ST);
+      }
     });
-  }
-  for (; t + 1 < n; t++) {
-    read(t, 1, x1, w1);
-    products(x0, w0, nothing);
-    wait_stages<L>(min(ST - 2, n - 2 - t));
-    meet();
-    read(t + 1, 0, x0, w0);
-    products(x1, w1, nothing);
+  };
+  // (stage t + 1 is there, for every wavefront once they met.  One loop for all stages takes 24 registers fewer, which 256
+  // columns do not have; 128 x 64, 4096 x 2048, 398 rows are 12.8 us with a loop for the last stages, 15.5 without)
+  if constexpr (BM * BN >= 192 * 256) {
+    for (; t + 1 < n; t++) {
+      const bool more = t + ST < n;
+      half0(t);
+      wait_stages<L>(more ? ST - 2 : min(ST - 2, n - 2 - t));
+      meet();
+      half1(t, more);
+    }
+  } else {
+    for (; t + ST < n; t++) {
+      half0(t);
+      wait_stages<L>(ST - 2);
+      meet();
+      half1(t, true);
+    }
+    for (; t + 1 < n; t++) {
+      half0(t);
+      wait_stages<L>(min(ST - 2, n - 2 - t));
+      meet();
+      half1(t, false);
+    }
   }
   if (WK == 1 || t * WK + kg < nk) {
     read(t, 1, x1, w1);

@@ -468,16 +468,17 @@ def _prompt_gemm(x, w, b, out, tanh_from=None, act: int = -1, limit: float = 0.0
 
 
 def linear(x, w, b=None, tanh_from=None, rows=None):
-    """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, on kernels of few rows (``_skinny``) and of more
+    """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, on kernels of few rows (``_skinny``) and of any
     (``_prompt_gemm_ok``).  tanh_from: columns from there on pass a tanh (of the rounded result).  rows: int32, which rows of
     x (default: all).  x may be ``NormedRows`` (whose only product this is).
 
-    Why not the library's above 16 rows: a call of it costs 21 us of host time, this one 6, and prompts of a few hundred rows
+    Why not the library's: a call of it costs 21 us of host time, this one 6, and prompts of a few hundred rows
     wait for the host; and it is slower itself, by 20 % on average over 192 to 16384 columns, K 128 to 8192 and 20 to 2644
     rows (10304 x 2048, 2048 rows 100 -> 84 us, 2048 x 8192, 2048 rows 82 -> 65, 2048 x 2048, 48 rows 8.6 -> 5.0; one of the few
-    the other way: 8192 x 2048, 1300 rows 43.5 -> 46)."""
+    the other way: 8192 x 2048, 1300 rows 43.5 -> 46).  8 rows of shapes that ``_skinny`` leaves: 2048 x 8192 11.2 -> 10.6, 96 x
+    4096 8.0 -> 6.1, 6144 x 3072 10.9 -> 8.6, 32000 x 4096 58 -> 51."""
     if rows is not None:
-        if (x.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and rows.shape[0] > 16 and b is None
+        if (x.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and rows.shape[0] > 0 and b is None
                 and tanh_from is None and x.shape[0] * x.stride(0) < 1 << 30 and _prompt_gemm_ok(x, w)):
             return _prompt_gemm(x, w, None, torch.empty(rows.shape[0], w.shape[0], device=x.device, dtype=x.dtype), rows=rows)
         x = x.index_select(0, rows)
@@ -488,7 +489,7 @@ def linear(x, w, b=None, tanh_from=None, rows=None):
         x = x.rows()
     if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
             b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
-        if x.dim() == 2 and x.shape[0] > 16 and _prompt_gemm_ok(x, w, b):
+        if _prompt_gemm_ok(x, w, b):
             return _prompt_gemm(x, w, b, torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype), tanh_from)
         y = F.linear(x, w, b)
         if tanh_from is not None:
