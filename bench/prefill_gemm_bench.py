@@ -21,7 +21,7 @@ def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--M", type=int, nargs="*", default=[36, 64, 288, 512, 2048, 8192])
     ap.add_argument("--deep", action="store_true",
-                    help="A/B the deep LDS pipeline: each variant with shallow stages (deep=0) "
+                    help="A/B the K slices: each variant with some 400 workgroups (deep=0) "
                          "and with the default rule (deep=1)")
     ap.add_argument("--deep-modes", type=int, nargs="*", default=[0, 1])
     ap.add_argument("--only", nargs="*", default=None, help="variant names to run")
@@ -32,13 +32,12 @@ def main():
                          "weights in the 256 MB Infinity Cache, as in a model's layer sequence")
     a = ap.parse_args()
     H, F = LLAMA31_8B.hidden, LLAMA31_8B.ffn
-    variants = [("v2_auto", (2, 0, 0)), ("v2_256x256_phased", (2, 1, 1)),
-                ("v2_256x256_2stage", (2, 1, 1, 0)),
+    variants = [("v2_auto", (2, 0, 0)), ("v2_256x256", (2, 1, 1)),
                 ("v2_128x256", (2, 2, 1)), ("v2_128x128", (2, 3, 1)),
                 ("v2_128x128_s2", (2, 3, 2)), ("v2_128x128_s4", (2, 3, 4)),
                 ("v2_128x192", (2, 9, 1)), ("v2_192x128", (2, 7, 1)),
-                ("v2_192x128_s2", (2, 7, 2)), ("v2_192x256", (2, 8, 1)), ("v2_192x256_s2", (2, 8, 2)), ("v2_192x256_auto", (2, 8, 0)), ("v2_256x256_s3", (2, 1, 3, 0)),
-                ("v2_256x256_s5", (2, 1, 5, 0)), ("v2_128x256_s2", (2, 2, 2)),
+                ("v2_192x128_s2", (2, 7, 2)), ("v2_192x256", (2, 8, 1)), ("v2_192x256_s2", (2, 8, 2)), ("v2_192x256_auto", (2, 8, 0)), ("v2_256x256_s3", (2, 1, 3)),
+                ("v2_256x256_s5", (2, 1, 5)), ("v2_128x256_s2", (2, 2, 2)),
                 ("v2_128x256_s3", (2, 2, 3)), ("v2_128x128_s2", (2, 3, 2))]
     L = __import__("p2p_llm_chat_go_amd.ops._lib", fromlist=["lib"]).lib()
     for M in a.M:
@@ -84,8 +83,7 @@ def main():
                 set_tiled_min_m(65 if cfg is None else 1)
                 L.p2p_prefill_deep(deep)
                 if cfg is not None:
-                    tiled_config(*cfg[:3])
-                    L.p2p_prefill_phased(cfg[3] if len(cfg) > 3 else 1)
+                    tiled_config(*cfg)
                 t = graph_time(lambda i: fn(Ws[i % ncp]), n_inner=10)
                 print(json.dumps({"M": M, "gemm": name, "variant": vname, "us": round(t, 1),
                                   "TFLOPs": round(flops / (t * 1e-6) / 1e12, 1),

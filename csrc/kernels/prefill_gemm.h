@@ -3,8 +3,7 @@
 //   out[m, n] = epilogue( rstd[m] * sum_k X[m, k] * W[n, k] )   (gemm_epilogue.h)
 //
 // Tiles BM x BN x 64 (launch_tile has the shapes, pick_tile the choice): 512 threads = 8 waves in a 2 (M) x 4 (N)
-// grid, wave tile (BM/2) x (BN/4) of v_mfma_f32_16x16x32_bf16 accumulators; 128 x 128 and 128 x 192 on 4 waves in a
-// 2 x 2 grid (reads_ahead below).
+// grid, wave tile (BM/2) x (BN/4) of v_mfma_f32_16x16x32_bf16 accumulators.
 // Both operands are staged with `global_load_lds_dwordx4` (one wave-instruction
 // = 1 KiB), so no VGPRs or VALU are spent on staging, and read by conflict-free
 // ds_read_b128:
@@ -122,17 +121,18 @@ __device__ __forceinline__ void pin_scalars(const T&... v) {
   (pin_scalar(v), ...);
 }
 
-// Tiles that read ahead (a workgroup has the CU to itself): 128 x 128 and 128 x 192 on four wavefronts of 64 x BN/2, each
-// the only one on its SIMD, 128 x 256 on eight of 64 x 64.  Eight in step read a half stage, waited, multiplied it, and
-// issued the copies between.  These read the next half stage under the products of the present one, and issue their copies
-// (a scalar address and a lane's constant offset) between the products, into the stage whose second half every wave has in
-// registers: down of llama3.1-8B at 1024 rows, in step 173 us, ahead 136 with 128 x 128 (37 % of the time on the matrix
-// cores: the copies' issue and the meeting of the waves are the rest; LDS reads take a fifth of the cycles, no bank
-// conflicts), 118 with 128 x 256, which copies a quarter less per product.  SwiGLU 28672 x 4096, 250 rows, 128 x 256 in
-// step / ahead 85 / 68.  A fifth wavefront that touched the lines of stages further ahead gave nothing; 256 x 128
-// measured as 128 x 256.
-template <int BM, int BN, int NWV>
-constexpr bool reads_ahead() { return NWV == 4 || BM * BN == 128 * 256; }
+// Tiles that read ahead (a workgroup has the CU to itself): 128 rows and more.  In step, eight wavefronts read a half stage,
+// waited, multiplied it, and issued the copies between.  These read the next half stage a fragment row at a time under the
+// products of the present one, and issue their copies (a scalar address and a lane's constant offset) between the products, into
+// the stage whose second half every wave has in registers.  llama3.1-8B, us: down, 1024 rows, in step 173, on four wavefronts
+// of 128 x 128 136, now 128 x 256 112 (1080 TFLOP/s); SwiGLU 28672 x 4096, 256 x 256 in four phases with a unit of copies
+// each 219, now 195 (1240 TFLOP/s), 398 rows 119, now 102; 4096 x 4096, 128 x 128 on four wavefronts 40, now 35, and with the
+// residual 50, now 36; 6144 x 4096, 128 x 192 on four 55, now 47.  256 x 128 measured as 128 x 256.
+template <int BM, int BN, int STAGES, bool NORM>
+constexpr bool reads_ahead() {
+  if (BM * BN == 256 * 256 && NORM) return false;   // (no registers for the sums)
+  return BM >= 128 && (STAGES >= 3 || BM * BN >= 192 * 256);
+}
 
 template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, int NWV = 8>
 __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
                                                           int up_off, void* __restrict__ out,
                                                           int ldo, float eps, EpiArgs ea,
                                                           SplitArgs sp) {
-  constexpr bool PIPE = reads_ahead<BM, BN, NWV>();
+  constexpr bool PIPE = reads_ahead<BM, BN, STAGES, NORM>();
   constexpr int NT = NWV * 64;
   constexpr int WN = NWV / 2;        // 2 x WN wave grid
   constexpr int FM = BM / 32;        // 16-row fragments per wave
@@ -151,8 +151,8 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
   constexpr int STAGE = (AB + BB) * 64;  // bf16x8 per stage
   constexpr int AI = AB / NWV, BI = BB / NWV;  // blocks per wave per stage
   constexpr int L = AI + BI;               // LDS-DMA instructions per thread per stage
+  constexpr bool RES_AHEAD = BM * BN <= 128 * 256;   // (larger tiles have no registers for them)
   static_assert(AB % NWV == 0 && BB % NWV == 0, "tile");
-  static_assert(!PIPE || STAGES >= 3, "the stage after the present one is read ahead");
   static_assert(FM >= 1 && FN >= 2, "tile");
   // PIPE: given at the launch.  A static 160 KiB tells the compiler that one wavefront per SIMD is all there can be, and it
   // moves the accumulators through AGPRs, four copies per product
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
   const bf16* asrc[AI];
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
-    // 8 rows x 128 bytes per block, 16-byte chunks of row R permuted by R & 7 (see the phased kernel)
+    // 8 rows x 128 bytes per block, 16-byte chunks of row R permuted by R & 7
     int row = m0 + 8 * (w + NWV * i) + (lane >> 3);
     row = row < M ? row : M - 1;
     asrc[i] = X + (size_t)row * ldx + 8 * ((lane & 7) ^ (lane >> 3));
@@ -223,6 +223,25 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
       bgi[j] = wn * FN + j;
     }
   }
+
+  // the residual values of fragment rows i0 .. i1 - 1 of the wave at (wm_, wn_)
+  auto residuals = [&](int wm_, int wn_, int i0, int i1, bf16(&res)[FM][4][FN]) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      if (i < i0 || i >= i1) continue;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const int m = min(m0 + wm_ * (BM / 2) + 16 * i + 4 * (lane >> 4) + jj, M - 1);
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          res[i][jj][j] = reinterpret_cast<const bf16*>(out)[(size_t)m * ldo + (nt_i * (BN / 16) + wn_ * FN + j) * 16 + (lane & 15)];
+      }
+    }
+  };
+  // They are loaded before the copies begin (behind the products they cost 7 us: 4096 x 4096, 1024 rows, 43 us where the plain
+  // product takes 36), by the slices of a reduction while they wait for each other
+  bf16 res[FM][4][FN];
+  if constexpr (EPI == EPI_RESID && !SPLIT && RES_AHEAD) residuals(wm, wn, 0, FM, res);
 
   f32x4 acc[FM][FN];
 #pragma unroll
@@ -266,13 +285,16 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int i = 0; i < L; ++i) copy(i, t);
     // (LDS reads as plain loads: the copies are asm, so the compiler waits for exactly what a product needs)
     const int ar = (wm * FM * 16 + (lane & 15)) * 8, aq = lane >> 4, ax = lane & 7;
-    auto read = [&](int t, int ks, bf16x8(&af)[FM], bf16x8(&bfr)[FN]) {
+    auto read_part = [&](int t, int ks, int i, bf16x8(&af)[FM], bf16x8(&bfr)[FN]) {   // fragment row i and its share of columns
       const bf16x8* sa = lds + (t % STAGES) * STAGE;
       const bf16x8* sb = sa + AB * 64 + lane;
+      af[i] = sa[ar + i * 128 + ((4 * ks + aq) ^ ax)];
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = sa[ar + i * 128 + ((4 * ks + aq) ^ ax)];
+      for (int j = i * FN / FM; j < (i + 1) * FN / FM; ++j) bfr[j] = sb[(bgi[j] * 2 + ks) * 64];
+    };
+    auto read = [&](int t, int ks, bf16x8(&af)[FM], bf16x8(&bfr)[FN]) {
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bfr[j] = sb[(bgi[j] * 2 + ks) * 64];
+      for (int i = 0; i < FM; ++i) read_part(t, ks, i, af, bfr);
       __builtin_amdgcn_sched_barrier(0);
     };
     // between(i): what is issued behind the products of fragment row i
@@ -314,25 +336,40 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
     // slot takes the next copies: a copy has STAGES - 1 stages' time
     auto used_up = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
     int t = 0;
-    for (; t + STAGES < n; ++t) {
-      read(t, 1, a1, b1);
-      products(a0, b0, nothing);
-      used_up();
-      wait_vmcnt<(STAGES - 2) * L>();   // stage t + 1 is there, for every wave once they met
-      meet();
-      read(t + 1, 0, a0, b0);
-      products(a1, b1, [&](int i) {
+    if constexpr (BM * BN >= 192 * 256) {   // one loop for all stages takes 24 registers fewer, which these tiles do not have
+      for (; t + 1 < n; ++t) {
+        const bool more = t + STAGES < n;
+        products(a0, b0, [&](int i) { read_part(t, 1, i, a1, b1); });
+        used_up();
+        wait_tiles<L, STAGES>(more ? STAGES - 2 : min(STAGES - 2, n - 2 - t));
+        meet();
+        products(a1, b1, [&](int i) {
+          read_part(t + 1, 0, i, a0, b0);
+          if (more)
 #pragma unroll
-        for (int c = i * L / FM; c < (i + 1) * L / FM; ++c) copy(c, t + STAGES);
-      });
-    }
-    for (; t + 1 < n; ++t) {
-      read(t, 1, a1, b1);
-      products(a0, b0, nothing);
-      wait_tiles<L, STAGES>(min(STAGES - 2, n - 2 - t));
-      meet();
-      read(t + 1, 0, a0, b0);
-      products(a1, b1, nothing);
+            for (int c = i * L / FM; c < (i + 1) * L / FM; ++c) copy(c, t + STAGES);
+        });
+      }
+    } else {
+      for (; t + STAGES < n; ++t) {
+        products(a0, b0, [&](int i) { read_part(t, 1, i, a1, b1); });
+        used_up();
+        wait_vmcnt<(STAGES - 2) * L>();   // stage t + 1 is there, for every wave once they met
+        meet();
+        products(a1, b1, [&](int i) {
+          read_part(t + 1, 0, i, a0, b0);
+#pragma unroll
+          for (int c = i * L / FM; c < (i + 1) * L / FM; ++c) copy(c, t + STAGES);
+        });
+      }
+      for (; t + 1 < n; ++t) {
+        read(t, 1, a1, b1);
+        products(a0, b0, nothing);
+        wait_tiles<L, STAGES>(min(STAGES - 2, n - 2 - t));
+        meet();
+        read(t + 1, 0, a0, b0);
+        products(a1, b1, nothing);
+      }
     }
     read(t, 1, a1, b1);
     products(a0, b0, nothing);
@@ -411,43 +448,40 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       if (i < i0 || i >= i1) continue;
-      // one fragment row's epilogue operands as one batch (residual values; the rows'
-      // positions -> (cos, sin) and KV slots): per element, between the stores they may
-      // alias, they were FN x 4 dependent round trips per fragment row
+      // a fragment row's epilogue operands as one batch (residual values; the rows' positions -> (cos, sin) and KV slots): per
+      // element, between the stores they may alias, they were FN x 4 dependent round trips per fragment row
       float resv[4][FN];
+      if constexpr (EPI == EPI_RESID) {
+        if constexpr (!RES_AHEAD) residuals(wm_, wn_, i, i + 1, res);
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) resv[jj][j] = (float)res[i][jj][j];
+      }
       float2 csv[4][FN];
       int slotv[4];
-      if constexpr (EPI == EPI_RESID || EPI == EPI_QKV_ROPE) {
+      if constexpr (EPI == EPI_QKV_ROPE) {
         int posv[4];
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
           const int m = m0 + wm_ * (BM / 2) + 16 * i + 4 * q + jj;
           posv[jj] = 0;
           slotv[jj] = -1;
-          if constexpr (EPI == EPI_QKV_ROPE)
-            if (m < M) {
-              posv[jj] = ea.pos[m];
-              slotv[jj] = ea.slots[m];
-            }
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            resv[jj][j] = 0.f;
-            if constexpr (EPI == EPI_RESID)
-              if (m < M) resv[jj][j] = (float)reinterpret_cast<const bf16*>(out)[(size_t)m * ldo + (nt_i * (BN / 16) + bg[j]) * 16 + r];
+          if (m < M) {
+            posv[jj] = ea.pos[m];
+            slotv[jj] = ea.slots[m];
           }
         }
-        if constexpr (EPI == EPI_QKV_ROPE) {
 #pragma unroll
-          for (int jj = 0; jj < 4; ++jj)
+        for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) {
-              const int g = nt_i * (BN / 16) + bg[j];
-              const int kk = g & 7;
-              const int dd = ((r < 8) ? 8 * kk + r : 64 + 8 * kk + (r - 8)) & 63;
-              const bool ok = m0 + wm_ * (BM / 2) + 16 * i + 4 * q + jj < M;
-              csv[jj][j] = ok ? ea.cs[(size_t)posv[jj] * 64 + dd] : float2{1.f, 0.f};
-            }
-        }
+          for (int j = 0; j < FN; ++j) {
+            const int g = nt_i * (BN / 16) + bg[j];
+            const int kk = g & 7;
+            const int dd = ((r < 8) ? 8 * kk + r : 64 + 8 * kk + (r - 8)) & 63;
+            const bool ok = m0 + wm_ * (BM / 2) + 16 * i + 4 * q + jj < M;
+            csv[jj][j] = ok ? ea.cs[(size_t)posv[jj] * 64 + dd] : float2{1.f, 0.f};
+          }
       }
       float scv[4];  // the rows' rstd (loads, with the operands above)
 #pragma unroll
@@ -505,7 +539,16 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int j = 0; j < FN; ++j)
           store_sc1(rsl, (int)((tile_v + ((size_t)split * FM * FN + i * FN + j) * NT + tid) * 16),
                     acc[i][j]);
+      // the tile's NWV * FM fragment rows go to the slices in equal runs (host guarantees splitk | 8), and a slice's
+      // run to its waves in shares that lie within one wave's rows
+      const int units = NWV * FM / splitk;
+      int share = (units + NWV - 1) / NWV;
+      while (FM % share || units % share) ++share;
+      const bool has = w * share < units;
+      const int unit = split * units + (has ? w * share : 0);
+      const int vw = unit / FM, i0 = unit % FM, i1 = has ? i0 + share : i0;  // whose accumulators this wave finishes
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains
+      if constexpr (EPI == EPI_RESID && RES_AHEAD) residuals(vw / WN, vw % WN, i0, i1, res);
       __syncthreads();
       if (tid == 0) {
         const unsigned g0 = __hip_atomic_load(&sp.gen[tile], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -528,14 +571,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
         }
       }
       __syncthreads();
-      // the tile's NWV * FM fragment rows go to the slices in equal runs (host guarantees splitk | 8), and a slice's
-      // run to its waves in shares that lie within one wave's rows
-      const int units = NWV * FM / splitk;
-      int share = (units + NWV - 1) / NWV;
-      while (FM % share || units % share) ++share;
-      if (w * share >= units) return;
-      const int unit = split * units + w * share;
-      const int vw = unit / FM, i0 = unit % FM, i1 = i0 + share;  // whose accumulators this wave finishes
+      if (!has) return;
       // acc is dead after the slab stores: it becomes the total (one fragment row of
       // loads in flight at a time keeps the 256x256 tile inside its register budget)
 #pragma unroll
@@ -618,6 +654,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
     // every slice has arrived: re-arm the ticket for the next launch (the workspace
     // counters are zeroed once at allocation, so no per-launch memset node is needed)
     if (tid == 0) sp.counters[tile] = 0;
+    if constexpr (EPI == EPI_RESID && RES_AHEAD) residuals(wm, wn, 0, FM, res);
   }
 
   epilogue(
@@ -628,282 +665,6 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) v
         return rstd_of(ss_row[rl]);
       },
       0, FM);
-}
-
-// ---------------------------------------------------------------------------------
-// 256 x 256 tile, phased pipeline (cdna_hip_programming.md §5 "The 256² 8-phase
-// template", re-derived for the fragment-major LDS image).  A K-tile (BK = 64) is
-// staged as four 16 KiB units -- A0/A1 (the two 64-row halves of every wave's 128
-// rows) and B0/B1 (the two 32-column halves of every wave's 64 columns) -- and
-// consumed in four phases of 16 MFMAs per wave, one C quadrant each:
-//   p0: (A0, B0)   p1: (A0, B1)   p2: (A1, B1)   p3: (A1, B0)
-// (B0 fragments stay in registers from p0 to p3).  Each phase issues ONE unit's
-// LDS-DMA (2 instructions per thread), in the order
-//   p0: A1(t+1)   p1: A0(t+2)   p2: B0(t+2)   p3: B1(t+2)
-// so a unit is re-staged one phase after its last read (behind that phase's
-// lgkmcnt(0) + barrier) and lands about five phases (> 1 K-tile) before it is
-// read: the counted vmcnt before a reading phase leaves 10 DMA instructions in
-// flight in the steady state and never drains the queue inside the loop.
-template <int EPI, bool NORM>
-__global__ __launch_bounds__(NT) void prefill_gemm8_kernel(const bf16x8* __restrict__ Wt,
-                                                           const bf16* __restrict__ X, int ldx,
-                                                           int M, int K, int m_tiles, int n_tiles,
-                                                           int up_off, void* __restrict__ out,
-                                                           int ldo, float eps, EpiArgs ea) {
-  constexpr int BM = 256, BN = 256, FM = 8, FN = 4;
-  constexpr int AB = 32, BB = 32, STAGE = (AB + BB) * 64;
-  __shared__ __attribute__((aligned(16))) bf16x8 lds[2 * STAGE];
-  const bool pre = !NORM && ea.rstd_in != nullptr;  // rows' rstd precomputed (see above)
-
-  const int nb = m_tiles * n_tiles;
-  const int b = xcd_remap(blockIdx.x, nb);
-  int mt_i, nt_i;
-  grouped_tile(b, m_tiles, n_tiles, mt_i, nt_i);
-  const int m0 = mt_i * BM;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 2, wn = w & 3;
-  const int S = K >> 5;
-  const int n = K / BK;
-
-  auto group_of = [&](int gi) -> int {
-    if constexpr (EPI == EPI_SILU) {
-      constexpr int H = BN / 32;
-      return gi < H ? nt_i * H + gi : nt_i * H + (gi - H) + up_off;
-    }
-    return nt_i * (BN / 16) + gi;
-  };
-  int bgi[FN];  // LDS B group slot of the wave's column fragment j
-#pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    if constexpr (EPI == EPI_SILU) {
-      bgi[j] = j < 2 ? wn * 2 + j : BN / 32 + wn * 2 + (j - 2);
-    } else {
-      bgi[j] = wn * FN + j;
-    }
-  }
-  // this thread's two DMA instructions of each unit: list index l = w + 8k (k = 0, 1)
-  //   A unit qa (full 128-B lines): 8 rows (l>>3)*128 + 64qa + 8(l&7) .. +7, lane ->
-  //     row + (lane>>3), LDS chunk p = lane&7 holding global chunk p ^ (row & 7)
-  //     (XOR swizzle: the A-fragment ds_read_b128 of 16 rows is conflict-free)
-  //   B unit qb: l = (wnb*2 + j2)*2 + ks -> slot of (wn = wnb, j = 2qb + j2)
-  const bf16* asrc[2][2];
-  int aslot[2][2];  // A: LDS offset in bf16x8 units
-  const bf16x8* bsrc[2][2];
-  int bslot[2][2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q)
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int l = w + 8 * k, ks = l & 1, x = l >> 1;
-      const int R = (l >> 3) * 128 + 64 * q + 8 * (l & 7) + (lane >> 3);
-      int row = m0 + R;
-      row = row < M ? row : M - 1;
-      asrc[q][k] = X + (size_t)row * ldx + 8 * ((lane & 7) ^ (R & 7));
-      aslot[q][k] = R * 8 + (lane & 7) - lane;  // + lane (per-lane DMA slot) = R*8 + p
-      const int wnb = x >> 1, j = 2 * q + (x & 1);
-      int gs;
-      if constexpr (EPI == EPI_SILU) gs = j < 2 ? wnb * 2 + j : BN / 32 + wnb * 2 + (j - 2);
-      else gs = wnb * FN + j;
-      bsrc[q][k] = Wt + ((size_t)group_of(gs) * S + ks) * 64 + lane;
-      bslot[q][k] = AB + gs * 2 + ks;
-    }
-  auto issue_a = [&](int q, int kt) {
-    bf16x8* base = lds + (kt & 1) * STAGE;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)  // wave-uniform LDS base: lane 0's slot (lane*16 B added by HW)
-      __builtin_amdgcn_global_load_lds((const void*)(asrc[q][k] + kt * BK),
-                                       (lds_ptr_t)(base + __builtin_amdgcn_readfirstlane(aslot[q][k])),
-                                       16, 0, 0);
-  };
-  auto issue_b = [&](int q, int kt) {
-    bf16x8* base = lds + (kt & 1) * STAGE;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      __builtin_amdgcn_global_load_lds((const void*)(bsrc[q][k] + (size_t)kt * 2 * 64),
-                                       (lds_ptr_t)(base + bslot[q][k] * 64), 16, 0, 0);
-  };
-  auto wait_units = [&](int units) {  // at most `units` of this thread's units in flight
-    switch (units) {
-      case 0: wait_vmcnt<0>(); break;
-      case 1: wait_vmcnt<2>(); break;
-      case 2: wait_vmcnt<4>(); break;
-      case 3: wait_vmcnt<6>(); break;
-      case 4: wait_vmcnt<8>(); break;
-      default: wait_vmcnt<10>(); break;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-  };
-
-  f32x4 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float ss[FM];
-#pragma unroll
-  for (int i = 0; i < FM; ++i) ss[i] = 0.f;
-
-  // prologue: A0 B0 B1 A1 of tile 0, A0 B0 B1 of tile 1 (the steady-state order)
-  issue_a(0, 0);
-  issue_b(0, 0);
-  issue_b(1, 0);
-  issue_a(1, 0);
-  if (n > 1) {
-    issue_a(0, 1);
-    issue_b(0, 1);
-    issue_b(1, 1);
-  }
-  bf16x8 af[4][2], bf0[2][2], bf1[2][2];
-  const int ar = lane & 15, aq = lane >> 4;
-  auto read_a = [&](const bf16x8* sa, int q) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)  // row (rg*16 + ar), global chunk 4ks + aq, swizzled
-        af[i][ks] = sa[((wm * FM + 4 * q + i) * 16 + ar) * 8 + ((4 * ks + aq) ^ (ar & 7))];
-    if constexpr (NORM) {  // RMSNorm sums: fragment i of a quadrant by wave wn == i
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (i != wn) continue;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-          ss[4 * q + i] = sumsq8(af[i][ks], ss[4 * q + i]);
-      }
-    }
-  };
-  auto read_b = [&](const bf16x8* sb, int q, bf16x8(&bfr)[2][2]) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) bfr[j][ks] = sb[(bgi[2 * q + j] * 2 + ks) * 64 + lane];
-  };
-  auto mma = [&](int qa, int qb, const bf16x8(&bfr)[2][2]) {
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[4 * qa + i][2 * qb + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              af[i][ks], bfr[j][ks], acc[4 * qa + i][2 * qb + j], 0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
-  };
-
-  for (int t = 0; t < n; ++t) {
-    const bf16x8* sa = lds + (t & 1) * STAGE;
-    const bf16x8* sb = sa + AB * 64;
-    const int more1 = t + 1 < n, more2 = t + 2 < n;
-    // p0: A0, B0
-    wait_units(2 + 3 * more1);
-    read_a(sa, 0);
-    read_b(sb, 0, bf0);
-    if (more1) issue_a(1, t + 1);
-    mma(0, 0, bf0);
-    // p1: B1 (A0 kept)
-    wait_units(1 + 4 * more1);
-    read_b(sb, 1, bf1);
-    if (more2) issue_a(0, t + 2);
-    mma(0, 1, bf1);
-    // p2: A1 (B1 kept)
-    wait_units(4 * more1 + more2);
-    read_a(sa, 1);
-    if (more2) issue_b(0, t + 2);
-    mma(1, 1, bf1);
-    // p3: (A1, B0), both in registers
-    if (more2) issue_b(1, t + 2);
-    mma(1, 0, bf0);
-  }
-  wait_vmcnt<0>();
-  __syncthreads();
-
-  float* ss_row = reinterpret_cast<float*>(lds);
-  if constexpr (NORM) {
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      if ((i & 3) != wn) continue;  // fragment i's rows were squared by wave (wm, i & 3)
-      float v = ss[i];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      if (lane < 16) ss_row[wm * (BM / 2) + 16 * i + lane] = v;
-    }
-    __syncthreads();
-  }
-  const int r = lane & 15, q = lane >> 4;
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    // one fragment row's epilogue operands as one batch (see prefill_gemm_kernel)
-    float resv[4][FN];
-    float2 csv[4][FN];
-    int slotv[4];
-    if constexpr (EPI == EPI_RESID || EPI == EPI_QKV_ROPE) {
-      int posv[4];
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int m = m0 + wm * (BM / 2) + 16 * i + 4 * q + jj;
-        posv[jj] = 0;
-        slotv[jj] = -1;
-        if constexpr (EPI == EPI_QKV_ROPE)
-          if (m < M) {
-            posv[jj] = ea.pos[m];
-            slotv[jj] = ea.slots[m];
-          }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          resv[jj][j] = 0.f;
-          if constexpr (EPI == EPI_RESID)
-            if (m < M) resv[jj][j] = (float)reinterpret_cast<const bf16*>(out)[(size_t)m * ldo + (nt_i * (BN / 16) + bgi[j]) * 16 + r];
-        }
-      }
-      if constexpr (EPI == EPI_QKV_ROPE) {
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const int g = nt_i * (BN / 16) + bgi[j];
-            const int kk = g & 7;
-            const int dd = ((r < 8) ? 8 * kk + r : 64 + 8 * kk + (r - 8)) & 63;
-            const bool ok = m0 + wm * (BM / 2) + 16 * i + 4 * q + jj < M;
-            csv[jj][j] = ok ? ea.cs[(size_t)posv[jj] * 64 + dd] : float2{1.f, 0.f};
-          }
-      }
-    }
-    float scv[4];  // the rows' precomputed rstd, loaded with the operands above
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj)
-      scv[jj] = pre ? ea.rstd_in[min(m0 + wm * (BM / 2) + 16 * i + 4 * q + jj, M - 1)] : 1.f;
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int rl = wm * (BM / 2) + 16 * i + 4 * q + jj;
-      const int m = m0 + rl;
-      const bool valid = m < M;
-      float scale = scv[jj];
-      if constexpr (NORM) scale = rsqrtf(ss_row[rl] / (float)K + eps);
-      if constexpr (EPI == EPI_SILU) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          epi_store<EPI>(m, valid, nt_i * (BN / 32) + wn * 2 + j, r, acc[i][j][jj] * scale,
-                         acc[i][j + 2][jj] * scale, out, ldo, ea);
-      } else if constexpr (EPI == EPI_QKV_ROPE) {
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          epi_store<EPI>(m, valid, nt_i * (BN / 16) + bgi[j], r, acc[i][j][jj] * scale, 0.f, out,
-                         ldo, ea, csv[jj][j], valid ? slotv[jj] : -1);
-      } else if constexpr (EPI == EPI_RESID) {
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          if (valid)
-            reinterpret_cast<bf16*>(out)[(size_t)m * ldo + (nt_i * (BN / 16) + bgi[j]) * 16 + r] =
-                f2bf(resv[jj][j] + acc[i][j][jj] * scale);
-      } else {
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          epi_store<EPI>(m, valid, nt_i * (BN / 16) + bgi[j], r, acc[i][j][jj] * scale, 0.f, out,
-                         ldo, ea);
-      }
-    }
-  }
 }
 
 // split-K workspace (device, grown on demand outside graph capture)
@@ -956,12 +717,6 @@ static int cu_count() {
   return cached[dev] > 0 ? cached[dev] : 0;
 }
 
-// Wavefronts of a tile shape: four (reads_ahead) where a workgroup has 128 rows and a CU to itself
-template <int BM, int BN>
-constexpr int waves_for() {
-  return BM == 128 && BN <= 192 ? 4 : 8;
-}
-
 // (128 x 192 leaves no registers for a reduction)
 template <int BM, int BN>
 constexpr bool splits_k() {
@@ -969,41 +724,24 @@ constexpr bool splits_k() {
 }
 
 // LDS stages per tile shape.  Measured on MI355X (bench/prefill_gemm_bench.py): the
-// 64-row tiles are latency-bound streams and want 3-4 stages in flight; tiles of 128 rows and more
-// on eight waves are MFMA-bound at large M, where two blocks share a CU and hide each other's
-// loads, and lose more to 1-block/CU occupancy than they gain from depth; those that read ahead have
-// the CU's LDS to themselves.
+// 64-row tiles are latency-bound streams and want 3-4 stages in flight; those that read ahead have the CU's LDS to
+// themselves.
 template <int BM, int BN>
 constexpr int stages_for() {
-  if constexpr (reads_ahead<BM, BN, waves_for<BM, BN>()>()) return (160 * 1024) / ((BM + BN) * BK * 2);
-  if constexpr (BM >= 128) return 2;
+  constexpr int most = (160 * 1024) / ((BM + BN) * BK * 2);
+  if constexpr (reads_ahead<BM, BN, most, false>()) return most;
   return BN <= 128 ? 4 : 3;
 }
 
-// Deep variant for grids of at most one block per CU (mid-M prompts, split-K tiles): one
-// resident block per CU is bound by its own bytes in flight (Little's law: one 128x128
-// stage is 32 KiB, a k-tile's MFMAs take ~0.05 us, an L2/MALL round trip ~1.5 us), so the
-// block keeps as many stages in flight as 160 KiB of LDS holds.
-// The 64-row tiles already run 3-4 stages and measured 4-9 % slower with 4-6
-// (profiles/r2_prefill_gemm_deep_stages.jsonl): deep applies from 128 rows.
-template <int BM, int BN>
-constexpr int deep_stages_for() {
-  if constexpr (BM < 128 || reads_ahead<BM, BN, waves_for<BM, BN>()>()) return stages_for<BM, BN>();
-  constexpr int stage_bytes = (BM + BN) * BK * 2;
-  constexpr int most = (160 * 1024) / stage_bytes;
-  return most > 6 ? 6 : (most < 2 ? 2 : most);
-}
-
-// 0 = shallow stages only, 1 = deep variant when the grid is <= one block per CU (default),
-// 2 = deep variant always (A/B).
-static int g_deep = 1;
+// 1: K slices fill one round of the CUs where a tile has a CU to itself; 0, 2 (A/B): some 400 workgroups whatever the tile
+static int g_fill = 1;
 
 template <int BM, int BN, int EPI, bool NORM, int STAGES>
 int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_tiles, int n_tiles,
                   int up_off, void* out, int ldo, float eps, const EpiArgs& ea, hipStream_t st,
                   int splitk, char* ws, int par) {
-  constexpr int NWV = waves_for<BM, BN>();
-  constexpr size_t SHM = reads_ahead<BM, BN, NWV>() ? (size_t)STAGES * (BM + BN) * BK * sizeof(bf16) : 0;
+  constexpr int NWV = 8;
+  constexpr size_t SHM = reads_ahead<BM, BN, STAGES, NORM>() ? (size_t)STAGES * (BM + BN) * BK * sizeof(bf16) : 0;
   const int tiles = m_tiles * n_tiles;
   auto with_lds = [](const void* k) {
     return SHM ? hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SHM) : hipSuccess;
@@ -1037,27 +775,27 @@ int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_ti
 template <int BM, int BN, int EPI, bool NORM>
 int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off, void* out,
            int ldo, float eps, const EpiArgs& ea, hipStream_t st) {
-  constexpr int SHALLOW = stages_for<BM, BN>();
-  constexpr int DEEP = deep_stages_for<BM, BN>();
+  constexpr int STAGES = stages_for<BM, BN>();
   const int m_tiles = (M + BM - 1) / BM;
   const int n_tiles = N / BN;
   const int tiles = m_tiles * n_tiles;
   const int nk = K / BK;
   const int cus = cu_count();
-  constexpr bool ALONE = reads_ahead<BM, BN, waves_for<BM, BN>()>();   // one workgroup per CU whatever the grid
-  const bool deep_auto = (DEEP > SHALLOW || ALONE) && g_deep == 1 && cus > 0 && tiles <= cus;
+  constexpr bool ALONE = BM >= 128 && BM * BN <= 128 * 256;   // one workgroup per CU whatever the grid
+  const bool fill = ALONE && g_fill == 1 && cus > 0 && tiles <= cus;
   // too few tiles to fill 256 CUs: split K so every CU gets work (>= 4 k-tiles per slice)
   // (measured on MI355X at 8B shapes: ~400 blocks, >= 16 k-tiles per slice); the deep
   // variant keeps the grid at one block per CU instead (power-of-two slices <= CUs/tiles)
   int splitk;
   if (g_splitk) {
     splitk = g_splitk;
-  } else if (deep_auto) {
+  } else if (fill) {
     const int cap = std::min(8, std::max(1, std::min(cus / tiles, nk / 16)));
     splitk = 1;
     while (splitk * 2 <= cap) splitk *= 2;
   } else {
-    splitk = std::min(8, std::max(1, std::min(400 / tiles, nk / 16)));
+    // (256 x 256: from 160 tiles on they fill the chip as they are)
+    splitk = BM * BN == 256 * 256 && tiles >= 160 ? 1 : std::min(8, std::max(1, std::min(400 / tiles, nk / 16)));
   }
   splitk = splits_k<BM, BN>() ? std::max(1, std::min(splitk, nk / 4)) : 1;
   char* ws = nullptr;
@@ -1070,26 +808,7 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
   } else {
     splitk = 1;
   }
-  const bool deep = DEEP > SHALLOW && (g_deep == 2 || (g_deep == 1 && cus > 0 && tiles * splitk <= cus));
-  if constexpr (DEEP > SHALLOW) {
-    if (deep)
-      return launch_stages<BM, BN, EPI, NORM, DEEP>(Wt, X, ldx, M, K, m_tiles, n_tiles, up_off, out,
-                                                    ldo, eps, ea, st, splitk, ws, par);
-  }
-  return launch_stages<BM, BN, EPI, NORM, SHALLOW>(Wt, X, ldx, M, K, m_tiles, n_tiles, up_off, out,
-                                                   ldo, eps, ea, st, splitk, ws, par);
-}
-
-static int g_phased = 1;  // 256x256 tiles: phased pipeline (1) or the 2-stage kernel (0)
-
-template <int EPI, bool NORM>
-int launch_phased(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off,
-                  void* out, int ldo, float eps, const EpiArgs& ea, hipStream_t st) {
-  const int m_tiles = (M + 255) / 256, n_tiles = N / 256;
-  hipLaunchKernelGGL((prefill_gemm8_kernel<EPI, NORM>), dim3(m_tiles * n_tiles), dim3(NT), 0, st,
-                     (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off, out,
-                     ldo, eps, ea);
-  return (int)hipGetLastError();
+  return launch_stages<BM, BN, EPI, NORM, STAGES>(Wt, X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, st, splitk, ws, par);
 }
 
 // 128 x 128 tiles of eight wavefronts and two stages, of which a CU takes two
@@ -1107,11 +826,7 @@ template <int EPI, bool NORM>
 int launch_tile(int tile, const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off,
                 void* out, int ldo, float eps, const EpiArgs& ea, hipStream_t st) {
   switch (tile) {
-    case 1:
-      // the phased kernel has no split-K: take it where the tiles already fill the chip
-      if (g_phased && (g_splitk == 1 || (!g_splitk && ((M + 255) / 256) * (N / 256) >= 160)))
-        return launch_phased<EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
-      return launch<256, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
+    case 1: return launch<256, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 2: return launch<128, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 3: return launch<128, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 4: return launch<64, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
@@ -1159,7 +874,7 @@ static int pick_tile(int M, int N, int K, int epi) {
   if (N >= 16384 && M > 128 && M <= 192) return 7;   // one row of tiles, 192 x 128: SwiGLU 28672 x 4096 62 us, 128 x 128 81
   // A residual product with a short K that gives 160 tiles of 256 x 256 and more waits for its residual and its first and last
   // stages: pairs of workgroups per CU hide that, but where the larger tiles' last round fills the CUs and K gives them time.
-  // us, pairs / 128 x 256 / phased 256 x 256: 8192 x 1024, 2048 rows 59 / 68 / 62, 8192 x 3072, 2048 rows 115 / 117 / 110,
+  // us, pairs / 128 x 256 / 256 x 256: 8192 x 1024, 2048 rows 59 / 68 / 62, 8192 x 3072, 2048 rows 115 / 117 / 110,
   // 1500 rows 93 / 106 / 104, 6144 x 2048, 4096 rows 124 / 131 / 160
   if (resid && K <= 3072 && N % 256 == 0 && tiles(256, 256) >= 160) {
     const long last = tiles(256, 256) % cus;
@@ -1167,13 +882,13 @@ static int pick_tile(int M, int N, int K, int epi) {
   }
   if (N % 256 == 0 && !(resid && K <= 3072)) {
     // More than a round of 128 x 128: the tile whose rounds of the CUs take the shortest time.  Relative times of a round,
-    // from SwiGLU of 16384 to 36864 columns and K = 2048 and 4096 (us at 4096, phased 256 x 256 / 192 x 256 / 128 x 256 /
+    // from SwiGLU of 16384 to 36864 columns and K = 2048 and 4096 (us at 4096, 256 x 256 / 192 x 256 / 128 x 256 /
     // 192 x 128; in brackets what the lines by rows before had): 28672 columns, 250 rows 126 / 95 / 68 / 91 [85], 300 rows
     // 107 / 94 / 108 / - [100], 512 rows 113 / 174 / 119 / 145 [119], 600 rows 202 / 179 / 161 / 174 [190], 1024 rows 211 /
     // 257 / 225 / - [213]; 22016 columns, 300 rows 104 / 130 / 98 / 85 [104], 600 rows 198 / 174 / 116 / 141 [188]; 36864
     // columns, 300 rows 203 / 176 / 116 / 145 [194]; 12288 x 2048, 400 rows 58 / - / 32 / 44 [43], 700 rows 98 / - / 57 /
     // 49 [79].  128 x 192, without SwiGLU: 6144 x 4096, 700 rows 46, 128 x 256 51, 192 x 128 52.  192 x 256 up to 200 tiles:
-    // launch() cuts K there as well (22016 columns above); phased: from 160 tiles (profiles/r2_prefill_gemm_phased.jsonl).
+    // launch() cuts K there as well (22016 columns above); 256 x 256 from 160 tiles.
     auto time = [&](int bm, int bn, int round) { return (tiles(bm, bn) + cus - 1) / cus * round; };
     int best = 2;
     long t = time(128, 256, 57);

@@ -201,17 +201,13 @@ static int g_tiled_version = 2;  // 2 = LDS-DMA 8-wave kernel (prefill_gemm.h), 
 // Benchmarks / A-B tests (p2p_tiled_gemm_config): version 1|2, tile 0 (heuristic) or 1..9 (256x256, 128x256, 128x128,
 // 64x128, 64x256, 128x128 two to a CU, 192x128, 192x256, 128x192),
 // splitk 0 (heuristic), 1 (off) or a forced K-slice count.
-// 256x256 prefill tiles: 1 = phased pipeline (default), 0 = the 2-stage kernel (A/B).
-P2P_API void p2p_prefill_phased(int on) { pgemm::g_phased = on ? 1 : 0; }
-
-// Deep LDS pipeline (A/B): 0 = shallow stages only, 1 = deep variant for grids of at most
-// one block per CU (default), 2 = deep variant always.
+// K slices of tiles that have a CU to themselves (A/B): 1 = a round of the CUs (default), 0 and 2 = some 400 workgroups.
+P2P_API void p2p_prefill_deep(int mode) { pgemm::g_fill = (mode >= 0 && mode <= 2) ? mode : 1; }
 // Precomputed per-row rstd for normed prefill GEMMs (A/B): 1 = on (default), 0 = in-loop sums.
 P2P_API void p2p_prefill_pre_rstd(int on) { pgemm::g_pre_rstd = on ? 1 : 0; }
 // 192 x 256 tiles where their rounds are the shortest (A/B): 1 = on (default)
 P2P_API void p2p_prefill_tile8(int on) { pgemm::g_tile8 = on ? 1 : 0; }
 
-P2P_API void p2p_prefill_deep(int mode) { pgemm::g_deep = (mode >= 0 && mode <= 2) ? mode : 1; }
 
 // Split-K reduction mode (A/B): 1 = parallel (every slice reduces a share, default where
 // residency allows), 0 = serial (the last arriving slice reduces the whole tile).
