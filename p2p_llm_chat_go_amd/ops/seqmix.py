@@ -52,7 +52,7 @@ _SIGS = {
     "p2p_sm_skinny": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                       c_void_p],
     "p2p_sm_prompt_gemm": [c_void_p, c_void_p, c_long, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
-                           c_int, c_float, c_float, c_int, c_void_p],
+                           c_int, c_float, c_float, c_int, c_int, c_void_p],
     "p2p_sm_skinny_logits": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_int,
                              c_void_p],
     "p2p_sm_skinny_conv": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
@@ -448,14 +448,19 @@ def _conv_args(M: int, N: int, dtype, c0: int, cw, cb, tail, ent, out):
 
 
 def _prompt_gemm_ok(x, w, b=None) -> bool:
-    """Products that ``csrc/seqmix/prompt_gemm.hip`` takes: bf16, K in steps of 64, rows that 16-byte copies can read."""
-    if x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda \
-            or x.device != w.device or x.requires_grad or w.requires_grad:
+    """Products that ``csrc/seqmix/prompt_gemm.h`` takes: K in stages of 128 bytes, rows that 16-byte copies can read."""
+    if x.dim() != 2 or w.dim() != 2 or x.dtype != w.dtype or not x.is_cuda or x.device != w.device or x.requires_grad \
+            or w.requires_grad:
         return False
     (M, K), ld = x.shape, x.stride(0)
-    return (M > 0 and K >= 64 and K % 64 == 0 and w.shape[1] == K and w.is_contiguous() and x.stride(1) == 1 and ld >= K
-            and ld % 8 == 0 and ld < 1 << 22 and K * (w.shape[0] + 256) < 1 << 30
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    if x.dtype == torch.bfloat16:
+        ok = K % 64 == 0 and ld % 8 == 0
+    elif x.dtype == torch.float32:
+        ok = K % 32 == 0 and ld % 4 == 0
+    else:
+        return False
+    return (ok and M > 0 and K > 0 and w.shape[1] == K and w.is_contiguous() and x.stride(1) == 1 and ld >= K
+            and ld < 1 << 21 and K * (w.shape[0] + 256) < 1 << 29 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and (b is None or b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and not b.requires_grad))
 
 
@@ -463,7 +468,7 @@ def _prompt_gemm(x, w, b, out, tanh_from=None, act: int = -1, limit: float = 0.0
     M, N = out.shape
     _chk(lib().p2p_sm_prompt_gemm(x.data_ptr(), _lib.ptr(rows), (x.shape[0] - 1) * x.stride(0) + x.shape[1], x.stride(0),
                                   w.data_ptr(), _lib.ptr(b), out.data_ptr(), out.stride(0), M, N, x.shape[1],
-                                  N if tanh_from is None else tanh_from, act, limit, alpha, tile, _st(x)), "prompt_gemm")
+                                  N if tanh_from is None else tanh_from, act, limit, alpha, tile, _f32(x), _st(x)), "prompt_gemm")
     return out
 
 
@@ -476,10 +481,10 @@ def linear(x, w, b=None, tanh_from=None, rows=None):
     wait for the host; and it is slower itself, by 20 % on average over 192 to 16384 columns, K 128 to 8192 and 20 to 2644
     rows (10304 x 2048, 2048 rows 100 -> 84 us, 2048 x 8192, 2048 rows 82 -> 65, 2048 x 2048, 48 rows 8.6 -> 5.0; one of the few
     the other way: 8192 x 2048, 1300 rows 43.5 -> 46).  8 rows of shapes that ``_skinny`` leaves: 2048 x 8192 11.2 -> 10.6, 96 x
-    4096 8.0 -> 6.1, 6144 x 3072 10.9 -> 8.6, 32000 x 4096 58 -> 51."""
+    4096 8.0 -> 6.1, 6144 x 3072 10.9 -> 8.6, 32000 x 4096 58 -> 51.  float32: 5 % (prompt_gemm_f32.hip)."""
     if rows is not None:
         if (x.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and rows.shape[0] > 0 and b is None
-                and tanh_from is None and x.shape[0] * x.stride(0) < 1 << 30 and _prompt_gemm_ok(x, w)):
+                and tanh_from is None and x.shape[0] * x.stride(0) < 1 << 29 and _prompt_gemm_ok(x, w)):
             return _prompt_gemm(x, w, None, torch.empty(rows.shape[0], w.shape[0], device=x.device, dtype=x.dtype), rows=rows)
         x = x.index_select(0, rows)
     if isinstance(x, NormedRows):
@@ -490,8 +495,12 @@ def linear(x, w, b=None, tanh_from=None, rows=None):
     if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
             b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
         if _prompt_gemm_ok(x, w, b):
-            return _prompt_gemm(x, w, b, torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype), tanh_from)
-        y = F.linear(x, w, b)
+            y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
+            if x.dtype == torch.bfloat16:
+                return _prompt_gemm(x, w, b, y, tanh_from)
+            _prompt_gemm(x, w, b, y)   # (float32: the pass has the better tanh)
+        else:
+            y = F.linear(x, w, b)
         if tanh_from is not None:
             tanh_(y[:, tanh_from:])
         return y

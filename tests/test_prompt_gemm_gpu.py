@@ -10,10 +10,10 @@ DEV = "cuda:0"
 TILES = 14
 
 
-def _case(M, N, K, ld=None, seed=0):
+def _case(M, N, K, ld=None, seed=0, dtype=torch.bfloat16):
     g = torch.Generator(device=DEV).manual_seed(seed + M * 7 + N)
-    x = torch.randn(M, ld or K, generator=g, device=DEV).bfloat16()[:, :K]
-    return x, (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    x = torch.randn(M, ld or K, generator=g, device=DEV).to(dtype)[:, :K]
+    return x, (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).to(dtype)
 
 
 def _close(got, ref):
@@ -60,6 +60,30 @@ def test_units(tile, act, limit):
     assert ((out.double() - want).norm() / want.norm()).item() < 2.0 ** -8
     got = sm.linear_unit(x, 3 * w, torch.empty_like(out), act, limit)
     assert ((got.double() - want).norm() / want.norm()).item() < 2.0 ** -8
+
+
+# fp32 sums of K products: against the library's sums of the same inputs, of which neither has another order's rounding on its
+# side (a chain of K / 4 sums each: their errors are alike, and twice the library's is far outside of what orders do)
+@pytest.mark.parametrize("tile", range(10))
+@pytest.mark.parametrize("M,N,K,ld", [(1, 8, 32, 32), (31, 100, 64, 68), (129, 132, 224, 224), (200, 77, 1056, 1060), (300, 520, 512, 512)])
+def test_float32(tile, M, N, K, ld):
+    x, w = _case(M, N, K, ld, dtype=torch.float32)
+    b = torch.randn(N, device=DEV)
+    ref = x.double() @ w.double().t() + b.double()
+    lib = ((F.linear(x, w, b).double() - ref).norm() / ref.norm()).item()
+    for shift in (0, 1):
+        whole = torch.full((M + 2, N + 8), 9.0, device=DEV)
+        out = whole[1:M + 1, shift:shift + N]
+        sm._prompt_gemm(x, w, b, out, tile=tile)
+        assert ((out.double() - ref).norm() / ref.norm()).item() <= 2 * lib + 6e-8
+        out.fill_(9.0)
+        assert bool((whole == 9.0).all())
+    if tile in (1, 7) or N % 2:
+        return
+    h = N // 2
+    want = F.silu(ref[:, :h] - b[:h].double()) * (ref[:, h:] - b[h:].double())
+    out = sm._prompt_gemm(x, w, None, torch.empty(M, h, device=DEV), act=0, tile=tile)
+    assert ((out.double() - want).norm() / want.norm()).item() < 1e-6
 
 
 def test_rows_and_other_rows():
