@@ -490,14 +490,15 @@ expert_gemm_mfma_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
 // fp32: four v_mfma_f32_16x16x4_f32, component by component.
 //
 // Bound by LDS reads and the copies' latency (two or three blocks per CU) and by the last round of the CUs.  8 experts,
-// 4096 slots, width 2048, gate and up of 1024: 50 us (690 TFLOP/s) and 29 us for the two products (160 rows) against 229 and
+// 4096 slots, width 2048, gate and up of 1024: 49 us (700 TFLOP/s) and 28 us for the two products (160 rows; 50 and 29 with one
+// number per store) against 229 and
 // 117 with register staging, one step at a time; 1212 slots at width 1024: 10.7 and 8.7 us (64 x 64 tiles) against 53
 // and 29; fp32, 1012 slots, width 1024 and 512: 37 and 21 us against 185 and 94 on vector instructions.
 template <typename T, int BM, int BN>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
 expert_gemm_tile_k(const T* __restrict__ x, int ldx, int x_div, const T* __restrict__ w,
                    const int* __restrict__ cnt, const int* __restrict__ rows, int ldr, T* __restrict__ out, int ldo,
-                   int N, int K, int E, int TMP, int epi, float limit, float alpha) {
+                   int N, int K, int E, int TMP, int epi, float limit, float alpha, int wide) {
   constexpr int EP = 16 / sizeof(T), KS = 8 * EP;          // numbers per piece, per step
   constexpr int FM = BM / 32, FN = BN / 32;                // 16 x 16 tiles of a wavefront
   constexpr int STAGE = (BM + BN) * 128;
@@ -569,30 +570,43 @@ expert_gemm_tile_k(const T* __restrict__ x, int ldx, int x_div, const T* __restr
       for (int a = 0; a < FM; a++)
         if (a < nmt) {
 #pragma unroll
-          for (int b = 0; b < FN; b++) acc[a][b] = mfma_piece<T>(af[kk][a], bf[kk][b], acc[a][b]);
+          for (int b = 0; b < FN; b++) acc[a][b] = mfma_piece<T>(bf[kk][b], af[kk][a], acc[a][b]);   // (see the stores)
         }
   }
+  // The weight rows are the products' left operand, so a lane ends with four neighbouring columns of one slot: one store for
+  // them, and little code behind the products (it is run once per tile, from memory).
 #pragma unroll
   for (int a = 0; a < FM; a++) {
     if (a >= nmt) continue;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int so = sslot[wm + a * 16 + quad * 4 + i];
-      if (so < 0) continue;
-      if (epi == 1 || epi == 3) {
-#pragma unroll
-        for (int b = 0; b < FN; b += 2) {
-          const int n = n0 + wn + b * 16;
-          if (n + 16 + n16 < N)
-            stf(out, (size_t)so * ldo + n / 2 + n16, glu_epi(acc[a][b][i], acc[a][b + 1][i], epi, limit, alpha));
-        }
-        continue;
+    const int so = sslot[wm + a * 16 + n16];
+    if (so < 0) continue;
+    T* o = out + (size_t)so * ldo;
+    auto put = [&](int n, int end, const float (&v)[4]) {
+      if (wide && n + 3 < end) {
+        stv<4>(o, n, v);
+        return;
       }
 #pragma unroll
-      for (int b = 0; b < FN; b++) {
-        const int n = n0 + wn + b * 16 + n16;
-        if (n < N) stf(out, (size_t)so * ldo + n, plain_epi(acc[a][b][i], epi));
+      for (int i = 0; i < 4; i++)
+        if (n + i < end) stf(o, n + i, v[i]);
+    };
+    if (epi == 1 || epi == 3) {
+#pragma unroll
+      for (int b = 0; b < FN; b += 2) {
+        const int n = n0 + wn + b * 16;            // (N is a multiple of 32)
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = glu_epi(acc[a][b][i], acc[a][b + 1][i], epi, limit, alpha);
+        put(n / 2 + quad * 4, N / 2, v);
       }
+      continue;
+    }
+#pragma unroll
+    for (int b = 0; b < FN; b++) {
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = plain_epi(acc[a][b][i], epi);
+      put(n0 + wn + b * 16 + quad * 4, N, v);
     }
   }
 }
@@ -674,7 +688,8 @@ static int launch_expert_tile(const void* x, int ldx, int x_div, const void* w, 
     if (e != hipSuccess) return (int)e;
   }
   hipLaunchKernelGGL((expert_gemm_tile_k<T, BM, BN>), dim3(tmp * ((N + BN - 1) / BN)), dim3(256), shm, st, (const T*)x,
-                     ldx, x_div, (const T*)w, cnt, rows, ldr, (T*)out, ldo, N, K, E, tmp, epi, limit, alpha);
+                     ldx, x_div, (const T*)w, cnt, rows, ldr, (T*)out, ldo, N, K, E, tmp, epi, limit, alpha,
+                     ldo % 4 == 0 && (size_t)out % (4 * sizeof(T)) == 0);
   return (int)hipGetLastError();
 }
 
