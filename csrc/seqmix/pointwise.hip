@@ -108,7 +108,50 @@ __global__ void copy_words_k(const int* src, int* dst, int n) {
   __hip_atomic_store(dst + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// What a step's layers derive from its entries (row0, n, start, slot), formed on the device: a copy of it from the host waits for
+// all that is under way, and the layers behind it for the host (a prompt of 40 rows, two or three of them: Regesun 893 -> 827 us,
+// Rasepel 880 -> 836, Tarunex 760 -> 719).  Entries of
+// `least` rows and more are cut into pieces of at most `size` consecutive rows: (row, rows) to units, or (row, rows, 1, piece) to
+// pieces and (first piece, pieces, start, slot) to whole; shorter ones go to rest as they are.
+__global__ void __launch_bounds__(256) step_tables_k(const int4* __restrict__ ent, int E, int size, int least, int2* __restrict__ units,
+                                                     int4* __restrict__ pieces, int4* __restrict__ whole, int4* __restrict__ rest) {
+  __shared__ int4 s[256];
+  int p0 = 0, w = 0, r = 0;   // pieces, whole and other entries so far
+  for (int base = 0; base < E; base += 256) {
+    __syncthreads();
+    if (base + (int)threadIdx.x < E) s[threadIdx.x] = ent[base + threadIdx.x];
+    __syncthreads();
+    for (int i = 0; i < min(256, E - base); i++) {
+      const int4 e = s[i];
+      if (e.y < least) {
+        if (threadIdx.x == 0) rest[r] = e;
+        r++;
+        continue;
+      }
+      const int n = (e.y + size - 1) / size;
+      for (int k = threadIdx.x; k < n; k += 256) {
+        const int row = e.x + k * size, rows = min(size, e.y - k * size);
+        if (units) units[p0 + k] = make_int2(row, rows);
+        else pieces[p0 + k] = make_int4(row, rows, 1, p0 + k);
+      }
+      if (!units && threadIdx.x == 0) whole[w] = make_int4(p0, n, e.z, e.w);
+      p0 += n, w++;
+    }
+  }
+}
+
 extern "C" {
+
+// units, or pieces, whole and rest (which may be null where no entry is shorter than `least`): see step_tables_k
+int p2p_sm_step_tables(const int* ent, int E, int size, int least, int* units, int* pieces, int* whole, int* rest, hipStream_t st) {
+  if (E <= 0) return 0;
+  if (size < 1 || (units ? least > 0 : !pieces || !whole) || (size_t)ent % 16 || (size_t)units % 8 ||
+      ((size_t)pieces | (size_t)whole | (size_t)rest) % 16)
+    return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(step_tables_k, dim3(1), dim3(256), 0, st, (const int4*)ent, E, size, least, (int2*)units, (int4*)pieces,
+                     (int4*)whole, (int4*)rest);
+  return (int)hipGetLastError();
+}
 
 int p2p_sm_copy_words(const int* src, int* dst, int n, hipStream_t st) {
   if (n <= 0) return 0;

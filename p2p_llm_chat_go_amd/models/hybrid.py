@@ -328,8 +328,7 @@ class StepBatch:
         """Row groups for the matrix-core attention kernel (``ops.seqmix.make_units``)."""
         u = self._units.get(rows_per_wave)
         if u is None:
-            u = self._units[rows_per_wave] = sm.make_units(self.ent_host, rows_per_wave).to(
-                self.ids.device)
+            u = self._units[rows_per_wave] = sm.device_units(self.ent_host, rows_per_wave, self.ent)
         return u
 
     def attn_units(self, rows_per_wave: int, shared: bool = True, latent: int = 0):

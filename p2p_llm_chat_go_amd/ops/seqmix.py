@@ -116,6 +116,7 @@ _SIGS = {
                         c_long, c_long, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                         c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                         c_int, c_int, c_int, c_void_p],
+    "p2p_sm_step_tables": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
     "p2p_sm_copy_words": [c_void_p, c_void_p, c_int, c_void_p],
     "p2p_sm_tanh": [c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "p2p_sm_sigmoid_gate": [c_void_p, c_long, c_long, c_void_p, c_int, c_void_p, c_int, c_int,
@@ -937,15 +938,36 @@ class Entries(list):
         self.tables = {}
 
 
-def chunk_tables(ent_host: list, chunk: int, device):
-    """``scan_chunks`` on the device, in one copy (kept with the step when it is an ``Entries``)."""
+def _on_device(ent, ent_host) -> bool:
+    """ent holds ent_host where a kernel can read it (``p2p_sm_step_tables``)."""
+    return (ent is not None and ent.is_cuda and ent.dtype == torch.int32 and ent.is_contiguous() and ent.shape == (len(ent_host), 4)
+            and ent.data_ptr() % 16 == 0)
+
+
+def _step_tables(ent, ent_host, chunk: int, least: int):
+    """``scan_chunks`` of the entries of at least ``least`` rows and the others as they are, formed on the device."""
+    whole = [e[1] for e in ent_host if e[1] >= least]
+    V, E = sum((n + chunk - 1) // chunk for n in whole), len(whole)
+    out = torch.empty(V + len(ent_host), 4, device=ent.device, dtype=torch.int32)
+    v, c, rest = out[:V], out[V:V + E], out[V + E:]
+    _chk(lib().p2p_sm_step_tables(ent.data_ptr(), len(ent_host), chunk, least, None, v.data_ptr(), c.data_ptr(), rest.data_ptr(),
+                                  _st(ent)), "step_tables")
+    return v, c, rest
+
+
+def chunk_tables(ent_host: list, chunk: int, device, ent=None):
+    """``scan_chunks`` on the device (kept with the step when it is an ``Entries``); ent: the entries there, which spare the
+    copy."""
     kept = getattr(ent_host, "tables", None)
     key = (chunk, str(device))
     if kept is not None and key in kept:
         return kept[key]
-    vent, cent = scan_chunks(ent_host, chunk)
-    both = torch.cat([vent, cent]).to(device)
-    out = both[:vent.shape[0]], both[vent.shape[0]:]
+    if _on_device(ent, ent_host):
+        out = _step_tables(ent, ent_host, chunk, 0)[:2]
+    else:
+        vent, cent = scan_chunks(ent_host, chunk)
+        both = torch.cat([vent, cent]).to(device)
+        out = both[:vent.shape[0]], both[vent.shape[0]:]
     if kept is not None:
         kept[key] = out
     return out
@@ -955,18 +977,22 @@ def _chunked(ent_host) -> bool:
     return SCAN_CHUNK > 0 and max(e[1] for e in ent_host) >= 2 * SCAN_CHUNK
 
 
-def portion_tables(ent_host: list, chunk: int, least: int, device):
+def portion_tables(ent_host: list, chunk: int, least: int, device, ent=None):
     """``chunk_tables`` of the portions of at least ``least`` tokens, and the other portions as entries (None where
     there are none), which walk in a launch of their own."""
     kept = getattr(ent_host, "tables", None)
     key = (chunk, least, str(device))
     if kept is not None and key in kept:
         return kept[key]
-    vent, cent = scan_chunks([e for e in ent_host if e[1] >= least], chunk)
-    short = [tuple(e) for e in ent_host if e[1] < least]
-    V, E = vent.shape[0], cent.shape[0]
-    every = torch.cat([vent, cent, torch.tensor(short, dtype=torch.int32).view(-1, 4)]).to(device)
-    out = every[:V], every[V:V + E], every[V + E:] if short else None
+    if _on_device(ent, ent_host) and any(e[1] >= least for e in ent_host):
+        v, c, rest = _step_tables(ent, ent_host, chunk, least)
+        out = v, c, rest if rest.shape[0] else None
+    else:
+        vent, cent = scan_chunks([e for e in ent_host if e[1] >= least], chunk)
+        short = [tuple(e) for e in ent_host if e[1] < least]
+        V, E = vent.shape[0], cent.shape[0]
+        every = torch.cat([vent, cent, torch.tensor(short, dtype=torch.int32).view(-1, 4)]).to(device)
+        out = every[:V], every[V:V + E], every[V + E:] if short else None
     if kept is not None:
         kept[key] = out
     return out
@@ -1058,7 +1084,7 @@ def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: 
         raise ValueError("gdelta_scan: head size %d > 256" % D)
     least = _gdelta_portions(ent_host, H, D)
     if least > 0:
-        vent, cent, ent = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, r.device)
+        vent, cent, ent = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, r.device, ent)
         tmp = torch.empty(4, vent.shape[0], H, 64, 64, device=r.device, dtype=torch.float32)
         _chk(lib().p2p_sm_gdelta_chunk(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), a.data_ptr(), ld,
@@ -1068,7 +1094,7 @@ def gdelta_scan(r, k, v, g, a, lo, w0, ab, normw, state, ent, ent_host, out, H: 
         if ent is None:
             return out
     elif _chunked(ent_host):
-        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, r.device)
+        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, r.device, ent)
         tmp = torch.empty(3, vent.shape[0], H, D, D, device=r.device, dtype=torch.float32)
         _chk(lib().p2p_sm_gdelta_scan_chunked(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), a.data_ptr(), ld,
@@ -1192,7 +1218,7 @@ def mamba_scan(conv, zx, xoff: int, dtoff: int, dt_bias, A_log, Dp, state, tail,
     walk, first = ent, 20.0 + 0.001 * N * P
     least = matrix_portions(ent_host, H, first, first, 1.3e-5 * N * P, 2.1 if N * P > 32768 else 0.8)
     if least > 0:
-        vent, cent, walk = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, zx.device)
+        vent, cent, walk = portion_tables(ent_host, min(SCAN_CHUNK, LIGHT_CHUNK), least, zx.device, ent)
         NV = vent.shape[0]
         # one buffer: the products of B and C that heads share (a group's 64 x 64 per chunk), the portions' states, their decays
         shared, states = NV * G * 64 * 64 if H > G else 0, NV * H * N * P
@@ -1268,7 +1294,7 @@ def selective_scan(x, xp, rank: int, wdt, dt_bias, A2, Dp, z, state, ent, ent_ho
     vent = cent = tmp = dtsum = None
     NV = 0
     if _chunked(ent_host):
-        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, y.device)
+        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, y.device, ent)
         NV = vent.shape[0]
         tmp = torch.empty(NV, N, I, device=y.device, dtype=torch.float32)
         dtsum = torch.empty(NV, I, device=y.device, dtype=torch.float32)
@@ -1301,6 +1327,17 @@ def make_units(ent_host: list, rows_per_wave: int) -> torch.Tensor:
     u = [(r, min(rows_per_wave, row0 + n - r)) for row0, n, _s, _sl in ent_host
          for r in range(row0, row0 + n, rows_per_wave)]
     return torch.tensor(u, dtype=torch.int32).view(-1, 2)
+
+
+def device_units(ent_host: list, rows_per_wave: int, ent) -> torch.Tensor:
+    """``make_units`` on the device of ent, the entries there."""
+    if not _on_device(ent, ent_host):
+        return make_units(ent_host, rows_per_wave).to(ent.device)
+    U = sum((e[1] + rows_per_wave - 1) // rows_per_wave for e in ent_host)
+    out = torch.empty(U, 2, device=ent.device, dtype=torch.int32)
+    _chk(lib().p2p_sm_step_tables(ent.data_ptr(), len(ent_host), rows_per_wave, 0, out.data_ptr(), None, None, None, _st(ent)),
+         "step_tables")
+    return out
 
 
 def latent_mfma_ok(qa, cache) -> bool:
@@ -2162,7 +2199,7 @@ def hgrn2_scan(proj, lower, fb, normw, state, ent, ent_host, out, H: int, D: int
     _vec(normw, V, "normw")
     _scan_state_ok(state, H, D, V, ent)
     if _chunked(ent_host):
-        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, proj.device)
+        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, proj.device, ent)
         NV = vent.shape[0]
         cs = torch.empty(NV, H, D, V, device=proj.device, dtype=torch.float32)
         cd = torch.empty(NV, H, D, device=proj.device, dtype=torch.float32)
@@ -2218,7 +2255,7 @@ def gla_scan(proj, low0: int, rank: int, wa2, za, inv_tau: float, normw, state, 
     NV = 0
     matrix = max(D, V) <= GLA_MAX
     if max(e[1] for e in ent_host) >= GLA_MIN if matrix else _chunked(ent_host):
-        vent, cent = chunk_tables(ent_host, LIGHT_CHUNK if matrix else SCAN_CHUNK, proj.device)
+        vent, cent = chunk_tables(ent_host, LIGHT_CHUNK if matrix else SCAN_CHUNK, proj.device, ent)
         NV = vent.shape[0]
         cs = torch.empty(NV, H, D, V, device=proj.device, dtype=torch.float32)
         cd = torch.empty(NV, H, D, device=proj.device, dtype=torch.float32)
@@ -2271,7 +2308,7 @@ def lightning_scan(proj, powers, state, ent, ent_host, out, H: int, D: int, V: i
     assert powers.dtype == torch.float32 and powers.is_contiguous() and powers.shape == (H, LIGHT_CHUNK + 1)
     _scan_state_ok(state, H, D, V, ent)
     if max(e[1] for e in ent_host) >= LIGHT_MIN:
-        vent, cent = chunk_tables(ent_host, LIGHT_CHUNK, proj.device)
+        vent, cent = chunk_tables(ent_host, LIGHT_CHUNK, proj.device, ent)
         NV = vent.shape[0]
         cs = torch.empty(NV, H, D, V, device=proj.device, dtype=torch.float32)
         _chk(lib().p2p_sm_lightning_chunked(proj.data_ptr(), proj.stride(0), powers.data_ptr(),
@@ -2333,7 +2370,7 @@ def gated_delta_scan(conv, araw, braw, gate, A_log, dt_bias, normw, state, ent, 
     assert H % G == 0
     _scan_state_ok(state, H, D, V, ent)
     if _chunked(ent_host):
-        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, conv.device)
+        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, conv.device, ent)
         NV = vent.shape[0]
         cs = torch.empty(NV, H, D, V, device=conv.device, dtype=torch.float32)
         ct = torch.empty(NV, H, D, D, device=conv.device, dtype=torch.float32)
@@ -2407,7 +2444,7 @@ def mlstm_scan(proj, bi, bf, cap: float, normw, state, mstate, ent, ent_host, ou
     vent = cent = cs = cd = None
     NV = 0
     if _chunked(ent_host):
-        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, proj.device)
+        vent, cent = chunk_tables(ent_host, SCAN_CHUNK, proj.device, ent)
         NV = vent.shape[0]
         cs = torch.empty(NV, H, D, V + 1, device=proj.device, dtype=torch.float32)
         cd = torch.empty(NV, H, D, device=proj.device, dtype=torch.float32)
