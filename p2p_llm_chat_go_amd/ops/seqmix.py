@@ -919,7 +919,9 @@ SCAN_CHUNK = int(os.environ.get("P2P_SCAN_CHUNK", "64"))
 
 def scan_chunks(ent_host: list, chunk: int):
     """(chunks as entries [(row0, n, 1, chunk index)], per entry (first chunk, chunks, first
-    position, slot)) as int32 tensors."""
+    position, slot)) as int32 tensors, of ``Portions`` on their device."""
+    if getattr(ent_host, "step", None) is not None:
+        return ent_host.tables(chunk)
     vent, cent = [], []
     for row0, n, start, slot in ent_host:
         c0 = len(vent)
@@ -927,6 +929,25 @@ def scan_chunks(ent_host: list, chunk: int):
             vent.append((r, min(chunk, row0 + n - r), 1, len(vent)))
         cent.append((c0, len(vent) - c0, start, slot))
     return torch.tensor(vent, dtype=torch.int32), torch.tensor(cent, dtype=torch.int32)
+
+
+class Portions(list):
+    """The entries of a step that have at least ``least`` rows.  step: all of the step's entries on the device, where a kernel
+    forms the tables (None: they are formed here and copied).  rest: the other entries, behind the tables there."""
+
+    def __init__(self, ent_host: list, least: int, ent):
+        super().__init__(e for e in ent_host if e[1] >= least)
+        on_device = ent is not None and ent.is_cuda and ent.dtype == torch.int32 and ent.is_contiguous() and \
+            ent.shape == (len(ent_host), 4) and ent.data_ptr() % 16 == 0
+        self.step, self.least, self.rest = ent if on_device and self else None, least, None
+
+    def tables(self, chunk: int):
+        V, E = sum((e[1] + chunk - 1) // chunk for e in self), len(self)
+        out = torch.empty(V + self.step.shape[0], 4, device=self.step.device, dtype=torch.int32)
+        v, c, self.rest = out[:V], out[V:V + E], out[V + E:]
+        _chk(lib().p2p_sm_step_tables(self.step.data_ptr(), self.step.shape[0], chunk, self.least, None, v.data_ptr(), c.data_ptr(),
+                                      self.rest.data_ptr(), _st(self.step)), "step_tables")
+        return v, c
 
 
 class Entries(list):
@@ -938,23 +959,6 @@ class Entries(list):
         self.tables = {}
 
 
-def _on_device(ent, ent_host) -> bool:
-    """ent holds ent_host where a kernel can read it (``p2p_sm_step_tables``)."""
-    return (ent is not None and ent.is_cuda and ent.dtype == torch.int32 and ent.is_contiguous() and ent.shape == (len(ent_host), 4)
-            and ent.data_ptr() % 16 == 0)
-
-
-def _step_tables(ent, ent_host, chunk: int, least: int):
-    """``scan_chunks`` of the entries of at least ``least`` rows and the others as they are, formed on the device."""
-    whole = [e[1] for e in ent_host if e[1] >= least]
-    V, E = sum((n + chunk - 1) // chunk for n in whole), len(whole)
-    out = torch.empty(V + len(ent_host), 4, device=ent.device, dtype=torch.int32)
-    v, c, rest = out[:V], out[V:V + E], out[V + E:]
-    _chk(lib().p2p_sm_step_tables(ent.data_ptr(), len(ent_host), chunk, least, None, v.data_ptr(), c.data_ptr(), rest.data_ptr(),
-                                  _st(ent)), "step_tables")
-    return v, c, rest
-
-
 def chunk_tables(ent_host: list, chunk: int, device, ent=None):
     """``scan_chunks`` on the device (kept with the step when it is an ``Entries``); ent: the entries there, which spare the
     copy."""
@@ -962,12 +966,11 @@ def chunk_tables(ent_host: list, chunk: int, device, ent=None):
     key = (chunk, str(device))
     if kept is not None and key in kept:
         return kept[key]
-    if _on_device(ent, ent_host):
-        out = _step_tables(ent, ent_host, chunk, 0)[:2]
-    else:
-        vent, cent = scan_chunks(ent_host, chunk)
-        both = torch.cat([vent, cent]).to(device)
-        out = both[:vent.shape[0]], both[vent.shape[0]:]
+    out = scan_chunks(Portions(ent_host, 0, ent), chunk)
+    if not out[0].is_cuda:
+        V = out[0].shape[0]
+        both = torch.cat(out).to(device)
+        out = both[:V], both[V:]
     if kept is not None:
         kept[key] = out
     return out
@@ -984,15 +987,14 @@ def portion_tables(ent_host: list, chunk: int, least: int, device, ent=None):
     key = (chunk, least, str(device))
     if kept is not None and key in kept:
         return kept[key]
-    if _on_device(ent, ent_host) and any(e[1] >= least for e in ent_host):
-        v, c, rest = _step_tables(ent, ent_host, chunk, least)
-        out = v, c, rest if rest.shape[0] else None
-    else:
-        vent, cent = scan_chunks([e for e in ent_host if e[1] >= least], chunk)
+    whole = Portions(ent_host, least, ent)
+    vent, cent = scan_chunks(whole, chunk)
+    if whole.rest is None:
         short = [tuple(e) for e in ent_host if e[1] < least]
         V, E = vent.shape[0], cent.shape[0]
         every = torch.cat([vent, cent, torch.tensor(short, dtype=torch.int32).view(-1, 4)]).to(device)
-        out = every[:V], every[V:V + E], every[V + E:] if short else None
+        vent, cent, whole.rest = every[:V], every[V:V + E], every[V + E:]
+    out = vent, cent, whole.rest if whole.rest.shape[0] else None
     if kept is not None:
         kept[key] = out
     return out
@@ -1331,7 +1333,7 @@ def make_units(ent_host: list, rows_per_wave: int) -> torch.Tensor:
 
 def device_units(ent_host: list, rows_per_wave: int, ent) -> torch.Tensor:
     """``make_units`` on the device of ent, the entries there."""
-    if not _on_device(ent, ent_host):
+    if Portions(ent_host, 0, ent).step is None:
         return make_units(ent_host, rows_per_wave).to(ent.device)
     U = sum((e[1] + rows_per_wave - 1) // rows_per_wave for e in ent_host)
     out = torch.empty(U, 2, device=ent.device, dtype=torch.int32)
