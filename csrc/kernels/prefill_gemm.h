@@ -864,12 +864,20 @@ static int pick_tile(int M, int N, int K, int epi) {
   if (small <= cus) {
     // One round of 128 x 128 tiles, K cut where they leave CUs idle.  128 x 256 tiles copy a quarter less per product and
     // take twice the slices: they pay where a slice keeps 2048 numbers and four slices fill the chip.  Residual, us,
-    // 128 x 128 / 128 x 256: 4096 x 14336, 300, 398, 512, 1024 rows 65 / 60, 73 / 62, 81 / 69, 135 / 118 (1020 TFLOP/s);
-    // 8192 x 28672, 256 rows 163 / 140; 4096 x 8192, 398 and 1024 rows 48 / 44, 82 / 77; 4096 x 6144, 700 rows (two
-    // slices) 60 / 56, 398 rows (four) 41 / 41; eight slices: 4096 x 14336, 256 rows 50 / 55; 4096 x 4096, 1024 rows
-    // 50 / 49.5, plain 40 / 44
+    // 128 x 128 / 128 x 256: 4096 x 14336, 300, 398, 512, 1024 rows 62 / 58, 68 / 61, 76 / 64, 125 / 111 (1080 TFLOP/s);
+    // 4096 x 8192, 398 and 1024 rows 43 / 41, 71 / 71; eight slices: 4096 x 14336, 72 and 128 rows 32 / 39, 34 / 42;
+    // 4096 x 4096, 1024 rows 37 / 43.  192 x 128 where its slices fill the chip and those of 128 x 256 leave a quarter of it idle
+    // (128 x 256 / 192 x 128, 4096 x 14336, 300, 350, 580, 700, 768 rows 58 / 52, 61 / 55, 97 / 85, 98 / 92, 104 / 92, 4096 x 8192,
+    // 700 rows 63 / 55)
     const long wide = N % 256 == 0 ? tiles(128, 256) : 0;
-    return wide * 8 > cus && K >= 6144 && K >= (wide * 4 > cus ? 2 : 4) * 2048 && wide <= cus ? 2 : 3;
+    if (!(wide * 8 > cus && K >= 6144 && K >= (wide * 4 > cus ? 2 : 4) * 2048 && wide <= cus)) return 3;
+    auto blocks = [&](long t) {   // with the slices that launch() cuts K into
+      long k = 1;
+      while (k * 2 <= std::min<long>(std::min<long>(8, cus / t), K / BK / 16)) k *= 2;
+      return t * k;
+    };
+    const long tall = tiles(192, 128);
+    return K >= 8192 && tall <= cus && blocks(wide) * 4 <= cus * 3l && blocks(tall) * 8 > cus * 7l ? 7 : 2;
   }
   if (N >= 16384 && M > 128 && M <= 192) return 7;   // one row of tiles, 192 x 128: SwiGLU 28672 x 4096 62 us, 128 x 128 81
   // A residual product with a short K that gives 160 tiles of 256 x 256 and more waits for its residual and its first and last
