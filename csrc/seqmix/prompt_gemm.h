@@ -69,18 +69,20 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
   const int tile = (xcd < over ? xcd * (per + 1) : over * (per + 1) + (xcd - over) * per) + blockIdx.x / 8;
   const int band = tile / (GM * a.n_tiles), first = band * GM, gm = min(a.m_tiles - first, GM), in = tile - band * GM * a.n_tiles;
   const int m0 = (first + in % gm) * BM, n0 = in / gm * (ACT ? BN / 2 : BN);
-  const int nk = a.K / KS, n = (nk + WK - 1) / WK;
+  const int nk = (a.K + KS - 1) / KS, n = (nk + WK - 1) / WK;
 
   // copies: an address of the wavefront's per stage, a lane's offset that stays
   const char* xs = (const char*)((const T*)a.x + (a.rows ? 0 : (size_t)m0 * a.ldx));
   const char* ws = (const char*)((const T*)a.w + (size_t)n0 * a.K);
   const int p8 = lane & 7, r8 = lane >> 3;
+  const bool half = a.K < KS;                  // rows of 64 bytes: their pieces twice, the second half stage is not multiplied
+  const int pieces = half ? 3 : 7;
   int at[L];
 #pragma unroll
   for (int i = 0; i < AI; i++) {
     const int r = 8 * (wk + WPK * i) + r8;
     const int m = min(m0 + r, a.M - 1);
-    at[i] = (a.rows ? a.rows[m] : m - m0) * a.ldx * (int)sizeof(T) + ((p8 ^ (r & 7)) << 4);
+    at[i] = (a.rows ? a.rows[m] : m - m0) * a.ldx * (int)sizeof(T) + (((p8 ^ (r & 7)) & pieces) << 4);
   }
   auto w_key = [](int r) { return (r & 3) | ((r / RUN) & 1) << 2; };   // r: row among those of a wavefront
 #pragma unroll
@@ -88,7 +90,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
     const int r = 8 * (wk + WPK * i) + r8, rw = r % (16 * FN);
     int row = ACT ? r / (16 * FN) * (8 * FN) + rw % (8 * FN) : r;
     row = min(n0 + row, a.N - 1) - n0 + (ACT && rw >= 8 * FN ? a.N : 0);
-    at[AI + i] = row * a.K * (int)sizeof(T) + ((p8 ^ w_key(rw)) << 4);
+    at[AI + i] = row * a.K * (int)sizeof(T) + (((p8 ^ w_key(rw)) & pieces) << 4);
   }
   const unsigned lds0 = lds_address(lds) + kg * KG + wk * 1024;
   auto copy = [&](int i, int t) {   // the i-th of this wavefront's copies of stage t
@@ -201,7 +203,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
   if (WK == 1 || t * WK + kg < nk) {
     read(t, 1, x1, w1);
     products(x0, w0, nothing);
-    products(x1, w1, nothing);
+    if (!half) products(x1, w1, nothing);
   }
   if constexpr (WK > 1) {   // the groups' sums, in their order
     used_up();

@@ -19,7 +19,7 @@ int p2p_sm_prompt_gemm(const void* x, const int* rows, long span, int ldx, const
                        int N, int K, int tanh_from, int act, float limit, float alpha, int tile, int f32, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   const int size = f32 ? 4 : 2, ks = 128 / size;
-  if (K < ks || K % ks || ldx < 0 || ldx % (16 / size) || (size_t)x % 16 || (size_t)w % 16 || act > 2 || (f32 && tanh_from < N) ||
+  if (K < 1 || (K % ks && K != ks / 2) || ldx < 0 || ldx % (16 / size) || (size_t)x % 16 || (size_t)w % 16 || act > 2 || (f32 && tanh_from < N) ||
       (rows ? span * size : (long)ldx * 256 * size) >= 1l << 31 || (long)K * size * (act >= 0 ? N + 256l : 256l) >= 1l << 31)
     return (int)hipErrorInvalidValue;
   // neighbours that a store takes at once
@@ -27,7 +27,7 @@ int p2p_sm_prompt_gemm(const void* x, const int* rows, long span, int ldx, const
                    : ldo % 4 == 0 && N % 4 == 0 && (size_t)out % (4 * size) == 0 ? 4 : 0;
   const GemmArgs a = {x, rows, ldx, w, bias, out, ldo, M, N, K, tanh_from, act, limit, alpha, 0, 0, wide};
   if (f32) return prompt_gemm_f32(a, tile, st);
-  switch (tile ? tile : pick_tile(TILES, M, act >= 0 ? 2 * N : N, K / ks, act >= 0)) {
+  switch (tile ? tile : pick_tile(TILES, M, act >= 0 ? 2 * N : N, (K + ks - 1) / ks, act >= 0)) {
     case 1: return launch_gemm<bf16, 32, 16, 1, 1, 4, 4>(a, st);
     case 2: return launch_gemm<bf16, 32, 32, 1, 1, 4, 4>(a, st);
     case 3: return launch_gemm<bf16, 32, 64, 1, 2, 2, 4>(a, st);

@@ -15,7 +15,7 @@ static const Tile TILES[] = {
     {128, 128, true, 6.5f, 4.8f, 1.894f, 1.904f}};
 
 int prompt_gemm_f32(const GemmArgs& a, int tile, hipStream_t st) {
-  switch (tile ? tile : pick_tile(TILES, a.M, a.act >= 0 ? 2 * a.N : a.N, a.K / 32, a.act >= 0)) {
+  switch (tile ? tile : pick_tile(TILES, a.M, a.act >= 0 ? 2 * a.N : a.N, (a.K + 31) / 32, a.act >= 0)) {
     case 1: return launch_gemm<float, 32, 16, 1, 1, 4, 4>(a, st);
     case 2: return launch_gemm<float, 32, 32, 1, 1, 4, 4>(a, st);
     case 3: return launch_gemm<float, 64, 32, 2, 1, 4, 3>(a, st);

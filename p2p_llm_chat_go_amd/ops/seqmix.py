@@ -449,15 +449,16 @@ def _conv_args(M: int, N: int, dtype, c0: int, cw, cb, tail, ent, out):
 
 
 def _prompt_gemm_ok(x, w, b=None) -> bool:
-    """Products that ``csrc/seqmix/prompt_gemm.h`` takes: K in stages of 128 bytes, rows that 16-byte copies can read."""
+    """Products that ``csrc/seqmix/prompt_gemm.h`` takes: K in stages of 128 bytes, rows that 16-byte copies can read; or one
+    stage of 64 (the low-rank decays, 1024 columns of K = 32: the host spends 20 us on the library's call and 10 on this)."""
     if x.dim() != 2 or w.dim() != 2 or x.dtype != w.dtype or not x.is_cuda or x.device != w.device or x.requires_grad \
             or w.requires_grad:
         return False
     (M, K), ld = x.shape, x.stride(0)
     if x.dtype == torch.bfloat16:
-        ok = K % 64 == 0 and ld % 8 == 0
+        ok = (K % 64 == 0 or K == 32) and ld % 8 == 0
     elif x.dtype == torch.float32:
-        ok = K % 32 == 0 and ld % 4 == 0
+        ok = (K % 32 == 0 or K == 16) and ld % 4 == 0
     else:
         return False
     return (ok and M > 0 and K > 0 and w.shape[1] == K and w.is_contiguous() and x.stride(1) == 1 and ld >= K

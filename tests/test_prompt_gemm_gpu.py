@@ -25,7 +25,7 @@ def _close(got, ref):
 
 # rows and columns at the edges of every tile (32 to 256), one 64 of K, fewer stages than a tile keeps, groups of K left over
 @pytest.mark.parametrize("tile", range(TILES + 1))
-@pytest.mark.parametrize("M,N,K,ld", [(1, 8, 64, 64), (31, 100, 128, 136), (33, 33, 192, 192), (257, 264, 448, 456),
+@pytest.mark.parametrize("M,N,K,ld", [(1, 8, 64, 64), (140, 200, 32, 40), (31, 100, 128, 136), (33, 33, 192, 192), (257, 264, 448, 456),
                                       (200, 77, 1088, 1088), (513, 520, 320, 320)])
 def test_tiles(tile, M, N, K, ld):
     x, w = _case(M, N, K, ld)
@@ -65,7 +65,7 @@ def test_units(tile, act, limit):
 # fp32 sums of K products: against the library's sums of the same inputs, of which neither has another order's rounding on its
 # side (a chain of K / 4 sums each: their errors are alike, and twice the library's is far outside of what orders do)
 @pytest.mark.parametrize("tile", range(10))
-@pytest.mark.parametrize("M,N,K,ld", [(1, 8, 32, 32), (31, 100, 64, 68), (129, 132, 224, 224), (200, 77, 1056, 1060), (300, 520, 512, 512)])
+@pytest.mark.parametrize("M,N,K,ld", [(1, 8, 32, 32), (140, 200, 16, 20), (31, 100, 64, 68), (129, 132, 224, 224), (200, 77, 1056, 1060), (300, 520, 512, 512)])
 def test_float32(tile, M, N, K, ld):
     x, w = _case(M, N, K, ld, dtype=torch.float32)
     b = torch.randn(N, device=DEV)
