@@ -326,7 +326,7 @@ def embed_rows(embed, ids, out, h_out=None, scale: float = 1.0):
 
 
 def _skinny(x, w) -> bool:
-    """Products that ``csrc/seqmix/skinny.hip`` takes from the library: at most 16 rows of one matrix instruction.  Where
+    """Products that ``csrc/seqmix/skinny.hip`` takes: at most 16 rows of one matrix instruction.  Where
     the lines lie (a captured graph, cold weights, library -> kernel in us, 8 rows unless others are named):
 
     * bf16, K up to 2048 (activations kept in registers where that pays, skinny.hip): 12288 x 2048 16.1 -> 12.1, 24576 x
@@ -336,7 +336,7 @@ def _skinny(x, w) -> bool:
       8192 x 256 5.7 -> 3.7, 8192 x 64 3.6 -> 2.5.
     * fp32, K up to 1024, the same kernel: 12288 x 1024 31.6 -> 12.9, 32000 x 512 19.0 -> 17.3, 65536 x 512 28.8 -> 31.8,
       32000 x 128 9.2 -> 8.3, 50257 x 128 10.7 -> 9.4, 128256 x 64 16.9 -> 13.6, 128256 x 1024 106 -> 92, 16384 x 768 13.8 ->
-      12.0; few columns stay with the library.
+      12.0; few columns are left to the kernel of any rows.
     * Longer K, one workgroup per tile walks all of it: bf16 2048 x 8192 12.9 -> 15.0, 2048 x 4096 12.5 -> 8.3, 4096 x
       4096 15.6 -> 9.9, 6144 x 3072 11.9 -> 13.0, 4 rows 12288 x 4096 24.1 -> 21.1, 16 rows 96 x 4096 7.9 -> 8.9, 8 rows
       7.9 -> 7.6; fp32 2048 x 4096 13.2 -> 15.0, 2048 x 2048 10.5 -> 8.5, 16 rows 4608 x 2048 14.1 -> 16.4, 1024 x 2048
