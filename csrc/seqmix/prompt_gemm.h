@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) prompt_gemm_k(GemmArgs a) {
 #pragma unroll
     for (int e = 0; e < RUN; e++) {
       float v = acc[i][e / 4][e % 4];
-      if constexpr (ACT) v = unit_act(a.act, v, acc[i][FN / 2 + e / 4][e % 4], a.limit, a.alpha);
+      if constexpr (ACT) v = unit_act<sizeof(T) == 4>(a.act, v, acc[i][FN / 2 + e / 4][e % 4], a.limit, a.alpha);
       else if (a.bias) v += bias[e];
       stf(o, e, v);
     }

@@ -86,6 +86,33 @@ def test_float32(tile, M, N, K, ld):
     assert ((out.double() - want).norm() / want.norm()).item() < 1e-6
 
 
+@pytest.mark.parametrize("act,limit", [("silu", None), ("gelu_tanh", None), ("silu", 7.0)])
+def test_float32_units_keep_the_bits_of_the_pass(act, limit):
+    # rows of one 1: every product is a number of w itself, so what is off is the unit's.  Gates of -40 to 40, where
+    # e^-g has lost all bits if its argument was rounded
+    n, K, M = 512, 32, 32
+    x = torch.eye(K, device=DEV)[:M]
+    gate = torch.linspace(-40, 40, n * M, device=DEV).view(n, M)
+    if act == "gelu_tanh":
+        gate = gate / 8                                       # (z + 0.044715 z^3: beyond 5 nothing but z or 0 is left)
+    up = torch.linspace(0.5, 2.0, n * M, device=DEV).view(n, M).flip(0)
+    w = torch.cat([gate, up], 0).contiguous()
+    g, u = gate.t().double(), up.t().double()
+    if limit is not None:
+        g = g.clamp(max=limit)
+        want, y = g * torch.sigmoid(1.702 * g) * (u.clamp(-limit, limit) + 1), 1.702 * g
+    elif act == "silu":
+        want, y = g * torch.sigmoid(g) * u, torch.zeros_like(g)
+    else:
+        y = 2 * (2 / torch.pi) ** 0.5 * (g + 0.044715 * g ** 3)
+        want = g * torch.sigmoid(y) * u
+    got = sm.linear_unit(x, w, torch.empty(M, n, device=DEV), act, limit)
+    # e^-y to 2^-23 of it, the sum, the division and two products each 2^-24 more; where y is formed (not for silu), its own
+    # roundings, up to four of 2^-24, reach e^-y by |y|
+    bound = (6 + 4 * y.abs()) * 2.0 ** -24 * want.abs() + 1e-37
+    assert bool(((got.double() - want).abs() <= bound).all())
+
+
 def test_rows_and_other_rows():
     x, w = _case(300, 96, 128, 160)
     rows = torch.randint(0, 300, (45,), device=DEV, dtype=torch.int32)
