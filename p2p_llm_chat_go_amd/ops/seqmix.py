@@ -34,6 +34,7 @@ import threading
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -448,28 +449,41 @@ def _conv_args(M: int, N: int, dtype, c0: int, cw, cb, tail, ent, out):
             _f32(out))
 
 
+_transforms, _modes, _tracing = (getattr(torch._C, n) for n in ("_are_functorch_transforms_active", "_len_torch_dispatch_stack",
+                                                               "_is_tracing"))
+_autocast, _compiling = torch.is_autocast_enabled, torch.compiler.is_compiling
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _by_address() -> bool:
+    """Whether a kernel may be launched by its operands' addresses: outside of function transforms (vmap, jvp), forward-mode
+    levels, dispatch modes, traces and autocast, all of which the library's call serves and such a launch passes by."""
+    return not (_transforms() or forward_ad._current_level >= 0 or _modes() or _tracing() or _autocast("cuda") or _compiling())
+
+
 def _prompt_gemm_ok(x, w, b=None) -> bool:
     """Products that ``csrc/seqmix/prompt_gemm.h`` takes: K in stages of 128 bytes, rows that 16-byte copies can read; or one
     stage of 64 (the low-rank decays, 1024 columns of K = 32: the host spends 20 us on the library's call and 10 on this)."""
-    if x.dim() != 2 or w.dim() != 2 or x.dtype != w.dtype or not x.is_cuda or x.device != w.device or x.requires_grad \
-            or w.requires_grad:
+    dt, xs, ws = x.dtype, x.shape, w.shape
+    if len(xs) != 2 or len(ws) != 2 or dt != w.dtype or not x.is_cuda or x.get_device() != w.get_device() or x.requires_grad \
+            or w.requires_grad or type(x) not in _PLAIN or type(w) not in _PLAIN or not _by_address():
         return False
-    (M, K), ld = x.shape, x.stride(0)
-    if x.dtype == torch.bfloat16:
+    (M, K), (ld, unit) = xs, x.stride()
+    if dt == torch.bfloat16:
         ok = (K % 64 == 0 or K == 32) and ld % 8 == 0
-    elif x.dtype == torch.float32:
+    elif dt == torch.float32:
         ok = (K % 32 == 0 or K == 16) and ld % 4 == 0
     else:
         return False
-    return (ok and M > 0 and K > 0 and w.shape[1] == K and w.is_contiguous() and x.stride(1) == 1 and ld >= K
-            and ld < 1 << 21 and K * (w.shape[0] + 256) < 1 << 29 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and (b is None or b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and not b.requires_grad))
+    return (ok and M > 0 and K > 0 and ws[1] == K and w.is_contiguous() and unit == 1 and ld >= K
+            and ld < 1 << 21 and K * (ws[0] + 256) < 1 << 29 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (b is None or b.dtype == dt and b.device == x.device and b.is_contiguous() and not b.requires_grad))
 
 
 def _prompt_gemm(x, w, b, out, tanh_from=None, act: int = -1, limit: float = 0.0, alpha: float = 0.0, rows=None, tile: int = 0):
-    M, N = out.shape
-    _chk(lib().p2p_sm_prompt_gemm(x.data_ptr(), _lib.ptr(rows), (x.shape[0] - 1) * x.stride(0) + x.shape[1], x.stride(0),
-                                  w.data_ptr(), _lib.ptr(b), out.data_ptr(), out.stride(0), M, N, x.shape[1],
+    (M, N), (n, K), ld = out.shape, x.shape, x.stride(0)
+    _chk(lib().p2p_sm_prompt_gemm(x.data_ptr(), None if rows is None else rows.data_ptr(), (n - 1) * ld + K, ld,
+                                  w.data_ptr(), None if b is None else b.data_ptr(), out.data_ptr(), out.stride(0), M, N, K,
                                   N if tanh_from is None else tanh_from, act, limit, alpha, tile, _f32(x), _st(x)), "prompt_gemm")
     return out
 

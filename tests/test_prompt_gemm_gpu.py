@@ -137,3 +137,28 @@ def test_other_forms_stay_with_the_library():
     sm.linear(x, w).sum().backward()
     assert w.grad is not None
     assert sm.linear(x[:0], w.detach()).shape == (0, 64)
+
+
+def test_transforms_and_modes_are_served_as_by_the_library():
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    x, w = _case(40, 64, 128, dtype=torch.float32)
+    xs = torch.stack([x, 2 * x, -x])
+    assert torch.equal(torch.func.vmap(lambda a: sm.linear(a, w))(xs), torch.func.vmap(lambda a: F.linear(a, w))(xs))
+    t = torch.randn_like(x)
+    y, dy = torch.func.jvp(lambda a: sm.linear(a, w), (x,), (t,))
+    assert torch.equal(y, F.linear(x, w)) and torch.equal(dy, F.linear(t, w))
+    with forward_ad.dual_level():
+        y, dy = forward_ad.unpack_dual(sm.linear(forward_ad.make_dual(x, t), w))
+        assert dy is not None and torch.equal(dy, F.linear(t, w))
+    assert torch.equal(torch.func.grad(lambda a: sm.linear(a, w).sum())(x), torch.func.grad(lambda a: F.linear(a, w).sum())(x))
+    traced = make_fx(lambda a: sm.linear(a, w))(x)            # a trace holds the product, not its result
+    assert torch.equal(traced(2 * x), F.linear(2 * x, w))
+    traced = torch.jit.trace(lambda a: sm.linear(a, w), (x,), check_trace=False)
+    assert torch.equal(traced(2 * x), F.linear(2 * x, w))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert sm.linear(x, w).dtype == torch.bfloat16 == F.linear(x, w).dtype
+    rows = torch.arange(3, 23, device=DEV, dtype=torch.int32)
+    assert torch.equal(torch.func.vmap(lambda a: sm.linear(a, w, rows=rows))(xs), F.linear(xs[:, 3:23], w))
+    assert sm._prompt_gemm_ok(x, w)                           # (nothing of that is left on)
