@@ -1301,11 +1301,16 @@ MIXERS = {c.kind: c for c in (GeneralDelta, Mamba2, LatentAttention, WindowAtten
                               ParallelGLA)}
 
 
+def _own_product(fill):
+    """Marks a ``fill`` or ``fill_routed`` that forms its product itself when it is given None (``ops.seqmix.linear_unit``).  One
+    that overrides it is not marked, and is given the product."""
+    fill.own_product = True
+    return fill
+
+
 class DenseFF:
     """Gated feed-forward W_down(act(W_gate h) * W_up h): silu-gated, or with a ``limit`` in its
     config the clamped unit of ``ops.seqmix.ff_act``.
-
-    ``fill`` without a product forms it itself (``ops.seqmix.linear_unit``).
 
     Every feed-forward offers two ways in: ``forward(h)``, or for a layer that runs the
     projections of its input and the output projections of its sublayers as one product each:
@@ -1328,8 +1333,9 @@ class DenseFF:
         self.w_in = self.w_gu
         self.w_down = self.w_out = get("down").to(dev, dtype).contiguous()
 
+    @_own_product
     def fill(self, gu, h, mid):
-        if gu is None:   # (the product is formed here)
+        if gu is None:
             sm.linear_unit(h, self.w_gu, mid, self.ACT, self.limit)
         elif self.limit is None:
             sm.glu_act(gu, mid, self.ACT)
@@ -1344,7 +1350,8 @@ class DenseFF:
         return sm.linear(act, self.w_down)
 
     def forward(self, h):
-        if isinstance(h, sm.NormedRows):
+        if isinstance(h, sm.NormedRows) or not hasattr(self.fill, "own_product") or \
+                type(self).forward_proj is not DenseFF.forward_proj:
             return self.forward_proj(sm.linear(h, self.w_gu))
         act = torch.empty(h.shape[0], self.F, device=h.device, dtype=h.dtype)
         self.fill(None, h, act)
@@ -1568,6 +1575,7 @@ class TopMoEFF:
         sm.expert_gemm(act, 1, self.w_down, cnt, rows, y, R * top)
         return y, wts
 
+    @_own_product
     def fill_routed(self, proj, h, mid, cnt=None):
         """``fill`` for a layer whose residual pass sums the routed experts itself."""
         if self.Fs:
@@ -1971,7 +1979,8 @@ class HybridModel:
                 y = L.mixer.forward(h, b, self.cache, i)
             elif moe[i]:
                 mid = torch.empty(R, L.ff.n_mid, device=dev, dtype=self.dtype) if L.ff.n_mid else None
-                routed = L.ff.fill_routed(None, h, mid, cnts[sum(moe[:i]), :L.ff.E])
+                proj = None if mid is None or hasattr(L.ff.fill_routed, "own_product") else sm.linear(h, L.ff.w_in)
+                routed = L.ff.fill_routed(proj, h, mid, cnts[sum(moe[:i]), :L.ff.E])
                 y = sm.linear(mid, L.ff.w_out) if mid is not None else None
             else:
                 y = L.ff.forward(h)
@@ -2025,7 +2034,7 @@ class HybridModel:
             L.mixer.mix(sm.linear(h1, L.mixer.w_in, L.mixer.b_in), b, self.cache, k, mid[:, :mm])
             extra = routed = None
             if L.ff is not None:
-                own = moe[k] or isinstance(L.ff, DenseFF) or L.ff.w_in is None   # (forms the product of its gated unit itself)
+                own = L.ff.w_in is None or hasattr(L.ff.fill_routed if moe[k] else L.ff.fill, "own_product")
                 proj = None if own else sm.linear(h2, L.ff.w_in)
                 if moe[k]:
                     routed = L.ff.fill_routed(proj, h2, mid[:, mm:], cnts[sum(moe[:k]), :L.ff.E])
