@@ -16,11 +16,19 @@ def _case(M, N, K, ld=None, seed=0, dtype=torch.bfloat16):
     return x, (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).to(dtype)
 
 
-def _close(got, ref):
-    # one rounding to bf16 (2^-9 of the value at most) of fp32 sums of K products: K 2^-24 of the products' magnitude, which
-    # rows ~ N(0, 1) and weights ~ N(0, 1/K) keep below sqrt(K) 2^-24 * 4 of the results' size
-    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * 4 * got.shape[1] ** 0.5 + 1e-3 * ref.abs().mean()
-    assert bool(((got.double() - ref).abs() <= bound).all())
+def _close(got, x, w, b):
+    """got = x w^T + b as one rounding to bf16 (2^-8 of the value at most) of fp32 sums of K products and b, whose roundings are
+    at most K 2^-24 of what the products' magnitudes sum to."""
+    ref = x.double() @ w.double().t() + b.double()
+    sums = (x.shape[1] + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    assert bool(((got.double() - ref).abs() <= 2.0 ** -8 * (ref.abs() + sums) + sums).all())
+
+
+def _tanh_close(got, z):
+    """got = tanh of the bf16 numbers z to 2e-6 of it, rounded to bf16: to half of the last of 8 bits."""
+    t = torch.tanh(z.double())
+    last = torch.exp2(torch.floor(torch.log2(t.abs().clamp(min=2.0 ** -126))) - 7)
+    assert bool(((got.double() - t).abs() <= last / 2 * (1 + 2.0 ** -20) + 2e-6 * t.abs()).all())
 
 
 # rows and columns at the edges of every tile (32 to 256), one 64 of K, fewer stages than a tile keeps, groups of K left over
@@ -33,13 +41,29 @@ def test_tiles(tile, M, N, K, ld):
     for shift in (0, 3, 4):   # 16-byte, 2-byte and 8-byte places of the rows
         whole = torch.full((M + 2, N + 16), 9.0, device=DEV, dtype=torch.bfloat16)
         out = whole[1:M + 1, shift:shift + N]
+        sm._prompt_gemm(x, w, b, out, tile=tile)
+        _close(out, x, w, b)
+        z = out.clone()
         sm._prompt_gemm(x, w, b, out, tanh_from=N - 5, tile=tile)
-        ref = x.double() @ w.double().t() + b.double()
-        _close(out[:, :N - 5], ref[:, :N - 5])
-        tail = torch.tanh(ref[:, N - 5:])   # of the rounded result: 2^-9 of it, then a rounding
-        assert (out[:, N - 5:].double() - tail).abs().max() <= 2.0 ** -7 * 4
+        assert torch.equal(out[:, :N - 5], z[:, :N - 5])
+        _tanh_close(out[:, N - 5:], z[:, N - 5:])
         out.fill_(9.0)
         assert bool((whole == 9.0).all())   # nothing beside it was written
+
+
+def test_tanh_of_every_number():
+    """All finite bf16 numbers as products of a row's one 1: around the switch of the two forms at 1/4, at their ends, beyond."""
+    every = torch.arange(1 << 16, device=DEV, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    every = every[every.isfinite() & ((every == 0) | (every.abs() >= 2.0 ** -126))]
+    n = every.numel() // 64
+    z = every[:64 * n].view(64, n)
+    out = sm.linear(torch.eye(64, device=DEV).bfloat16(), z.t().contiguous(), tanh_from=0)
+    _tanh_close(out, z)
+    odd = torch.tensor([float("inf"), float("-inf"), float("nan")], device=DEV).bfloat16().repeat_interleave(16)[:, None]
+    x = torch.zeros(48, 64, device=DEV).bfloat16()
+    x[:, :1] = odd
+    out = sm.linear(x, torch.ones(8, 64, device=DEV).bfloat16(), tanh_from=0).float()
+    assert bool((out[:16] == 1).all() and (out[16:32] == -1).all() and out[32:].isnan().all())
 
 
 @pytest.mark.parametrize("tile", [0] + list(range(2, TILES - 1)))
