@@ -410,7 +410,7 @@ class NormedRows:
     def linear(self, w, b=None, tanh_from=None, conv=None):
         """The rows times w transposed (plus b), and behind it a convolution (``_conv_args``).  None where no kernel does
         all that."""
-        if not self._fits(w) or (b is not None and not (b.dtype == self.dtype and b.is_cuda and b.is_contiguous())):
+        if not self._fits(w) or not _bias_ok(b, w, self.y):
             return None
         x, y, spare = self.x, self.y, self.spare
         (M, K), N = x.shape, w.shape[0]
@@ -461,6 +461,12 @@ def _by_address() -> bool:
     return not (_transforms() or forward_ad._current_level >= 0 or _modes() or _tracing() or _autocast("cuda") or _compiling())
 
 
+def _bias_ok(b, w, x) -> bool:
+    """Whether kernels can read b: one number per row of w.  (The library takes one for all of them too, and refuses the rest.)"""
+    return b is None or (b.dtype == x.dtype and b.shape == w.shape[:1] and b.is_contiguous() and b.device == x.device
+                         and type(b) in _PLAIN)
+
+
 def _prompt_gemm_ok(x, w, b=None) -> bool:
     """Products that ``csrc/seqmix/prompt_gemm.h`` takes: K in stages of 128 bytes, rows that 16-byte copies can read; or one
     stage of 64 (the low-rank decays, 1024 columns of K = 32: the host spends 20 us on the library's call and 10 on this)."""
@@ -477,7 +483,7 @@ def _prompt_gemm_ok(x, w, b=None) -> bool:
         return False
     return (ok and M > 0 and K > 0 and ws[1] == K and w.is_contiguous() and unit == 1 and ld >= K
             and ld < 1 << 21 and K * (ws[0] + 256) < 1 << 29 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and (b is None or b.dtype == dt and b.device == x.device and b.is_contiguous() and not b.requires_grad))
+            and _bias_ok(b, w, x) and (b is None or not b.requires_grad))
 
 
 def _prompt_gemm(x, w, b, out, tanh_from=None, act: int = -1, limit: float = 0.0, alpha: float = 0.0, rows=None, tile: int = 0):
@@ -508,8 +514,7 @@ def linear(x, w, b=None, tanh_from=None, rows=None):
         if y is not None:
             return y
         x = x.rows()
-    if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or (b is not None and not (
-            b.dtype == x.dtype and b.is_cuda and b.is_contiguous())):
+    if x.dim() != 2 or x.shape[0] > 16 or not _skinny(x, w) or not _bias_ok(b, w, x):
         if _prompt_gemm_ok(x, w, b):
             y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
             if x.dtype == torch.bfloat16:

@@ -163,6 +163,17 @@ def test_other_forms_stay_with_the_library():
     assert sm.linear(x[:0], w.detach()).shape == (0, 64)
 
 
+@pytest.mark.parametrize("M", [3, 16, 40])
+def test_biases_of_other_shapes(M):
+    x, w = _case(M, 64, 128)
+    for b in (torch.full((1,), 0.75, device=DEV).bfloat16(), torch.randn(1, 64, device=DEV).bfloat16()):
+        assert not sm._bias_ok(b, w, x)
+        assert torch.equal(sm.linear(x, w, b), F.linear(x, w, b))
+    for b in (torch.randn(63, device=DEV).bfloat16(), torch.randn(65, device=DEV).bfloat16()):
+        with pytest.raises(RuntimeError):
+            sm.linear(x, w, b)
+
+
 def test_transforms_and_modes_are_served_as_by_the_library():
     from torch.autograd import forward_ad
     from torch.fx.experimental.proxy_tensor import make_fx
