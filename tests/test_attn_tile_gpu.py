@@ -39,7 +39,9 @@ def _close(got, want):
 
 @pytest.mark.parametrize("step", sorted(STEPS))
 @pytest.mark.parametrize("H,G,D,V", [(8, 2, 128, 128), (3, 1, 24, 40), (4, 4, 16, 8), (34, 2, 8, 16),
-                                     (4, 2, 136, 200), (16, 1, 64, 256)])
+                                     (4, 2, 136, 200), (16, 1, 64, 256),
+                                     # windows alone with both sides of 33 to 128: two sizes, padded ones, groups of 3 and 5
+                                     (6, 2, 64, 128), (6, 2, 128, 64), (8, 2, 72, 40), (10, 2, 96, 104)])
 @pytest.mark.parametrize("form", ["window", "sink", "biased", "blocks", "kept", "maps"])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_window_attention_tiles(step, H, G, D, V, form, dt):

@@ -104,11 +104,11 @@ def test_shared_tiles_are_as_exact_as_a_wavefront_each(scale, win, form):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("bad", [INF, -INF, NAN])
 @pytest.mark.parametrize("max_keys", [None, 700])
-@pytest.mark.parametrize("form", ["window", "blocks", "kept", "maps", "latent", "latent512"])
+@pytest.mark.parametrize("form", ["window", "padded", "blocks", "kept", "maps", "latent", "latent512"])
 def test_attention_keeps_values_that_are_not_finite_to_later_rows(dt, bad, max_keys, form):
     """Position 70's value is not finite: rows before it, and rows whose window has passed it, are as they were."""
     ent, row_ent, pos, bt, R, g = _step([150, 40], [0, 37], 2)
-    H, D = 4, 64 if form != "latent512" else 512
+    H, D = 4, {"latent512": 512, "padded": 72}.get(form, 64)
     M = 2 if form == "maps" else 1
     win = 50 if form != "window" else 1 << 30
     latent = form.startswith("latent")

@@ -1093,19 +1093,19 @@ def test_tiled_gemm_read_ahead(epi, tile, splitk, nk):
         tiled_config(2, 0, 0)
 
 
-@pytest.mark.parametrize("deep", [0, 2])
-@pytest.mark.parametrize("splitk", [1, 4])
-@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
+# whole K, four slices that were asked for, and the slices of either rule (18 tiles of 128 x 128: three without a round of
+# the CUs in mind, added up one after the other, and two that fill it, side by side)
+@pytest.mark.parametrize("splitk,deep,K", [(1, 1, 1024), (4, 1, 1024), (0, 0, 3072), (0, 1, 3072)])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("epi", ["store_norm", "silu", "resid"])
-def test_tiled_gemm_deep_stages(epi, tile, splitk, deep):
-    """Shallow (deep=0) and deep LDS pipelines (deep=2: as many stages as 160 KiB holds)
-    of every tile shape against the fp32 reference."""
+def test_tiled_gemm_slices(epi, tile, splitk, deep, K):
+    """Every tile shape with K whole and cut, by both rules (p2p_prefill_deep), against the fp32 reference."""
     from p2p_llm_chat_go_amd.ops import _lib
     from p2p_llm_chat_go_amd.ops.gemm import set_tiled_min_m, tiled_config
 
     L = _lib.lib()
     torch.manual_seed(tile * 10 + splitk)
-    M, K, N = 300, 1024, 768
+    M, N = 300, 768
     W = (torch.randn(N, K) * 0.05).to(torch.bfloat16)
     x = torch.randn(M, K).to(torch.bfloat16)
     Wt = ops.tile_weight(W).to(DEV)
