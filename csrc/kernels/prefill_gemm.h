@@ -811,13 +811,16 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
   return launch_stages<BM, BN, EPI, NORM, STAGES>(Wt, X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, st, splitk, ws, par);
 }
 
-// 128 x 128 tiles of eight wavefronts and two stages, of which a CU takes two
-template <int EPI, bool NORM>
+// Tiles of eight wavefronts and two stages, of which a CU takes two: one's start and end lie under the other's products.  192 x 128
+// of more than one round of the CUs run so (us, a workgroup with the CU to itself / two: normed 16640 x 512, 470 rows 25 / 21,
+// 10112 x 768, 2167 rows 62 / 49, SwiGLU 12288 x 2048, 700 rows 55 / 48, 22016 x 4096, 300 rows 96 / 93, 16640 x 7488, 569 rows
+// 169 / 157; over 60 shapes with K of 256 to 8192 between 28 % less and, 10240 x 8192, 878 rows, 163 / 168, 3 % more)
+template <int BM, int EPI, bool NORM>
 int launch_pairs(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off, void* out, int ldo, float eps,
                  const EpiArgs& ea, hipStream_t st) {
-  const int m_tiles = (M + 127) / 128, n_tiles = N / 128;
+  const int m_tiles = (M + BM - 1) / BM, n_tiles = N / 128;
   SplitArgs none{1, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-  hipLaunchKernelGGL((prefill_gemm_kernel<128, 128, EPI, NORM, false, 2>), dim3(m_tiles * n_tiles), dim3(NT), 0, st,
+  hipLaunchKernelGGL((prefill_gemm_kernel<BM, 128, EPI, NORM, false, 2>), dim3(m_tiles * n_tiles), dim3(NT), 0, st,
                      (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, none);
   return (int)hipGetLastError();
 }
@@ -831,8 +834,12 @@ int launch_tile(int tile, const void* Wt, const void* X, int ldx, int M, int K, 
     case 3: return launch<128, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 4: return launch<64, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 5: return launch<64, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
-    case 6: return launch_pairs<EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
-    case 7: return launch<192, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
+    case 6: return launch_pairs<128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
+    case 7:
+      if constexpr (EPI != EPI_RESID)   // (a residual read ahead leaves registers for one workgroup)
+        if (g_splitk <= 1 && (long)((M + 191) / 192) * (N / 128) > cu_count())
+          return launch_pairs<192, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
+      return launch<192, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 8: return launch<192, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 9:
       if constexpr (EPI != EPI_SILU)

@@ -1135,6 +1135,40 @@ def test_tiled_gemm_slices(epi, tile, splitk, deep, K):
     assert ops.tiled_split_fault() == 0
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 448])       # one stage of K, two, and more than are there at once
+@pytest.mark.parametrize("M", [257, 385])                # ragged rows of the second and the third tile
+@pytest.mark.parametrize("epi", ["store", "store_norm", "silu", "resid"])
+def test_tiled_gemm_rounds_of_192_rows(epi, M, K):
+    """192 x 128 tiles of more than a round of the CUs, which share a CU in pairs, against the fp32 product."""
+    from p2p_llm_chat_go_amd.ops.gemm import set_tiled_min_m, tiled_config
+
+    torch.manual_seed(M + K)
+    N = 128 * 130
+    W = (torch.randn(N, K) * 0.05).to(torch.bfloat16)
+    x = torch.randn(M, K).to(torch.bfloat16)
+    h = torch.randn(M, N).to(torch.bfloat16)
+    Wt, xd, hd = ops.tile_weight(W).to(DEV), x.to(DEV), h.to(DEV)
+    acc = x.float() @ W.float().t()
+    if epi in ("store_norm", "silu"):
+        acc = acc * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)
+    tiled_config(2, 7, 0)
+    set_tiled_min_m(1)
+    try:
+        if epi == "resid":
+            ops.skinny_gemm(Wt, xd, ops.EPI_RESID, out=hd)
+            out, ref = hd, h.float() + acc
+        elif epi == "silu":
+            out = ops.skinny_gemm(Wt, xd, ops.EPI_SILU, norm=True)
+            ref = torch.nn.functional.silu(acc[:, :N // 2]) * acc[:, N // 2:]
+        else:
+            out, ref = ops.skinny_gemm(Wt, xd, ops.EPI_STORE, norm=epi == "store_norm"), acc
+    finally:
+        set_tiled_min_m(65)
+        tiled_config(2, 0, 0)
+    # (one rounding to bf16, 2^-9 of each number at most, of fp32 sums of up to 448 products)
+    assert _rel(out.cpu(), ref) < 2 ** -8
+
+
 @pytest.mark.parametrize("cfg", [(2, 1, 1), (2, 1, 0), (2, 2, 1), (2, 3, 1), (2, 3, 2)])
 @pytest.mark.parametrize("epi", ["store_norm", "silu", "resid"])
 def test_tiled_gemm_grouped_order(epi, cfg):
