@@ -46,7 +46,12 @@ def test_every_width_of_128_columns_has_a_tile(epi):
     assert L.p2p_prefill_tile(2048, 3072, 1024, G.EPI_RESID) == 6     # short rows: two tiles to a CU
     # long rows: 128 x 256 in two slices of K, in four of 2048 and more, 128 x 128 where they would be shorter or eight
     for M, N, K, tile in ((1024, 4096, 14336, 2), (398, 4096, 14336, 2), (200, 4096, 14336, 3), (700, 4096, 6144, 2),
-                          (398, 4096, 6144, 3), (1024, 4096, 4096, 3)):
+                          (398, 4096, 6144, 3), (1024, 4096, 4096, 3),
+                          # 192 x 128 where 128 x 256 leaves a quarter of the CUs idle, from K = 8192 on
+                          (256, 4096, 14336, 3), (257, 4096, 14336, 7), (300, 4096, 14336, 7), (350, 4096, 14336, 7),
+                          (384, 4096, 14336, 7), (385, 4096, 14336, 2), (576, 4096, 14336, 2), (577, 4096, 14336, 7),
+                          (700, 4096, 14336, 7), (768, 4096, 14336, 7), (769, 4096, 14336, 2), (700, 4096, 8192, 7),
+                          (700, 4096, 8128, 2)):
         assert L.p2p_prefill_tile(M, N, K, G.EPI_RESID) == tile, (M, N, K)
     # SwiGLU widths: the tile whose rounds of 256 CUs are the shortest
     for M, N, tile in ((128, 28672, 3), (150, 28672, 7), (250, 28672, 2), (300, 28672, 8), (500, 28672, 1), (700, 28672, 2),

@@ -1135,6 +1135,27 @@ def test_tiled_gemm_slices(epi, tile, splitk, deep, K):
     assert ops.tiled_split_fault() == 0
 
 
+@pytest.mark.parametrize("M,tile", [(257, 7), (300, 7), (384, 7), (385, 2), (700, 7), (769, 2)])
+def test_residual_products_of_long_rows(M, tile):
+    """Where 192 x 128 tiles with four (two) slices of K take over from 128 x 256 and back: their slices add up shares of one,
+    two and three fragment rows each and have read the residual ahead."""
+    from p2p_llm_chat_go_amd.ops import _lib
+
+    N, K = 4096, 14336
+    assert _lib.lib().p2p_prefill_tile(M, N, K, ops.EPI_RESID) == tile
+    torch.manual_seed(M)
+    W = (torch.randn(N, K) * 0.01).to(torch.bfloat16)
+    x, h = torch.randn(M, K, device=DEV).to(torch.bfloat16), torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    Wt, Wd = ops.tile_weight(W).to(DEV), W.to(DEV)
+    want = h.double() + x.double() @ Wd.double().t()
+    mag = h.double().abs() + x.double().abs() @ Wd.double().abs().t()
+    ops.skinny_gemm(Wt, x, ops.EPI_RESID, out=h)
+    assert ops.tiled_split_fault() == 0
+    # one rounding to bf16 of fp32 sums: each of K additions off by 2^-24 of what the magnitudes sum to at most
+    sums = K * 2.0 ** -24 * mag
+    assert bool(((h.double() - want).abs() <= 2.0 ** -8 * (want.abs() + sums) + sums).all())
+
+
 @pytest.mark.parametrize("K", [64, 128, 192, 448])       # one stage of K, two, and more than are there at once
 @pytest.mark.parametrize("M", [257, 385])                # ragged rows of the second and the third tile
 @pytest.mark.parametrize("epi", ["store", "store_norm", "silu", "resid"])
@@ -1165,7 +1186,7 @@ def test_tiled_gemm_rounds_of_192_rows(epi, M, K):
     finally:
         set_tiled_min_m(65)
         tiled_config(2, 0, 0)
-    # (one rounding to bf16, 2^-9 of each number at most, of fp32 sums of up to 448 products)
+    # (one rounding to bf16, 2^-8 of each number at most, of fp32 sums of up to 448 products)
     assert _rel(out.cpu(), ref) < 2 ** -8
 
 
