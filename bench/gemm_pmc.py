@@ -1,6 +1,6 @@
 """PMC target: the prefill GEMM at two operating points, each launched 5 times with
 the tile forced -- gate_up at 288 rows on the 192x256 tile (mid-M) and at
-8192 rows on the phased 256x256 tile (large M) -- so rocprofv3 --pmc rows can be
+8192 rows on the 256x256 tile (large M) -- so rocprofv3 --pmc rows can be
 compared per k-step (scripts/gemm_pmc.sh)."""
 import os
 import sys

@@ -1,5 +1,5 @@
 """End-to-end A/B of a kernel library switch (a p2p_prefill_* setter in tiled_gemm.hip:
-pre_rstd, tile8, deep, phased), set before the engine is built, around bench.py.
+pre_rstd, tile8, deep), set before the engine is built, around bench.py.
 Run on the GPU: python bench/switch_ab.py p2p_prefill_tile8 {0|1} [bench.py args]"""
 import os
 import sys

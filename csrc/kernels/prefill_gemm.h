@@ -12,7 +12,7 @@
 //   * X is row-major: a block is 8 rows x 128 bytes, whole lines (a CU takes those
 //     in at 95 to 100 KB/us, the 16 rows x 64 bytes of a fragment at 58), 16-byte
 //     piece p of row R at p ^ (R & 7).
-// LDS holds two to six stages of (BM+BN) x 64 bf16 (stages_for, deep_stages_for): later
+// LDS holds two to five stages of (BM+BN) x 64 bf16 (stages_for, launch_pairs): later
 // stages are in flight while the MFMAs consume stage kt; one barrier per
 // k-tile.  Blocks sharing a weight n-tile are consecutive after the XCD remap.
 // NORM: the waves of column 0 also square the A fragments they read; a lane
@@ -121,7 +121,7 @@ __device__ __forceinline__ void pin_scalars(const T&... v) {
   (pin_scalar(v), ...);
 }
 
-// Tiles that read ahead (a workgroup has the CU to itself): 128 rows and more.  In step, eight wavefronts read a half stage,
+// Tiles that read ahead (a workgroup has the CU to itself): 128 rows and more (but see launch_pairs).  In step, eight wavefronts read a half stage,
 // waited, multiplied it, and issued the copies between.  These read the next half stage a fragment row at a time under the
 // products of the present one, and issue their copies (a scalar address and a lane's constant offset) between the products, into
 // the stage whose second half every wave has in registers.  llama3.1-8B, us: down, 1024 rows, in step 173, on four wavefronts
@@ -134,16 +134,15 @@ constexpr bool reads_ahead() {
   return BM >= 128 && (STAGES >= 3 || BM * BN >= 192 * 256);
 }
 
-template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES, int NWV = 8>
-__global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
+template <int BM, int BN, int EPI, bool NORM, bool SPLIT, int STAGES>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void prefill_gemm_kernel(const bf16x8* __restrict__ Wt,
                                                           const bf16* __restrict__ X, int ldx,
                                                           int M, int K, int m_tiles, int n_tiles,
                                                           int up_off, void* __restrict__ out,
                                                           int ldo, float eps, EpiArgs ea,
                                                           SplitArgs sp) {
   constexpr bool PIPE = reads_ahead<BM, BN, STAGES, NORM>();
-  constexpr int NT = NWV * 64;
-  constexpr int WN = NWV / 2;        // 2 x WN wave grid
+  constexpr int NWV = NT / 64, WN = NWV / 2;   // 2 x WN wave grid
   constexpr int FM = BM / 32;        // 16-row fragments per wave
   constexpr int FN = BN / (16 * WN);  // 16-col groups per wave
   constexpr int AB = BM / 16 * 2;    // A fragment blocks per stage (x 1 KiB)
@@ -733,14 +732,13 @@ constexpr int stages_for() {
   return BN <= 128 ? 4 : 3;
 }
 
-// 1: K slices fill one round of the CUs where a tile has a CU to itself; 0, 2 (A/B): some 400 workgroups whatever the tile
-static int g_fill = 1;
+// K slices fill one round of the CUs where a tile has a CU to itself; not (A/B): some 400 workgroups whatever the tile
+static bool g_fill = true;
 
 template <int BM, int BN, int EPI, bool NORM, int STAGES>
 int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_tiles, int n_tiles,
                   int up_off, void* out, int ldo, float eps, const EpiArgs& ea, hipStream_t st,
                   int splitk, char* ws, int par) {
-  constexpr int NWV = 8;
   constexpr size_t SHM = reads_ahead<BM, BN, STAGES, NORM>() ? (size_t)STAGES * (BM + BN) * BK * sizeof(bf16) : 0;
   const int tiles = m_tiles * n_tiles;
   auto with_lds = [](const void* k) {
@@ -748,7 +746,7 @@ int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_ti
   };
   if constexpr (splits_k<BM, BN>()) {
     if (splitk > 1) {
-      constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, true, STAGES, NWV>;
+      constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, true, STAGES>;
       if (const hipError_t e = with_lds((const void*)kernel)) return (int)e;
       const size_t slab = (size_t)tiles * splitk * BM * BN * sizeof(float);
       // counters live at the END of the workspace at a fixed offset from the end so a
@@ -759,15 +757,15 @@ int launch_stages(const void* Wt, const void* X, int ldx, int M, int K, int m_ti
       int* fw = p2p_split_fault_word_ptr(st);
       SplitArgs sp{splitk, (f32x4*)ws, (float*)(ws + slab), ctr, ctr + nw / 2,
                    fw ? fw : (int*)(ctr + nw - 1), par};
-      hipLaunchKernelGGL(kernel, dim3(tiles * splitk), dim3(NWV * 64), SHM, st, (const bf16x8*)Wt,
+      hipLaunchKernelGGL(kernel, dim3(tiles * splitk), dim3(NT), SHM, st, (const bf16x8*)Wt,
                          (const bf16*)X, ldx, M, K, m_tiles, n_tiles, up_off, out, ldo, eps, ea, sp);
       return (int)hipGetLastError();
     }
   }
   SplitArgs none{1, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-  constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, false, STAGES, NWV>;
+  constexpr auto kernel = prefill_gemm_kernel<BM, BN, EPI, NORM, false, STAGES>;
   if (const hipError_t e = with_lds((const void*)kernel)) return (int)e;
-  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(NWV * 64), SHM, st, (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles,
+  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(NT), SHM, st, (const bf16x8*)Wt, (const bf16*)X, ldx, M, K, m_tiles,
                      n_tiles, up_off, out, ldo, eps, ea, none);
   return (int)hipGetLastError();
 }
@@ -782,10 +780,10 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
   const int nk = K / BK;
   const int cus = cu_count();
   constexpr bool ALONE = BM >= 128 && BM * BN <= 128 * 256;   // one workgroup per CU whatever the grid
-  const bool fill = ALONE && g_fill == 1 && cus > 0 && tiles <= cus;
+  const bool fill = ALONE && g_fill && cus > 0 && tiles <= cus;
   // too few tiles to fill 256 CUs: split K so every CU gets work (>= 4 k-tiles per slice)
-  // (measured on MI355X at 8B shapes: ~400 blocks, >= 16 k-tiles per slice); the deep
-  // variant keeps the grid at one block per CU instead (power-of-two slices <= CUs/tiles)
+  // (measured on MI355X at 8B shapes: ~400 blocks, >= 16 k-tiles per slice); tiles that have a
+  // CU to themselves keep to one block per CU instead (power-of-two slices <= CUs/tiles)
   int splitk;
   if (g_splitk) {
     splitk = g_splitk;
@@ -864,18 +862,19 @@ static int pick_tile(int M, int N, int K, int epi) {
   const int cus = cu_count() > 0 ? cu_count() : 256;
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * (N / bn); };
   // (one-m-tile 384 / 448-row tiles for 321-448 rows measured 1.1-1.3x SLOWER than the
-  // 128x128 split-K / phased 256x256 picks below and were removed:
+  // 128x128 split-K / 256x256 picks of that time and were removed:
   // profiles/r3_prefill_tiles_384_448.jsonl)
   const long small = tiles(128, 128);
   const bool resid = epi == EPI_RESID;
   if (small <= cus) {
     // One round of 128 x 128 tiles, K cut where they leave CUs idle.  128 x 256 tiles copy a quarter less per product and
     // take twice the slices: they pay where a slice keeps 2048 numbers and four slices fill the chip.  Residual, us,
-    // 128 x 128 / 128 x 256: 4096 x 14336, 300, 398, 512, 1024 rows 62 / 58, 68 / 61, 76 / 64, 125 / 111 (1080 TFLOP/s);
-    // 4096 x 8192, 398 and 1024 rows 43 / 41, 71 / 71; eight slices: 4096 x 14336, 72 and 128 rows 32 / 39, 34 / 42;
-    // 4096 x 4096, 1024 rows 37 / 43.  192 x 128 where its slices fill the chip and those of 128 x 256 leave a quarter of it idle
-    // (128 x 256 / 192 x 128, 4096 x 14336, 300, 350, 580, 700, 768 rows 58 / 52, 61 / 55, 97 / 85, 98 / 92, 104 / 92, 4096 x 8192,
-    // 700 rows 63 / 55)
+    // 128 x 128 / 128 x 256: 4096 x 14336, 300, 398, 512, 1024 rows 62 / 57, 66 / 61, 76 / 65, 126 / 111 (1080 TFLOP/s);
+    // 4096 x 8192, 398 and 1024 rows 43 / 42, 73 / 71; eight slices: 4096 x 14336, 72 and 128 rows 33 / 39, 34 / 42;
+    // 4096 x 4096, 1024 rows 40 / 44.  192 x 128 where its slices fill the chip and those of 128 x 256 leave a quarter of it idle
+    // (128 x 256 / 192 x 128, 4096 x 14336, 300, 350, 580, 700, 768 rows 57 / 52, 61 / 55, 96 / 84, 99 / 89, 104 / 93, 4096 x 8192,
+    // 700 rows 65 / 57).  The lengths between 6144 and 8191 were measured later and say the same, the line does not yet: 4096 x
+    // 6144, 580, 700, 768 rows 49 / 45, 50 / 47, 52 / 48, 4096 x 7168 56 / 50, 57 / 52, 59 / 54
     const long wide = N % 256 == 0 ? tiles(128, 256) : 0;
     if (!(wide * 8 > cus && K >= 6144 && K >= (wide * 4 > cus ? 2 : 4) * 2048 && wide <= cus)) return 3;
     auto blocks = [&](long t) {   // with the slices that launch() cuts K into
@@ -886,24 +885,25 @@ static int pick_tile(int M, int N, int K, int epi) {
     const long tall = tiles(192, 128);
     return K >= 8192 && tall <= cus && blocks(wide) * 4 <= cus * 3l && blocks(tall) * 8 > cus * 7l ? 7 : 2;
   }
-  if (N >= 16384 && M > 128 && M <= 192) return 7;   // one row of tiles, 192 x 128: SwiGLU 28672 x 4096 62 us, 128 x 128 81
+  if (N >= 16384 && M > 128 && M <= 192) return 7;   // one row of tiles, 192 x 128: SwiGLU 28672 x 4096 60 us, 128 x 128 80
   // A residual product with a short K that gives 160 tiles of 256 x 256 and more waits for its residual and its first and last
   // stages: pairs of workgroups per CU hide that, but where the larger tiles' last round fills the CUs and K gives them time.
-  // us, pairs / 128 x 256 / 256 x 256: 8192 x 1024, 2048 rows 59 / 68 / 62, 8192 x 3072, 2048 rows 115 / 117 / 110,
-  // 1500 rows 93 / 106 / 104, 6144 x 2048, 4096 rows 124 / 131 / 160
+  // The line was drawn when tiles loaded the residual behind their products (us, pairs / 128 x 256 / 256 x 256: 8192 x 1024, 2048
+  // rows 59 / 68 / 62, 8192 x 3072, 2048 rows 115 / 117 / 110, 1500 rows 93 / 106 / 104, 6144 x 2048, 4096 rows 124 / 131 / 160).
+  // They load it before them now, and the larger ones have gained more: 44 / 46 / 40, 110 / 99 / 87, 94 / 89 / 76, 113 / 104 / 112
   if (resid && K <= 3072 && N % 256 == 0 && tiles(256, 256) >= 160) {
     const long last = tiles(256, 256) % cus;
     return K >= 2560 && (last == 0 || last * 6 > cus * 5) ? 1 : 6;
   }
   if (N % 256 == 0 && !(resid && K <= 3072)) {
-    // More than a round of 128 x 128: the tile whose rounds of the CUs take the shortest time.  Relative times of a round,
-    // from SwiGLU of 16384 to 36864 columns and K = 2048 and 4096 (us at 4096, 256 x 256 / 192 x 256 / 128 x 256 /
-    // 192 x 128; in brackets what the lines by rows before had): 28672 columns, 250 rows 126 / 95 / 68 / 91 [85], 300 rows
-    // 107 / 94 / 108 / - [100], 512 rows 113 / 174 / 119 / 145 [119], 600 rows 202 / 179 / 161 / 174 [190], 1024 rows 211 /
-    // 257 / 225 / - [213]; 22016 columns, 300 rows 104 / 130 / 98 / 85 [104], 600 rows 198 / 174 / 116 / 141 [188]; 36864
-    // columns, 300 rows 203 / 176 / 116 / 145 [194]; 12288 x 2048, 400 rows 58 / - / 32 / 44 [43], 700 rows 98 / - / 57 /
-    // 49 [79].  128 x 192, without SwiGLU: 6144 x 4096, 700 rows 46, 128 x 256 51, 192 x 128 52.  192 x 256 up to 200 tiles:
-    // launch() cuts K there as well (22016 columns above); 256 x 256 from 160 tiles.
+    // More than a round of 128 x 128: the tile whose rounds of the CUs take the shortest time.  The relative times of a round are
+    // from SwiGLU of 16384 to 36864 columns and K = 2048 and 4096 on kernels of which 256 x 256 and 192 x 256 have become 10 %
+    // faster; what they pick is the best, or 1 % from it, on these too.  us with norm, 256 x 256 / 192 x 256 / 128 x 256 / 192 x
+    // 128 at K = 4096: 28672 columns, 250 rows 125 / 93 / 69 / 97, 300 rows 101 / 93 / 111 / 96, 398 rows 104 / 159 / 114 / 147,
+    // 512 rows 104 / 164 / 122 / 148, 600 rows 183 / 168 / 168 / 178, 1024 rows 201 / 242 / 229 / 264; 22016 columns, 300 rows
+    // 94 / 129 / 101 / 90, 600 rows 169 / 159 / 116 / 144; 36864 columns, 300 rows 180 / 166 / 117 / 146; 12288 x 2048, 400 rows
+    // 56 / 71 / 33 / 45, 700 rows 92 / 91 / 59 / 50.  128 x 192, without SwiGLU: 6144 x 4096, 700 rows 48, 128 x 256 54, 192 x
+    // 128 48.  192 x 256 from 200 tiles: launch() cuts K below; 256 x 256 from 160 tiles.
     auto time = [&](int bm, int bn, int round) { return (tiles(bm, bn) + cus - 1) / cus * round; };
     int best = 2;
     long t = time(128, 256, 57);
@@ -917,15 +917,16 @@ static int pick_tile(int M, int N, int K, int epi) {
     return best;
   }
   // 128 x 128 takes more than one round, a workgroup per CU: a larger tile that takes one.  us, 128 x 128 / 192 x 128 /
-  // 128 x 192: normed 9216 x 4096, 448 rows 74 / 68 / 50; residual 6144 x 2048, 700 rows 57 / 47 / 44
+  // 128 x 192: normed 9216 x 4096, 448 rows 71 / 49 / 49; residual 6144 x 2048, 700 rows 37 / 26 / 25
   const bool tall = tiles(192, 128) <= cus;
   if (!(resid && K <= 1024) && tile_fits(9, N, epi) && tiles(128, 192) <= cus) return 9;
   if (tall) return 7;
-  // no tile takes one.  Two workgroups on a CU hide what one waits for: the reads of the residual, the first and the last
-  // stages of a short K (pairs / 128 x 192 / 128 x 256: residual 3072 x 1024, 2048 rows 35 / 37 / 38, 11264 x 2368, 456
-  // rows 57 / - / 64, 22016 x 4096, 256 rows 95 / - / 91; pairs / 128 x 128: 8320 x 1024, 600 rows 28 / 31,
-  // 8320 x 4096, 600 rows 77 / 72, residual 86 / 91); over more rounds 192 x 128 has fewer (10112 x 768, 2167 rows
-  // 55 / 58 / 69 with 128 x 128, 8320 x 4096, 1042 rows 110 / 137 / 105)
+  // no tile takes one.  Two workgroups on a CU hide what one waits for: the first and the last stages of a short K, and, when
+  // the lines were drawn, the reads of the residual, which are ahead of the products now (us then; now: pairs / 128 x 192 / 128 x
+  // 256: residual 3072 x 1024, 2048 rows 35 / 37 / 38; 22 / 20 / 21, 11264 x 2368, 456 rows 57 / - / 64; 43 / - / 37, SwiGLU 22016
+  // x 4096, 256 rows 95 / - / 91; 78 / - / 64; pairs / 128 x 128: 8320 x 1024, 600 rows 28 / 31; 20 / 23, 8320 x 4096, 600 rows
+  // 77 / 72; 61 / 70, residual 86 / 91; 63 / 71); over more rounds 192 x 128 has fewer (192 x 128 / pairs / 128 x 128 now: 10112
+  // x 768, 2167 rows 46 / 48 / 61, residual 66 / 53 / 68, 8320 x 4096, 1042 rows 90 / 115 / 101)
   const bool two = small <= 2 * cus;
   if (N % 256 == 0) return resid && two && K <= 3072 ? 6 : 2;
   if (two) return K <= (resid ? 4096 : 1024) ? 6 : 3;

@@ -201,8 +201,8 @@ static int g_tiled_version = 2;  // 2 = LDS-DMA 8-wave kernel (prefill_gemm.h), 
 // Benchmarks / A-B tests (p2p_tiled_gemm_config): version 1|2, tile 0 (heuristic) or 1..9 (256x256, 128x256, 128x128,
 // 64x128, 64x256, 128x128 two to a CU, 192x128, 192x256, 128x192),
 // splitk 0 (heuristic), 1 (off) or a forced K-slice count.
-// K slices of tiles that have a CU to themselves (A/B): 1 = a round of the CUs (default), 0 and 2 = some 400 workgroups.
-P2P_API void p2p_prefill_deep(int mode) { pgemm::g_fill = (mode >= 0 && mode <= 2) ? mode : 1; }
+// K slices of tiles that have a CU to themselves (A/B): 1 = a round of the CUs (default), 0 (or 2) = some 400 workgroups.
+P2P_API void p2p_prefill_deep(int mode) { pgemm::g_fill = mode != 0 && mode != 2; }
 // Precomputed per-row rstd for normed prefill GEMMs (A/B): 1 = on (default), 0 = in-loop sums.
 P2P_API void p2p_prefill_pre_rstd(int on) { pgemm::g_pre_rstd = on ? 1 : 0; }
 // 192 x 256 tiles where their rounds are the shortest (A/B): 1 = on (default)

@@ -41,8 +41,8 @@ class HybridDecodeGraph:
     a captured hipGraph: metadata in, forward, greedy argmax, tokens out.  A step writes its
     metadata into page-locked memory that the graph's first kernel reads, replays, and finds its
     tokens where the last kernel left them; rows beyond the live ones are padding on the
-    null page and the null state slot.  (Around the replay, 8 rows: metadata as tensors, a copy before it and one behind it
-    96 us of host time, page-locked memory 40.)"""
+    null page and the null state slot.  (A step of 8 rows beside its replay and the wait for it: metadata as
+    tensors, a copy before it and one behind it 66 us, page-locked memory 8.)"""
 
     def __init__(self, model: HybridModel, rows: int, maxp: int):
         self.model, self.rows, self.maxp = model, rows, maxp

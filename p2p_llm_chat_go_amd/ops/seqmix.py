@@ -327,21 +327,24 @@ def embed_rows(embed, ids, out, h_out=None, scale: float = 1.0):
 
 
 def _skinny(x, w) -> bool:
-    """Products that ``csrc/seqmix/skinny.hip`` takes: at most 16 rows of one matrix instruction.  Where
-    the lines lie (a captured graph, cold weights, library -> kernel in us, 8 rows unless others are named):
+    """Products that ``csrc/seqmix/skinny.hip`` takes: at most 16 rows of one matrix instruction.  The lines were drawn against
+    the library, which took the rest; ``csrc/seqmix/prompt_gemm.h`` takes it now.  us in a captured graph, cold weights, library /
+    this kernel / prompt_gemm.h, 8 rows unless others are named:
 
-    * bf16, K up to 2048 (activations kept in registers where that pays, skinny.hip): 12288 x 2048 16.1 -> 12.1, 24576 x
-      2048 37.3 -> 21.8, 128256 x 2048 109 -> 97, 16 rows 108 -> 97; up to 1536 by N, because a tile is small against the
-      sums and barrier that end it: 32000 x 1536 25.7 -> 20.9, 65536 x 1536 40.8 -> 40.5, 128256 x 1536 75 -> 79, 32000 x
-      640 15.2 -> 13.4, 65536 x 640 19.7 -> 27.7; up to 256 sooner: 16384 x 256 6.4 -> 4.3, 16384 x 64 4.5 -> 3.0, 16 rows
-      8192 x 256 5.7 -> 3.7, 8192 x 64 3.6 -> 2.5.
-    * fp32, K up to 1024, the same kernel: 12288 x 1024 31.6 -> 12.9, 32000 x 512 19.0 -> 17.3, 65536 x 512 28.8 -> 31.8,
-      32000 x 128 9.2 -> 8.3, 50257 x 128 10.7 -> 9.4, 128256 x 64 16.9 -> 13.6, 128256 x 1024 106 -> 92, 16384 x 768 13.8 ->
-      12.0; few columns are left to the kernel of any rows.
-    * Longer K, one workgroup per tile walks all of it: bf16 2048 x 8192 12.9 -> 15.0, 2048 x 4096 12.5 -> 8.3, 4096 x
-      4096 15.6 -> 9.9, 6144 x 3072 11.9 -> 13.0, 4 rows 12288 x 4096 24.1 -> 21.1, 16 rows 96 x 4096 7.9 -> 8.9, 8 rows
-      7.9 -> 7.6; fp32 2048 x 4096 13.2 -> 15.0, 2048 x 2048 10.5 -> 8.5, 16 rows 4608 x 2048 14.1 -> 16.4, 1024 x 2048
-      8.6 -> 9.8, 8 rows 8.7 -> 8.5, 96 x 2048 6.7 -> 7.7.
+    * bf16, K up to 2048 (activations kept in registers where that pays, skinny.hip): 12288 x 2048 15.1 / 11.3 / 12.4, 24576 x
+      2048 37.3 / 20.6 / 25.1, 128256 x 2048 110 / 96 / 100, 16 rows 109 / 100 / 104; up to 1536 by N, because a tile is small
+      against the sums and barrier that end it: 32000 x 1536 25.8 / 19.7 / 21.6, 65536 x 1536 40.7 / 37.6 / 38.7, 128256 x 1536
+      76 / 73 / 74, 32000 x 640 15.0 / 12.0 / 10.1, 65536 x 640 18.9 / 20.9 / 18.3; up to 256 sooner: 16384 x 256 6.3 / 4.1 / 4.0,
+      16384 x 64 4.4 / 2.8 / 3.1, 16 rows 8192 x 256 5.5 / 3.5 / 3.6, 8192 x 64 3.9 / 2.2 / 2.7.
+    * fp32, K up to 1024, the same kernel: 12288 x 1024 31.0 / 11.8 / 17.1, 32000 x 512 17.5 / 15.3 / 21.8, 65536 x 512 26.9 /
+      29.7 / 41.7, 32000 x 128 9.2 / 6.5 / 8.8, 50257 x 128 10.4 / 8.7 / 15.3, 128256 x 64 16.9 / 13.9 / 17.8, 128256 x 1024
+      121 / 96 / 127, 16384 x 768 14.1 / 11.8 / 16.1; few columns are left to the kernel of any rows.
+    * Longer K, one workgroup per tile walks all of it: bf16 2048 x 8192 12.9 / 15.0 / 12.1, 2048 x 4096 14.7 / 8.7 / 7.5, 4096 x
+      4096 15.4 / 10.5 / 9.0, one row 15.6 / 9.3 / 9.0, 6144 x 3072 13.2 / 13.5 / 10.0, 4 rows 12288 x 4096 29.0 / 23.7 / 22.8, 16
+      rows 96 x 4096 7.6 / 8.7 / 5.9, 8 rows 7.7 / 7.4 / 5.9; fp32 2048 x 4096 13.0 / 14.6 / 15.1, 2048 x 2048 11.9 / 8.8 / 9.2, 16
+      rows 4608 x 2048 14.8 / 19.0 / 14.3, 1024 x 2048 8.3 / 9.3 / 8.6, 8 rows 8.4 / 8.0 / 8.5, 96 x 2048 6.5 / 7.5 / 8.1.
+
+    So bf16 of K above 2048, and 32000 x 640, would be 1 to 2 us better off there; the lines do not say so yet.
 
     The rest: what 16-byte loads need."""
     M, K = x.shape
@@ -469,7 +472,7 @@ def _bias_ok(b, w, x) -> bool:
 
 def _prompt_gemm_ok(x, w, b=None) -> bool:
     """Products that ``csrc/seqmix/prompt_gemm.h`` takes: K in stages of 128 bytes, rows that 16-byte copies can read; or one
-    stage of 64 (the low-rank decays, 1024 columns of K = 32: the host spends 20 us on the library's call and 10 on this)."""
+    stage of 64 (the low-rank decays, 1024 columns of K = 32: the host spends 18 us on the library's call and 8 on this)."""
     dt, xs, ws = x.dtype, x.shape, w.shape
     if len(xs) != 2 or len(ws) != 2 or dt != w.dtype or not x.is_cuda or x.get_device() != w.get_device() or x.requires_grad \
             or w.requires_grad or type(x) not in _PLAIN or type(w) not in _PLAIN or not _by_address():
@@ -499,11 +502,11 @@ def linear(x, w, b=None, tanh_from=None, rows=None):
     (``_prompt_gemm_ok``).  tanh_from: columns from there on pass a tanh (of the rounded result).  rows: int32, which rows of
     x (default: all).  x may be ``NormedRows`` (whose only product this is).
 
-    Why not the library's: a call of it costs 21 us of host time, this one 6, and prompts of a few hundred rows
+    Why not the library's: a call of it costs 18 us of host time, this one 8 with its checks, and prompts of a few hundred rows
     wait for the host; and it is slower itself, by 20 % on average over 192 to 16384 columns, K 128 to 8192 and 20 to 2644
     rows (10304 x 2048, 2048 rows 100 -> 84 us, 2048 x 8192, 2048 rows 82 -> 65, 2048 x 2048, 48 rows 8.6 -> 5.0; one of the few
-    the other way: 8192 x 2048, 1300 rows 43.5 -> 46).  8 rows of shapes that ``_skinny`` leaves: 2048 x 8192 11.2 -> 10.6, 96 x
-    4096 8.0 -> 6.1, 6144 x 3072 10.9 -> 8.6, 32000 x 4096 58 -> 51.  float32: 5 % (prompt_gemm_f32.hip)."""
+    the other way: 8192 x 2048, 1300 rows 43.5 -> 46).  8 rows of shapes that ``_skinny`` leaves: 2048 x 8192 12.9 -> 12.1,
+    6144 x 3072 13.2 -> 10.0, 32000 x 4096 60 -> 51, 16 rows of 96 x 4096 7.6 -> 5.9.  float32: 5 % (prompt_gemm_f32.hip)."""
     if rows is not None:
         if (x.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and rows.shape[0] > 0 and b is None
                 and tanh_from is None and x.shape[0] * x.stride(0) < 1 << 29 and _prompt_gemm_ok(x, w)):
@@ -1536,7 +1539,10 @@ def latent_forms(ent_host: list, win: int) -> bool:
     layer's attention with its products, in latent space / formed, us (latents of 512 and a window of 1024, of 448 with a rotated
     part; 16 heads of 128, the latter also 8): 16 rows 38 / 37, 51 / 46, 40 / 37, 32 rows 50 / 40, 66 / 52, 55 / 43, 256 rows
     85 / 58, 95 / 65, 85 / 53, 2048 rows 181 / 90, 259 / 118; 256 rows behind 1024 100 / 75, 112 / 85, 95 / 77; 512 rows behind 3072
-    110 / 78, 174 / 136, 122 / 121."""
+    110 / 78, 174 / 136, 122 / 121.  A running sequence beside a prompt is walked by one workgroup per head, and the rule holds all
+    the same: whole steps of two latent layers among others (widths 2048, 2048 and 1024), 256 rows + one behind 1000 1280 / 1226, 1123 / 1009, 1100 / 983, 512 + one behind
+    2400 1566 / 1513, 1441 / 1286, 1154 / 1048, 2048 + one behind 3900 3360 / 3303, 3198 / 2501, 2202 / 1610, 300 + four behind 350
+    1418 / 1399, 1213 / 1101, 1226 / 1084."""
     rows = sum(e[1] for e in ent_host)
     keys = sum(min(e[2], win - 1) + e[1] for e in ent_host)
     return rows >= 32 and max(e[1] for e in ent_host) > 1 and keys <= 6 * rows
