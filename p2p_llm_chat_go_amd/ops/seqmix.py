@@ -499,14 +499,16 @@ def _prompt_gemm(x, w, b, out, tanh_from=None, act: int = -1, limit: float = 0.0
 
 def linear(x, w, b=None, tanh_from=None, rows=None):
     """x [M, K] times w [N, K] transposed, plus b [N]: ``F.linear``, on kernels of few rows (``_skinny``) and of any
-    (``_prompt_gemm_ok``).  tanh_from: columns from there on pass a tanh (of the rounded result).  rows: int32, which rows of
-    x (default: all).  x may be ``NormedRows`` (whose only product this is).
+    (``_prompt_gemm_ok``).  tanh_from: columns from there on (negative: that many from the end) pass a tanh (of the rounded
+    result).  rows: int32, which rows of x (default: all).  x may be ``NormedRows`` (whose only product this is).
 
     Why not the library's: a call of it costs 18 us of host time, this one 8 with its checks, and prompts of a few hundred rows
     wait for the host; and it is slower itself, by 20 % on average over 192 to 16384 columns, K 128 to 8192 and 20 to 2644
     rows (10304 x 2048, 2048 rows 100 -> 84 us, 2048 x 8192, 2048 rows 82 -> 65, 2048 x 2048, 48 rows 8.6 -> 5.0; one of the few
     the other way: 8192 x 2048, 1300 rows 43.5 -> 46).  8 rows of shapes that ``_skinny`` leaves: 2048 x 8192 12.9 -> 12.1,
     6144 x 3072 13.2 -> 10.0, 32000 x 4096 60 -> 51, 16 rows of 96 x 4096 7.6 -> 5.9.  float32: 5 % (prompt_gemm_f32.hip)."""
+    if tanh_from is not None and tanh_from < 0:
+        tanh_from = max(0, w.shape[0] + tanh_from)
     if rows is not None:
         if (x.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and rows.shape[0] > 0 and b is None
                 and tanh_from is None and x.shape[0] * x.stride(0) < 1 << 29 and _prompt_gemm_ok(x, w)):

@@ -174,6 +174,17 @@ def test_biases_of_other_shapes(M):
             sm.linear(x, w, b)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [3, 40])
+def test_tanh_of_the_last_columns(M, dt):
+    x, w = _case(M, 64, 128, dtype=dt)
+    z = sm.linear(x, w)
+    for n in (5, 64, 70):
+        y = sm.linear(x, w, tanh_from=-n)
+        assert torch.equal(y, sm.linear(x, w, tanh_from=max(0, 64 - n)))
+        assert torch.equal(y[:, :max(0, 64 - n)], z[:, :max(0, 64 - n)]) and not torch.equal(y, z)
+
+
 def test_transforms_and_modes_are_served_as_by_the_library():
     from torch.autograd import forward_ad
     from torch.fx.experimental.proxy_tensor import make_fx
