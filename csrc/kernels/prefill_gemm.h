@@ -812,7 +812,9 @@ int launch(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_o
 // Tiles of eight wavefronts and two stages, of which a CU takes two: one's start and end lie under the other's products.  192 x 128
 // of more than one round of the CUs run so (us, a workgroup with the CU to itself / two: normed 16640 x 512, 470 rows 25 / 21,
 // 10112 x 768, 2167 rows 62 / 49, SwiGLU 12288 x 2048, 700 rows 55 / 48, 22016 x 4096, 300 rows 96 / 93, 16640 x 7488, 569 rows
-// 169 / 157; over 60 shapes with K of 256 to 8192 between 28 % less and, 10240 x 8192, 878 rows, 163 / 168, 3 % more)
+// 169 / 157; over 60 shapes with K of 256 to 8192 between 28 % less and, 10240 x 8192, 878 rows, 163 / 168, 3 % more.  So do SwiGLU's
+// of a short K in one round, which end before four stages pay (7424 x 320, 557 rows 13.9 / 12.8, 7680 x 832, 692 rows 18.9 / 18.4,
+// but 18176 x 1216, 137 rows 23.6 / 26.8; without SwiGLU 8320 x 384, 537 rows 14.6 / 14.8)
 template <int BM, int EPI, bool NORM>
 int launch_pairs(const void* Wt, const void* X, int ldx, int M, int K, int N, int up_off, void* out, int ldo, float eps,
                  const EpiArgs& ea, hipStream_t st) {
@@ -835,7 +837,7 @@ int launch_tile(int tile, const void* Wt, const void* X, int ldx, int M, int K, 
     case 6: return launch_pairs<128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 7:
       if constexpr (EPI != EPI_RESID)   // (a residual read ahead leaves registers for one workgroup)
-        if (g_splitk <= 1 && (long)((M + 191) / 192) * (N / 128) > cu_count())
+        if (g_splitk <= 1 && ((EPI == EPI_SILU && K <= 832) || (long)((M + 191) / 192) * (N / 128) > cu_count()))
           return launch_pairs<192, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
       return launch<192, 128, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);
     case 8: return launch<192, 256, EPI, NORM>(Wt, X, ldx, M, K, N, up_off, out, ldo, eps, ea, st);

@@ -1157,10 +1157,11 @@ def test_residual_products_of_long_rows(M, tile):
 
 
 @pytest.mark.parametrize("K", [64, 128, 192, 448])       # one stage of K, two, and more than are there at once
-@pytest.mark.parametrize("M", [257, 385])                # ragged rows of the second and the third tile
+@pytest.mark.parametrize("M", [100, 257, 385])           # one round; ragged rows of the second and the third tile
 @pytest.mark.parametrize("epi", ["store", "store_norm", "silu", "resid"])
 def test_tiled_gemm_rounds_of_192_rows(epi, M, K):
-    """192 x 128 tiles of more than a round of the CUs, which share a CU in pairs, against the fp32 product."""
+    """192 x 128 tiles of more than a round of the CUs, and SwiGLU's of a short K, which share a CU in pairs, and the others of
+    one round, against the fp32 product."""
     from p2p_llm_chat_go_amd.ops.gemm import set_tiled_min_m, tiled_config
 
     torch.manual_seed(M + K)
